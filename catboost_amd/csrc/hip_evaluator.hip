@@ -436,6 +436,10 @@ TBucketGrid MakeBucketGrid(const std::vector<float>& borders) {
 
 constexpr size_t kMaxTileLdsBytes = 160 * 1024;
 
+// Workgroups wanted of a leaf index launch: 200 000 documents * 1000 trees (782 blocks, 2 workgroups per CU) take 180 us as
+// 782 workgroups, 165 as 2346, 199 as 4692 (shorter runs of a row, the bins read more often).
+constexpr size_t kLeafIndexWorkgroups = 2048;
+
 // LDS of the tile kernel without leaf regions: the bins of 256 documents and the accumulator
 size_t TileLdsBytes(uint32_t buckets, int dchunk) {
     return ((static_cast<size_t>(buckets) * dev::kDocsPerBlock + 7) & ~size_t(7)) +
@@ -3067,18 +3071,28 @@ void THipEvaluator::LeafIndexesQuantizedDevice(const uint8_t* bins, size_t docCo
     CBAMD_ENSURE(bins != nullptr && indexes != nullptr, "null pointer passed to leaf index calculation");
     hipStream_t s = m.Pick(stream);
     const size_t blocks = (docCount + 255) / 256;
-    const size_t tileLds = static_cast<size_t>(m.LayoutBuckets) * dev::kDocsPerBlock + dev::kWave * dev::kLeafIndexPitch * 4;
-    if (m.Oblivious && m.MaxDepth <= 8 && m.PackedTrees.Get() != nullptr && tileLds <= kMaxTileLdsBytes) {
+    const size_t tileLds = static_cast<size_t>(m.LayoutBuckets) * dev::kDocsPerBlock + dev::kDocsPerBlock * dev::kLeafIndexPitch * 4;
+    if (m.Oblivious && m.MaxDepth <= 8 && m.PackedTrees.Get() != nullptr && tileLds <= kMaxTileLdsBytes &&
+        docCount < (size_t(1) << 31)) {
+        // shares of the trees: enough workgroups for the chip's 256 CUs to go through them a few times over
+        const size_t groups = (treeEnd - treeStart + dev::kLeafIndexGroup - 1) / dev::kLeafIndexGroup;
+        const size_t wanted = std::max<size_t>(1, std::min<size_t>(groups, (kLeafIndexWorkgroups + blocks - 1) / blocks));
+        const size_t shareGroups = (groups + wanted - 1) / wanted;
+        const size_t shares = (groups + shareGroups - 1) / shareGroups;
+        CBAMD_ENSURE(blocks * shares < (size_t(1) << 31), "batch is too large for one leaf index launch");
         const auto launch = [&](auto kernel) {
             EnsureDynamicLds(reinterpret_cast<const void*>(kernel), tileLds);
-            hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks)), dim3(256), tileLds, s,
-                               reinterpret_cast<const uint32_t*>(bins), docCount, m.LayoutBuckets, m.PackedTrees.Get(),
-                               static_cast<uint32_t>(treeStart), static_cast<uint32_t>(treeEnd), indexes);
+            hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks * shares)), dim3(dev::kLeafIndexThreads), tileLds, s,
+                               reinterpret_cast<const uint32_t*>(bins), static_cast<uint32_t>(docCount), m.LayoutBuckets,
+                               m.PackedTrees.Get(), static_cast<uint32_t>(treeStart), static_cast<uint32_t>(treeEnd),
+                               static_cast<uint32_t>(shares), static_cast<uint32_t>(shareGroups * dev::kLeafIndexGroup), indexes);
         };
-        if (m.PackedSevenBit) {
-            launch(dev::LeafIndexesTileKernel<true>);
+        if (m.PackedSevenBit && m.MaxDepth <= 6) {
+            launch(dev::LeafIndexesTileKernel<true, 6>);
+        } else if (m.PackedSevenBit) {
+            launch(dev::LeafIndexesTileKernel<true, 8>);
         } else {
-            launch(dev::LeafIndexesTileKernel<false>);
+            launch(dev::LeafIndexesTileKernel<false, 8>);
         }
         HIP_CHECK(hipGetLastError());
         return;

@@ -859,6 +859,32 @@ __device__ __forceinline__ uint32_t TreeIndexes(const uint8_t* laneTile, uint32_
     return idx4 >> (8 - MAXD);
 }
 
+// The same for four trees whose packed rows sit side by side in the lanes of `packedRows` (kPackedTreeDwords lanes
+// each): all LDS reads of the four trees are in flight before the first compare.
+template <bool SEVEN_BIT, int MAXD>
+__device__ __forceinline__ void FourTreesIndexes(const uint8_t* laneTile, uint32_t packedRows, uint32_t (&idx)[4]) {
+    uint32_t a[4][MAXD];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int d = 0; d < MAXD; ++d) {
+            const uint32_t level = __builtin_amdgcn_readlane(packedRows, i * kPackedTreeDwords + d);
+            a[i][d] = *reinterpret_cast<const uint32_t*>(laneTile + LevelTileOffset<SEVEN_BIT>(level));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t idx4 = 0;
+#pragma unroll
+        for (int d = 0; d < MAXD; ++d) {
+            const uint32_t level = __builtin_amdgcn_readlane(packedRows, i * kPackedTreeDwords + d);
+            const uint32_t r = CompareBytes<SEVEN_BIT>(a[i][d], level);
+            idx4 = (r & 0x80808080u) | ((idx4 >> 1) & 0x7f7f7f7fu);
+        }
+        idx[i] = idx4 >> (8 - MAXD);
+    }
+}
+
 // Oblivious trees of depth <= MAXD <= 8 whose bins fit an LDS tile: one workgroup of kTileWaves
 // waves per 256-document block. The block's bins (buckets x 256 bytes) are copied to LDS once;
 // the waves share the tile and split the trees among themselves (tree t goes to wave
@@ -2805,53 +2831,130 @@ __global__ __launch_bounds__(256) void LeafIndexesKernel(const uint8_t* __restri
     }
 }
 
-// Leaf indexes of oblivious trees of depth <= 8 whose 256-document tile of bins fits LDS: the byte-parallel walk of
-// the tile kernel (four documents per lane, a tree per wave and turn), and rows of the output written whole. A
-// workgroup of four waves takes a block of 256 documents and the trees in groups of 64: wave w walks trees
-// 16 w .. 16 w + 15 of the group and leaves each tree's four index bytes per lane in LDS ([lane][tree], 65 dwords
-// per lane); then wave j writes, document by document, the 64 indexes of documents 64 j .. 64 j + 63: one 256-byte
-// store per document and group where the plain kernel stores four bytes per (document, tree) a row apart.
-// packedTrees as in EvalObliviousTileKernel. grid = doc blocks, block = 256, dynamic LDS = buckets * 256 + 64 * 65 * 4.
+// Leaf indexes of oblivious trees of depth <= MAXD <= 8 whose 256-document tile of bins fits LDS: the byte-parallel walk
+// of the tile kernels (four documents per lane, a tree per wave and turn, its levels broadcast from a lane's register), and
+// rows of the output written whole. What bounds it is the output, four bytes per document and tree. A workgroup of eight
+// waves takes a block of 256 documents and a share of the trees in groups of 64: wave w walks trees 8 w .. 8 w + 7 of
+// the group, four at a time, turns the four bytes of four trees into the four bytes of a document (a 4 x 4 transpose of
+// bytes) and leaves them in LDS, a ring of 128 trees per document, a byte each; then sixteen threads write 64 indexes of
+// a document, 16 bytes a thread. The 64 indexes are those that fill whole 128-byte lines of the output, up to 31 trees
+// behind the group, which the ring still holds: rows of 4 * trees bytes start anywhere in a line, and lines written in two
+// parts cost the memory twice. 200 000 documents * 1000 trees of depth 6 over 100 features: 466 us with a workgroup per
+// block and 4-byte stores, 227 with shares and 16-byte stores, 165 with whole lines (4.85 TB/s).
+// A share is some groups of 64 trees: the grid is blocks * shares, so that a batch of a few hundred blocks still fills
+// the chip a few times over (one workgroup per block left a last generation nearly empty).
+// packedTrees as in EvalObliviousTileKernel. block = 512 threads, dynamic LDS = buckets * 256 + 256 * 33 * 4.
 constexpr int kLeafIndexGroup = 64;
-constexpr int kLeafIndexPitch = kLeafIndexGroup + 1;
+constexpr int kLeafIndexThreads = 512;
+constexpr int kLeafIndexRing = 2 * kLeafIndexGroup / 4;   // dwords of a document's ring
+constexpr int kLeafIndexPitch = kLeafIndexRing + 1;
+constexpr int kLeafIndexLine = 32;                        // dwords of a line of the output
 
-template <bool SEVEN_BIT>
-__global__ __launch_bounds__(256) void LeafIndexesTileKernel(const uint32_t* __restrict__ bins, size_t docCount,
-                                                             uint32_t bucketCount, const uint32_t* __restrict__ packedTrees,
-                                                             uint32_t treeBegin, uint32_t treeEnd,
-                                                             uint32_t* __restrict__ out) {
+template <bool SEVEN_BIT, int MAXD>
+__global__ __launch_bounds__(kLeafIndexThreads) void LeafIndexesTileKernel(
+    const uint32_t* __restrict__ bins, uint32_t docCount, uint32_t bucketCount, const uint32_t* __restrict__ packedTrees,
+    uint32_t treeBegin, uint32_t treeEnd, uint32_t shares, uint32_t shareTrees, uint32_t* __restrict__ out) {
     extern __shared__ uint32_t sTile[];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (kWave - 1);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const size_t block = blockIdx.x;
-    const uint32_t tileDwords = bucketCount * kWave;
-    const uint32_t* src = bins + block * tileDwords;
-    for (uint32_t i = tid; i < tileDwords; i += 256) {
-        sTile[i] = src[i];
+    // the shares of a block go to one XCD one after the other, so that they read its bins from one L2
+    const uint32_t perXcd = gridDim.x / kXcdCount, extra = gridDim.x % kXcdCount;
+    const uint32_t xcd = blockIdx.x % kXcdCount;
+    const uint32_t work = xcd * perXcd + min(xcd, extra) + blockIdx.x / kXcdCount;
+    const uint32_t block = work / shares;
+    // A share ends, document by document, where a line ends; the next one walks the trees of a line more in front.
+    const bool firstShare = work % shares == 0, lastShare = work % shares == shares - 1;
+    const int32_t lead = firstShare ? 0 : kLeafIndexLine;
+    const uint32_t firstTree = treeBegin + (work % shares) * shareTrees - lead;
+    const int32_t count = lastShare ? treeEnd - firstTree : shareTrees + lead;  // trees that are walked
+    const uint32_t tilePieces = bucketCount * (kWave / 4);
+    const uint4* src = reinterpret_cast<const uint4*>(bins) + static_cast<size_t>(block) * tilePieces;
+    for (uint32_t i = tid; i < tilePieces; i += kLeafIndexThreads) {
+        reinterpret_cast<uint4*>(sTile)[i] = src[i];
     }
-    uint32_t* stage = sTile + tileDwords;
+    uint32_t* ring = sTile + bucketCount * kWave;
     const uint8_t* laneTile = reinterpret_cast<const uint8_t*>(sTile) + lane * 4;
-    const uint32_t slot = lane & (kPackedTreeDwords - 1);
     const size_t treeCount = treeEnd - treeBegin;
-    const size_t firstDoc = block * kDocsPerBlock + wave * kWave;  // of the 64 documents this wave writes
-    for (uint32_t group = treeBegin; group < treeEnd; group += kLeafIndexGroup) {
+    const uint32_t blockDocs = min(static_cast<uint32_t>(kDocsPerBlock), docCount - block * kDocsPerBlock);
+    uint32_t* blockOut = out + static_cast<size_t>(block) * kDocsPerBlock * treeCount + (firstTree - treeBegin);
+    constexpr int kWaves = kLeafIndexThreads / kWave;
+    constexpr int kPerWave = kLeafIndexGroup / kWaves;
+    // the packed rows of the wave's trees of a group, four trees to a register, fetched a group ahead; trees past
+    // the share are walked as its last tree and not written
+    uint32_t rows[kPerWave / 4];
+    const auto fetchRows = [&](int32_t group) {
+#pragma unroll
+        for (int q = 0; q < kPerWave / 4; ++q) {
+            const int32_t t = min(group + static_cast<int32_t>(wave * kPerWave + q * 4 + lane / kPackedTreeDwords), count - 1);
+            rows[q] = packedTrees[static_cast<size_t>(firstTree + t) * kPackedTreeDwords + lane % kPackedTreeDwords];
+        }
+    };
+    fetchRows(0);
+    for (int32_t group = 0; group < count; group += kLeafIndexGroup) {
         __syncthreads();  // the tile is loaded; the previous group's indexes are written
-        constexpr int kPerWave = kLeafIndexGroup / 4;
-#pragma unroll 4
-        for (int k = 0; k < kPerWave; ++k) {
-            const uint32_t t = group + wave * kPerWave + k;
-            if (t < treeEnd) {
-                const uint32_t row = packedTrees[static_cast<size_t>(t) * kPackedTreeDwords + slot];
-                stage[lane * kLeafIndexPitch + wave * kPerWave + k] = TreeIndexes<SEVEN_BIT, 8>(laneTile, row);
-            }
+#pragma unroll
+        for (int q = 0; q < kPerWave / 4; ++q) {
+            uint32_t idx[4];
+            FourTreesIndexes<SEVEN_BIT, MAXD>(laneTile, rows[q], idx);
+            const uint32_t low01 = __builtin_amdgcn_perm(idx[1], idx[0], 0x05010400u);  // documents 0 and 1, trees 0 and 1
+            const uint32_t high01 = __builtin_amdgcn_perm(idx[1], idx[0], 0x07030602u);
+            const uint32_t low23 = __builtin_amdgcn_perm(idx[3], idx[2], 0x05010400u);
+            const uint32_t high23 = __builtin_amdgcn_perm(idx[3], idx[2], 0x07030602u);
+            uint32_t* cell = ring + lane * kLeafIndexPitch + (group / 4 + wave * (kPerWave / 4) + q) % kLeafIndexRing;
+            cell[0 * kWave * kLeafIndexPitch] = __builtin_amdgcn_perm(low23, low01, 0x05040100u);
+            cell[1 * kWave * kLeafIndexPitch] = __builtin_amdgcn_perm(low23, low01, 0x07060302u);
+            cell[2 * kWave * kLeafIndexPitch] = __builtin_amdgcn_perm(high23, high01, 0x05040100u);
+            cell[3 * kWave * kLeafIndexPitch] = __builtin_amdgcn_perm(high23, high01, 0x07060302u);
         }
         __syncthreads();
-        const uint32_t tree = group + lane;
-        for (uint32_t d = 0; d < kWave; ++d) {
-            const size_t doc = firstDoc + d;
-            if (doc < docCount && tree < treeEnd) {
-                out[doc * treeCount + (tree - treeBegin)] = (stage[d * kLeafIndexPitch + lane] >> (8 * wave)) & 0xffu;
+        fetchRows(group + kLeafIndexGroup);
+        const int32_t done = min(group + kLeafIndexGroup, count);  // trees whose indexes are in the ring
+        const int32_t quadTree = group + static_cast<int32_t>(tid % 16) * 4;
+        // the indexes of trees `tree` .. tree + 3 of the document whose ring starts at `cells`
+        const auto ringQuad = [&](const uint32_t* cells, int32_t tree) {
+            const uint32_t at = static_cast<uint32_t>(tree + 4 * kLeafIndexRing) / 4;
+            const uint32_t bytes = __builtin_amdgcn_alignbyte(cells[(at + 1) % kLeafIndexRing], cells[at % kLeafIndexRing],
+                                                              static_cast<uint32_t>(tree) & 3u);
+            return make_uint4(bytes & 0xffu, (bytes >> 8) & 0xffu, (bytes >> 16) & 0xffu, bytes >> 24);
+        };
+        constexpr uint32_t kDocsPerPass = kLeafIndexThreads / 16;
+        if (group > 0 && (done < count || !lastShare)) {
+            // inside a row: two whole lines per document (fewer behind a share's last, shorter group)
+            uint32_t* row = blockOut + (tid / 16) * treeCount;
+            const uint32_t* cells = ring + (tid / 16) * kLeafIndexPitch;
+            const int32_t groupTrees = done - group;
+#pragma unroll
+            for (uint32_t pass = 0; pass < kDocsPerBlock / kDocsPerPass; ++pass) {
+                const int32_t behind = static_cast<int32_t>((reinterpret_cast<uintptr_t>(row) / 4) % kLeafIndexLine);
+                const uint4 quad = ringQuad(cells, quadTree - behind);
+                if (pass * kDocsPerPass + tid / 16 < blockDocs && quadTree - group < groupTrees) {
+                    *reinterpret_cast<uint4*>(row + (quadTree - behind)) = quad;
+                }
+                row += kDocsPerPass * treeCount;
+                cells += kDocsPerPass * kLeafIndexPitch;
+            }
+            continue;
+        }
+        for (uint32_t d = tid / 16; d < blockDocs; d += kDocsPerPass) {
+            uint32_t* row = blockOut + d * treeCount;
+            const int32_t behind = static_cast<int32_t>((reinterpret_cast<uintptr_t>(row) / 4) % kLeafIndexLine);
+            // whole lines only, but for the row's first and last
+            const int32_t begin = group > 0 ? group - behind : firstShare ? 0 : lead - behind;
+            const int32_t end = done == count && lastShare ? count : done - behind;
+            for (int32_t tree = quadTree - behind; tree < end; tree += kLeafIndexGroup) {
+                const uint4 quad = ringQuad(ring + d * kLeafIndexPitch, tree);
+                if (tree >= begin && tree + 4 <= end) {
+                    *reinterpret_cast<uint4*>(row + tree) = quad;
+                } else {
+                    const uint32_t values[4] = {quad.x, quad.y, quad.z, quad.w};
+#pragma unroll
+                    for (int32_t i = 0; i < 4; ++i) {
+                        if (tree + i >= begin && tree + i < end) {
+                            row[tree + i] = values[i];
+                        }
+                    }
+                }
             }
         }
     }
