@@ -9,6 +9,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <limits>
+#include <numeric>
 #include <string>
 #include <thread>
 #include <tuple>
@@ -806,24 +807,113 @@ struct TFeaturePositions {
     }
 };
 
+// One feature's value of one row of its table, static_ctr_provider.cpp:52-126: one branch per CTR type, the row null
+// where the table does not know the hash. Single roundings throughout, as TModelCtr::Calc (online_ctr.h:290-293).
+float CtrValueOfRow(const TModelCtr& ctr, const TCtrValueTable& table, const uint8_t* row) {
+    const auto counter = [&](size_t i) {
+        uint32_t v;
+        std::memcpy(&v, row + 4 * i, 4);
+        return v;
+    };
+    const auto asFloat = [](uint32_t v) { return static_cast<float>(static_cast<int32_t>(v)); };
+    const int classes = table.TargetClassesCount;
+    switch (ctr.Base.CtrType) {
+        case ECtrType::BinarizedTargetMeanValue:
+        case ECtrType::FloatTargetMeanValue: {
+            if (!row) {
+                return ctr.Calc(0.f, 0.f);
+            }
+            float sum;
+            std::memcpy(&sum, row, 4);
+            return ctr.Calc(sum, asFloat(counter(1)));
+        }
+        case ECtrType::Counter:
+        case ECtrType::FeatureFreq:
+            return ctr.Calc(row ? asFloat(counter(0)) : 0.f, static_cast<float>(table.CounterDenominator));
+        case ECtrType::Buckets: {
+            if (!row) {
+                return ctr.Calc(0.f, 0.f);
+            }
+            uint32_t total = 0;
+            for (int c = 0; c < classes; ++c) {
+                total += counter(c);
+            }
+            return ctr.Calc(asFloat(counter(ctr.TargetBorderIdx)), asFloat(total));
+        }
+        case ECtrType::Borders: {
+            if (!row) {
+                return ctr.Calc(0.f, 0.f);
+            }
+            if (classes <= 2) {
+                return ctr.Calc(asFloat(counter(1)), asFloat(counter(0) + counter(1)));
+            }
+            uint32_t good = 0, total = 0;
+            for (int c = 0; c < classes; ++c) {
+                total += counter(c);
+                good += c > ctr.TargetBorderIdx ? counter(c) : 0u;
+            }
+            return ctr.Calc(asFloat(good), asFloat(total));
+        }
+    }
+    return 0.f;
+}
+
+// The rows of a table in the order in which TDenseIndexHashView::GetIndex (helpers/dense_hash_view.h:46-56) would come
+// upon them: `found(hash, row)` for every bucket that a look-up of its own hash reaches before an empty bucket.
+template <typename TFound>
+void ForEachCtrRow(const TCtrValueTable& table, const TFound& found) {
+    const size_t bucketCount = table.IndexHashRaw.size() / 12, mask = bucketCount - 1;
+    const auto bucket = [&](size_t at, uint64_t* hash, uint32_t* row) {
+        std::memcpy(hash, table.IndexHashRaw.data() + 12 * at, 8);
+        std::memcpy(row, table.IndexHashRaw.data() + 12 * at + 8, 4);
+    };
+    constexpr uint64_t kEmpty = ~uint64_t(0);
+    uint64_t hash;
+    uint32_t row;
+    size_t start = 0;
+    for (; start < bucketCount; ++start) {
+        bucket(start, &hash, &row);
+        if (hash == kEmpty) {
+            break;
+        }
+    }
+    size_t run = 0;  // taken buckets between the last empty one and this one
+    for (size_t i = 1; i < bucketCount; ++i) {
+        const size_t at = (start + i) & mask;
+        bucket(at, &hash, &row);
+        if (hash == kEmpty) {
+            run = 0;
+            continue;
+        }
+        if (((at - hash) & mask) <= run) {
+            found(hash, row);
+        }
+        ++run;
+    }
+}
+
 // Device tables of the model's CTR features (TStaticCtrProvider, catboost/libs/model/static_ctr_provider.cpp):
-// per feature a descriptor and its projection (SetupBinFeatureIndexes, :142-178, resolved to bucket
-// numbers and input columns), all index buckets and all rows. Every row index and class index the kernel
-// can reach is checked here, so a damaged model fails at load instead of reading out of bounds.
+// per projection a descriptor, the projection itself (SetupBinFeatureIndexes, :142-178, resolved to bucket
+// numbers and input columns) and one hash table that holds, per hash that any of the projection's tables of learned
+// statistics knows, the bins of all the projection's CTR features (dev::TCtrGroupDev). Every row index and class index
+// is checked here, so a damaged model fails at load instead of reading out of bounds.
 // Appends one bucket entry per 254 borders of a CTR feature to the binarize bucket tables.
+struct TCtrDeviceTables {
+    TDeviceVec<uint32_t> Groups, Items, Table, Buckets, CatColumnsFlat, CatColumnsSplit;
+    uint32_t CatColumnCount = 0;
+    uint32_t GroupCount = 0;
+};
+
 void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions,
                     const std::vector<TCtrValueTable>& tables, std::vector<uint32_t>* srcFlat,
                     std::vector<uint32_t>* srcSplit, std::vector<uint32_t>* offsets, std::vector<uint32_t>* flags,
-                    std::vector<uint32_t>* values, TDeviceVec<uint32_t>* featuresOut, TDeviceVec<uint32_t>* itemsOut,
-                    TDeviceVec<uint32_t>* indexOut, TDeviceVec<uint32_t>* blobOut, TDeviceVec<uint32_t>* catColumnsFlatOut,
-                    TDeviceVec<uint32_t>* catColumnsSplitOut, uint32_t* catColumnCountOut) {
-    static_assert(sizeof(dev::TCtrFeatureDev) == 64 && sizeof(dev::TCtrItemDev) == 16, "device CTR records changed size");
-    std::vector<dev::TCtrFeatureDev> features;
+                    std::vector<uint32_t>* values, TCtrDeviceTables* result) {
+    static_assert(sizeof(dev::TCtrGroupDev) == 32 && sizeof(dev::TCtrItemDev) == 16, "device CTR records changed size");
+    std::vector<dev::TCtrGroupDev> groups;
     std::vector<dev::TCtrItemDev> items;
-    std::vector<uint32_t> index, blob;
     std::vector<uint32_t> catColumnsFlat, catColumnsSplit;  // distinct categorical columns of all projections
-    std::vector<uint32_t> tableIndexBegin(tables.size(), 0), tableBlobBegin(tables.size(), 0), tableRows(tables.size(), 0);
-    std::vector<bool> tableUploaded(tables.size(), false);
+    std::vector<bool> tableChecked(tables.size(), false);
+    std::vector<uint32_t> tableRows(tables.size(), 0);
 
     // first bucket of every used float feature and of every one-hot feature
     std::vector<uint32_t> floatFirstBucket(trees.FloatFeatures.size(), 0), oneHotFirstBucket(trees.OneHotFeatures.size(), 0);
@@ -837,6 +927,14 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
         bucket += static_cast<uint32_t>((trees.OneHotFeatures[i].Values.size() + kMaxValuesPerBin - 1) / kMaxValuesPerBin);
     }
 
+    // the features: their tables, checked, and their buckets
+    struct TFeature {
+        size_t Table = 0;
+        size_t RowBytes = 0;
+        uint32_t FirstBucket = 0, BucketCount = 0;
+    };
+    std::vector<TFeature> features;
+    std::vector<std::vector<size_t>> groupFeatures;
     for (const auto& feature : trees.CtrFeatures) {
         const TModelCtr& ctr = feature.Ctr;
         size_t t = 0;
@@ -876,17 +974,14 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
                 }
                 break;
         }
-        if (!tableUploaded[t]) {
-            tableUploaded[t] = true;
-            tableIndexBegin[t] = static_cast<uint32_t>(index.size() / 3);
-            tableBlobBegin[t] = static_cast<uint32_t>(blob.size());
+        if (!tableChecked[t]) {
+            tableChecked[t] = true;
             bool hasEmpty = false;
             uint32_t maxRow = 0;
             bool anyRow = false;
             for (size_t b = 0; b < bucketCount; ++b) {
                 uint32_t w[3];
                 std::memcpy(w, table.IndexHashRaw.data() + 12 * b, 12);
-                index.insert(index.end(), w, w + 3);
                 if ((w[0] & w[1]) == 0xffffffffu) {
                     hasEmpty = true;
                 } else {
@@ -895,19 +990,53 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
                 }
             }
             CBAMD_ENSURE(hasEmpty, "CTR index hash table has no empty bucket");
+            CBAMD_ENSURE(maxRow != 0xffffffffu || !anyRow, "CTR value table is shorter than its index");
             tableRows[t] = anyRow ? maxRow + 1 : 0;
-            blob.resize(blob.size() + (table.CTRBlob.size() + 3) / 4, 0);
-            if (!table.CTRBlob.empty()) {
-                std::memcpy(blob.data() + tableBlobBegin[t], table.CTRBlob.data(), table.CTRBlob.size());
-            }
-            CBAMD_ENSURE(index.size() / 3 < (size_t(1) << 32) && blob.size() < (size_t(1) << 32), "CTR tables are too large");
         }
         CBAMD_ENSURE(static_cast<size_t>(tableRows[t]) * rowBytes <= table.CTRBlob.size(),
                      "CTR value table is shorter than its index");
+        TFeature f;
+        f.Table = t;
+        f.RowBytes = rowBytes;
+        f.FirstBucket = static_cast<uint32_t>(srcFlat->size());
+        for (size_t begin = 0; begin < feature.Borders.size(); begin += kMaxValuesPerBin) {
+            const size_t end = std::min(begin + kMaxValuesPerBin, feature.Borders.size());
+            std::vector<float> b;
+            for (size_t i = begin; i < end; ++i) {
+                if (!std::isnan(feature.Borders[i])) {
+                    b.push_back(feature.Borders[i]);
+                }
+            }
+            std::sort(b.begin(), b.end());
+            for (float x : b) {
+                uint32_t bits;
+                std::memcpy(&bits, &x, 4);
+                values->push_back(bits);
+            }
+            offsets->push_back(static_cast<uint32_t>(values->size()));
+            srcFlat->push_back(0);
+            srcSplit->push_back(0);
+            flags->push_back(dev::kBucketFlagCtr);
+        }
+        f.BucketCount = static_cast<uint32_t>(srcFlat->size()) - f.FirstBucket;
+        size_t g = 0;
+        while (g < groupFeatures.size() &&
+               !(trees.CtrFeatures[groupFeatures[g].front()].Ctr.Base.Projection == ctr.Base.Projection)) {
+            ++g;
+        }
+        if (g == groupFeatures.size()) {
+            groupFeatures.emplace_back();
+        }
+        groupFeatures[g].push_back(features.size());
+        features.push_back(f);
+    }
 
-        dev::TCtrFeatureDev f{};
-        f.ItemBegin = static_cast<uint32_t>(items.size());
-        for (int catIndex : ctr.Base.Projection.CatFeatures) {
+    std::vector<uint32_t> table, buckets;
+    for (const std::vector<size_t>& members : groupFeatures) {
+        const TFeatureCombination& projection = trees.CtrFeatures[members.front()].Ctr.Base.Projection;
+        dev::TCtrGroupDev group{};
+        group.ItemBegin = static_cast<uint32_t>(items.size());
+        for (int catIndex : projection.CatFeatures) {
             const TCatFeature* cat = nullptr;
             for (const auto& c : trees.CatFeatures) {
                 if (c.Index == catIndex && c.UsedInModel) {
@@ -930,7 +1059,7 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
             }
             items.push_back({dev::kCtrItemCat, static_cast<uint32_t>(at.FlatIndex), static_cast<uint32_t>(at.Index), tileRow});
         }
-        for (const auto& split : ctr.Base.Projection.BinFeatures) {
+        for (const auto& split : projection.BinFeatures) {
             bool found = false;
             for (size_t i = 0; i < trees.FloatFeatures.size() && !found; ++i) {
                 const auto& ff = trees.FloatFeatures[i];
@@ -948,7 +1077,7 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
             }
             CBAMD_ENSURE(found, "CTR projection refers to a float split the model does not have");
         }
-        for (const auto& split : ctr.Base.Projection.OneHotFeatures) {
+        for (const auto& split : projection.OneHotFeatures) {
             bool found = false;
             for (size_t i = 0; i < trees.OneHotFeatures.size() && !found; ++i) {
                 const auto& oh = trees.OneHotFeatures[i];
@@ -966,57 +1095,123 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
             }
             CBAMD_ENSURE(found, "CTR projection refers to a one-hot split the model does not have");
         }
-        f.ItemEnd = static_cast<uint32_t>(items.size());
-        f.HashBuckets = tableIndexBegin[t];
-        f.HashMask = static_cast<uint32_t>(bucketCount - 1);
-        f.BlobOffset = tableBlobBegin[t];
-        f.Type = static_cast<uint32_t>(ctr.Base.CtrType);
-        f.TargetBorderIdx = ctr.TargetBorderIdx;
-        f.TargetClassesCount = table.TargetClassesCount;
-        f.CounterDenominator = table.CounterDenominator;
-        f.PriorNum = ctr.PriorNum;
-        f.PriorDenom = ctr.PriorDenom;
-        f.Shift = ctr.Shift;
-        f.Scale = ctr.Scale;
-        f.FirstBucket = static_cast<uint32_t>(srcFlat->size());
-        for (size_t begin = 0; begin < feature.Borders.size(); begin += kMaxValuesPerBin) {
-            const size_t end = std::min(begin + kMaxValuesPerBin, feature.Borders.size());
-            std::vector<float> b;
-            for (size_t i = begin; i < end; ++i) {
-                if (!std::isnan(feature.Borders[i])) {
-                    b.push_back(feature.Borders[i]);
-                }
+        group.ItemEnd = static_cast<uint32_t>(items.size());
+        group.FirstBucket = static_cast<uint32_t>(buckets.size());
+        std::vector<uint32_t> firstByte;  // of every member's bins in an entry
+        for (size_t i : members) {
+            firstByte.push_back(group.BucketCount);
+            for (uint32_t k = 0; k < features[i].BucketCount; ++k) {
+                buckets.push_back(features[i].FirstBucket + k);
             }
-            std::sort(b.begin(), b.end());
-            for (float x : b) {
-                uint32_t bits;
-                std::memcpy(&bits, &x, 4);
-                values->push_back(bits);
-            }
-            offsets->push_back(static_cast<uint32_t>(values->size()));
-            srcFlat->push_back(0);
-            srcSplit->push_back(0);
-            flags->push_back(dev::kBucketFlagCtr);
+            group.BucketCount += features[i].BucketCount;
         }
-        f.BucketCount = static_cast<uint32_t>(srcFlat->size()) - f.FirstBucket;
-        f.SameProjectionAsPrevious =
-            !features.empty() && trees.CtrFeatures[features.size() - 1].Ctr.Base.Projection == ctr.Base.Projection ? 1u : 0u;
-        features.push_back(f);
+        // the bins of member i for a row of its table (null: unknown hash)
+        const auto fillBins = [&](size_t i, const uint8_t* row, uint8_t* bins) {
+            const TFeature& f = features[members[i]];
+            const float value = CtrValueOfRow(trees.CtrFeatures[members[i]].Ctr, tables[f.Table], row);
+            for (uint32_t k = 0; k < f.BucketCount; ++k) {
+                const uint32_t begin = (*offsets)[f.FirstBucket + k], end = (*offsets)[f.FirstBucket + k + 1];
+                const float* borders = reinterpret_cast<const float*>(values->data());
+                // the number of borders below the value (none below a NaN)
+                bins[firstByte[i] + k] = static_cast<uint8_t>(std::lower_bound(borders + begin, borders + end, value) - (borders + begin));
+            }
+        };
+        // members of one table follow each other, so that each table is gone through once
+        std::vector<size_t> order(members.size());
+        std::iota(order.begin(), order.end(), size_t(0));
+        std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return features[members[a]].Table < features[members[b]].Table; });
+        size_t keys = 0;  // at most: a hash known to several tables is counted for each
+        for (size_t i = 0; i < order.size(); ++i) {
+            const size_t t = features[members[order[i]]].Table;
+            if (i == 0 || t != features[members[order[i - 1]]].Table) {
+                size_t rows = 0;
+                ForEachCtrRow(tables[t], [&](uint64_t, uint32_t) { ++rows; });
+                keys = std::max(keys, rows);
+            }
+        }
+        group.EntryPieces = (8 + group.BucketCount + 15) / 16;
+        const size_t entryDwords = 4 * static_cast<size_t>(group.EntryPieces);
+        const size_t firstDword = table.size();
+        CBAMD_ENSURE(firstDword / 4 < (size_t(1) << 32), "CTR tables are too large");
+        group.FirstPiece = static_cast<uint32_t>(firstDword / 4);
+        std::vector<uint32_t> unknown(entryDwords, 0);
+        unknown[0] = unknown[1] = 0xffffffffu;
+        for (size_t i = 0; i < members.size(); ++i) {
+            fillBins(i, nullptr, reinterpret_cast<uint8_t*>(unknown.data() + 2));
+        }
+        // Tables of one projection were learned on the same documents and know the same hashes; where they do not, the
+        // union may pass half of the entries, and the table is built again with twice as many.
+        size_t entries = 2;
+        while (entries < 2 * keys) {
+            entries *= 2;
+        }
+        const auto build = [&] {
+            CBAMD_ENSURE(entries <= (size_t(1) << 31), "CTR tables are too large");
+            table.resize(firstDword);
+            table.reserve(firstDword + entries * entryDwords);
+            for (size_t e = 0; e < entries; ++e) {
+                table.insert(table.end(), unknown.begin(), unknown.end());
+            }
+            group.HashMask = static_cast<uint32_t>(entries - 1);
+            std::vector<uint32_t> filledBy(entries, 0);  // a hash that a damaged table holds twice: the first one counts
+            size_t taken = 0;
+            bool fits = true;
+            for (size_t first = 0, last = 0; first < order.size(); first = last) {
+                const size_t t = features[members[order[first]]].Table;
+                while (last < order.size() && features[members[order[last]]].Table == t) {
+                    ++last;
+                }
+                ForEachCtrRow(tables[t], [&](uint64_t hash, uint32_t row) {
+                    size_t at = static_cast<size_t>(hash) & (entries - 1);
+                    const auto hashAt = [&] {
+                        const uint32_t* e = table.data() + firstDword + at * entryDwords;
+                        return e[0] | (static_cast<uint64_t>(e[1]) << 32);
+                    };
+                    while (hashAt() != hash && hashAt() != ~uint64_t(0)) {
+                        at = (at + 1) & (entries - 1);
+                    }
+                    uint32_t* entry = table.data() + firstDword + at * entryDwords;
+                    if (hashAt() != hash) {
+                        if (!fits || 2 * (taken + 1) > entries) {
+                            fits = false;
+                            return;
+                        }
+                        ++taken;
+                        entry[0] = static_cast<uint32_t>(hash);
+                        entry[1] = static_cast<uint32_t>(hash >> 32);
+                    }
+                    if (filledBy[at] == last) {
+                        return;
+                    }
+                    filledBy[at] = static_cast<uint32_t>(last);
+                    for (size_t i = first; i < last; ++i) {
+                        fillBins(order[i], tables[t].CTRBlob.data() + static_cast<size_t>(row) * features[members[order[i]]].RowBytes,
+                                 reinterpret_cast<uint8_t*>(entry + 2));
+                    }
+                });
+            }
+            return fits;
+        };
+        while (!build()) {
+            entries *= 2;
+        }
+        groups.push_back(group);
     }
-    std::vector<uint32_t> raw(features.size() * (sizeof(dev::TCtrFeatureDev) / 4));
-    std::memcpy(raw.data(), features.data(), raw.size() * 4);
-    featuresOut->Upload(raw);
-    raw.assign(std::max<size_t>(items.size(), 1) * (sizeof(dev::TCtrItemDev) / 4), 0);
-    std::memcpy(raw.data(), items.data(), items.size() * sizeof(dev::TCtrItemDev));
-    itemsOut->Upload(raw);
-    indexOut->Upload(index);
-    if (blob.empty()) {
-        blob.push_back(0);
-    }
-    blobOut->Upload(blob);
-    *catColumnCountOut = static_cast<uint32_t>(catColumnsFlat.size());
-    catColumnsFlatOut->Upload(catColumnsFlat);
-    catColumnsSplitOut->Upload(catColumnsSplit);
+    const auto upload = [](const void* data, size_t bytes, TDeviceVec<uint32_t>* out) {
+        std::vector<uint32_t> raw(std::max<size_t>(bytes / 4, 1), 0);
+        if (bytes) {
+            std::memcpy(raw.data(), data, bytes);
+        }
+        out->Upload(raw);
+    };
+    upload(groups.data(), groups.size() * sizeof(dev::TCtrGroupDev), &result->Groups);
+    upload(items.data(), items.size() * sizeof(dev::TCtrItemDev), &result->Items);
+    upload(buckets.data(), buckets.size() * 4, &result->Buckets);
+    result->Table.Upload(table);
+    result->CatColumnsFlat.Upload(catColumnsFlat);
+    result->CatColumnsSplit.Upload(catColumnsSplit);
+    result->CatColumnCount = static_cast<uint32_t>(catColumnsFlat.size());
+    result->GroupCount = static_cast<uint32_t>(groups.size());
 }
 
 }  // namespace
@@ -1052,10 +1247,8 @@ struct THipEvaluator::TImpl {
     TDeviceVec<uint32_t> BucketGrid;  // 4 dwords per bucket: lowest border, cells per unit, search steps, 0
     TDeviceVec<uint32_t> BucketLut;   // kLutCells bytes per bucket
     TDeviceVec<unsigned long long> ExpMantissa;  // the table of the prediction types' exponent
-    // CTR tables: feature descriptors, projection items, the index buckets and the rows of all tables
-    TDeviceVec<uint32_t> CtrFeatures, CtrItems, CtrIndexBuckets, CtrBlob, CtrCatColumnsFlat, CtrCatColumnsSplit;
-    uint32_t CtrCatColumnCount = 0;
-    bool CtrTileUsable = false;  // the projections' categorical columns fit the LDS tile of CtrBinarizeTileKernel
+    TCtrDeviceTables Ctr;
+    bool CtrTileUsable = false;  // the projections' categorical columns fit the LDS tile of CtrBinarizeKernel
     // tree tables
     TDeviceVec<uint32_t> Splits, TreeStart, TreeSize, FirstLeaf, StepNodes, NodeToLeaf;
     TDeviceVec<double> Leaves, Bias;
@@ -1273,14 +1466,14 @@ struct THipEvaluator::TImpl {
     }
     dev::TCtrTablesDev CtrTables() const {
         dev::TCtrTablesDev t;
-        t.Features = reinterpret_cast<const dev::TCtrFeatureDev*>(CtrFeatures.Get());
-        t.Items = reinterpret_cast<const dev::TCtrItemDev*>(CtrItems.Get());
-        t.IndexBuckets = CtrIndexBuckets.Get();
-        t.Blob = CtrBlob.Get();
-        t.CatColumnsFlat = CtrCatColumnsFlat.Get();
-        t.CatColumnsSplit = CtrCatColumnsSplit.Get();
-        t.CatColumnCount = CtrCatColumnCount;
-        t.FeatureCount = CtrCount;
+        t.Groups = reinterpret_cast<const dev::TCtrGroupDev*>(Ctr.Groups.Get());
+        t.Items = reinterpret_cast<const dev::TCtrItemDev*>(Ctr.Items.Get());
+        t.Table = reinterpret_cast<const uint4*>(Ctr.Table.Get());
+        t.Buckets = Ctr.Buckets.Get();
+        t.CatColumnsFlat = Ctr.CatColumnsFlat.Get();
+        t.CatColumnsSplit = Ctr.CatColumnsSplit.Get();
+        t.CatColumnCount = Ctr.CatColumnCount;
+        t.GroupCount = Ctr.GroupCount;
         return t;
     }
     dev::TTreeTables TreeTables() const {
@@ -1410,10 +1603,9 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     CBAMD_ENSURE(m.BinarizeBuckets == trees.CtrFirstBucket, "internal error: bucket count mismatch");
     if (!trees.CtrFeatures.empty()) {
         CBAMD_ENSURE(ctrTables != nullptr, "Model has CTR features but no tables of learned statistics");
-        BuildCtrTables(trees, positions, *ctrTables, &srcFlat, &srcSplit, &offsets, &flags, &values, &m.CtrFeatures, &m.CtrItems,
-                       &m.CtrIndexBuckets, &m.CtrBlob, &m.CtrCatColumnsFlat, &m.CtrCatColumnsSplit, &m.CtrCatColumnCount);
+        BuildCtrTables(trees, positions, *ctrTables, &srcFlat, &srcSplit, &offsets, &flags, &values, &m.Ctr);
         m.CtrCount = static_cast<uint32_t>(trees.CtrFeatures.size());
-        m.CtrTileUsable = m.CtrCatColumnCount <= dev::kCtrMaxTileColumns && switches.CtrTile;
+        m.CtrTileUsable = m.Ctr.CatColumnCount <= dev::kCtrMaxTileColumns && switches.CtrTile;
     }
     CBAMD_ENSURE(srcFlat.size() == BucketCount, "internal error: bucket count mismatch");
     for (size_t b = 0; b + 1 < offsets.size(); ++b) {
@@ -2424,17 +2616,18 @@ void THipEvaluator::QuantizeDevice(const TFeatureBatch& batch, size_t docCount, 
             cats.DocStride = 1;
             cats.ColumnStride = batch.Stride;
         }
-        CBAMD_ENSURE(m.CtrCount <= 65535, "too many CTR features for one launch");
-        const dev::TBinarizeTables tab = m.BinarizeTables(batch.Layout != TFeatureBatch::SplitRows);
+        // shares of the projections: a small batch has fewer blocks than the chip has room for workgroups
+        const uint32_t groups = m.Ctr.GroupCount;
+        const uint32_t wanted = static_cast<uint32_t>(std::max<size_t>(1, std::min<size_t>((groups + 3) / 4, 2048 / blocks)));
+        const uint32_t groupsPerShare = (groups + wanted - 1) / wanted;
+        const dim3 grid(static_cast<uint32_t>(blocks), (groups + groupsPerShare - 1) / groupsPerShare);
         if (m.CtrTileUsable) {
-            const dim3 grid(static_cast<uint32_t>(blocks), (m.CtrCount + dev::kCtrGroup - 1) / dev::kCtrGroup);
-            const size_t lds = static_cast<size_t>(std::max<uint32_t>(m.CtrCatColumnCount, 1)) * dev::kCtrTilePitch * 4;
-            hipLaunchKernelGGL(dev::CtrBinarizeTileKernel, grid, dim3(256), lds, s, cats, static_cast<uint32_t>(docCount),
-                               m.CtrTables(), tab, reinterpret_cast<uint32_t*>(bins));
+            const size_t lds = static_cast<size_t>(std::max<uint32_t>(m.Ctr.CatColumnCount, 1)) * dev::kCtrTilePitch * 4;
+            hipLaunchKernelGGL(dev::CtrBinarizeKernel<true>, grid, dim3(256), lds, s, cats, static_cast<uint32_t>(docCount),
+                               m.CtrTables(), m.LayoutBuckets, groupsPerShare, reinterpret_cast<uint32_t*>(bins));
         } else {
-            const dim3 grid(static_cast<uint32_t>(blocks), m.CtrCount);
-            hipLaunchKernelGGL(dev::CtrBinarizeKernel, grid, dim3(64), 0, s, cats, static_cast<uint32_t>(docCount),
-                               m.CtrTables(), tab, reinterpret_cast<uint32_t*>(bins));
+            hipLaunchKernelGGL(dev::CtrBinarizeKernel<false>, grid, dim3(256), 0, s, cats, static_cast<uint32_t>(docCount),
+                               m.CtrTables(), m.LayoutBuckets, groupsPerShare, reinterpret_cast<uint32_t*>(bins));
         }
         HIP_CHECK(hipGetLastError());
     }
@@ -3016,7 +3209,7 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
                                ? "BinarizeColumnsKernel"
                                : "BinarizeRowsKernel<" + std::to_string(BinarizeLog2Slots(m.MaxBucketValues)) + ">";
     if (m.CtrCount > 0) {
-        binarize += m.CtrTileUsable ? "+CtrBinarizeTileKernel" : "+CtrBinarizeKernel";
+        binarize += m.CtrTileUsable ? "+CtrBinarizeKernel<true>" : "+CtrBinarizeKernel<false>";
     }
     const int dchunk = TileChunk(m.Dim);
     std::string evaluate;

@@ -396,20 +396,19 @@ __global__ __launch_bounds__(256) void BinarizeColumnsKernel(const float* __rest
 
 // ---- CTR (target statistics) features -------------------------------------------------------
 // What TStaticCtrProvider::CalcCtrs (catboost/libs/model/static_ctr_provider.cpp:14-131) and the
-// binarization of its results (cpu/quantization.h:304-325) do per block, done per document here.
-
-struct TCtrFeatureDev {
+// binarization of its results (cpu/quantization.h:304-325) do per block, done per document here. A CTR's value
+// depends on the document only through the row of the learned statistics that the hash of its projection finds, so
+// the host computes the bins of every row once, when the tables are uploaded (BuildCtrTables in hip_evaluator.hip):
+// all CTR features of one projection share one hash table whose entries hold the hash and, a byte each, the bins of
+// the projection's buckets. An empty entry holds the bins of a hash that no table knows.
+struct TCtrGroupDev {             // the CTR features of one projection
     uint32_t ItemBegin, ItemEnd;  // the projection: entries of TCtrTablesDev::Items
-    uint32_t HashBuckets;         // first 12-byte bucket of the CTR's table in IndexBuckets
-    uint32_t HashMask;            // buckets of the table - 1
-    uint32_t BlobOffset;          // first dword of the table's rows in Blob
-    uint32_t Type;                // ECtrType
-    int32_t TargetBorderIdx;
-    int32_t TargetClassesCount;
-    int32_t CounterDenominator;
-    float PriorNum, PriorDenom, Shift, Scale;
-    uint32_t FirstBucket, BucketCount;  // where the binarized CTR goes
-    uint32_t SameProjectionAsPrevious;  // the feature before this one hashes the same items
+    uint32_t FirstPiece;          // the group's table in TCtrTablesDev::Table, in pieces of 16 bytes
+    uint32_t HashMask;            // entries of the table - 1
+    uint32_t EntryPieces;         // pieces of an entry: hash low, hash high, then the bins
+    uint32_t FirstBucket;         // of the group's list in TCtrTablesDev::Buckets
+    uint32_t BucketCount;
+    uint32_t Unused;
 };
 
 constexpr uint32_t kCtrItemCat = 0;       // hashed categorical value of column SrcFlat / SrcSplit
@@ -421,15 +420,15 @@ struct TCtrItemDev {
 };
 
 struct TCtrTablesDev {
-    const TCtrFeatureDev* Features;
+    const TCtrGroupDev* Groups;
     const TCtrItemDev* Items;
-    const uint32_t* IndexBuckets;  // {hash low, hash high, row} per bucket (helpers/dense_hash_view.h:12-26)
-    const uint32_t* Blob;
+    const uint4* Table;
+    const uint32_t* Buckets;  // per byte of an entry's bins the bucket it goes to
     // the categorical columns the projections read, as flat and as categorical feature indexes
     const uint32_t* CatColumnsFlat;
     const uint32_t* CatColumnsSplit;
     uint32_t CatColumnCount;
-    uint32_t FeatureCount;
+    uint32_t GroupCount;
 };
 
 // hashed categorical values of a batch: Base[doc * DocStride + column * ColumnStride]
@@ -439,268 +438,138 @@ struct TCatSource {
     uint32_t SplitColumns;  // columns are categorical feature indexes (not flat feature indexes)
 };
 
-__device__ __forceinline__ uint64_t CtrCalcHash(uint64_t a, uint64_t b) {  // catboost/libs/model/hash.h:11-14
-    constexpr uint64_t kMagicMult = 0x4906ba494954cb65ull;
-    return kMagicMult * (a + kMagicMult * b);
+// CalcHash(a, b) = magic * (a + magic * b), catboost/libs/model/hash.h:11-14, as magic * a + magic^2 * b
+constexpr uint64_t kCtrMagic = 0x4906ba494954cb65ull;
+constexpr uint64_t kCtrMagicSquared = kCtrMagic * kCtrMagic;
+
+// b: a hashed categorical value, sign-extended
+__device__ __forceinline__ uint64_t CtrHashOfCat(uint32_t v) {
+    constexpr uint32_t kLow = static_cast<uint32_t>(kCtrMagicSquared), kHigh = static_cast<uint32_t>(kCtrMagicSquared >> 32);
+    const uint64_t product = static_cast<uint64_t>(v) * kLow;
+    const uint32_t high = static_cast<uint32_t>(product >> 32) + v * kHigh - (static_cast<int32_t>(v) < 0 ? kLow : 0u);
+    return (static_cast<uint64_t>(high) << 32) | static_cast<uint32_t>(product);
 }
 
-// TModelCtr::Calc, online_ctr.h:290-293: two roundings each for the quotient and the affine map
-__device__ __forceinline__ float CtrCalc(const TCtrFeatureDev& f, float countInClass, float totalCount) {
-    const float ctr = __fdiv_rn(__fadd_rn(countInClass, f.PriorNum), __fadd_rn(totalCount, f.PriorDenom));
-    return __fmul_rn(__fadd_rn(ctr, f.Shift), f.Scale);
-}
-
-constexpr uint32_t kCtrNotFound = 0xffffffffu;
-
-// TDenseIndexHashView::GetIndex, helpers/dense_hash_view.h:46-56; the probe sequence ends at the first
-// empty bucket, and after one pass over the table at the latest
-__device__ __forceinline__ uint32_t CtrTableRow(const TCtrTablesDev& ctr, const TCtrFeatureDev& f, uint64_t hash) {
-    const uint32_t lo = static_cast<uint32_t>(hash), hi = static_cast<uint32_t>(hash >> 32);
-    uint32_t zz = lo & f.HashMask;
-    for (uint32_t probes = 0; probes <= f.HashMask; ++probes) {
-        const uint32_t* bucket = ctr.IndexBuckets + 3 * (static_cast<size_t>(f.HashBuckets) + zz);
-        const uint32_t blo = bucket[0], bhi = bucket[1];
-        if ((blo & bhi) == 0xffffffffu) {
-            return kCtrNotFound;
-        }
-        if (blo == lo && bhi == hi) {
-            return bucket[2];
-        }
-        zz = (zz + 1) & f.HashMask;
-    }
-    return kCtrNotFound;
-}
-
-// static_ctr_provider.cpp:52-126, one branch per CTR type
-__device__ __forceinline__ float CtrValue(const TCtrTablesDev& ctr, const TCtrFeatureDev& f, uint32_t row) {
-    const uint32_t* blob = ctr.Blob + f.BlobOffset;
-    if (f.Type == 2 || f.Type == 3) {  // mean of the target: {float Sum; int Count}
-        if (row == kCtrNotFound) {
-            return CtrCalc(f, 0.f, 0.f);
-        }
-        return CtrCalc(f, __uint_as_float(blob[2 * static_cast<size_t>(row)]),
-                       static_cast<float>(static_cast<int32_t>(blob[2 * static_cast<size_t>(row) + 1])));
-    }
-    if (f.Type == 4 || f.Type == 5) {  // Counter, FeatureFreq
-        const float denominator = static_cast<float>(f.CounterDenominator);
-        if (row == kCtrNotFound) {
-            return CtrCalc(f, 0.f, denominator);
-        }
-        return CtrCalc(f, static_cast<float>(static_cast<int32_t>(blob[row])), denominator);
-    }
-    const int32_t classes = f.TargetClassesCount;
-    if (f.Type == 1) {  // Buckets
-        if (row == kCtrNotFound) {
-            return CtrCalc(f, 0.f, 0.f);
-        }
-        const uint32_t* history = blob + static_cast<size_t>(row) * classes;
-        int32_t total = 0;
-        for (int32_t c = 0; c < classes; ++c) {
-            total += static_cast<int32_t>(history[c]);
-        }
-        return CtrCalc(f, static_cast<float>(static_cast<int32_t>(history[f.TargetBorderIdx])), static_cast<float>(total));
-    }
-    // Borders
-    if (classes > 2) {
-        int32_t good = 0, total = 0;
-        if (row != kCtrNotFound) {
-            const uint32_t* history = blob + static_cast<size_t>(row) * classes;
-            for (int32_t c = 0; c < f.TargetBorderIdx + 1; ++c) {
-                total += static_cast<int32_t>(history[c]);
-            }
-            for (int32_t c = f.TargetBorderIdx + 1; c < classes; ++c) {
-                good += static_cast<int32_t>(history[c]);
-            }
-            total += good;
-        }
-        return CtrCalc(f, static_cast<float>(good), static_cast<float>(total));
-    }
-    if (row == kCtrNotFound) {
-        return CtrCalc(f, 0.f, 0.f);
-    }
-    const int32_t n0 = static_cast<int32_t>(blob[2 * static_cast<size_t>(row)]);
-    const int32_t n1 = static_cast<int32_t>(blob[2 * static_cast<size_t>(row) + 1]);
-    return CtrCalc(f, static_cast<float>(n1), static_cast<float>(n0 + n1));
-}
-
-// Tables whose row is one or two dwords (all but the class histograms of more than two classes): the dwords of
-// a row, read once for all the features of the table, and the value of a feature from them (as CtrValue).
-__device__ __forceinline__ bool CtrRowIsShort(const TCtrFeatureDev& f) {
-    return (f.Type >= 2 && f.Type <= 5) || (f.Type != 1 && f.TargetClassesCount <= 2);
-}
-
-__device__ __forceinline__ uint2 CtrShortRow(const TCtrTablesDev& ctr, const TCtrFeatureDev& f, uint32_t row) {
-    const uint32_t* blob = ctr.Blob + f.BlobOffset;
-    if (row == kCtrNotFound) {
-        return make_uint2(0u, 0u);
-    }
-    if (f.Type == 4 || f.Type == 5) {
-        return make_uint2(blob[row], 0u);
-    }
-    return make_uint2(blob[2 * static_cast<size_t>(row)], blob[2 * static_cast<size_t>(row) + 1]);
-}
-
-__device__ __forceinline__ float CtrValueOfShortRow(const TCtrFeatureDev& f, uint32_t row, uint2 dwords) {
-    if (f.Type == 2 || f.Type == 3) {
-        if (row == kCtrNotFound) {
-            return CtrCalc(f, 0.f, 0.f);
-        }
-        return CtrCalc(f, __uint_as_float(dwords.x), static_cast<float>(static_cast<int32_t>(dwords.y)));
-    }
-    if (f.Type == 4 || f.Type == 5) {
-        const float denominator = static_cast<float>(f.CounterDenominator);
-        if (row == kCtrNotFound) {
-            return CtrCalc(f, 0.f, denominator);
-        }
-        return CtrCalc(f, static_cast<float>(static_cast<int32_t>(dwords.x)), denominator);
-    }
-    if (row == kCtrNotFound) {
-        return CtrCalc(f, 0.f, 0.f);
-    }
-    const int32_t n0 = static_cast<int32_t>(dwords.x), n1 = static_cast<int32_t>(dwords.y);
-    return CtrCalc(f, static_cast<float>(n1), static_cast<float>(n0 + n1));
-}
-
-// grid = (document blocks, CTR features), one wave per workgroup: lane l computes the CTR of documents
-// l, l + 64, l + 128, l + 192 of the block from the block's float / one-hot bins (already written)
-// and the hashed categorical values, and writes the bins of the CTR's buckets.
-__global__ __launch_bounds__(64) void CtrBinarizeKernel(TCatSource cats, uint32_t docCount, TCtrTablesDev ctr,
-                                                        TBinarizeTables tab, uint32_t* __restrict__ bins) {
-    const uint32_t block = blockIdx.x, lane = threadIdx.x;
-    const TCtrFeatureDev f = ctr.Features[blockIdx.y];
-    uint64_t hash[4] = {0, 0, 0, 0};
-    for (uint32_t i = f.ItemBegin; i < f.ItemEnd; ++i) {
-        const TCtrItemDev item = ctr.Items[i];
-        if (item.Kind == kCtrItemCat) {
-            const size_t column = cats.SplitColumns ? item.SrcSplit : item.SrcFlat;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const size_t doc = min(block * kDocsPerBlock + j * kWave + lane, docCount - 1);
-                const int32_t v = static_cast<int32_t>(cats.Base[doc * cats.DocStride + column * cats.ColumnStride]);
-                hash[j] = CtrCalcHash(hash[j], static_cast<uint64_t>(static_cast<int64_t>(v)));
-            }
-        } else {
-            const uint32_t word = bins[(static_cast<size_t>(block) * tab.BucketPitch + item.SrcFlat) * kWave + lane];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t bin = (word >> (8 * j)) & 0xffu;
-                const bool holds = item.Kind == kCtrItemBinGe ? bin >= item.Value : bin == item.Value;
-                hash[j] = CtrCalcHash(hash[j], holds ? 1u : 0u);
-            }
-        }
-    }
-    float value[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        value[j] = CtrValue(ctr, f, CtrTableRow(ctr, f, hash[j]));
-    }
-    for (uint32_t k = 0; k < f.BucketCount; ++k) {
-        const uint32_t bucket = f.FirstBucket + k;
-        const uint32_t begin = tab.BucketOffset[bucket], end = tab.BucketOffset[bucket + 1];
-        uint32_t count[4] = {0, 0, 0, 0};
-        for (uint32_t b = begin; b < end; ++b) {
-            const float border = __uint_as_float(tab.Values[b]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                count[j] += value[j] > border ? 1u : 0u;
-            }
-        }
-        bins[(static_cast<size_t>(block) * tab.BucketPitch + bucket) * kWave + lane] =
-            count[0] | (count[1] << 8) | (count[2] << 16) | (count[3] << 24);
-    }
-}
-
-// The same for models whose CTR projections read at most kCtrMaxTileColumns categorical columns:
-// grid = (document blocks, groups of kCtrGroup CTR features), 4 waves per workgroup. The block's hashed
-// categorical values are staged once per workgroup into LDS ([column][document], read without bank
-// conflicts), each wave then works through kCtrGroup / 4 consecutive CTR features and keeps the hash
-// when the next feature has the same projection (features are sorted by projection).
-constexpr uint32_t kCtrGroup = 16;
+// The bins of a lane's four documents ({lane, lane + 64, lane + 128, lane + 192} of the block) in the buckets of CTR
+// features. What bounds it is the gathers of table entries (a line of L2 each for tables beyond the L1): one 16-byte
+// read finds and answers a lookup of up to eight buckets, where a table per CTR feature, its rows and a division and a
+// count of borders per feature used to take some ten times as long (1M documents, 16 categorical columns, 24 projections
+// with 96 CTR features: 620 us before).
+// grid = (document blocks, shares of the groups), 4 waves per workgroup, each wave a run of the share's groups.
+// TILE: the block's hashed categorical values are staged once per workgroup into LDS ([column][document]); without
+// it (more than kCtrMaxTileColumns columns) they are read from the batch where a projection needs them.
 constexpr uint32_t kCtrMaxTileColumns = 60;
-constexpr uint32_t kCtrTilePitch = kDocsPerBlock + 1;
+constexpr uint32_t kCtrTilePitch = kDocsPerBlock + 4;  // 16 columns * 4 documents, stored at once, fall on 64 banks
 
-__global__ __launch_bounds__(256) void CtrBinarizeTileKernel(TCatSource cats, uint32_t docCount, TCtrTablesDev ctr,
-                                                             TBinarizeTables tab, uint32_t* __restrict__ bins) {
+template <bool TILE>
+__global__ __launch_bounds__(256) void CtrBinarizeKernel(TCatSource cats, uint32_t docCount, TCtrTablesDev ctr,
+                                                         uint32_t bucketPitch, uint32_t groupsPerShare,
+                                                         uint32_t* __restrict__ bins) {
     extern __shared__ uint32_t sCats[];  // [CatColumnCount][kCtrTilePitch]
     const uint32_t block = blockIdx.x, tid = threadIdx.x;
-    const uint32_t lane = tid & (kWave - 1), wave = tid / kWave;
-    const uint32_t columns = ctr.CatColumnCount;
-    const uint32_t* columnList = cats.SplitColumns ? ctr.CatColumnsSplit : ctr.CatColumnsFlat;
-    const size_t firstDoc = static_cast<size_t>(block) * kDocsPerBlock;
-    for (uint32_t i = tid; i < columns * kDocsPerBlock; i += 256) {
-        // neighbouring threads read neighbouring addresses: columns of one row, or documents of one column
-        const uint32_t c = cats.ColumnStride == 1 ? i % columns : i / kDocsPerBlock;
-        const uint32_t d = cats.ColumnStride == 1 ? i / columns : i % kDocsPerBlock;
-        const size_t doc = min(firstDoc + d, static_cast<size_t>(docCount) - 1);
-        sCats[c * kCtrTilePitch + d] = cats.Base[doc * cats.DocStride + static_cast<size_t>(columnList[c]) * cats.ColumnStride];
-    }
-    __syncthreads();
-    constexpr uint32_t kPerWave = kCtrGroup / 4;
-    const uint32_t first = blockIdx.y * kCtrGroup + wave * kPerWave;
-    uint64_t hash[4] = {0, 0, 0, 0};
-    uint32_t row[4] = {kCtrNotFound, kCtrNotFound, kCtrNotFound, kCtrNotFound};
-    uint2 rowDwords[4] = {};
-    uint32_t tableOfRows = 0;  // HashBuckets of the table that row[] was looked up in
-    for (uint32_t k = 0; k < kPerWave && first + k < ctr.FeatureCount; ++k) {
-        const TCtrFeatureDev f = ctr.Features[first + k];
-        if (k == 0 || !f.SameProjectionAsPrevious) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                hash[j] = 0;
-            }
-            for (uint32_t i = f.ItemBegin; i < f.ItemEnd; ++i) {
-                const TCtrItemDev item = ctr.Items[i];
-                if (item.Kind == kCtrItemCat) {
-                    const uint32_t* column = sCats + item.Value * kCtrTilePitch + lane;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int32_t v = static_cast<int32_t>(column[j * kWave]);
-                        hash[j] = CtrCalcHash(hash[j], static_cast<uint64_t>(static_cast<int64_t>(v)));
-                    }
-                } else {
-                    const uint32_t word = bins[(static_cast<size_t>(block) * tab.BucketPitch + item.SrcFlat) * kWave + lane];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const uint32_t bin = (word >> (8 * j)) & 0xffu;
-                        const bool holds = item.Kind == kCtrItemBinGe ? bin >= item.Value : bin == item.Value;
-                        hash[j] = CtrCalcHash(hash[j], holds ? 1u : 0u);
-                    }
+    const uint32_t lane = tid & (kWave - 1);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const uint32_t firstDoc = block * kDocsPerBlock;
+    // documents past the last one are read as the last one (their bins are never used)
+    if (TILE) {
+        const uint32_t columns = ctr.CatColumnCount;
+        const uint32_t* columnList = cats.SplitColumns ? ctr.CatColumnsSplit : ctr.CatColumnsFlat;
+        if (cats.ColumnStride == 1) {  // sixteen columns of a row side by side
+            for (uint32_t c = tid % 16; c < columns; c += 16) {
+                const uint32_t* column = cats.Base + columnList[c];
+#pragma unroll 4
+                for (uint32_t d = tid / 16; d < kDocsPerBlock; d += 16) {
+                    sCats[c * kCtrTilePitch + d] = column[static_cast<size_t>(min(firstDoc + d, docCount - 1)) * cats.DocStride];
                 }
             }
-        }
-        // features that differ only in prior, target border, shift or scale read the same row of the same table
-        const bool shortRow = CtrRowIsShort(f);
-        if (k == 0 || !f.SameProjectionAsPrevious || f.HashBuckets != tableOfRows) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                row[j] = CtrTableRow(ctr, f, hash[j]);
+        } else {
+            const size_t doc = min(firstDoc + tid, docCount - 1);
+            for (uint32_t c = 0; c < columns; ++c) {
+                sCats[c * kCtrTilePitch + tid] = cats.Base[doc * cats.DocStride + columnList[c] * cats.ColumnStride];
             }
-            if (shortRow) {
+        }
+        __syncthreads();
+    }
+    const uint32_t* blockBins = bins + static_cast<size_t>(block) * bucketPitch * kWave + lane;
+    const uint32_t shareBegin = blockIdx.y * groupsPerShare;
+    const uint32_t shareEnd = min(shareBegin + groupsPerShare, ctr.GroupCount);
+    const uint32_t groupsPerWave = (shareEnd - shareBegin + 3) / 4;
+    const uint32_t end = min(shareBegin + (wave + 1) * groupsPerWave, shareEnd);
+    for (uint32_t g = shareBegin + wave * groupsPerWave; g < end; ++g) {
+        const TCtrGroupDev group = ctr.Groups[g];
+        uint64_t hash[4] = {0, 0, 0, 0};
+        for (uint32_t i = group.ItemBegin; i < group.ItemEnd; ++i) {
+            const TCtrItemDev item = ctr.Items[i];
+            if (item.Kind == kCtrItemCat) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    rowDwords[j] = CtrShortRow(ctr, f, row[j]);
+                    uint32_t v;
+                    if (TILE) {
+                        v = sCats[item.Value * kCtrTilePitch + j * kWave + lane];
+                    } else {
+                        const size_t column = cats.SplitColumns ? item.SrcSplit : item.SrcFlat;
+                        const size_t doc = min(firstDoc + j * kWave + lane, docCount - 1);
+                        v = cats.Base[doc * cats.DocStride + column * cats.ColumnStride];
+                    }
+                    const uint64_t h = CtrHashOfCat(v);
+                    hash[j] = i == group.ItemBegin ? h : kCtrMagic * hash[j] + h;
+                }
+            } else {
+                const uint32_t word = blockBins[item.SrcFlat * kWave];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t bin = (word >> (8 * j)) & 0xffu;
+                    const bool holds = item.Kind == kCtrItemBinGe ? bin >= item.Value : bin == item.Value;
+                    hash[j] = kCtrMagic * hash[j] + (holds ? kCtrMagicSquared : 0u);
                 }
             }
-            tableOfRows = f.HashBuckets;
         }
-        float value[4];
+        // the four documents' first probes are in flight together; at most half of a table's entries are taken, so
+        // that every probe sequence ends at its hash or at an empty entry (all ones) soon
+        const uint4* table = ctr.Table + group.FirstPiece;
+        uint32_t at[4];
+        uint4 entry[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            value[j] = shortRow ? CtrValueOfShortRow(f, row[j], rowDwords[j]) : CtrValue(ctr, f, row[j]);
+            at[j] = static_cast<uint32_t>(hash[j]) & group.HashMask;
+            entry[j] = table[static_cast<size_t>(at[j]) * group.EntryPieces];
         }
-        for (uint32_t b = 0; b < f.BucketCount; ++b) {
-            const uint32_t bucket = f.FirstBucket + b;
-            const uint32_t begin = tab.BucketOffset[bucket], end = tab.BucketOffset[bucket + 1];
-            uint32_t count[4] = {0, 0, 0, 0};
-            for (uint32_t x = begin; x < end; ++x) {
-                const float border = __uint_as_float(tab.Values[x]);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    count[j] += value[j] > border ? 1u : 0u;
+        for (int j = 0; j < 4; ++j) {
+            while ((entry[j].x != static_cast<uint32_t>(hash[j]) || entry[j].y != static_cast<uint32_t>(hash[j] >> 32)) &&
+                   (entry[j].x & entry[j].y) != 0xffffffffu) {
+                at[j] = (at[j] + 1) & group.HashMask;
+                entry[j] = table[static_cast<size_t>(at[j]) * group.EntryPieces];
+            }
+        }
+        // bytes of four documents and four buckets -> a dword of four documents per bucket
+        const uint32_t* buckets = ctr.Buckets + group.FirstBucket;
+        const auto store = [&](uint32_t first, uint32_t d0, uint32_t d1, uint32_t d2, uint32_t d3) {
+            const uint32_t low01 = __builtin_amdgcn_perm(d1, d0, 0x05010400u), high01 = __builtin_amdgcn_perm(d1, d0, 0x07030602u);
+            const uint32_t low23 = __builtin_amdgcn_perm(d3, d2, 0x05010400u), high23 = __builtin_amdgcn_perm(d3, d2, 0x07030602u);
+            const uint32_t out[4] = {__builtin_amdgcn_perm(low23, low01, 0x05040100u), __builtin_amdgcn_perm(low23, low01, 0x07060302u),
+                                     __builtin_amdgcn_perm(high23, high01, 0x05040100u), __builtin_amdgcn_perm(high23, high01, 0x07060302u)};
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                if (first + k < group.BucketCount) {
+                    bins[(static_cast<size_t>(block) * bucketPitch + buckets[first + k]) * kWave + lane] = out[k];
                 }
             }
-            bins[(static_cast<size_t>(block) * tab.BucketPitch + bucket) * kWave + lane] =
-                count[0] | (count[1] << 8) | (count[2] << 16) | (count[3] << 24);
+        };
+        store(0, entry[0].z, entry[1].z, entry[2].z, entry[3].z);
+        if (group.BucketCount > 4) {
+            store(4, entry[0].w, entry[1].w, entry[2].w, entry[3].w);
+        }
+        for (uint32_t piece = 1; piece < group.EntryPieces; ++piece) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                entry[j] = table[static_cast<size_t>(at[j]) * group.EntryPieces + piece];
+            }
+            const uint32_t first = piece * 16 - 8;
+            store(first, entry[0].x, entry[1].x, entry[2].x, entry[3].x);
+            store(first + 4, entry[0].y, entry[1].y, entry[2].y, entry[3].y);
+            store(first + 8, entry[0].z, entry[1].z, entry[2].z, entry[3].z);
+            store(first + 12, entry[0].w, entry[1].w, entry[2].w, entry[3].w);
         }
     }
 }

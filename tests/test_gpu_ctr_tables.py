@@ -1,0 +1,38 @@
+"""CTR features of one projection share a hash table of bins: entries of one and of several 16-byte pieces, features of
+more than 254 borders (several buckets), tables of one projection that know different hashes, batches whose workgroups
+share the projections out. Needs an MI355X."""
+import numpy as np
+import pytest
+
+import catboost_amd as cb
+from oracle.oracle import OracleModel
+from oracle.cbm_reader import read_cbm
+
+from tests import ctr_models
+from tests.cbm_writer import write_cbm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tile", ["1", "0"])
+@pytest.mark.parametrize("copies,wide", [(1, False), (4, False), (13, False), (5, True)])
+def test_projections_of_many_buckets(monkeypatch, tile, copies, wide):
+    monkeypatch.setenv("CATBOOST_AMD_CTR_TILE", tile)
+    model, known = ctr_models.random_ctr_model(21, n_cat=6, n_bases=15, n_trees=30)
+    rng = np.random.default_rng(copies)
+    features = []
+    for c in model["ctr_features"]:
+        for k in range(copies):
+            lo, hi = float(c["shift"] * c["scale"]), float((1 + c["shift"]) * c["scale"])
+            count = 300 if wide and k == 2 else int(rng.integers(1, 20))
+            features.append(dict(c, prior_num=np.float32(k / 8.0),
+                                 borders=np.unique(rng.uniform(lo, hi, size=count).astype(np.float32))))
+    model["ctr_features"], model["ctr_feature_count"] = features, len(features)
+    total = (sum(f["borders"].size for f in model["float_features"]) +
+             sum(o["values"].size for o in model["one_hot_features"]) + sum(c["borders"].size for c in features))
+    model["tree_splits"] = rng.integers(0, total, size=len(model["tree_splits"])).astype(np.int32)
+    data = write_cbm(model)
+    o, g = OracleModel(read_cbm(data)), cb.ModelCalcer(buffer=data)
+    for docs in (1, 257, 5000):
+        floats, cats = ctr_models.random_documents(model, known, docs, 3 + docs)
+        np.testing.assert_array_equal(g.quantize_hashed(floats, cats), o.binarize(floats, cats, layout="split"))
