@@ -72,6 +72,10 @@ public:
     // index of the fused kernel tables that such a call would use (0 flat rows, 1 split rows), -1 when it takes
     // the two launches: the one test that EvalRowsFusedDevice, the host pipeline and DescribeKernels share
     int FusedLayoutFor(int layout, size_t stride, size_t docCount, size_t treeStart, size_t treeEnd, bool anyBatchSize) const;
+    // Batches of oblivious models that are too small to fill the chip: one launch from the features to the results,
+    // the trees in the slices of TreeSlicesFor. `source` and `results` may be device or pinned host memory. True when
+    // such a call takes it.
+    bool TakesSmallBatchKernel(size_t docCount, size_t treeStart, size_t treeEnd) const;
     // Small batches (fewer than 256 workgroups of the register kernels) are cut into slices of the trees by the
     // calls that own their scratch memory; off: every sum is one pass in tree order, the CPU evaluator's
     // order of additions, at the price of the small-batch speed-up. Set it before the calls it should govern.
@@ -119,12 +123,17 @@ public:
     struct TImpl;
 
 private:
+    // what every launch that reads features asks of its batch
+    void CheckBatch(const TFeatureBatch& batch, size_t docCount) const;
     void SetLastTimes(const TKernelTimes& times);
+    // ... of a small-batch launch: its context, whose clock stamps are read when the times are asked for
+    void SetLastTimes(const void* smallContext);
     std::unique_ptr<TImpl> Impl;
     size_t TreeCount = 0;
     int ApproxDimension = 1;
     uint32_t BucketCount = 0;
     TKernelTimes LastTimes;
+    const void* LastSmallContext = nullptr;  // a THostContext of Impl
     mutable std::mutex TimesLock;  // callers of one evaluator run side by side; the last one to finish leaves its times
 };
 

@@ -3,12 +3,15 @@
 #include "fast_exp.h"
 #include "kernels.hip.h"
 
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <cmath>
 #include <condition_variable>
 #include <cstdlib>
 #include <cstring>
 #include <limits>
+#include <map>
 #include <numeric>
 #include <string>
 #include <thread>
@@ -447,6 +450,15 @@ TBucketGrid MakeBucketGrid(const std::vector<float>& borders) {
 }
 
 constexpr size_t kMaxTileLdsBytes = 160 * 1024;
+
+// Batches of SmallBatchKernel and FewDocumentsKernel, in documents times passes over the dimensions; beyond, the binarize
+// and register kernels in slices of the trees are faster. Whole call, 1000 trees of depth 8 over 200 features: 8192
+// documents 31 us against 46 on those, 16384 48 against 49, 32768 82 against 62 (200 trees of depth 6: 26 against 33 and
+// 39 against 37). FewDocumentsKernel against SmallBatchKernel: 512 documents 18 against 21 us, 1024 24 against 21.
+constexpr size_t kSmallBatchDocs = 16384;
+constexpr size_t kFewDocs = 640;
+// host calls read features of at most so many bytes from pinned memory
+constexpr size_t kSmallHostBytes = size_t(16) << 20;
 
 // Workgroups wanted of a leaf index launch: 200 000 documents * 1000 trees (782 blocks, 2 workgroups per CU) take 180 us as
 // 782 workgroups, 165 as 2346, 199 as 4692 (shorter runs of a row, the bins read more often).
@@ -1350,6 +1362,28 @@ struct THipEvaluator::TImpl {
     const char* RegKernelName = "";
     const char* FusedKernelName = "";
 
+    // small-batch kernel: tree rows of sixteen dwords, and from these dwords on the cells of its tile and the first leaves
+    bool SmallUsable = false;
+    uint32_t SmallCellCount = 0;
+    TDeviceVec<uint32_t> SmallTable;
+    size_t SmallCellsAt = 0, SmallFirstLeafAt = 0;
+    // (no slices on a model too short for them: its one slice is the whole model)
+    uint32_t SmallSliceTrees(size_t treeCount) const {
+        const uint32_t slice = RegKernelUsable ? RegSliceTrees(RegTreeBlockSize) : 32;
+        return treeCount < 2 * static_cast<size_t>(slice) ? static_cast<uint32_t>(treeCount) : slice;
+    }
+    int SmallDims() const { return Dim == 1 ? 1 : Dim == 2 ? 2 : 4; }
+    uint32_t SmallPasses() const { return static_cast<uint32_t>((Dim + SmallDims() - 1) / SmallDims()); }
+    size_t SmallLdsBytes(size_t treeCount) const {
+        const size_t sliceTrees = SmallSliceTrees(treeCount);
+        const size_t tile = static_cast<size_t>(dev::SmallDocPitch(SmallCellCount)) * dev::kSmallDocs * 4;
+        return tile + (treeCount + sliceTrees - 1) / sliceTrees * dev::kSmallDocs * SmallDims() * 8;
+    }
+    size_t FewLdsBytes(size_t treeCount) const {
+        const size_t sliceTrees = SmallSliceTrees(treeCount);
+        return (static_cast<size_t>(SmallCellCount) + 1) / 2 * 8 + (treeCount + sliceTrees - 1) / sliceTrees * (sliceTrees + 2) * SmallDims() * 8;
+    }
+
     // Staging of the calls that own their buffers (CalcDevice and the host entry points): a call borrows a
     // context - a stream, a bin buffer and two slots of pinned and device staging memory - from a small pool,
     // so that a few callers of one evaluator run side by side and later ones wait for a free context.
@@ -1373,6 +1407,8 @@ struct THipEvaluator::TImpl {
         TDeviceVec<double> SlicePartials;  // raw sums per slice of the trees (small batches)
         THostSlot Slots[2];
         hipEvent_t Ev[3] = {nullptr, nullptr, nullptr};
+        TDeviceVec<unsigned long long> Stamps;  // start and end of every workgroup of the last small-batch launch
+        size_t StampCount = 0;
         bool Busy = false;
 
         THostContext() {
@@ -1667,6 +1703,73 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     m.BucketOffset.Upload(offsets);
     m.BucketFlags.Upload(flags);
     m.Values.Upload(values);
+
+    // ---- small-batch kernel: every split as "cell of the tile above a border"
+    if (m.Oblivious && m.MaxDepth <= 8 && TreeCount > 0 && m.CtrCount == 0 && BucketCount > 0) {
+        std::vector<dev::TSmallCell> cells;
+        std::vector<uint32_t> cellOfBucket(BucketCount, UINT32_MAX);
+        std::map<std::pair<uint32_t, uint32_t>, uint32_t> cellOfValue;  // one-hot: (bucket, value's index) -> cell
+        // rows of null trees behind the model's, for a last slice that ends inside a turn: no level is above +inf or NaN
+        std::vector<uint32_t> rows((TreeCount + dev::kSmallNullTrees) * 16, 0);
+        std::vector<uint32_t> first(TreeCount + dev::kSmallNullTrees, static_cast<uint32_t>(trees.LeafValues.size()));
+        const uint32_t never = 0x7f800000u;
+        bool usable = trees.LeafValues.size() < (size_t(1) << 32);
+        for (size_t t = 0; t < TreeCount + dev::kSmallNullTrees && usable; ++t) {
+            const int depth = t < TreeCount ? trees.TreeSizes[t] : 0;
+            uint32_t* row = rows.data() + t * 16;
+            if (t < TreeCount) {
+                first[t] = static_cast<uint32_t>(trees.TreeFirstLeafOffsets[t]);
+            }
+            for (int d = 0; d < 8; ++d) {
+                row[8 + d] = never;
+                if (d >= depth) {
+                    continue;
+                }
+                const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + d];
+                const uint32_t b = rb.FeatureIndex, n = offsets[b + 1] - offsets[b];
+                // a damaged model may name a border that is not there: such a split stays with the kernels on bins
+                const bool oneHot = (flags[b] & dev::kBucketFlagOneHot) != 0;
+                const uint32_t at = oneHot ? static_cast<uint8_t>(~rb.XorMask) : rb.SplitIdx;
+                if (at == 0 || at > n || (oneHot ? rb.SplitIdx != 0xff : rb.XorMask != 0)) {
+                    usable = false;
+                    break;
+                }
+                uint32_t cell;
+                if (oneHot) {
+                    // "bin = at", and no other value of the bucket is the same one
+                    const uint32_t value = values[offsets[b] + at - 1];
+                    usable = usable &&
+                             std::count(values.begin() + offsets[b], values.begin() + offsets[b + 1], value) == 1;
+                    const auto found = cellOfValue.emplace(std::make_pair(b, at), static_cast<uint32_t>(cells.size()));
+                    if (found.second) {
+                        cells.push_back({srcFlat[b], srcSplit[b], 2u, value});
+                    }
+                    cell = found.first->second;
+                    row[8 + d] = 0x3f000000u;  // 0.5
+                } else {
+                    if (cellOfBucket[b] == UINT32_MAX) {
+                        cellOfBucket[b] = static_cast<uint32_t>(cells.size());
+                        cells.push_back({srcFlat[b], srcSplit[b], (flags[b] & dev::kBucketFlagNanToInf) ? 1u : 0u, 0u});
+                    }
+                    cell = cellOfBucket[b];
+                    row[8 + d] = values[offsets[b] + at - 1];
+                }
+                row[d] = cell * 4;
+            }
+        }
+        if (usable && !cells.empty()) {
+            // one allocation: the rows, the cells, the first leaves
+            std::vector<uint32_t> table(std::move(rows));
+            m.SmallCellsAt = table.size();
+            const uint32_t* cellDwords = reinterpret_cast<const uint32_t*>(cells.data());
+            table.insert(table.end(), cellDwords, cellDwords + cells.size() * (sizeof(dev::TSmallCell) / 4));
+            m.SmallFirstLeafAt = table.size();
+            table.insert(table.end(), first.begin(), first.end());
+            m.SmallTable.Upload(table);
+            m.SmallCellCount = static_cast<uint32_t>(cells.size());
+            m.SmallUsable = true;
+        }
+    }
 
     // ---- tree tables
     std::vector<uint32_t> splits(trees.RepackedBins.size());
@@ -2554,6 +2657,35 @@ void LaunchBinarizeColumns(uint32_t maxBucketValues, size_t blocks, const float*
 
 }  // namespace
 
+void THipEvaluator::CheckBatch(const TFeatureBatch& batch, size_t docCount) const {
+    const TImpl& m = *Impl;
+    CBAMD_ENSURE(batch.Floats != nullptr || (batch.Layout == TFeatureBatch::SplitRows && m.MinFloatSize == 0),
+                 "float features pointer is null");
+    switch (batch.Layout) {
+        case TFeatureBatch::FlatRows:
+            CBAMD_ENSURE(batch.Stride >= m.FlatVectorSize, "insufficient flat features vector size: " +
+                                                                std::to_string(batch.Stride) + " expected: " +
+                                                                std::to_string(m.FlatVectorSize));
+            break;
+        case TFeatureBatch::SplitRows:
+            CBAMD_ENSURE(batch.Stride >= m.MinFloatSize, "insufficient float features vector size: " +
+                                                             std::to_string(batch.Stride) + " expected: " +
+                                                             std::to_string(m.MinFloatSize));
+            if (m.HasCats) {
+                CBAMD_ENSURE(batch.Cats != nullptr, "Model has categorical features but no categorical features provided");
+                CBAMD_ENSURE(batch.CatStride >= m.MinCatSize, "insufficient cat features vector size: " +
+                                                                  std::to_string(batch.CatStride) + " expected: " +
+                                                                  std::to_string(m.MinCatSize));
+            }
+            break;
+        case TFeatureBatch::FlatColumns:
+            CBAMD_ENSURE(batch.Stride >= docCount, "column stride is shorter than the document count");
+            break;
+        default:
+            CBAMD_ENSURE(false, "unknown feature layout");
+    }
+}
+
 void THipEvaluator::QuantizeDevice(const TFeatureBatch& batch, size_t docCount, uint8_t* bins, void* stream) {
     TImpl& m = *Impl;
     if (docCount == 0) {
@@ -2572,42 +2704,23 @@ void THipEvaluator::QuantizeDevice(const TFeatureBatch& batch, size_t docCount, 
         return;
     }
     CBAMD_ENSURE(bins != nullptr, "quantized buffer is null");
-    CBAMD_ENSURE(batch.Floats != nullptr || (batch.Layout == TFeatureBatch::SplitRows && m.MinFloatSize == 0),
-                 "float features pointer is null");
+    CheckBatch(batch, docCount);
     switch (batch.Layout) {
-        case TFeatureBatch::FlatRows: {
-            CBAMD_ENSURE(batch.Stride >= m.FlatVectorSize, "insufficient flat features vector size: " +
-                                                                std::to_string(batch.Stride) + " expected: " +
-                                                                std::to_string(m.FlatVectorSize));
+        case TFeatureBatch::FlatRows:
             LaunchBinarizeRows(m.MaxBucketValues, blocks, batch.Floats, batch.Stride, nullptr, 0, docCount,
                                m.BinarizeTables(true), reinterpret_cast<uint32_t*>(bins), s);
             break;
-        }
-        case TFeatureBatch::SplitRows: {
-            CBAMD_ENSURE(batch.Stride >= m.MinFloatSize, "insufficient float features vector size: " +
-                                                             std::to_string(batch.Stride) + " expected: " +
-                                                             std::to_string(m.MinFloatSize));
-            if (m.HasCats) {
-                CBAMD_ENSURE(batch.Cats != nullptr, "Model has categorical features but no categorical features provided");
-                CBAMD_ENSURE(batch.CatStride >= m.MinCatSize, "insufficient cat features vector size: " +
-                                                                  std::to_string(batch.CatStride) + " expected: " +
-                                                                  std::to_string(m.MinCatSize));
-            }
+        case TFeatureBatch::SplitRows:
             // a model with one-hot buckets always reads them from the categorical matrix here
             LaunchBinarizeRows(m.MaxBucketValues, blocks, batch.Floats, batch.Stride, m.HasCats ? batch.Cats : nullptr,
                                batch.CatStride, docCount, m.BinarizeTables(false), reinterpret_cast<uint32_t*>(bins), s);
             break;
-        }
-        case TFeatureBatch::FlatColumns: {
-            CBAMD_ENSURE(batch.Stride >= docCount, "column stride is shorter than the document count");
+        case TFeatureBatch::FlatColumns:
             if (m.BinarizeBuckets > 0) {
                 LaunchBinarizeColumns(m.MaxBucketValues, blocks, batch.Floats, batch.Stride, docCount,
                                       m.BinarizeTables(true), reinterpret_cast<uint32_t*>(bins), s);
             }
             break;
-        }
-        default:
-            CBAMD_ENSURE(false, "unknown feature layout");
     }
     HIP_CHECK(hipGetLastError());
     if (m.CtrCount > 0) {
@@ -3158,6 +3271,71 @@ void THipEvaluator::EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCou
     HIP_CHECK(hipGetLastError());
 }
 
+// The largest batch of the small-batch kernel: see kSmallBatchDocs.
+bool THipEvaluator::TakesSmallBatchKernel(size_t docCount, size_t treeStart, size_t treeEnd) const {
+    const TImpl& m = *Impl;
+    return m.SmallUsable && m.SmallBatchSlices && docCount > 0 && docCount * m.SmallPasses() <= kSmallBatchDocs && treeStart == 0 &&
+           treeEnd == TreeCount && m.SmallLdsBytes(TreeCount) <= kMaxTileLdsBytes;
+}
+
+// One launch of the small-batch kernel whose end `stop` marks. `batch` and `results` may be device or pinned host memory.
+static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THostContext& ctx, const TFeatureBatch& batch,
+                             size_t docCount, size_t treeCount, double* results, hipStream_t s, hipEvent_t stop) {
+    CBAMD_ENSURE(results != nullptr, "results pointer is null");
+    dev::TSmallSource src = {};
+    src.Floats = reinterpret_cast<const uint32_t*>(batch.Floats);
+    const bool columns = batch.Layout == TFeatureBatch::FlatColumns;
+    src.DocStride = columns ? 1 : batch.Stride;
+    src.ColumnStride = columns ? batch.Stride : 1;
+    src.Cats = reinterpret_cast<const uint32_t*>(batch.Cats);
+    src.CatStride = batch.CatStride;
+    src.Split = batch.Layout == TFeatureBatch::SplitRows ? 1u : 0u;
+    dev::TSmallTables tab = {};
+    tab.Cells = reinterpret_cast<const dev::TSmallCell*>(m.SmallTable.Get() + m.SmallCellsAt);
+    tab.TreeRows = m.SmallTable.Get();
+    tab.FirstLeaf = m.SmallTable.Get() + m.SmallFirstLeafAt;
+    tab.Leaves = m.Leaves.Get();
+    tab.Bias = m.Bias.Get();
+    tab.Scale = m.Scale;
+    tab.CellCount = m.SmallCellCount;
+    tab.Dim = static_cast<uint32_t>(m.Dim);
+    tab.TreeCount = static_cast<uint32_t>(treeCount);
+    tab.SliceTrees = m.SmallSliceTrees(treeCount);
+    tab.SliceCount = (tab.TreeCount + tab.SliceTrees - 1) / tab.SliceTrees;
+    const uint32_t dims = static_cast<uint32_t>(m.SmallDims());
+    const uint32_t passes = m.SmallPasses();
+    const auto launch = [&](auto kernel, size_t groups, uint32_t threads, size_t lds) {
+        ctx.Stamps.Reserve(2 * groups * passes);
+        ctx.StampCount = groups * passes;
+        EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds);
+        hipExtLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups), passes), dim3(threads), lds, s, nullptr, stop, 0, src,
+                              static_cast<uint32_t>(docCount), tab, results, reinterpret_cast<ulonglong2*>(ctx.Stamps.Get()));
+    };
+    const auto launchFew = [&](auto kernel) {
+        launch(kernel, docCount, std::min<uint32_t>(dev::kFewThreads, (tab.TreeCount + 63) / 64 * 64), m.FewLdsBytes(treeCount));
+    };
+    const auto launchSmall = [&](auto kernel) {
+        launch(kernel, (docCount + dev::kSmallDocs - 1) / dev::kSmallDocs, dev::kSmallThreads, m.SmallLdsBytes(treeCount));
+    };
+    const bool shallow = m.MaxDepth <= 6;
+    if (docCount * passes <= kFewDocs && m.FewLdsBytes(treeCount) <= kMaxTileLdsBytes) {
+        if (dims == 1) {
+            shallow ? launchFew(dev::FewDocumentsKernel<6, 1>) : launchFew(dev::FewDocumentsKernel<8, 1>);
+        } else if (dims == 2) {
+            shallow ? launchFew(dev::FewDocumentsKernel<6, 2>) : launchFew(dev::FewDocumentsKernel<8, 2>);
+        } else {
+            shallow ? launchFew(dev::FewDocumentsKernel<6, 4>) : launchFew(dev::FewDocumentsKernel<8, 4>);
+        }
+    } else if (dims == 1) {
+        shallow ? launchSmall(dev::SmallBatchKernel<6, 1>) : launchSmall(dev::SmallBatchKernel<8, 1>);
+    } else if (dims == 2) {
+        shallow ? launchSmall(dev::SmallBatchKernel<6, 2>) : launchSmall(dev::SmallBatchKernel<8, 2>);
+    } else {
+        shallow ? launchSmall(dev::SmallBatchKernel<6, 4>) : launchSmall(dev::SmallBatchKernel<8, 4>);
+    }
+    HIP_CHECK(hipGetLastError());
+}
+
 int THipEvaluator::FusedLayoutFor(int layout, size_t stride, size_t docCount, size_t treeStart, size_t treeEnd, bool anyBatchSize) const {
     const TImpl& m = *Impl;
     const int layoutIndex = layout == TFeatureBatch::FlatRows ? 0 : layout == TFeatureBatch::SplitRows ? 1 : -1;
@@ -3214,6 +3392,12 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
     // whole-model calls only: a call for a range of the trees may take other kernels
     if (FusedLayoutFor(layout, stride, docCount, 0, TreeCount, false) >= 0) {
         return std::string("fused=") + m.FusedKernelName;
+    }
+    if (TakesSmallBatchKernel(docCount, 0, TreeCount)) {
+        const uint32_t sliceTrees = m.SmallSliceTrees(TreeCount);
+        const bool few = docCount * m.SmallPasses() <= kFewDocs && m.FewLdsBytes(TreeCount) <= kMaxTileLdsBytes;
+        return std::string("binarize=none;evaluate=") + (few ? "FewDocumentsKernel<" : "SmallBatchKernel<") + std::to_string(m.MaxDepth <= 6 ? 6 : 8) + ", " + std::to_string(m.SmallDims()) +
+               ">, " + std::to_string((TreeCount + sliceTrees - 1) / sliceTrees) + " slices of the trees";
     }
     std::string binarize = m.BinarizeBuckets == 0 ? "none"
                            : layout == TFeatureBatch::FlatColumns
@@ -3354,6 +3538,13 @@ void THipEvaluator::CalcDevice(const TFeatureBatch& batch, size_t docCount, size
     HIP_CHECK(hipSetDevice(m.DeviceId));
     TImpl::TContextLease ctx(m);
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : m.Stream;
+    if (TakesSmallBatchKernel(docCount, treeStart, treeEnd)) {
+        CheckBatch(batch, docCount);
+        LaunchSmallBatch(m, *ctx, batch, docCount, TreeCount, results, s, ctx->Ev[2]);
+        HIP_CHECK(hipEventSynchronize(ctx->Ev[2]));
+        SetLastTimes(&*ctx);
+        return;
+    }
     TKernelTimes times;
     HIP_CHECK(hipEventRecord(ctx->Ev[0], s));
     if (EvalRowsFusedDevice(batch, docCount, treeStart, treeEnd, results, s)) {
@@ -3452,6 +3643,17 @@ void GatherRows(const T* const* rows, size_t count, size_t rowLen, T* dst) {
     });
 }
 
+// documents [begin, begin + n) of columns [first, last), each given by pointer (null: zeros), into [column][n]
+void CopyColumns(const float* const* columns, size_t begin, size_t n, size_t first, size_t last, float* dst) {
+    for (size_t f = first; f < last; ++f) {
+        if (columns[f] != nullptr) {
+            std::memcpy(dst + f * n, columns[f] + begin, n * sizeof(float));
+        } else {
+            std::memset(dst + f * n, 0, n * sizeof(float));
+        }
+    }
+}
+
 // A model without trees answers with its bias whatever the prediction type: the reference fills the result
 // array with the bias values in turn and returns before any post-processing (cpu/formula_evaluator.cpp:29-41).
 void FillBiasOnly(const std::vector<double>& bias, size_t count, double* results) {
@@ -3493,11 +3695,34 @@ void RunPipeline(size_t docCount, size_t chunk, hipEvent_t (&done)[2], const TSt
 void THipEvaluator::SetLastTimes(const TKernelTimes& times) {
     std::lock_guard<std::mutex> guard(TimesLock);
     LastTimes = times;
+    LastSmallContext = nullptr;
+}
+
+void THipEvaluator::SetLastTimes(const void* smallContext) {
+    std::lock_guard<std::mutex> guard(TimesLock);
+    LastSmallContext = smallContext;
 }
 
 TKernelTimes THipEvaluator::LastKernelTimes() const {
     std::lock_guard<std::mutex> guard(TimesLock);
-    return LastTimes;
+    if (LastSmallContext == nullptr) {
+        return LastTimes;
+    }
+    // a small-batch launch left its workgroups' clock stamps on the device; they are fetched when somebody asks
+    const TImpl::THostContext& ctx = *static_cast<const TImpl::THostContext*>(LastSmallContext);
+    std::vector<unsigned long long> stamps(2 * ctx.StampCount);
+    int clockKhz = 0;
+    HIP_CHECK(hipSetDevice(Impl->DeviceId));
+    HIP_CHECK(hipDeviceGetAttribute(&clockKhz, hipDeviceAttributeWallClockRate, Impl->DeviceId));
+    HIP_CHECK(hipMemcpy(stamps.data(), ctx.Stamps.Get(), stamps.size() * sizeof(stamps[0]), hipMemcpyDeviceToHost));
+    unsigned long long begin = ~0ull, end = 0;
+    for (size_t i = 0; i + 1 < stamps.size(); i += 2) {
+        begin = std::min(begin, stamps[i]);
+        end = std::max(end, stamps[i + 1]);
+    }
+    TKernelTimes times;
+    times.EvalMs = end > begin && clockKhz > 0 ? static_cast<float>(end - begin) / static_cast<float>(clockKhz) : 0.f;
+    return times;
 }
 
 // Stages one chunk of rows given by pointer (the reference API's float** / hashed int**) and returns the
@@ -3560,6 +3785,29 @@ static void RunPredictionChunk(THipEvaluator& ev, THipEvaluator::TImpl::THostCon
     HIP_CHECK(hipEventRecord(slot.Ev[3], s));
 }
 
+// A small batch whose features are in the context's pinned memory: the kernel reads them there and writes the results to
+// pinned memory, so that nothing is copied by a command of its own.
+static void CalcSmallHostBatch(THipEvaluator& ev, THipEvaluator::TImpl& m, THipEvaluator::TImpl::THostContext& ctx,
+                               const TFeatureBatch& batch, size_t docCount, int predictionType, double* results) {
+    THipEvaluator::TImpl::THostSlot& slot = ctx.Slots[0];
+    const size_t dim = static_cast<size_t>(m.Dim);
+    const size_t outDim = predictionType == dev::kPredClass ? 1 : dim;
+    const bool raw = predictionType == dev::kPredRaw;
+    slot.PinnedResults.Reserve(docCount * dim);
+    if (!raw) {
+        slot.StageResults.Reserve(docCount * dim);
+    }
+    LaunchSmallBatch(m, ctx, batch, docCount, ev.GetTreeCount(), raw ? slot.PinnedResults.Get() : slot.StageResults.Get(), ctx.Stream,
+                     slot.Ev[3]);
+    if (raw) {
+        HIP_CHECK(hipEventSynchronize(slot.Ev[3]));
+    } else {
+        ev.ApplyPredictionTypeDevice(predictionType, 0, docCount, docCount, slot.StageResults.Get(), slot.PinnedResults.Get(), ctx.Stream);
+        HIP_CHECK(hipStreamSynchronize(ctx.Stream));
+    }
+    std::memcpy(results, slot.PinnedResults.Get(), docCount * outDim * sizeof(double));
+}
+
 void THipEvaluator::CalcHostRows(const float* const* rows, size_t rowLen, bool flat, const int32_t* const* catRows,
                                  size_t catRowLen, size_t docCount, size_t treeStart, size_t treeEnd, double* results,
                                  int predictionType) {
@@ -3580,6 +3828,24 @@ void THipEvaluator::CalcHostRows(const float* const* rows, size_t rowLen, bool f
     }
     HIP_CHECK(hipSetDevice(m.DeviceId));
     TImpl::TContextLease ctx(m);
+    if (TakesSmallBatchKernel(docCount, treeStart, treeEnd) && docCount * (needFloats + needCats) * 4 <= kSmallHostBytes) {
+        TImpl::THostSlot& slot = ctx->Slots[0];
+        slot.PinnedFloats.Reserve(std::max<size_t>(1, docCount * needFloats));
+        GatherRows(rows, docCount, needFloats, slot.PinnedFloats.Get());
+        TFeatureBatch batch;
+        batch.Layout = flat ? TFeatureBatch::FlatRows : TFeatureBatch::SplitRows;
+        batch.Floats = slot.PinnedFloats.Get();
+        batch.Stride = needFloats;
+        if (needCats) {
+            slot.PinnedCats.Reserve(docCount * needCats);
+            GatherRows(catRows, docCount, needCats, slot.PinnedCats.Get());
+            batch.Cats = slot.PinnedCats.Get();
+            batch.CatStride = needCats;
+        }
+        CalcSmallHostBatch(*this, m, *ctx, batch, docCount, predictionType, results);
+        SetLastTimes(&*ctx);
+        return;
+    }
     const size_t chunk = PipelineDocs((needFloats + needCats) * 4);
     const size_t stageDocs = std::min(chunk, docCount);
     for (int i = 0; i < (docCount > chunk ? 2 : 1); ++i) {
@@ -3629,6 +3895,18 @@ void THipEvaluator::CalcHostColumns(const float* const* columns, size_t columnCo
     }
     HIP_CHECK(hipSetDevice(m.DeviceId));
     TImpl::TContextLease ctx(m);
+    if (TakesSmallBatchKernel(docCount, treeStart, treeEnd) && docCount * need * 4 <= kSmallHostBytes) {
+        TImpl::THostSlot& slot = ctx->Slots[0];
+        slot.PinnedFloats.Reserve(std::max<size_t>(1, docCount * need));
+        CopyColumns(columns, 0, docCount, 0, need, slot.PinnedFloats.Get());
+        TFeatureBatch batch;
+        batch.Layout = TFeatureBatch::FlatColumns;
+        batch.Floats = slot.PinnedFloats.Get();
+        batch.Stride = docCount;
+        CalcSmallHostBatch(*this, m, *ctx, batch, docCount, predictionType, results);
+        SetLastTimes(&*ctx);
+        return;
+    }
     const size_t chunk = PipelineDocs(need * 4);
     const size_t stageDocs = std::min(chunk, docCount);
     for (int i = 0; i < (docCount > chunk ? 2 : 1); ++i) {
@@ -3646,15 +3924,8 @@ void THipEvaluator::CalcHostColumns(const float* const* columns, size_t columnCo
         [&](int i, size_t begin, size_t n) {
             TImpl::THostSlot& slot = ctx->Slots[i];
             float* dst = slot.PinnedFloats.Get();
-            ParallelCopy(need, need * n * sizeof(float), [=](size_t first, size_t last) {
-                for (size_t f = first; f < last; ++f) {
-                    if (columns[f] != nullptr) {
-                        std::memcpy(dst + f * n, columns[f] + begin, n * sizeof(float));
-                    } else {
-                        std::memset(dst + f * n, 0, n * sizeof(float));
-                    }
-                }
-            });
+            ParallelCopy(need, need * n * sizeof(float),
+                         [=](size_t first, size_t last) { CopyColumns(columns, begin, n, first, last, dst); });
             if (need) {
                 HIP_CHECK(hipMemcpyAsync(slot.StageFloats.Get(), dst, n * need * sizeof(float), hipMemcpyHostToDevice, ctx->Stream));
             }

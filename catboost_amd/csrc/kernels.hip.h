@@ -680,6 +680,339 @@ __global__ __launch_bounds__(256) void CombineSlicesKernel(const double* __restr
     out[i] = Finish(sum, scale, bias[i % static_cast<size_t>(dim)], true);
 }
 
+// ---- small batches of oblivious models: one launch from the features to the results ---------
+// A batch of a few thousand documents does not fill the chip, and its time is that of launches and of chains of dependent
+// loads, so it takes one kernel that compares the features with the splits' borders directly (no bins) and writes the
+// finished values; it may read the features from, and write the results to, pinned host memory. The values of the model's
+// features of a workgroup's documents go to LDS (a cell each); a tree is a row of sixteen dwords, eight levels' cells and
+// eight borders. The trees are summed in slices and the slices in slice order - the sums and the order of
+// CombineSlicesKernel, so that a document's value does not depend on which kernel took it. Two forms:
+//   FewDocumentsKernel  a workgroup per document, a lane per tree; the leaf values meet in LDS, where a thread per slice
+//                       adds its slice. What bounds it: the chain of loads cell -> feature -> leaf value, a few us.
+//   SmallBatchKernel    a workgroup per sixteen documents; a row of sixteen lanes (lane = document) walks a slice, the
+//                       lane's dword of a tree's row is handed round with DPP row broadcasts (every lane reading the
+//                       whole row would hold the texture path for 64 cycles per tree and wave). What bounds it: vector
+//                       issue, some 40 instructions per four trees * sixteen documents at two waves per SIMD.
+struct TSmallCell {       // a cell of the tile
+    uint32_t SrcFlat;     // column in flat rows or columns
+    uint32_t SrcSplit;    // column of the float (kind 0, 1) or categorical (kind 2) matrix
+    uint32_t Kind;        // 0: the value; 1: the value, NaN as +inf; 2: 1 where the hash is Value, else 0
+    uint32_t Value;
+};
+
+struct TSmallTables {
+    const TSmallCell* Cells;
+    const uint32_t* TreeRows;   // [trees + kSmallNullTrees null trees][16]: levels' cells, borders
+    const uint32_t* FirstLeaf;  // of a tree in Leaves, the null trees' too
+    const double* Leaves;
+    const double* Bias;
+    double Scale;
+    uint32_t CellCount;
+    uint32_t Dim;
+    uint32_t TreeCount;
+    uint32_t SliceTrees;
+    uint32_t SliceCount;
+};
+
+struct TSmallSource {     // value of feature f of document d: Floats[d * DocStride + f * ColumnStride], in dwords
+    const uint32_t* Floats;
+    size_t DocStride, ColumnStride;
+    const uint32_t* Cats;  // split rows: the hashed categorical values, else null
+    size_t CatStride;
+    uint32_t Split;        // split rows: columns are float and categorical indexes
+};
+
+constexpr int kSmallDocs = 16;                   // documents of a workgroup of SmallBatchKernel
+constexpr int kSmallNullTrees = 32;
+constexpr int kSmallThreads = 512;
+constexpr int kFewThreads = 1024;
+
+// Dwords between two documents of SmallBatchKernel's tile, [document][cell] so that a level's cell is one byte offset in
+// both kernels. Odd multiples of four: the sixteen documents of a cell fall on sixteen of the 64 banks.
+__host__ __device__ __forceinline__ uint32_t SmallDocPitch(uint32_t cells) {
+    return (cells + 3) / 8 * 8 + 4;
+}
+
+__device__ __forceinline__ uint32_t SmallCellValue(const TSmallSource& src, const TSmallCell& c, size_t doc) {
+    uint32_t v;
+    if (src.Split && c.Kind == 2) {
+        v = src.Cats[doc * src.CatStride + c.SrcSplit];
+    } else {
+        v = src.Floats[doc * src.DocStride + (src.Split ? c.SrcSplit : c.SrcFlat) * src.ColumnStride];
+    }
+    if (c.Kind == 1) {
+        v = isnan(__uint_as_float(v)) ? 0x7f800000u : v;
+    } else if (c.Kind == 2) {
+        v = v == c.Value ? 0x3f800000u : 0u;
+    }
+    return v;
+}
+
+// Start and end of a workgroup on the device's wall clock: stamps[workgroup][2]. (One pair for the launch, minimum and
+// maximum by atomics, held a launch of 256 workgroups back by some 5 us.)
+__device__ __forceinline__ void SmallStamp(ulonglong2* stamps, unsigned long long began) {
+    stamps[blockIdx.y * gridDim.x + blockIdx.x] = make_ulonglong2(began, wall_clock64());
+}
+
+// grid = (documents, ceil(dim / DIMS)), block = whole waves, at most kFewThreads; dynamic LDS = CellCount * 4 rounded up
+// to 8 + DIMS * SliceCount * (SliceTrees + 2) * 8 bytes.
+template <int DEPTH, int DIMS>
+__global__ __launch_bounds__(kFewThreads) void FewDocumentsKernel(TSmallSource src, uint32_t docCount, TSmallTables tab,
+                                                                  double* __restrict__ out, ulonglong2* __restrict__ stamps) {
+    extern __shared__ uint32_t sSmall[];
+    const unsigned long long began = wall_clock64();
+    const uint32_t tid = threadIdx.x, threads = blockDim.x;
+    const uint32_t doc = blockIdx.x, d0 = blockIdx.y * DIMS;
+    const uint32_t pitch = tab.SliceTrees + 1;  // the slices' values, one behind another, fall on different banks
+    double* values = reinterpret_cast<double*>(sSmall + (tab.CellCount + 1) / 2 * 2);  // [k][slice][pitch]
+    double* sums = values + static_cast<size_t>(DIMS) * tab.SliceCount * pitch;        // [k][slice]
+    uint4 cells[2], borders[2];
+    uint32_t first = 0;
+    const auto fetch = [&](uint32_t t) {
+        const uint4* row = reinterpret_cast<const uint4*>(tab.TreeRows) + static_cast<size_t>(t) * 4;
+        cells[0] = row[0];
+        borders[0] = row[2];
+        cells[1] = row[1];
+        borders[1] = row[3];
+        first = tab.FirstLeaf[t];
+    };
+    fetch(min(tid, tab.TreeCount - 1));  // in flight while the cells are filled
+    for (uint32_t i = tid; i < tab.CellCount; i += threads) {
+        sSmall[i] = SmallCellValue(src, tab.Cells[i], doc);
+    }
+    __syncthreads();
+    const uint8_t* tile = reinterpret_cast<const uint8_t*>(sSmall);
+    for (uint32_t t = tid; t < tab.TreeCount; t += threads) {
+        if (t != tid) {
+            fetch(t);
+        }
+        const uint32_t at[8] = {cells[0].x, cells[0].y, cells[0].z, cells[0].w, cells[1].x, cells[1].y, cells[1].z, cells[1].w};
+        const uint32_t border[8] = {borders[0].x, borders[0].y, borders[0].z, borders[0].w,
+                                    borders[1].x, borders[1].y, borders[1].z, borders[1].w};
+        uint32_t idx = 0;
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            const float x = *reinterpret_cast<const float*>(tile + at[d]);
+            idx |= (x > __uint_as_float(border[d]) ? 1u : 0u) << d;
+        }
+        const double* p = tab.Leaves + first + static_cast<size_t>(idx) * tab.Dim + d0;
+        const uint32_t slice = t / tab.SliceTrees, cell = slice * pitch + (t - slice * tab.SliceTrees);
+#pragma unroll
+        for (int k = 0; k < DIMS; ++k) {
+            if (DIMS == 1 || d0 + k < tab.Dim) {
+                values[k * tab.SliceCount * pitch + cell] = p[k];
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t dims = DIMS == 1 ? 1 : min(static_cast<uint32_t>(DIMS), tab.Dim - d0);
+    for (uint32_t i = tid; i < tab.SliceCount * dims; i += threads) {
+        const uint32_t slice = i % tab.SliceCount;
+        const uint32_t count = min(tab.SliceTrees, tab.TreeCount - slice * tab.SliceTrees);
+        const double* v = values + static_cast<size_t>(i) * pitch;
+        double sum = 0.0;
+#pragma unroll 8
+        for (uint32_t t = 0; t < count; ++t) {
+            sum = __dadd_rn(sum, v[t]);
+        }
+        sums[i] = sum;
+    }
+    __syncthreads();
+    if (tid < dims) {
+        const double* v = sums + tid * tab.SliceCount;
+        double sum = v[0];
+#pragma unroll 8
+        for (uint32_t slice = 1; slice < tab.SliceCount; ++slice) {
+            sum = __dadd_rn(sum, v[slice]);
+        }
+        out[static_cast<size_t>(doc) * tab.Dim + d0 + tid] = Finish(sum, tab.Scale, tab.Bias[d0 + tid], true);
+        if (tid == 0) {
+            SmallStamp(stamps, began);
+        }
+    }
+}
+
+// the value of lane N of the lane's row of sixteen
+template <int N>
+__device__ __forceinline__ uint32_t RowBroadcast(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x150 + N, 0xf, 0xf, true));
+}
+
+// leaf indexes of trees FIRST .. FIRST + 3 of a turn; level d decides bit d
+template <int D, int FIRST, int N>
+__device__ __forceinline__ void SmallLevels(const uint8_t* docTile, const uint32_t (&row)[N], uint32_t (&idx)[4]) {
+    if constexpr (D >= 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float x = *reinterpret_cast<const float*>(docTile + RowBroadcast<D>(row[FIRST + i]));
+            idx[i] = idx[i] + idx[i] + (x > __uint_as_float(RowBroadcast<8 + D>(row[FIRST + i])) ? 1u : 0u);
+        }
+        SmallLevels<D - 1, FIRST>(docTile, row, idx);
+    }
+}
+
+// The leaf values of a turn's trees, four trees at a time: the scheduler would otherwise start the reads of all of them
+// and spill. `leafOfLane`: first leaf of tree i in lane i of the row.
+template <int DEPTH, int DIMS, int FIRST, int N>
+__device__ __forceinline__ void SmallLeafValues(const uint8_t* docTile, const uint32_t (&row)[N], uint32_t leafOfLane,
+                                                const double* leaves, uint32_t dim, uint32_t dimsLeft, double (&value)[N][DIMS]) {
+    if constexpr (FIRST < N) {
+        uint32_t idx[4] = {0, 0, 0, 0};
+        SmallLevels<DEPTH - 1, FIRST>(docTile, row, idx);
+        const uint32_t leaf[4] = {RowBroadcast<FIRST>(leafOfLane), RowBroadcast<FIRST + 1>(leafOfLane),
+                                  RowBroadcast<FIRST + 2>(leafOfLane), RowBroadcast<FIRST + 3>(leafOfLane)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const double* p = leaves + (DIMS == 1 ? leaf[i] + idx[i] : leaf[i] + static_cast<size_t>(idx[i]) * dim);
+#pragma unroll
+            for (int k = 0; k < DIMS; ++k) {
+                value[FIRST + i][k] = DIMS == 1 || static_cast<uint32_t>(k) < dimsLeft ? p[k] : 0.0;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        SmallLeafValues<DEPTH, DIMS, FIRST + 4>(docTile, row, leafOfLane, leaves, dim, dimsLeft, value);
+    }
+}
+
+// grid = (ceil(documents / 16), ceil(dim / DIMS)), block = kSmallThreads: 32 slices at a time;
+// dynamic LDS = 16 * SmallDocPitch(CellCount) * 4 + SliceCount * 16 * DIMS * 8 bytes.
+template <int DEPTH, int DIMS>
+__global__ __launch_bounds__(kSmallThreads) void SmallBatchKernel(TSmallSource src, uint32_t docCount, TSmallTables tab,
+                                                                  double* __restrict__ out, ulonglong2* __restrict__ stamps) {
+    // trees of a turn: their rows, and the leaf values of the turn before, are in flight together
+    constexpr int kTurn = DIMS == 1 ? 16 : DIMS == 2 ? 8 : 4;
+    static_assert(2 * kTurn <= kSmallNullTrees, "rows are fetched up to a turn past the last one");
+    extern __shared__ uint32_t sSmall[];
+    const unsigned long long began = wall_clock64();
+    constexpr uint32_t threads = kSmallThreads;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t firstDoc = blockIdx.x * kSmallDocs;
+    const uint32_t docs = min(static_cast<uint32_t>(kSmallDocs), docCount - firstDoc);
+    const uint32_t d0 = blockIdx.y * DIMS;
+    const uint32_t lane = tid % kSmallDocs;
+    const uint32_t docPitch = SmallDocPitch(tab.CellCount);
+    double* sums = reinterpret_cast<double*>(sSmall + docPitch * kSmallDocs);  // [slice][k][document]
+    uint32_t next[kTurn], nextLeaf;
+    const auto fetch = [&](uint32_t t) {
+#pragma unroll
+        for (int i = 0; i < kTurn; ++i) {
+            next[i] = tab.TreeRows[static_cast<size_t>(t + i) * 16 + lane];
+        }
+        nextLeaf = tab.FirstLeaf[t + lane % kTurn];  // lane i: tree i's
+    };
+    fetch(min(tid / kSmallDocs * tab.SliceTrees, tab.TreeCount));  // in flight while the tile is filled
+    // Neighbouring threads read neighbouring addresses: cells of a document, or documents of a column. A thread's cells of
+    // a turn are asked for together, then their values: two trips to memory for up to 256 (128) cells.
+    constexpr uint32_t kCells = 4;
+    if (src.ColumnStride == 1) {
+        constexpr uint32_t kDocs = kSmallDocs / (kSmallThreads / kWave);
+        for (uint32_t cell = tid % kWave; cell < tab.CellCount; cell += kCells * kWave) {
+            TSmallCell c[kCells];
+            uint32_t v[kCells][kDocs];
+#pragma unroll
+            for (uint32_t i = 0; i < kCells; ++i) {
+                c[i] = tab.Cells[min(cell + i * kWave, tab.CellCount - 1)];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kCells; ++i) {
+#pragma unroll
+                for (uint32_t j = 0; j < kDocs; ++j) {
+                    v[i][j] = SmallCellValue(src, c[i], firstDoc + min(tid / kWave * kDocs + j, docs - 1));
+                }
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kCells; ++i) {
+#pragma unroll
+                for (uint32_t j = 0; j < kDocs; ++j) {
+                    if (cell + i * kWave < tab.CellCount) {
+                        sSmall[(cell + i * kWave) + (tid / kWave * kDocs + j) * docPitch] = v[i][j];
+                    }
+                }
+            }
+        }
+    } else {
+        constexpr uint32_t kRows = kSmallThreads / kSmallDocs;
+        for (uint32_t cell = tid / kSmallDocs; cell < tab.CellCount; cell += kCells * kRows) {
+            TSmallCell c[kCells];
+            uint32_t v[kCells];
+#pragma unroll
+            for (uint32_t i = 0; i < kCells; ++i) {
+                c[i] = tab.Cells[min(cell + i * kRows, tab.CellCount - 1)];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kCells; ++i) {
+                v[i] = SmallCellValue(src, c[i], firstDoc + min(lane, docs - 1));
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kCells; ++i) {
+                if (cell + i * kRows < tab.CellCount) {
+                    sSmall[(cell + i * kRows) + lane * docPitch] = v[i];
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const uint8_t* docTile = reinterpret_cast<const uint8_t*>(sSmall + lane * docPitch);  // (documents past the last one: the last one again)
+    const double* leaves = tab.Leaves + d0;
+    for (uint32_t slice = tid / kSmallDocs; slice < tab.SliceCount; slice += threads / kSmallDocs) {
+        const uint32_t begin = slice * tab.SliceTrees;
+        const uint32_t end = min(begin + tab.SliceTrees, tab.TreeCount);
+        if (slice != tid / kSmallDocs) {
+            fetch(begin);
+        }
+        double acc[DIMS], value[kTurn][DIMS];
+#pragma unroll
+        for (int k = 0; k < DIMS; ++k) {
+            acc[k] = 0.0;
+        }
+        // Slices are a multiple of a turn, or the whole model: trees past the end of it are null trees, whose leaf is zero.
+        const auto add = [&] {
+#pragma unroll
+            for (int i = 0; i < kTurn; ++i) {
+#pragma unroll
+                for (int k = 0; k < DIMS; ++k) {
+                    acc[k] = __dadd_rn(acc[k], value[i][k]);
+                }
+            }
+        };
+        for (uint32_t t = begin; t < end; t += kTurn) {
+            uint32_t row[kTurn];
+#pragma unroll
+            for (int i = 0; i < kTurn; ++i) {
+                row[i] = next[i];
+            }
+            const uint32_t leafOfLane = nextLeaf;
+            if (t + kTurn < end) {
+                fetch(t + kTurn);
+            }
+            if (t > begin) {
+                add();  // the values of the turn before
+            }
+            SmallLeafValues<DEPTH, DIMS, 0>(docTile, row, leafOfLane, leaves, tab.Dim, tab.Dim - d0, value);
+        }
+        add();
+#pragma unroll
+        for (int k = 0; k < DIMS; ++k) {
+            sums[(slice * DIMS + k) * kSmallDocs + lane] = acc[k];
+        }
+    }
+    __syncthreads();
+    if (tid < kSmallDocs * DIMS) {
+        const uint32_t k = tid / kSmallDocs;
+        if (lane < docs && d0 + k < tab.Dim) {
+            double sum = sums[tid];
+#pragma unroll 8
+            for (uint32_t slice = 1; slice < tab.SliceCount; ++slice) {
+                sum = __dadd_rn(sum, sums[slice * DIMS * kSmallDocs + tid]);
+            }
+            out[static_cast<size_t>(firstDoc + lane) * tab.Dim + d0 + k] = Finish(sum, tab.Scale, tab.Bias[d0 + k], true);
+        }
+        if (tid == 0) {
+            SmallStamp(stamps, began);
+        }
+    }
+}
+
 // Packed tree table of the tile kernel: 16 dwords per tree. Slots 0..7 hold the tree's levels
 // (slot d = split d, unused levels padded with a split that is false for every bin), slot 8 the
 // index of the tree's first leaf value. A level is

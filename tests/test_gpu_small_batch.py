@@ -86,3 +86,75 @@ def test_small_batch_slicing_switched_off_through_the_api():
     ev.set_small_batch_slicing(True)
     assert "slices" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, 3000)["evaluate"]
     np.testing.assert_array_equal(model.calc_flat(host), sliced)
+
+
+@pytest.mark.parametrize("seed,n_float,n_cat,trees,depth,dim,many,docs", [
+    (1, 7, 2, 1, 6, 1, False, (1, 2)),
+    (2, 20, 0, 31, 4, 1, False, (1, 15, 16, 17)),
+    (3, 9, 6, 63, 8, 1, True, (5, 640, 641)),        # a slice of two turns and a ragged one; one-hot; more than 254 borders
+    (4, 130, 3, 64, 7, 1, False, (33, 1000)),        # two slices; cells of three turns of the tile
+    (5, 300, 4, 97, 6, 2, False, (3, 320, 321)),     # two dimensions: documents count twice
+    (6, 40, 2, 1100, 5, 3, False, (17, 700)),        # more slices than rows of a workgroup
+    (7, 12, 1, 33, 8, 9, False, (16, 400)),          # three passes over the dimensions, the last of one
+    (8, 700, 10, 200, 8, 1, False, (1, 64, 1500)),   # wider than the register kernels
+])
+def test_small_kernels_against_the_oracle(seed, n_float, n_cat, trees, depth, dim, many, docs):
+    """One launch from the features to the results: a lane per tree for few documents, sixteen lanes of documents per
+    slice of the trees beyond. Every layout, device and host entry points, NaN modes, one-hot splits."""
+    import torch
+
+    from tests.test_oracle import _random_flat_data, _random_oblivious
+
+    rng = np.random.default_rng(seed)
+    model, cat_values = _random_oblivious(rng, n_float=n_float, n_cat=n_cat, trees=trees, max_depth=depth, dim=dim,
+                                          many_borders=many, scale=0.5, bias=rng.normal(size=dim))
+    o = OracleModel(model)
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    float_at = [f["flat_index"] for f in model["float_features"]]
+    cat_at = [c["flat_index"] for c in model["cat_features"]]
+    for n in docs:
+        kernel = ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, n)["evaluate"]
+        passes = 1 if dim <= 2 else (dim + 3) // 4
+        assert kernel.startswith("FewDocumentsKernel" if n * passes <= 640 else "SmallBatchKernel"), kernel
+        x = _random_flat_data(rng, model, cat_values, n)
+        expected = o.calc(x)
+        close = dict(rtol=1e-9, atol=1e-12)
+        np.testing.assert_allclose(g.calc_flat(x), expected, **close)
+        np.testing.assert_allclose(g.calc_flat_transposed(np.ascontiguousarray(x.T)), expected, **close)
+        floats, cats = np.ascontiguousarray(x[:, float_at]), np.ascontiguousarray(x[:, cat_at]).view(np.int32)
+        if n_cat:
+            np.testing.assert_allclose(g.calc_hashed(floats, cats), expected, **close)
+        flat, columns = torch.from_numpy(x).to("cuda:0"), torch.from_numpy(np.ascontiguousarray(x.T)).to("cuda:0")
+        f, c = torch.from_numpy(floats).to("cuda:0"), torch.from_numpy(cats).to("cuda:0")
+        for feats in (ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), flat.shape[1]),
+                      ev.features(cb.LAYOUT_FLAT_COLUMNS, columns.data_ptr(), n),
+                      ev.features(cb.LAYOUT_SPLIT_ROWS, f.data_ptr(), f.shape[1], c.data_ptr(), c.shape[1])):
+            out = torch.full((n * dim + 8,), -3.0, dtype=torch.float64, device="cuda:0")
+            torch.cuda.synchronize()
+            ev.eval_data(feats, n, out.data_ptr())
+            np.testing.assert_allclose(out.cpu().numpy()[:n * dim], expected, **close)
+            assert (out.cpu().numpy()[n * dim:] == -3.0).all()
+        assert ev.last_kernel_times()[1] > 0.0
+
+
+def test_a_documents_value_does_not_depend_on_the_small_kernel_that_took_it():
+    """The slices of the trees and the order of their sums are those of the register kernels' small batches."""
+    import torch
+
+    model, info = syn.build_model("C1", trees=150)
+    model.enable_gpu_evaluation(0)
+    ev = model.evaluator()
+    x = syn.device_features(info, 20_000)
+    values = {}
+    for docs in (3, 640, 641, 16_384, 20_000):
+        part = x[:docs].contiguous()
+        out = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, part.data_ptr(), part.shape[1]), docs, out.data_ptr())
+        values[docs] = out.cpu().numpy()
+    assert "cbamd_eval_reg" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, 20_000)["evaluate"]
+    for docs, v in values.items():
+        np.testing.assert_array_equal(v, values[20_000][:docs])
