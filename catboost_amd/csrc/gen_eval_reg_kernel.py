@@ -47,14 +47,16 @@ Kernel arguments (80 bytes):
   48 scale       double          56 bias const double* (first dimension of this launch)
   64 bucketCount uint32 (1 .. BUCKETS)                68 dim uint32
   72 first dimension of this launch uint32            76 dimensions to store uint32 (1 .. PITCH)
-  80 tree blocks per slice uint32 (kernels that are not fused)
+  80 tree blocks per slice uint32                     84 slices per workgroup uint32 (kernels that are not fused)
   88 map of the bins registers const uint32* (kernels that are not fused, read when flags bit 3 is set;
      96 bytes in all)
-grid = (ceil(blockCount / WAVES), slices) workgroups of WAVES * 64 threads, LDS = 2 * TREE_BLOCK * LEAVES *
-PITCH * 8 bytes. Slice y of the grid takes the tree blocks from y * (tree blocks per slice) on, at most that
-many, and writes to out + y * docCount * dim: a small batch is spread over the chip by giving every slice
-of the trees its own workgroups, which store raw sums (flags bit 2) that a second kernel adds up in slice
-order. One slice (grid.y = 1, tree blocks per slice = treeBlocks) is the plain launch.
+grid = (ceil(blockCount / WAVES), ceil(slices / slices per workgroup)) workgroups of WAVES * 64 threads, LDS =
+2 * TREE_BLOCK * LEAVES * PITCH * 8 bytes. Slice s takes the tree blocks from s * (tree blocks per slice) on, at most
+that many, and writes to out + s * docCount * dim: a small batch is spread over the chip by giving the slices of
+the trees to different workgroups, which store raw sums (flags bit 2) that a second kernel adds up in slice
+order. A workgroup of several slices loads its bins once and walks on from slice to slice (an even number of tree
+blocks each), storing and clearing its sums in between. One slice (grid.y = 1, tree blocks per slice = treeBlocks) is
+the plain launch.
 
 Fused variants ("cbamd_fused_..."; one-dimensional float-only models, plain and six-bit forms) take the
 documents' fp32 rows instead of bins and binarize them into the bins registers themselves, so the bins
@@ -549,6 +551,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  s_load_dwordx4 s[96:99], s[0:1], 0x40")
     if not fused:
         e("  s_load_dword s101, s[0:1], 0x50")         # tree blocks per slice
+        e("  s_load_dword s34, s[0:1], 0x54")          # slices of a workgroup
     if fused:
         e("  s_load_dwordx4 s[84:87], s[0:1], 0x50")   # floats, unit records
         e("  s_load_dwordx2 s[88:89], s[0:1], 0x60")   # row stride in bytes, units
@@ -577,10 +580,14 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  v_add_u32_e32 v2, s28, v2")
     e("  s_waitcnt lgkmcnt(0)")
     if not fused:
-        # the slice of the trees that this row of the grid takes (s3: workgroup id y)
+        # the slices of the trees that this row of the grid takes (s3: workgroup id y)
+        e("  s_mul_i32 s3, s3, s34")                 # its first slice
         e("  s_mul_i32 s24, s3, s101")               # its first tree block
         e("  s_sub_u32 s25, s14, s24")
-        e("  s_min_u32 s14, s25, s101")              # its tree blocks
+        e("  s_mul_i32 s28, s34, s101")
+        e("  s_min_u32 s35, s25, s28")               # its tree blocks
+        e("  s_min_u32 s14, s35, s101")              # those of the first slice,
+        e("  s_sub_u32 s35, s35, s14")               # and behind it
         e("  s_mul_i32 s25, s24, %d" % (block * tree_row_bytes))
         e("  s_add_u32 s6, s6, s25")
         e("  s_addc_u32 s7, s7, 0")
@@ -604,6 +611,8 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  s_add_u32 s21, s21, s20")
     e("  s_add_u32 s24, s13, -1")
     e("  s_min_u32 s24, s21, s24")
+    if not fused:
+        e("  s_mov_b32 s13, s35")                    # tree blocks of the workgroup behind the slice's
     if fused:
         fused_binarize()
     else:
@@ -617,7 +626,10 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  s_bitcmp1_b32 s15, 3")
         e("  s_cbranch_scc1 %s_mapped" % name)
         for i in range(buckets):
-            # registers past the model's bucket count reload the last bucket and are never indexed
+            # registers past the model's bucket count reload the last bucket or stay as they are: never indexed
+            if i and i % 16 == 0:
+                e("  s_cmp_le_u32 s96, %d" % i)
+                e("  s_cbranch_scc1 %s_loaded" % name)
             e("  s_min_u32 s24, %d, s28" % i)
             e("  s_lshl_b32 s24, s24, 8")
             e("  s_add_u32 s34, s32, s24")
@@ -816,13 +828,14 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             e("  v_add_f64 v[%d:%d], v[%d:%d], s[%d:%d]" % (ac(j, k), ac(j, k) + 1, ac(j, k), ac(j, k) + 1,
                                                              32 + 2 * k, 33 + 2 * k))
     e("%s_store:" % name)
+    # (the tables' position, the next trees' rows and a deep tree's byte selectors are still needed if a slice follows)
     e("  v_and_b32_e32 v5, 63, v0")
-    e("  s_lshl_b32 s24, s21, 8")
-    e("  v_add_u32_e32 v5, s24, v5")
+    e("  s_lshl_b32 s28, s21, 8")
+    e("  v_add_u32_e32 v5, s28, v5")
     for j in range(4):
         e("  v_add_u32_e32 v%d, %d, v5" % (te0, 64 * j))
         e("  v_cmp_gt_u32_e32 vcc, s12, v%d" % te0)
-        e("  s_and_saveexec_b64 s[30:31], vcc")
+        e("  s_and_saveexec_b64 s[4:5], vcc")
         e("  v_mul_lo_u32 v%d, v%d, s97" % (te0 + 1, te0))               # document * dim
         e("  v_add_lshl_u32 v%d, v%d, s98, 3" % (te0 + 1, te0 + 1))     # + first dimension, in bytes
         for k in range(pitch):
@@ -831,7 +844,28 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 e("  s_cbranch_scc0 %s_stored_%d" % (name, j))
             e("  global_store_dwordx2 v%d, v[%d:%d], s[10:11] offset:%d" % (te0 + 1, ac(j, k), ac(j, k) + 1, 8 * k))
         e("%s_stored_%d:" % (name, j))
-        e("  s_mov_b64 exec, s[30:31]")
+        e("  s_mov_b64 exec, s[4:5]")
+    if not fused:
+        # The workgroup's next slice: a slice ends behind the second buffer, so its first tree block sits in the first
+        # one and its first rows in their registers, as at the end of a turn of the loop. The sums start again at
+        # zero, at the next slice's place in `out`.
+        e("  s_cmp_eq_u32 s13, 0")
+        e("  s_cbranch_scc1 %s_end" % name)
+        e("  s_min_u32 s14, s13, s101")
+        e("  s_sub_u32 s13, s13, s14")
+        e("  s_mul_i32 s28, s12, s97")
+        e("  s_lshl_b32 s28, s28, 3")
+        e("  s_add_u32 s10, s10, s28")
+        e("  s_addc_u32 s11, s11, 0")
+        e("  s_add_u32 s6, s6, %d" % (2 * block * tree_row_bytes))
+        e("  s_addc_u32 s7, s7, 0")
+        e("  s_add_u32 s30, s30, %d" % (2 * block * tree_row_bytes))
+        e("  s_addc_u32 s31, s31, 0")
+        for r in list(range(lv0, ga0)) + (list(range(lw0, lw0 + 8)) if two_sets else []):
+            e("  v_mov_b32_e32 v%d, 0" % r)
+        e("  s_set_gpr_idx_on s22, 0x1")
+        e("  s_branch %s_loop" % name)
+        e("%s_end:" % name)
     e("  s_endpgm")
     e(".Lend_%s:" % name)
     e(".size %s, .Lend_%s-%s" % (name, name, name))

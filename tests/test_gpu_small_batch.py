@@ -158,3 +158,42 @@ def test_a_documents_value_does_not_depend_on_the_small_kernel_that_took_it():
     assert "cbamd_eval_reg" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, 20_000)["evaluate"]
     for docs, v in values.items():
         np.testing.assert_array_equal(v, values[20_000][:docs])
+
+
+@pytest.mark.parametrize("seed,n_float,n_cat,trees,depth,dim,many,docs", [
+    (1, 40, 0, 150, 6, 1, False, 131_073),    # five slices, the last of 22 trees; 16-tree blocks
+    (2, 150, 0, 500, 8, 1, False, 60_001),    # sixteen slices, the last of 20 trees
+    (3, 30, 6, 330, 8, 1, True, 100_000),     # bins in mapped registers, one-hot splits
+    (4, 60, 0, 200, 7, 6, False, 70_007),     # several dimensions: small tree blocks, many to a slice
+    (5, 50, 0, 161, 10, 1, False, 90_001),    # deep trees: byte selectors in scalar registers; a slice of one tree
+])
+def test_workgroups_that_walk_several_slices(seed, n_float, n_cat, trees, depth, dim, many, docs):
+    """A batch of more (document, slice) pairs than the chip holds workgroups has workgroups walk several slices: the
+    same bits as batches whose workgroups take one slice each."""
+    import torch
+
+    from tests.test_oracle import _random_flat_data, _random_oblivious
+
+    rng = np.random.default_rng(seed)
+    model, cat_values = _random_oblivious(rng, n_float=n_float, n_cat=n_cat, trees=trees, max_depth=depth, dim=dim,
+                                          many_borders=many, scale=0.5, bias=rng.normal(size=dim))
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    kernels = ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"]
+    assert "cbamd_eval_reg" in kernels and "slices" in kernels, kernels
+    x = _random_flat_data(rng, model, cat_values, docs)
+    flat = torch.from_numpy(x).to("cuda:0")
+    out = torch.full((docs * dim + 8,), -3.0, dtype=torch.float64, device="cuda:0")
+    parts = torch.zeros(docs * dim, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), flat.shape[1]), docs, out.data_ptr())
+    for begin in range(0, docs, 2048):
+        n = min(2048, docs - begin)
+        ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, flat[begin:].data_ptr(), flat.shape[1]), n, parts[begin * dim:].data_ptr())
+    assert torch.equal(out[:docs * dim], parts)
+    assert bool((out[docs * dim:] == -3.0).all())
+    sample = rng.choice(docs, size=2000, replace=False)
+    np.testing.assert_allclose(out.cpu().numpy()[:docs * dim].reshape(docs, dim)[sample],
+                               OracleModel(model).calc(x[sample]).reshape(-1, dim), rtol=1e-9, atol=1e-12)
