@@ -607,11 +607,11 @@ uint32_t QuadTileWaves(uint32_t rows, int maxd) {
     return QuadTileLdsBytes(rows, maxd, 8) <= kMaxTileLdsBytes ? 8u : QuadTileLdsBytes(rows, maxd, 4) <= kMaxTileLdsBytes ? 4u : 0u;
 }
 
-// LDS of the pair-tile kernel: 128 documents' bins, then per wave the leaf values of two trees; the same area
-// takes one partial sum per wave, lane group and document at the end
+// LDS of the pair-tile kernel: 128 documents' bins, then per wave the leaf values of one tree of 256 leaves or two of 64;
+// the same area takes one partial sum per wave and document at the end
 size_t PairTileLdsBytes(uint32_t buckets, int maxd) {
     return ((static_cast<size_t>(buckets) * 128 + 15) & ~size_t(15)) +
-           static_cast<size_t>(dev::kTileWaves) * 2 * std::max<size_t>(size_t(1) << maxd, 128) * sizeof(double);
+           static_cast<size_t>(dev::kPairWaves) * std::max<size_t>(size_t(1) << maxd, 128) * sizeof(double);
 }
 
 // dimensions the tile kernel accumulates per pass over the trees (and the pitch of its padded leaf rows)
@@ -3089,7 +3089,7 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
             const size_t lds = PairTileLdsBytes(m.TileRowCount, maxd);
             const auto launch = [&](auto kernel) {
                 EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds);
-                hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(2 * blocks)), dim3(64 * dev::kTileWaves), lds, s,
+                hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(2 * blocks)), dim3(64 * dev::kPairWaves), lds, s,
                                    reinterpret_cast<const uint16_t*>(bins), docCount, m.LayoutBuckets, m.TileMap.Get(),
                                    m.TileRowCount, reinterpret_cast<const uint4*>(m.PairRows.Get()),
                                    reinterpret_cast<const double2*>(m.HalfTileLeaves.Get()), m.Bias.Get(), m.Scale, tb, te,

@@ -1433,23 +1433,30 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousHalfTileKernel(
 // bit 7 exactly when bin == value).
 // `pairRows` holds 8 dwords per tree, one per level: byte offset of the level's bucket in the tile (bucket * 128,
 // bits 7-16) | xor byte (bits 0-6) | the value added to each of the four bins << 24, slot 0 also bit 23 when some
-// level of the tree xors (PackedPairTreeIndexes). Levels past the tree's depth are zero (bucket 0, add 0: never
+// level of the tree xors (WalkPackedPairLevels). Levels past the tree's depth are zero (bucket 0, add 0: never
 // true). A lane keeps its tree's row in registers (two 16-byte loads, the same addresses for the 32 lanes of a
 // group; with offsets and values to add as a dword each the row took four, and the kernel, which is bound by the
 // bytes its lanes receive over the vector memory path, 49 ms instead of 41 on 10M documents x 5000 trees) and the wave
-// publishes the two trees' leaf values, which are contiguous in `leaves` (1 << MAXD doubles per tree), in its
-// own LDS region. Waves take the pairs round robin; a last tree without a partner is done by wave 0 with both
-// groups on the same tree and only the first one adding. Partial sums (one per wave and group) are added in a
-// fixed order at the end. The fetches run kPairAhead rounds ahead of the walk without looking at the tree range:
-// both tables end with kPairTreePadding trees' worth of zeros. The LDS reads of a pair's levels are issued a round
-// before the arithmetic on them, behind the previous pair's leaf values going into the region, so a round's
-// instructions never wait for reads of its own (a null tree's levels read row 0).
+// publishes the trees' leaf values (1 << MAXD doubles per tree, a pair's side by side in `leaves`) in its own LDS
+// region, one tree after the other: before the gathers the two groups swap half of their indexes, so that every lane
+// has two documents of either tree (documents j * 64 + 2 * m + group, j = 0, 1), gathers them from the first tree's
+// values, and the second tree's then go to the same place (LDS serves a wave's requests in order). With 2 KB per wave
+// instead of a pair's 4 KB sixteen waves find room beside the widest tile instead of eight. That is what the kernel
+// lacked: a wave issues an instruction about every nine cycles, and two waves per SIMD left half of the SIMD's issue
+// cycles empty (PAIR_NUMBERS).
+// Waves take the pairs round robin; a last tree without a partner is done by wave 0 with both groups on the same tree
+// and its values added once. Partial sums (one per wave) are added in a fixed order at the end. The fetches run
+// kPairAhead rounds ahead of the walk without looking at the tree range: both tables end with kPairTreePadding trees'
+// worth of zeros (a null tree's levels read row 0).
 // With `tileMap` the tile has rowCount rows (MapTileBins) and the offsets in pairRows name rows, not buckets.
-// grid = 2 * doc blocks, block = 64 * kTileWaves threads, dynamic LDS = rows * 128 (rounded up to 16) +
-// kTileWaves * 2 * max(1 << MAXD, 128) * 8 bytes (the leaf regions, later the partial sums).
+// The two halves of a block read the same lines of `bins`, two bytes of every four, so they go to workgroups of one
+// XCD that start one after the other (workgroups go round-robin to the XCDs).
+// grid = 2 * doc blocks, block = 64 * kPairWaves threads, dynamic LDS = rows * 128 (rounded up to 16) +
+// kPairWaves * max(1 << MAXD, 128) * 8 bytes (the leaf regions, later the partial sums).
 constexpr uint32_t kPairRowXorFlag = 1u << 23;  // slot 0 of a tree's row: some level xors
+constexpr int kPairWaves = 16;
 constexpr int kPairAhead = 3;
-constexpr int kPairTreePadding = 2 * kTileWaves * kPairAhead;
+constexpr int kPairTreePadding = 2 * kPairWaves * kPairAhead;
 
 // Rows of a tile that splits the buckets of more than 127 values in two (`tileMap`, a dword per row: bits 0-15 the
 // bucket, bits 16.. what becomes of its bins: 0 as they are, 1 min(bin, 127), 2 max(bin - 127, 0)), byte-parallel.
@@ -1484,50 +1491,7 @@ __device__ __forceinline__ uint32_t MapTileBins(uint32_t bins4, uint32_t mode) {
 // lands in bit 6 while the following level's lands in bit 7, and a pair of levels joins the index with one shift
 // and two bit-field inserts: eighteen instructions for eight levels where the one-level-at-a-time form takes
 // twenty-four (a one-hot level on an even position xors with the low six bits of its mask).
-template <bool XOR, int MAXD, bool SIX>
-__device__ __forceinline__ uint32_t PackedPairTreeIndexes(uint32_t laneOffset, const uint4 (&desc)[2]) {
-    const uint32_t levels[8] = {desc[0].x, desc[0].y, desc[0].z, desc[0].w, desc[1].x, desc[1].y, desc[1].z, desc[1].w};
-    uint32_t a[MAXD];
-#pragma unroll
-    for (int d = 0; d < MAXD; ++d) {
-        a[d] = *reinterpret_cast<const __attribute__((address_space(3))) uint32_t*>((levels[d] & 0x1ff80u) | laneOffset);
-    }
-    // one wait for the eight reads (lgkmcnt 0, the other counters untouched)
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_sched_barrier(0);
-    uint32_t r[MAXD];
-#pragma unroll
-    for (int d = 0; d < MAXD; ++d) {
-        uint32_t v = a[d];
-        if (XOR) {
-            const uint32_t x = levels[d] & 0x7fu;
-            v ^= __builtin_amdgcn_perm(x, x, 0u);  // the xor byte four times
-        }
-        r[d] = v + __builtin_amdgcn_perm(levels[d], levels[d], 0x03030303u);  // byte 3 four times
-    }
-    uint32_t idx4 = 0;
-    if constexpr (SIX) {
-        static_assert(MAXD % 2 == 0, "levels in pairs");
-#pragma unroll
-        for (int d = 0; d < MAXD; d += 2) {
-            // bit 7 of the odd level, bit 6 of the even one; below them what is left of the even level's sum, which
-            // only the first pair lets through: those six bits leave the byte with the shifts that follow (MAXD 8)
-            // or end below the six bits that index the leaves (MAXD 6)
-            const uint32_t pair = (r[d + 1] & 0x80808080u) | (r[d] & 0x7f7f7f7fu);
-            idx4 = d == 0 ? pair : (pair & 0xc0c0c0c0u) | ((idx4 >> 2) & 0x3f3f3f3fu);
-        }
-    } else {
-#pragma unroll
-        for (int d = 0; d < MAXD; ++d) {
-            idx4 = (r[d] & 0x80808080u) | (idx4 >> 1);
-        }
-    }
-    return idx4;
-}
-
-// The two halves of PackedPairTreeIndexes for a kernel that keeps the reads of a tree's levels one round ahead of
-// the arithmetic on them: the reads alone, and the walk on what they returned.
+// In two halves: the LDS reads of a tree's levels, and the walk on what they returned.
 template <int MAXD>
 __device__ __forceinline__ void ReadPackedPairLevels(uint32_t laneOffset, const uint4 (&desc)[2], uint32_t (&a)[MAXD]) {
     const uint32_t levels[8] = {desc[0].x, desc[0].y, desc[0].z, desc[0].w, desc[1].x, desc[1].y, desc[1].z, desc[1].w};
@@ -1555,6 +1519,9 @@ __device__ __forceinline__ uint32_t WalkPackedPairLevels(const uint32_t (&a)[MAX
         static_assert(MAXD % 2 == 0, "levels in pairs");
 #pragma unroll
         for (int d = 0; d < MAXD; d += 2) {
+            // bit 7 of the odd level, bit 6 of the even one; below them what is left of the even level's sum, which
+            // only the first pair lets through: those six bits leave the byte with the shifts that follow (MAXD 8)
+            // or end below the six bits that index the leaves (MAXD 6)
             const uint32_t pair = (r[d + 1] & 0x80808080u) | (r[d] & 0x7f7f7f7fu);
             idx4 = d == 0 ? pair : (pair & 0xc0c0c0c0u) | ((idx4 >> 2) & 0x3f3f3f3fu);
         }
@@ -1597,37 +1564,38 @@ __device__ __forceinline__ uint32_t PairTreeIndexes(const uint8_t* laneTile, con
 }
 
 template <int MAXD, bool SIX>
-__global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousPairTileKernel(
+__global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     const uint16_t* __restrict__ bins, size_t docCount, uint32_t bucketCount, const uint32_t* __restrict__ tileMap,
     uint32_t rowCount, const uint4* __restrict__ pairRows, const double2* __restrict__ leaves2,
     const double* __restrict__ bias, double scale, uint32_t treeBegin, uint32_t treeEnd, double* __restrict__ out) {
     constexpr uint32_t kLeaves = 1u << MAXD;
-    constexpr int kLeafRegs = MAXD == 8 ? 4 : 1;  // 16-byte pieces of a pair's 2 * kLeaves leaf values per lane
+    constexpr int kLeafRegs = MAXD == 8 ? 4 : 1;       // 16-byte pieces of a pair's 2 * kLeaves leaf values per lane
+    constexpr int kPublishRegs = MAXD == 8 ? 2 : 1;    // pieces that go to LDS at a time: one tree's, or both trees'
+    constexpr uint32_t kRegion = MAXD == 8 ? kLeaves : 2 * kLeaves;  // doubles of a wave's region
     static_assert(MAXD == 8 || MAXD == 6, "64 or 256 leaves per tree");
-    // s_waitcnt that lets the loads of two pairs (two 16-byte pieces of a row and kLeafRegs of leaf values each)
-    // stay in flight: vmcnt in bits 0-3 and 14-15, the other counters untouched
-    // (of the pair behind the oldest, its row has to be there as well: its levels are read a round early)
-    constexpr int kLoadsBehind = kLeafRegs + (2 + kLeafRegs);
-    constexpr int kWaitForOldestPair = (kLoadsBehind & 0xf) | ((kLoadsBehind >> 4) << 14) | 0x0f70;
-    // s_waitcnt for the level reads of this round: the previous round's gathers and this round's stores were issued
-    // behind them (LDS serves a wave's requests in order); vmcnt and expcnt untouched
-    constexpr int kWaitForLevelReads = 0xc07f | ((4 + kLeafRegs) << 8);
-    constexpr int kWaitForGathers = 0xc07f | ((kLeafRegs + MAXD) << 8);
+    // s_waitcnt for the level reads and, issued before them, the last round's gathers: only the stores behind them
+    // stay under way (lgkmcnt in bits 8-11; vmcnt and expcnt untouched)
+    constexpr int kWaitForLevelReads = 0xc07f | (kPublishRegs << 8);
     extern __shared__ uint32_t sTile[];
     uint16_t* sTile16 = reinterpret_cast<uint16_t*>(sTile);
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (kWave - 1);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const size_t block = blockIdx.x >> 1;
-    const uint32_t half = blockIdx.x & 1;
+    // sixteen workgroups take eight blocks, one per XCD, their first halves before their second ones; the blocks of a
+    // last group that is not full come half by half
+    const uint32_t turn = blockIdx.x / (2 * kXcdCount), inTurn = blockIdx.x % (2 * kXcdCount);
+    const bool wholeTurn = gridDim.x - turn * (2 * kXcdCount) >= 2 * kXcdCount;
+    const size_t block = turn * kXcdCount + (wholeTurn ? inTurn % kXcdCount : inTurn >> 1);
+    const uint32_t half = wholeTurn ? inTurn / kXcdCount : inTurn & 1;
     const uint32_t tileWords = rowCount * kWave;  // rowCount = bucketCount without a map
     const uint16_t* src = bins + block * (bucketCount * kWave) * 2 + half;
     if (tileMap == nullptr) {
-        for (uint32_t i = tid; i < tileWords; i += 64 * kTileWaves) {
+#pragma unroll 16
+        for (uint32_t i = tid; i < tileWords; i += 64 * kPairWaves) {
             sTile16[i] = src[2 * i];
         }
     } else {
-        for (uint32_t row = wave; row < rowCount; row += kTileWaves) {
+        for (uint32_t row = wave; row < rowCount; row += kPairWaves) {
             const uint32_t entry = tileMap[row];
             const uint32_t bins2 = src[2 * ((entry & 0xffffu) * kWave + lane)];
             sTile16[row * kWave + lane] = static_cast<uint16_t>(MapTileBins(bins2, entry >> 16));
@@ -1636,14 +1604,15 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousPairTileKernel(
     const uint32_t group = lane >> 5;
     const uint32_t tileBytes = (tileWords * 2 + 15) & ~15u;
     double* leafArea = reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(sTile) + tileBytes);
-    double2* sLeafWave2 = reinterpret_cast<double2*>(leafArea + wave * 2 * kLeaves);
-    const double* sLeafMine = leafArea + wave * 2 * kLeaves + group * kLeaves;
+    double* sLeafWave = leafArea + wave * kRegion;
+    double2* sLeafWave2 = reinterpret_cast<double2*>(sLeafWave) + lane;
+    const double* sLeafSecond = sLeafWave + (MAXD == 8 ? 0 : kLeaves);  // where the second tree's values are published
     const uint32_t laneOffset = (lane & 31) * 4;
     __syncthreads();  // tile is loaded
 
     const uint32_t treeCount = treeEnd - treeBegin;
     const uint32_t pairCount = treeCount / 2;
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    double acc[2] = {0.0, 0.0};
     constexpr int kAhead = kPairAhead;
     uint4 rows[kAhead][2];
     double2 pref[kAhead][kLeafRegs];
@@ -1657,7 +1626,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousPairTileKernel(
         _Pragma("unroll") for (int i = 0; i < 2; ++i) {                                            \
             rows[k][i] = row[i];                                                                   \
         }                                                                                          \
-        /* the row first: the round before the pair's own waits for it alone */                   \
+        /* the row first: its levels are read before the leaf values go to LDS */                 \
         __builtin_amdgcn_sched_barrier(0);                                                         \
         const double2* values = myLeaves + static_cast<size_t>(first) * (kLeaves / 2);             \
         _Pragma("unroll") for (int i = 0; i < kLeafRegs; ++i) {                                    \
@@ -1665,69 +1634,64 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousPairTileKernel(
         }                                                                                          \
         __builtin_amdgcn_sched_barrier(0);                                                         \
     } while (0)
-    // the pair's leaf values into the wave's LDS region (the previous pair's gathers were issued before these
-    // stores and LDS serves one wave's requests in order), then the levels: four leaf indexes per lane
-#define CBAMD_PUBLISH_AND_WALK(k, idx4)                                                            \
+    // pieces of the pair's leaf values into the wave's LDS region: gathers of what it held were issued before these
+    // stores, and LDS serves one wave's requests in order
+#define CBAMD_PUBLISH(k, begin)                                                                    \
     do {                                                                                           \
-        _Pragma("unroll") for (int i = 0; i < kLeafRegs; ++i) {                                    \
-            sLeafWave2[i * kWave + lane] = pref[k][i];                                             \
+        __builtin_amdgcn_wave_barrier();                                                           \
+        _Pragma("unroll") for (int i = 0; i < kPublishRegs; ++i) {                                 \
+            sLeafWave2[i * kWave] = pref[k][(begin) + i];                                          \
         }                                                                                          \
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");                                     \
         __builtin_amdgcn_wave_barrier();                                                           \
+    } while (0)
+    // The indexes of the pair, four documents of its group's tree per lane, then two documents of either tree:
+    // first and second tree's in the low sixteen bits of idxA and idxB.
+#define CBAMD_WALK(k, levelBins, idxA, idxB)                                                       \
+    do {                                                                                           \
         const uint32_t flags =                                                                     \
             __builtin_amdgcn_readlane(rows[k][0].x, 0) | __builtin_amdgcn_readlane(rows[k][0].x, 32); \
+        uint32_t idx4;                                                                             \
         if (flags & kPairRowXorFlag) {                                                             \
-            idx4 = PackedPairTreeIndexes<true, MAXD, SIX>(laneOffset, rows[k]);                    \
+            idx4 = WalkPackedPairLevels<true, MAXD, SIX>(levelBins, rows[k]);                      \
         } else {                                                                                   \
-            idx4 = PackedPairTreeIndexes<false, MAXD, SIX>(laneOffset, rows[k]);                   \
+            idx4 = WalkPackedPairLevels<false, MAXD, SIX>(levelBins, rows[k]);                     \
         }                                                                                          \
+        const auto swapped = __builtin_amdgcn_permlane32_swap(idx4, idx4 >> 16, false, false);     \
+        idxA = swapped[0];                                                                         \
+        idxB = swapped[1];                                                                         \
     } while (0)
+#define CBAMD_LEAF(idx, j) (((idx) >> (8 * (j) + 8 - MAXD)) & (kLeaves - 1))
 
-    // One round of a wave: the leaf values that the previous round gathered are added while this round's LDS
-    // reads are under way; the registers of this pair take the pair kAhead rounds ahead as soon as every level
-    // has read them (the loads then land in those registers), and the gathers go out last.
-    double gathered[4] = {0.0, 0.0, 0.0, 0.0};
-    uint32_t levelBins[kAhead][MAXD];  // what the reads of a pair's levels returned, issued a round before their use
+    // One round of a wave: the leaf values that the previous round gathered are added once this round's level reads,
+    // issued behind them, have returned; the gathers go out last, and the registers of this pair take the pair kAhead
+    // rounds ahead.
+    double gathered[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
 #define CBAMD_PAIR_ROUND(k)                                                                        \
     do {                                                                                           \
-        constexpr int kn = (k + 1) % kAhead;                                                       \
-        uint32_t idx4;                                                                             \
-        /* one wait for this pair's loads and the next pair's row: the later loads stay in flight */ \
-        __builtin_amdgcn_s_waitcnt(kWaitForOldestPair);                                            \
+        uint32_t levelBins[MAXD], idxA, idxB;                                                      \
+        ReadPackedPairLevels<MAXD>(laneOffset, rows[k], levelBins);                                \
         __builtin_amdgcn_sched_barrier(0);                                                         \
-        _Pragma("unroll") for (int i = 0; i < kLeafRegs; ++i) {                                    \
-            sLeafWave2[i * kWave + lane] = pref[k][i];                                             \
-        }                                                                                          \
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");                                     \
-        __builtin_amdgcn_wave_barrier();                                                           \
+        CBAMD_PUBLISH(k, 0);                                                                       \
         __builtin_amdgcn_sched_barrier(0);                                                         \
         __builtin_amdgcn_s_waitcnt(kWaitForLevelReads);                                            \
         __builtin_amdgcn_sched_barrier(0);                                                         \
-        /* the next pair's levels are read while this pair's are worked on */                     \
-        ReadPackedPairLevels<MAXD>(laneOffset, rows[kn], levelBins[kn]);                           \
-        __builtin_amdgcn_sched_barrier(0);                                                         \
-        const uint32_t flags =                                                                     \
-            __builtin_amdgcn_readlane(rows[k][0].x, 0) | __builtin_amdgcn_readlane(rows[k][0].x, 32); \
-        if (flags & kPairRowXorFlag) {                                                             \
-            idx4 = WalkPackedPairLevels<true, MAXD, SIX>(levelBins[k], rows[k]);                   \
-        } else {                                                                                   \
-            idx4 = WalkPackedPairLevels<false, MAXD, SIX>(levelBins[k], rows[k]);                  \
+        _Pragma("unroll") for (int j = 0; j < 2; ++j) {                                            \
+            acc[j] = __dadd_rn(__dadd_rn(acc[j], gathered[0][j]), gathered[1][j]);                 \
         }                                                                                          \
-        /* the previous round's gathers: this round's stores and reads were issued behind them */ \
-        __builtin_amdgcn_sched_barrier(0);                                                         \
-        __builtin_amdgcn_s_waitcnt(kWaitForGathers);                                               \
-        __builtin_amdgcn_sched_barrier(0);                                                         \
-        _Pragma("unroll") for (int q = 0; q < 4; ++q) {                                            \
-            acc[q] = __dadd_rn(acc[q], gathered[q]);                                               \
+        CBAMD_WALK(k, levelBins, idxA, idxB);                                                      \
+        _Pragma("unroll") for (int j = 0; j < 2; ++j) {                                            \
+            gathered[0][j] = sLeafWave[CBAMD_LEAF(idxA, j)];                                       \
+        }                                                                                          \
+        if constexpr (MAXD == 8) {                                                                 \
+            CBAMD_PUBLISH(k, kLeafRegs / 2);                                                       \
+        }                                                                                          \
+        _Pragma("unroll") for (int j = 0; j < 2; ++j) {                                            \
+            gathered[1][j] = sLeafSecond[CBAMD_LEAF(idxB, j)];                                     \
         }                                                                                          \
         __builtin_amdgcn_sched_barrier(0);                                                         \
-        CBAMD_FETCH_PAIR(k, treeBegin + 2 * (p + kAhead * kTileWaves));                            \
-        __builtin_amdgcn_sched_barrier(0);                                                         \
-        _Pragma("unroll") for (int q = 0; q < 4; ++q) {                                            \
-            gathered[q] = sLeafMine[(idx4 >> (8 * q + 8 - MAXD)) & (kLeaves - 1)];                 \
-        }                                                                                          \
-        __builtin_amdgcn_wave_barrier();                                                           \
-        p += kTileWaves;                                                                           \
+        CBAMD_FETCH_PAIR(k, treeBegin + 2 * (p + kAhead * kPairWaves));                            \
+        p += kPairWaves;                                                                           \
     } while (0)
 
     uint32_t p = wave;
@@ -1738,21 +1702,12 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousPairTileKernel(
         for (int i = 0; i < kLeafRegs; ++i) {
             pref[k][i] = {0.0, 0.0};
         }
-        CBAMD_FETCH_PAIR(k, treeBegin + 2 * (p + k * kTileWaves));
+        CBAMD_FETCH_PAIR(k, treeBegin + 2 * (p + k * kPairWaves));
     }
     static_assert(kAhead == 3, "the rounds below are written out for three register sets");
-#pragma unroll
-    for (int k = 1; k < kAhead; ++k) {
-#pragma unroll
-        for (int d = 0; d < MAXD; ++d) {
-            levelBins[k][d] = 0;
-        }
-    }
-    ReadPackedPairLevels<MAXD>(laneOffset, rows[0], levelBins[0]);  // the first pair's levels
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // (so that the rounds' waits need not cover this way into the loop)
     // whole turns of the three register sets without a branch between the rounds, so that the waits for
     // the loads count only the loads that are older than the one needed
-    while (p + 2 * kTileWaves < pairCount) {
+    while (p + 2 * kPairWaves < pairCount) {
         CBAMD_PAIR_ROUND(0);
         CBAMD_PAIR_ROUND(1);
         CBAMD_PAIR_ROUND(2);
@@ -1764,11 +1719,11 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousPairTileKernel(
         }
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        acc[q] = __dadd_rn(acc[q], gathered[q]);
+    for (int j = 0; j < 2; ++j) {
+        acc[j] = __dadd_rn(__dadd_rn(acc[j], gathered[0][j]), gathered[1][j]);
     }
     if ((treeCount & 1) && wave == 0) {
-        // the last tree has no partner: both groups walk it (its row and its leaf values twice), the first adds
+        // the last tree has no partner: both groups walk it (its row and its leaf values, twice with 64 leaves)
         const uint4* row = pairRows + static_cast<size_t>(treeEnd - 1) * 2;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -1776,35 +1731,36 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousPairTileKernel(
         }
         const double2* values = leaves2 + static_cast<size_t>(treeEnd - 1) * (kLeaves / 2);
 #pragma unroll
-        for (int i = 0; i < kLeafRegs; ++i) {
+        for (int i = 0; i < kPublishRegs; ++i) {
             pref[0][i] = values[(i * kWave + lane) & (kLeaves / 2 - 1)];
         }
-        uint32_t idx4;
-        CBAMD_PUBLISH_AND_WALK(0, idx4);
+        uint32_t levelBins[MAXD], idxA, idxB;
+        ReadPackedPairLevels<MAXD>(laneOffset, rows[0], levelBins);
+        CBAMD_PUBLISH(0, 0);
+        CBAMD_WALK(0, levelBins, idxA, idxB);
+        static_cast<void>(idxB);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const double v = sLeafMine[(idx4 >> (8 * q + 8 - MAXD)) & (kLeaves - 1)];
-            acc[q] = __dadd_rn(acc[q], group == 0 ? v : 0.0);
+        for (int j = 0; j < 2; ++j) {
+            acc[j] = __dadd_rn(acc[j], sLeafWave[CBAMD_LEAF(idxA, j)]);
         }
-        __builtin_amdgcn_wave_barrier();
     }
 #undef CBAMD_PAIR_ROUND
 #undef CBAMD_FETCH_PAIR
-#undef CBAMD_PUBLISH_AND_WALK
+#undef CBAMD_PUBLISH
+#undef CBAMD_WALK
+#undef CBAMD_LEAF
     __syncthreads();  // every wave is through with its leaf region: the area now takes the partial sums
-    // partial sums as [wave][group][document of the tile], then one thread per document adds the sixteen
+    // partial sums as [wave][document of the tile], then one thread per document adds the sixteen
     double* sRed = leafArea;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        // byte q of a lane's dword: document (q & 1) * 64 + 2 * (lane & 31) + (q >> 1) of the tile
-        const uint32_t docInTile = (q & 1) * kWave + 2 * (lane & 31) + (q >> 1);
-        sRed[(wave * 2 + group) * 128 + docInTile] = acc[q];
+    for (int j = 0; j < 2; ++j) {
+        sRed[wave * 128 + j * kWave + 2 * (lane & 31) + group] = acc[j];
     }
     __syncthreads();
     if (tid < 128) {
         double sum = sRed[tid];
 #pragma unroll
-        for (int part = 1; part < 2 * kTileWaves; ++part) {
+        for (int part = 1; part < kPairWaves; ++part) {
             sum = __dadd_rn(sum, sRed[part * 128 + tid]);
         }
         const size_t doc = block * kDocsPerBlock + (2 * half + (tid >> 6)) * kWave + (tid & 63);
@@ -1823,6 +1779,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousPairTileKernel(
 // grid = 4 * doc blocks, block = 64 * WAVES threads, dynamic LDS = rows * 64 (rounded up to 16) +
 // WAVES * 4 * (1 << MAXD) * 8 bytes (the leaf regions, later the partial sums).
 constexpr int kQuadTreePadding = 4 * kTileWaves * kPairAhead;
+static_assert(kPairTreePadding <= kQuadTreePadding, "the tables of the two kernels are padded alike");
 
 template <int MAXD, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void EvalObliviousQuadTileKernel(
