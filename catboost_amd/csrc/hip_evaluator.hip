@@ -1297,9 +1297,9 @@ struct THipEvaluator::TImpl {
     TDeviceVec<uint32_t> PackedTrees;  // tile kernel: 16 dwords per oblivious tree of depth <= 8
     TDeviceVec<uint32_t> PackedMixed;  // half-tile kernel: packed rows in the form chosen per tree
     TDeviceVec<double> HalfTileLeaves; // half-tile kernel: 64 or 256 leaf values per tree at a fixed pitch
-    TDeviceVec<uint32_t> PairRows;     // pair-tile kernel: 8 dwords per tree, empty when the model does not qualify
+    TDeviceVec<uint32_t> PairRows;     // pair-tile kernel: 32 dwords per tree, empty when the model does not qualify
     bool PairSix = false;              // ... in the six-bit form (every bin below 64)
-    TDeviceVec<uint32_t> QuadRows;     // quad-tile kernel: the same with 64 bytes per row of the tile
+    TDeviceVec<uint32_t> QuadRows;     // quad-tile kernel: 16 dwords per tree, 64 bytes per row of the tile
     TDeviceVec<uint32_t> TileRows;     // row-tile kernel (whole tile, one tree per wave): the same with 256 bytes per bucket
     TDeviceVec<double> TileLeaves;     // its leaf values: [slice of the dimensions][tree][pair of dimensions][leaf][2]
     size_t TileSliceStride = 0;        // 16-byte pairs of TileLeaves per slice
@@ -1889,17 +1889,14 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         return rows;
     };
 
-    // The pair-tile kernel's rows: 8 dwords per tree, a level's row offset (128-byte rows), xor byte (bits 0-6) and
-    // the byte added to the bins (bits 24-31) in one dword
-    const auto packedPairRows = [&](bool six) {
-        constexpr uint32_t kDwords = 8;
-        std::vector<uint32_t> rows((trees.GetTreeCount() + dev::kQuadTreePadding) * kDwords, 0);
+    // The pair-tile kernel's rows: sixteen entries of two dwords per tree, entry d a level's row offset (128-byte rows)
+    // and its xor byte four times, entry 8 + d the value added to the four bins of a dword
+    const auto pairTileRows = [&](bool six) {
+        std::vector<uint32_t> rows((trees.GetTreeCount() + dev::kPairTreePadding) * dev::kPairRowDwords, 0);
         for (size_t t = 0; t < trees.GetTreeCount(); ++t) {
-            uint32_t* row = rows.data() + t * kDwords;
-            bool anyXor = false;
+            uint32_t* row = rows.data() + t * dev::kPairRowDwords;
             for (int d = 0; d < trees.TreeSizes[t]; ++d) {
                 const TTileLevel level = tileLevelOf(trees.RepackedBins[trees.TreeStartOffsets[t] + d]);
-                CBAMD_ENSURE(level.Row < 1024 && level.Xor < 128 && (level.Add & 0xffu) <= 128, "level does not fit the packed row");
                 uint32_t xorByte = level.Xor, addByte = level.Add & 0xffu;
                 if (six && d % 2 == 0) {
                     // the six-bit form of an even level: its result goes to bit 6 of the byte
@@ -1910,11 +1907,9 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                         addByte -= 64;
                     }
                 }
-                row[d] = level.Row * 128u | xorByte | addByte << 24;
-                anyXor = anyXor || level.IsXor;
-            }
-            if (anyXor) {
-                row[0] |= dev::kPairRowXorFlag;
+                row[2 * d] = level.Row * 128u;
+                row[2 * d + 1] = xorByte * 0x01010101u;
+                row[2 * (8 + d)] = addByte * 0x01010101u;
             }
         }
         return rows;
@@ -2015,7 +2010,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     if (pairFits) {
                         // every bin below 64: the walk joins two levels at a time
                         m.PairSix = m.MaxBucketValues <= 63 && !tileRowsSplit && switches.RegSix;
-                        m.PairRows.Upload(packedPairRows(m.PairSix));
+                        m.PairRows.Upload(pairTileRows(m.PairSix));
                     } else {
                         m.QuadRows.Upload(rowsInRegisters(64));
                     }
@@ -3091,7 +3086,7 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
                 EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds);
                 hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(2 * blocks)), dim3(64 * dev::kPairWaves), lds, s,
                                    reinterpret_cast<const uint16_t*>(bins), docCount, m.LayoutBuckets, m.TileMap.Get(),
-                                   m.TileRowCount, reinterpret_cast<const uint4*>(m.PairRows.Get()),
+                                   m.TileRowCount, reinterpret_cast<const uint2*>(m.PairRows.Get()),
                                    reinterpret_cast<const double2*>(m.HalfTileLeaves.Get()), m.Bias.Get(), m.Scale, tb, te,
                                    results);
             };

@@ -1431,19 +1431,22 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousHalfTileKernel(
 // and one byte-parallel compare for 2 x 128 (tree, document) pairs instead of 128. Needs every bin of the
 // tile below 128 (the 7-bit compare; a one-hot level xors first: (bin ^ (~value & 0x7f)) + 1 carries into
 // bit 7 exactly when bin == value).
-// `pairRows` holds 8 dwords per tree, one per level: byte offset of the level's bucket in the tile (bucket * 128,
-// bits 7-16) | xor byte (bits 0-6) | the value added to each of the four bins << 24, slot 0 also bit 23 when some
-// level of the tree xors (WalkPackedPairLevels). Levels past the tree's depth are zero (bucket 0, add 0: never
-// true). A lane keeps its tree's row in registers (two 16-byte loads, the same addresses for the 32 lanes of a
-// group; with offsets and values to add as a dword each the row took four, and the kernel, which is bound by the
-// bytes its lanes receive over the vector memory path, 49 ms instead of 41 on 10M documents x 5000 trees) and the wave
+// `pairRows` holds sixteen 8-byte entries per tree, one per lane of a row of sixteen lanes: entry d < 8 the byte offset
+// of level d's bucket in the tile (bucket * 128) and the xor byte four times, entry 8 + d the value added to each of the
+// four bins (the byte four times) and 0. Levels past the tree's depth are zero (bucket 0, add 0: never true). A lane
+// holds one entry of its group's tree, and the levels take their operands from the row's lanes by DPP (row_newbcast),
+// which costs no instruction of its own: 512 bytes per pair over the vector memory path, where a packed row in every
+// lane took 2 KB beside the 4 KB of leaf values, and an instruction per level fewer than unpacking it (two on a one-hot level). The wave
 // publishes the trees' leaf values (1 << MAXD doubles per tree, a pair's side by side in `leaves`) in its own LDS
 // region, one tree after the other: before the gathers the two groups swap half of their indexes, so that every lane
 // has two documents of either tree (documents j * 64 + 2 * m + group, j = 0, 1), gathers them from the first tree's
 // values, and the second tree's then go to the same place (LDS serves a wave's requests in order). With 2 KB per wave
 // instead of a pair's 4 KB sixteen waves find room beside the widest tile instead of eight. That is what the kernel
 // lacked: a wave issues an instruction about every nine cycles, and two waves per SIMD left half of the SIMD's issue
-// cycles empty (PAIR_NUMBERS).
+// cycles empty. 10M documents * 5000 trees of depth 8 over 1016 buckets, whole call with 10.3 ms of binarize: 57.1 ms with
+// eight waves, 51.1 with sixteen, 49.4 with the rows by DPP. What is left per pair and CU, of 123 cycles: vector issue
+// 82, LDS about 78 (32 of them the values going in, 30 the gathers), vector memory 72 (the values' 4 KB at 64 bytes a
+// cycle): 128 documents share a copy of 256 values, and no wider tile fits.
 // Waves take the pairs round robin; a last tree without a partner is done by wave 0 with both groups on the same tree
 // and its values added once. Partial sums (one per wave) are added in a fixed order at the end. The fetches run
 // kPairAhead rounds ahead of the walk without looking at the tree range: both tables end with kPairTreePadding trees'
@@ -1453,7 +1456,8 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousHalfTileKernel(
 // XCD that start one after the other (workgroups go round-robin to the XCDs).
 // grid = 2 * doc blocks, block = 64 * kPairWaves threads, dynamic LDS = rows * 128 (rounded up to 16) +
 // kPairWaves * max(1 << MAXD, 128) * 8 bytes (the leaf regions, later the partial sums).
-constexpr uint32_t kPairRowXorFlag = 1u << 23;  // slot 0 of a tree's row: some level xors
+constexpr uint32_t kPairRowXorFlag = 1u << 23;  // slot 0 of a tree's row in registers: some level xors
+constexpr int kPairRowDwords = 32;
 constexpr int kPairWaves = 16;
 constexpr int kPairAhead = 3;
 constexpr int kPairTreePadding = 2 * kPairWaves * kPairAhead;
@@ -1482,38 +1486,48 @@ __device__ __forceinline__ uint32_t MapTileBins(uint32_t bins4, uint32_t mode) {
     return bins4;
 }
 
-// The same walk on a tree's row in its packed form, one dword per level: bits 7-16 the byte offset of the level's
-// row in a tile of 128-byte rows, bits 0-6 the xor byte, bits 24-31 the value added to each of the four bins (bit
-// 23 of slot 0: some level of the tree xors). laneOffset is the lane's offset inside a row; the tile starts at LDS
-// address 0 (the kernel has no other LDS). A pair of trees then costs a lane two 16-byte loads instead of four:
-// the pair-tile kernel is bound by the bytes that the vector memory path delivers to its lanes.
+// The value that lane N of each row of sixteen lanes holds, in every lane of the row.
+template <int N>
+__device__ __forceinline__ uint32_t FromRowLane(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x150 + N, 0xf, 0xf, true));
+}
+
+// The walk of the pair-tile kernel, in two halves: the LDS reads of a tree's levels (laneOffset is the lane's offset
+// inside a row of the tile, which starts at LDS address 0: the kernel has no other LDS), and the leaf indexes of four
+// documents, one per byte, from what they returned. `row` is the lane's entry of pairRows.
 // SIX: every bin of the tile is below 64. The even levels then carry the byte (64 - split), so that their result
 // lands in bit 6 while the following level's lands in bit 7, and a pair of levels joins the index with one shift
-// and two bit-field inserts: eighteen instructions for eight levels where the one-level-at-a-time form takes
-// twenty-four (a one-hot level on an even position xors with the low six bits of its mask).
-// In two halves: the LDS reads of a tree's levels, and the walk on what they returned.
-template <int MAXD>
-__device__ __forceinline__ void ReadPackedPairLevels(uint32_t laneOffset, const uint4 (&desc)[2], uint32_t (&a)[MAXD]) {
-    const uint32_t levels[8] = {desc[0].x, desc[0].y, desc[0].z, desc[0].w, desc[1].x, desc[1].y, desc[1].z, desc[1].w};
-#pragma unroll
-    for (int d = 0; d < MAXD; ++d) {
-        a[d] = *reinterpret_cast<const __attribute__((address_space(3))) uint32_t*>((levels[d] & 0x1ff80u) | laneOffset);
+// and two bit-field inserts (a one-hot level on an even position xors with the low six bits of its mask).
+template <int MAXD, int D = 0>
+__device__ __forceinline__ void ReadPairLevels(uint32_t laneOffset, uint32_t row, uint32_t (&a)[MAXD]) {
+    if constexpr (D < MAXD) {
+        a[D] = *reinterpret_cast<const __attribute__((address_space(3))) uint32_t*>(FromRowLane<D>(row) + laneOffset);
+        ReadPairLevels<MAXD, D + 1>(laneOffset, row, a);
     }
 }
 
-template <bool XOR, int MAXD, bool SIX>
-__device__ __forceinline__ uint32_t WalkPackedPairLevels(const uint32_t (&a)[MAXD], const uint4 (&desc)[2]) {
-    const uint32_t levels[8] = {desc[0].x, desc[0].y, desc[0].z, desc[0].w, desc[1].x, desc[1].y, desc[1].z, desc[1].w};
-    uint32_t r[MAXD];
-#pragma unroll
-    for (int d = 0; d < MAXD; ++d) {
-        uint32_t v = a[d];
-        if (XOR) {
-            const uint32_t x = levels[d] & 0x7fu;
-            v ^= __builtin_amdgcn_perm(x, x, 0u);  // the xor byte four times
-        }
-        r[d] = v + __builtin_amdgcn_perm(levels[d], levels[d], 0x03030303u);  // byte 3 four times
+template <int MAXD, int D = 0>
+__device__ __forceinline__ void XorPairLevels(uint32_t xors, uint32_t (&a)[MAXD]) {
+    if constexpr (D < MAXD) {
+        a[D] ^= FromRowLane<D>(xors);
+        XorPairLevels<MAXD, D + 1>(xors, a);
     }
+}
+
+template <int MAXD, int D = 0>
+__device__ __forceinline__ void AddPairLevels(uint32_t adds, uint32_t (&a)[MAXD]) {
+    if constexpr (D < MAXD) {
+        a[D] += FromRowLane<8 + D>(adds);
+        AddPairLevels<MAXD, D + 1>(adds, a);
+    }
+}
+
+template <int MAXD, bool SIX>
+__device__ __forceinline__ uint32_t WalkPairLevels(uint2 row, uint32_t (&r)[MAXD]) {
+    if (__any(row.y != 0)) {
+        XorPairLevels<MAXD>(row.y, r);
+    }
+    AddPairLevels<MAXD>(row.x, r);
     uint32_t idx4 = 0;
     if constexpr (SIX) {
         static_assert(MAXD % 2 == 0, "levels in pairs");
@@ -1566,7 +1580,7 @@ __device__ __forceinline__ uint32_t PairTreeIndexes(const uint8_t* laneTile, con
 template <int MAXD, bool SIX>
 __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     const uint16_t* __restrict__ bins, size_t docCount, uint32_t bucketCount, const uint32_t* __restrict__ tileMap,
-    uint32_t rowCount, const uint4* __restrict__ pairRows, const double2* __restrict__ leaves2,
+    uint32_t rowCount, const uint2* __restrict__ pairRows, const double2* __restrict__ leaves2,
     const double* __restrict__ bias, double scale, uint32_t treeBegin, uint32_t treeEnd, double* __restrict__ out) {
     constexpr uint32_t kLeaves = 1u << MAXD;
     constexpr int kLeafRegs = MAXD == 8 ? 4 : 1;       // 16-byte pieces of a pair's 2 * kLeaves leaf values per lane
@@ -1604,9 +1618,9 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     const uint32_t group = lane >> 5;
     const uint32_t tileBytes = (tileWords * 2 + 15) & ~15u;
     double* leafArea = reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(sTile) + tileBytes);
-    double* sLeafWave = leafArea + wave * kRegion;
-    double2* sLeafWave2 = reinterpret_cast<double2*>(sLeafWave) + lane;
-    const double* sLeafSecond = sLeafWave + (MAXD == 8 ? 0 : kLeaves);  // where the second tree's values are published
+    double2* sLeafWave2 = reinterpret_cast<double2*>(leafArea + wave * kRegion) + lane;
+    // LDS addresses of the first and the second tree's values
+    const uint32_t leafFirst = tileBytes + wave * kRegion * 8, leafSecond = leafFirst + (MAXD == 8 ? 0 : kLeaves * 8);
     const uint32_t laneOffset = (lane & 31) * 4;
     __syncthreads();  // tile is loaded
 
@@ -1614,18 +1628,15 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     const uint32_t pairCount = treeCount / 2;
     double acc[2] = {0.0, 0.0};
     constexpr int kAhead = kPairAhead;
-    uint4 rows[kAhead][2];
+    uint2 rows[kAhead];
     double2 pref[kAhead][kLeafRegs];
-    // what a lane fetches of the pair that starts at tree `first`: its group's row and its pieces of the
-    // two trees' leaf values
-    const uint4* myRows = pairRows + group * 2;
+    // what a lane fetches of the pair that starts at tree `first`: its entry of its group's row and its pieces of
+    // the two trees' leaf values
+    const uint2* myRows = pairRows + group * 16 + (lane & 15);
     const double2* myLeaves = leaves2 + lane;
 #define CBAMD_FETCH_PAIR(k, first)                                                                 \
     do {                                                                                           \
-        const uint4* row = myRows + static_cast<size_t>(first) * 2;                                \
-        _Pragma("unroll") for (int i = 0; i < 2; ++i) {                                            \
-            rows[k][i] = row[i];                                                                   \
-        }                                                                                          \
+        rows[k] = myRows[static_cast<size_t>(first) * 16];                                         \
         /* the row first: its levels are read before the leaf values go to LDS */                 \
         __builtin_amdgcn_sched_barrier(0);                                                         \
         const double2* values = myLeaves + static_cast<size_t>(first) * (kLeaves / 2);             \
@@ -1649,19 +1660,19 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     // first and second tree's in the low sixteen bits of idxA and idxB.
 #define CBAMD_WALK(k, levelBins, idxA, idxB)                                                       \
     do {                                                                                           \
-        const uint32_t flags =                                                                     \
-            __builtin_amdgcn_readlane(rows[k][0].x, 0) | __builtin_amdgcn_readlane(rows[k][0].x, 32); \
-        uint32_t idx4;                                                                             \
-        if (flags & kPairRowXorFlag) {                                                             \
-            idx4 = WalkPackedPairLevels<true, MAXD, SIX>(levelBins, rows[k]);                      \
-        } else {                                                                                   \
-            idx4 = WalkPackedPairLevels<false, MAXD, SIX>(levelBins, rows[k]);                     \
+        uint32_t idx4 = WalkPairLevels<MAXD, SIX>(rows[k], levelBins);                             \
+        if constexpr (MAXD == 6) {                                                                 \
+            idx4 &= 0xfcfcfcfcu;                                                                   \
         }                                                                                          \
         const auto swapped = __builtin_amdgcn_permlane32_swap(idx4, idx4 >> 16, false, false);     \
         idxA = swapped[0];                                                                         \
         idxB = swapped[1];                                                                         \
     } while (0)
-#define CBAMD_LEAF(idx, j) (((idx) >> (8 * (j) + 8 - MAXD)) & (kLeaves - 1))
+    // the leaf value that byte j of idx names: eight times its index (two times the byte with 64 leaves, whose index is
+    // in the upper six bits) and the values' address in one instruction
+#define CBAMD_LEAF(base, idx, j)                                                                   \
+    (*reinterpret_cast<const __attribute__((address_space(3))) double*>(                           \
+        __builtin_amdgcn_udot4(idx, (MAXD == 8 ? 8u : 2u) << (8 * (j)), base, false)))
 
     // One round of a wave: the leaf values that the previous round gathered are added once this round's level reads,
     // issued behind them, have returned; the gathers go out last, and the registers of this pair take the pair kAhead
@@ -1670,7 +1681,7 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
 #define CBAMD_PAIR_ROUND(k)                                                                        \
     do {                                                                                           \
         uint32_t levelBins[MAXD], idxA, idxB;                                                      \
-        ReadPackedPairLevels<MAXD>(laneOffset, rows[k], levelBins);                                \
+        ReadPairLevels<MAXD>(laneOffset, rows[k].x, levelBins);                                    \
         __builtin_amdgcn_sched_barrier(0);                                                         \
         CBAMD_PUBLISH(k, 0);                                                                       \
         __builtin_amdgcn_sched_barrier(0);                                                         \
@@ -1681,13 +1692,13 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
         }                                                                                          \
         CBAMD_WALK(k, levelBins, idxA, idxB);                                                      \
         _Pragma("unroll") for (int j = 0; j < 2; ++j) {                                            \
-            gathered[0][j] = sLeafWave[CBAMD_LEAF(idxA, j)];                                       \
+            gathered[0][j] = CBAMD_LEAF(leafFirst, idxA, j);                                       \
         }                                                                                          \
         if constexpr (MAXD == 8) {                                                                 \
             CBAMD_PUBLISH(k, kLeafRegs / 2);                                                       \
         }                                                                                          \
         _Pragma("unroll") for (int j = 0; j < 2; ++j) {                                            \
-            gathered[1][j] = sLeafSecond[CBAMD_LEAF(idxB, j)];                                     \
+            gathered[1][j] = CBAMD_LEAF(leafSecond, idxB, j);                                      \
         }                                                                                          \
         __builtin_amdgcn_sched_barrier(0);                                                         \
         CBAMD_FETCH_PAIR(k, treeBegin + 2 * (p + kAhead * kPairWaves));                            \
@@ -1724,24 +1735,20 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     }
     if ((treeCount & 1) && wave == 0) {
         // the last tree has no partner: both groups walk it (its row and its leaf values, twice with 64 leaves)
-        const uint4* row = pairRows + static_cast<size_t>(treeEnd - 1) * 2;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            rows[0][i] = row[i];
-        }
+        rows[0] = pairRows[static_cast<size_t>(treeEnd - 1) * 16 + (lane & 15)];
         const double2* values = leaves2 + static_cast<size_t>(treeEnd - 1) * (kLeaves / 2);
 #pragma unroll
         for (int i = 0; i < kPublishRegs; ++i) {
             pref[0][i] = values[(i * kWave + lane) & (kLeaves / 2 - 1)];
         }
         uint32_t levelBins[MAXD], idxA, idxB;
-        ReadPackedPairLevels<MAXD>(laneOffset, rows[0], levelBins);
+        ReadPairLevels<MAXD>(laneOffset, rows[0].x, levelBins);
         CBAMD_PUBLISH(0, 0);
         CBAMD_WALK(0, levelBins, idxA, idxB);
         static_cast<void>(idxB);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            acc[j] = __dadd_rn(acc[j], sLeafWave[CBAMD_LEAF(idxA, j)]);
+            acc[j] = __dadd_rn(acc[j], CBAMD_LEAF(leafFirst, idxA, j));
         }
     }
 #undef CBAMD_PAIR_ROUND
@@ -1772,8 +1779,9 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
 
 // The same with four trees per wave on a quarter of a block, for models whose rows do not fit the half tile: the
 // tile holds the bins of 64 documents (documents quarter * 64 + l of the block in byte l of a row), lanes 16 g ..
-// 16 g + 15 walk tree g of a quad of trees, each lane for the four documents of one dword. The rows are pairRows
-// with 64 bytes per row of the tile; rows and leaf values are fetched three rounds ahead, so both tables end with
+// 16 g + 15 walk tree g of a quad of trees, each lane for the four documents of one dword. The rows are
+// sixteen dwords per tree in every lane of its group: slot d the byte offset of level d's bucket (bucket * 64) | xor byte
+// << 24, slot 8 + d the value added to the bins, slot 0 also kPairRowXorFlag. Rows and leaf values are fetched three rounds ahead, so both tables end with
 // kQuadTreePadding null trees.
 // WAVES = 8, or 4 when the rows leave LDS for four waves' regions only.
 // grid = 4 * doc blocks, block = 64 * WAVES threads, dynamic LDS = rows * 64 (rounded up to 16) +
@@ -1961,7 +1969,7 @@ __global__ __launch_bounds__(64 * WAVES) void EvalObliviousQuadTileKernel(
 }
 
 // Models of 7-bit bins whose 256-document tile fits LDS, one tree per wave: the walk of
-// EvalObliviousPairTileKernel on the whole tile. A tree's row is `tileRows` (the format of pairRows with
+// EvalObliviousPairTileKernel on the whole tile. A tree's row is `tileRows` (the quad-tile kernel's format with
 // bucket * 256 as the byte offset); its address is the same in every lane, so it comes through scalar loads
 // and a level is an LDS read and three vector instructions with no lane reads and no scalar arithmetic. The
 // leaf values go through the wave's LDS region; rows and values are fetched kPairAhead rounds ahead without

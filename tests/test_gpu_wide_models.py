@@ -316,3 +316,26 @@ def test_one_hot_bucket_of_more_than_127_values_on_the_tile_kernels(seed, n_floa
         np.testing.assert_allclose(g.calc_flat(x, tree_start=begin, tree_end=end),
                                    o.calc(x, tree_start=begin, tree_end=end), rtol=RTOL, atol=ATOL,
                                    err_msg="trees %d..%d" % (begin, end))
+
+
+@pytest.mark.parametrize("max_depth,n_cat", [(8, 0), (8, 9), (6, 9)])
+def test_pair_tile_kernel_at_the_ends_of_its_turns(max_depth, n_cat):
+    """Documents in 7 to 9 and 17 blocks (halves of eight blocks are dealt out over the dies, those of a last group of
+    fewer blocks one by one) and tree ranges around its sixteen waves' rounds of one to three pairs."""
+    rng = np.random.default_rng(81)
+    model, cat_values = _random_oblivious(rng, n_float=900, n_cat=n_cat, trees=500, max_depth=max_depth)
+    o = OracleModel(model)
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    x = _random_flat_data(rng, model, cat_values, 17 * 256)
+    assert g.evaluator().describe_kernels(cb.LAYOUT_FLAT_ROWS, len(x))["evaluate"] == "EvalObliviousPairTileKernel"
+    want = o.calc(x)
+    for docs in (1, 7 * 256 - 1, 7 * 256, 8 * 256, 8 * 256 + 1, 17 * 256):
+        # the sums differ by their order alone: 500 values of about one, 1e-16 each
+        np.testing.assert_allclose(g.calc_flat(x[:docs]), want[:docs], rtol=RTOL, atol=ATOL, err_msg="%d documents" % docs)
+    few = x[:300]
+    for begin, length in ((0, 31), (1, 32), (2, 33), (0, 65), (3, 95), (0, 96), (5, 97), (404, 96), (403, 97)):
+        np.testing.assert_allclose(g.calc_flat(few, tree_start=begin, tree_end=begin + length),
+                                   o.calc(few, tree_start=begin, tree_end=begin + length), rtol=RTOL, atol=ATOL,
+                                   err_msg="trees %d..%d" % (begin, begin + length))
