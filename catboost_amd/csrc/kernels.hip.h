@@ -1444,9 +1444,11 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalObliviousHalfTileKernel(
 // instead of a pair's 4 KB sixteen waves find room beside the widest tile instead of eight. That is what the kernel
 // lacked: a wave issues an instruction about every nine cycles, and two waves per SIMD left half of the SIMD's issue
 // cycles empty. 10M documents * 5000 trees of depth 8 over 1016 buckets, whole call with 10.3 ms of binarize: 57.1 ms with
-// eight waves, 51.1 with sixteen, 49.4 with the rows by DPP. What is left per pair and CU, of 123 cycles: vector issue
-// 82, LDS about 78 (32 of them the values going in, 30 the gathers), vector memory 72 (the values' 4 KB at 64 bytes a
-// cycle): 128 documents share a copy of 256 values, and no wider tile fits.
+// eight waves, 51.1 with sixteen, 49.4 with the rows by DPP, 46.9 with the tile in 16-byte pieces. What is left per pair
+// and CU, of 115 cycles: vector issue 82, LDS about 78 (32 of them the values going in, 30 the gathers), vector memory 72
+// (the values' 4 KB at 64 bytes a cycle): 128 documents share a copy of 256 values, and no wider tile fits.
+// The tile of a workgroup that has its CU to itself arrives while nothing else runs there: it is read in 16-byte pieces,
+// eight per thread in flight (two bytes a load from bins that do not start at such an address, or through `tileMap`).
 // Waves take the pairs round robin; a last tree without a partner is done by wave 0 with both groups on the same tree
 // and its values added once. Partial sums (one per wave) are added in a fixed order at the end. The fetches run
 // kPairAhead rounds ahead of the walk without looking at the tree range: both tables end with kPairTreePadding trees'
@@ -1603,18 +1605,6 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     const uint32_t half = wholeTurn ? inTurn / kXcdCount : inTurn & 1;
     const uint32_t tileWords = rowCount * kWave;  // rowCount = bucketCount without a map
     const uint16_t* src = bins + block * (bucketCount * kWave) * 2 + half;
-    if (tileMap == nullptr) {
-#pragma unroll 16
-        for (uint32_t i = tid; i < tileWords; i += 64 * kPairWaves) {
-            sTile16[i] = src[2 * i];
-        }
-    } else {
-        for (uint32_t row = wave; row < rowCount; row += kPairWaves) {
-            const uint32_t entry = tileMap[row];
-            const uint32_t bins2 = src[2 * ((entry & 0xffffu) * kWave + lane)];
-            sTile16[row * kWave + lane] = static_cast<uint16_t>(MapTileBins(bins2, entry >> 16));
-        }
-    }
     const uint32_t group = lane >> 5;
     const uint32_t tileBytes = (tileWords * 2 + 15) & ~15u;
     double* leafArea = reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(sTile) + tileBytes);
@@ -1622,8 +1612,6 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     // LDS addresses of the first and the second tree's values
     const uint32_t leafFirst = tileBytes + wave * kRegion * 8, leafSecond = leafFirst + (MAXD == 8 ? 0 : kLeaves * 8);
     const uint32_t laneOffset = (lane & 31) * 4;
-    __syncthreads();  // tile is loaded
-
     const uint32_t treeCount = treeEnd - treeBegin;
     const uint32_t pairCount = treeCount / 2;
     double acc[2] = {0.0, 0.0};
@@ -1645,6 +1633,38 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
         }                                                                                          \
         __builtin_amdgcn_sched_barrier(0);                                                         \
     } while (0)
+    uint32_t p = wave;
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+        // (written before the loads so that the arrays stay in registers)
+#pragma unroll
+        for (int i = 0; i < kLeafRegs; ++i) {
+            pref[k][i] = {0.0, 0.0};
+        }
+        CBAMD_FETCH_PAIR(k, treeBegin + 2 * (p + k * kPairWaves));
+    }
+    // the tile, behind the requests for the first pairs
+    if (tileMap == nullptr && (reinterpret_cast<uintptr_t>(bins) & 15) == 0) {
+        const uint4* src4 = reinterpret_cast<const uint4*>(src - half);
+        const uint32_t select = half ? 0x07060302u : 0x05040100u;  // the upper or the lower halves of two dwords
+#pragma unroll 8
+        for (uint32_t i = tid; i < tileWords / 4; i += 64 * kPairWaves) {
+            const uint4 v = src4[i];
+            reinterpret_cast<uint2*>(sTile)[i] = make_uint2(__builtin_amdgcn_perm(v.y, v.x, select), __builtin_amdgcn_perm(v.w, v.z, select));
+        }
+    } else if (tileMap == nullptr) {
+        for (uint32_t i = tid; i < tileWords; i += 64 * kPairWaves) {
+            sTile16[i] = src[2 * i];
+        }
+    } else {
+        for (uint32_t row = wave; row < rowCount; row += kPairWaves) {
+            const uint32_t entry = tileMap[row];
+            const uint32_t bins2 = src[2 * ((entry & 0xffffu) * kWave + lane)];
+            sTile16[row * kWave + lane] = static_cast<uint16_t>(MapTileBins(bins2, entry >> 16));
+        }
+    }
+    __syncthreads();  // tile is loaded
+
     // pieces of the pair's leaf values into the wave's LDS region: gathers of what it held were issued before these
     // stores, and LDS serves one wave's requests in order
 #define CBAMD_PUBLISH(k, begin)                                                                    \
@@ -1705,16 +1725,6 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
         p += kPairWaves;                                                                           \
     } while (0)
 
-    uint32_t p = wave;
-#pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-        // (written before the loads so that the arrays stay in registers)
-#pragma unroll
-        for (int i = 0; i < kLeafRegs; ++i) {
-            pref[k][i] = {0.0, 0.0};
-        }
-        CBAMD_FETCH_PAIR(k, treeBegin + 2 * (p + k * kPairWaves));
-    }
     static_assert(kAhead == 3, "the rounds below are written out for three register sets");
     // whole turns of the three register sets without a branch between the rounds, so that the waits for
     // the loads count only the loads that are older than the one needed
