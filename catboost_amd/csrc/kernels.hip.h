@@ -584,6 +584,46 @@ __device__ __forceinline__ double Finish(double sum, double scale, double bias, 
     return r;
 }
 
+// Copies of a document block's bins into LDS by a workgroup of THREADS threads. A workgroup of the tile kernels has its
+// CU to itself or shares it with one other, so nothing else hides the loads: eight of them per thread are issued before
+// the first is stored, where a plain loop waits for every one. 4M documents * 500 non-symmetric trees over 300 features
+// 7.01 -> 6.50 ms, 970 640 documents * 2934 trees of depth 6 over 614 features (EvalObliviousRowTileKernel) 2.87 -> 2.59.
+template <int THREADS, typename T, typename TStore>
+__device__ __forceinline__ void CopyInBatches(const T* __restrict__ src, uint32_t count, uint32_t tid, const TStore& store) {
+    constexpr int kBatch = 8;
+    for (uint32_t first = tid; first < count; first += kBatch * THREADS) {
+        T v[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            v[j] = src[min(first + j * THREADS, count - 1)];  // past the end: the last piece again, not stored
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            if (first + j * THREADS < count) {
+                store(first + j * THREADS, v[j]);
+            }
+        }
+    }
+}
+
+// All `rows` of a block (256 bytes each), row r to the 64 dwords from tile + 64 * place(r) on; in pieces of 16 bytes
+// unless the bins start at an address that does not allow it (a caller's buffer).
+template <int THREADS, typename TPlace>
+__device__ __forceinline__ void CopyTile(const uint32_t* src, uint32_t rows, uint32_t tid, uint32_t* tile, const TPlace& place) {
+    if ((reinterpret_cast<uintptr_t>(src) & 15) == 0) {
+        CopyInBatches<THREADS>(reinterpret_cast<const uint4*>(src), rows * (kWave / 4), tid, [&](uint32_t i, const uint4& v) {
+            reinterpret_cast<uint4*>(tile)[place(i / (kWave / 4)) * (kWave / 4) + i % (kWave / 4)] = v;
+        });
+    } else {
+        CopyInBatches<THREADS>(src, rows * kWave, tid, [&](uint32_t i, uint32_t v) { tile[place(i / kWave) * kWave + i % kWave] = v; });
+    }
+}
+
+template <int THREADS>
+__device__ __forceinline__ void CopyTile(const uint32_t* src, uint32_t rows, uint32_t tid, uint32_t* tile) {
+    CopyTile<THREADS>(src, rows, tid, tile, [](uint32_t row) { return row; });
+}
+
 // Oblivious trees, any model: one wave per 256-document block, four documents per lane, leaf
 // sums kept in registers in fp64 and accumulated in tree order (as the CPU evaluator does).
 // DCHUNK output dimensions are accumulated per pass over the trees.
@@ -1133,9 +1173,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 4
     const size_t block = blockIdx.x;
     const uint32_t tileDwords = bucketCount * kWave;
     const uint32_t* src = bins + block * tileDwords;
-    for (uint32_t i = tid; i < tileDwords; i += 64 * WAVES) {
-        sTile[i] = src[i];
-    }
+    CopyTile<64 * WAVES>(src, bucketCount, tid, sTile);
     const bool addBias = treeBegin == 0;
     const uint8_t* laneTile = reinterpret_cast<const uint8_t*>(sTile) + lane * 4;
     const uint32_t slot = lane & (kPackedTreeDwords - 1);
@@ -1488,6 +1526,31 @@ __device__ __forceinline__ uint32_t MapTileBins(uint32_t bins4, uint32_t mode) {
     return bins4;
 }
 
+// The rows of a tile with `tileMap` (MapTileBins), a wave per row, eight rows of a wave in flight; load(i) and
+// store(row, bins) take the dword (or the half of it) that is the lane's.
+template <int WAVES, typename TLoad, typename TStore>
+__device__ __forceinline__ void CopyMappedRows(const uint32_t* __restrict__ tileMap, uint32_t rowCount, uint32_t wave,
+                                               const TLoad& load, const TStore& store) {
+    constexpr int kBatch = 8;
+    for (uint32_t first = wave; first < rowCount; first += kBatch * WAVES) {
+        uint32_t entry[kBatch], bins4[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            entry[j] = tileMap[min(first + j * WAVES, rowCount - 1)];  // past the end: the last row again, not stored
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            bins4[j] = load(entry[j] & 0xffffu);
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            if (first + j * WAVES < rowCount) {
+                store(first + j * WAVES, MapTileBins(bins4[j], entry[j] >> 16));
+            }
+        }
+    }
+}
+
 // The value that lane N of each row of sixteen lanes holds, in every lane of the row.
 template <int N>
 __device__ __forceinline__ uint32_t FromRowLane(uint32_t v) {
@@ -1647,21 +1710,17 @@ __global__ __launch_bounds__(64 * kPairWaves) void EvalObliviousPairTileKernel(
     if (tileMap == nullptr && (reinterpret_cast<uintptr_t>(bins) & 15) == 0) {
         const uint4* src4 = reinterpret_cast<const uint4*>(src - half);
         const uint32_t select = half ? 0x07060302u : 0x05040100u;  // the upper or the lower halves of two dwords
-#pragma unroll 8
-        for (uint32_t i = tid; i < tileWords / 4; i += 64 * kPairWaves) {
-            const uint4 v = src4[i];
+        CopyInBatches<64 * kPairWaves>(src4, tileWords / 4, tid, [&](uint32_t i, const uint4& v) {
             reinterpret_cast<uint2*>(sTile)[i] = make_uint2(__builtin_amdgcn_perm(v.y, v.x, select), __builtin_amdgcn_perm(v.w, v.z, select));
-        }
+        });
     } else if (tileMap == nullptr) {
         for (uint32_t i = tid; i < tileWords; i += 64 * kPairWaves) {
             sTile16[i] = src[2 * i];
         }
     } else {
-        for (uint32_t row = wave; row < rowCount; row += kPairWaves) {
-            const uint32_t entry = tileMap[row];
-            const uint32_t bins2 = src[2 * ((entry & 0xffffu) * kWave + lane)];
-            sTile16[row * kWave + lane] = static_cast<uint16_t>(MapTileBins(bins2, entry >> 16));
-        }
+        CopyMappedRows<kPairWaves>(
+            tileMap, rowCount, wave, [&](uint32_t bucket) { return uint32_t(src[2 * (bucket * kWave + lane)]); },
+            [&](uint32_t row, uint32_t bins2) { sTile16[row * kWave + lane] = static_cast<uint16_t>(bins2); });
     }
     __syncthreads();  // tile is loaded
 
@@ -2020,14 +2079,11 @@ __global__ __launch_bounds__(64 * WAVES) void EvalObliviousRowTileKernel(
     const uint32_t tileDwords = rowCount * kWave;  // rowCount = bucketCount without a map
     const uint32_t* src = bins + block * (bucketCount * kWave);
     if (tileMap == nullptr) {
-        for (uint32_t i = tid; i < tileDwords; i += 64 * WAVES) {
-            sTile[i] = src[i];
-        }
+        CopyTile<64 * WAVES>(src, rowCount, tid, sTile);
     } else {
-        for (uint32_t row = wave; row < rowCount; row += WAVES) {
-            const uint32_t entry = tileMap[row];
-            sTile[row * kWave + lane] = MapTileBins(src[(entry & 0xffffu) * kWave + lane], entry >> 16);
-        }
+        CopyMappedRows<WAVES>(
+            tileMap, rowCount, wave, [&](uint32_t bucket) { return src[bucket * kWave + lane]; },
+            [&](uint32_t row, uint32_t bins4) { sTile[row * kWave + lane] = bins4; });
     }
     const uint32_t tileBytes = (tileDwords * 4 + 15) & ~15u;
     double* sRed = reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(sTile) + tileBytes);  // [DIMS][256 documents]
@@ -2214,14 +2270,11 @@ __global__ __launch_bounds__(64 * WAVES) void EvalObliviousDeepTileKernel(
     const uint32_t tileDwords = rowCount * kWave;  // rowCount = bucketCount without a map
     const uint32_t* src = bins + block * (bucketCount * kWave);
     if (tileMap == nullptr) {
-        for (uint32_t i = tid; i < tileDwords; i += 64 * WAVES) {
-            sTile[i] = src[i];
-        }
+        CopyTile<64 * WAVES>(src, rowCount, tid, sTile);
     } else {
-        for (uint32_t row = wave; row < rowCount; row += WAVES) {
-            const uint32_t entry = tileMap[row];
-            sTile[row * kWave + lane] = MapTileBins(src[(entry & 0xffffu) * kWave + lane], entry >> 16);
-        }
+        CopyMappedRows<WAVES>(
+            tileMap, rowCount, wave, [&](uint32_t bucket) { return src[bucket * kWave + lane]; },
+            [&](uint32_t row, uint32_t bins4) { sTile[row * kWave + lane] = bins4; });
     }
     const uint32_t tileBytes = (tileDwords * 4 + 15) & ~15u;
     double* sRed = reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(sTile) + tileBytes);  // [256 documents]
@@ -2329,14 +2382,11 @@ __global__ __launch_bounds__(64 * WAVES) void EvalObliviousDeepTilePairsKernel(
     const uint32_t tileDwords = rowCount * kWave;  // rowCount = bucketCount without a map
     const uint32_t* src = bins + block * (bucketCount * kWave);
     if (tileMap == nullptr) {
-        for (uint32_t i = tid; i < tileDwords; i += 64 * WAVES) {
-            sTile[i] = src[i];
-        }
+        CopyTile<64 * WAVES>(src, rowCount, tid, sTile);
     } else {
-        for (uint32_t row = wave; row < rowCount; row += WAVES) {
-            const uint32_t entry = tileMap[row];
-            sTile[row * kWave + lane] = MapTileBins(src[(entry & 0xffffu) * kWave + lane], entry >> 16);
-        }
+        CopyMappedRows<WAVES>(
+            tileMap, rowCount, wave, [&](uint32_t bucket) { return src[bucket * kWave + lane]; },
+            [&](uint32_t row, uint32_t bins4) { sTile[row * kWave + lane] = bins4; });
     }
     const uint32_t tileBytes = (tileDwords * 4 + 15) & ~15u;
     double* sRed = reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(sTile) + tileBytes);  // [DIMS][256 documents]
@@ -2531,9 +2581,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalNonSymmetricTileKernel(
     const size_t block = blockIdx.x;
     const uint32_t tileDwords = bucketCount * kWave;
     const uint32_t* src = bins + block * tileDwords;
-    for (uint32_t i = tid; i < tileDwords; i += 64 * kTileWaves) {
-        sTile[i] = src[i];
-    }
+    CopyTile<64 * kTileWaves>(src, bucketCount, tid, sTile);
     const bool addBias = treeBegin == 0;
     const uint8_t* laneTile = reinterpret_cast<const uint8_t*>(sTile) + lane * 4;
     double* sRed = reinterpret_cast<double*>(sTile + ((tileDwords + 1) & ~1u));
@@ -2728,15 +2776,10 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
     const size_t block = blockIdx.x;
     const uint32_t tileDwords = bucketCount * kWave;
     const uint32_t* src = bins + block * tileDwords;
-    for (uint32_t i = tid; i < tileDwords; i += 64 * WAVES) {
-        sTile[NsLdsTileRow(i / kWave, WAVES, ENTRIES) * kWave + (i & (kWave - 1))] = src[i];
-    }
     const uint32_t laneOff = lane * 4;
     double* sRed = reinterpret_cast<double*>(sTile + NsLdsTileRows(bucketCount, WAVES, ENTRIES) * kWave);
     uint32_t* sEntries = sTile + wave * kNsLdsEntries;  // 8 KB per wave, the first ENTRIES * 4 bytes of them
     const uint32_t bucketMask = 0x3ff00u;
-    __syncthreads();  // tile is loaded
-
     // A unit's entries come as whole rounds, whatever its size: a unit starts at a multiple of four entries and
     // the table ends with ENTRIES spare ones, so the copy needs neither a bound nor a branch (entries past the
     // unit's are never followed).
@@ -2758,6 +2801,17 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
             fetched[i] = fSource[i * kWave];                                                                \
         }                                                                                                   \
     } while (0)
+
+    uint32_t u = wave;
+    uint4 row = make_uint4(0, 0, 0, 0), row2 = make_uint4(0, 0, 0, 0);
+    if (u < unitCount) {
+        row = unitRows[2 * u];
+        row2 = unitRows[2 * u + 1];
+        CBAMD_FETCH_UNIT(row);
+    }
+    // the tile, behind the request for the first unit
+    CopyTile<64 * WAVES>(src, bucketCount, tid, sTile, [](uint32_t bucket) { return NsLdsTileRow(bucket, WAVES, ENTRIES); });
+    __syncthreads();  // tile is loaded
 
     double acc[4][DIMS];
 #pragma unroll
@@ -2784,13 +2838,6 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
     int lastSet = -1;  // the set whose values are not added yet
     const uint32_t d0 = blockIdx.y * DIMS;
     const double* sliceValues = valuesByEntry + static_cast<size_t>(blockIdx.y) * entryCount * DIMS;
-    uint32_t u = wave;
-    uint4 row = make_uint4(0, 0, 0, 0), row2 = make_uint4(0, 0, 0, 0);
-    if (u < unitCount) {
-        row = unitRows[2 * u];
-        row2 = unitRows[2 * u + 1];
-        CBAMD_FETCH_UNIT(row);
-    }
     const auto walkUnit = [&](double (&mineSet)[kNsUnitTrees][4], const double (&otherSet)[kNsUnitTrees][4]) {
         const uint32_t first = __builtin_amdgcn_readfirstlane(row.x);
         const uint32_t height = __builtin_amdgcn_readfirstlane(row.y);

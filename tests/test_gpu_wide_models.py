@@ -339,3 +339,35 @@ def test_pair_tile_kernel_at_the_ends_of_its_turns(max_depth, n_cat):
         np.testing.assert_allclose(g.calc_flat(few, tree_start=begin, tree_end=begin + length),
                                    o.calc(few, tree_start=begin, tree_end=begin + length), rtol=RTOL, atol=ATOL,
                                    err_msg="trees %d..%d" % (begin, begin + length))
+
+
+@pytest.mark.parametrize("config,trees,features,kernel", [
+    ("C4", 40, 90, "EvalNonSymmetricLdsKernel"),
+    ("C2", 150, 300, "EvalObliviousRowTileKernel"),
+    ("C2", 400, 900, "EvalObliviousPairTileKernel"),
+])
+def test_bins_at_an_address_that_is_no_multiple_of_sixteen(monkeypatch, config, trees, features, kernel):
+    """The tile kernels read bins in 16-byte pieces where their address allows it; a caller's buffer need not."""
+    import torch
+
+    from catboost_amd import synthetic as syn
+    monkeypatch.setitem(syn.CONFIGS, "narrowed", dict(syn.CONFIGS[config], floats=features))
+    model, info = syn.build_model("narrowed", trees=trees)
+    model.enable_gpu_evaluation(0)
+    ev = model.evaluator()
+    docs = 1301
+    assert kernel in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"]
+    x = syn.device_features(info, docs)
+    size = ev.quantized_bytes(docs)
+    bins = torch.zeros(size, dtype=torch.uint8, device="cuda:0")
+    shifted = torch.zeros(size + 16, dtype=torch.uint8, device="cuda:0")
+    out, out2 = (torch.zeros(docs, dtype=torch.float64, device="cuda:0") for _ in range(2))
+    torch.cuda.synchronize()
+    ev.quantize(ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), x.shape[1]), docs, bins.data_ptr())
+    ev.synchronize()
+    shifted[4:4 + size] = bins
+    torch.cuda.synchronize()
+    ev.eval_quantized(bins.data_ptr(), docs, out.data_ptr())
+    ev.eval_quantized(shifted.data_ptr() + 4, docs, out2.data_ptr())
+    ev.synchronize()
+    assert torch.equal(out, out2)
