@@ -126,14 +126,14 @@ private:
     // what every launch that reads features asks of its batch
     void CheckBatch(const TFeatureBatch& batch, size_t docCount) const;
     void SetLastTimes(const TKernelTimes& times);
-    // ... of a small-batch launch: its context, whose clock stamps are read when the times are asked for
-    void SetLastTimes(const void* smallContext);
+    // ... of a small-batch launch on a THostContext, whose clock stamps are read when the times are asked for
+    void SetLastSmallTimes(void* smallContext);
     std::unique_ptr<TImpl> Impl;
     size_t TreeCount = 0;
     int ApproxDimension = 1;
     uint32_t BucketCount = 0;
     TKernelTimes LastTimes;
-    const void* LastSmallContext = nullptr;  // a THostContext of Impl
+    const void* LastSmallStamps = nullptr;  // a TSmallStamps of one of Impl's contexts (they live as long as Impl)
     mutable std::mutex TimesLock;  // callers of one evaluator run side by side; the last one to finish leaves its times
 };
 

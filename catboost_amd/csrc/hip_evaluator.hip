@@ -1420,14 +1420,20 @@ struct THipEvaluator::TImpl {
         // binarize start, binarize end, evaluate end, results on the host
         hipEvent_t Ev[4] = {nullptr, nullptr, nullptr, nullptr};
     };
+    // Start and end of every workgroup of a small-batch launch. LastKernelTimes of one thread may read those of a call that
+    // has returned while another thread's call runs on the same context: the two never share a buffer.
+    struct TSmallStamps {
+        TDeviceVec<unsigned long long> Values;
+        size_t Count = 0;
+    };
     struct THostContext {
         hipStream_t Stream = nullptr;
         TDeviceVec<uint8_t> ScratchBins;
         TDeviceVec<double> SlicePartials;  // raw sums per slice of the trees (small batches)
         THostSlot Slots[2];
         hipEvent_t Ev[3] = {nullptr, nullptr, nullptr};
-        TDeviceVec<unsigned long long> Stamps;  // start and end of every workgroup of the last small-batch launch
-        size_t StampCount = 0;
+        TSmallStamps Stamps[2];  // the last small-batch launch's, and those that the next one writes
+        int NextStamps = 0;
         bool Busy = false;
 
         THostContext() {
@@ -3322,11 +3328,12 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
     const uint32_t dims = static_cast<uint32_t>(m.SmallDims());
     const uint32_t passes = m.SmallPasses();
     const auto launch = [&](auto kernel, size_t groups, uint32_t threads, size_t lds) {
-        ctx.Stamps.Reserve(2 * groups * passes);
-        ctx.StampCount = groups * passes;
+        THipEvaluator::TImpl::TSmallStamps& stamps = ctx.Stamps[ctx.NextStamps];
+        stamps.Values.Reserve(2 * groups * passes);
+        stamps.Count = groups * passes;
         EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds);
         hipExtLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups), passes), dim3(threads), lds, s, nullptr, stop, 0, src,
-                              static_cast<uint32_t>(docCount), tab, results, reinterpret_cast<ulonglong2*>(ctx.Stamps.Get()));
+                              static_cast<uint32_t>(docCount), tab, results, reinterpret_cast<ulonglong2*>(stamps.Values.Get()));
     };
     const auto launchFew = [&](auto kernel) {
         launch(kernel, docCount, std::min<uint32_t>(dev::kFewThreads, (tab.TreeCount + 63) / 64 * 64), m.FewLdsBytes(treeCount));
@@ -3559,7 +3566,7 @@ void THipEvaluator::CalcDevice(const TFeatureBatch& batch, size_t docCount, size
         CheckBatch(batch, docCount);
         LaunchSmallBatch(m, *ctx, batch, docCount, TreeCount, results, s, ctx->Ev[2]);
         HIP_CHECK(hipEventSynchronize(ctx->Ev[2]));
-        SetLastTimes(&*ctx);
+        SetLastSmallTimes(&*ctx);
         return;
     }
     TKernelTimes times;
@@ -3712,26 +3719,28 @@ void RunPipeline(size_t docCount, size_t chunk, hipEvent_t (&done)[2], const TSt
 void THipEvaluator::SetLastTimes(const TKernelTimes& times) {
     std::lock_guard<std::mutex> guard(TimesLock);
     LastTimes = times;
-    LastSmallContext = nullptr;
+    LastSmallStamps = nullptr;
 }
 
-void THipEvaluator::SetLastTimes(const void* smallContext) {
+void THipEvaluator::SetLastSmallTimes(void* smallContext) {
+    TImpl::THostContext& ctx = *static_cast<TImpl::THostContext*>(smallContext);
     std::lock_guard<std::mutex> guard(TimesLock);
-    LastSmallContext = smallContext;
+    LastSmallStamps = &ctx.Stamps[ctx.NextStamps];
+    ctx.NextStamps ^= 1;
 }
 
 TKernelTimes THipEvaluator::LastKernelTimes() const {
     std::lock_guard<std::mutex> guard(TimesLock);
-    if (LastSmallContext == nullptr) {
+    if (LastSmallStamps == nullptr) {
         return LastTimes;
     }
     // a small-batch launch left its workgroups' clock stamps on the device; they are fetched when somebody asks
-    const TImpl::THostContext& ctx = *static_cast<const TImpl::THostContext*>(LastSmallContext);
-    std::vector<unsigned long long> stamps(2 * ctx.StampCount);
+    const TImpl::TSmallStamps& last = *static_cast<const TImpl::TSmallStamps*>(LastSmallStamps);
+    std::vector<unsigned long long> stamps(2 * last.Count);
     int clockKhz = 0;
     HIP_CHECK(hipSetDevice(Impl->DeviceId));
     HIP_CHECK(hipDeviceGetAttribute(&clockKhz, hipDeviceAttributeWallClockRate, Impl->DeviceId));
-    HIP_CHECK(hipMemcpy(stamps.data(), ctx.Stamps.Get(), stamps.size() * sizeof(stamps[0]), hipMemcpyDeviceToHost));
+    HIP_CHECK(hipMemcpy(stamps.data(), last.Values.Get(), stamps.size() * sizeof(stamps[0]), hipMemcpyDeviceToHost));
     unsigned long long begin = ~0ull, end = 0;
     for (size_t i = 0; i + 1 < stamps.size(); i += 2) {
         begin = std::min(begin, stamps[i]);
@@ -3860,7 +3869,7 @@ void THipEvaluator::CalcHostRows(const float* const* rows, size_t rowLen, bool f
             batch.CatStride = needCats;
         }
         CalcSmallHostBatch(*this, m, *ctx, batch, docCount, predictionType, results);
-        SetLastTimes(&*ctx);
+        SetLastSmallTimes(&*ctx);
         return;
     }
     const size_t chunk = PipelineDocs((needFloats + needCats) * 4);
@@ -3921,7 +3930,7 @@ void THipEvaluator::CalcHostColumns(const float* const* columns, size_t columnCo
         batch.Floats = slot.PinnedFloats.Get();
         batch.Stride = docCount;
         CalcSmallHostBatch(*this, m, *ctx, batch, docCount, predictionType, results);
-        SetLastTimes(&*ctx);
+        SetLastSmallTimes(&*ctx);
         return;
     }
     const size_t chunk = PipelineDocs(need * 4);

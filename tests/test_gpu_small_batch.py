@@ -140,6 +140,44 @@ def test_small_kernels_against_the_oracle(seed, n_float, n_cat, trees, depth, di
         assert ev.last_kernel_times()[1] > 0.0
 
 
+def test_kernel_times_beside_running_small_batches():
+    """The last call's times are read from its launch's clock stamps while other threads' launches of growing size write
+    theirs: each reading is one launch's own."""
+    import threading
+
+    model, info = syn.build_model("C1", trees=150)
+    model.enable_gpu_evaluation(0)
+    ev = model.evaluator()
+    host = syn.device_features(info, 8000).cpu().numpy()
+    expected = model.calc_flat(host)
+    failures, running = [], threading.Event()
+    running.set()
+
+    def read_times():
+        try:
+            while running.is_set():
+                assert 0.0 < ev.last_kernel_times()[1] < 1000.0
+        except Exception as e:  # noqa: BLE001 (reported below)
+            failures.append(repr(e))
+
+    def call(offset):
+        try:
+            for docs in range(1 + offset, 8000, 601):
+                assert np.array_equal(model.calc_flat(host[:docs]), expected[:docs])
+        except Exception as e:  # noqa: BLE001
+            failures.append(repr(e))
+
+    reader = threading.Thread(target=read_times)
+    callers = [threading.Thread(target=call, args=(i,)) for i in range(3)]
+    for t in [reader] + callers:
+        t.start()
+    for t in callers:
+        t.join()
+    running.clear()
+    reader.join()
+    assert not failures, failures
+
+
 def test_a_documents_value_does_not_depend_on_the_small_kernel_that_took_it():
     """The slices of the trees and the order of their sums are those of the register kernels' small batches."""
     import torch
