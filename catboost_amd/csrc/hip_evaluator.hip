@@ -376,7 +376,7 @@ struct TKernelSwitches {
     bool PairTile = true;         // CATBOOST_AMD_PAIR_TILE=0: the half-tile kernel with one tree per wave
     bool RowTile = true;          // CATBOOST_AMD_ROW_TILE=0: the tile kernel that broadcasts a tree's levels from a lane
     bool RegSplit = true;         // CATBOOST_AMD_REG_SPLIT=0: buckets of more than 127 values send a model to the mixed kernels
-    uint32_t NsWaves = 0;         // CATBOOST_AMD_NS_WAVES=4|6|8|12|16: that shape of the non-symmetric LDS kernel or none
+    uint32_t NsWaves = 0;         // CATBOOST_AMD_NS_WAVES=4|6|8|10|11|12|16: shapes of the non-symmetric LDS kernel with so many waves or none
 
     static TKernelSwitches FromEnvironment() {
         const auto off = [](const char* name) {
@@ -501,12 +501,24 @@ uint32_t NsLdsDims(int dim) {
     return dim == 1 ? 1 : dim == 2 ? 2 : 4;
 }
 
+// Few buckets leave LDS for larger regions (fewer units, larger trees) at a given number of waves, and 249 to 312 buckets
+// for ten or eleven waves where trees of more than 1536 entries used to leave eight. Evaluate launch, 1M documents, trees
+// of depth 10: 500 trees over 100 features 1224 us with eight waves of 2048 entries, 1103 with twelve of 1536, 1061 with
+// twelve of 2048, 1025 with sixteen of 2048; 500 over 300 features 1285 with eight, 1207 with ten, 1199 with eleven of 1792,
+// 1150 to 1181 with twelve of 1536. The speeds of the larger regions lie below what they measured, as their units differ.
 struct TNsLdsShape {
     uint32_t Waves;
     uint32_t Entries;
     double Speed;  // steps of a unit per unit of time, relative to the 8-wave shape
 };
-constexpr TNsLdsShape kNsLdsShapes[] = {{16, 1024, 1.45}, {12, 1536, 1.26}, {8, 2048, 1.0}, {6, 2048, 0.8}, {4, 2048, 0.55}};
+constexpr TNsLdsShape kNsLdsShapes[] = {{16, 1024, 1.45}, {16, 1536, 1.37}, {16, 2048, 1.35}, {12, 1536, 1.26}, {12, 2048, 1.2},
+                                        {11, 1792, 1.08}, {10, 2048, 1.04}, {8, 2048, 1.0},   {6, 2048, 0.8},   {4, 2048, 0.55}};
+
+// Calls `tryShape` with the waves and the entries of one shape after another until it returns true.
+template <typename TTry, size_t... I>
+bool LaunchOfShape(const TTry& tryShape, std::index_sequence<I...>) {
+    return (tryShape(std::integral_constant<int, kNsLdsShapes[I].Waves>(), std::integral_constant<int, kNsLdsShapes[I].Entries>()) || ...);
+}
 
 // A unit of EvalNonSymmetricLdsKernel: up to three trees that a wave walks side by side out of its LDS region
 struct TNsUnit {
@@ -3135,31 +3147,22 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
                                m.NsUnitCount, m.NsValuesByEntry.Get(), m.Bias.Get(), m.Scale,
                                static_cast<uint32_t>(m.Dim), m.NsEntryCount, tb, te, results);
         };
-        const auto launchDims = [&](auto one, auto two, auto four) {
-            if (dims == 1) {
-                launch(one);
-            } else if (dims == 2) {
-                launch(two);
-            } else {
-                launch(four);
+        const auto tryShape = [&](auto waves, auto entries) {
+            constexpr int W = decltype(waves)::value, E = decltype(entries)::value;
+            if (m.NsLdsShape.Waves != W || m.NsLdsShape.Entries != E) {
+                return false;
             }
+            if (dims == 1) {
+                launch(dev::EvalNonSymmetricLdsKernel<W, E, 1>);
+            } else if (dims == 2) {
+                launch(dev::EvalNonSymmetricLdsKernel<W, E, 2>);
+            } else {
+                launch(dev::EvalNonSymmetricLdsKernel<W, E, 4>);
+            }
+            return true;
         };
-        if (m.NsLdsShape.Waves == 16) {
-            launchDims(dev::EvalNonSymmetricLdsKernel<16, 1024, 1>, dev::EvalNonSymmetricLdsKernel<16, 1024, 2>,
-                       dev::EvalNonSymmetricLdsKernel<16, 1024, 4>);
-        } else if (m.NsLdsShape.Waves == 12) {
-            launchDims(dev::EvalNonSymmetricLdsKernel<12, 1536, 1>, dev::EvalNonSymmetricLdsKernel<12, 1536, 2>,
-                       dev::EvalNonSymmetricLdsKernel<12, 1536, 4>);
-        } else if (m.NsLdsShape.Waves == 6) {
-            launchDims(dev::EvalNonSymmetricLdsKernel<6, 2048, 1>, dev::EvalNonSymmetricLdsKernel<6, 2048, 2>,
-                       dev::EvalNonSymmetricLdsKernel<6, 2048, 4>);
-        } else if (m.NsLdsShape.Waves == 4) {
-            launchDims(dev::EvalNonSymmetricLdsKernel<4, 2048, 1>, dev::EvalNonSymmetricLdsKernel<4, 2048, 2>,
-                       dev::EvalNonSymmetricLdsKernel<4, 2048, 4>);
-        } else {
-            launchDims(dev::EvalNonSymmetricLdsKernel<8, 2048, 1>, dev::EvalNonSymmetricLdsKernel<8, 2048, 2>,
-                       dev::EvalNonSymmetricLdsKernel<8, 2048, 4>);
-        }
+        const bool launched = LaunchOfShape(tryShape, std::make_index_sequence<std::size(kNsLdsShapes)>());
+        CBAMD_ENSURE(launched, "internal error: no kernel of this shape");
         HIP_CHECK(hipGetLastError());
         return;
     }

@@ -2716,7 +2716,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalNonSymmetricTileKernel(
 // the tile here and for the entries on the host.
 // The kernel is bound by the latency of this chain of LDS reads, so the workgroup has as many waves as LDS has
 // room for: WAVES regions of ENTRIES entries, ENTRIES at least the largest tree of the model
-// (16 x 1024, 12 x 1536 or 8 x 2048).
+// (kNsLdsShapes in hip_evaluator.hip; 16 x 1024 to 4 x 2048).
 // The two children of a node sit side by side at an even index (the root is entry 0, entry 1 is
 // unused), so one 8-byte LDS read, issued together with the read of the node's bin, brings both
 // and the compare only selects: one LDS round trip per level. A terminal entry points at its own

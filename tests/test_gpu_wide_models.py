@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import catboost_amd as cb
+from oracle.cbm_reader import read_cbm
 from oracle.oracle import OracleModel
 from tests.test_oracle import _random_flat_data, _random_oblivious
 
@@ -371,3 +372,26 @@ def test_bins_at_an_address_that_is_no_multiple_of_sixteen(monkeypatch, config, 
     ev.eval_quantized(shifted.data_ptr() + 4, docs, out2.data_ptr())
     ev.synchronize()
     assert torch.equal(out, out2)
+
+
+@pytest.mark.parametrize("waves,features,depth", [
+    (16, 120, 10), (16, 121, 9), (16, 248, 9), (12, 248, 10), (12, 249, 9), (11, 324, 9), (10, 312, 10), (10, 30, 10),
+])
+def test_shapes_of_the_non_symmetric_kernel_at_the_ends_of_their_buckets(monkeypatch, waves, features, depth):
+    """Regions of 1024 to 2048 entries for ten to sixteen waves, up to the last bucket that LDS has room for."""
+    import torch
+
+    from catboost_amd import synthetic as syn
+    monkeypatch.setenv("CATBOOST_AMD_NS_WAVES", str(waves))
+    monkeypatch.setitem(syn.CONFIGS, "narrowed", dict(syn.CONFIGS["C4"], floats=features, depth=depth))
+    model, info = syn.build_model("narrowed", trees=60)
+    model.enable_gpu_evaluation(0)
+    ev = model.evaluator()
+    docs = 1301
+    assert ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"].startswith("EvalNonSymmetricLdsKernel<%d, " % waves)
+    x = syn.device_features(info, docs)
+    out = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), x.shape[1]), docs, out.data_ptr())
+    expected = OracleModel(read_cbm(model.save_to_buffer())).calc(x.cpu().numpy())
+    np.testing.assert_allclose(out.cpu().numpy(), expected, rtol=RTOL, atol=ATOL)
