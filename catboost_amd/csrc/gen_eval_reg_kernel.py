@@ -394,7 +394,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             unit, j = seq[n]
             lo, scale, flags = rec_lo[n % 2], rec_scale[n % 2], rec_fo[n % 2]
             label = "%s_u%d_%d" % (name, unit, j)
-            e("  s_waitcnt lgkmcnt(0)")                # the unit's record
             # NaN counts as +inf in the columns whose flag says so
             e("  s_lshr_b32 s3, s%d, 16" % flags)
             e("  s_cmp_eq_u32 s3, 0")
@@ -517,6 +516,9 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                     wait_loads(pair[-1])
                 for n in pair:
                     unit, j = seq[n]
+                    # The unit's record, also that of a unit the model lacks: scalar loads return in any order, and the
+                    # record after next goes to the same registers.
+                    e("  s_waitcnt lgkmcnt(0)")
                     if unit > 0:
                         e("  s_cmp_le_u32 s28, %d" % unit)
                         e("  s_cbranch_scc1 %s_u%d_%d_skip" % (name, unit, j))

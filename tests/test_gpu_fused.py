@@ -213,3 +213,32 @@ def test_fused_split_rows_layout(monkeypatch):
     assert torch.equal(a, b)
     np.testing.assert_array_equal(a.cpu().numpy(), oracle.calc(x, layout="split", threads=8))
     np.testing.assert_array_equal(fm.calc_hashed(x, np.zeros((x.shape[0], 0), np.int32)), a.cpu().numpy())
+
+
+@pytest.mark.parametrize("columns,depth,shape", [(24, 8, 64), (24, 6, 64), (12, 7, 64), (150, 8, 208), (150, 6, 208), (130, 7, 208)])
+def test_fused_images_with_units_that_the_model_lacks(columns, depth, shape, monkeypatch):
+    """Six-bit models of one, two, nine and ten units of sixteen columns: the last image then holds two or three units in a
+    row that the model lacks. All documents of a batch that keeps every CU busy against the two launches, bit for bit."""
+    import torch
+
+    rng = np.random.default_rng(columns * 10 + depth)
+    width = max(columns, 16)
+    model = _random_model(rng, width, list(range(columns)), trees=60, depth=depth,
+                          borders_of=lambda f: rng.normal(0, 1, size=rng.integers(20, 60)))
+    (_, fev), (_, tev) = _evaluators(_bytes(model), monkeypatch)
+    docs = 1_000_003 if columns < 100 else 400_009
+    name = fev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs).get("fused", "")
+    assert name.startswith("cbamd_fused_b%d_w" % shape) and name.endswith("_s")
+    generator = torch.Generator(device="cuda:0")
+    generator.manual_seed(columns)
+    dx = torch.randn(docs, width, device="cuda:0", generator=generator)
+    a = torch.full((docs,), -1.0, dtype=torch.float64, device="cuda:0")
+    b = torch.full((docs,), -2.0, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    for _ in range(3):
+        fev.eval_data(fev.features(cb.LAYOUT_FLAT_ROWS, dx.data_ptr(), width), docs, a.data_ptr())
+        tev.eval_data(tev.features(cb.LAYOUT_FLAT_ROWS, dx.data_ptr(), width), docs, b.data_ptr())
+        assert fev.last_kernel_times()[0] == 0.0 and tev.last_kernel_times()[0] > 0.0
+        assert torch.equal(a, b)
+        a.fill_(-1.0)
+        torch.cuda.synchronize()

@@ -96,3 +96,83 @@ def test_staging_copies_stay_inside_the_tables(fused):
             if is_fused:
                 assert [b for b, _ in staged[:images]] == list(range(images)), (name, staged)
                 assert [buffer for _, buffer in staged[:images]] == [i % 2 for i in range(images)], (name, staged)
+
+
+def _registers(text):
+    """Scalar registers that an instruction's operands name."""
+    found = set()
+    for first, last in re.findall(r"\bs\[(\d+):(\d+)\]", text):
+        found.update(range(int(first), int(last) + 1))
+    found.update(int(r) for r in re.findall(r"\bs(\d+)\b", text))
+    return found
+
+
+def _scalar_load_faults(lines, units):
+    """Follows scalar loads, which return in any order, along every path of a kernel (of a fused kernel: every path of a
+    model of `units` units, whose number sits in s28 while the rows are binarized): instructions that name a register
+    which a load may still write, and loads into such a register."""
+    code, label_at = [], {}
+    for line in lines:
+        line = line.strip()
+        if line.startswith(".Lend"):
+            break
+        if line.endswith(":"):
+            label_at[line[:-1]] = len(code)
+        elif line and not line.startswith((".", ";", "#")):
+            code.append(line)
+    loop_at = next(at for label, at in label_at.items() if label.endswith("_loop"))
+    # the loop's loads into s3 only pull lines into the cache: nothing reads the register there or behind it
+    sink = re.compile(r"s_load_dword s3, ")
+    assert not any(3 in _registers(c) for c in code[loop_at:] if not sink.match(c))
+    unit_phase = [at for at, c in enumerate(code) if c == "s_mov_b32 s28, s89"]
+    state = {0: frozenset()}  # registers with a load in flight on arrival at an instruction
+    work, faults = [0], set()
+    while work:
+        at = work.pop()
+        c, flying = code[at], state[at]
+        op, _, operands = c.partition(" ")
+        after, targets = flying, [at + 1]
+        if op == "s_waitcnt":
+            after = frozenset() if "lgkmcnt(0)" in c else flying
+        elif op.startswith("s_load_"):
+            destination = _registers(operands.split(",")[0])
+            if _registers(operands) & flying:
+                faults.add((at, c))
+            after = flying if at >= loop_at and sink.match(c) else flying | destination
+        elif op == "s_branch":
+            targets = [label_at[operands]]
+        elif op.startswith("s_cbranch"):
+            targets.append(label_at[operands])
+            compared = re.match(r"s_cmp_le_u32 s28, (\d+)$", code[at - 1])
+            if units is not None and compared and unit_phase and at > unit_phase[0] and op == "s_cbranch_scc1":
+                targets = [targets[1] if units <= int(compared.group(1)) else targets[0]]
+        elif op == "s_endpgm":
+            targets = []
+        elif op.startswith(("s_", "v_", "ds_", "global_")):
+            if _registers(operands) & flying:
+                faults.add((at, c))
+        else:
+            raise AssertionError("unknown instruction: " + c)
+        for target in targets:
+            merged = after | state.get(target, frozenset())
+            if target not in state or merged != state[target]:
+                state[target] = merged
+                work.append(target)
+    return sorted(faults)
+
+
+def test_scalar_loads_in_flight_keep_their_registers():
+    """A record of a unit that the model lacks must have arrived before the record after next is requested into its
+    registers: images with two such units in a row (one or two units beyond a multiple of four in the six-bit form)
+    would otherwise binarize sixteen columns with whichever record came last."""
+    gen = _generator()
+    for variant in gen.VARIANTS:
+        text, _ = gen.gen_kernel(*variant)
+        assert not _scalar_load_faults(text.split("\n"), None), gen.kernel_name(*variant)
+    for buckets, waves in gen.FUSED_SHAPES:
+        for six in (False, True):
+            for levels in (None, 6):
+                text, _ = gen.gen_kernel(buckets, waves, 1, 256, False, six, fused=True, levels=levels)
+                name = gen.kernel_name(buckets, waves, 1, 256, False, six, True, levels)
+                for units in range(1, buckets // 16 + 1):
+                    assert not _scalar_load_faults(text.split("\n"), units), (name, units)
