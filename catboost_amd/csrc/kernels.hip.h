@@ -3102,11 +3102,7 @@ __global__ __launch_bounds__(kLeafIndexThreads) void LeafIndexesTileKernel(
     const int32_t lead = firstShare ? 0 : kLeafIndexLine;
     const uint32_t firstTree = treeBegin + (work % shares) * shareTrees - lead;
     const int32_t count = lastShare ? treeEnd - firstTree : shareTrees + lead;  // trees that are walked
-    const uint32_t tilePieces = bucketCount * (kWave / 4);
-    const uint4* src = reinterpret_cast<const uint4*>(bins) + static_cast<size_t>(block) * tilePieces;
-    for (uint32_t i = tid; i < tilePieces; i += kLeafIndexThreads) {
-        reinterpret_cast<uint4*>(sTile)[i] = src[i];
-    }
+    CopyTile<kLeafIndexThreads>(bins + static_cast<size_t>(block) * (bucketCount * kWave), bucketCount, tid, sTile);
     uint32_t* ring = sTile + bucketCount * kWave;
     const uint8_t* laneTile = reinterpret_cast<const uint8_t*>(sTile) + lane * 4;
     const size_t treeCount = treeEnd - treeBegin;

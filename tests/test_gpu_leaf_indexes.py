@@ -36,3 +36,29 @@ def test_leaf_indexes_at_the_edges_of_groups_shares_and_lines(cfg, trees, docs):
             got = out.cpu().numpy()
             np.testing.assert_array_equal(got[shift:shift + count].reshape(docs, end - begin), expected[:, begin:end])
             assert (got[:shift] == -7).all() and (got[shift + count:] == -7).all()
+
+
+@pytest.mark.parametrize("cfg", ["C1", "C2", "C2B"])
+def test_leaf_indexes_of_bins_at_an_address_that_is_no_multiple_of_sixteen(cfg):
+    """A caller's buffer of bins may start at any multiple of four."""
+    import torch
+
+    trees, docs = 130, 700
+    model, info = syn.build_model(cfg, trees=trees)
+    model.enable_gpu_evaluation(0)
+    ev = model.evaluator()
+    x = syn.device_features(info, docs)
+    expected = OracleModel(read_cbm(model.save_to_buffer())).leaf_indexes(x.cpu().numpy())
+    size = ev.quantized_bytes(docs)
+    bins = torch.zeros(size, dtype=torch.uint8, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.quantize(ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), x.shape[1]), docs, bins.data_ptr())
+    ev.synchronize()
+    for shift in (4, 8, 12):
+        moved = torch.full((size + 16,), 0xff, dtype=torch.uint8, device="cuda:0")
+        moved[shift:shift + size] = bins
+        out = torch.full((docs, trees), -7, dtype=torch.int32, device="cuda:0")
+        torch.cuda.synchronize()
+        ev.leaf_indexes_quantized(moved.data_ptr() + shift, docs, out.data_ptr(), 0, trees)
+        ev.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), expected)
