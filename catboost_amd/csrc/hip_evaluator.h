@@ -133,7 +133,6 @@ private:
     int ApproxDimension = 1;
     uint32_t BucketCount = 0;
     TKernelTimes LastTimes;
-    const void* LastSmallStamps = nullptr;  // a TSmallStamps of one of Impl's contexts (they live as long as Impl)
     mutable std::mutex TimesLock;  // callers of one evaluator run side by side; the last one to finish leaves its times
 };
 

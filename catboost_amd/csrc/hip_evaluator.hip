@@ -96,6 +96,34 @@ private:
     size_t Cap = 0;
 };
 
+// The calling thread's current device for as long as this lives; its own again afterwards.
+class TDeviceGuard {
+public:
+    explicit TDeviceGuard(int deviceId) {
+        HIP_CHECK(hipGetDevice(&Previous));
+        HIP_CHECK(hipSetDevice(deviceId));
+    }
+    ~TDeviceGuard() { (void)hipSetDevice(Previous); }
+    TDeviceGuard(const TDeviceGuard&) = delete;
+    TDeviceGuard& operator=(const TDeviceGuard&) = delete;
+
+private:
+    int Previous = 0;
+};
+
+// Calls that a capture elsewhere in the process would forbid (waits, copies) on streams of this file's own, which no
+// capture knows: this thread may make them for as long as this lives.
+class TCaptureGuard {
+public:
+    TCaptureGuard() { HIP_CHECK(hipThreadExchangeStreamCaptureMode(&Mode)); }
+    ~TCaptureGuard() { (void)hipThreadExchangeStreamCaptureMode(&Mode); }
+    TCaptureGuard(const TCaptureGuard&) = delete;
+    TCaptureGuard& operator=(const TCaptureGuard&) = delete;
+
+private:
+    hipStreamCaptureMode Mode = hipStreamCaptureModeRelaxed;
+};
+
 // A kernel that uses more than 64 KB of dynamic LDS has to be told so once (per device); the largest size asked
 // for so far is remembered, so that the attribute is not set again on every launch.
 // The code object of the assembly kernels, loaded once per device and kept for the life of the process: every
@@ -1432,8 +1460,10 @@ struct THipEvaluator::TImpl {
         // binarize start, binarize end, evaluate end, results on the host
         hipEvent_t Ev[4] = {nullptr, nullptr, nullptr, nullptr};
     };
-    // Start and end of every workgroup of a small-batch launch. LastKernelTimes of one thread may read those of a call that
-    // has returned while another thread's call runs on the same context: the two never share a buffer.
+    // Start and end of every workgroup of a small-batch launch. (In pinned memory, which the kernel would write over PCIe,
+    // they cost a call 0.2 to 0.6 us; an event in front of the launch cost 19 us.) LastKernelTimes of one thread may read
+    // those of a call that has returned while another thread's call runs on the same context: a launch takes a buffer that
+    // nobody else refers to.
     struct TSmallStamps {
         TDeviceVec<unsigned long long> Values;
         size_t Count = 0;
@@ -1444,9 +1474,24 @@ struct THipEvaluator::TImpl {
         TDeviceVec<double> SlicePartials;  // raw sums per slice of the trees (small batches)
         THostSlot Slots[2];
         hipEvent_t Ev[3] = {nullptr, nullptr, nullptr};
-        TSmallStamps Stamps[2];  // the last small-batch launch's, and those that the next one writes
-        int NextStamps = 0;
+        std::vector<std::shared_ptr<TSmallStamps>> Stamps;  // of this context's launches; at most one more than refer to them
+        std::shared_ptr<TSmallStamps> RunningStamps;        // those that the running launch writes
         bool Busy = false;
+
+        TSmallStamps& StampsForLaunch(size_t workgroups) {
+            RunningStamps.reset();
+            for (const auto& stamps : Stamps) {
+                if (stamps.use_count() == 1) {
+                    RunningStamps = stamps;
+                }
+            }
+            if (!RunningStamps) {
+                RunningStamps = Stamps.emplace_back(std::make_shared<TSmallStamps>());
+            }
+            RunningStamps->Values.Reserve(2 * workgroups);
+            RunningStamps->Count = workgroups;
+            return *RunningStamps;
+        }
 
         THostContext() {
             try {
@@ -1495,6 +1540,9 @@ struct THipEvaluator::TImpl {
     std::mutex ContextLock;
     std::condition_variable ContextFree;
     std::vector<std::unique_ptr<THostContext>> Contexts;
+    std::shared_ptr<const TSmallStamps> LastSmallStamps;  // the last call's if it was a small batch; under TimesLock
+    hipStream_t TimesStream = nullptr;                    // reads them
+    std::mutex TimesStreamLock;
 
     // A context of the pool for the time of one call.
     class TContextLease {
@@ -1584,8 +1632,10 @@ struct THipEvaluator::TImpl {
             (void)hipStreamSynchronize(Stream);
         }
         Contexts.clear();
-        if (Stream) {
-            (void)hipStreamDestroy(Stream);
+        for (hipStream_t s : {Stream, TimesStream}) {
+            if (s) {
+                (void)hipStreamDestroy(s);
+            }
         }
     }
 };
@@ -3331,9 +3381,7 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
     const uint32_t dims = static_cast<uint32_t>(m.SmallDims());
     const uint32_t passes = m.SmallPasses();
     const auto launch = [&](auto kernel, size_t groups, uint32_t threads, size_t lds) {
-        THipEvaluator::TImpl::TSmallStamps& stamps = ctx.Stamps[ctx.NextStamps];
-        stamps.Values.Reserve(2 * groups * passes);
-        stamps.Count = groups * passes;
+        const THipEvaluator::TImpl::TSmallStamps& stamps = ctx.StampsForLaunch(groups * passes);
         EnsureDynamicLds(reinterpret_cast<const void*>(kernel), lds);
         hipExtLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups), passes), dim3(threads), lds, s, nullptr, stop, 0, src,
                               static_cast<uint32_t>(docCount), tab, results, reinterpret_cast<ulonglong2*>(stamps.Values.Get()));
@@ -3722,28 +3770,40 @@ void RunPipeline(size_t docCount, size_t chunk, hipEvent_t (&done)[2], const TSt
 void THipEvaluator::SetLastTimes(const TKernelTimes& times) {
     std::lock_guard<std::mutex> guard(TimesLock);
     LastTimes = times;
-    LastSmallStamps = nullptr;
+    Impl->LastSmallStamps.reset();
 }
 
 void THipEvaluator::SetLastSmallTimes(void* smallContext) {
-    TImpl::THostContext& ctx = *static_cast<TImpl::THostContext*>(smallContext);
     std::lock_guard<std::mutex> guard(TimesLock);
-    LastSmallStamps = &ctx.Stamps[ctx.NextStamps];
-    ctx.NextStamps ^= 1;
+    Impl->LastSmallStamps = static_cast<TImpl::THostContext*>(smallContext)->RunningStamps;
 }
 
 TKernelTimes THipEvaluator::LastKernelTimes() const {
-    std::lock_guard<std::mutex> guard(TimesLock);
-    if (LastSmallStamps == nullptr) {
-        return LastTimes;
+    TImpl& m = *Impl;
+    std::shared_ptr<const TImpl::TSmallStamps> last;
+    {
+        std::lock_guard<std::mutex> guard(TimesLock);
+        if (!m.LastSmallStamps) {
+            return LastTimes;
+        }
+        last = m.LastSmallStamps;
     }
-    // a small-batch launch left its workgroups' clock stamps on the device; they are fetched when somebody asks
-    const TImpl::TSmallStamps& last = *static_cast<const TImpl::TSmallStamps*>(LastSmallStamps);
-    std::vector<unsigned long long> stamps(2 * last.Count);
+    // A small-batch launch left its workgroups' clock stamps on the device. They are fetched when somebody asks, on a stream
+    // that nothing else uses, while calls go on and publish theirs.
+    TDeviceGuard device(m.DeviceId);
+    TCaptureGuard capture;
+    std::vector<unsigned long long> stamps(2 * last->Count);
     int clockKhz = 0;
-    HIP_CHECK(hipSetDevice(Impl->DeviceId));
-    HIP_CHECK(hipDeviceGetAttribute(&clockKhz, hipDeviceAttributeWallClockRate, Impl->DeviceId));
-    HIP_CHECK(hipMemcpy(stamps.data(), last.Values.Get(), stamps.size() * sizeof(stamps[0]), hipMemcpyDeviceToHost));
+    HIP_CHECK(hipDeviceGetAttribute(&clockKhz, hipDeviceAttributeWallClockRate, m.DeviceId));
+    {
+        std::lock_guard<std::mutex> guard(m.TimesStreamLock);
+        if (m.TimesStream == nullptr) {
+            HIP_CHECK(hipStreamCreateWithFlags(&m.TimesStream, hipStreamNonBlocking));
+        }
+        HIP_CHECK(hipMemcpyAsync(stamps.data(), last->Values.Get(), stamps.size() * sizeof(stamps[0]), hipMemcpyDeviceToHost,
+                                 m.TimesStream));
+        HIP_CHECK(hipStreamSynchronize(m.TimesStream));
+    }
     unsigned long long begin = ~0ull, end = 0;
     for (size_t i = 0; i + 1 < stamps.size(); i += 2) {
         begin = std::min(begin, stamps[i]);

@@ -170,9 +170,11 @@ bool CbHipApplyPredictionTypeDevice(CbHipEvaluatorHandle* evaluator, int predict
 
 bool CbHipSynchronize(CbHipEvaluatorHandle* evaluator, void* hipStream);
 
-/* hipEvent-measured duration of the binarize and evaluate kernels of the last CbHipEvalData or
- * host-level prediction call (summed over its chunks). A call that ran as one fused launch reports the
- * whole launch as evalMs and 0 as binarizeMs, whatever the entry point. */
+/* Duration of the binarize and evaluate kernels of the last CbHipEvalData or host-level prediction call
+ * (summed over its chunks), measured with hipEvents. A call that ran as one fused launch reports the
+ * whole launch as evalMs and 0 as binarizeMs, whatever the entry point; so does a small batch of an oblivious
+ * model that ran as one launch, whose evalMs is the time from its first workgroup's start to its last one's
+ * end on the device's clock. The call only reads what was measured: it waits for no stream and no other call. */
 bool CbHipLastKernelTimes(CbHipEvaluatorHandle* evaluator, float* binarizeMs, float* evalMs);
 
 /* Which kernels a whole-model CbHipEvalData (or host entry point) call on docCount documents of `layout`

@@ -235,3 +235,35 @@ def test_workgroups_that_walk_several_slices(seed, n_float, n_cat, trees, depth,
     sample = rng.choice(docs, size=2000, replace=False)
     np.testing.assert_allclose(out.cpu().numpy()[:docs * dim].reshape(docs, dim)[sample],
                                OracleModel(model).calc(x[sample]).reshape(-1, dim), rtol=1e-9, atol=1e-12)
+
+
+def test_kernel_times_are_read_without_waiting_for_other_streams():
+    """A small-batch call's times come at once while the null stream is busy, and leave a capture alone."""
+    import torch
+
+    model, info = syn.build_model("C1", trees=150)
+    model.enable_gpu_evaluation(0)
+    ev = model.evaluator()
+    docs = 2000
+    x = syn.device_features(info, docs)
+    out = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+    feats = ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), x.shape[1])
+    torch.cuda.synchronize()
+    ev.eval_data(feats, docs, out.data_ptr())
+    expected = ev.last_kernel_times()
+    assert expected[0] == 0.0 and 0.0 < expected[1] < 100.0
+    busy = torch.cuda.Event()
+    torch.cuda._sleep(500_000_000)  # some 0.2 s on the null stream
+    busy.record()
+    assert ev.last_kernel_times() == expected
+    assert not busy.query(), "the times waited for the null stream"
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    ones = torch.ones(16, device="cuda:0")
+    with torch.cuda.graph(graph):
+        ones += 1.0
+        assert ev.last_kernel_times() == expected
+    for i in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((ones == 2.0 + i).all())
