@@ -3534,28 +3534,38 @@ void THipEvaluator::LeafIndexesQuantizedDevice(const uint8_t* bins, size_t docCo
     CBAMD_ENSURE(bins != nullptr && indexes != nullptr, "null pointer passed to leaf index calculation");
     hipStream_t s = m.Pick(stream);
     const size_t blocks = (docCount + 255) / 256;
-    const size_t tileLds = static_cast<size_t>(m.LayoutBuckets) * dev::kDocsPerBlock + dev::kDocsPerBlock * dev::kLeafIndexPitch * 4;
-    if (m.Oblivious && m.MaxDepth <= 8 && m.PackedTrees.Get() != nullptr && tileLds <= kMaxTileLdsBytes &&
-        docCount < (size_t(1) << 31)) {
-        // shares of the trees: enough workgroups for the chip's 256 CUs to go through them a few times over
-        const size_t groups = (treeEnd - treeStart + dev::kLeafIndexGroup - 1) / dev::kLeafIndexGroup;
-        const size_t wanted = std::max<size_t>(1, std::min<size_t>(groups, (kLeafIndexWorkgroups + blocks - 1) / blocks));
-        const size_t shareGroups = (groups + wanted - 1) / wanted;
-        const size_t shares = (groups + shareGroups - 1) / shareGroups;
-        CBAMD_ENSURE(blocks * shares < (size_t(1) << 31), "batch is too large for one leaf index launch");
-        const auto launch = [&](auto kernel) {
-            EnsureDynamicLds(reinterpret_cast<const void*>(kernel), tileLds);
-            hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks * shares)), dim3(dev::kLeafIndexThreads), tileLds, s,
+    const auto tileLds = [&](int group) {
+        return static_cast<size_t>(m.LayoutBuckets) * dev::kDocsPerBlock + static_cast<size_t>(dev::kDocsPerBlock) * dev::LeafIndexPitch(group) * 4;
+    };
+    if (m.Oblivious && m.MaxDepth <= 8 && m.PackedTrees.Get() != nullptr &&
+        tileLds(dev::kLeafIndexSmallGroup) <= kMaxTileLdsBytes && docCount < (size_t(1) << 31)) {
+        const auto launch = [&](auto kernel, int group) {
+            // shares of the trees: enough workgroups for the chip's 256 CUs to go through them a few times over
+            const size_t groups = (treeEnd - treeStart + group - 1) / group;
+            const size_t wanted = std::max<size_t>(1, std::min<size_t>(groups, (kLeafIndexWorkgroups + blocks - 1) / blocks));
+            const size_t shareGroups = (groups + wanted - 1) / wanted;
+            const size_t shares = (groups + shareGroups - 1) / shareGroups;
+            CBAMD_ENSURE(blocks * shares < (size_t(1) << 31), "batch is too large for one leaf index launch");
+            EnsureDynamicLds(reinterpret_cast<const void*>(kernel), tileLds(group));
+            hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks * shares)), dim3(dev::kLeafIndexThreads), tileLds(group), s,
                                reinterpret_cast<const uint32_t*>(bins), static_cast<uint32_t>(docCount), m.LayoutBuckets,
                                m.PackedTrees.Get(), static_cast<uint32_t>(treeStart), static_cast<uint32_t>(treeEnd),
-                               static_cast<uint32_t>(shares), static_cast<uint32_t>(shareGroups * dev::kLeafIndexGroup), indexes);
+                               static_cast<uint32_t>(shares), static_cast<uint32_t>(shareGroups * group), indexes);
         };
-        if (m.PackedSevenBit && m.MaxDepth <= 6) {
-            launch(dev::LeafIndexesTileKernel<true, 6>);
-        } else if (m.PackedSevenBit) {
-            launch(dev::LeafIndexesTileKernel<true, 8>);
+        const auto launchGroup = [&](auto group) {
+            constexpr int G = decltype(group)::value;
+            if (m.PackedSevenBit && m.MaxDepth <= 6) {
+                launch(dev::LeafIndexesTileKernel<true, 6, G>, G);
+            } else if (m.PackedSevenBit) {
+                launch(dev::LeafIndexesTileKernel<true, 8, G>, G);
+            } else {
+                launch(dev::LeafIndexesTileKernel<false, 8, G>, G);
+            }
+        };
+        if (tileLds(dev::kLeafIndexGroup) <= kMaxTileLdsBytes) {
+            launchGroup(std::integral_constant<int, dev::kLeafIndexGroup>());
         } else {
-            launch(dev::LeafIndexesTileKernel<false, 8>);
+            launchGroup(std::integral_constant<int, dev::kLeafIndexSmallGroup>());
         }
         HIP_CHECK(hipGetLastError());
         return;

@@ -3077,14 +3077,22 @@ __global__ __launch_bounds__(256) void LeafIndexesKernel(const uint8_t* __restri
 // block and 4-byte stores, 227 with shares and 16-byte stores, 165 with whole lines (4.85 TB/s).
 // A share is some groups of 64 trees: the grid is blocks * shares, so that a batch of a few hundred blocks still fills
 // the chip a few times over (one workgroup per block left a last generation nearly empty).
-// packedTrees as in EvalObliviousTileKernel. block = 512 threads, dynamic LDS = buckets * 256 + 256 * 33 * 4.
+// GROUP = 32 is for tiles that leave less than 33 KB of LDS (509 to 576 buckets): half the trees per group, a line of a
+// document at a time, a ring of 64 trees in 16 KB. Its documents' rings have no spare dword between them; each starts a
+// dword further on than that of four documents before, so that the lanes' stores fall on all banks. 200 000 documents * 500
+// trees of depth 8, whole call: 540 buckets 250 us, 2540 through LeafIndexesKernel; 508 buckets, groups of 64, 251.
+// packedTrees as in EvalObliviousTileKernel. block = 512 threads, dynamic LDS = buckets * 256 + 256 * LeafIndexPitch * 4.
 constexpr int kLeafIndexGroup = 64;
+constexpr int kLeafIndexSmallGroup = 32;
 constexpr int kLeafIndexThreads = 512;
-constexpr int kLeafIndexRing = 2 * kLeafIndexGroup / 4;   // dwords of a document's ring
-constexpr int kLeafIndexPitch = kLeafIndexRing + 1;
 constexpr int kLeafIndexLine = 32;                        // dwords of a line of the output
 
-template <bool SEVEN_BIT, int MAXD>
+// dwords between two documents' rings of two groups of trees
+__host__ __device__ constexpr int LeafIndexPitch(int group) {
+    return group == kLeafIndexSmallGroup ? 2 * group / 4 : 2 * group / 4 + 1;
+}
+
+template <bool SEVEN_BIT, int MAXD, int GROUP>
 __global__ __launch_bounds__(kLeafIndexThreads) void LeafIndexesTileKernel(
     const uint32_t* __restrict__ bins, uint32_t docCount, uint32_t bucketCount, const uint32_t* __restrict__ packedTrees,
     uint32_t treeBegin, uint32_t treeEnd, uint32_t shares, uint32_t shareTrees, uint32_t* __restrict__ out) {
@@ -3109,7 +3117,13 @@ __global__ __launch_bounds__(kLeafIndexThreads) void LeafIndexesTileKernel(
     const uint32_t blockDocs = min(static_cast<uint32_t>(kDocsPerBlock), docCount - block * kDocsPerBlock);
     uint32_t* blockOut = out + static_cast<size_t>(block) * kDocsPerBlock * treeCount + (firstTree - treeBegin);
     constexpr int kWaves = kLeafIndexThreads / kWave;
-    constexpr int kPerWave = kLeafIndexGroup / kWaves;
+    constexpr int kPerWave = GROUP / kWaves;
+    constexpr int kRing = 2 * GROUP / 4, kPitch = LeafIndexPitch(GROUP);  // dwords of a document's ring, and to the next one
+    constexpr uint32_t kDocThreads = GROUP / 4;                           // threads that write a document
+    constexpr uint32_t kDocsPerPass = kLeafIndexThreads / kDocThreads;
+    // where the ring of document d of the block starts, the same for every kWave documents
+    const auto ringStart = [](uint32_t d) { return kPitch == kRing ? d / 4 : 0u; };
+    static_assert(kPitch != kRing || (kWave / 4 % kRing == 0 && kDocsPerPass / 4 % kRing == 0), "documents that share a start");
     // the packed rows of the wave's trees of a group, four trees to a register, fetched a group ahead; trees past
     // the share are walked as its last tree and not written
     uint32_t rows[kPerWave / 4];
@@ -3121,7 +3135,7 @@ __global__ __launch_bounds__(kLeafIndexThreads) void LeafIndexesTileKernel(
         }
     };
     fetchRows(0);
-    for (int32_t group = 0; group < count; group += kLeafIndexGroup) {
+    for (int32_t group = 0; group < count; group += GROUP) {
         __syncthreads();  // the tile is loaded; the previous group's indexes are written
 #pragma unroll
         for (int q = 0; q < kPerWave / 4; ++q) {
@@ -3131,49 +3145,48 @@ __global__ __launch_bounds__(kLeafIndexThreads) void LeafIndexesTileKernel(
             const uint32_t high01 = __builtin_amdgcn_perm(idx[1], idx[0], 0x07030602u);
             const uint32_t low23 = __builtin_amdgcn_perm(idx[3], idx[2], 0x05010400u);
             const uint32_t high23 = __builtin_amdgcn_perm(idx[3], idx[2], 0x07030602u);
-            uint32_t* cell = ring + lane * kLeafIndexPitch + (group / 4 + wave * (kPerWave / 4) + q) % kLeafIndexRing;
-            cell[0 * kWave * kLeafIndexPitch] = __builtin_amdgcn_perm(low23, low01, 0x05040100u);
-            cell[1 * kWave * kLeafIndexPitch] = __builtin_amdgcn_perm(low23, low01, 0x07060302u);
-            cell[2 * kWave * kLeafIndexPitch] = __builtin_amdgcn_perm(high23, high01, 0x05040100u);
-            cell[3 * kWave * kLeafIndexPitch] = __builtin_amdgcn_perm(high23, high01, 0x07060302u);
+            uint32_t* cell = ring + lane * kPitch + (group / 4 + wave * (kPerWave / 4) + q + ringStart(lane)) % kRing;
+            cell[0 * kWave * kPitch] = __builtin_amdgcn_perm(low23, low01, 0x05040100u);
+            cell[1 * kWave * kPitch] = __builtin_amdgcn_perm(low23, low01, 0x07060302u);
+            cell[2 * kWave * kPitch] = __builtin_amdgcn_perm(high23, high01, 0x05040100u);
+            cell[3 * kWave * kPitch] = __builtin_amdgcn_perm(high23, high01, 0x07060302u);
         }
         __syncthreads();
-        fetchRows(group + kLeafIndexGroup);
-        const int32_t done = min(group + kLeafIndexGroup, count);  // trees whose indexes are in the ring
-        const int32_t quadTree = group + static_cast<int32_t>(tid % 16) * 4;
-        // the indexes of trees `tree` .. tree + 3 of the document whose ring starts at `cells`
-        const auto ringQuad = [&](const uint32_t* cells, int32_t tree) {
-            const uint32_t at = static_cast<uint32_t>(tree + 4 * kLeafIndexRing) / 4;
-            const uint32_t bytes = __builtin_amdgcn_alignbyte(cells[(at + 1) % kLeafIndexRing], cells[at % kLeafIndexRing],
+        fetchRows(group + GROUP);
+        const int32_t done = min(group + GROUP, count);  // trees whose indexes are in the ring
+        const int32_t quadTree = group + static_cast<int32_t>(tid % kDocThreads) * 4;
+        // the indexes of trees `tree` .. tree + 3 of the document whose ring is `cells` and starts at `start`
+        const auto ringQuad = [&](const uint32_t* cells, uint32_t start, int32_t tree) {
+            const uint32_t at = static_cast<uint32_t>(tree + 4 * kRing) / 4 + start;
+            const uint32_t bytes = __builtin_amdgcn_alignbyte(cells[(at + 1) % kRing], cells[at % kRing],
                                                               static_cast<uint32_t>(tree) & 3u);
             return make_uint4(bytes & 0xffu, (bytes >> 8) & 0xffu, (bytes >> 16) & 0xffu, bytes >> 24);
         };
-        constexpr uint32_t kDocsPerPass = kLeafIndexThreads / 16;
         if (group > 0 && (done < count || !lastShare)) {
-            // inside a row: two whole lines per document (fewer behind a share's last, shorter group)
-            uint32_t* row = blockOut + (tid / 16) * treeCount;
-            const uint32_t* cells = ring + (tid / 16) * kLeafIndexPitch;
+            // inside a row: a group's whole lines per document (fewer behind a share's last, shorter group)
+            uint32_t* row = blockOut + (tid / kDocThreads) * treeCount;
+            const uint32_t* cells = ring + (tid / kDocThreads) * kPitch;
             const int32_t groupTrees = done - group;
 #pragma unroll
             for (uint32_t pass = 0; pass < kDocsPerBlock / kDocsPerPass; ++pass) {
                 const int32_t behind = static_cast<int32_t>((reinterpret_cast<uintptr_t>(row) / 4) % kLeafIndexLine);
-                const uint4 quad = ringQuad(cells, quadTree - behind);
-                if (pass * kDocsPerPass + tid / 16 < blockDocs && quadTree - group < groupTrees) {
+                const uint4 quad = ringQuad(cells, ringStart(tid / kDocThreads), quadTree - behind);
+                if (pass * kDocsPerPass + tid / kDocThreads < blockDocs && quadTree - group < groupTrees) {
                     *reinterpret_cast<uint4*>(row + (quadTree - behind)) = quad;
                 }
                 row += kDocsPerPass * treeCount;
-                cells += kDocsPerPass * kLeafIndexPitch;
+                cells += kDocsPerPass * kPitch;
             }
             continue;
         }
-        for (uint32_t d = tid / 16; d < blockDocs; d += kDocsPerPass) {
+        for (uint32_t d = tid / kDocThreads; d < blockDocs; d += kDocsPerPass) {
             uint32_t* row = blockOut + d * treeCount;
             const int32_t behind = static_cast<int32_t>((reinterpret_cast<uintptr_t>(row) / 4) % kLeafIndexLine);
             // whole lines only, but for the row's first and last
             const int32_t begin = group > 0 ? group - behind : firstShare ? 0 : lead - behind;
             const int32_t end = done == count && lastShare ? count : done - behind;
-            for (int32_t tree = quadTree - behind; tree < end; tree += kLeafIndexGroup) {
-                const uint4 quad = ringQuad(ring + d * kLeafIndexPitch, tree);
+            for (int32_t tree = quadTree - behind; tree < end; tree += GROUP) {
+                const uint4 quad = ringQuad(ring + d * kPitch, ringStart(d), tree);
                 if (tree >= begin && tree + 4 <= end) {
                     *reinterpret_cast<uint4*>(row + tree) = quad;
                 } else {
