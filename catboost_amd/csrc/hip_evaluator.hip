@@ -1426,21 +1426,35 @@ struct THipEvaluator::TImpl {
     uint32_t SmallCellCount = 0;
     TDeviceVec<uint32_t> SmallTable;
     size_t SmallCellsAt = 0, SmallFirstLeafAt = 0;
-    // (no slices on a model too short for them: its one slice is the whole model)
-    uint32_t SmallSliceTrees(size_t treeCount) const {
-        const uint32_t slice = RegKernelUsable ? RegSliceTrees(RegTreeBlockSize) : 32;
-        return treeCount < 2 * static_cast<size_t>(slice) ? static_cast<uint32_t>(treeCount) : slice;
-    }
+    // rows of the table without the null trees at its end, and those of a slice: a slice of the register kernels' (the whole
+    // model when it is too short for slices), or a partial sum of SumOrder() with null trees up to the length of the longest
+    uint32_t SmallTreeCount = 0, SmallSliceTrees = 0;
+    uint32_t SmallSliceCount() const { return (SmallTreeCount + SmallSliceTrees - 1) / SmallSliceTrees; }
+
+    // The order in which a whole-model launch of EvalQuantizedDevice adds the trees of an oblivious model of depth <= 8 that
+    // the register kernels do not take: partial sums, each in tree order, added one after the other.
+    struct TSumOrder {
+        uint32_t Waves = 1;     // of a workgroup
+        uint32_t Side = 1;      // consecutive trees that a wave takes at a time; a last group that is not full is wave 0's
+        bool PerTree = false;   // ... each to a sum of its own
+        uint32_t Parts() const { return PerTree ? Waves * Side : Waves; }
+        uint32_t PartOf(size_t tree, size_t treeCount) const {
+            const size_t group = tree / Side;
+            const size_t wave = (group + 1) * Side <= treeCount ? group % Waves : 0;
+            return static_cast<uint32_t>(PerTree ? wave * Side + tree % Side : wave);
+        }
+    };
+    TSumOrder SumOrder() const;
+
     int SmallDims() const { return Dim == 1 ? 1 : Dim == 2 ? 2 : 4; }
     uint32_t SmallPasses() const { return static_cast<uint32_t>((Dim + SmallDims() - 1) / SmallDims()); }
-    size_t SmallLdsBytes(size_t treeCount) const {
-        const size_t sliceTrees = SmallSliceTrees(treeCount);
+    size_t SmallLdsBytes() const {
         const size_t tile = static_cast<size_t>(dev::SmallDocPitch(SmallCellCount)) * dev::kSmallDocs * 4;
-        return tile + (treeCount + sliceTrees - 1) / sliceTrees * dev::kSmallDocs * SmallDims() * 8;
+        return tile + static_cast<size_t>(SmallSliceCount()) * dev::kSmallDocs * SmallDims() * 8;
     }
-    size_t FewLdsBytes(size_t treeCount) const {
-        const size_t sliceTrees = SmallSliceTrees(treeCount);
-        return (static_cast<size_t>(SmallCellCount) + 1) / 2 * 8 + (treeCount + sliceTrees - 1) / sliceTrees * (sliceTrees + 2) * SmallDims() * 8;
+    size_t FewLdsBytes() const {
+        return (static_cast<size_t>(SmallCellCount) + 1) / 2 * 8 +
+               static_cast<size_t>(SmallSliceCount()) * (SmallSliceTrees + 2) * SmallDims() * 8;
     }
 
     // Staging of the calls that own their buffers (CalcDevice and the host entry points): a call borrows a
@@ -1790,73 +1804,6 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     m.BucketOffset.Upload(offsets);
     m.BucketFlags.Upload(flags);
     m.Values.Upload(values);
-
-    // ---- small-batch kernel: every split as "cell of the tile above a border"
-    if (m.Oblivious && m.MaxDepth <= 8 && TreeCount > 0 && m.CtrCount == 0 && BucketCount > 0) {
-        std::vector<dev::TSmallCell> cells;
-        std::vector<uint32_t> cellOfBucket(BucketCount, UINT32_MAX);
-        std::map<std::pair<uint32_t, uint32_t>, uint32_t> cellOfValue;  // one-hot: (bucket, value's index) -> cell
-        // rows of null trees behind the model's, for a last slice that ends inside a turn: no level is above +inf or NaN
-        std::vector<uint32_t> rows((TreeCount + dev::kSmallNullTrees) * 16, 0);
-        std::vector<uint32_t> first(TreeCount + dev::kSmallNullTrees, static_cast<uint32_t>(trees.LeafValues.size()));
-        const uint32_t never = 0x7f800000u;
-        bool usable = trees.LeafValues.size() < (size_t(1) << 32);
-        for (size_t t = 0; t < TreeCount + dev::kSmallNullTrees && usable; ++t) {
-            const int depth = t < TreeCount ? trees.TreeSizes[t] : 0;
-            uint32_t* row = rows.data() + t * 16;
-            if (t < TreeCount) {
-                first[t] = static_cast<uint32_t>(trees.TreeFirstLeafOffsets[t]);
-            }
-            for (int d = 0; d < 8; ++d) {
-                row[8 + d] = never;
-                if (d >= depth) {
-                    continue;
-                }
-                const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + d];
-                const uint32_t b = rb.FeatureIndex, n = offsets[b + 1] - offsets[b];
-                // a damaged model may name a border that is not there: such a split stays with the kernels on bins
-                const bool oneHot = (flags[b] & dev::kBucketFlagOneHot) != 0;
-                const uint32_t at = oneHot ? static_cast<uint8_t>(~rb.XorMask) : rb.SplitIdx;
-                if (at == 0 || at > n || (oneHot ? rb.SplitIdx != 0xff : rb.XorMask != 0)) {
-                    usable = false;
-                    break;
-                }
-                uint32_t cell;
-                if (oneHot) {
-                    // "bin = at", and no other value of the bucket is the same one
-                    const uint32_t value = values[offsets[b] + at - 1];
-                    usable = usable &&
-                             std::count(values.begin() + offsets[b], values.begin() + offsets[b + 1], value) == 1;
-                    const auto found = cellOfValue.emplace(std::make_pair(b, at), static_cast<uint32_t>(cells.size()));
-                    if (found.second) {
-                        cells.push_back({srcFlat[b], srcSplit[b], 2u, value});
-                    }
-                    cell = found.first->second;
-                    row[8 + d] = 0x3f000000u;  // 0.5
-                } else {
-                    if (cellOfBucket[b] == UINT32_MAX) {
-                        cellOfBucket[b] = static_cast<uint32_t>(cells.size());
-                        cells.push_back({srcFlat[b], srcSplit[b], (flags[b] & dev::kBucketFlagNanToInf) ? 1u : 0u, 0u});
-                    }
-                    cell = cellOfBucket[b];
-                    row[8 + d] = values[offsets[b] + at - 1];
-                }
-                row[d] = cell * 4;
-            }
-        }
-        if (usable && !cells.empty()) {
-            // one allocation: the rows, the cells, the first leaves
-            std::vector<uint32_t> table(std::move(rows));
-            m.SmallCellsAt = table.size();
-            const uint32_t* cellDwords = reinterpret_cast<const uint32_t*>(cells.data());
-            table.insert(table.end(), cellDwords, cellDwords + cells.size() * (sizeof(dev::TSmallCell) / 4));
-            m.SmallFirstLeafAt = table.size();
-            table.insert(table.end(), first.begin(), first.end());
-            m.SmallTable.Upload(table);
-            m.SmallCellCount = static_cast<uint32_t>(cells.size());
-            m.SmallUsable = true;
-        }
-    }
 
     // ---- tree tables
     std::vector<uint32_t> splits(trees.RepackedBins.size());
@@ -2637,6 +2584,106 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             m.TileMap.Upload(tileMap);
         }
     }
+
+    // ---- small-batch kernel: every split as "cell of the tile above a border"
+    if (m.Oblivious && m.MaxDepth <= 8 && TreeCount > 0 && m.CtrCount == 0 && BucketCount > 0) {
+        std::vector<dev::TSmallCell> cells;
+        std::vector<uint32_t> cellOfBucket(BucketCount, UINT32_MAX);
+        std::map<std::pair<uint32_t, uint32_t>, uint32_t> cellOfValue;  // one-hot: (bucket, value's index) -> cell
+        // The trees in slices that are added as larger batches' kernels add them: consecutive trees for the register kernels'
+        // slices, else the trees of a wave's partial sum.
+        std::vector<size_t> order;
+        const size_t nullTree = TreeCount;
+        if (m.RegKernelUsable) {
+            order.resize(TreeCount);
+            std::iota(order.begin(), order.end(), size_t(0));
+            const uint32_t slice = RegSliceTrees(m.RegTreeBlockSize);
+            m.SmallSliceTrees = TreeCount < 2 * static_cast<size_t>(slice) ? static_cast<uint32_t>(TreeCount) : slice;
+        } else {
+            const TImpl::TSumOrder sums = m.SumOrder();
+            std::vector<std::vector<size_t>> parts(sums.Parts());
+            size_t longest = 0;
+            for (size_t t = 0; t < TreeCount; ++t) {
+                std::vector<size_t>& part = parts[sums.PartOf(t, TreeCount)];
+                part.push_back(t);
+                longest = std::max(longest, part.size());
+            }
+            while (parts.back().empty()) {
+                parts.pop_back();  // sums of zero
+            }
+            if (parts.size() > 1) {
+                longest = (longest + dev::kSmallTurn - 1) / dev::kSmallTurn * dev::kSmallTurn;
+            }
+            for (std::vector<size_t>& part : parts) {
+                part.resize(longest, nullTree);
+                order.insert(order.end(), part.begin(), part.end());
+            }
+            m.SmallSliceTrees = static_cast<uint32_t>(longest);
+        }
+        m.SmallTreeCount = static_cast<uint32_t>(order.size());
+        // rows of null trees at the end, for a last slice that ends inside a turn: no level is above +inf or NaN
+        order.resize(order.size() + dev::kSmallNullTrees, nullTree);
+        std::vector<uint32_t> rows(order.size() * 16, 0);
+        std::vector<uint32_t> first(order.size(), static_cast<uint32_t>(trees.LeafValues.size()));
+        const uint32_t never = 0x7f800000u;
+        bool usable = trees.LeafValues.size() < (size_t(1) << 32);
+        for (size_t place = 0; place < order.size() && usable; ++place) {
+            const size_t t = order[place];
+            const int depth = t < TreeCount ? trees.TreeSizes[t] : 0;
+            uint32_t* row = rows.data() + place * 16;
+            if (t < TreeCount) {
+                first[place] = static_cast<uint32_t>(trees.TreeFirstLeafOffsets[t]);
+            }
+            for (int d = 0; d < 8; ++d) {
+                row[8 + d] = never;
+                if (d >= depth) {
+                    continue;
+                }
+                const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + d];
+                const uint32_t b = rb.FeatureIndex, n = offsets[b + 1] - offsets[b];
+                // a damaged model may name a border that is not there: such a split stays with the kernels on bins
+                const bool oneHot = (flags[b] & dev::kBucketFlagOneHot) != 0;
+                const uint32_t at = oneHot ? static_cast<uint8_t>(~rb.XorMask) : rb.SplitIdx;
+                if (at == 0 || at > n || (oneHot ? rb.SplitIdx != 0xff : rb.XorMask != 0)) {
+                    usable = false;
+                    break;
+                }
+                uint32_t cell;
+                if (oneHot) {
+                    // "bin = at", and no other value of the bucket is the same one
+                    const uint32_t value = values[offsets[b] + at - 1];
+                    usable = usable &&
+                             std::count(values.begin() + offsets[b], values.begin() + offsets[b + 1], value) == 1;
+                    const auto found = cellOfValue.emplace(std::make_pair(b, at), static_cast<uint32_t>(cells.size()));
+                    if (found.second) {
+                        cells.push_back({srcFlat[b], srcSplit[b], 2u, value});
+                    }
+                    cell = found.first->second;
+                    row[8 + d] = 0x3f000000u;  // 0.5
+                } else {
+                    if (cellOfBucket[b] == UINT32_MAX) {
+                        cellOfBucket[b] = static_cast<uint32_t>(cells.size());
+                        cells.push_back({srcFlat[b], srcSplit[b], (flags[b] & dev::kBucketFlagNanToInf) ? 1u : 0u, 0u});
+                    }
+                    cell = cellOfBucket[b];
+                    row[8 + d] = values[offsets[b] + at - 1];
+                }
+                row[d] = cell * 4;
+            }
+        }
+        if (usable && !cells.empty()) {
+            // one allocation: the rows, the cells, the first leaves
+            std::vector<uint32_t> table(std::move(rows));
+            m.SmallCellsAt = table.size();
+            const uint32_t* cellDwords = reinterpret_cast<const uint32_t*>(cells.data());
+            table.insert(table.end(), cellDwords, cellDwords + cells.size() * (sizeof(dev::TSmallCell) / 4));
+            m.SmallFirstLeafAt = table.size();
+            table.insert(table.end(), first.begin(), first.end());
+            m.SmallTable.Upload(table);
+            m.SmallCellCount = static_cast<uint32_t>(cells.size());
+            m.SmallUsable = true;
+        }
+    }
 }
 
 THipEvaluator::~THipEvaluator() = default;
@@ -2853,6 +2900,24 @@ size_t TileLeafLdsBytes(int maxd, int dchunk, int waves = dev::kTileWaves) {
     return static_cast<size_t>(waves) * (size_t(1) << maxd) * dchunk * sizeof(double);
 }
 
+// leaf values go through LDS whenever the tile, the accumulator and the per-wave leaf regions
+// fit the 160 KB of a CU (gathers from global memory cost ~50 L1 accesses per wave instruction)
+bool TileLeavesInLds(uint32_t buckets, int maxd, int dchunk, bool pairAligned) {
+    return pairAligned && TileLdsBytes(buckets, dchunk) + TileLeafLdsBytes(maxd, dchunk) <= kMaxTileLdsBytes;
+}
+
+// a tile of which only one workgroup fits a CU gets sixteen waves instead of eight, LDS permitting
+int TileWaves(uint32_t buckets, int maxd, int dchunk, bool leavesInLds) {
+    const size_t narrow = TileLdsBytes(buckets, dchunk) + (leavesInLds ? TileLeafLdsBytes(maxd, dchunk) : 0);
+    const size_t wide = TileLdsBytes(buckets, dchunk) + (leavesInLds ? TileLeafLdsBytes(maxd, dchunk, dev::kWideTileWaves) : 0);
+    return 2 * narrow > kMaxTileLdsBytes && wide <= kMaxTileLdsBytes ? dev::kWideTileWaves : dev::kTileWaves;
+}
+
+// the levels that EvalObliviousTileKernel walks
+int TileLevels(uint32_t maxDepth) {
+    return maxDepth <= 4 ? 4 : maxDepth <= 6 ? 6 : 8;
+}
+
 struct TTileArgs {
     const uint8_t* Bins;
     size_t DocCount;
@@ -2881,10 +2946,7 @@ void LaunchEvalTileW(const TTileArgs& a) {
 
 template <bool SEVEN_BIT, int MAXD, int DCHUNK, bool LEAF_LDS>
 void LaunchEvalTileL(const TTileArgs& a) {
-    // a tile of which only one workgroup fits a CU gets sixteen waves instead of eight, LDS permitting
-    const size_t narrow = TileLdsBytes(a.Buckets, DCHUNK) + (LEAF_LDS ? TileLeafLdsBytes(MAXD, DCHUNK) : 0);
-    const size_t wide = TileLdsBytes(a.Buckets, DCHUNK) + (LEAF_LDS ? TileLeafLdsBytes(MAXD, DCHUNK, dev::kWideTileWaves) : 0);
-    if (2 * narrow > kMaxTileLdsBytes && wide <= kMaxTileLdsBytes) {
+    if (TileWaves(a.Buckets, MAXD, DCHUNK, LEAF_LDS) == dev::kWideTileWaves) {
         LaunchEvalTileW<SEVEN_BIT, MAXD, DCHUNK, LEAF_LDS, dev::kWideTileWaves>(a);
     } else {
         LaunchEvalTileW<SEVEN_BIT, MAXD, DCHUNK, LEAF_LDS, dev::kTileWaves>(a);
@@ -2893,10 +2955,7 @@ void LaunchEvalTileL(const TTileArgs& a) {
 
 template <bool SEVEN_BIT, int MAXD, int DCHUNK>
 void LaunchEvalTile(const TTileArgs& a) {
-    // leaf values go through LDS whenever the tile, the accumulator and the per-wave leaf regions
-    // fit the 160 KB of a CU (gathers from global memory cost ~50 L1 accesses per wave instruction)
-    const size_t withLeaves = TileLdsBytes(a.Buckets, DCHUNK) + TileLeafLdsBytes(MAXD, DCHUNK);
-    if (a.LeavesPairAligned && withLeaves <= kMaxTileLdsBytes) {
+    if (TileLeavesInLds(a.Buckets, MAXD, DCHUNK, a.LeavesPairAligned)) {
         LaunchEvalTileL<SEVEN_BIT, MAXD, DCHUNK, true>(a);
     } else {
         LaunchEvalTileL<SEVEN_BIT, MAXD, DCHUNK, false>(a);
@@ -2917,12 +2976,10 @@ void LaunchEvalTileD(int dchunk, const TTileArgs& a) {
 
 template <bool SEVEN_BIT>
 void LaunchEvalTileM(uint32_t maxDepth, int dchunk, const TTileArgs& a) {
-    if (maxDepth <= 4) {
-        LaunchEvalTileD<SEVEN_BIT, 4>(dchunk, a);
-    } else if (maxDepth <= 6) {
-        LaunchEvalTileD<SEVEN_BIT, 6>(dchunk, a);
-    } else {
-        LaunchEvalTileD<SEVEN_BIT, 8>(dchunk, a);
+    switch (TileLevels(maxDepth)) {
+        case 4: LaunchEvalTileD<SEVEN_BIT, 4>(dchunk, a); break;
+        case 6: LaunchEvalTileD<SEVEN_BIT, 6>(dchunk, a); break;
+        default: LaunchEvalTileD<SEVEN_BIT, 8>(dchunk, a); break;
     }
 }
 
@@ -2971,6 +3028,27 @@ void LaunchEval(bool oblivious, const uint8_t* bins, size_t docCount, uint32_t b
 }
 
 }  // namespace
+
+// One branch per kernel, in the order in which EvalQuantizedDevice comes to them.
+THipEvaluator::TImpl::TSumOrder THipEvaluator::TImpl::SumOrder() const {
+    const int dchunk = TileChunk(Dim);
+    TSumOrder order;
+    if (TileRows.Get() != nullptr) {
+        order.Waves = RowTileWaves(TileRowCount, MaxDepth, Dim);
+    } else if (TileLdsBytes(LayoutBuckets, dchunk) <= kMaxTileLdsBytes) {
+        const int levels = TileLevels(MaxDepth);
+        const bool leavesInLds = TileLeavesInLds(LayoutBuckets, levels, dchunk, Dim > 1 || LeavesPairAligned);
+        order.Waves = static_cast<uint32_t>(TileWaves(LayoutBuckets, levels, dchunk, leavesInLds));
+    } else if (QuadRows.Get() != nullptr) {
+        order.Waves = QuadTileWaves(TileRowCount, MaxDepth <= 6 ? 6 : 8);
+        order.Side = 4;
+        order.PerTree = true;
+    } else if (Dim == 1 && HalfTileLeaves.Get() != nullptr && HalfTileLdsBytes(LayoutBuckets, 8) <= kMaxTileLdsBytes) {
+        order.Waves = PairRows.Get() != nullptr ? dev::kPairWaves : dev::kTileWaves;
+        order.Side = PairRows.Get() != nullptr ? 2 : 1;
+    }
+    return order;
+}
 
 void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, size_t treeStart, size_t treeEnd,
                                         double* results, void* stream) {
@@ -3351,12 +3429,12 @@ void THipEvaluator::EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCou
 bool THipEvaluator::TakesSmallBatchKernel(size_t docCount, size_t treeStart, size_t treeEnd) const {
     const TImpl& m = *Impl;
     return m.SmallUsable && m.SmallBatchSlices && docCount > 0 && docCount * m.SmallPasses() <= kSmallBatchDocs && treeStart == 0 &&
-           treeEnd == TreeCount && m.SmallLdsBytes(TreeCount) <= kMaxTileLdsBytes;
+           treeEnd == TreeCount && m.SmallLdsBytes() <= kMaxTileLdsBytes;
 }
 
 // One launch of the small-batch kernel whose end `stop` marks. `batch` and `results` may be device or pinned host memory.
 static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THostContext& ctx, const TFeatureBatch& batch,
-                             size_t docCount, size_t treeCount, double* results, hipStream_t s, hipEvent_t stop) {
+                             size_t docCount, double* results, hipStream_t s, hipEvent_t stop) {
     CBAMD_ENSURE(results != nullptr, "results pointer is null");
     dev::TSmallSource src = {};
     src.Floats = reinterpret_cast<const uint32_t*>(batch.Floats);
@@ -3375,9 +3453,9 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
     tab.Scale = m.Scale;
     tab.CellCount = m.SmallCellCount;
     tab.Dim = static_cast<uint32_t>(m.Dim);
-    tab.TreeCount = static_cast<uint32_t>(treeCount);
-    tab.SliceTrees = m.SmallSliceTrees(treeCount);
-    tab.SliceCount = (tab.TreeCount + tab.SliceTrees - 1) / tab.SliceTrees;
+    tab.TreeCount = m.SmallTreeCount;
+    tab.SliceTrees = m.SmallSliceTrees;
+    tab.SliceCount = m.SmallSliceCount();
     const uint32_t dims = static_cast<uint32_t>(m.SmallDims());
     const uint32_t passes = m.SmallPasses();
     const auto launch = [&](auto kernel, size_t groups, uint32_t threads, size_t lds) {
@@ -3387,13 +3465,13 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
                               static_cast<uint32_t>(docCount), tab, results, reinterpret_cast<ulonglong2*>(stamps.Values.Get()));
     };
     const auto launchFew = [&](auto kernel) {
-        launch(kernel, docCount, std::min<uint32_t>(dev::kFewThreads, (tab.TreeCount + 63) / 64 * 64), m.FewLdsBytes(treeCount));
+        launch(kernel, docCount, std::min<uint32_t>(dev::kFewThreads, (tab.TreeCount + 63) / 64 * 64), m.FewLdsBytes());
     };
     const auto launchSmall = [&](auto kernel) {
-        launch(kernel, (docCount + dev::kSmallDocs - 1) / dev::kSmallDocs, dev::kSmallThreads, m.SmallLdsBytes(treeCount));
+        launch(kernel, (docCount + dev::kSmallDocs - 1) / dev::kSmallDocs, dev::kSmallThreads, m.SmallLdsBytes());
     };
     const bool shallow = m.MaxDepth <= 6;
-    if (docCount * passes <= kFewDocs && m.FewLdsBytes(treeCount) <= kMaxTileLdsBytes) {
+    if (docCount * passes <= kFewDocs && m.FewLdsBytes() <= kMaxTileLdsBytes) {
         if (dims == 1) {
             shallow ? launchFew(dev::FewDocumentsKernel<6, 1>) : launchFew(dev::FewDocumentsKernel<8, 1>);
         } else if (dims == 2) {
@@ -3469,10 +3547,9 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
         return std::string("fused=") + m.FusedKernelName;
     }
     if (TakesSmallBatchKernel(docCount, 0, TreeCount)) {
-        const uint32_t sliceTrees = m.SmallSliceTrees(TreeCount);
-        const bool few = docCount * m.SmallPasses() <= kFewDocs && m.FewLdsBytes(TreeCount) <= kMaxTileLdsBytes;
+        const bool few = docCount * m.SmallPasses() <= kFewDocs && m.FewLdsBytes() <= kMaxTileLdsBytes;
         return std::string("binarize=none;evaluate=") + (few ? "FewDocumentsKernel<" : "SmallBatchKernel<") + std::to_string(m.MaxDepth <= 6 ? 6 : 8) + ", " + std::to_string(m.SmallDims()) +
-               ">, " + std::to_string((TreeCount + sliceTrees - 1) / sliceTrees) + " slices of the trees";
+               ">, " + std::to_string(m.SmallSliceCount()) + " slices of the trees";
     }
     std::string binarize = m.BinarizeBuckets == 0 ? "none"
                            : layout == TFeatureBatch::FlatColumns
@@ -3625,7 +3702,7 @@ void THipEvaluator::CalcDevice(const TFeatureBatch& batch, size_t docCount, size
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : m.Stream;
     if (TakesSmallBatchKernel(docCount, treeStart, treeEnd)) {
         CheckBatch(batch, docCount);
-        LaunchSmallBatch(m, *ctx, batch, docCount, TreeCount, results, s, ctx->Ev[2]);
+        LaunchSmallBatch(m, *ctx, batch, docCount, results, s, ctx->Ev[2]);
         HIP_CHECK(hipEventSynchronize(ctx->Ev[2]));
         SetLastSmallTimes(&*ctx);
         return;
@@ -3896,7 +3973,7 @@ static void CalcSmallHostBatch(THipEvaluator& ev, THipEvaluator::TImpl& m, THipE
     if (!raw) {
         slot.StageResults.Reserve(docCount * dim);
     }
-    LaunchSmallBatch(m, ctx, batch, docCount, ev.GetTreeCount(), raw ? slot.PinnedResults.Get() : slot.StageResults.Get(), ctx.Stream,
+    LaunchSmallBatch(m, ctx, batch, docCount, raw ? slot.PinnedResults.Get() : slot.StageResults.Get(), ctx.Stream,
                      slot.Ev[3]);
     if (raw) {
         HIP_CHECK(hipEventSynchronize(slot.Ev[3]));

@@ -735,8 +735,11 @@ __global__ __launch_bounds__(256) void CombineSlicesKernel(const double* __restr
 // loads, so it takes one kernel that compares the features with the splits' borders directly (no bins) and writes the
 // finished values; it may read the features from, and write the results to, pinned host memory. The values of the model's
 // features of a workgroup's documents go to LDS (a cell each); a tree is a row of sixteen dwords, eight levels' cells and
-// eight borders. The trees are summed in slices and the slices in slice order - the sums and the order of
-// CombineSlicesKernel, so that a document's value does not depend on which kernel took it. Two forms:
+// eight borders. The trees are summed in slices and the slices in slice order: those of CombineSlicesKernel, or, for models
+// that the register kernels do not take, the partial sums of the kernel that larger batches take (each slice the trees of
+// one, brought to one length with null trees), so that a document's value does not depend on which kernel took it. The
+// sixteen sums of 1000 trees over 700 buckets against slices of 32 trees: 24 us and 22 for 2048 documents, 62 and 60 for
+// 16384 (49 and 60 on the binarize and pair-tile kernels). Two forms:
 //   FewDocumentsKernel  a workgroup per document, a lane per tree; the leaf values meet in LDS, where a thread per slice
 //                       adds its slice. What bounds it: the chain of loads cell -> feature -> leaf value, a few us.
 //   SmallBatchKernel    a workgroup per sixteen documents; a row of sixteen lanes (lane = document) walks a slice, the
@@ -773,7 +776,8 @@ struct TSmallSource {     // value of feature f of document d: Floats[d * DocStr
 };
 
 constexpr int kSmallDocs = 16;                   // documents of a workgroup of SmallBatchKernel
-constexpr int kSmallNullTrees = 32;
+constexpr int kSmallTurn = 16;                   // trees that one of its lanes has in flight, one dimension at a time
+constexpr int kSmallNullTrees = 2 * kSmallTurn;
 constexpr int kSmallThreads = 512;
 constexpr int kFewThreads = 1024;
 
@@ -930,7 +934,7 @@ template <int DEPTH, int DIMS>
 __global__ __launch_bounds__(kSmallThreads) void SmallBatchKernel(TSmallSource src, uint32_t docCount, TSmallTables tab,
                                                                   double* __restrict__ out, ulonglong2* __restrict__ stamps) {
     // trees of a turn: their rows, and the leaf values of the turn before, are in flight together
-    constexpr int kTurn = DIMS == 1 ? 16 : DIMS == 2 ? 8 : 4;
+    constexpr int kTurn = kSmallTurn / DIMS;
     static_assert(2 * kTurn <= kSmallNullTrees, "rows are fetched up to a turn past the last one");
     extern __shared__ uint32_t sSmall[];
     const unsigned long long began = wall_clock64();

@@ -141,9 +141,9 @@ bool CbHipEvalData(CbHipEvaluatorHandle* evaluator, const CbHipFeatures* deviceF
  * 32 MiB (the error names the largest document count for the model); a model that runs on a fused
  * kernel keeps its bins in registers there, uses no buffer and has no such limit (a batch of such a model
  * that does not fit the buffer takes the fused kernel at any size). The call never cuts the trees into
- * slices (it has no memory for partial sums): every sum is one pass in tree order, the CPU evaluator's order
- * of additions, so for small batches it may differ in the last bits from CbHipEvalData with slicing on, and
- * it has none of that call's small-batch speed-up. All calls on one GPU share the array, so calls that
+ * slices (it has no memory for partial sums): its sums are those of CbHipEvalQuantized, so for small batches
+ * it may differ in the last bits from CbHipEvalData with slicing on, and it has none of that call's
+ * small-batch speed-up. All calls on one GPU share the array, so calls that
  * overlap there (two streams, two threads, two evaluators) race; calls in stream order on one stream are
  * safe. */
 bool CbHipEvalDataNoAlloc(CbHipEvaluatorHandle* evaluator, const CbHipFeatures* deviceFeatures, size_t docCount,
@@ -182,16 +182,19 @@ bool CbHipLastKernelTimes(CbHipEvaluatorHandle* evaluator, float* binarizeMs, fl
  * and benchmarks; no counterpart in the reference. */
 bool CbHipDescribeKernels(CbHipEvaluatorHandle* evaluator, int layout, size_t docCount, char* buffer, size_t bufferSize);
 
-/* Batches of fewer than 256 workgroups (65 536 to 262 144 documents, by the kernel) are spread over the GPU by
- * cutting the trees into slices that run side by side; a slice adds its leaves in tree order and the slices'
- * sums are then added in slice order. The result is the same for every call and every batch size below that
- * limit, and differs in the last bits (inside 1e-9 relative) from the single pass in tree order that larger
- * batches, CbHipEvalQuantized and the CPU evaluator make (cpu/evaluator_impl.cpp:362-460; single document:
- * c_api.cpp:383-384). enabled = false turns the slices off for later calls: every sum is then one pass in tree
- * order whatever the batch size, at the price of the small-batch speed-up (C2 model, 4096 documents: 0.13
- * instead of 0.04 ms per call). No counterpart in the reference. The first form acts on a bare evaluator, the
- * second on a model handle (kept across Load* calls and rebuilt evaluators). Not to be called while another
- * thread evaluates on the same handle. */
+/* Small batches are spread over the GPU by cutting the trees into slices that run side by side.
+ * Models of the register kernels (up to 224 buckets): a slice adds its leaves in tree order and the slices' sums
+ * are then added in slice order. The result is the same for every call and every batch size below 256 workgroups
+ * (262 144 documents, 524 288 with at most 96 buckets), and differs in the last bits (inside 1e-9 relative) from
+ * the single pass in tree order that larger batches, CbHipEvalQuantized and the CPU evaluator make
+ * (cpu/evaluator_impl.cpp:362-460; single document: c_api.cpp:383-384). Wider oblivious models: the slices are the
+ * partial sums that the kernels of larger batches and of CbHipEvalQuantized add, so the result of a whole-model
+ * call is the same for every batch size.
+ * enabled = false turns the slices off for later calls: a batch of any size then takes the kernels of large ones,
+ * which for the register kernels' models means one pass in tree order, at the price of the small-batch speed-up
+ * (1000 trees of depth 8 over 200 features, 4096 documents: 0.15 instead of 0.023 ms per call). No counterpart in
+ * the reference. The first form acts on a bare evaluator, the second on a model handle (kept across Load* calls and
+ * rebuilt evaluators). Not to be called while another thread evaluates on the same handle. */
 bool CbHipEvaluatorSetSmallBatchSlicing(CbHipEvaluatorHandle* evaluator, bool enabled);
 bool CbHipSetSmallBatchSlicing(void* modelHandle, bool enabled);
 

@@ -10,6 +10,7 @@ import pytest
 
 import catboost_amd as cb
 from catboost_amd import synthetic as syn
+from oracle import model_builder as mb
 from oracle.cbm_reader import read_cbm
 from oracle.oracle import OracleModel
 
@@ -267,3 +268,100 @@ def test_kernel_times_are_read_without_waiting_for_other_streams():
         graph.replay()
         torch.cuda.synchronize()
         assert bool((ones == 2.0 + i).all())
+
+
+def _model_of_buckets(rng, buckets, cats, trees, depth, dim, borders_of_first):
+    """Every one of `buckets` columns is split on, the last `cats` of them one-hot; trees of different depths."""
+    floats = buckets - cats
+    hashes = rng.integers(-2**31, 2**31, size=(cats, 5), dtype=np.int64).astype(np.int32)
+    columns = list(rng.permutation(buckets)) + [0] * (borders_of_first if borders_of_first > 1 else 0)
+    tree_list = []
+    for t in range(trees):
+        size = depth if len(columns) > 0 or t % 5 else int(rng.integers(0, depth + 1))
+        splits = []
+        for _ in range(size):
+            c = int(columns.pop() if columns else rng.integers(0, buckets))
+            splits.append(("float", c, float(np.float32(rng.normal()))) if c < floats
+                          else ("onehot", c - floats, int(rng.choice(hashes[c - floats]))))
+        tree_list.append((splits, rng.normal(size=dim << size)))
+    assert not columns
+    model = mb.build_oblivious([mb.float_feature(f) for f in range(floats)], [mb.cat_feature(i, floats + i) for i in range(cats)],
+                               dim, tree_list, scale=0.5, bias=rng.normal(size=dim))
+    return model, hashes
+
+
+@pytest.mark.parametrize("buckets,cats,trees,depth,dim,first,switch,kernel", [
+    (400, 2, 301, 8, 1, 1, "", "EvalObliviousRowTileKernel"),
+    (230, 0, 203, 6, 1, 1, "", "EvalObliviousRowTileKernel"),          # eight waves
+    (560, 0, 117, 8, 1, 200, "", "EvalObliviousRowTileKernel"),        # a bucket of more than 127 values
+    (330, 0, 150, 8, 3, 1, "", "EvalObliviousRowTileKernel"),
+    (260, 3, 90, 6, 10, 1, "", "EvalObliviousRowTileKernel"),
+    (300, 3, 170, 8, 1, 200, "ROW_TILE", "EvalObliviousTileKernel"),
+    (500, 3, 333, 8, 1, 1, "ROW_TILE", "EvalObliviousTileKernel"),
+    (300, 0, 77, 4, 5, 1, "ROW_TILE", "EvalObliviousTileKernel"),
+    (700, 10, 201, 8, 1, 1, "", "EvalObliviousPairTileKernel"),        # a last tree without a partner
+    (1000, 0, 250, 6, 1, 1, "", "EvalObliviousPairTileKernel"),
+    (700, 10, 205, 8, 1, 1, "PAIR_TILE", "EvalObliviousHalfTileKernel"),
+    (1150, 0, 303, 8, 1, 1, "", "EvalObliviousQuadTileKernel"),        # three trees behind the last four
+    (1150, 5, 250, 6, 1, 1, "", "EvalObliviousQuadTileKernel"),
+    (2100, 5, 420, 6, 1, 1, "", "EvalObliviousQuadTileKernel"),        # four waves
+    (900, 0, 150, 7, 2, 1, "", "EvalObliviousKernel"),                 # one pass in tree order
+])
+def test_wide_models_round_alike_at_every_batch_size(buckets, cats, trees, depth, dim, first, switch, kernel, monkeypatch):
+    """Models that the register kernels do not take: the small kernels add a document's trees in the order of the kernel
+    that takes larger batches, so its value is the same bits whatever came with it."""
+    import torch
+
+    if switch:
+        monkeypatch.setenv("CATBOOST_AMD_" + switch, "0")
+    rng = np.random.default_rng(buckets)
+    model, hashes = _model_of_buckets(rng, buckets, cats, trees, depth, dim, first)
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    docs = 17_000
+    assert ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"] == kernel
+    x = rng.normal(size=(docs, buckets)).astype(np.float32)
+    for i in range(cats):
+        x[:, buckets - cats + i] = rng.choice(hashes[i], size=docs).view(np.float32)
+    flat = torch.from_numpy(x).to("cuda:0")
+    feats = ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), flat.shape[1])
+    expected = torch.zeros(docs * dim, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.eval_data(feats, docs, expected.data_ptr())
+    sample = rng.choice(docs, size=500, replace=False)
+    np.testing.assert_allclose(expected.cpu().numpy().reshape(docs, dim)[sample], OracleModel(model).calc(x[sample]).reshape(-1, dim),
+                               rtol=1e-9, atol=1e-12)
+    small = set()
+    for n in (1, 33, 700, 1500, 4001):
+        small.add(ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, n)["evaluate"].split("<")[0])
+        out = torch.full((n * dim,), -3.0, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        ev.eval_data(feats, n, out.data_ptr())
+        assert torch.equal(out, expected[:n * dim]), n
+    assert {"FewDocumentsKernel", "SmallBatchKernel"} <= small, small
+
+
+def test_fewer_trees_than_waves_round_alike(monkeypatch):
+    import torch
+
+    monkeypatch.setenv("CATBOOST_AMD_REG_KERNEL", "0")
+    rng = np.random.default_rng(5)
+    for trees in (1, 2, 3, 5, 7):
+        g = cb.ModelCalcer()
+        g.load_from_dict(mb.build_oblivious([mb.float_feature(f) for f in range(60)], [], 1, [
+            ([("float", int(f), float(np.float32(rng.normal()))) for f in rng.choice(60, size=8, replace=False)],
+             rng.normal(size=256)) for _ in range(trees)]))
+        g.enable_gpu_evaluation(0)
+        ev = g.evaluator()
+        assert ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, 17_000)["evaluate"] == "EvalObliviousRowTileKernel"
+        x = torch.from_numpy(rng.normal(size=(17_000, 60)).astype(np.float32)).to("cuda:0")
+        feats = ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), 60)
+        out = torch.zeros(17_000, dtype=torch.float64, device="cuda:0")
+        part = torch.zeros(900, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        ev.eval_data(feats, 17_000, out.data_ptr())
+        for n in (1, 900):
+            ev.eval_data(feats, n, part.data_ptr())
+            assert torch.equal(part[:n], out[:n])
