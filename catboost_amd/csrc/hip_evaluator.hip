@@ -504,7 +504,7 @@ constexpr size_t kMaxTileLdsBytes = 160 * 1024;
 // 39 against 37). FewDocumentsKernel against SmallBatchKernel: 512 documents 18 against 21 us, 1024 24 against 21.
 constexpr size_t kSmallBatchDocs = 16384;
 constexpr size_t kFewDocs = 640;
-// host calls read features of at most so many bytes from pinned memory
+// ... of host calls, whose features are at most so many bytes: more go through the pipeline of chunks
 constexpr size_t kSmallHostBytes = size_t(16) << 20;
 
 // Workgroups wanted of a leaf index launch: 200 000 documents * 1000 trees (782 blocks, 2 workgroups per CU) take 180 us as
@@ -1455,6 +1455,10 @@ struct THipEvaluator::TImpl {
     size_t FewLdsBytes() const {
         return (static_cast<size_t>(SmallCellCount) + 1) / 2 * 8 +
                static_cast<size_t>(SmallSliceCount()) * (SmallSliceTrees + 2) * SmallDims() * 8;
+    }
+    // of the batches that TakesSmallBatchKernel lets through
+    bool TakesFewDocumentsKernel(size_t docCount) const {
+        return docCount * SmallPasses() <= kFewDocs && FewLdsBytes() <= kMaxTileLdsBytes;
     }
 
     // Staging of the calls that own their buffers (CalcDevice and the host entry points): a call borrows a
@@ -3471,7 +3475,7 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
         launch(kernel, (docCount + dev::kSmallDocs - 1) / dev::kSmallDocs, dev::kSmallThreads, m.SmallLdsBytes());
     };
     const bool shallow = m.MaxDepth <= 6;
-    if (docCount * passes <= kFewDocs && m.FewLdsBytes() <= kMaxTileLdsBytes) {
+    if (m.TakesFewDocumentsKernel(docCount)) {
         if (dims == 1) {
             shallow ? launchFew(dev::FewDocumentsKernel<6, 1>) : launchFew(dev::FewDocumentsKernel<8, 1>);
         } else if (dims == 2) {
@@ -3547,7 +3551,7 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
         return std::string("fused=") + m.FusedKernelName;
     }
     if (TakesSmallBatchKernel(docCount, 0, TreeCount)) {
-        const bool few = docCount * m.SmallPasses() <= kFewDocs && m.FewLdsBytes() <= kMaxTileLdsBytes;
+        const bool few = m.TakesFewDocumentsKernel(docCount);
         return std::string("binarize=none;evaluate=") + (few ? "FewDocumentsKernel<" : "SmallBatchKernel<") + std::to_string(m.MaxDepth <= 6 ? 6 : 8) + ", " + std::to_string(m.SmallDims()) +
                ">, " + std::to_string(m.SmallSliceCount()) + " slices of the trees";
     }
@@ -3961,11 +3965,40 @@ static void RunPredictionChunk(THipEvaluator& ev, THipEvaluator::TImpl::THostCon
     HIP_CHECK(hipEventRecord(slot.Ev[3], s));
 }
 
-// A small batch whose features are in the context's pinned memory: the kernel reads them there and writes the results to
-// pinned memory, so that nothing is copied by a command of its own.
+// Whether the features of a small host batch go to device memory before the launch, instead of being read from pinned memory
+// by the kernel. Rows: the kernel reads them once per pass over the dimensions, so a copy (some 20 us) pays when the
+// passes behind the first would move much. Columns: one document's values, or sixteen documents' of a column, are a request
+// over PCIe each, so it pays soon. Whole call, 100 columns, read by the kernel and copied: rows, one dimension, 5000
+// documents 98 and 117 us; ten dimensions (three passes), 2048 documents 66 and 82, 5000 195 and 157. Columns, 128 documents
+// 30 and 37, 512 61 and 45; 1024 (SmallBatchKernel) 50 and 56, 5000 162 and 112; 600 columns, 512 documents 265 and 83.
+static bool CopiesSmallHostBatch(const THipEvaluator::TImpl& m, bool columns, size_t docCount) {
+    const size_t values = docCount * m.SmallCellCount;
+    if (columns) {
+        return values > (m.TakesFewDocumentsKernel(docCount) ? size_t(24) << 10 : size_t(144) << 10);
+    }
+    return values * (m.SmallPasses() - 1) * 4 > (size_t(5) << 19);
+}
+
+// A small batch whose features (`floatCount` and `catCount` values) are in the context's pinned memory; the results come to
+// pinned memory, too.
 static void CalcSmallHostBatch(THipEvaluator& ev, THipEvaluator::TImpl& m, THipEvaluator::TImpl::THostContext& ctx,
-                               const TFeatureBatch& batch, size_t docCount, int predictionType, double* results) {
+                               TFeatureBatch batch, size_t floatCount, size_t catCount, size_t docCount, int predictionType,
+                               double* results) {
     THipEvaluator::TImpl::THostSlot& slot = ctx.Slots[0];
+    if (CopiesSmallHostBatch(m, batch.Layout == TFeatureBatch::FlatColumns, docCount)) {
+        const auto toDevice = [&](auto& stage, auto& pinned, size_t count) {
+            stage.Reserve(std::max<size_t>(1, count));
+            if (count) {
+                HIP_CHECK(hipMemcpyAsync(stage.Get(), pinned.Get(), count * 4, hipMemcpyHostToDevice, ctx.Stream));
+            }
+        };
+        toDevice(slot.StageFloats, slot.PinnedFloats, floatCount);
+        batch.Floats = slot.StageFloats.Get();
+        if (batch.Cats != nullptr) {
+            toDevice(slot.StageCats, slot.PinnedCats, catCount);
+            batch.Cats = slot.StageCats.Get();
+        }
+    }
     const size_t dim = static_cast<size_t>(m.Dim);
     const size_t outDim = predictionType == dev::kPredClass ? 1 : dim;
     const bool raw = predictionType == dev::kPredRaw;
@@ -4018,7 +4051,7 @@ void THipEvaluator::CalcHostRows(const float* const* rows, size_t rowLen, bool f
             batch.Cats = slot.PinnedCats.Get();
             batch.CatStride = needCats;
         }
-        CalcSmallHostBatch(*this, m, *ctx, batch, docCount, predictionType, results);
+        CalcSmallHostBatch(*this, m, *ctx, batch, docCount * needFloats, docCount * needCats, docCount, predictionType, results);
         SetLastSmallTimes(&*ctx);
         return;
     }
@@ -4074,12 +4107,14 @@ void THipEvaluator::CalcHostColumns(const float* const* columns, size_t columnCo
     if (TakesSmallBatchKernel(docCount, treeStart, treeEnd) && docCount * need * 4 <= kSmallHostBytes) {
         TImpl::THostSlot& slot = ctx->Slots[0];
         slot.PinnedFloats.Reserve(std::max<size_t>(1, docCount * need));
-        CopyColumns(columns, 0, docCount, 0, need, slot.PinnedFloats.Get());
+        float* dst = slot.PinnedFloats.Get();
+        ParallelCopy(need, need * docCount * sizeof(float),
+                     [=](size_t first, size_t last) { CopyColumns(columns, 0, docCount, first, last, dst); });
         TFeatureBatch batch;
         batch.Layout = TFeatureBatch::FlatColumns;
         batch.Floats = slot.PinnedFloats.Get();
         batch.Stride = docCount;
-        CalcSmallHostBatch(*this, m, *ctx, batch, docCount, predictionType, results);
+        CalcSmallHostBatch(*this, m, *ctx, batch, docCount * need, 0, docCount, predictionType, results);
         SetLastSmallTimes(&*ctx);
         return;
     }

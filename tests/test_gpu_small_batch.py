@@ -365,3 +365,36 @@ def test_fewer_trees_than_waves_round_alike(monkeypatch):
         for n in (1, 900):
             ev.eval_data(feats, n, part.data_ptr())
             assert torch.equal(part[:n], out[:n])
+
+
+@pytest.mark.parametrize("n_float,n_cat,dim,docs", [
+    (100, 0, 1, (245, 246, 600, 1474, 1475, 5000)),  # columns: 24 K values of few documents, 144 K of more
+    (300, 0, 2, (40, 82, 700)),
+    (90, 10, 10, (60, 213, 700, 2500, 5461)),        # three passes: rows beyond 2.5 MB of repeated reads
+])
+def test_host_batches_read_in_place_and_copied(n_float, n_cat, dim, docs):
+    """Small host batches on either side of the sizes from which the features are copied to the device first: the bits
+    of the device call, rows, columns and split rows."""
+    import torch
+
+    rng = np.random.default_rng(n_float)
+    model, hashes = _model_of_buckets(rng, n_float + n_cat, n_cat, 200, 6, dim, 1)
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    for n in docs + docs[:1]:
+        x = rng.normal(size=(n, n_float + n_cat)).astype(np.float32)
+        for i in range(n_cat):
+            x[:, n_float + i] = rng.choice(hashes[i], size=n).view(np.float32)
+        assert "slices" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, n)["evaluate"]
+        flat = torch.from_numpy(x).to("cuda:0")
+        out = torch.zeros(n * dim, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), flat.shape[1]), n, out.data_ptr())
+        expected = out.cpu().numpy()
+        np.testing.assert_allclose(expected, OracleModel(model).calc(x), rtol=1e-9, atol=1e-12)
+        np.testing.assert_array_equal(g.calc_flat(x), expected)
+        np.testing.assert_array_equal(g.calc_flat_transposed(np.ascontiguousarray(x.T)), expected)
+        floats, cats = np.ascontiguousarray(x[:, :n_float]), np.ascontiguousarray(x[:, n_float:]).view(np.int32)
+        np.testing.assert_array_equal(g.calc_hashed(floats, cats), expected)
