@@ -36,3 +36,27 @@ def test_projections_of_many_buckets(monkeypatch, tile, copies, wide):
     for docs in (1, 257, 5000):
         floats, cats = ctr_models.random_documents(model, known, docs, 3 + docs)
         np.testing.assert_array_equal(g.quantize_hashed(floats, cats), o.binarize(floats, cats, layout="split"))
+
+
+def test_large_tables_are_built_side_by_side():
+    """Tables of 20 000 further hashes each, so that the projections' tables are made by several host threads."""
+    model, known = ctr_models.random_ctr_model(22, n_cat=6, n_bases=15, n_trees=30)
+    rng = np.random.default_rng(22)
+    for table in model["ctr_tables"]:
+        index = table["index_hash_raw"].view(np.dtype([("hash", "<u8"), ("row", "<u4")]))
+        index = np.sort(index[index["hash"] != np.uint64(ctr_models.MASK64)], order="row")
+        rows = table["ctr_blob"].reshape(len(index), -1)
+        assert (index["row"] == np.arange(len(index))).all()
+        more = rng.integers(0, 2**63, size=20_000, dtype=np.uint64)
+        table["index_hash_raw"] = ctr_models.build_index_hash([int(h) for h in np.unique(np.concatenate([index["hash"], more]))])
+        order = np.argsort(np.argsort(np.concatenate([index["hash"], more])))
+        blob = np.concatenate([rows, rows[rng.integers(0, len(rows), size=len(more))]])
+        placed = np.empty_like(blob)
+        placed[order] = blob
+        table["ctr_blob"] = placed.ravel().copy()
+    data = write_cbm(model)
+    o, g = OracleModel(read_cbm(data)), cb.ModelCalcer(buffer=data)
+    floats, cats = ctr_models.random_documents(model, known, 3000, 5)
+    bins = g.quantize_hashed(floats, cats)
+    np.testing.assert_array_equal(bins, o.binarize(floats, cats, layout="split"))
+    np.testing.assert_allclose(g.calc_hashed(floats, cats), o.calc(floats, cats, layout="split"), rtol=1e-9, atol=1e-12)
