@@ -1,7 +1,7 @@
 """Seeded sweep over random model shapes on the GPU: the library against the oracle, through the C ABI.
 
 Each seed draws a model (oblivious, the same converted to non-symmetric, or one with CTR features of every
-kind), a document count around the block sizes, and the switches that pick between kernels of equal
+kind), a document count around the block sizes or beyond the smallest batches, and the switches that pick between kernels of equal
 results; bins and leaf indexes must be equal, predictions within 1e-9 rel / 1e-12 abs. The default run
 takes a few seconds; CATBOOST_AMD_SWEEP_SEEDS=first:count widens it (tens of thousands of seeds fit in
 minutes).
@@ -49,6 +49,8 @@ def _tree_model_case(seed, rng, asymmetric):
     max_depth = int(rng.choice([1, 3, 6, 8, 10, 12]))
     many = bool(rng.integers(0, 2))
     docs = int(rng.choice([1, 2, 63, 64, 65, 255, 256, 257, 1000, 3333, 9000]))
+    if not asymmetric and rng.integers(0, 6) == 0:
+        docs = 16_641  # beyond the one-launch kernels of small batches: the register kernels in slices of the trees
     trees = min(trees, max(1, 40000 // n_float))
     tag = "seed %d dim %d floats %d cats %d trees %d depth<=%d many borders %s docs %d non-symmetric %s" % (
         seed, dim, n_float, n_cat, trees, max_depth, many, docs, asymmetric)
@@ -99,8 +101,8 @@ def test_random_model_shapes(monkeypatch, capsys):
         monkeypatch.setenv("CATBOOST_AMD_SMALL_BATCH", str(int(rng.integers(0, 2))))
         monkeypatch.setenv("CATBOOST_AMD_REG_SPLIT", str(int(rng.integers(0, 2))))
         monkeypatch.setenv("CATBOOST_AMD_ROW_TILE", str(int(rng.integers(0, 2))))
-        # the shape of the non-symmetric LDS kernel: chosen by the model, or one of the five
-        monkeypatch.setenv("CATBOOST_AMD_NS_WAVES", str(int(rng.choice([0, 4, 6, 8, 12, 16]))))
+        # the shape of the non-symmetric LDS kernel: chosen by the model, or among those of so many waves
+        monkeypatch.setenv("CATBOOST_AMD_NS_WAVES", str(int(rng.choice([0, 4, 6, 8, 10, 11, 12, 16]))))
         if kind == 2:
             _ctr_model_case(seed, rng, monkeypatch)
         else:
