@@ -534,13 +534,22 @@ uint32_t NsLdsDims(int dim) {
 
 // Few buckets leave LDS for larger regions (fewer units, larger trees) at a given number of waves, and 249 to 312 buckets
 // for ten or eleven waves where trees of more than 1536 entries used to leave eight. Evaluate launch, 1M documents, trees
-// of depth 10: 500 trees over 100 features 1224 us with eight waves of 2048 entries, 1103 with twelve of 1536, 1061 with
-// twelve of 2048, 1025 with sixteen of 2048; 500 over 300 features 1285 with eight, 1207 with ten, 1199 with eleven of 1792,
-// 1150 to 1181 with twelve of 1536. The speeds of the larger regions lie below what they measured, as their units differ.
+// of depth 10: 500 trees over 100 features 1250 us with eight waves of 2048 entries, 1131 with twelve of 1536, 1062 with
+// twelve of 2048, 1027 with sixteen of 2048; 500 over 300 features 1298 with eight, 1223 with ten, 1201 with eleven of 1792,
+// 1196 with twelve of 1536; 300 of three dimensions over 100 features 975 with eight, 832 with twelve of 2048, 812 with
+// sixteen of 1536.
+// The model's shape is the one with the least steps / speed. Steps (a unit takes as many as its tallest tree) per time,
+// relative to eight waves, measured over eleven models of depth 6 to 10, 20 to 300 features, one and three dimensions:
+//   16 x 1024 1.33 .. 1.41   16 x 1536 1.23 .. 1.40   16 x 2048 1.18 .. 1.25   12 x 1536 1.14 .. 1.32
+//   12 x 2048 1.12 .. 1.19   11 x 1792 1.11 .. 1.18   10 x 2048 1.05 .. 1.09
+// (a region that is fuller takes longer per step, so a shape's speed falls as its units shrink). The figures below, set on
+// two models, differ from these by up to 0.1; they gave nine of the eleven models the fastest shape and one (three
+// dimensions over 100 features) the second, 2 % behind. The last one has 20 features: there two workgroups of eight waves
+// share a CU (870 us against 999 with the 16 x 2048 that is taken), which the rule does not know.
 struct TNsLdsShape {
     uint32_t Waves;
     uint32_t Entries;
-    double Speed;  // steps of a unit per unit of time, relative to the 8-wave shape
+    double Speed;  // steps per unit of time, relative to the 8-wave shape
 };
 constexpr TNsLdsShape kNsLdsShapes[] = {{16, 1024, 1.45}, {16, 1536, 1.37}, {16, 2048, 1.35}, {12, 1536, 1.26}, {12, 2048, 1.2},
                                         {11, 1792, 1.08}, {10, 2048, 1.04}, {8, 2048, 1.0},   {6, 2048, 0.8},   {4, 2048, 0.55}};

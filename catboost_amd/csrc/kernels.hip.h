@@ -808,10 +808,11 @@ __device__ __forceinline__ void SmallStamp(ulonglong2* stamps, unsigned long lon
     stamps[blockIdx.y * gridDim.x + blockIdx.x] = make_ulonglong2(began, wall_clock64());
 }
 
+// (The second argument is SmallBatchKernel's number of documents; here the grid has it.)
 // grid = (documents, ceil(dim / DIMS)), block = whole waves, at most kFewThreads; dynamic LDS = CellCount * 4 rounded up
 // to 8 + DIMS * SliceCount * (SliceTrees + 2) * 8 bytes.
 template <int DEPTH, int DIMS>
-__global__ __launch_bounds__(kFewThreads) void FewDocumentsKernel(TSmallSource src, uint32_t docCount, TSmallTables tab,
+__global__ __launch_bounds__(kFewThreads) void FewDocumentsKernel(TSmallSource src, uint32_t, TSmallTables tab,
                                                                   double* __restrict__ out, ulonglong2* __restrict__ stamps) {
     extern __shared__ uint32_t sSmall[];
     const unsigned long long began = wall_clock64();
