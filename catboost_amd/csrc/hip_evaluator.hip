@@ -510,8 +510,8 @@ constexpr size_t kFewDocs = 640;
 // ... of host calls, whose features are at most so many bytes: more go through the pipeline of chunks
 constexpr size_t kSmallHostBytes = size_t(16) << 20;
 
-// Workgroups wanted of a leaf index launch: 200 000 documents * 1000 trees (782 blocks, 2 workgroups per CU) take 180 us as
-// 782 workgroups, 165 as 2346, 199 as 4692 (shorter runs of a row, the bins read more often).
+// Workgroups wanted of a leaf index launch: 200 000 documents * 1000 trees (782 blocks, 2 workgroups per CU) take 225 us as
+// 782 workgroups, 200 as 2346, 216 as 4692 (shorter runs of a row, the bins read more often), launches back to back.
 constexpr size_t kLeafIndexWorkgroups = 2048;
 
 // LDS of the tile kernel without leaf regions: the bins of 256 documents and the accumulator

@@ -463,8 +463,8 @@ __device__ __forceinline__ uint64_t CtrHashOfCat(uint32_t v) {
 // The bins of a lane's four documents ({lane, lane + 64, lane + 128, lane + 192} of the block) in the buckets of CTR
 // features. What bounds it is the gathers of table entries (a line of L2 each for tables beyond the L1): one 16-byte
 // read finds and answers a lookup of up to eight buckets, where a table per CTR feature, its rows and a division and a
-// count of borders per feature used to take some ten times as long (1M documents, 16 categorical columns, 24 projections
-// with 96 CTR features: 620 us before).
+// count of borders per feature took five times as long (1M documents, 16 categorical columns, 24 projections with 96 CTR
+// features: 620 us then, 125 now).
 // grid = (document blocks, shares of the groups), 4 waves per workgroup, each wave a run of the share's groups.
 // TILE: the block's hashed categorical values are staged once per workgroup into LDS ([column][document]); without
 // it (more than kCtrMaxTileColumns columns) they are read from the batch where a projection needs them.
@@ -3079,7 +3079,8 @@ __global__ __launch_bounds__(256) void LeafIndexesKernel(const uint8_t* __restri
 // a document, 16 bytes a thread. The 64 indexes are those that fill whole 128-byte lines of the output, up to 31 trees
 // behind the group, which the ring still holds: rows of 4 * trees bytes start anywhere in a line, and lines written in two
 // parts cost the memory twice. 200 000 documents * 1000 trees of depth 6 over 100 features: 466 us with a workgroup per
-// block and 4-byte stores, 227 with shares and 16-byte stores, 165 with whole lines (4.85 TB/s).
+// block and 4-byte stores, 227 with shares and 16-byte stores, 165 with whole lines, one after another on one box; traced in
+// whole calls 183 us (4.4 TB/s), back to back 200.
 // A share is some groups of 64 trees: the grid is blocks * shares, so that a batch of a few hundred blocks still fills
 // the chip a few times over (one workgroup per block left a last generation nearly empty).
 // GROUP = 32 is for tiles that leave less than 33 KB of LDS (509 to 576 buckets): half the trees per group, a line of a

@@ -174,7 +174,8 @@ bool CbHipSynchronize(CbHipEvaluatorHandle* evaluator, void* hipStream);
  * (summed over its chunks), measured with hipEvents. A call that ran as one fused launch reports the
  * whole launch as evalMs and 0 as binarizeMs, whatever the entry point; so does a small batch of an oblivious
  * model that ran as one launch, whose evalMs is the time from its first workgroup's start to its last one's
- * end on the device's clock. The call only reads what was measured: it waits for no stream and no other call. */
+ * end on the device's clock, fetched by this call. It waits for no stream of the caller's and no other call, and may
+ * be made while a stream is being captured. */
 bool CbHipLastKernelTimes(CbHipEvaluatorHandle* evaluator, float* binarizeMs, float* evalMs);
 
 /* Which kernels a whole-model CbHipEvalData (or host entry point) call on docCount documents of `layout`
