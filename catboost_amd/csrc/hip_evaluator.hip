@@ -4116,7 +4116,9 @@ void THipEvaluator::CalcHostRows(const float* const* rows, size_t rowLen, bool f
     if (TakesSmallBatchKernel(docCount, treeStart, treeEnd) && docCount * (needFloats + needCats) * 4 <= kSmallHostBytes) {
         TImpl::THostSlot& slot = ctx->Slots[0];
         slot.PinnedFloats.Reserve(std::max<size_t>(1, docCount * needFloats));
-        GatherRows(rows, docCount, needFloats, slot.PinnedFloats.Get());
+        if (needFloats) {  // a model of categorical features may come without float rows
+            GatherRows(rows, docCount, needFloats, slot.PinnedFloats.Get());
+        }
         TFeatureBatch batch;
         batch.Layout = flat ? TFeatureBatch::FlatRows : TFeatureBatch::SplitRows;
         batch.Floats = slot.PinnedFloats.Get();

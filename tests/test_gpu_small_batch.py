@@ -398,3 +398,17 @@ def test_host_batches_read_in_place_and_copied(n_float, n_cat, dim, docs):
         np.testing.assert_array_equal(g.calc_flat_transposed(np.ascontiguousarray(x.T)), expected)
         floats, cats = np.ascontiguousarray(x[:, :n_float]), np.ascontiguousarray(x[:, n_float:]).view(np.int32)
         np.testing.assert_array_equal(g.calc_hashed(floats, cats), expected)
+
+
+def test_categorical_features_without_float_rows():
+    """One-hot features alone: the float rows may be a null pointer, in small batches as in large ones."""
+    rng = np.random.default_rng(3)
+    model, hashes = _model_of_buckets(rng, 12, 12, 80, 6, 1, 1)
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    oracle = OracleModel(model)
+    for n in (1, 700, 17_000):
+        cats = np.stack([rng.choice(h, size=n) for h in hashes], axis=1)
+        np.testing.assert_allclose(g.calc_hashed(np.zeros((n, 0), np.float32), cats),
+                                   oracle.calc(np.zeros((n, 0), np.float32), cats, layout="split"), rtol=1e-9, atol=1e-12)
