@@ -3439,7 +3439,8 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
 
 uint32_t THipEvaluator::TreeSlicesFor(size_t docCount) const {
     const TImpl& m = *Impl;
-    if (!m.RegKernelUsable || !m.SmallBatchSlices || docCount == 0) {
+    // (a slice's results are addressed with 32 bits, as a launch's are: models of more than 2047 dimensions can pass that)
+    if (!m.RegKernelUsable || !m.SmallBatchSlices || docCount == 0 || docCount >= (size_t(1) << 29) / m.Dim) {
         return 1;
     }
     // Workgroups of a plain launch; below one per CU the launch lasts as long as one wave's walk through the

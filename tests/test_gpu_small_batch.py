@@ -412,3 +412,27 @@ def test_categorical_features_without_float_rows():
         cats = np.stack([rng.choice(h, size=n) for h in hashes], axis=1)
         np.testing.assert_allclose(g.calc_hashed(np.zeros((n, 0), np.float32), cats),
                                    oracle.calc(np.zeros((n, 0), np.float32), cats, layout="split"), rtol=1e-9, atol=1e-12)
+
+
+def test_results_of_a_batch_that_a_slice_cannot_address():
+    """262 000 documents of 2080 dimensions: more result bytes than a launch addresses, so the trees are not sliced."""
+    import torch
+
+    rng = np.random.default_rng(9)
+    dim, docs = 2080, 262_000
+    model, _ = _model_of_buckets(rng, 4, 0, 70, 1, dim, 1)
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    assert "slices" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs - 6000)["evaluate"]
+    assert "slices" not in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"]
+    x = torch.randn(docs, 4, device="cuda:0")
+    out = torch.full((docs * dim + 64,), -3.0, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), 4), docs, out.data_ptr())
+    assert bool((out[docs * dim:] == -3.0).all())
+    out = out[:docs * dim].reshape(docs, dim)
+    sample = np.concatenate([rng.choice(docs, size=100, replace=False), [0, docs - 1]])
+    np.testing.assert_allclose(out[torch.from_numpy(sample).to("cuda:0")].cpu().numpy(),
+                               OracleModel(model).calc(x.cpu().numpy()[sample]).reshape(-1, dim), rtol=1e-9, atol=1e-12)
