@@ -185,9 +185,9 @@ bool CbHipDescribeKernels(CbHipEvaluatorHandle* evaluator, int layout, size_t do
 
 /* Small batches are spread over the GPU by cutting the trees into slices that run side by side.
  * Models of the register kernels (up to 224 buckets): a slice adds its leaves in tree order and the slices' sums
- * are then added in slice order. The result is the same for every call and every batch size below 256 workgroups
- * (262 144 documents, 524 288 with at most 96 buckets) and 4 GiB of results, and differs in the last bits (inside
- * 1e-9 relative) from the single pass in tree order that larger batches, CbHipEvalQuantized and the CPU evaluator make
+ * are then added in slice order. The result is the same for every call and every batch of up to 261 120 documents
+ * (and 4 GiB of results), and differs in the last bits (inside 1e-9 relative) from the single pass in tree order
+ * that larger batches, CbHipEvalQuantized and the CPU evaluator make
  * (cpu/evaluator_impl.cpp:362-460; single document: c_api.cpp:383-384). Wider oblivious models: the slices are the
  * partial sums that the kernels of larger batches and of CbHipEvalQuantized add, so the result of a whole-model
  * call is the same for every batch size.
