@@ -64,7 +64,7 @@ def end_to_end_c_abi(model, info, docs):
 
 def host_threads():
     """Worker threads for the CPU legs: every host core, unless the machine's environment caps worker pools
-    (OMP_NUM_THREADS: a GPU box gives one GPU's job a share of its cores)."""
+    (OMP_NUM_THREADS: a job with one GPU of several has a share of the cores)."""
     cap = os.environ.get("OMP_NUM_THREADS", "")
     cores = os.cpu_count() or 1
     return max(1, min(cores, int(cap))) if cap.isdigit() else cores
