@@ -53,9 +53,11 @@ public:
     size_t QuantizedBytes(size_t docCount) const;
 
     // ---- device-resident data; `stream` is a hipStream_t (nullptr = the evaluator's own stream)
-    void QuantizeDevice(const TFeatureBatch& batch, size_t docCount, uint8_t* bins, void* stream);
+    // `end`: an event that the last launch takes along when it can (the caller records it otherwise)
+    struct TStageEnd;
+    void QuantizeDevice(const TFeatureBatch& batch, size_t docCount, uint8_t* bins, void* stream, TStageEnd* end = nullptr);
     void EvalQuantizedDevice(const uint8_t* bins, size_t docCount, size_t treeStart, size_t treeEnd,
-                             double* results, void* stream);
+                             double* results, void* stream, TStageEnd* end = nullptr);
     // Small batches on the register-resident kernels: the trees are cut into TreeSlicesFor(docCount) slices that
     // run on workgroups of their own and store raw sums into `partials` (TreeSliceScratchDoubles(docCount)
     // doubles, the caller's), which a second kernel adds up in slice order. One slice: the plain launch. The
@@ -63,12 +65,13 @@ public:
     // trees (within the 1e-9 relative bar, the same for every call).
     uint32_t TreeSlicesFor(size_t docCount) const;
     size_t TreeSliceScratchDoubles(size_t docCount) const;
-    void EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCount, double* results, double* partials, void* stream);
+    void EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCount, double* results, double* partials, void* stream,
+                                   TStageEnd* end = nullptr);
     // binarize + evaluate in one launch of a fused kernel, the bins in registers only; false (and nothing
     // launched) when the model, the batch layout or the tree range has no fused kernel
     // (anyBatchSize: also below the batch size from which the fused launch is the faster one)
     bool EvalRowsFusedDevice(const TFeatureBatch& batch, size_t docCount, size_t treeStart, size_t treeEnd,
-                             double* results, void* stream, bool anyBatchSize = false);
+                             double* results, void* stream, bool anyBatchSize = false, TStageEnd* end = nullptr);
     // index of the fused kernel tables that such a call would use (0 flat rows, 1 split rows), -1 when it takes
     // the two launches: the one test that EvalRowsFusedDevice, the host pipeline and DescribeKernels share
     int FusedLayoutFor(int layout, size_t stride, size_t docCount, size_t treeStart, size_t treeEnd, bool anyBatchSize) const;
