@@ -564,6 +564,9 @@ constexpr size_t kSmallHostBytes = size_t(16) << 20;
 // 782 workgroups, 200 as 2346, 216 as 4692 (shorter runs of a row, the bins read more often), launches back to back.
 constexpr size_t kLeafIndexWorkgroups = 2048;
 
+// The cache between the L2s and HBM. What is larger is not found there by its next reader.
+constexpr size_t kMemorySideCacheBytes = size_t(256) << 20;
+
 // LDS of the tile kernel without leaf regions: the bins of 256 documents and the accumulator
 size_t TileLdsBytes(uint32_t buckets, int dchunk) {
     return ((static_cast<size_t>(buckets) * dev::kDocsPerBlock + 7) & ~size_t(7)) +
@@ -3766,12 +3769,20 @@ void THipEvaluator::LeafIndexesQuantizedDevice(const uint8_t* bins, size_t docCo
         };
         const auto launchGroup = [&](auto group) {
             constexpr int G = decltype(group)::value;
-            if (m.PackedSevenBit && m.MaxDepth <= 6) {
-                launch(dev::LeafIndexesTileKernel<true, 6, G>, G);
-            } else if (m.PackedSevenBit) {
-                launch(dev::LeafIndexesTileKernel<true, 8, G>, G);
+            const auto launchStores = [&](auto stream) {
+                constexpr bool STREAM = decltype(stream)::value;
+                if (m.PackedSevenBit && m.MaxDepth <= 6) {
+                    launch(dev::LeafIndexesTileKernel<true, 6, G, STREAM>, G);
+                } else if (m.PackedSevenBit) {
+                    launch(dev::LeafIndexesTileKernel<true, 8, G, STREAM>, G);
+                } else {
+                    launch(dev::LeafIndexesTileKernel<false, 8, G, STREAM>, G);
+                }
+            };
+            if (docCount * (treeEnd - treeStart) * sizeof(uint32_t) > kMemorySideCacheBytes) {
+                launchStores(std::true_type());
             } else {
-                launch(dev::LeafIndexesTileKernel<false, 8, G>, G);
+                launchStores(std::false_type());
             }
         };
         if (tileLds(dev::kLeafIndexGroup) <= kMaxTileLdsBytes) {

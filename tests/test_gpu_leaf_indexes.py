@@ -114,3 +114,28 @@ def test_leaf_indexes_of_wide_models(buckets, trees, depth, one_hot, docs):
             got = out.cpu().numpy()
             np.testing.assert_array_equal(got[shift:shift + count].reshape(docs, end - begin), expected[:, begin:end])
             assert (got[:shift] == -7).all() and (got[shift + count:] == -7).all()
+
+
+@pytest.mark.parametrize("cfg,trees,docs", [("C1", 200, 336_001), ("C2B", 131, 513_000), ("C2", 416, 161_500)])
+def test_leaf_indexes_larger_than_the_memory_side_cache(cfg, trees, docs):
+    """More than 256 MB of indexes take streaming stores: the same indexes as two calls for halves of the documents."""
+    import torch
+
+    model, info = syn.build_model(cfg, trees=trees)
+    model.enable_gpu_evaluation(0)
+    ev = model.evaluator()
+    x = syn.device_features(info, docs)
+    half = docs // 512 * 256
+    assert docs * trees * 4 > 256 << 20 > (docs - half) * trees * 4
+    pitch = ev.quantized_bytes(256)
+    bins = torch.zeros(ev.quantized_bytes(docs), dtype=torch.uint8, device="cuda:0")
+    out = torch.full((2, docs, trees), -7, dtype=torch.int32, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.quantize(ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), x.shape[1]), docs, bins.data_ptr())
+    ev.leaf_indexes_quantized(bins.data_ptr(), docs, out[0].data_ptr())
+    ev.leaf_indexes_quantized(bins.data_ptr(), half, out[1].data_ptr())
+    ev.leaf_indexes_quantized(bins.data_ptr() + half // 256 * pitch, docs - half, out[1, half:].data_ptr())
+    ev.synchronize()
+    assert torch.equal(out[0], out[1])
+    expected = OracleModel(read_cbm(model.save_to_buffer())).leaf_indexes(x[-700:].cpu().numpy())
+    np.testing.assert_array_equal(out[0, -700:].cpu().numpy(), expected)
