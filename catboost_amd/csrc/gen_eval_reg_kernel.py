@@ -76,7 +76,7 @@ go through the same two LDS buffers as the tree blocks that follow them:
 Additional kernel arguments (104 bytes in all):
   80 floats const float*  88 units const uint32* [BUCKETS / 16 + 1][40] + [16]  96 row stride in bytes uint32
  100 unitCount uint32 (1 .. BUCKETS / 16)
-and argument 0 is unused, argument 16 points at the border table images.
+and argument 0 is the delay of workgroups 256 .. 511 in turns of 4096 cycles, argument 16 points at the border table images.
 
 Usage: gen_eval_reg_kernel.py OUT.s
 """
@@ -622,6 +622,19 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  s_lshl_b32 s25, s96, 8")                # bytes of bins per document block
         e("  s_mul_hi_u32 s31, s24, s25")
         e("  s_mul_i32 s30, s24, s25")
+        # Workgroups 256 .. 511, the second ones of the CUs, start late by argument 0 turns of 4096 cycles: the first
+        # ones' rows then arrive at the full rate and their trees are walked while the second ones' rows arrive,
+        # where both would wait for rows together and walk together.
+        e("  s_sub_u32 s25, s2, 0x100")
+        e("  s_cmp_lt_u32 s25, 0x100")
+        e("  s_cselect_b32 s25, s4, 0")
+        e("%s_late:" % name)
+        e("  s_cmp_eq_u32 s25, 0")
+        e("  s_cbranch_scc1 %s_prompt" % name)
+        e("  s_sleep 64")
+        e("  s_sub_u32 s25, s25, 1")
+        e("  s_branch %s_late" % name)
+        e("%s_prompt:" % name)
         e("  s_add_u32 s32, s4, s30")
         e("  s_addc_u32 s33, s5, s31")
         e("  s_add_u32 s28, s96, -1")
