@@ -91,6 +91,12 @@ SHAPES = [
     (224, 4, 1, 256), (208, 4, 1, 256), (200, 4, 1, 256), (96, 8, 1, 256),
     (224, 4, 1, 64), (208, 4, 1, 64), (200, 4, 1, 64), (128, 4, 1, 64), (96, 8, 1, 64),
     (192, 4, 2, 64), (160, 4, 4, 64), (128, 4, 6, 64),
+    # Fewer buckets: three or four waves per SIMD instead of two; and three dimensions, whose odd one is a piece of eight
+    # bytes per leaf: LDS bounds these kernels, and a fourth dimension of padding is a quarter of its reads. 1M documents,
+    # 1000 trees: three dimensions, 60 buckets 559 -> 446 us, 100 621 -> 506, 120 636 -> 528; seven as 4 + 3 1125 -> 1009,
+    # nine as 6 + 3 1388 -> 1271; two over 70 buckets 367 -> 350, six over 50 812 -> 791. (Of eight waves per workgroup: 30 000
+    # documents 2 to 4 % slower than before. Four dimensions over 48 buckets at four waves: 1 %, not kept.)
+    (80, 4, 2, 64), (104, 4, 3, 64), (176, 4, 3, 64), (56, 4, 6, 64),
     (192, 4, 2, 256), (160, 4, 4, 256), (128, 4, 6, 256),
 ]
 # trees of depth 9 and 10 (1024 leaf rows, one dimension): plain and six-bit forms only
@@ -148,7 +154,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     row_dwords = 32 if mixed or deep else 16      # level table of a tree
     tree_row_bytes = row_dwords * 4
     rows_a, rows_b = 32, 32 + row_dwords  # the two sets of scalar registers holding level tables
-    assert pitch == 1 or pitch % 2 == 0
+    odd = pitch > 1 and pitch % 2 == 1    # the last dimension's values stand alone, eight bytes per leaf
     threads = waves * 64
     row_bytes = threads * 16              # one 16-byte piece per thread of a leaf table copy
     tree_bytes = leaves * pitch * 8
@@ -574,7 +580,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     # (a six-level index sits in bits 2..7 of its byte)
     # (tables of several dimensions hold a tree's values as pieces of two dimensions, each piece an array of
     # 16 bytes per leaf: a wave's 16-byte gathers then spread over all sixteen groups of four LDS banks, which
-    # leaf rows of 32 bytes would not)
+    # leaf rows of 32 bytes would not; an odd last dimension is a piece of eight bytes per leaf)
     e("  s_mov_b32 s23, %d" % ((8 if pitch == 1 else 16) >> max(8 - depth, 0)))
     e("  s_mul_i32 s100, s20, %d" % wave_bytes)  # offset of the wave's share of a tree block
     # one step back: every group of copies steps forward first
@@ -616,12 +622,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     if not fused:
         e("  s_mov_b32 s13, s35")                    # tree blocks of the workgroup behind the slice's
     if fused:
-        fused_binarize()
-    else:
-        # (the level table registers are free until the first tables are loaded)
-        e("  s_lshl_b32 s25, s96, 8")                # bytes of bins per document block
-        e("  s_mul_hi_u32 s31, s24, s25")
-        e("  s_mul_i32 s30, s24, s25")
         # Workgroups 256 .. 511, the second ones of the CUs, start late by argument 0 turns of 4096 cycles: the first
         # ones' rows then arrive at the full rate and their trees are walked while the second ones' rows arrive,
         # where both would wait for rows together and walk together.
@@ -635,6 +635,12 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  s_sub_u32 s25, s25, 1")
         e("  s_branch %s_late" % name)
         e("%s_prompt:" % name)
+        fused_binarize()
+    else:
+        # (the level table registers are free until the first tables are loaded)
+        e("  s_lshl_b32 s25, s96, 8")                # bytes of bins per document block
+        e("  s_mul_hi_u32 s31, s24, s25")
+        e("  s_mul_i32 s30, s24, s25")
         e("  s_add_u32 s32, s4, s30")
         e("  s_addc_u32 s33, s5, s31")
         e("  s_add_u32 s28, s96, -1")
@@ -738,6 +744,8 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  s_lshl_b32 s28, s28, 6")
     e("  s_add_u32 s30, s6, s28")
     e("  s_addc_u32 s31, s7, 0")
+    if odd:
+        e("  s_mov_b32 s24, %d" % (8 >> max(8 - depth, 0)))  # the odd dimension's piece (s24 and s25 are free from here to the epilogue)
     if deep:
         # byte selectors of the two index words (s24 and s25 are free from here to the epilogue)
         e("  s_mov_b32 s24, 0x05010400")
@@ -763,13 +771,13 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 levels_high(rows)
             tree_offset = buf * buf_bytes + i * tree_bytes
 
-            def gather_address(j):
+            def gather_address(j, scale="s23"):
                 if deep:
                     e("  v_mul_u32_u24_sdwa v%d, s23, v%d dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_%d"
                       % (ga0 + j, wd0 + j // 2, j % 2))
                 else:
-                    e("  v_mul_u32_u24_sdwa v%d, s23, v3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_%d"
-                      % (ga0 + j, j))
+                    e("  v_mul_u32_u24_sdwa v%d, %s, v3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_%d"
+                      % (ga0 + j, scale, j))
             if two_sets:
                 # The trees of a block alternate between the two sets of leaf values (a block has an even number
                 # of trees, so the first tree of a block finds the last one's values in the second set). The wait
@@ -793,9 +801,13 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                     if pitch == 1:
                         e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, 0), lv(j, 0) + 1, ga0 + j, tree_offset))
                     else:
-                        for k in range(0, pitch, 2):
+                        for k in range(0, pitch - 1, 2):
                             e("  ds_read_b128 v[%d:%d], v%d offset:%d" % (lv(j, k), lv(j, k) + 3, ga0 + j,
                                                                          tree_offset + (k // 2) * leaves * 16))
+                        if odd:
+                            gather_address(j, "s24")
+                            e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, pitch - 1), lv(j, pitch - 1) + 1, ga0 + j,
+                                                                        tree_offset + (pitch // 2) * leaves * 16))
                 load_rows(rows, buf * block + i + 2)
             # copy of the next tree block into the other buffer, spread over this block's trees
             staged = False

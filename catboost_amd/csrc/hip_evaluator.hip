@@ -243,6 +243,10 @@ constexpr TEvalRegVariant kEvalRegVariants[] = {
     {200, 4, 1, 256, false, false, "cbamd_eval_reg_b200_w4_p1_l256"},
     {208, 4, 1, 256, false, false, "cbamd_eval_reg_b208_w4_p1_l256"},
     {224, 4, 1, 256, false, false, "cbamd_eval_reg_b224_w4_p1_l256"},
+    {80, 4, 2, 64, false, false, "cbamd_eval_reg_b80_w4_p2_l64"},
+    {104, 4, 3, 64, false, false, "cbamd_eval_reg_b104_w4_p3_l64"},
+    {176, 4, 3, 64, false, false, "cbamd_eval_reg_b176_w4_p3_l64"},
+    {56, 4, 6, 64, false, false, "cbamd_eval_reg_b56_w4_p6_l64"},
     {192, 4, 2, 64, false, false, "cbamd_eval_reg_b192_w4_p2_l64"},
     {160, 4, 4, 64, false, false, "cbamd_eval_reg_b160_w4_p4_l64"},
     {128, 4, 6, 64, false, false, "cbamd_eval_reg_b128_w4_p6_l64"},
@@ -258,6 +262,10 @@ constexpr TEvalRegVariant kEvalRegVariants[] = {
     {200, 4, 1, 256, true, false, "cbamd_eval_reg_b200_w4_p1_l256_m"},
     {208, 4, 1, 256, true, false, "cbamd_eval_reg_b208_w4_p1_l256_m"},
     {224, 4, 1, 256, true, false, "cbamd_eval_reg_b224_w4_p1_l256_m"},
+    {80, 4, 2, 64, true, false, "cbamd_eval_reg_b80_w4_p2_l64_m"},
+    {104, 4, 3, 64, true, false, "cbamd_eval_reg_b104_w4_p3_l64_m"},
+    {176, 4, 3, 64, true, false, "cbamd_eval_reg_b176_w4_p3_l64_m"},
+    {56, 4, 6, 64, true, false, "cbamd_eval_reg_b56_w4_p6_l64_m"},
     {192, 4, 2, 64, true, false, "cbamd_eval_reg_b192_w4_p2_l64_m"},
     {160, 4, 4, 64, true, false, "cbamd_eval_reg_b160_w4_p4_l64_m"},
     {128, 4, 6, 64, true, false, "cbamd_eval_reg_b128_w4_p6_l64_m"},
@@ -273,6 +281,10 @@ constexpr TEvalRegVariant kEvalRegVariants[] = {
     {200, 4, 1, 256, false, true, "cbamd_eval_reg_b200_w4_p1_l256_s"},
     {208, 4, 1, 256, false, true, "cbamd_eval_reg_b208_w4_p1_l256_s"},
     {224, 4, 1, 256, false, true, "cbamd_eval_reg_b224_w4_p1_l256_s"},
+    {80, 4, 2, 64, false, true, "cbamd_eval_reg_b80_w4_p2_l64_s"},
+    {104, 4, 3, 64, false, true, "cbamd_eval_reg_b104_w4_p3_l64_s"},
+    {176, 4, 3, 64, false, true, "cbamd_eval_reg_b176_w4_p3_l64_s"},
+    {56, 4, 6, 64, false, true, "cbamd_eval_reg_b56_w4_p6_l64_s"},
     {192, 4, 2, 64, false, true, "cbamd_eval_reg_b192_w4_p2_l64_s"},
     {160, 4, 4, 64, false, true, "cbamd_eval_reg_b160_w4_p4_l64_s"},
     {128, 4, 6, 64, false, true, "cbamd_eval_reg_b128_w4_p6_l64_s"},
@@ -332,16 +344,17 @@ uint32_t RegSliceTrees(uint32_t treeBlock) {
     return std::max(2 * treeBlock, 32u);
 }
 
-// Slices that one workgroup of a sliced launch walks. The chip holds 512 workgroups at a time (two per CU, every variant),
-// and a workgroup pays for its bins, its first tables and its end what about one slice costs: the number with the
-// cheapest sum over the generations is taken (half a slice to two and a half as the price measured the same). A slice
-// per workgroup -> this rule, 1000 trees of depth 8 over 200 features, whole device call: 50 000 documents 99 -> 78 us,
-// 100 000 151 -> 100, 200 000 255 -> 157; 20 000 (no more workgroups than fit) 62 -> 57.
-uint32_t RegSlicesPerGroup(size_t groups, uint32_t slices) {
+// Slices that one workgroup of a sliced launch walks. The chip holds `resident` workgroups at a time (two to four per CU, by
+// the variant's registers and LDS), and a workgroup pays for its bins, its first tables and its end what about one slice
+// costs: the number with the cheapest sum over the generations is taken (half a slice to two and a half as the price
+// measured the same). A slice per workgroup -> this rule, 1000 trees of depth 8 over 200 features, whole device call:
+// 50 000 documents 99 -> 78 us, 100 000 151 -> 100, 200 000 255 -> 157; 20 000 (no more workgroups than fit) 62 -> 57.
+// Two per CU assumed where three fit: 100 003 documents of 500 trees and three dimensions 87.3 us instead of 81.3.
+uint32_t RegSlicesPerGroup(size_t groups, uint32_t slices, size_t resident) {
     uint32_t best = 1;
     size_t bestCost = std::numeric_limits<size_t>::max();
     for (uint32_t k = 1; k <= slices; ++k) {
-        const size_t generations = (groups * ((slices + k - 1) / k) + 511) / 512;
+        const size_t generations = (groups * ((slices + k - 1) / k) + resident - 1) / resident;
         const size_t cost = generations * (k + 1);
         if (cost < bestCost) {
             best = k;
@@ -1522,6 +1535,7 @@ struct THipEvaluator::TImpl {
         uint32_t FirstDim = 0;
         uint32_t StoreDims = 1;
         uint32_t TreeBlock = 16;         // trees per LDS buffer of this kernel
+        uint32_t GroupsPerCu = 1;        // workgroups that a CU holds at a time
         size_t TreeLeafDoubles = 0;      // doubles of a tree in Leaves
         const double* Leaves = nullptr;  // the launch's leaf table
     };
@@ -2447,9 +2461,10 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     for (int d = 0; d < depth; ++d) {
                         modelLeaf |= ((leaf >> d) & 1) << levelOrder[t][d];
                     }
-                    // one-dimensional: a value per leaf; else pieces of two dimensions, 16 bytes per leaf and piece
+                    // pieces of two dimensions, 16 bytes per leaf and piece; an odd last dimension, as one alone: a value per leaf
                     for (size_t k = 0; k < launchPitch && launch * pitch + k < static_cast<size_t>(m.Dim); ++k) {
-                        const size_t slot = launchPitch == 1 ? leaf : (k / 2) * rowsPerTree * 2 + leaf * 2 + k % 2;
+                        const bool alone = k + 1 == launchPitch && k % 2 == 0;  // the odd last dimension
+                        const size_t slot = (k / 2) * rowsPerTree * 2 + (alone ? leaf : leaf * 2 + k % 2);
                         table[slot] = values[modelLeaf * m.Dim + launch * pitch + k];
                     }
                 }
@@ -2486,6 +2501,9 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 l.TreeLeafDoubles = rowsPerTree * pitch;
                 l.Leaves = m.RegLeaves.Get() + launch * m.RegLaunchLeaves;
             }
+            int groupsPerCu = 0;
+            HIP_CHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&groupsPerCu, l.Function, static_cast<int>(64 * l.Waves), 0));
+            l.GroupsPerCu = static_cast<uint32_t>(std::max(1, groupsPerCu));
             m.RegLaunches.push_back(l);
         }
         m.RegKernelUsable = true;
@@ -3555,7 +3573,7 @@ void THipEvaluator::EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCou
         args.FirstDim = l.FirstDim;
         args.StoreDims = l.StoreDims;
         const uint32_t grid = (args.BlockCount + l.Waves - 1) / l.Waves;
-        launchArgs.SlicesPerGroup = RegSlicesPerGroup(grid, slices);
+        launchArgs.SlicesPerGroup = RegSlicesPerGroup(grid, slices, size_t(256) * l.GroupsPerCu);
         const uint32_t shares = (slices + launchArgs.SlicesPerGroup - 1) / launchArgs.SlicesPerGroup;
         LaunchModuleWithEnd(l.Function, grid, shares, 64 * l.Waves, s, nullptr, launchArgs);
     }
@@ -3673,7 +3691,17 @@ bool THipEvaluator::EvalRowsFusedDevice(const TFeatureBatch& batch, size_t docCo
     args.Units = f.Units.Get();
     args.StrideBytes = static_cast<uint32_t>(batch.Stride * sizeof(float));
     args.UnitCount = f.UnitCount;
+    // Workgroups that start together wait for their rows together and walk their trees together. The second ones of the
+    // CUs start when the rows of the first ones have arrived (6 TB/s: early rather than late), so that one set walks while
+    // the other loads; a part of them waits less. Rows from HBM, whole call: 1M documents of 50 features, 200 trees of depth 6
+    // (one generation) 106.0 -> 101.6 us; 4M of 200 features, 1000 trees of depth 8 1564 -> 1545, 520 000 245.3 -> 242.2,
+    // 300 000 233.4 -> 232.9 (4 % longer with the whole delay for its 37 second workgroups). At 4.5 TB/s the same within
+    // 1 %, at 3.5 the one-generation batches lose what they gained.
     const uint32_t grid = (args.Reg.BlockCount + m.FusedWaves - 1) / m.FusedWaves;
+    const double secondGroups = std::min(256.0, std::max(256.0, static_cast<double>(grid)) - 256.0);
+    const double rowBytes = std::min(args.StrideBytes, f.UnitCount * kFusedUnitColumns * 4);
+    const double loadSeconds = secondGroups * m.FusedWaves * dev::kDocsPerBlock * rowBytes / 6e12, turnSeconds = 4096 / 2.4e9;
+    args.Reg.Bins = reinterpret_cast<const void*>(static_cast<uintptr_t>(std::min(loadSeconds / turnSeconds, 64.0)));
     LaunchModuleWithEnd(m.FusedFunction, grid, 1, 64 * m.FusedWaves, m.Pick(stream), TakeEnd(end), args);
     return true;
 }
@@ -3691,17 +3719,7 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
     }
     std::string binarize = m.BinarizeBuckets == 0 ? "none"
                            : layout == TFeatureBatch::FlatColumns
-    // Workgroups that start together wait for their rows together and walk their trees together. The second ones of the
-    // CUs start when the rows of the first ones have arrived (6 TB/s: early rather than late), so that one set walks while
-    // the other loads; a part of them waits less. Rows from HBM, whole call: 1M documents of 50 features, 200 trees of depth 6
-    // (one generation) 106.0 -> 101.6 us; 4M of 200 features, 1000 trees of depth 8 1564 -> 1545, 520 000 245.3 -> 242.2,
-    // 300 000 233.4 -> 232.9 (4 % longer with the whole delay for its 37 second workgroups). At 4.5 TB/s the same within
-    // 1 %, at 3.5 the one-generation batches lose what they gained.
                                ? "BinarizeColumnsKernel"
-    const double secondGroups = std::min(256.0, std::max(256.0, static_cast<double>(grid)) - 256.0);
-    const double rowBytes = std::min(args.StrideBytes, f.UnitCount * kFusedUnitColumns * 4);
-    const double loadSeconds = secondGroups * m.FusedWaves * dev::kDocsPerBlock * rowBytes / 6e12, turnSeconds = 4096 / 2.4e9;
-    args.Reg.Bins = reinterpret_cast<const void*>(static_cast<uintptr_t>(std::min(loadSeconds / turnSeconds, 64.0)));
                                : "BinarizeRowsKernel<" + std::to_string(BinarizeLog2Slots(m.MaxBucketValues)) + ">";
     if (m.CtrCount > 0) {
         binarize += m.CtrTileUsable ? "+CtrBinarizeKernel<true>" : "+CtrBinarizeKernel<false>";

@@ -549,11 +549,19 @@ __global__ __launch_bounds__(256) void CtrBinarizeKernel(TCatSource cats, uint32
         for (;;) {
             bool open[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            while ((entry[j].x != static_cast<uint32_t>(hash[j]) || entry[j].y != static_cast<uint32_t>(hash[j] >> 32)) &&
-                   (entry[j].x & entry[j].y) != 0xffffffffu) {
-                at[j] = (at[j] + 1) & group.HashMask;
-                entry[j] = table[static_cast<size_t>(at[j]) * group.EntryPieces];
+            for (int j = 0; j < 4; ++j) {
+                open[j] = (entry[j].x != static_cast<uint32_t>(hash[j]) || entry[j].y != static_cast<uint32_t>(hash[j] >> 32)) &&
+                          (entry[j].x & entry[j].y) != 0xffffffffu;
+            }
+            if (!(open[0] || open[1] || open[2] || open[3])) {
+                break;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (open[j]) {
+                    at[j] = (at[j] + 1) & group.HashMask;
+                    entry[j] = table[static_cast<size_t>(at[j]) * group.EntryPieces];
+                }
             }
         }
         // bytes of four documents and four buckets -> a dword of four documents per bucket
