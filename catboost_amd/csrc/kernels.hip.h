@@ -820,12 +820,20 @@ __device__ __forceinline__ void SmallStamp(ulonglong2* stamps, unsigned long lon
     stamps[blockIdx.y * gridDim.x + blockIdx.x] = make_ulonglong2(began, wall_clock64());
 }
 
+// How a host call of few documents learns that a workgroup is done: its results are in (coherent, pinned) host memory when its
+// flag is the ticket. Looking at the flags is shorter than waiting until the launch is retired.
+struct TSmallDone {
+    uint32_t* Flags;  // [workgroup]; null: the end of the launch says so
+    uint32_t Ticket;
+};
+
 // (The second argument is SmallBatchKernel's number of documents; here the grid has it.)
 // grid = (documents, ceil(dim / DIMS)), block = whole waves, at most kFewThreads; dynamic LDS = CellCount * 4 rounded up
 // to 8 + DIMS * SliceCount * (SliceTrees + 2) * 8 bytes.
 template <int DEPTH, int DIMS>
 __global__ __launch_bounds__(kFewThreads) void FewDocumentsKernel(TSmallSource src, uint32_t, TSmallTables tab,
-                                                                  double* __restrict__ out, ulonglong2* __restrict__ stamps) {
+                                                                  double* __restrict__ out, ulonglong2* __restrict__ stamps,
+                                                                  TSmallDone done) {
     extern __shared__ uint32_t sSmall[];
     const unsigned long long began = wall_clock64();
     const uint32_t tid = threadIdx.x, threads = blockDim.x;
@@ -895,6 +903,12 @@ __global__ __launch_bounds__(kFewThreads) void FewDocumentsKernel(TSmallSource s
         out[static_cast<size_t>(doc) * tab.Dim + d0 + tid] = Finish(sum, tab.Scale, tab.Bias[d0 + tid], true);
         if (tid == 0) {
             SmallStamp(stamps, began);
+        }
+        if (done.Flags != nullptr) {
+            __threadfence_system();  // the results, which lanes of this one wave wrote, and the stamps first
+            if (tid == 0) {
+                __hip_atomic_store(done.Flags + blockIdx.y * gridDim.x + blockIdx.x, done.Ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
         }
     }
 }

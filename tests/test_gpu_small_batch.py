@@ -436,3 +436,52 @@ def test_results_of_a_batch_that_a_slice_cannot_address():
     sample = np.concatenate([rng.choice(docs, size=100, replace=False), [0, docs - 1]])
     np.testing.assert_allclose(out[torch.from_numpy(sample).to("cuda:0")].cpu().numpy(),
                                OracleModel(model).calc(x.cpu().numpy()[sample]).reshape(-1, dim), rtol=1e-9, atol=1e-12)
+
+
+@pytest.mark.parametrize("dim,n_float", [(1, 100), (3, 40), (9, 30)])
+def test_few_host_documents_whose_workgroups_set_flags(dim, n_float):
+    """Host batches of up to sixteen workgroups return when the workgroups' flags are set, larger ones with the launch: rows
+    and columns, call after call with other values, other calls in between, kernel times, and callers side by side."""
+    import threading
+
+    rng = np.random.default_rng(dim)
+    ffs = [mb.float_feature(i, i) for i in range(n_float)]
+    trees = []
+    for t in range(150):
+        splits = [("float", int(f), float(np.float32(b))) for f, b in zip(rng.integers(0, n_float, 6), rng.normal(size=6))]
+        trees.append((splits, rng.normal(size=64 * dim)))
+    model = mb.build_oblivious(ffs, [], dim, trees, scale=0.5, bias=list(rng.normal(size=dim)))
+    m = cb.ModelCalcer()
+    m.load_from_dict(model)
+    m.enable_gpu_evaluation(0)
+    x = rng.normal(size=(400, n_float)).astype(np.float32)
+    expected = m.calc_flat(x).reshape(400, dim)  # the launch's event
+    np.testing.assert_allclose(expected.ravel(), OracleModel(model).calc(x), rtol=1e-9, atol=1e-12)
+
+    def check(seed):
+        own = np.random.default_rng(seed)
+        for _ in range(60):
+            docs = int(own.integers(1, 19))
+            at = int(own.integers(0, 400 - docs))
+            rows = x[at:at + docs]
+            got = m.calc_flat(rows) if own.integers(0, 2) else m.calc_flat_transposed(np.ascontiguousarray(rows.T))
+            np.testing.assert_array_equal(got.reshape(docs, dim), expected[at:at + docs])
+
+    check(0)
+    m.calc_flat(x[:1])
+    binarize_ms, eval_ms = m.evaluator().last_kernel_times()
+    assert binarize_ms == 0.0 and 0.0 < eval_ms < 5.0
+    failures = []
+
+    def caller(seed):
+        try:
+            check(seed)
+        except BaseException as e:  # noqa: B902
+            failures.append(e)
+
+    threads = [threading.Thread(target=caller, args=(s,)) for s in range(1, 7)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures[0]
