@@ -1640,7 +1640,8 @@ struct THipEvaluator::TImpl {
     };
     struct THostContext {
         hipStream_t Stream = nullptr;
-        hipStream_t CopyStream = nullptr;  // features of the next chunk, while the kernels of the one before run on Stream
+        hipStream_t CopyStream = nullptr;  // features of the next chunk, while the kernels of the one before run on Stream;
+                                           // made by the first call of several chunks
         TDeviceVec<uint8_t> ScratchBins;
         TDeviceVec<double> SlicePartials;  // raw sums per slice of the trees (small batches)
         THostSlot Slots[2];
@@ -1664,16 +1665,27 @@ struct THipEvaluator::TImpl {
             return *RunningStamps;
         }
 
-        // What Stream does from here on finds the slot's features, sent on CopyStream, on the device.
-        void AwaitCopies(int slot) {
-            HIP_CHECK(hipEventRecord(Slots[slot].Ev[4], CopyStream));
-            HIP_CHECK(hipStreamWaitEvent(Stream, Slots[slot].Ev[4], 0));
+        // The stream for the features of a call's chunks.
+        hipStream_t CopiesOf(bool severalChunks) {
+            if (!severalChunks) {
+                return Stream;
+            }
+            if (CopyStream == nullptr) {
+                HIP_CHECK(hipStreamCreateWithFlags(&CopyStream, hipStreamNonBlocking));
+            }
+            return CopyStream;
+        }
+        // What Stream does from here on finds the slot's features, sent on `copies`, on the device.
+        void AwaitCopies(int slot, hipStream_t copies) {
+            if (copies != Stream) {
+                HIP_CHECK(hipEventRecord(Slots[slot].Ev[4], copies));
+                HIP_CHECK(hipStreamWaitEvent(Stream, Slots[slot].Ev[4], 0));
+            }
         }
 
         THostContext() {
             try {
                 HIP_CHECK(hipStreamCreateWithFlags(&Stream, hipStreamNonBlocking));
-                HIP_CHECK(hipStreamCreateWithFlags(&CopyStream, hipStreamNonBlocking));
                 for (auto& e : Ev) {
                     HIP_CHECK(hipEventCreate(&e));
                 }
@@ -4185,8 +4197,11 @@ void RunPipeline(size_t docCount, size_t chunk, THipEvaluator::TImpl::THostConte
         finish(static_cast<int>((index + 1) & 1));
     } catch (...) {
         // the context goes back to the pool: nothing of this call may touch its buffers any more
-        (void)hipStreamSynchronize(ctx.CopyStream);
-        (void)hipStreamSynchronize(ctx.Stream);
+        for (hipStream_t s : {ctx.CopyStream, ctx.Stream}) {
+            if (s) {
+                (void)hipStreamSynchronize(s);
+            }
+        }
         throw;
     }
 }
@@ -4409,11 +4424,12 @@ void THipEvaluator::CalcHostRows(const float* const* rows, size_t rowLen, bool f
     }
     ctx->ScratchBins.Reserve(QuantizedBytes(stageDocs));
     TKernelTimes times;
+    const hipStream_t copies = ctx->CopiesOf(docCount > chunk);
     RunPipeline(
         docCount, chunk, *ctx,
         [&](int i, size_t begin, size_t n) {
-            const TFeatureBatch batch = StageRowChunk(ctx->Slots[i], ctx->CopyStream, rows, catRows, begin, n, needFloats, needCats, flat);
-            ctx->AwaitCopies(i);
+            const TFeatureBatch batch = StageRowChunk(ctx->Slots[i], copies, rows, catRows, begin, n, needFloats, needCats, flat);
+            ctx->AwaitCopies(i, copies);
             RunPredictionChunk(*this, *ctx, i, batch, begin, n, docCount, stageDocs, treeStart, treeEnd, predictionType);
         },
         [&](int i, size_t begin, size_t n) {
@@ -4468,20 +4484,20 @@ void THipEvaluator::CalcHostColumns(const float* const* columns, size_t columnCo
     }
     ctx->ScratchBins.Reserve(QuantizedBytes(stageDocs));
     TKernelTimes times;
+    const hipStream_t copies = ctx->CopiesOf(docCount > chunk);
     RunPipeline(
         docCount, chunk, *ctx,
         [&](int i, size_t begin, size_t n) {
             TImpl::THostSlot& slot = ctx->Slots[i];
             float* dst = slot.PinnedFloats.Get();
             float* device = slot.StageFloats.Get();
-            const hipStream_t copies = ctx->CopyStream;
             FillAndSend(
                 need, n * sizeof(float), [=](size_t first, size_t last) { CopyColumns(columns, begin, n, first, last, dst); },
                 [=](size_t first, size_t last) {
                     HIP_CHECK(hipMemcpyAsync(device + first * n, dst + first * n, (last - first) * n * sizeof(float),
                                              hipMemcpyHostToDevice, copies));
                 });
-            ctx->AwaitCopies(i);
+            ctx->AwaitCopies(i, copies);
             TFeatureBatch batch;
             batch.Layout = TFeatureBatch::FlatColumns;
             batch.Floats = slot.StageFloats.Get();
