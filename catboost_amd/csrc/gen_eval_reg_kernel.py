@@ -73,6 +73,8 @@ go through the same two LDS buffers as the tree blocks that follow them:
   * per unit a record of 40 dwords: sixteen lo, sixteen scale, a flags dword (bit q: the unit's q-th four
     columns need four steps, bit 4 + q: three or more, bit 8 + q: two or more, bit 16 + i: NaN counts
     as +inf in column i); behind the BUCKETS / 16 + 1 records, the units' byte offsets in a row.
+Column-major documents ("cbamd_fused_cols_..."): the bins registers follow the buckets, sixteen to a unit; behind the records
+sit, per unit, its sixteen columns instead of the units' byte offsets, and argument 96 is the bytes from a column to the next.
 Additional kernel arguments (104 bytes in all):
   80 floats const float*  88 units const uint32* [BUCKETS / 16 + 1][40] + [16]  96 row stride in bytes uint32
  100 unitCount uint32 (1 .. BUCKETS / 16)
@@ -111,6 +113,12 @@ FUSED_SHAPES = [(208, 4), (64, 8), (80, 8)]
 # Every shape also in a form that walks six levels ("_d6": models of depth <= 6; the leaf tables keep the 256 rows
 # per tree that the border images' buffers are sized for, the index reaches the first 64 of them).
 FUSED_SIX_LEVEL_BUCKETS = 208
+# Fused kernels of column-major documents ("cbamd_fused_cols_..."), every shape in the same four forms. A load is a column's value
+# for 64 neighbouring documents, so every line comes once and whole; what bounds them is vector issue at two waves per SIMD (four
+# for the shapes of 64 and 80) and the columns' arrival, as for rows. Against two launches, whole call: 1M documents, 1000
+# trees of depth 6 over 150 features 398 -> 338 us, 200 trees over 50 124 -> 90, 100 over 120 181 -> 132; 4M, 1000 trees of
+# depth 8 over 200 1800 -> 1465 (the same model on rows 1545); 270 000, 300 trees over 50 72.3 -> 66.7.
+FUSED_COLUMN_SHAPES = [(208, 4), (160, 4), (64, 8), (80, 8)]
 FUSED_MAX_STEPS = 4
 FUSED_EXTRA_SETS = 1
 FUSED_UNIT_DWORDS = 40
@@ -129,9 +137,10 @@ def fused_chunks(buckets, six):
     return chunks + chunks % 2
 
 
-def kernel_name(buckets, waves, pitch, leaves, mixed, six=False, fused=False, levels=None):
+def kernel_name(buckets, waves, pitch, leaves, mixed, six=False, fused=False, levels=None, columns=False):
     if fused:
-        return "cbamd_fused_b%d_w%d%s%s" % (buckets, waves, "_d6" if levels == 6 else "", "_s" if six else "")
+        return "cbamd_fused_%sb%d_w%d%s%s" % ("cols_" if columns else "", buckets, waves, "_d6" if levels == 6 else "",
+                                              "_s" if six else "")
     return "cbamd_eval_reg_b%d_w%d_p%d_l%d%s" % (buckets, waves, pitch, leaves, "_m" if mixed else "_s" if six else "")
 
 
@@ -143,11 +152,12 @@ def tree_block(pitch, leaves):
     return block
 
 
-def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, levels=None):
+def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, levels=None, columns=False):
     assert not (mixed and six)
+    assert fused or not columns
     assert not fused or (pitch == 1 and leaves == 256 and not mixed and buckets % 16 == 0)
     assert levels is None or (fused and levels == 6)
-    name = kernel_name(buckets, waves, pitch, leaves, mixed, six, fused, levels)
+    name = kernel_name(buckets, waves, pitch, leaves, mixed, six, fused, levels, columns)
     depth = levels or {64: 6, 256: 8, 1024: 10}[leaves]
     deep = depth > 8                      # levels 8 and 9 go into a second index word
     assert not deep or (pitch == 1 and not mixed and not fused)
@@ -319,6 +329,194 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 e("  v_lshrrev_b32_e32 v3, 1, v3")
                 e("  v_bfi_b32 v3, s22, v4, v3")
 
+    # ---- the binarize phase's search, shared by the rows' and the columns' form
+    out_of_line = []
+
+    def search_step(step, vals):
+        """Step `step` (counted from the last one, 1) of the four searches: looks at the border 2^(step-1)
+        places on and moves on behind it when it lies below the value."""
+        size = 4 << (step - 1)
+        for d in range(4):
+            e("  ds_read_b32 v%d, v%d offset:%d" % (srch_b[d], srch_p[d], search_step.border_at[d] + size - 4))
+        e("  s_waitcnt lgkmcnt(0)")
+        for d in range(4):
+            e("  v_cmp_lt_f32_e32 vcc, v%d, v%d" % (srch_b[d], vals + d))
+            e("  v_cndmask_b32_e64 v%d, 0, %d, vcc" % (srch_b[d], size))
+            e("  v_add_u32_e32 v%d, v%d, v%d" % (srch_p[d], srch_p[d], srch_b[d]))
+
+    def search_group(label, unit, j, q, vals, lo, scale, flags, buf):
+        """Columns 4 q .. 4 q + 3 of a unit for the lane's document j, whose values are in v[vals] .. v[vals + 3]: their
+        bins into byte j of the bins registers."""
+        local = (unit % (fused_layout(six)[0] // 16)) * 16 + 4 * q
+        search_step.border_at = [buf * buf_bytes + (local + d) * fused_layout(six)[1] for d in range(4)]
+        for d in range(4):
+            i = 4 * q + d
+            # the value's cell in the column's grid and the search start stored for it
+            e("  v_subrev_f32_e32 v%d, s%d, v%d" % (srch_b[d], lo + i, vals + d))
+            e("  v_mul_f32_e32 v%d, s%d, v%d" % (srch_b[d], scale + i, srch_b[d]))
+            e("  v_cvt_u32_f32_e32 v%d, v%d" % (srch_b[d], srch_b[d]))
+            e("  v_min_u32_e32 v%d, 0xff, v%d" % (srch_b[d], srch_b[d]))
+            e("  ds_read_u8 v%d, v%d offset:%d" % (srch_p[d], srch_b[d],
+                                                   buf * buf_bytes + 16384 + (local + d) * 256))
+        e("  s_waitcnt lgkmcnt(0)")
+        if not six:
+            for d in range(4):
+                e("  v_lshlrev_b32_e32 v%d, 2, v%d" % (srch_p[d], srch_p[d]))
+        # the search: steps above two are rare and sit out of line
+        e("  s_bitcmp1_b32 s%d, %d" % (flags, 4 + q))
+        e("  s_cbranch_scc1 %s_q%d_hi" % (label, q))
+        e("%s_q%d_back:" % (label, q))
+        e("  s_bitcmp1_b32 s%d, %d" % (flags, 8 + q))
+        e("  s_cbranch_scc0 %s_q%d_one" % (label, q))
+        search_step(2, vals)
+        e("%s_q%d_one:" % (label, q))
+        search_step(1, vals)
+        for d in range(4):
+            reg = b0 + unit * 16 + 4 * q + d
+            if j == 0:
+                e("  v_lshrrev_b32_e32 v%d, 2, v%d" % (reg, srch_p[d]))
+            else:
+                e("  v_lshl_add_u32 v%d, v%d, %d, v%d" % (reg, srch_p[d], 8 * j - 2, reg))
+        out_of_line.append((label, q, vals, list(search_step.border_at), flags))
+
+    def emit_out_of_line():
+        for label, q, vals, border_at, flags in out_of_line:
+            search_step.border_at = border_at
+            e("%s_q%d_hi:" % (label, q))
+            e("  s_bitcmp1_b32 s%d, %d" % (flags, q))
+            e("  s_cbranch_scc0 %s_q%d_three" % (label, q))
+            search_step(4, vals)
+            e("%s_q%d_three:" % (label, q))
+            search_step(3, vals)
+            e("  s_branch %s_q%d_back" % (label, q))
+        del out_of_line[:]
+
+    def binarize_columns(rec_lo, rec_scale, rec_fo):
+        """The phase for column-major documents, behind the prologue that it shares with the rows' form. A turn is
+        eight columns (half a unit) of the lane's four documents: a load is a column's value for one of them, 256
+        contiguous bytes per wave. s6: bytes between columns, s[8:15]: the columns of the turn whose loads come next."""
+        units_per_chunk = fused_layout(six)[0] // 16
+        max_units = buckets // 16
+        chunks = fused_chunks(buckets, six)
+        columns_at = (max_units + 1) * FUSED_UNIT_DWORDS * 4
+        order = [(unit, half) for unit in range(max_units) for half in (0, 1)]
+        after = dict(zip(order, order[1:]))
+
+        def load_record(unit):
+            x, at = unit % 2, unit * FUSED_UNIT_DWORDS * 4
+            e("  s_load_dwordx16 s[%d:%d], s[24:25], 0x%x" % (rec_lo[x], rec_lo[x] + 15, at))
+            e("  s_load_dwordx16 s[%d:%d], s[24:25], 0x%x" % (rec_scale[x], rec_scale[x] + 15, at + 64))
+            e("  s_load_dwordx2 s[%d:%d], s[24:25], 0x%x" % (rec_fo[x], rec_fo[x] + 1, at + 128))
+
+        def load_columns(turn):
+            e("  s_load_dwordx8 s[8:15], s[24:25], 0x%x" % (columns_at + turn[0] * 64 + turn[1] * 32))
+
+        value_set, pending, issued, done = {}, [], set(), set()
+
+        def issue_loads(turn):
+            e("  s_waitcnt lgkmcnt(0)")                # the turn's columns
+            for c in range(8):
+                e("  s_mul_i32 s30, s%d, s6" % (8 + c))
+                e("  s_mul_hi_u32 s31, s%d, s6" % (8 + c))
+                e("  s_add_u32 s30, s30, s4")
+                e("  s_addc_u32 s31, s31, s5")
+                for j in range(4):
+                    e("  global_load_dword v%d, v%d, s[30:31]" % (value_set[turn][2 * j + c // 4] + c % 4, row_off[j]))
+                    pending.append(("turn", turn))
+            issued.add(turn)
+            if turn in after:
+                load_columns(after[turn])
+
+        def wait_loads(turn):
+            last = max((i for i, op in enumerate(pending) if op == ("turn", turn)), default=None)
+            if last is not None:
+                e("  s_waitcnt vmcnt(%d)" % min(63, len(pending) - 1 - last))
+                del pending[:last + 1]
+
+        def process(turn, buf):
+            unit, half = turn
+            lo, scale, flags = rec_lo[unit % 2], rec_scale[unit % 2], rec_fo[unit % 2]
+            label = "%s_u%d_%d" % (name, unit, half)
+            # NaN counts as +inf in the columns whose flag says so
+            e("  s_bfe_u32 s3, s%d, 0x%x" % (flags, (8 << 16) | (16 + 8 * half)))
+            e("  s_cmp_eq_u32 s3, 0")
+            e("  s_cbranch_scc1 %s_n" % label)
+            e("  v_mov_b32_e32 v%d, 0x7f800000" % srch_b[0])
+            for c in range(8):
+                e("  s_bitcmp1_b32 s%d, %d" % (flags, 16 + 8 * half + c))
+                e("  s_cbranch_scc0 %s_n%d" % (label, c))
+                for j in range(4):
+                    reg = value_set[turn][2 * j + c // 4] + c % 4
+                    e("  v_cmp_u_f32_e32 vcc, v%d, v%d" % (reg, reg))
+                    e("  v_cndmask_b32_e32 v%d, v%d, v%d, vcc" % (reg, reg, srch_b[0]))
+                e("%s_n%d:" % (label, c))
+            e("%s_n:" % label)
+            for j in range(4):
+                for h in (0, 1):
+                    search_group("%s_%d" % (label, j), unit, j, 2 * half + h, value_set[turn][2 * j + h], lo, scale, flags, buf)
+
+        # sets of registers for the turns in flight, as in the rows' form
+        plan = []
+        for c in range(chunks):
+            turns = [t for t in order if t[0] // units_per_chunk == c]
+            later_units = [u for u in range(max_units - 1, -1, -1) if u // units_per_chunk > c]
+            sets = [values[0] + values[1]]
+            for k in range(min(FUSED_EXTRA_SETS, len(later_units) // 2)):
+                sets.append([b0 + 16 * u + 4 * q for u in later_units[2 * k:2 * k + 2] for q in range(4)])
+            for k, turn in enumerate(turns):
+                value_set[turn] = sets[k % len(sets)]
+            plan.append((turns, len(sets), bool(turns) and len(sets) > 1 and (len(turns) - 1) % len(sets) != 0))
+
+        load_record(0)
+        if max_units > 1:
+            load_record(1)
+        load_columns(order[0])
+        issue_loads(order[0])
+        e("  s_waitcnt vmcnt(0)")                      # the first image (and the first loads)
+        e("  s_barrier")
+        del pending[:]
+        done.add(order[0])
+        for c, (turns, set_count, cross) in enumerate(plan):
+            buf = c % 2
+            for g in range(len(groups)):
+                stage((1 - buf) * buf_bytes, g)
+                pending.extend([("stage", c)] * groups[g][1])
+            if turns:
+                # the model has no unit in this image: nothing to do but to pass it on
+                e("  s_cmp_le_u32 s28, %d" % turns[0][0])
+                e("  s_cbranch_scc1 %s_c%d_end" % (name, c))
+            for k, turn in enumerate(turns):
+                ahead = [t for t in turns[k:k + set_count] if t not in issued]
+                if k == len(turns) - 1 and cross and c + 1 < len(plan) and plan[c + 1][0]:
+                    ahead.append(plan[c + 1][0][0])
+                for t in ahead:
+                    issue_loads(t)
+                if turn in done:
+                    done.discard(turn)
+                else:
+                    wait_loads(turn)
+                e("  s_waitcnt lgkmcnt(0)")            # the unit's record, also that of a unit the model lacks
+                if turn[0] > 0:
+                    e("  s_cmp_le_u32 s28, %d" % turn[0])
+                    e("  s_cbranch_scc1 %s_u%d_%d_skip" % (name, turn[0], turn[1]))
+                process(turn, buf)
+                e("%s_u%d_%d_skip:" % (name, turn[0], turn[1]))
+                if turn[1] == 1 and turn[0] + 2 < max_units:
+                    load_record(turn[0] + 2)
+            e("  s_branch %s_c%d_end" % (name, c))
+            emit_out_of_line()
+            e("%s_c%d_end:" % (name, c))
+            e("  s_waitcnt vmcnt(0) lgkmcnt(0)")
+            e("  s_barrier")
+            done.update(op[1] for op in pending if op[0] == "turn")
+            del pending[:]
+        assert len(issued) == len(order)
+        # the record and column registers held these arguments
+        e("  s_load_dwordx4 s[96:99], s[0:1], 0x40")
+        e("  s_load_dwordx8 s[4:11], s[0:1], 0x0")
+        e("  s_load_dwordx8 s[12:19], s[0:1], 0x20")
+        e("  s_waitcnt lgkmcnt(0)")                    # the level tables are loaded through s[6:7] next
+
     def fused_binarize():
         """The binarize phase of a fused kernel: fills the bins registers from the documents' rows. On
         entry the first border table image is on its way into buffer 0 and s24 holds the wave's document
@@ -333,8 +531,13 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  s_sub_u32 s31, s12, s30")
         e("  s_add_u32 s31, s31, -1")
         e("  s_min_u32 s31, s31, 0xff")               # last row of the batch, counted from the block's first, at most 255
-        e("  s_mul_hi_u32 s3, s30, s88")
-        e("  s_mul_i32 s25, s30, s88")
+        if columns:
+            e("  s_mov_b32 s3, 0")                    # a document's value is four bytes from its neighbours'
+            e("  s_lshl_b32 s25, s30, 2")
+            e("  s_mov_b32 s6, s88")                  # bytes from one column to the next
+        else:
+            e("  s_mul_hi_u32 s3, s30, s88")
+            e("  s_mul_i32 s25, s30, s88")
         e("  s_add_u32 s4, s84, s25")                 # s[4:5]: the block's first row
         e("  s_addc_u32 s5, s85, s3")
         e("  v_and_b32_e32 v%d, 63, v0" % srch_p[0])
@@ -342,10 +545,16 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             # rows past the last document are read as the last document
             e("  v_add_u32_e32 v%d, %d, v%d" % (row_off[j], 64 * j, srch_p[0]))
             e("  v_min_u32_e32 v%d, s31, v%d" % (row_off[j], row_off[j]))
-            e("  v_mul_lo_u32 v%d, v%d, s88" % (row_off[j], row_off[j]))
+            if columns:
+                e("  v_lshlrev_b32_e32 v%d, 2, v%d" % (row_off[j], row_off[j]))
+            else:
+                e("  v_mul_lo_u32 v%d, v%d, s88" % (row_off[j], row_off[j]))
         e("  s_mov_b32 s24, s86")                     # s[24:25]: unit records, s28: units of the model
         e("  s_mov_b32 s25, s87")
         e("  s_mov_b32 s28, s89")
+        if columns:
+            binarize_columns(rec_lo, rec_scale, rec_fo)
+            return
         # the units' byte offsets in a row (they follow the records) stay in s6 .. s19 for the whole phase;
         # the arguments that sat there are loaded again behind it
         assert max_units <= 14
@@ -384,18 +593,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 e("  s_waitcnt vmcnt(%d)" % (len(pending) - 1 - last))
                 del pending[:last + 1]
 
-        def search_step(step, vals):
-            """Step `step` (counted from the last one, 1) of the four searches: looks at the border 2^(step-1)
-            places on and moves on behind it when it lies below the value."""
-            size = 4 << (step - 1)
-            for d in range(4):
-                e("  ds_read_b32 v%d, v%d offset:%d" % (srch_b[d], srch_p[d], search_step.border_at[d] + size - 4))
-            e("  s_waitcnt lgkmcnt(0)")
-            for d in range(4):
-                e("  v_cmp_lt_f32_e32 vcc, v%d, v%d" % (srch_b[d], vals + d))
-                e("  v_cndmask_b32_e64 v%d, 0, %d, vcc" % (srch_b[d], size))
-                e("  v_add_u32_e32 v%d, v%d, v%d" % (srch_p[d], srch_p[d], srch_b[d]))
-
         def process(n, buf):
             unit, j = seq[n]
             lo, scale, flags = rec_lo[n % 2], rec_scale[n % 2], rec_fo[n % 2]
@@ -414,50 +611,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 e("%s_n%d:" % (label, i))
             e("%s_n:" % label)
             for q in range(4):
-                vals = value_set[n][q]
-                local = (unit % units_per_chunk) * 16 + 4 * q
-                search_step.border_at = [buf * buf_bytes + (local + d) * border_bytes for d in range(4)]
-                for d in range(4):
-                    i = 4 * q + d
-                    # the value's cell in the column's grid and the search start stored for it
-                    e("  v_subrev_f32_e32 v%d, s%d, v%d" % (srch_b[d], lo + i, vals + d))
-                    e("  v_mul_f32_e32 v%d, s%d, v%d" % (srch_b[d], scale + i, srch_b[d]))
-                    e("  v_cvt_u32_f32_e32 v%d, v%d" % (srch_b[d], srch_b[d]))
-                    e("  v_min_u32_e32 v%d, 0xff, v%d" % (srch_b[d], srch_b[d]))
-                    e("  ds_read_u8 v%d, v%d offset:%d" % (srch_p[d], srch_b[d],
-                                                           buf * buf_bytes + 16384 + (local + d) * 256))
-                e("  s_waitcnt lgkmcnt(0)")
-                if not six:
-                    for d in range(4):
-                        e("  v_lshlrev_b32_e32 v%d, 2, v%d" % (srch_p[d], srch_p[d]))
-                # the search: steps above two are rare and sit out of line
-                e("  s_bitcmp1_b32 s%d, %d" % (flags, 4 + q))
-                e("  s_cbranch_scc1 %s_q%d_hi" % (label, q))
-                e("%s_q%d_back:" % (label, q))
-                e("  s_bitcmp1_b32 s%d, %d" % (flags, 8 + q))
-                e("  s_cbranch_scc0 %s_q%d_one" % (label, q))
-                search_step(2, vals)
-                e("%s_q%d_one:" % (label, q))
-                search_step(1, vals)
-                for d in range(4):
-                    reg = b0 + unit * 16 + 4 * q + d
-                    if j == 0:
-                        e("  v_lshrrev_b32_e32 v%d, 2, v%d" % (reg, srch_p[d]))
-                    else:
-                        e("  v_lshl_add_u32 v%d, v%d, %d, v%d" % (reg, srch_p[d], 8 * j - 2, reg))
-                out_of_line.append((label, q, vals, list(search_step.border_at), flags))
-
-        def emit_out_of_line():
-            for label, q, vals, border_at, flags in out_of_line:
-                search_step.border_at = border_at
-                e("%s_q%d_hi:" % (label, q))
-                e("  s_bitcmp1_b32 s%d, %d" % (flags, q))
-                e("  s_cbranch_scc0 %s_q%d_three" % (label, q))
-                search_step(4, vals)
-                e("%s_q%d_three:" % (label, q))
-                search_step(3, vals)
-                e("  s_branch %s_q%d_back" % (label, q))
-            del out_of_line[:]
+                search_group(label, unit, j, q, value_set[n][q], lo, scale, flags, buf)
 
         # Two neighbouring units of a document (128 bytes of its row) are loaded together, eight loads one
         # behind the other, so that a line of the row is asked for once (the cache merges requests that
@@ -486,7 +640,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             cross = bool(pairs) and len(sets) > 1 and (len(pairs) - 1) % len(sets) != 0
             plan.append((pairs, len(sets), cross))
 
-        out_of_line = []
         load_record(0)
         if len(seq) > 1:
             load_record(1)
@@ -969,12 +1122,13 @@ def generate():
         text, meta = gen_kernel(buckets, waves, pitch, leaves, mixed, six)
         parts.append(text)
         metas.append(meta)
-    for buckets, waves in FUSED_SHAPES:
-        for six in (False, True):
-            for levels in (None, 6) if buckets <= FUSED_SIX_LEVEL_BUCKETS else (None,):
-                text, meta = gen_kernel(buckets, waves, 1, 256, False, six, fused=True, levels=levels)
-                parts.append(text)
-                metas.append(meta)
+    for columns, shapes in ((False, FUSED_SHAPES), (True, FUSED_COLUMN_SHAPES)):
+        for buckets, waves in shapes:
+            for six in (False, True):
+                for levels in (None, 6) if buckets <= FUSED_SIX_LEVEL_BUCKETS else (None,):
+                    text, meta = gen_kernel(buckets, waves, 1, 256, False, six, fused=True, levels=levels, columns=columns)
+                    parts.append(text)
+                    metas.append(meta)
     parts.append(".amdgpu_metadata")
     parts.append("---")
     parts.append("amdhsa.kernels:")

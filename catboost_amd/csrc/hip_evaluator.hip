@@ -312,6 +312,7 @@ struct TFusedVariant {
     bool Six;
     uint32_t Levels;
     const char* Name;
+    bool Columns = false;  // column-major documents
 };
 constexpr TFusedVariant kFusedVariants[] = {
     {64, 8, false, 6, "cbamd_fused_b64_w8_d6"},
@@ -326,6 +327,22 @@ constexpr TFusedVariant kFusedVariants[] = {
     {208, 4, true, 6, "cbamd_fused_b208_w4_d6_s"},
     {208, 4, false, 8, "cbamd_fused_b208_w4"},
     {208, 4, true, 8, "cbamd_fused_b208_w4_s"},
+    {64, 8, false, 6, "cbamd_fused_cols_b64_w8_d6", true},
+    {64, 8, true, 6, "cbamd_fused_cols_b64_w8_d6_s", true},
+    {64, 8, false, 8, "cbamd_fused_cols_b64_w8", true},
+    {64, 8, true, 8, "cbamd_fused_cols_b64_w8_s", true},
+    {80, 8, false, 6, "cbamd_fused_cols_b80_w8_d6", true},
+    {80, 8, true, 6, "cbamd_fused_cols_b80_w8_d6_s", true},
+    {80, 8, false, 8, "cbamd_fused_cols_b80_w8", true},
+    {80, 8, true, 8, "cbamd_fused_cols_b80_w8_s", true},
+    {160, 4, false, 6, "cbamd_fused_cols_b160_w4_d6", true},
+    {160, 4, true, 6, "cbamd_fused_cols_b160_w4_d6_s", true},
+    {160, 4, false, 8, "cbamd_fused_cols_b160_w4", true},
+    {160, 4, true, 8, "cbamd_fused_cols_b160_w4_s", true},
+    {208, 4, false, 6, "cbamd_fused_cols_b208_w4_d6", true},
+    {208, 4, true, 6, "cbamd_fused_cols_b208_w4_d6_s", true},
+    {208, 4, false, 8, "cbamd_fused_cols_b208_w4", true},
+    {208, 4, true, 8, "cbamd_fused_cols_b208_w4_s", true},
 };
 constexpr uint32_t kFusedUnitColumns = 16;
 constexpr uint32_t kFusedUnitDwords = 40;   // sixteen lo, sixteen scale, flags, padding
@@ -576,6 +593,11 @@ constexpr size_t kSmallBatchDocs = 16384;
 constexpr size_t kFewDocs = 640;
 // ... of host calls, whose features are at most so many bytes: more go through the pipeline of chunks
 constexpr size_t kSmallHostBytes = size_t(16) << 20;
+
+// Workgroups up to which a host batch's launch sets flags: every one of them orders its results before its flag, over PCIe.
+// 1000 trees of depth 6 over 100 features, whole call with the launch's event and with flags: 1 row 20.6 and 18.3 us, 4 rows
+// 20.5 and 18.5, 16 20.8 and 19.8, 24 21.0 and 20.2, 200 23.6 and 28.3.
+constexpr size_t kFlaggedGroups = 16;
 
 // Workgroups wanted of a leaf index launch: 200 000 documents * 1000 trees (782 blocks, 2 workgroups per CU) take 225 us as
 // 782 workgroups, 200 as 2346, 216 as 4692 (shorter runs of a row, the bins read more often), launches back to back.
@@ -1549,24 +1571,23 @@ struct THipEvaluator::TImpl {
     // min(bin, 127) and max(bin - 127, 0), so that every level is a 7-bit compare (the kernels' register map)
     TDeviceVec<uint32_t> RegMap;
 
-    // fused kernels, per row layout (0: flat rows, 1: split rows of a model without categorical features)
+    // fused kernels, per layout (0: flat rows, 1: split rows of a model without categorical features, 2: flat columns)
     struct TFused {
-        bool Usable = false;
+        hipFunction_t Function = nullptr;
+        uint32_t Waves = 0;
+        const char* Name = "";
         uint32_t UnitCount = 0;
         TDeviceVec<uint32_t> Rows;    // level rows that name bins registers of the fused layout
         TDeviceVec<uint32_t> Units;   // unit records
         TDeviceVec<uint8_t> Table;    // border table images, then a copy of the leaf table
     };
-    TFused Fused[2];
-    hipFunction_t FusedFunction = nullptr;
-    uint32_t FusedWaves = 0;
+    std::shared_ptr<TFused> Fused[3];  // null: two launches
     // Below about one wave per SIMD a fused launch lasts as long as one wave's binarize phase and tree walk,
     // and two launches (the binarize kernel spreads a block over many waves) are shorter.
     size_t FusedMinDocs() const {
         return SmallBatchSlices ? size_t(1024) * dev::kDocsPerBlock : 0;
     }
     const char* RegKernelName = "";
-    const char* FusedKernelName = "";
 
     // small-batch kernel: tree rows of sixteen dwords, and from these dwords on the cells of its tile and the first leaves
     bool SmallUsable = false;
@@ -1615,9 +1636,10 @@ struct THipEvaluator::TImpl {
         TPinnedVec<float> PinnedFloats;
         TPinnedVec<int32_t> PinnedCats;
         TPinnedVec<double> PinnedResults;
-        // results of a small host batch and the flags of its workgroups, which the host looks at while the launch runs
-        TPinnedVec<double, hipHostMallocCoherent> SmallResults;
-        TPinnedVec<uint32_t, hipHostMallocCoherent> SmallFlags;
+        // flags of the workgroups of a small host batch and its results, which the host looks at while the launch runs
+        TPinnedVec<double, hipHostMallocCoherent> SmallMemory;
+        uint32_t* SmallFlags() const { return reinterpret_cast<uint32_t*>(SmallMemory.Get()); }
+        double* SmallResults() const { return SmallMemory.Get() + kFlaggedGroups * sizeof(uint32_t) / sizeof(double); }
         uint32_t SmallTicket = 0;
         size_t SmallGroups = 0;  // workgroups of the running launch
         TPinnedVec<uint32_t> PinnedIndexes;
@@ -2562,10 +2584,15 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             }
         }
         const std::vector<double>& fusedLeafTable = variant->Leaves == 64 ? fusedLeaves : leaves;
-        for (int layoutIndex = 0; layoutIndex < 2 && fusedCandidate; ++layoutIndex) {
-            const std::vector<uint32_t>& columns = layoutIndex == 0 ? srcFlat : srcSplit;
-            const size_t rowWidth = layoutIndex == 0 ? m.FlatVectorSize : m.MinFloatSize;
-            if (rowWidth < kFusedUnitColumns) {
+        for (int layoutIndex = 0; layoutIndex < 3 && fusedCandidate; ++layoutIndex) {
+            const bool columnMajor = layoutIndex == 2;  // a value is a load of its own: units of any sixteen buckets
+            const std::vector<uint32_t>& columns = layoutIndex == 1 ? srcSplit : srcFlat;
+            const size_t rowWidth = layoutIndex == 1 ? m.MinFloatSize : m.FlatVectorSize;
+            if (rowWidth < kFusedUnitColumns && !columnMajor) {
+                continue;
+            }
+            if (layoutIndex == 1 && m.MinFloatSize == m.FlatVectorSize && srcSplit == srcFlat) {
+                m.Fused[1] = m.Fused[0];  // the same rows
                 continue;
             }
             std::vector<std::pair<uint32_t, uint32_t>> byColumn;  // (column, bucket)
@@ -2577,12 +2604,18 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             for (size_t i = 1; i < byColumn.size(); ++i) {
                 distinct = distinct && byColumn[i].first != byColumn[i - 1].first;
             }
-            if (!distinct) {
+            if (!distinct && !columnMajor) {
                 continue;
             }
             // units: sixteen columns from a used column on, moved back where they would leave the row
             std::vector<uint32_t> unitStart, slotOfBucket(BucketCount, 0);
-            for (size_t i = 0; i < byColumn.size();) {
+            for (uint32_t b = 0; b < BucketCount && columnMajor; ++b) {
+                slotOfBucket[b] = b;
+            }
+            if (columnMajor) {
+                unitStart.assign((BucketCount + kFusedUnitColumns - 1) / kFusedUnitColumns, 0);
+            }
+            for (size_t i = 0; i < byColumn.size() && !columnMajor;) {
                 const uint32_t start = static_cast<uint32_t>(std::min<size_t>(byColumn[i].first, rowWidth - kFusedUnitColumns));
                 const uint32_t unit = static_cast<uint32_t>(unitStart.size());
                 unitStart.push_back(start);
@@ -2593,13 +2626,14 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             }
             const TFusedVariant* fused = nullptr;
             for (const auto& v : kFusedVariants) {
-                // (the wide fused shape is for the models of the wide evaluate kernels)
-                if (v.Six == variant->Six && unitStart.size() * kFusedUnitColumns <= v.Buckets && !fused &&
-                    (variant->Waves == 4 || v.Buckets <= 80) && m.MaxDepth <= v.Levels) {
+                // (of the rows' shapes the wide one is for the models of the wide evaluate kernels; columns over 85 to 90
+                // buckets: 1M documents, 200 trees 160 us on two launches, 134 on the shape of 160, 1000 trees 316 and 309)
+                if (v.Columns == columnMajor && v.Six == variant->Six && unitStart.size() * kFusedUnitColumns <= v.Buckets && !fused &&
+                    (variant->Waves == 4 || v.Buckets <= 80 || columnMajor) && m.MaxDepth <= v.Levels) {
                     fused = &v;
                 }
             }
-            if (!fused || (m.FusedFunction && m.FusedWaves != fused->Waves)) {
+            if (!fused) {
                 continue;
             }
             const uint32_t slots = fused->Six ? 64 : 128;           // border slots of a bucket in an image
@@ -2635,10 +2669,16 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             if (!fits) {
                 continue;
             }
-            // the records of all units the kernel has code for, one more, and the units' byte offsets in a row
-            std::vector<uint32_t> units((static_cast<size_t>(maxUnits) + 1) * kFusedUnitDwords + 16, 0);
-            for (size_t u = 0; u < unitStart.size(); ++u) {
-                units[(static_cast<size_t>(maxUnits) + 1) * kFusedUnitDwords + u] = unitStart[u] * 4;
+            // the records of all units the kernel has code for, one more, and the units' byte offsets in a row or every
+            // unit's columns (places that no bucket has read the first bucket's)
+            const size_t recordDwords = (static_cast<size_t>(maxUnits) + 1) * kFusedUnitDwords;
+            std::vector<uint32_t> units(recordDwords + (columnMajor ? (maxUnits + 1) * kFusedUnitColumns : 16), 0);
+            std::fill(units.begin() + recordDwords, units.end(), columnMajor ? columns[0] : 0);
+            for (size_t u = 0; u < unitStart.size() && !columnMajor; ++u) {
+                units[recordDwords + u] = unitStart[u] * 4;
+            }
+            for (uint32_t b = 0; b < BucketCount && columnMajor; ++b) {
+                units[recordDwords + b] = columns[b];
             }
             std::vector<uint8_t> table(images * kFusedImageBytes + fusedLeafTable.size() * sizeof(double), 0);
             for (uint32_t slot = 0; slot < fused->Buckets; ++slot) {
@@ -2684,17 +2724,15 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     row[2 * d] = row[0];
                 }
             }
-            if (!m.FusedFunction) {
-                HIP_CHECK(hipModuleGetFunction(&m.FusedFunction, m.RegModule, fused->Name));
-                m.FusedWaves = fused->Waves;
-                m.FusedKernelName = fused->Name;
-            }
-            TImpl::TFused& f = m.Fused[layoutIndex];
+            m.Fused[layoutIndex] = std::make_shared<TImpl::TFused>();
+            TImpl::TFused& f = *m.Fused[layoutIndex];
+            HIP_CHECK(hipModuleGetFunction(&f.Function, m.RegModule, fused->Name));
+            f.Waves = fused->Waves;
+            f.Name = fused->Name;
             f.UnitCount = static_cast<uint32_t>(unitStart.size());
             f.Rows.Upload(fusedRows);
             f.Units.Upload(units);
             f.Table.Upload(table);
-            f.Usable = true;
         }
     }
 
@@ -3626,11 +3664,6 @@ bool THipEvaluator::TakesSmallBatchKernel(size_t docCount, size_t treeStart, siz
            treeEnd == TreeCount && m.SmallLdsBytes() <= kMaxTileLdsBytes;
 }
 
-// Workgroups up to which a host batch's launch sets flags: every one of them orders its results before its flag, over PCIe.
-// 1000 trees of depth 6 over 100 features, whole call with the launch's event and with flags: 1 row 20.6 and 18.3 us, 4 rows
-// 20.5 and 18.5, 16 20.8 and 19.8, 24 21.0 and 20.2, 200 23.6 and 28.3.
-constexpr size_t kFlaggedGroups = 16;
-
 // One launch of the small-batch kernel whose end `stop` marks. `batch` and `results` may be device or pinned host memory.
 // `flagged`: the slot whose flags the workgroups of FewDocumentsKernel set (AwaitSmallBatch).
 static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THostContext& ctx, const TFeatureBatch& batch,
@@ -3670,11 +3703,11 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
         if (flagged != nullptr) {
             const size_t groups = docCount * passes;
             CBAMD_ENSURE(groups <= kFlaggedGroups, "internal error: more workgroups than flags");
-            if (flagged->SmallFlags.Reserve(kFlaggedGroups) || ++flagged->SmallTicket == 0) {
-                std::memset(flagged->SmallFlags.Get(), 0, kFlaggedGroups * sizeof(uint32_t));
+            if (++flagged->SmallTicket == 0) {
+                std::memset(flagged->SmallFlags(), 0, kFlaggedGroups * sizeof(uint32_t));
                 flagged->SmallTicket = 1;
             }
-            done.Flags = flagged->SmallFlags.Get();
+            done.Flags = flagged->SmallFlags();
             done.Ticket = flagged->SmallTicket;
             flagged->SmallGroups = groups;
         }
@@ -3705,7 +3738,7 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
 // Waits for the workgroups of a launch with flags. The launch itself may not have been retired when this returns; what follows
 // on its stream is ordered behind it. A launch that takes long (or has failed) is waited for as usual.
 static void AwaitSmallBatch(const THipEvaluator::TImpl::THostSlot& slot, hipEvent_t stop) {
-    const uint32_t* flags = slot.SmallFlags.Get();
+    const uint32_t* flags = slot.SmallFlags();
     const auto started = std::chrono::steady_clock::now();
     size_t group = 0;
     for (uint32_t turn = 0; group < slot.SmallGroups; ++turn) {
@@ -3720,9 +3753,9 @@ static void AwaitSmallBatch(const THipEvaluator::TImpl::THostSlot& slot, hipEven
 
 int THipEvaluator::FusedLayoutFor(int layout, size_t stride, size_t docCount, size_t treeStart, size_t treeEnd, bool anyBatchSize) const {
     const TImpl& m = *Impl;
-    const int layoutIndex = layout == TFeatureBatch::FlatRows ? 0 : layout == TFeatureBatch::SplitRows ? 1 : -1;
-    if (layoutIndex < 0 || !m.Fused[layoutIndex].Usable || docCount == 0 || treeStart != 0 || treeEnd != TreeCount ||
-        docCount >= (size_t(1) << 29) || stride >= (size_t(1) << 20)) {
+    const int layoutIndex = layout == TFeatureBatch::FlatRows ? 0 : layout == TFeatureBatch::SplitRows ? 1 : layout == TFeatureBatch::FlatColumns ? 2 : -1;
+    if (layoutIndex < 0 || !m.Fused[layoutIndex] || docCount == 0 || treeStart != 0 || treeEnd != TreeCount ||
+        docCount >= (size_t(1) << 29) || stride >= (size_t(1) << (layoutIndex == 2 ? 30 : 20))) {
         return -1;
     }
     if (!anyBatchSize && docCount < m.FusedMinDocs()) {
@@ -3738,10 +3771,13 @@ bool THipEvaluator::EvalRowsFusedDevice(const TFeatureBatch& batch, size_t docCo
     if (layoutIndex < 0) {
         return false;
     }
-    const TImpl::TFused& f = m.Fused[layoutIndex];
+    const TImpl::TFused& f = *m.Fused[layoutIndex];
     CBAMD_ENSURE(results != nullptr, "results pointer is null");
     CBAMD_ENSURE(batch.Floats != nullptr, "float features pointer is null");
-    const size_t need = layoutIndex == 0 ? m.FlatVectorSize : m.MinFloatSize;
+    if (layoutIndex == 2) {
+        CheckBatch(batch, docCount);
+    }
+    const size_t need = layoutIndex == 0 ? m.FlatVectorSize : layoutIndex == 1 ? m.MinFloatSize : 0;
     CBAMD_ENSURE(batch.Stride >= need, (layoutIndex == 0 ? "insufficient flat features vector size: " : "insufficient float features vector size: ") +
                                            std::to_string(batch.Stride) + " expected: " + std::to_string(need));
     TEvalFusedArgs args = {};
@@ -3768,20 +3804,21 @@ bool THipEvaluator::EvalRowsFusedDevice(const TFeatureBatch& batch, size_t docCo
     // (one generation) 106.0 -> 101.6 us; 4M of 200 features, 1000 trees of depth 8 1564 -> 1545, 520 000 245.3 -> 242.2,
     // 300 000 233.4 -> 232.9 (4 % longer with the whole delay for its 37 second workgroups). At 4.5 TB/s the same within
     // 1 %, at 3.5 the one-generation batches lose what they gained.
-    const uint32_t grid = (args.Reg.BlockCount + m.FusedWaves - 1) / m.FusedWaves;
+    const uint32_t grid = (args.Reg.BlockCount + f.Waves - 1) / f.Waves;
     const double secondGroups = std::min(256.0, std::max(256.0, static_cast<double>(grid)) - 256.0);
-    const double rowBytes = std::min(args.StrideBytes, f.UnitCount * kFusedUnitColumns * 4);
-    const double loadSeconds = secondGroups * m.FusedWaves * dev::kDocsPerBlock * rowBytes / 6e12, turnSeconds = 4096 / 2.4e9;
+    const uint32_t unitsBytes = f.UnitCount * kFusedUnitColumns * 4;
+    const double rowBytes = layoutIndex == 2 ? unitsBytes : std::min(args.StrideBytes, unitsBytes);
+    const double loadSeconds = secondGroups * f.Waves * dev::kDocsPerBlock * rowBytes / 6e12, turnSeconds = 4096 / 2.4e9;
     args.Reg.Bins = reinterpret_cast<const void*>(static_cast<uintptr_t>(std::min(loadSeconds / turnSeconds, 64.0)));
-    LaunchModuleWithEnd(m.FusedFunction, grid, 1, 64 * m.FusedWaves, m.Pick(stream), TakeEnd(end), args);
+    LaunchModuleWithEnd(f.Function, grid, 1, 64 * f.Waves, m.Pick(stream), TakeEnd(end), args);
     return true;
 }
 
 std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t stride) const {
     const TImpl& m = *Impl;
     // whole-model calls only: a call for a range of the trees may take other kernels
-    if (FusedLayoutFor(layout, stride, docCount, 0, TreeCount, false) >= 0) {
-        return std::string("fused=") + m.FusedKernelName;
+    if (const int fused = FusedLayoutFor(layout, stride, docCount, 0, TreeCount, false); fused >= 0) {
+        return std::string("fused=") + m.Fused[fused]->Name;
     }
     if (TakesSmallBatchKernel(docCount, 0, TreeCount)) {
         const bool few = m.TakesFewDocumentsKernel(docCount);
@@ -4353,10 +4390,13 @@ static void CalcSmallHostBatch(THipEvaluator& ev, THipEvaluator::TImpl& m, THipE
     const size_t outDim = predictionType == dev::kPredClass ? 1 : dim;
     const bool raw = predictionType == dev::kPredRaw;
     if (raw && m.TakesFewDocumentsKernel(docCount) && docCount * m.SmallPasses() <= kFlaggedGroups) {
-        slot.SmallResults.Reserve(docCount * dim);
-        LaunchSmallBatch(m, ctx, batch, docCount, slot.SmallResults.Get(), ctx.Stream, slot.Ev[3], &slot);
+        if (slot.SmallMemory.Reserve(kFlaggedGroups * sizeof(uint32_t) / sizeof(double) + docCount * dim)) {
+            std::memset(slot.SmallFlags(), 0, kFlaggedGroups * sizeof(uint32_t));
+            slot.SmallTicket = 0;
+        }
+        LaunchSmallBatch(m, ctx, batch, docCount, slot.SmallResults(), ctx.Stream, slot.Ev[3], &slot);
         AwaitSmallBatch(slot, slot.Ev[3]);
-        std::memcpy(results, slot.SmallResults.Get(), docCount * dim * sizeof(double));
+        std::memcpy(results, slot.SmallResults(), docCount * dim * sizeof(double));
     } else if (raw) {
         slot.PinnedResults.Reserve(docCount * dim);
         LaunchSmallBatch(m, ctx, batch, docCount, slot.PinnedResults.Get(), ctx.Stream, slot.Ev[3]);

@@ -176,3 +176,61 @@ def test_scalar_loads_in_flight_keep_their_registers():
                 name = gen.kernel_name(buckets, waves, 1, 256, False, six, True, levels)
                 for units in range(1, buckets // 16 + 1):
                     assert not _scalar_load_faults(text.split("\n"), units), (name, units)
+
+
+@pytest.mark.parametrize("levels", [None, 6])
+@pytest.mark.parametrize("six", [False, True])
+def test_fused_kernels_of_columns(six, levels):
+    """The column-major fused kernels: their copies follow the rows' ones, scalar loads keep their registers for any
+    number of units, and every load goes to registers that no bin and no value in flight holds."""
+    gen = _generator()
+    for buckets, waves in gen.FUSED_COLUMN_SHAPES:
+        text, _ = gen.gen_kernel(buckets, waves, 1, 256, False, six, fused=True, levels=levels, columns=True)
+        lines = text.split("\n")
+        name = gen.kernel_name(buckets, waves, 1, 256, False, six, True, levels, True)
+        assert lines[1] == ".globl " + name
+        wave_bytes = 32 * 1024 // waves
+        images = gen.fused_chunks(buckets, six)
+        rows_shape = next((b, w) for b, w in gen.FUSED_SHAPES if w == waves)
+        rows, _ = gen.gen_kernel(*rows_shape, 1, 256, False, six, fused=True, levels=levels)
+        for wave, lane in ((0, 0), (waves - 1, 63)):
+            copies, loop_at = _copies(lines, wave, lane, wave_bytes)
+            assert loop_at == (images + 1) * (wave_bytes // 1024), name
+            share = wave * wave_bytes + lane * 16
+            for index, (source, lds) in enumerate(copies):
+                assert 0 <= lds and lds + 16 <= 64 * 1024 and source < (images + 3) * 32 * 1024, (name, index)
+                assert lds % 32768 == source % 32768 == share + (index % (wave_bytes // 1024)) * 1024, (name, index)
+            expected, _ = _copies(rows.split("\n"), wave, lane, wave_bytes)
+            assert len(copies) - loop_at == len(expected) - (gen.fused_chunks(rows_shape[0], six) + 1) * (wave_bytes // 1024)
+        for units in range(1, buckets // 16 + 1):
+            assert not _scalar_load_faults(lines, units), (name, units)
+        # every column of every unit is loaded once for each of the four documents, and waited for before its search reads it
+        flying, loads, bins, aside = [], 0, set(), None
+        for line in lines[:next(i for i, l in enumerate(lines) if l == name + "_loop:")]:
+            line = line.strip()
+            found = re.match(r"s_branch (%s_c\d+_end)$" % name, line)
+            if found:  # what follows is jumped to from a turn's search, before the next loads
+                aside = found.group(1) + ":"
+            if aside is not None:
+                aside = None if line == aside else aside
+                continue
+            found = re.match(r"global_load_dword v(\d+), v\d+, s\[30:31\]$", line)
+            if found:
+                register = int(found.group(1))
+                assert register not in flying and register not in bins, (name, line)
+                flying.append(register)
+                loads += 1
+            elif line.startswith("global_load_lds"):
+                flying.append(None)
+            elif "vmcnt(" in line:
+                keep = int(re.search(r"vmcnt\((\d+)\)", line).group(1))
+                del flying[:max(0, len(flying) - keep)]
+            else:
+                used = {int(r) for r in re.findall(r"\bv(\d+)\b", line)}
+                for first, last in re.findall(r"\bv\[(\d+):(\d+)\]", line):
+                    used.update(range(int(first), int(last) + 1))
+                assert not used & set(flying), (name, line)
+                found = re.match(r"v_lshrrev_b32_e32 v(\d+), 2, v(6|7|8|9)$", line)
+                if found:
+                    bins.add(int(found.group(1)))
+        assert loads == buckets * 4 and len(bins) == buckets, (name, loads, len(bins))
