@@ -116,8 +116,8 @@ FUSED_SIX_LEVEL_BUCKETS = 208
 # Fused kernels of column-major documents ("cbamd_fused_cols_..."), every shape in the same four forms. A load is a column's value
 # for 64 neighbouring documents, so every line comes once and whole; what bounds them is vector issue at two waves per SIMD (four
 # for the shapes of 64 and 80) and the columns' arrival, as for rows. Against two launches, whole call: 1M documents, 1000
-# trees of depth 6 over 150 features 398 -> 338 us, 200 trees over 50 124 -> 90, 100 over 120 181 -> 132; 4M, 1000 trees of
-# depth 8 over 200 1800 -> 1465 (the same model on rows 1545); 270 000, 300 trees over 50 72.3 -> 66.7.
+# trees of depth 6 over 150 features 398 -> 327 us, 200 trees over 50 124 -> 89, 100 over 120 181 -> 128; 4M, 1000 trees of
+# depth 8 over 200 1800 -> 1369 (the same model on rows 1545); 270 000, 300 trees over 50 72.3 -> 66.7.
 FUSED_COLUMN_SHAPES = [(208, 4), (160, 4), (64, 8), (80, 8)]
 FUSED_MAX_STEPS = 4
 FUSED_EXTRA_SETS = 1
@@ -421,7 +421,10 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 e("  s_add_u32 s30, s30, s4")
                 e("  s_addc_u32 s31, s31, s5")
                 for j in range(4):
-                    e("  global_load_dword v%d, v%d, s[30:31]" % (value_set[turn][2 * j + c // 4] + c % 4, row_off[j]))
+                    # a line is read once, by this load: nontemporal, so that the leaf tables stay in the L2s (150 features, 1M
+                    # documents 338.7 -> 326.8 us; 200 features, 4M 1468 -> 1369; the rows' loads, which meet in lines, took
+                    # 2584 us with it instead of 1593)
+                    e("  global_load_dword v%d, v%d, s[30:31] nt" % (value_set[turn][2 * j + c // 4] + c % 4, row_off[j]))
                     pending.append(("turn", turn))
             issued.add(turn)
             if turn in after:

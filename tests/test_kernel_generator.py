@@ -214,7 +214,7 @@ def test_fused_kernels_of_columns(six, levels):
             if aside is not None:
                 aside = None if line == aside else aside
                 continue
-            found = re.match(r"global_load_dword v(\d+), v\d+, s\[30:31\]$", line)
+            found = re.match(r"global_load_dword v(\d+), v\d+, s\[30:31\] nt$", line)
             if found:
                 register = int(found.group(1))
                 assert register not in flying and register not in bins, (name, line)
