@@ -464,7 +464,7 @@ __device__ __forceinline__ uint64_t CtrHashOfCat(uint32_t v) {
 // features. What bounds it is the gathers of table entries (a line of L2 each for tables beyond the L1): one 16-byte
 // read finds and answers a lookup of up to eight buckets, where a table per CTR feature, its rows and a division and a
 // count of borders per feature took five times as long (1M documents, 16 categorical columns, 24 projections with 96 CTR
-// features: 620 us then, 107 now).
+// features: 620 us then, 107 with tables up to half full, 83 now).
 // grid = (document blocks, shares of the groups), 4 waves per workgroup, each wave a run of the share's groups.
 // TILE: the block's hashed categorical values are staged once per workgroup into LDS ([column][document]); without
 // it (more than kCtrMaxTileColumns columns) they are read from the batch where a projection needs them.
@@ -534,7 +534,8 @@ __global__ __launch_bounds__(256) void CtrBinarizeKernel(TCatSource cats, uint32
                 }
             }
         }
-        // the four documents' first probes are in flight together; at most half of a table's entries are taken, so
+        // the four documents' first probes are in flight together; at most half of a table's entries are taken (a quarter of small
+        // ones), so
         // that every probe sequence ends at its hash or at an empty entry (all ones) soon
         const uint4* table = ctr.Table + group.FirstPiece;
         uint32_t at[4];
