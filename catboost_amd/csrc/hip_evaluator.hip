@@ -2949,10 +2949,11 @@ void LaunchBinarizeRowsPC(size_t blocks, const float* floats, size_t stride, con
     // A workgroup keeps its tile's borders in LDS over up to kBinarizeBlocksPerGroup document blocks; a smaller batch gives
     // each fewer blocks, so that there are still a few generations of workgroups, whose phases overlap: 200 000 documents of
     // 100 features, 1000 trees 111.8 us with about 1024 workgroups, 109.5 with 4096; leaf indexes of 200 000 documents 218.0
-    // and 214.9; 30 000 to 100 000 documents the same. (Column-major batches, which have no tile to fill: 100 000 documents
+    // and 214.9; 30 000 to 100 000 documents the same. Tables of 256 slots (20 KB) cost a workgroup more than that gives:
+    // a CTR model of 1M documents 364 us with 1024 and 373 with 4096. (Column-major batches, which have no tile to fill: 100 000 documents
     // 69.6 and 71.7, so those keep 1024.)
     const uint32_t blocksPerGroup = static_cast<uint32_t>(
-        std::max<size_t>(1, std::min<size_t>(kBinarizeBlocksPerGroup, blocks * tiles / 4096)));
+        std::max<size_t>(1, std::min<size_t>(kBinarizeBlocksPerGroup, blocks * tiles / (LOG2P < 8 ? 4096 : 1024))));
     const size_t groups = (blocks + blocksPerGroup - 1) / blocksPerGroup;
     CBAMD_ENSURE(groups * tiles < (size_t(1) << 31), "batch is too large for one binarize launch");
     const dim3 grid(static_cast<uint32_t>(groups * tiles));
