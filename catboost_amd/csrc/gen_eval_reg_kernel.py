@@ -114,7 +114,9 @@ FUSED_SHAPES = [(208, 4), (64, 8), (80, 8)]
 # per tree that the border images' buffers are sized for, the index reaches the first 64 of them).
 FUSED_SIX_LEVEL_BUCKETS = 208
 # Fused kernels of column-major documents ("cbamd_fused_cols_..."), every shape in the same four forms. A load is a column's value
-# for 64 neighbouring documents, so every line comes once and whole; what bounds them is vector issue at two waves per SIMD (four
+# for 64 neighbouring documents: a line comes whole and, where the columns start on line boundaries, once (else a wave's load
+# shares its first and last line with its neighbours'; places of the last unit that no bucket has read the first bucket's
+# column again). What bounds them is vector issue at two waves per SIMD (four
 # for the shapes of 64 and 80) and the columns' arrival, as for rows. Against two launches, whole call: 1M documents, 1000
 # trees of depth 6 over 150 features 398 -> 327 us, 200 trees over 50 124 -> 89, 100 over 120 181 -> 128; 4M, 1000 trees of
 # depth 8 over 200 1800 -> 1369 (the same model on rows 1545); 270 000, 300 trees over 50 72.3 -> 66.7.
@@ -415,6 +417,11 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
 
         def issue_loads(turn):
             e("  s_waitcnt lgkmcnt(0)")                # the turn's columns
+            if turn[0] > 0:
+                # a unit that the model lacks: its loads are counted but fetch nothing (4M documents, 16 buckets on the shape
+                # of 64, 30 trees: 109.5 us when they read the first bucket's column, 92.8 now; 24 buckets 127 and 117)
+                e("  s_cmp_gt_u32 s28, %d" % turn[0])
+                e("  s_cselect_b64 exec, -1, 0")
             for c in range(8):
                 e("  s_mul_i32 s30, s%d, s6" % (8 + c))
                 e("  s_mul_hi_u32 s31, s%d, s6" % (8 + c))
@@ -426,6 +433,8 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                     # 2584 us with it instead of 1593)
                     e("  global_load_dword v%d, v%d, s[30:31] nt" % (value_set[turn][2 * j + c // 4] + c % 4, row_off[j]))
                     pending.append(("turn", turn))
+            if turn[0] > 0:
+                e("  s_mov_b64 exec, -1")
             issued.add(turn)
             if turn in after:
                 load_columns(after[turn])

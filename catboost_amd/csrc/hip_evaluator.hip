@@ -1596,6 +1596,15 @@ struct THipEvaluator::TImpl {
     size_t FusedMinDocs() const {
         return SmallBatchSlices ? size_t(1024) * dev::kDocsPerBlock : 0;
     }
+    // Column-major documents of models with few buckets and few trees: a fused launch loads and searches sixteen columns
+    // whatever the model has of them, and there is little else to do. Two launches against one, trees of depth 6, 4M documents:
+    // one bucket, 30 trees 55 and 78 us, 300 trees 233 and 243; four buckets, 30 trees 67 and 78, 100 trees 120 and 128; eight,
+    // 30 trees 83 and 83, 300 trees 261 and 249; twelve, 30 trees 98 and 88. 530 000 documents: one bucket, 30 trees 25 and 29,
+    // eight, 100 trees 42.8 and 43.5. (Smaller batches' trees would be cut into slices, one more launch: 500 000 documents,
+    // one bucket, 100 trees 45 and 33.)
+    bool FewColumnsForFused(size_t docCount, size_t treeCount) const {
+        return SmallBatchSlices && docCount >= (size_t(1) << 19) && BinarizeBuckets < 12 && BinarizeBuckets * treeCount < 1600;
+    }
     const char* RegKernelName = "";
 
     // small-batch kernel: tree rows of sixteen dwords, and from these dwords on the cells of its tile and the first leaves
@@ -3769,6 +3778,9 @@ int THipEvaluator::FusedLayoutFor(int layout, size_t stride, size_t docCount, si
         return -1;
     }
     if (!anyBatchSize && docCount < m.FusedMinDocs()) {
+        return -1;
+    }
+    if (!anyBatchSize && layoutIndex == 2 && m.FewColumnsForFused(docCount, TreeCount)) {
         return -1;
     }
     return layoutIndex;

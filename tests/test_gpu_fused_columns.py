@@ -105,3 +105,20 @@ def test_refused_columns_stay_refused():
     out = torch.zeros(300, dtype=torch.float64, device="cuda:0")
     with pytest.raises(Exception, match="column stride is shorter"):
         ev.eval_data(ev.features(cb.LAYOUT_FLAT_COLUMNS, x.data_ptr(), 299), 300, out.data_ptr())
+
+
+@pytest.mark.small_batch
+@pytest.mark.parametrize("used,trees,docs,fused", [
+    (1, 30, 530_000, False), (4, 100, 530_001, False), (11, 30, 600_000, False), (8, 300, 530_000, True), (12, 30, 530_000, True),
+    (4, 30, 520_000, True), (16, 30, 530_000, True), (17, 30, 530_000, True),
+])
+def test_models_of_few_columns(monkeypatch, used, trees, docs, fused):
+    """Large column-major batches of models with few buckets and few trees take two launches; both give the sums of one pass."""
+    rng = np.random.default_rng(used + trees)
+    model, _ = _model(rng, used, used, 6, 6, trees, nans=False)
+    x = rng.standard_normal((docs, used), dtype=np.float32)
+    x[::7, 0] = np.nan
+    _, ev, a = _eval(model, x, docs, monkeypatch, "1")
+    assert ("fused" in ev.describe_kernels(cb.LAYOUT_FLAT_COLUMNS, docs)) == fused
+    assert (ev.last_kernel_times()[0] == 0.0) == fused
+    np.testing.assert_array_equal(a, OracleModel(model).calc(x, threads=8))

@@ -234,3 +234,23 @@ def test_fused_kernels_of_columns(six, levels):
                 if found:
                     bins.add(int(found.group(1)))
         assert loads == buckets * 4 and len(bins) == buckets, (name, loads, len(bins))
+
+
+def test_fused_kernels_of_columns_fetch_nothing_for_units_that_the_model_lacks():
+    """The loads of every unit but the first run under a mask that is empty for a unit beyond the model's, and full again
+    behind them."""
+    gen = _generator()
+    for buckets, waves in gen.FUSED_COLUMN_SHAPES:
+        text, _ = gen.gen_kernel(buckets, waves, 1, 256, False, True, fused=True, columns=True)
+        masked, unit_loads = None, {}
+        for line in (line.strip() for line in text.split("\n")):
+            found = re.match(r"s_cmp_gt_u32 s28, (\d+)$", line)
+            if found:
+                masked = int(found.group(1))
+            elif line == "s_mov_b64 exec, -1":
+                masked = None
+            elif line.startswith("global_load_dword v") and line.endswith(" nt"):
+                unit_loads[masked] = unit_loads.get(masked, 0) + 1
+        # (the first unit, which every model has, is loaded without a mask)
+        assert unit_loads == {unit or None: 64 for unit in range(buckets // 16)}
+        assert text.count("s_cselect_b64 exec, -1, 0") == text.count("s_mov_b64 exec, -1")
