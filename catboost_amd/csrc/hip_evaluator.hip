@@ -1605,6 +1605,18 @@ struct THipEvaluator::TImpl {
     bool FewColumnsForFused(size_t docCount, size_t treeCount) const {
         return SmallBatchSlices && docCount >= (size_t(1) << 19) && BinarizeBuckets < 12 && BinarizeBuckets * treeCount < 1600;
     }
+    // Column-major batches that leave CUs without a workgroup of the fused shapes of eight waves, which last as long as one
+    // workgroup's walk whatever the batch: two launches with the trees in slices fill the chip and save about 0.3 us per 1000
+    // trees and 1000 documents below 460 000, at the price of the bins' way through memory and two more launches, about 8 us and a
+    // quarter of one per bucket. Beyond 192 workgroups the slices take another generation of them. Slices and fused, depth 6:
+    // 262 144 documents, 8 buckets, 200 trees 40 and 42 us, 20 buckets, 600 trees 68 and 93, 60, 1000 trees 113 and 145, 80, 300
+    // trees 73 and 71; 300 000, 8 buckets, 200 trees 48 and 43, 20, 600 trees 83 and 94, 60, 300 trees 76 and 67; 350 000, 20, 600
+    // trees 86 and 94, 80, 1000 trees of depth 8 165 and 166; 390 000, 20, 600 trees 90 and 94, 60, 1000 trees 150 and 146; 420 000,
+    // 20, 600 trees 107 and 94. (The shape of 160 over 92 buckets, 1000 trees: 262 144 121 and 124, 350 000 160 and 150.)
+    bool SlicesBeforeFusedColumns(size_t docCount, size_t treeCount) const {
+        return Fused[2]->Waves == 8 && docCount < size_t(192) * 8 * dev::kDocsPerBlock &&
+               (460000 - docCount) * treeCount > 26000000 + 830000 * size_t(BinarizeBuckets);
+    }
     const char* RegKernelName = "";
 
     // small-batch kernel: tree rows of sixteen dwords, and from these dwords on the cells of its tile and the first leaves
@@ -3780,7 +3792,8 @@ int THipEvaluator::FusedLayoutFor(int layout, size_t stride, size_t docCount, si
     if (!anyBatchSize && docCount < m.FusedMinDocs()) {
         return -1;
     }
-    if (!anyBatchSize && layoutIndex == 2 && m.FewColumnsForFused(docCount, TreeCount)) {
+    if (!anyBatchSize && layoutIndex == 2 &&
+        (m.FewColumnsForFused(docCount, TreeCount) || (TreeSlicesFor(docCount) > 1 && m.SlicesBeforeFusedColumns(docCount, TreeCount)))) {
         return -1;
     }
     return layoutIndex;
@@ -4053,8 +4066,10 @@ void THipEvaluator::CalcDeviceNoAlloc(const TFeatureBatch& batch, size_t docCoun
     TImpl& m = *Impl;
     const size_t maxDocs = kNoAllocScratchBytes / (static_cast<size_t>(m.LayoutBuckets) * dev::kDocsPerBlock) * dev::kDocsPerBlock;
     // the fused kernel keeps the bins in registers: no buffer at all. A batch whose bins do not fit the fixed
-    // buffer takes it whatever its size (below the size from which it is the faster as well)
-    if (EvalRowsFusedDevice(batch, docCount, treeStart, treeEnd, results, stream, docCount > maxDocs)) {
+    // buffer takes it whatever its size (below the size from which it is the faster as well),
+    // and so does one that CalcDevice would cut into slices, which this call has no memory for
+    const bool anyBatchSize = docCount > maxDocs || (docCount >= m.FusedMinDocs() && TreeSlicesFor(docCount) > 1);
+    if (EvalRowsFusedDevice(batch, docCount, treeStart, treeEnd, results, stream, anyBatchSize)) {
         return;
     }
     CBAMD_ENSURE(docCount <= maxDocs, "batch of " + std::to_string(docCount) + " documents exceeds the fixed bin buffer: at most " +

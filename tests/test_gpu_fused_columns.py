@@ -122,3 +122,30 @@ def test_models_of_few_columns(monkeypatch, used, trees, docs, fused):
     assert ("fused" in ev.describe_kernels(cb.LAYOUT_FLAT_COLUMNS, docs)) == fused
     assert (ev.last_kernel_times()[0] == 0.0) == fused
     np.testing.assert_array_equal(a, OracleModel(model).calc(x, threads=8))
+
+
+@pytest.mark.small_batch
+@pytest.mark.parametrize("used,trees,docs,fused", [(20, 1000, 262_144, False), (30, 600, 300_001, False), (20, 1000, 393_215, False), (20, 1000, 393_217, True),
+                                                   (20, 100, 262_144, True), (60, 300, 290_000, True), (80, 1200, 270_000, False),
+                                                   (150, 1000, 262_144, True)])
+def test_medium_batches_of_many_trees(monkeypatch, used, trees, docs, fused):
+    """Medium column-major batches of models with many trees are cut into slices, as smaller ones are."""
+    import torch
+
+    rng = np.random.default_rng(used + trees)
+    model, _ = _model(rng, used, used, 6, 6, trees, nans=False)
+    x = rng.standard_normal((docs, used), dtype=np.float32)
+    _, ev, a = _eval(model, x, docs, monkeypatch, "1")
+    kernels = ev.describe_kernels(cb.LAYOUT_FLAT_COLUMNS, docs)
+    assert ("fused" in kernels) == fused and ("slices" in kernels.get("evaluate", "")) != fused
+    assert (ev.last_kernel_times()[0] == 0.0) == fused
+    pick = np.r_[0:600, docs - 600:docs]
+    expected = OracleModel(model).calc(x[pick])
+    np.testing.assert_allclose(a[pick], expected, rtol=1e-9, atol=1e-12)
+    # without memory for slices: one pass, fused whatever the trees
+    columns = torch.from_numpy(np.ascontiguousarray(x.T)).to("cuda:0")
+    out = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.eval_data_no_alloc(ev.features(cb.LAYOUT_FLAT_COLUMNS, columns.data_ptr(), docs), docs, out.data_ptr())
+    ev.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy()[pick], expected)
