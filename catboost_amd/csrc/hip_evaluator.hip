@@ -344,6 +344,7 @@ constexpr TFusedVariant kFusedVariants[] = {
     {208, 4, false, 8, "cbamd_fused_cols_b208_w4", true},
     {208, 4, true, 8, "cbamd_fused_cols_b208_w4_s", true},
 };
+constexpr uint32_t kLateStartCus = 256;     // CUs of the device whose second workgroups the fused kernels of rows start late
 constexpr uint32_t kFusedUnitColumns = 16;
 constexpr uint32_t kFusedUnitDwords = 40;   // sixteen lo, sixteen scale, flags, padding
 constexpr uint32_t kFusedMaxSteps = 4;
@@ -351,7 +352,7 @@ constexpr size_t kFusedImageBytes = 32 * 1024;
 constexpr size_t kFusedLutOffset = 16 * 1024;
 
 struct TEvalFusedArgs {
-    TEvalRegArgs Reg;       // Bins: the delay of the CUs' second workgroups; Leaves: the border table images, then the leaf table
+    TEvalRegArgs Reg;       // Bins: the delay of the CUs' second workgroups (rows); Leaves: the border table images, then the leaf table
     const void* Floats;
     const void* Units;
     uint32_t StrideBytes;
@@ -1486,6 +1487,7 @@ int GetHipDeviceCount() {
 
 struct THipEvaluator::TImpl {
     int DeviceId = 0;
+    uint32_t CuCount = 0;
     hipStream_t Stream = nullptr;
     uint8_t* NoAllocScratch = nullptr;  // this device's copy of the file-scope array `scratch`
     bool Oblivious = true;
@@ -1898,6 +1900,9 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     HIP_CHECK(hipSetDevice(deviceId));
     TImpl& m = *Impl;
     m.DeviceId = deviceId;
+    int cus = 0;
+    HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, deviceId));
+    m.CuCount = static_cast<uint32_t>(cus);
     m.SmallBatchSlices = switches.SmallBatch;
     m.NoAllocScratch = NoAllocScratchOfCurrentDevice(deviceId);
     HIP_CHECK(hipStreamCreateWithFlags(&m.Stream, hipStreamNonBlocking));
@@ -3833,18 +3838,30 @@ bool THipEvaluator::EvalRowsFusedDevice(const TFeatureBatch& batch, size_t docCo
     args.Units = f.Units.Get();
     args.StrideBytes = static_cast<uint32_t>(batch.Stride * sizeof(float));
     args.UnitCount = f.UnitCount;
-    // Workgroups that start together wait for their rows together and walk their trees together. The second ones of the
-    // CUs start when the rows of the first ones have arrived (6 TB/s: early rather than late), so that one set walks while
-    // the other loads; a part of them waits less. Rows from HBM, whole call: 1M documents of 50 features, 200 trees of depth 6
-    // (one generation) 106.0 -> 101.6 us; 4M of 200 features, 1000 trees of depth 8 1564 -> 1545, 520 000 245.3 -> 242.2,
-    // 300 000 233.4 -> 232.9 (4 % longer with the whole delay for its 37 second workgroups). At 4.5 TB/s the same within
-    // 1 %, at 3.5 the one-generation batches lose what they gained.
     const uint32_t grid = (args.Reg.BlockCount + f.Waves - 1) / f.Waves;
-    const double secondGroups = std::min(256.0, std::max(256.0, static_cast<double>(grid)) - 256.0);
-    const uint32_t unitsBytes = f.UnitCount * kFusedUnitColumns * 4;
-    const double rowBytes = layoutIndex == 2 ? unitsBytes : std::min(args.StrideBytes, unitsBytes);
-    const double loadSeconds = secondGroups * f.Waves * dev::kDocsPerBlock * rowBytes / 6e12, turnSeconds = 4096 / 2.4e9;
-    args.Reg.Bins = reinterpret_cast<const void*>(static_cast<uintptr_t>(std::min(loadSeconds / turnSeconds, 64.0)));
+    // Workgroups that start together wait for their rows together and walk their trees together. The second ones of the
+    // CUs start when the rows of the first ones have arrived (6 TB/s: early rather than late; 4.5 gives the same within
+    // 1 %, with 3.5 batches of one generation lose what they gain), so that one set walks while the other loads; a part of
+    // them waits less. Rows from HBM, whole call, without and with the delay: 1M documents of 50 features, trees of depth 6:
+    // 10 trees 75.8 and 74.3 us, 100 89.4 and 87.6, 200 105.8 and 102.9, 500 158.7 and 154.9; 700 000 of 200 features, depth 8:
+    // 10 trees 152.2 and 152.2, 30 194.6 and 189.2, 500 275.0 and 264.6; 4M of 200 features, 1000 trees 1608 and 1598; rows of
+    // 64 features and up to 30 trees lose, 2M documents 127.8 and 130.5. Two to eight callers at a time gain as one does (1M
+    // documents of 200 features, 100 trees 248 and 240 us a call).
+    // Batches of one generation whose rows arrive at the full rate as they are, as columns do, would only end later: rows
+    // of up to a line or two (1M documents of 17 features, 30 trees 36.8 and 38.8 us), and, in the shapes of four waves,
+    // rows that are whole pieces of 64 bytes (520 000 documents, 1000 trees of depth 8: 128 features 208.9 and 219.8 us, 160
+    // 222.4 and 231.4, 192 220.3 and 232.3; 127 246.7 and 240.8, 145 246.7 and 243.8, 193 261.7 and 258.2; of eight waves: 1M
+    // documents of 80 features, 500 trees 177.7 and 172.9). In several generations those rows gain or lose 1 to 2 %, but
+    // rows of 512 bytes lose (128 features: 700 000 documents, 100 trees 112.7 and 118.2, 1M, 1000 trees 391.8 and 399.9).
+    const bool wholePieces = (reinterpret_cast<uintptr_t>(batch.Floats) | args.StrideBytes) % 64 == 0;
+    const bool oneGeneration = grid <= 2 * kLateStartCus;
+    const bool fullRate = f.Waves == 4 && wholePieces ? oneGeneration || args.StrideBytes % 512 == 0 : oneGeneration && args.StrideBytes <= 128;
+    if (layoutIndex != 2 && m.CuCount == kLateStartCus && !fullRate) {
+        const double secondGroups = std::min<double>(kLateStartCus, std::max<double>(kLateStartCus, grid) - kLateStartCus);
+        const double rowBytes = std::min(args.StrideBytes, f.UnitCount * kFusedUnitColumns * 4);
+        const double loadSeconds = secondGroups * f.Waves * dev::kDocsPerBlock * rowBytes / 6e12, turnSeconds = 4096 / 2.4e9;
+        args.Reg.Bins = reinterpret_cast<const void*>(static_cast<uintptr_t>(std::min(loadSeconds / turnSeconds, 64.0)));
+    }
     LaunchModuleWithEnd(f.Function, grid, 1, 64 * f.Waves, m.Pick(stream), TakeEnd(end), args);
     return true;
 }

@@ -254,3 +254,11 @@ def test_fused_kernels_of_columns_fetch_nothing_for_units_that_the_model_lacks()
         # (the first unit, which every model has, is loaded without a mask)
         assert unit_loads == {unit or None: 64 for unit in range(buckets // 16)}
         assert text.count("s_cselect_b64 exec, -1, 0") == text.count("s_mov_b64 exec, -1")
+
+
+def test_only_the_fused_kernels_of_rows_start_late():
+    gen = _generator()
+    for columns, shapes in ((False, gen.FUSED_SHAPES), (True, gen.FUSED_COLUMN_SHAPES)):
+        for buckets, waves in shapes:
+            text, _ = gen.gen_kernel(buckets, waves, 1, 256, False, True, fused=True, columns=columns)
+            assert ("s_sleep" in text) == (not columns)
