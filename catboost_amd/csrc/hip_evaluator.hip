@@ -604,8 +604,12 @@ constexpr size_t kFlaggedGroups = 16;
 // 782 workgroups, 200 as 2346, 216 as 4692 (shorter runs of a row, the bins read more often), launches back to back.
 constexpr size_t kLeafIndexWorkgroups = 2048;
 
-// Size up to which a projection's table of CTR bins is at most a quarter full instead of half.
-constexpr size_t kCtrRoomyTableBytes = size_t(16) << 20;
+// Size of all tables of CTR bins together up to which they are (usually) at most a quarter full instead of half: three times
+// an L2. Half and a quarter full, 1M documents, whole call: 36 projections of 1000 hashes (2.3 MB a quarter full) 408 and
+// 315 us, 4000 (9 MB) 459 and 421, 8000 (19 MB) 527 and 561, 16 000 (38 MB) 624 and 687; 12 projections of 8000 (6 MB) 225 and
+// 208, 16 000 (13 MB) 247 and 245, 32 000 (25 MB) 274 and 293, 115 000 (100 MB) 356 and 352. (Batches of 100 000 documents
+// gain up to 10 % at any of these sizes, by 7 to 14 us.)
+constexpr size_t kCtrRoomyBytes = size_t(12) << 20;
 
 // The cache between the L2s and HBM. What is larger is not found there by its next reader.
 constexpr size_t kMemorySideCacheBytes = size_t(256) << 20;
@@ -1334,6 +1338,45 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
         groups.push_back(group);
     }
 
+    // What the groups' tables take when the hashes of a projection's largest table fill at most half of one. Members of one
+    // table follow each other, so that each table is gone through once.
+    std::vector<std::vector<size_t>> groupOrder(groups.size());
+    std::vector<size_t> groupEntries(groups.size(), 2);
+    size_t indexBytes = 0;
+    for (const TCtrValueTable& t : tables) {
+        indexBytes += t.IndexHashRaw.size();
+    }
+    RunOnThreads(groups.size(), indexBytes >> 20, [&](size_t g) {
+        const std::vector<size_t>& members = groupFeatures[g];
+        std::vector<size_t>& order = groupOrder[g];
+        order.resize(members.size());
+        std::iota(order.begin(), order.end(), size_t(0));
+        std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return features[members[a]].Table < features[members[b]].Table; });
+        size_t keys = 0;  // of the largest table
+        for (size_t i = 0; i < order.size(); ++i) {
+            const size_t t = features[members[order[i]]].Table;
+            if (i == 0 || t != features[members[order[i - 1]]].Table) {
+                size_t rows = 0;
+                ForEachCtrRow(tables[t], [&](uint64_t, uint32_t) { ++rows; });
+                keys = std::max(keys, rows);
+            }
+        }
+        while (groupEntries[g] < 2 * keys) {
+            groupEntries[g] *= 2;
+        }
+    });
+    // A quarter where all tables together then take no more than kCtrRoomyBytes: a wave's lookups take as many rounds as the
+    // longest of its 256 probe sequences.
+    size_t tableBytes = 0;
+    for (size_t g = 0; g < groups.size(); ++g) {
+        tableBytes += groupEntries[g] * groups[g].EntryPieces * 16;
+    }
+    if (2 * tableBytes <= kCtrRoomyBytes) {
+        for (size_t& entries : groupEntries) {
+            entries *= 2;
+        }
+    }
+
     // the table of group g: entries of a hash and its bins
     const auto buildTable = [&](size_t g) {
         dev::TCtrGroupDev& group = groups[g];
@@ -1355,19 +1398,6 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
                 bins[firstByte[i] + k] = static_cast<uint8_t>(std::lower_bound(borders + begin, borders + end, value) - (borders + begin));
             }
         };
-        // members of one table follow each other, so that each table is gone through once
-        std::vector<size_t> order(members.size());
-        std::iota(order.begin(), order.end(), size_t(0));
-        std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return features[members[a]].Table < features[members[b]].Table; });
-        size_t keys = 0;  // of the largest table
-        for (size_t i = 0; i < order.size(); ++i) {
-            const size_t t = features[members[order[i]]].Table;
-            if (i == 0 || t != features[members[order[i - 1]]].Table) {
-                size_t rows = 0;
-                ForEachCtrRow(tables[t], [&](uint64_t, uint32_t) { ++rows; });
-                keys = std::max(keys, rows);
-            }
-        }
         const size_t entryDwords = 4 * static_cast<size_t>(group.EntryPieces);
         std::vector<uint32_t> unknown(entryDwords, 0);
         unknown[0] = unknown[1] = 0xffffffffu;
@@ -1376,16 +1406,8 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
         }
         // Tables of one projection were learned on the same documents and know the same hashes; where they do not, the
         // union may pass half of the entries, and the table is built again with twice as many.
-        size_t entries = 2;
-        while (entries < 2 * keys) {
-            entries *= 2;
-        }
-        // At most a quarter full where that takes no more than kCtrRoomyTableBytes: a wave's lookups take as many rounds as
-        // the longest of its 256 probe sequences. 1M documents, 24 projections 397 -> 373 us, 300 000, 36 projections
-        // 138.7 -> 115.2, 2M, 12 projections 345 -> 320 (an eighth full: 376, 116, 318).
-        if (entries * 2 * entryDwords * sizeof(uint32_t) <= kCtrRoomyTableBytes) {
-            entries *= 2;
-        }
+        const std::vector<size_t>& order = groupOrder[g];
+        size_t entries = groupEntries[g];
         const auto build = [&] {
             CBAMD_ENSURE(entries <= (size_t(1) << 31), "CTR tables are too large");
             table.clear();
@@ -1441,10 +1463,6 @@ void BuildCtrTables(const TModelTrees& trees, const TFeaturePositions& positions
     // The groups' tables, side by side on the host's threads: 8 categorical columns of 400 000 values each and 4 pairs of
     // them, 48 CTR features, 0.10 s; 0.87 on one thread.
     std::vector<std::vector<uint32_t>> groupTables(groups.size());
-    size_t indexBytes = 0;
-    for (const TCtrValueTable& t : tables) {
-        indexBytes += t.IndexHashRaw.size();
-    }
     RunOnThreads(groups.size(), indexBytes >> 18, [&](size_t g) { groupTables[g] = buildTable(g); });
     size_t pieces = 0;
     for (size_t g = 0; g < groups.size(); ++g) {

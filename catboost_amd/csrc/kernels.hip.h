@@ -534,9 +534,8 @@ __global__ __launch_bounds__(256) void CtrBinarizeKernel(TCatSource cats, uint32
                 }
             }
         }
-        // the four documents' first probes are in flight together; at most half of a table's entries are taken (a quarter of small
-        // ones), so
-        // that every probe sequence ends at its hash or at an empty entry (all ones) soon
+        // the four documents' first probes are in flight together; at most half of a table's entries are taken (a quarter where
+        // the tables are small together), so that every probe sequence ends at its hash or at an empty entry (all ones) soon
         const uint4* table = ctr.Table + group.FirstPiece;
         uint32_t at[4];
         uint4 entry[4];

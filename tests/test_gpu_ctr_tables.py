@@ -60,3 +60,47 @@ def test_large_tables_are_built_side_by_side():
     bins = g.quantize_hashed(floats, cats)
     np.testing.assert_array_equal(bins, o.binarize(floats, cats, layout="split"))
     np.testing.assert_allclose(g.calc_hashed(floats, cats), o.calc(floats, cats, layout="split"), rtol=1e-9, atol=1e-12)
+
+
+def _model_of_large_tables(more_hashes):
+    model, known = ctr_models.random_ctr_model(23, n_cat=6, n_bases=15, n_trees=30)
+    for table in model["ctr_tables"]:
+        rng = np.random.default_rng(23)  # the same hashes in every table of a projection
+        index = table["index_hash_raw"].view(np.dtype([("hash", "<u8"), ("row", "<u4")]))
+        index = np.sort(index[index["hash"] != np.uint64(ctr_models.MASK64)], order="row")
+        rows = table["ctr_blob"].reshape(len(index), -1)
+        keys = np.unique(np.concatenate([index["hash"], rng.integers(0, 2**63, size=more_hashes, dtype=np.uint64)]))
+        row_of = {int(h): int(r) for h, r in index}
+        table["index_hash_raw"] = ctr_models.build_index_hash([int(h) for h in keys])
+        table["ctr_blob"] = rows[[row_of.get(int(h), i % len(rows)) for i, h in enumerate(keys)]].ravel().copy()
+    return model, known
+
+
+@pytest.mark.parametrize("more_hashes,roomy", [(3000, True), (60_000, False)])
+def test_tables_are_roomy_only_while_they_are_small_together(more_hashes, roomy):
+    """Tables a quarter full cost lookups more than they give once all of them together outgrow the L2s."""
+    import torch
+
+    model, known = _model_of_large_tables(more_hashes)
+    data = write_cbm(model)
+    projections = {(tuple(c["base"]["cat_features"]), tuple(c["base"]["float_splits"]), tuple(c["base"]["one_hot_splits"]))
+                   for c in model["ctr_features"]}
+    entries = 2
+    while entries < 2 * more_hashes:
+        entries *= 2
+    half = len(projections) * entries * 16  # (entries of one piece, and of two where a projection has many features)
+    assert (2 * half <= 10 << 20) == roomy and (half > 12 << 20) != roomy
+    warm = cb.ModelCalcer(buffer=write_cbm(_model_of_large_tables(10)[0]))
+    warm.enable_gpu_evaluation(0)
+    warm.evaluator()
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    g = cb.ModelCalcer(buffer=data)
+    g.enable_gpu_evaluation(0)
+    g.evaluator()
+    used = before - torch.cuda.mem_get_info()[0]
+    if not roomy:
+        assert half <= used < 1.9 * half, (used, half)
+    o = OracleModel(read_cbm(data))
+    floats, cats = ctr_models.random_documents(model, known, 3000, 5)
+    np.testing.assert_array_equal(g.quantize_hashed(floats, cats), o.binarize(floats, cats, layout="split"))
