@@ -83,12 +83,15 @@ def test_columns_further_apart_than_32_bits_reach(monkeypatch):
     np.testing.assert_array_equal(a, OracleModel(model).calc(x))
 
 
-def test_large_batch_of_columns_with_late_second_workgroups(monkeypatch):
-    """More than 256 workgroups: the second ones of the CUs start late."""
+@pytest.mark.parametrize("docs", [410_003, 1_100_003])
+def test_large_batches_of_columns(monkeypatch, docs):
+    """More workgroups than CUs, and more than the chip holds at a time."""
     rng = np.random.default_rng(4)
     model, _ = _model(rng, 120, 120, 40, 6, 100, nans=False)
-    x = rng.standard_normal((410_003, 120), dtype=np.float32)
-    _, _, a = _eval(model, x, 410_003, monkeypatch, "1")
+    x = rng.standard_normal((docs, 120), dtype=np.float32)
+    _, ev, a = _eval(model, x, docs, monkeypatch, "1")
+    assert ev.describe_kernels(cb.LAYOUT_FLAT_COLUMNS, docs)["fused"] == "cbamd_fused_cols_b160_w4_d6_s"
+    assert ev.last_kernel_times()[0] == 0.0, "the fused kernel did not run"
     np.testing.assert_array_equal(a, OracleModel(model).calc(x, threads=8))
 
 
