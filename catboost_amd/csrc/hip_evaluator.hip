@@ -493,6 +493,9 @@ struct TKernelSwitches {
     bool RowTile = true;          // CATBOOST_AMD_ROW_TILE=0: the tile kernel that broadcasts a tree's levels from a lane
     bool RegSplit = true;         // CATBOOST_AMD_REG_SPLIT=0: buckets of more than 127 values send a model to the mixed kernels
     uint32_t NsWaves = 0;         // CATBOOST_AMD_NS_WAVES=4|6|8|10|11|12|16: shapes of the non-symmetric LDS kernel with so many waves or none
+    uint32_t FlagTicket = 0;      // CATBOOST_AMD_FLAG_TICKET=n: the first ticket of few host documents' flags is n + 1; their waits are counted
+    bool CountFlagged = false;
+    uint32_t FlagWaitUs = 200;    // CATBOOST_AMD_FLAG_WAIT_US=n: microseconds after which such a call waits for its launch instead
 
     static TKernelSwitches FromEnvironment() {
         const auto off = [](const char* name) {
@@ -515,6 +518,13 @@ struct TKernelSwitches {
         k.RegSplit = !off("CATBOOST_AMD_REG_SPLIT");
         if (const char* v = std::getenv("CATBOOST_AMD_NS_WAVES")) {
             k.NsWaves = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
+        }
+        if (const char* v = std::getenv("CATBOOST_AMD_FLAG_TICKET")) {
+            k.FlagTicket = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
+            k.CountFlagged = true;
+        }
+        if (const char* v = std::getenv("CATBOOST_AMD_FLAG_WAIT_US")) {
+            k.FlagWaitUs = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
         }
         if (const char* v = std::getenv("CATBOOST_AMD_REG_MIN_BUCKETS")) {
             k.RegMinBuckets = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
@@ -1506,6 +1516,10 @@ int GetHipDeviceCount() {
 struct THipEvaluator::TImpl {
     int DeviceId = 0;
     uint32_t CuCount = 0;
+    // flags of few host documents (the switches of tests): first ticket, longest wait, calls that their flags ended
+    uint32_t FlagTicket = 0, FlagWaitUs = 200;
+    bool CountFlagged = false;
+    std::atomic<uint64_t> FlaggedCalls{0};
     hipStream_t Stream = nullptr;
     uint8_t* NoAllocScratch = nullptr;  // this device's copy of the file-scope array `scratch`
     bool Oblivious = true;
@@ -1922,6 +1936,9 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, deviceId));
     m.CuCount = static_cast<uint32_t>(cus);
     m.SmallBatchSlices = switches.SmallBatch;
+    m.FlagTicket = switches.FlagTicket;
+    m.CountFlagged = switches.CountFlagged;
+    m.FlagWaitUs = switches.FlagWaitUs;
     m.NoAllocScratch = NoAllocScratchOfCurrentDevice(deviceId);
     HIP_CHECK(hipStreamCreateWithFlags(&m.Stream, hipStreamNonBlocking));
     TreeCount = trees.GetTreeCount();
@@ -3791,17 +3808,20 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
 
 // Waits for the workgroups of a launch with flags. The launch itself may not have been retired when this returns; what follows
 // on its stream is ordered behind it. A launch that takes long (or has failed) is waited for as usual.
-static void AwaitSmallBatch(const THipEvaluator::TImpl::THostSlot& slot, hipEvent_t stop) {
+static void AwaitSmallBatch(THipEvaluator::TImpl& m, const THipEvaluator::TImpl::THostSlot& slot, hipEvent_t stop) {
     const uint32_t* flags = slot.SmallFlags();
     const auto started = std::chrono::steady_clock::now();
     size_t group = 0;
     for (uint32_t turn = 0; group < slot.SmallGroups; ++turn) {
         if (__atomic_load_n(flags + group, __ATOMIC_ACQUIRE) == slot.SmallTicket) {
             ++group;
-        } else if (turn % 256 == 255 && std::chrono::steady_clock::now() - started > std::chrono::microseconds(200)) {
+        } else if ((turn % 256 == 255 || m.FlagWaitUs == 0) && std::chrono::steady_clock::now() - started >= std::chrono::microseconds(m.FlagWaitUs)) {
             HIP_CHECK(hipEventSynchronize(stop));
             return;
         }
+    }
+    if (m.CountFlagged) {
+        m.FlaggedCalls.fetch_add(1, std::memory_order_relaxed);
     }
 }
 
@@ -3893,7 +3913,8 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
     if (TakesSmallBatchKernel(docCount, 0, TreeCount)) {
         const bool few = m.TakesFewDocumentsKernel(docCount);
         return std::string("binarize=none;evaluate=") + (few ? "FewDocumentsKernel<" : "SmallBatchKernel<") + std::to_string(m.MaxDepth <= 6 ? 6 : 8) + ", " + std::to_string(m.SmallDims()) +
-               ">, " + std::to_string(m.SmallSliceCount()) + " slices of the trees";
+               ">, " + std::to_string(m.SmallSliceCount()) + " slices of the trees" +
+               (m.CountFlagged ? ";flagged=" + std::to_string(m.FlaggedCalls.load()) : "");
     }
     std::string binarize = m.BinarizeBuckets == 0 ? "none"
                            : layout == TFeatureBatch::FlatColumns
@@ -4464,10 +4485,10 @@ static void CalcSmallHostBatch(THipEvaluator& ev, THipEvaluator::TImpl& m, THipE
     if (raw && m.TakesFewDocumentsKernel(docCount) && docCount * m.SmallPasses() <= kFlaggedGroups) {
         if (slot.SmallMemory.Reserve(kFlaggedGroups * sizeof(uint32_t) / sizeof(double) + docCount * dim)) {
             std::memset(slot.SmallFlags(), 0, kFlaggedGroups * sizeof(uint32_t));
-            slot.SmallTicket = 0;
+            slot.SmallTicket = m.FlagTicket;
         }
         LaunchSmallBatch(m, ctx, batch, docCount, slot.SmallResults(), ctx.Stream, slot.Ev[3], &slot);
-        AwaitSmallBatch(slot, slot.Ev[3]);
+        AwaitSmallBatch(m, slot, slot.Ev[3]);
         std::memcpy(results, slot.SmallResults(), docCount * dim * sizeof(double));
     } else if (raw) {
         slot.PinnedResults.Reserve(docCount * dim);

@@ -98,7 +98,11 @@ typedef struct CbHipFeatures {
  *   CATBOOST_AMD_NS_WAVES=4|6|8|12|16 non-symmetric models walked out of LDS: only that many waves per workgroup
  *                                    (regions of 2048, 1536 or 1024 tree entries) instead of the most that hold
  *                                    the model's largest tree
- *   CATBOOST_AMD_CTR_TILE=0          the plain CTR kernel instead of the LDS tile one */
+ *   CATBOOST_AMD_CTR_TILE=0          the plain CTR kernel instead of the LDS tile one
+ *   CATBOOST_AMD_FLAG_TICKET=n       calls of few host documents, which return when their workgroups have set flags in
+ *                                    host memory: the flags' first ticket is n + 1, and CbHipDescribeKernels for a small
+ *                                    batch ends with ";flagged=<calls that their flags have ended>"
+ *   CATBOOST_AMD_FLAG_WAIT_US=n      such a call waits for its launch after n microseconds instead of 200 */
 
 /* Model upload: validates the tables, derives buckets / repacked splits / leaf offsets and
  * copies SoA tables to device `deviceId` (takes the place of the TGpuEvaluator constructor,

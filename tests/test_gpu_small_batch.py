@@ -485,3 +485,39 @@ def test_few_host_documents_whose_workgroups_set_flags(dim, n_float):
     for t in threads:
         t.join()
     assert not failures, failures[0]
+
+
+@pytest.mark.small_batch
+@pytest.mark.parametrize("ticket,wait_us", [(0, "1000000"), (2**32 - 21, "1000000"), (0, "0")])
+def test_which_wait_ends_calls_of_few_host_documents(monkeypatch, ticket, wait_us):
+    """Up to sixteen workgroups the flags end a call, also where the ticket wraps around; above, and where the flags take
+    longer than the wait for them, the launch's event does."""
+    monkeypatch.setenv("CATBOOST_AMD_FLAG_TICKET", str(ticket))
+    monkeypatch.setenv("CATBOOST_AMD_FLAG_WAIT_US", wait_us)
+    rng = np.random.default_rng(ticket % 1000)
+    ffs = [mb.float_feature(i, i) for i in range(60)]
+    trees = []
+    for _ in range(300):
+        splits = [("float", int(f), float(np.float32(b))) for f, b in zip(rng.integers(0, 60, 6), rng.normal(size=6))]
+        trees.append((splits, rng.normal(size=64)))
+    model = mb.build_oblivious(ffs, [], 1, trees, bias=[0.25])
+    m = cb.ModelCalcer()
+    m.load_from_dict(model)
+    m.enable_gpu_evaluation(0)
+    x = rng.normal(size=(40, 60)).astype(np.float32)
+    expected = m.calc_flat(x)  # the launch's event
+    np.testing.assert_allclose(expected, OracleModel(model).calc(x), rtol=1e-9, atol=1e-12)
+
+    def flagged():
+        return int(m.evaluator().describe_kernels(cb.LAYOUT_FLAT_ROWS, 1)["flagged"])
+
+    assert flagged() == 0
+    m.calc_flat(x[:16])  # (makes the memory, which takes longer than the launch)
+    began = flagged()
+    for call in range(50):
+        docs = 1 + call % 16
+        np.testing.assert_array_equal(m.calc_flat(x[call % 24:call % 24 + docs]), expected[call % 24:call % 24 + docs])
+    assert flagged() - began == (50 if wait_us != "0" else 0)
+    for docs in (17, 40):
+        np.testing.assert_array_equal(m.calc_flat(x[:docs]), expected[:docs])
+    assert flagged() - began == (50 if wait_us != "0" else 0)
