@@ -2,9 +2,9 @@
 
 The kernels evaluate oblivious trees of depth <= 8 (LEAVES = 64 or 256; LEAVES = 1024: depth <= 10, one
 dimension, plain and six-bit forms, level tables of 32 dwords of which the first 20 are used, the two extra
-levels' bits in a second index byte per document). The plain variants take models whose bins and
-split indexes all fit 7 bits (no xor masks), the case of float-feature models with at most 127
-used borders per feature; the "_s" variants take such models when no feature uses more than 63
+levels' bits in a second index byte per document). The plain variants take models without xor masks
+whose bins are at most 128, the case of float-feature models with at most 128 used borders per
+feature (others are split over two registers); the "_s" variants take such models when no feature uses more than 64
 borders, which lets two levels share their merge; the "_m" (mixed) variants take any bins and xor masks (one-hot splits)
 and choose the compare per tree. One launch produces PITCH consecutive dimensions of the result
 (1 for a one-dimensional model).
@@ -23,9 +23,9 @@ Layout of the work:
   * a tree's levels come from a table of 16 dwords per tree, (bucket, (128 - splitIdx) * 0x01010101)
     per level, read with one scalar load two trees ahead; kernels for LEAVES = 64 use the first six.
     Six-bit variants: the even levels' constant is (64 - splitIdx) * 0x01010101, which puts the level's
-    bit in bit 6 of every byte (all bins are below 64), next to the following level's in bit 7.
+    bit in bit 6 of every byte (all bins are at most 64), next to the following level's in bit 7.
     Mixed variants: 32 dwords per tree. Bit 31 of the first dword clear: the 7-bit form above (the
-    tree has no xor mask and all bins of its buckets fit 7 bits). Set: 4 dwords per level, bucket,
+    tree has no xor mask and no bin of its buckets is above 128). Set: 4 dwords per level, bucket,
     xorMask, splitIdx & 0x7f (both times 0x01010101) and 0x80808080 if splitIdx < 128 else 0; the
     unsigned byte compare (bin ^ xorMask) >= splitIdx is then bit 7 of
     majority(x, (x | 0x80) - (splitIdx & 0x7f), splitIdx < 128) taken per byte, x = bin ^ xorMask;
@@ -119,7 +119,7 @@ FUSED_SIX_LEVEL_BUCKETS = 208
 # column again). What bounds them is vector issue at two waves per SIMD (four
 # for the shapes of 64 and 80) and the columns' arrival, as for rows. Against two launches, whole call: 1M documents, 1000
 # trees of depth 6 over 150 features 398 -> 327 us, 200 trees over 50 124 -> 89, 100 over 120 181 -> 128; 4M, 1000 trees of
-# depth 8 over 200 1800 -> 1369 (the same model on rows 1545); 270 000, 300 trees over 50 72.3 -> 66.7.
+# depth 8 over 200 1800 -> 1369 (the same model on rows 1593); 270 000, 300 trees over 50 72.3 -> 66.7.
 FUSED_COLUMN_SHAPES = [(208, 4), (160, 4), (64, 8), (80, 8)]
 FUSED_MAX_STEPS = 4
 FUSED_EXTRA_SETS = 1
@@ -294,7 +294,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 e("  v_bfi_b32 v3, s22, v4, v3")
 
     def levels_six_bit(rows):
-        """Bins below 64 everywhere: the host gives the even levels the constant (64 - splitIdx), whose sum
+        """Bins of at most 64 everywhere: the host gives the even levels the constant (64 - splitIdx), whose sum
         has the level's bit in bit 6 (and bit 7 clear), the odd levels (128 - splitIdx) as in the 7-bit
         form. A pair of levels is then merged into the index with one shift: five instructions for two
         levels instead of six. What the first pair leaves below its two bits goes the way the 7-bit
@@ -827,7 +827,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         if True:
             # Flags bit 3: the bins registers follow a map, one dword per register: bits 0..15 the bucket it
             # is loaded from, bits 16.. what becomes of the bins there: 0 as they are, 1 min(bin, 127), 2
-            # max(bin - 127, 0). A float bucket with more than 127 values then takes two registers, and a level
+            # max(bin - 127, 0). A float bucket with more than 128 values then takes two registers, and a level
             # "bin >= s" reads the first (s <= 127) or the second (with s - 127): every tree without xor
             # masks runs in the 7-bit form. The map has ceil(BUCKETS / 16) * 16 entries.
             e("  s_branch %s_loaded" % name)

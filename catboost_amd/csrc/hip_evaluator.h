@@ -67,13 +67,14 @@ public:
     size_t TreeSliceScratchDoubles(size_t docCount) const;
     void EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCount, double* results, double* partials, void* stream,
                                    TStageEnd* end = nullptr);
-    // binarize + evaluate in one launch of a fused kernel, the bins in registers only; false (and nothing
-    // launched) when the model, the batch layout or the tree range has no fused kernel
-    // (anyBatchSize: also below the batch size from which the fused launch is the faster one)
-    bool EvalRowsFusedDevice(const TFeatureBatch& batch, size_t docCount, size_t treeStart, size_t treeEnd,
-                             double* results, void* stream, bool anyBatchSize = false, TStageEnd* end = nullptr);
-    // index of the fused kernel tables that such a call would use (0 flat rows, 1 split rows), -1 when it takes
-    // the two launches: the one test that EvalRowsFusedDevice, the host pipeline and DescribeKernels share
+    // binarize + evaluate in one launch of a fused kernel (rows or columns), the bins in registers only; false (and nothing
+    // launched) when the model, the batch layout or the tree range has no fused kernel, or two launches are the faster way
+    // (anyBatchSize: also where they are)
+    bool EvalFusedDevice(const TFeatureBatch& batch, size_t docCount, size_t treeStart, size_t treeEnd,
+                         double* results, void* stream, bool anyBatchSize = false, TStageEnd* end = nullptr);
+    // index of the fused kernel tables that such a call would use (0 flat rows, 1 split rows, 2 flat columns), -1 when it
+    // takes the two launches (always with a stride of 2^20 floats or more between rows, of 2^30 or more between columns, and
+    // from 2^29 documents on): the one test that EvalFusedDevice, the host pipeline and DescribeKernels share
     int FusedLayoutFor(int layout, size_t stride, size_t docCount, size_t treeStart, size_t treeEnd, bool anyBatchSize) const;
     // Batches of oblivious models that are too small to fill the chip: one launch from the features to the results,
     // the trees in the slices of TreeSlicesFor. `source` and `results` may be device or pinned host memory. True when

@@ -234,7 +234,7 @@ struct TEvalRegVariant {
     uint32_t Pitch;   // dimensions per launch = doubles per leaf row
     uint32_t Leaves;  // leaf rows per tree (64: trees of depth <= 6)
     bool Mixed;       // 32-dword level tables, compare form chosen per tree
-    bool Six;         // every bin below 64: even levels compare into bit 6, two levels share a merge
+    bool Six;         // every bin at most 64: even levels compare into bit 6, two levels share a merge
     const char* Name;
 };
 constexpr TEvalRegVariant kEvalRegVariants[] = {
@@ -397,7 +397,7 @@ uint32_t RegTreeBlock(const TEvalRegVariant& v) {
 
 // The variant for a model: one-dimensional models take the smallest register file that holds
 // their buckets; others the pitch that needs the fewest launches (then the smallest such pitch).
-// mixed: the model has one-hot splits or bins above 127.
+// mixed: the model has one-hot splits, or bins above 128 that stay in one register.
 const TEvalRegVariant* PickRegVariant(uint32_t buckets, uint32_t dim, uint32_t maxDepth, bool mixed, bool six,
                                       uint32_t minVariantBuckets = 0) {
     const TEvalRegVariant* best = nullptr;
@@ -491,7 +491,7 @@ struct TKernelSwitches {
     bool LevelOrder = true;       // CATBOOST_AMD_LEVEL_ORDER=0: register kernels keep the model's order of a tree's levels
     bool PairTile = true;         // CATBOOST_AMD_PAIR_TILE=0: the half-tile kernel with one tree per wave
     bool RowTile = true;          // CATBOOST_AMD_ROW_TILE=0: the tile kernel that broadcasts a tree's levels from a lane
-    bool RegSplit = true;         // CATBOOST_AMD_REG_SPLIT=0: buckets of more than 127 values send a model to the mixed kernels
+    bool RegSplit = true;         // CATBOOST_AMD_REG_SPLIT=0: a bucket keeps to one register: more than 127 values send a model to the mixed kernels
     uint32_t NsWaves = 0;         // CATBOOST_AMD_NS_WAVES=4|6|8|10|11|12|16: shapes of the non-symmetric LDS kernel with so many waves or none
     uint32_t FlagTicket = 0;      // CATBOOST_AMD_FLAG_TICKET=n: the first ticket of few host documents' flags is n + 1; their waits are counted
     bool CountFlagged = false;
@@ -1610,7 +1610,7 @@ struct THipEvaluator::TImpl {
     };
     std::vector<TRegLaunch> RegLaunches;
     TDeviceVec<double> RegTailLeaves;  // leaf table of a last launch that uses another kernel
-    // Models without xor masks whose buckets hold more than 127 values: such a bucket takes two bins registers,
+    // Models without xor masks whose buckets hold more than 128 values: such a bucket takes two bins registers,
     // min(bin, 127) and max(bin - 127, 0), so that every level is a 7-bit compare (the kernels' register map)
     TDeviceVec<uint32_t> RegMap;
 
@@ -2414,7 +2414,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     // none (constant 0) would then be true for the largest bin: the leaf tables repeat a tree's values in the rows
     // that such levels choose between. 1M documents, 1000 trees of depth 6, 116 buckets of which 20 have 128 values:
     // 136 registers and two waves per SIMD before, 116 and three now, evaluate launch 243 -> 216 us.
-    // Both limits are the only difference to 127 and 63 values, so nothing else of the dispatch depends on them.
+    // (The tile kernels keep to 127 and 63 values: their leaf tables have no rows to repeat.)
     const uint32_t sevenBitValues = switches.RegSplit ? 128 : 127;
     const bool regSevenBit = m.Oblivious && !m.HasOneHot && m.MaxBucketValues <= sevenBitValues;
     const bool six = regSevenBit && m.MaxBucketValues <= 64 && switches.RegSix;
@@ -2486,7 +2486,10 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         const size_t tailTableTrees = ((TreeCount + tailBlock - 1) / tailBlock + 2) * tailBlock;
         // tree ranges are cut at blocks of the kernel with the larger block (both are powers of two)
         m.RegTreeBlockSize = std::max(block, tailBlock);
-        std::vector<uint32_t> rows(std::max(tableTrees, tailTableTrees) * rowDwords, 0);  // 7-bit form (bucket 0, add 0): false for every bin
+        // A level that stands for none (bucket 0 or the tree's first one, add 0) is true for the bins from 128 on, in the six-bit form
+        // from 64 on at its even levels. Nothing may depend on it: the leaf tables repeat a tree's values in all rows that such
+        // levels choose between, and the trees that fill up the last block have zeros in all of theirs.
+        std::vector<uint32_t> rows(std::max(tableTrees, tailTableTrees) * rowDwords, 0);
         std::vector<double> leaves((tailVariant ? launches - 1 : launches) * m.RegLaunchLeaves, 0.0);
         std::vector<double> tailLeaves(tailVariant ? tailTableTrees * rowsPerTree * tailPitch : 0, 0.0);
         // Order of a tree's levels in these tables (levelOrder[t][position] = level of the model). The leaf
@@ -2540,10 +2543,6 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                            (regMapped || offsets[rb.FeatureIndex + 1] - offsets[rb.FeatureIndex] <= sevenBitValues);
             }
             CBAMD_ENSURE(sevenBit || variant->Mixed, "internal error: tree needs the 8-bit compare");
-            // a mixed model's bucket 0 may hold bins above 127, which the 7-bit padding level
-            // (bucket 0, add 0) would take for true: a tree without levels goes the 8-bit way and
-            // the padding levels of the others use the tree's own first bucket
-            sevenBit = sevenBit && (depth > 0 || !variant->Mixed);
             uint32_t* row = rows.data() + t * rowDwords;
             if (sevenBit) {
                 for (int d = 0; d < depth; ++d) {
@@ -3842,8 +3841,8 @@ int THipEvaluator::FusedLayoutFor(int layout, size_t stride, size_t docCount, si
     return layoutIndex;
 }
 
-bool THipEvaluator::EvalRowsFusedDevice(const TFeatureBatch& batch, size_t docCount, size_t treeStart, size_t treeEnd,
-                                        double* results, void* stream, bool anyBatchSize, TStageEnd* end) {
+bool THipEvaluator::EvalFusedDevice(const TFeatureBatch& batch, size_t docCount, size_t treeStart, size_t treeEnd,
+                                    double* results, void* stream, bool anyBatchSize, TStageEnd* end) {
     TImpl& m = *Impl;
     const int layoutIndex = FusedLayoutFor(batch.Layout, batch.Stride, docCount, treeStart, treeEnd, anyBatchSize);
     if (layoutIndex < 0) {
@@ -4083,7 +4082,7 @@ void THipEvaluator::CalcDevice(const TFeatureBatch& batch, size_t docCount, size
     TKernelTimes times;
     TStageEnd binarizeEnd{ctx->Ev[1]}, evalEnd{ctx->Ev[2]};
     HIP_CHECK(hipEventRecord(ctx->Ev[0], s));
-    if (EvalRowsFusedDevice(batch, docCount, treeStart, treeEnd, results, s, false, &evalEnd)) {
+    if (EvalFusedDevice(batch, docCount, treeStart, treeEnd, results, s, false, &evalEnd)) {
         // one launch does both: its whole duration is reported as the evaluate time
         evalEnd.Close(s);
         HIP_CHECK(hipEventSynchronize(ctx->Ev[2]));
@@ -4125,7 +4124,7 @@ void THipEvaluator::CalcDeviceNoAlloc(const TFeatureBatch& batch, size_t docCoun
     // buffer takes it whatever its size (below the size from which it is the faster as well),
     // and so does one that CalcDevice would cut into slices, which this call has no memory for
     const bool anyBatchSize = docCount > maxDocs || (docCount >= m.FusedMinDocs() && TreeSlicesFor(docCount) > 1);
-    if (EvalRowsFusedDevice(batch, docCount, treeStart, treeEnd, results, stream, anyBatchSize)) {
+    if (EvalFusedDevice(batch, docCount, treeStart, treeEnd, results, stream, anyBatchSize)) {
         return;
     }
     CBAMD_ENSURE(docCount <= maxDocs, "batch of " + std::to_string(docCount) + " documents exceeds the fixed bin buffer: at most " +
@@ -4422,7 +4421,7 @@ static void RunPredictionChunk(THipEvaluator& ev, THipEvaluator::TImpl::THostCon
     if (ev.FusedLayoutFor(batch.Layout, batch.Stride, n, treeStart, treeEnd, false) >= 0) {
         // one launch does both: its whole duration is reported as the evaluate time, as CalcDevice does
         binarizeEnd.Close(s);
-        ev.EvalRowsFusedDevice(batch, n, treeStart, treeEnd, slot.StageResults.Get(), s, false, &evalEnd);
+        ev.EvalFusedDevice(batch, n, treeStart, treeEnd, slot.StageResults.Get(), s, false, &evalEnd);
     } else {
         ev.QuantizeDevice(batch, n, ctx.ScratchBins.Get(), s, &binarizeEnd);
         binarizeEnd.Close(s);

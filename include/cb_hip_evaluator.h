@@ -85,8 +85,8 @@ typedef struct CbHipFeatures {
  *   CATBOOST_AMD_REG_KERNEL=0        no register-resident assembly kernels (the LDS tile kernels instead)
  *   CATBOOST_AMD_REG_SIX=0           no six-bit form of the register-resident kernels and of the pair-tile kernel
  *   CATBOOST_AMD_REG_MIN_BUCKETS=n   only register-resident kernel shapes that hold n buckets or more
- *   CATBOOST_AMD_REG_SPLIT=0         a float feature with more than 127 used borders sends the model to the mixed
- *                                    (8-bit compare) kernels instead of taking two bins registers
+ *   CATBOOST_AMD_REG_SPLIT=0         a float feature keeps to one bins register: more than 127 used borders send the
+ *                                    model to the mixed (8-bit compare) kernels (else: more than 128 take two)
  *   CATBOOST_AMD_SMALL_BATCH=0       the start value of CbHipSetSmallBatchSlicing is "off"
  *   CATBOOST_AMD_LEVEL_ORDER=0       register-resident kernels keep the model's order of a tree's levels
  *   CATBOOST_AMD_FUSED=0             binarize and evaluate always as two launches (no fused kernels)
