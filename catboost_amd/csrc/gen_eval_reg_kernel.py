@@ -118,8 +118,8 @@ FUSED_SIX_LEVEL_BUCKETS = 208
 # shares its first and last line with its neighbours'; places of the last unit that no bucket has read the first bucket's
 # column again). What bounds them is vector issue at two waves per SIMD (four
 # for the shapes of 64 and 80) and the columns' arrival, as for rows. Against two launches, whole call: 1M documents, 1000
-# trees of depth 6 over 150 features 398 -> 327 us, 200 trees over 50 124 -> 89, 100 over 120 181 -> 128; 4M, 1000 trees of
-# depth 8 over 200 1800 -> 1369 (the same model on rows 1593); 270 000, 300 trees over 50 72.3 -> 66.7.
+# trees of depth 6 over 150 features 398 -> 317 us, 200 trees over 50 124 -> 87, 100 over 120 181 -> 123; 4M, 1000 trees of
+# depth 8 over 200 1799 -> 1418 (the same model on rows 1602); 270 000, 300 trees over 50 72.7 -> 66.6.
 FUSED_COLUMN_SHAPES = [(208, 4), (160, 4), (64, 8), (80, 8)]
 FUSED_MAX_STEPS = 4
 FUSED_EXTRA_SETS = 1
@@ -428,9 +428,10 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 e("  s_add_u32 s30, s30, s4")
                 e("  s_addc_u32 s31, s31, s5")
                 for j in range(4):
-                    # a line is read once, by this load: nontemporal, so that the leaf tables stay in the L2s (150 features, 1M
-                    # documents 338.7 -> 326.8 us; 200 features, 4M 1468 -> 1369; the rows' loads, which meet in lines, took
-                    # 2584 us with it instead of 1593)
+                    # a line is read by this load and at most one neighbour's: nontemporal, so that the leaf tables stay in the
+                    # L2s (150 features, 1M documents 327.6 -> 315.8 us; 200 features, 4M 1526 -> 1418; 300 000 documents of 100
+                    # features, one batch again and again 67.5 -> 64.6; the rows' loads, which meet in lines, took 2584 us with it
+                    # instead of 1593)
                     e("  global_load_dword v%d, v%d, s[30:31] nt" % (value_set[turn][2 * j + c // 4] + c % 4, row_off[j]))
                     pending.append(("turn", turn))
             if turn[0] > 0:

@@ -2695,8 +2695,8 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             }
             const TFusedVariant* fused = nullptr;
             for (const auto& v : kFusedVariants) {
-                // (of the rows' shapes the wide one is for the models of the wide evaluate kernels; columns over 85 to 90
-                // buckets: 1M documents, 200 trees 160 us on two launches, 134 on the shape of 160, 1000 trees 316 and 309)
+                // (of the rows' shapes the wide one is for the models of the wide evaluate kernels; columns over 88
+                // buckets: 1M documents, 200 trees 164 us on two launches, 126 on the shape of 160, 1000 trees 329 and 301)
                 if (v.Columns == columnMajor && v.Six == variant->Six && unitStart.size() * kFusedUnitColumns <= v.Buckets && !fused &&
                     (variant->Waves == 4 || v.Buckets <= 80 || columnMajor) && m.MaxDepth <= v.Levels) {
                     fused = &v;
@@ -3007,11 +3007,11 @@ void LaunchBinarizeRowsPC(size_t blocks, const float* floats, size_t stride, con
                           size_t docCount, const dev::TBinarizeTables& tab, uint32_t* bins, hipStream_t s, hipEvent_t end) {
     const size_t tiles = (tab.BucketCount + dev::kBucketTile - 1) / dev::kBucketTile;
     // A workgroup keeps its tile's borders in LDS over up to kBinarizeBlocksPerGroup document blocks; a smaller batch gives
-    // each fewer blocks, so that there are still a few generations of workgroups, whose phases overlap: 200 000 documents of
-    // 100 features, 1000 trees 111.8 us with about 1024 workgroups, 109.5 with 4096; leaf indexes of 200 000 documents 218.0
-    // and 214.9; 30 000 to 100 000 documents the same. Tables of 256 slots (20 KB) cost a workgroup more than that gives:
-    // a CTR model of 1M documents 364 us with 1024 and 373 with 4096. (Column-major batches, which have no tile to fill: 100 000 documents
-    // 69.6 and 71.7, so those keep 1024.)
+    // each fewer blocks, so that there are still a few generations of workgroups, whose phases overlap: whole call with about
+    // 1024 workgroups and with 4096, 100 000 documents of 250 features, 300 trees 71.9 and 67.3 us, 200 000 119.0 and 111.9,
+    // 200 000 of 100 features, four dimensions 94.2 and 91.3, 50 000 of 600 features 91.3 and 87.3; 100 000 of 50 to 200 features
+    // the same within 1 %. Tables of 256 slots (20 KB) cost a workgroup more than that gives: a CTR model of 1M documents 364 us with 1024
+    // and 373 with 4096. (Column-major batches, which have no tile to fill: 100 000 documents 69.6 and 71.7, so those keep 1024.)
     const uint32_t blocksPerGroup = static_cast<uint32_t>(
         std::max<size_t>(1, std::min<size_t>(kBinarizeBlocksPerGroup, blocks * tiles / (LOG2P < 8 ? 4096 : 1024))));
     const size_t groups = (blocks + blocksPerGroup - 1) / blocksPerGroup;

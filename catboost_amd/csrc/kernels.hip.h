@@ -464,7 +464,8 @@ __device__ __forceinline__ uint64_t CtrHashOfCat(uint32_t v) {
 // features. What bounds it is the gathers of table entries (a line of L2 each for tables beyond the L1): one 16-byte
 // read finds and answers a lookup of up to eight buckets, where a table per CTR feature, its rows and a division and a
 // count of borders per feature took five times as long (1M documents, 16 categorical columns, 24 projections with 96 CTR
-// features: 620 us then, 107 with tables up to half full, 83 now).
+// features: 620 us then; 87 to 97 now, three batches in turn; with tables half full instead of a quarter the call takes 252
+// us instead of 215).
 // grid = (document blocks, shares of the groups), 4 waves per workgroup, each wave a run of the share's groups.
 // TILE: the block's hashed categorical values are staged once per workgroup into LDS ([column][document]); without
 // it (more than kCtrMaxTileColumns columns) they are read from the batch where a projection needs them.
