@@ -3812,7 +3812,7 @@ static void AwaitSmallBatch(THipEvaluator::TImpl& m, const THipEvaluator::TImpl:
     const auto started = std::chrono::steady_clock::now();
     size_t group = 0;
     for (uint32_t turn = 0; group < slot.SmallGroups; ++turn) {
-        if (__atomic_load_n(flags + group, __ATOMIC_ACQUIRE) == slot.SmallTicket) {
+        if (m.FlagWaitUs != 0 && __atomic_load_n(flags + group, __ATOMIC_ACQUIRE) == slot.SmallTicket) {
             ++group;
         } else if ((turn % 256 == 255 || m.FlagWaitUs == 0) && std::chrono::steady_clock::now() - started >= std::chrono::microseconds(m.FlagWaitUs)) {
             HIP_CHECK(hipEventSynchronize(stop));

@@ -102,7 +102,7 @@ typedef struct CbHipFeatures {
  *   CATBOOST_AMD_FLAG_TICKET=n       calls of few host documents, which return when their workgroups have set flags in
  *                                    host memory: the flags' first ticket is n + 1, and CbHipDescribeKernels for a small
  *                                    batch ends with ";flagged=<calls that their flags have ended>"
- *   CATBOOST_AMD_FLAG_WAIT_US=n      such a call waits for its launch after n microseconds instead of 200 */
+ *   CATBOOST_AMD_FLAG_WAIT_US=n      such a call waits for its launch after n microseconds instead of 200 (0: at once) */
 
 /* Model upload: validates the tables, derives buckets / repacked splits / leaf offsets and
  * copies SoA tables to device `deviceId` (takes the place of the TGpuEvaluator constructor,
