@@ -1,0 +1,443 @@
+#include "exchange_plan.h"
+
+#include <algorithm>
+#include <cstring>
+#include <utility>
+
+namespace cbamd {
+
+namespace {
+
+// A level of the model as an edge of the multigraph trees x groups
+struct TEdge {
+    uint32_t Tree = 0, Group = 0;
+    const TExchangeLevel* Level = nullptr;
+    uint32_t ModelLevel = 0;  // which level of its tree
+    bool High = false;        // one of the places behind the first five
+    int Place = -1;           // place in its group, later the order of the compares
+};
+
+struct TGroup {
+    std::vector<uint32_t> Edges;
+    uint32_t FirstRound = ~0u, LastRound = 0;  // rounds whose trees look at it
+    uint32_t Slot = 0;
+};
+
+// Gives the places behind the first kEvenPlaces to the levels that split the documents unevenly: the five low bits of a leaf index
+// choose the pair of LDS banks of a gather, lanes with the same index share an access, and lopsided levels in the high bits
+// leave fewer different leaves per bank (borders drawn evenly, 16 lanes a cycle: 12.0 cycles per gather of 64 lanes in the model's order,
+// 8.5 so). A tree and a group have at most as many edges on either side as there are places; trees start within that,
+// groups are brought there by swapping pairs of a tree's levels, the cheapest first.
+constexpr uint32_t kEvenPlaces = 5;
+
+class TSides {
+public:
+    TSides(std::vector<TEdge>* edges, const std::vector<std::vector<uint32_t>>& ofTree, const std::vector<TGroup>& groups,
+           uint32_t places)
+        : Edges(*edges), OfTree(ofTree), Groups(groups), Places{kEvenPlaces, places - kEvenPlaces}, TreeCount{std::vector<uint32_t>(ofTree.size(), 0), std::vector<uint32_t>(ofTree.size(), 0)}
+        , GroupCount{std::vector<uint32_t>(groups.size(), 0), std::vector<uint32_t>(groups.size(), 0)} {
+    }
+
+    bool Assign() {
+        for (size_t t = 0; t < OfTree.size(); ++t) {
+            std::vector<uint32_t> order(OfTree[t]);
+            std::stable_sort(order.begin(), order.end(),
+                             [&](uint32_t a, uint32_t b) { return Edges[a].Level->Lopsided < Edges[b].Level->Lopsided; });
+            for (size_t i = 0; i < order.size(); ++i) {
+                Edges[order[i]].High = i >= kEvenPlaces;
+                Count(order[i], 1);
+            }
+        }
+        for (uint32_t g = 0; g < Groups.size(); ++g) {
+            for (int side = 0; side < 2; ++side) {
+                while (GroupCount[side][g] > Places[side]) {
+                    if (!Relieve(g, side != 0)) {
+                        return false;
+                    }
+                }
+            }
+        }
+        return true;
+    }
+
+private:
+    void Count(uint32_t e, int by) {
+        TreeCount[Edges[e].High][Edges[e].Tree] += by;
+        GroupCount[Edges[e].High][Edges[e].Group] += by;
+    }
+    void Flip(uint32_t e) {
+        Count(e, -1);
+        Edges[e].High = !Edges[e].High;
+        Count(e, 1);
+    }
+    double Cost(uint32_t e) const {  // of moving the edge to the other side
+        return Edges[e].High ? -Edges[e].Level->Lopsided : Edges[e].Level->Lopsided;
+    }
+
+    // One edge of `side` less in group g: along a shortest chain of swaps (an edge of the group leaves `side`, another
+    // edge of its tree takes its place there, and so on) that ends at a tree or a group with room.
+    bool Relieve(uint32_t g, bool side) {
+        Steps.clear();
+        At.assign(1, g);
+        Via.assign(1, -1);
+        Seen.assign(1, g);
+        while (!At.empty()) {
+            double bestCost = 0.0;
+            int best = -1;
+            Next.clear();
+            NextVia.clear();
+            for (size_t i = 0; i < At.size(); ++i) {
+                for (uint32_t out : Groups[At[i]].Edges) {
+                    if (Edges[out].High != side) {
+                        continue;
+                    }
+                    const uint32_t t = Edges[out].Tree;
+                    if (TreeCount[!side][t] < Places[!side]) {
+                        Steps.push_back({out, ~0u, Via[i]});
+                        if (best < 0 || Cost(out) < bestCost) {
+                            best = static_cast<int>(Steps.size()) - 1;
+                            bestCost = Cost(out);
+                        }
+                        continue;
+                    }
+                    for (uint32_t in : OfTree[t]) {
+                        const uint32_t to = Edges[in].Group;
+                        if (Edges[in].High == side || to == At[i]) {
+                            continue;
+                        }
+                        if (GroupCount[side][to] < Places[side]) {
+                            const double cost = Cost(out) + Cost(in);
+                            Steps.push_back({out, in, Via[i]});
+                            if (best < 0 || cost < bestCost) {
+                                best = static_cast<int>(Steps.size()) - 1;
+                                bestCost = cost;
+                            }
+                        } else if (std::find(Seen.begin(), Seen.end(), to) == Seen.end()) {
+                            Seen.push_back(to);
+                            Steps.push_back({out, in, Via[i]});
+                            Next.push_back(to);
+                            NextVia.push_back(static_cast<int>(Steps.size()) - 1);
+                        }
+                    }
+                }
+            }
+            if (best >= 0) {
+                for (int s = best; s >= 0; s = Steps[s].Parent) {
+                    Flip(Steps[s].Out);
+                    if (Steps[s].In != ~0u) {
+                        Flip(Steps[s].In);
+                    }
+                }
+                return true;
+            }
+            At.swap(Next);
+            Via.swap(NextVia);
+        }
+        return false;
+    }
+
+    struct TStep {
+        uint32_t Out, In;  // edges that leave and enter the side
+        int Parent;        // step before
+    };
+    std::vector<TStep> Steps;              // of Relieve
+    std::vector<uint32_t> At, Next, Seen;  // groups of the frontier, of the next one, and all that were on one
+    std::vector<int> Via, NextVia;         // steps that led there
+    std::vector<TEdge>& Edges;
+    const std::vector<std::vector<uint32_t>>& OfTree;
+    const std::vector<TGroup>& Groups;
+    const uint32_t Places[2];
+    std::vector<uint32_t> TreeCount[2], GroupCount[2];
+};
+
+// Places base .. base + colours - 1 for the edges of one side: each edge takes a place that is free at its tree and at its group, after
+// swapping two places along the alternating path that starts at the group when there is no such place.
+void Colour(std::vector<TEdge>* edges, size_t treeCount, size_t groupCount, bool high, uint32_t colours, uint32_t base) {
+    std::vector<int> tree(treeCount * colours, -1), group(groupCount * colours, -1);
+    const auto slot = [&](bool isTree, uint32_t vertex, uint32_t colour) -> int& {
+        return (isTree ? tree : group)[vertex * colours + colour];
+    };
+    for (size_t i = 0; i < edges->size(); ++i) {
+        TEdge& e = (*edges)[i];
+        if (e.High != high) {
+            continue;
+        }
+        int atTree = -1, atGroup = -1, both = -1;
+        for (uint32_t c = 0; c < colours; ++c) {
+            const bool freeTree = slot(true, e.Tree, c) < 0, freeGroup = slot(false, e.Group, c) < 0;
+            if (freeTree && atTree < 0) {
+                atTree = static_cast<int>(c);
+            }
+            if (freeGroup && atGroup < 0) {
+                atGroup = static_cast<int>(c);
+            }
+            if (freeTree && freeGroup && both < 0) {
+                both = static_cast<int>(c);
+            }
+        }
+        if (both < 0) {
+            // the path from the group along the colours atTree, atGroup, atTree ... never comes to the edge's tree
+            std::vector<uint32_t> path;
+            bool isTree = false;
+            uint32_t vertex = e.Group;
+            int colour = atTree;
+            for (int next = slot(isTree, vertex, colour); next >= 0; next = slot(isTree, vertex, colour)) {
+                path.push_back(static_cast<uint32_t>(next));
+                isTree = !isTree;
+                vertex = isTree ? (*edges)[next].Tree : (*edges)[next].Group;
+                colour = colour == atTree ? atGroup : atTree;
+            }
+            for (uint32_t p : path) {
+                const TEdge& on = (*edges)[p];
+                slot(true, on.Tree, on.Place - base) = -1;
+                slot(false, on.Group, on.Place - base) = -1;
+            }
+            for (uint32_t p : path) {
+                TEdge& on = (*edges)[p];
+                on.Place = static_cast<int>(base) + (on.Place - static_cast<int>(base) == atTree ? atGroup : atTree);
+                slot(true, on.Tree, on.Place - base) = static_cast<int>(p);
+                slot(false, on.Group, on.Place - base) = static_cast<int>(p);
+            }
+            both = atTree;
+        }
+        e.Place = static_cast<int>(base) + both;
+        slot(true, e.Tree, both) = static_cast<int>(i);
+        slot(false, e.Group, both) = static_cast<int>(i);
+    }
+}
+
+}  // namespace
+
+bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketCount, uint32_t maxDepth, bool six,
+                       TExchangePlan* plan) {
+    const size_t treeCount = trees.size();
+    // ---- buckets to waves: the busiest first, each to the wave that compares the least
+    std::vector<uint32_t> levelsOf(bucketCount, 0);
+    for (const TExchangeTree& t : trees) {
+        for (const TExchangeLevel& l : t.Levels) {
+            if (l.Bucket >= bucketCount) {
+                return false;  // a damaged model
+            }
+            ++levelsOf[l.Bucket];
+        }
+    }
+    std::vector<uint32_t> byLevels;
+    for (uint32_t b = 0; b < bucketCount; ++b) {
+        if (levelsOf[b] > 0) {
+            byLevels.push_back(b);
+        }
+    }
+    if (treeCount == 0 || byLevels.size() > size_t(kExchangeWaves) * kExchangeWaveBuckets) {
+        return false;
+    }
+    std::stable_sort(byLevels.begin(), byLevels.end(), [&](uint32_t a, uint32_t b) { return levelsOf[a] > levelsOf[b]; });
+    std::vector<uint32_t> waveOf(bucketCount, 0), registerOf(bucketCount, 0);
+    std::vector<uint32_t> taken(kExchangeWaves, 0);
+    std::vector<size_t> load(kExchangeWaves, 0);
+    plan->WaveTable.assign(size_t(kExchangeWaves) * kExchangeWaveDwords, 0);
+    for (uint32_t b : byLevels) {
+        uint32_t best = kExchangeWaves;
+        for (uint32_t w = 0; w < kExchangeWaves; ++w) {
+            if (taken[w] < kExchangeWaveBuckets && (best == kExchangeWaves || load[w] < load[best])) {
+                best = w;
+            }
+        }
+        waveOf[b] = best;
+        registerOf[b] = taken[best]++;
+        load[best] += levelsOf[b];
+        plan->WaveTable[best * kExchangeWaveDwords + registerOf[b]] = b * 256u;
+    }
+
+    // ---- trees to the waves that sum them, and to steps
+    std::vector<std::vector<uint32_t>> treesOf(kExchangeWaves);
+    for (size_t t = 0; t < treeCount / 2 * 2; ++t) {
+        treesOf[t / 2 % kExchangeWaves].push_back(static_cast<uint32_t>(t));
+    }
+    if (treeCount % 2 != 0) {
+        treesOf[0].push_back(static_cast<uint32_t>(treeCount - 1));
+    }
+    size_t longest = 0;
+    std::vector<uint32_t> stepOf(treeCount, 0), sumWaveOf(treeCount, 0);
+    for (uint32_t w = 0; w < kExchangeWaves; ++w) {
+        longest = std::max(longest, treesOf[w].size());
+        for (size_t i = 0; i < treesOf[w].size(); ++i) {
+            stepOf[treesOf[w][i]] = static_cast<uint32_t>(i);
+            sumWaveOf[treesOf[w][i]] = w;
+        }
+    }
+    plan->Rounds = static_cast<uint32_t>((longest + kExchangeRoundSteps - 1) / kExchangeRoundSteps);
+    const size_t steps = size_t(plan->Rounds) * kExchangeRoundSteps;
+
+    // ---- levels to groups: a wave's levels in the order of their trees' steps
+    std::vector<uint32_t> byStep(treeCount);
+    for (size_t t = 0; t < treeCount; ++t) {
+        byStep[t] = static_cast<uint32_t>(t);
+    }
+    std::stable_sort(byStep.begin(), byStep.end(), [&](uint32_t a, uint32_t b) { return stepOf[a] < stepOf[b]; });
+    std::vector<TEdge> edges;
+    std::vector<TGroup> groups;
+    std::vector<std::vector<uint32_t>> edgesOfTree(treeCount), groupsOf(kExchangeWaves);
+    for (uint32_t t : byStep) {
+        edgesOfTree[t].reserve(trees[t].Levels.size());
+        for (uint32_t d = 0; d < trees[t].Levels.size(); ++d) {
+            const TExchangeLevel& level = trees[t].Levels[d];
+            const uint32_t w = waveOf[level.Bucket];
+            if (groupsOf[w].empty() || groups[groupsOf[w].back()].Edges.size() == maxDepth) {
+                groupsOf[w].push_back(static_cast<uint32_t>(groups.size()));
+                groups.emplace_back();
+                groups.back().Edges.reserve(maxDepth);
+            }
+            TEdge edge;
+            edge.Tree = t;
+            edge.Group = groupsOf[w].back();
+            edge.Level = &level;
+            edge.ModelLevel = d;
+            TGroup& group = groups[edge.Group];
+            const uint32_t round = stepOf[t] / kExchangeRoundSteps;
+            group.FirstRound = std::min(group.FirstRound, round);
+            group.LastRound = std::max(group.LastRound, round);
+            group.Edges.push_back(static_cast<uint32_t>(edges.size()));
+            edgesOfTree[t].push_back(static_cast<uint32_t>(edges.size()));
+            edges.push_back(edge);
+        }
+    }
+
+    // ---- places in the groups
+    if (!TSides(&edges, edgesOfTree, groups, maxDepth).Assign()) {
+        return false;
+    }
+    Colour(&edges, treeCount, groups.size(), false, kEvenPlaces, 0);
+    Colour(&edges, treeCount, groups.size(), true, maxDepth - kEvenPlaces, kEvenPlaces);
+
+    // ---- when a group is compared, and in which slot it stands. A wave compares a group at the end of a step. The barrier of
+    // round r stands at the beginning of its last step; behind it come the reads for the next round's first tree. So
+    // the last step of round p - 1 and the first three of round p make up *phase* p: a group for the trees of round r
+    // is compared in phase r - 1 or before (phase -1: before the first step), and its slot is free again from phase r + 1 on, r
+    // the last round that looks at it. As far as slots go a wave compares a group in every step and so stays ahead of the need.
+    std::vector<std::vector<uint32_t>> groupsAt(steps * kExchangeWaves), early(kExchangeWaves);
+    std::vector<uint32_t> freeSlots;
+    for (uint32_t s = kExchangeSlots; s-- > 0;) {
+        freeSlots.push_back(s);
+    }
+    std::vector<std::vector<uint32_t>> freedAfter(plan->Rounds);
+    std::vector<size_t> next(kExchangeWaves, 0);
+    const int64_t rounds = plan->Rounds;
+    for (int64_t phase = -1; phase < rounds; ++phase) {
+        std::vector<std::vector<uint32_t>> now(kExchangeWaves);
+        const auto nextRound = [&](uint32_t w) {  // first round that needs the wave's next group
+            return next[w] < groupsOf[w].size() ? static_cast<int64_t>(groups[groupsOf[w][next[w]]].FirstRound) : rounds + 2;
+        };
+        const auto place = [&](uint32_t w) {
+            TGroup& group = groups[groupsOf[w][next[w]]];
+            group.Slot = freeSlots.back();
+            freeSlots.pop_back();
+            freedAfter[group.LastRound].push_back(group.Slot);
+            now[w].push_back(groupsOf[w][next[w]++]);
+        };
+        for (uint32_t w = 0; w < kExchangeWaves; ++w) {
+            while (nextRound(w) <= phase + 1) {
+                if (freeSlots.empty()) {
+                    return false;
+                }
+                place(w);
+            }
+        }
+        const int64_t firstStep = std::max<int64_t>(phase * kExchangeRoundSteps - 1, 0);
+        const uint32_t stepCount = phase < 0 ? 0 : static_cast<uint32_t>(phase * kExchangeRoundSteps + kExchangeRoundSteps - 1 - firstStep);
+        // ahead of the need, not the slots that the next phases' groups may want
+        for (uint32_t turn = 0; turn < kExchangeRoundSteps; ++turn) {
+            for (uint32_t w = 0; w < kExchangeWaves; ++w) {
+                if ((phase < 0 ? turn == 0 : now[w].size() < stepCount) && nextRound(w) <= phase + 2 && freeSlots.size() > 4 * kExchangeWaves) {
+                    place(w);
+                }
+            }
+        }
+        for (uint32_t w = 0; w < kExchangeWaves; ++w) {
+            for (size_t i = 0; i < now[w].size(); ++i) {
+                (phase < 0 ? early[w] : groupsAt[(firstStep + i % stepCount) * kExchangeWaves + w]).push_back(now[w][i]);
+            }
+        }
+        if (phase >= 0) {
+            freeSlots.insert(freeSlots.end(), freedAfter[phase].begin(), freedAfter[phase].end());
+        }
+    }
+
+    // ---- tables
+    const auto writeGroup = [&](uint32_t g, uint32_t* row) {
+        std::fill(row, row + kExchangeGroupDwords, 0u);
+        row[0] = groups[g].Slot * 256u << 16;
+        for (uint32_t e : groups[g].Edges) {
+            const TEdge& edge = edges[e];
+            uint32_t xorByte = edge.Level->Xor, addByte = edge.Level->Add;
+            if (six && edge.Place % 2 == 0) {
+                // the result goes to bit 6
+                if (edge.Level->IsXor) {
+                    xorByte &= 0x3fu;
+                } else {
+                    addByte -= 64;
+                }
+            }
+            row[2 * edge.Place] |= registerOf[edge.Level->Bucket] | xorByte << 8;
+            row[2 * edge.Place + 1] = (addByte & 0xffu) * 0x01010101u;
+            row[2] |= edge.Level->IsXor ? kExchangeXorFlag : 0u;
+        }
+    };
+    const auto recordOf = [&](size_t step, uint32_t w) {
+        return plan->Records.data() + (step / kExchangeRoundSteps * kExchangeWaves + w) * kExchangeRecordDwords;
+    };
+    plan->Records.assign((size_t(plan->Rounds) + 1) * kExchangeWaves * kExchangeRecordDwords, 0);
+    plan->ExtraRows.clear();
+    for (uint32_t w = 0; w < kExchangeWaves; ++w) {
+        uint32_t* wave = plan->WaveTable.data() + w * kExchangeWaveDwords;
+        wave[kExchangeWaveBuckets] = static_cast<uint32_t>(plan->ExtraRows.size() * sizeof(uint32_t));
+        wave[kExchangeWaveBuckets + 1] = static_cast<uint32_t>(early[w].size());
+        const auto addExtra = [&](uint32_t g) {
+            plan->ExtraRows.resize(plan->ExtraRows.size() + kExchangeGroupDwords);
+            uint32_t* row = plan->ExtraRows.data() + plan->ExtraRows.size() - kExchangeGroupDwords;
+            writeGroup(g, row);
+            return row;
+        };
+        for (uint32_t g : early[w]) {
+            addExtra(g);
+        }
+        for (size_t step = 0; step < steps; ++step) {
+            const std::vector<uint32_t>& at = groupsAt[step * kExchangeWaves + w];
+            uint32_t* row = recordOf(step, w) + step % kExchangeRoundSteps * kExchangeGroupDwords;
+            if (at.empty()) {
+                row[2] = kExchangeSkipFlag;
+                continue;
+            }
+            writeGroup(at[0], row);
+            row[2] |= at.size() > 1 ? kExchangeMoreFlag : 0u;
+            for (size_t i = 1; i < at.size(); ++i) {
+                addExtra(at[i])[2] |= i + 1 < at.size() ? kExchangeMoreFlag : 0u;
+            }
+        }
+    }
+    plan->ExtraRows.resize(plan->ExtraRows.size() + kExchangeEarlyRows * kExchangeGroupDwords, 0);
+    const size_t leafCount = size_t(1) << maxDepth;
+    plan->Leaves.assign((size_t(plan->Rounds) + 1) * kExchangeWaves * kExchangeRoundSteps * leafCount, 0.0);
+    for (size_t t = 0; t < treeCount; ++t) {
+        const size_t step = stepOf[t], inRound = step % kExchangeRoundSteps;
+        const uint32_t w = sumWaveOf[t];
+        uint32_t* row = recordOf(step, w) + kExchangeRoundSteps * kExchangeGroupDwords + inRound * kExchangeTreeDwords;
+        double* values = plan->Leaves.data() + ((step / kExchangeRoundSteps * kExchangeWaves + w) * kExchangeRoundSteps + inRound) * leafCount;
+        for (uint32_t e : edgesOfTree[t]) {
+            row[edges[e].Place] = groups[edges[e].Group].Slot * 256u;
+        }
+        // a place without a level holds another group's bit: the values are the same for either
+        uint32_t low[16] = {}, high[16] = {};  // what the lower and the upper four bits of an index say of the leaf
+        for (uint32_t i = 0; i < 16; ++i) {
+            for (uint32_t e : edgesOfTree[t]) {
+                const uint32_t place = static_cast<uint32_t>(edges[e].Place);
+                (place < 4 ? low : high)[i] |= (i >> place % 4 & 1) << edges[e].ModelLevel;
+            }
+        }
+        for (size_t i = 0; i < leafCount; ++i) {
+            values[i] = trees[t].Leaves[low[i & 15] | high[i >> 4]];
+        }
+    }
+    return true;
+}
+
+}  // namespace cbamd

@@ -1,0 +1,62 @@
+// Host tables of the exchange kernels (gen_eval_exchange_kernel.py): one-dimensional oblivious models of depth <= 8 whose
+// bins of 256 documents fit the registers of a workgroup's sixteen waves (64 buckets each).
+//
+// Every wave compares the levels that look at its own buckets and packs their results, one bit per document, into dwords:
+// a *group* is MaxDepth levels (8 or 6), whose bits stand in different positions of a byte per document. The dwords meet in
+// LDS slots; the wave that sums a tree picks the tree's bits out of the dwords of its levels' groups, the bit at position p
+// from the dword that the tree's row names for p. Two levels must therefore stand in different positions if they belong to one tree or to
+// one group: a proper edge colouring of the multigraph trees x groups (an edge is a level), whose degrees are at most
+// MaxDepth, and such a graph has one with MaxDepth colours (Koenig).
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+namespace cbamd {
+
+constexpr uint32_t kExchangeWaves = 16;          // waves per workgroup, one workgroup per CU
+constexpr uint32_t kExchangeWaveBuckets = 64;    // bins registers per wave
+constexpr uint32_t kExchangeRoundSteps = 4;      // trees that a wave sums between two barriers
+constexpr uint32_t kExchangeSlots = 224;         // LDS slots of 256 bytes for the groups' dwords
+constexpr uint32_t kExchangeGroupDwords = 16;    // a group's row: per place (register | xor byte << 8, added bytes); the first dword
+                                                 // also slot * 256 << 16, the third one the flags
+constexpr uint32_t kExchangeXorFlag = 0x80000000u;   // a level of the group xors
+constexpr uint32_t kExchangeMoreFlag = 0x40000000u;  // another group in this step, from the wave's row of extra ones
+constexpr uint32_t kExchangeSkipFlag = 0x20000000u;  // no group in this step
+constexpr uint32_t kExchangeEarlyRows = 3;       // rows of the groups before the first step that are fetched together
+constexpr uint32_t kExchangeTreeDwords = 8;      // a tree's row: per place the byte offset of the slot that holds its level's group
+// per round and wave: four group rows, four tree rows
+constexpr uint32_t kExchangeRecordDwords = kExchangeRoundSteps * (kExchangeGroupDwords + kExchangeTreeDwords);
+constexpr uint32_t kExchangeWaveDwords = 80;     // per wave: 64 bucket offsets in bytes, offset of its first extra group row in
+                                                 // bytes, how many of those come before the first step
+
+struct TExchangeLevel {
+    uint32_t Bucket = 0;
+    uint32_t Add = 0;       // byte added to the (xored) bin: the level's result is the carry into bit 7
+    uint32_t Xor = 0;       // seven bits
+    bool IsXor = false;
+    double Lopsided = 0.0;  // 0: splits the documents evenly
+};
+
+struct TExchangeTree {
+    std::vector<TExchangeLevel> Levels;
+    const double* Leaves = nullptr;  // 1 << Levels.size() values
+};
+
+struct TExchangePlan {
+    uint32_t Rounds = 0;
+    std::vector<uint32_t> WaveTable;  // [wave][kExchangeWaveDwords]
+    std::vector<uint32_t> Records;    // [round + 1][wave][kExchangeRecordDwords]: rows are fetched ahead
+    std::vector<uint32_t> ExtraRows;  // [wave][its extra groups][kExchangeGroupDwords], and kExchangeEarlyRows spare ones
+    std::vector<double> Leaves;       // [round + 1][wave][step][1 << maxDepth]
+};
+
+// maxDepth: 6 or 8, at least the deepest tree's. six: all bins are at most 63, and the levels of even places in a group
+// have their results in bit 6. Tree t of pair p = t / 2 is summed by wave p % 16, the last tree of an odd number by wave 0
+// behind its others: the sums and their order are the pair-tile kernel's. Returns false if the model does not fit (too many
+// buckets, or groups that no slot is left for).
+bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketCount, uint32_t maxDepth, bool six,
+                       TExchangePlan* plan);
+
+}  // namespace cbamd

@@ -82,7 +82,11 @@ and argument 0 is the delay of workgroups 256 .. 511 in turns of 4096 cycles (ro
 
 Usage: gen_eval_reg_kernel.py OUT.s
 """
+import os
 import sys
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import gen_eval_exchange_kernel  # noqa: E402
 
 
 LDS_BUFFER_LIMIT = 32 * 1024
@@ -1145,6 +1149,10 @@ def generate():
                     text, meta = gen_kernel(buckets, waves, 1, 256, False, six, fused=True, levels=levels, columns=columns)
                     parts.append(text)
                     metas.append(meta)
+    for depth, six in gen_eval_exchange_kernel.SHAPES:
+        text, meta = gen_eval_exchange_kernel.gen_kernel(depth, six)
+        parts.append(text)
+        metas.append(meta)
     parts.append(".amdgpu_metadata")
     parts.append("---")
     parts.append("amdhsa.kernels:")

@@ -1,5 +1,6 @@
 // Host side of the HIP evaluator: model upload, kernel launches, host staging.
 #include "hip_evaluator.h"
+#include "exchange_plan.h"
 #include "fast_exp.h"
 #include "kernels.hip.h"
 
@@ -227,6 +228,23 @@ static_assert(sizeof(TEvalRegLaunchArgs) == 96, "kernel argument block of the re
 constexpr uint32_t kRegFlagMapped = 8;
 // what a mapped bins register holds of its bucket's bins (bits 16.. of a map entry)
 constexpr uint32_t kRegMapAsIs = 0, kRegMapLow = 1, kRegMapHigh = 2;  // bin, min(bin, 127), max(bin - 127, 0)
+
+// argument block of the exchange kernels (gen_eval_exchange_kernel.py)
+struct TEvalExchangeArgs {
+    const void* Bins;
+    const void* WaveTable;
+    const void* Records;
+    const void* ExtraRows;
+    const void* Leaves;
+    double* Out;
+    const double* Bias;
+    double Scale;
+    uint32_t DocCount;
+    uint32_t Rounds;
+    uint32_t BlockBytes;
+    uint32_t Unused;
+};
+static_assert(sizeof(TEvalExchangeArgs) == 80, "kernel argument block of the exchange kernels");
 
 struct TEvalRegVariant {
     uint32_t Buckets;
@@ -490,6 +508,7 @@ struct TKernelSwitches {
     bool SmallBatch = true;       // CATBOOST_AMD_SMALL_BATCH=0: small batches are not spread over slices of the trees
     bool LevelOrder = true;       // CATBOOST_AMD_LEVEL_ORDER=0: register kernels keep the model's order of a tree's levels
     bool PairTile = true;         // CATBOOST_AMD_PAIR_TILE=0: the half-tile kernel with one tree per wave
+    bool Exchange = true;         // CATBOOST_AMD_EXCHANGE=0: the pair-tile kernel for batches of every size
     bool RowTile = true;          // CATBOOST_AMD_ROW_TILE=0: the tile kernel that broadcasts a tree's levels from a lane
     bool RegSplit = true;         // CATBOOST_AMD_REG_SPLIT=0: a bucket keeps to one register: more than 127 values send a model to the mixed kernels
     uint32_t NsWaves = 0;         // CATBOOST_AMD_NS_WAVES=4|6|8|10|11|12|16: shapes of the non-symmetric LDS kernel with so many waves or none
@@ -514,6 +533,7 @@ struct TKernelSwitches {
         k.LevelOrder = !off("CATBOOST_AMD_LEVEL_ORDER");
         k.SmallBatch = !off("CATBOOST_AMD_SMALL_BATCH");
         k.PairTile = !off("CATBOOST_AMD_PAIR_TILE");
+        k.Exchange = !off("CATBOOST_AMD_EXCHANGE");
         k.RowTile = !off("CATBOOST_AMD_ROW_TILE");
         k.RegSplit = !off("CATBOOST_AMD_REG_SPLIT");
         if (const char* v = std::getenv("CATBOOST_AMD_NS_WAVES")) {
@@ -1550,6 +1570,12 @@ struct THipEvaluator::TImpl {
     TDeviceVec<double> HalfTileLeaves; // half-tile kernel: 64 or 256 leaf values per tree at a fixed pitch
     TDeviceVec<uint32_t> PairRows;     // pair-tile kernel: 32 dwords per tree, empty when the model does not qualify
     bool PairSix = false;              // ... in the six-bit form (every bin below 64)
+    TDeviceVec<uint32_t> ExchangeWaves, ExchangeRecords, ExchangeExtra;  // exchange kernel (exchange_plan.h)
+    TDeviceVec<double> ExchangeLeaves;
+    uint32_t ExchangeRounds = 0;
+    bool PairBeforeTile = false;       // the tile kernel would hold the model's bins, but the pair-tile kernel takes it
+    hipFunction_t ExchangeFunction = nullptr;  // nullptr: the model does not qualify
+    const char* ExchangeName = "";
     TDeviceVec<uint32_t> QuadRows;     // quad-tile kernel: 16 dwords per tree, 64 bytes per row of the tile
     TDeviceVec<uint32_t> TileRows;     // row-tile kernel (whole tile, one tree per wave): the same with 256 bytes per bucket
     TDeviceVec<double> TileLeaves;     // its leaf values: [slice of the dimensions][tree][pair of dimensions][leaf][2]
@@ -1677,6 +1703,26 @@ struct THipEvaluator::TImpl {
         }
     };
     TSumOrder SumOrder() const;
+
+    // The exchange kernel instead of the pair-tile kernel, whose sums it gives: a workgroup per block of 256 documents where the other
+    // has one per half block, one per CU in both. A generation of its workgroups lasts as long as 1.2 to 1.45 generations of the
+    // other's (trees of depth 7 and 8) or 1.6 to 1.8 (up to 6), measured with 500 to 5000 trees; the batch decides how many of
+    // each there are. 5000 trees of depth 8 over 1016 features, evaluate launch, pair-tile -> exchange: 33 000 documents
+    // 240 -> 170 us, 66 000 363 -> 334, 130 000 493 -> 351, 1M 3633 -> 2659; 2000 of depth 5 over 700: 50 000 documents 61 -> 52 us,
+    // 130 000 124 -> 113, 1M 887 -> 810, but 66 000 88 -> 96 and 140 000 147 -> 155, which stay where they were.
+    bool TakesExchangeKernel(size_t docCount) const {
+        if (ExchangeFunction == nullptr || docCount >= (size_t(1) << 32)) {
+            return false;
+        }
+        const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
+        const size_t generations = (blocks + CuCount - 1) / CuCount, others = (2 * blocks + CuCount - 1) / CuCount;
+        return generations * (MaxDepth <= 6 ? 36 : 29) < others * 20;
+    }
+
+    // The tile kernel takes the model (of kernels on bins in an LDS tile of whole blocks, the one without a tree's row in registers).
+    bool TileFits() const {
+        return !PairBeforeTile && TileLdsBytes(LayoutBuckets, TileChunk(Dim)) <= kMaxTileLdsBytes;
+    }
 
     int SmallDims() const { return Dim == 1 ? 1 : Dim == 2 ? 2 : 4; }
     uint32_t SmallPasses() const { return static_cast<uint32_t>((Dim + SmallDims() - 1) / SmallDims()); }
@@ -2279,7 +2325,11 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 }
             }
             m.PackedMixed.Upload(mixed);
-            if (TileLdsBytes(m.LayoutBuckets, 1) > kMaxTileLdsBytes) {
+            // Some 577 to 632 buckets: the tile fits LDS, but not with the regions of the row-tile kernel. Two trees per wave on
+            // half a tile, or the exchange kernel, are the faster there.
+            m.PairBeforeTile = switches.RowTile && switches.PairTile && PairTileLdsBytes(tileRowCount, 8) <= kMaxTileLdsBytes &&
+                               RowTileWaves(tileRowCount, m.MaxDepth, 1) == 0;
+            if (!m.TileFits()) {
                 const size_t pitch = m.MaxDepth <= 6 ? 64 : 256;
                 // zeros at the end: the pair-tile and quad-tile kernels fetch ahead of their trees without a bound
                 std::vector<double> fixed((trees.GetTreeCount() + dev::kQuadTreePadding) * pitch, 0.0);
@@ -2298,6 +2348,32 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                         // every bin below 64: the walk joins two levels at a time
                         m.PairSix = m.MaxBucketValues <= 63 && !tileRowsSplit && switches.RegSix;
                         m.PairRows.Upload(pairTileRows(m.PairSix));
+                        if (switches.Exchange && !tileRowsSplit) {
+                            std::vector<TExchangeTree> levels(trees.GetTreeCount());
+                            for (size_t t = 0; t < levels.size(); ++t) {
+                                levels[t].Leaves = trees.LeafValues.data() + trees.TreeFirstLeafOffsets[t];
+                                for (int d = 0; d < trees.TreeSizes[t]; ++d) {
+                                    const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + d];
+                                    const TTileLevel level = tileLevelOf(rb);
+                                    // how evenly a level splits, estimated as for the register kernels (levelOrder below)
+                                    const uint32_t n = offsets[rb.FeatureIndex + 1] - offsets[rb.FeatureIndex];
+                                    const double share = level.IsXor ? 0.05 : static_cast<double>(rb.SplitIdx) / (n + 1.0);
+                                    levels[t].Levels.push_back({level.Row, level.Add & 0xffu, level.Xor, level.IsXor,
+                                                                switches.LevelOrder ? std::fabs(share - 0.5) : 0.0});
+                                }
+                            }
+                            TExchangePlan plan;
+                            if (BuildExchangePlan(levels, m.LayoutBuckets, static_cast<uint32_t>(maxd), m.PairSix, &plan)) {
+                                m.ExchangeRounds = plan.Rounds;
+                                m.ExchangeWaves.Upload(plan.WaveTable);
+                                m.ExchangeRecords.Upload(plan.Records);
+                                m.ExchangeExtra.Upload(plan.ExtraRows);
+                                m.ExchangeLeaves.Upload(plan.Leaves);
+                                m.ExchangeName = maxd == 6 ? (m.PairSix ? "cbamd_eval_exchange_d6_s" : "cbamd_eval_exchange_d6")
+                                                           : (m.PairSix ? "cbamd_eval_exchange_d8_s" : "cbamd_eval_exchange_d8");
+                                HIP_CHECK(hipModuleGetFunction(&m.ExchangeFunction, SharedRegModule(kEvalRegCodeObject), m.ExchangeName));
+                            }
+                        }
                     } else {
                         m.QuadRows.Upload(rowsInRegisters(64));
                     }
@@ -3341,7 +3417,7 @@ THipEvaluator::TImpl::TSumOrder THipEvaluator::TImpl::SumOrder() const {
     TSumOrder order;
     if (TileRows.Get() != nullptr) {
         order.Waves = RowTileWaves(TileRowCount, MaxDepth, Dim);
-    } else if (TileLdsBytes(LayoutBuckets, dchunk) <= kMaxTileLdsBytes) {
+    } else if (TileFits()) {
         const int levels = TileLevels(MaxDepth);
         const bool leavesInLds = TileLeavesInLds(LayoutBuckets, levels, dchunk, Dim > 1 || LeavesPairAligned);
         order.Waves = static_cast<uint32_t>(TileWaves(LayoutBuckets, levels, dchunk, leavesInLds));
@@ -3489,7 +3565,7 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
         HIP_CHECK(hipGetLastError());
         return;
     }
-    if (m.Oblivious && m.MaxDepth <= 8 && TileLdsBytes(m.LayoutBuckets, dchunk) <= kMaxTileLdsBytes) {
+    if (m.Oblivious && m.MaxDepth <= 8 && m.TileFits()) {
         // byte-parallel kernel over an LDS tile of bins
         const TTileArgs args{bins, docCount, m.LayoutBuckets, m.PackedTrees.Get(),
                              m.Dim == 1 ? m.Leaves.Get() : m.LeavesPadded.Get(), m.Bias.Get(), m.Scale, m.Dim, tb, te,
@@ -3530,6 +3606,13 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
         // the bins of a block exceed the 256-document tile: half blocks
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
         const int maxd = m.MaxDepth <= 6 ? 6 : 8;
+        if (m.TakesExchangeKernel(docCount) && tb == 0 && te == TreeCount && (reinterpret_cast<uintptr_t>(bins) & 3) == 0) {
+            TEvalExchangeArgs args = {bins, m.ExchangeWaves.Get(), m.ExchangeRecords.Get(), m.ExchangeExtra.Get(), m.ExchangeLeaves.Get(),
+                                      results, m.Bias.Get(), m.Scale, static_cast<uint32_t>(docCount), m.ExchangeRounds,
+                                      m.LayoutBuckets * dev::kDocsPerBlock, 0};
+            LaunchModuleWithEnd(m.ExchangeFunction, static_cast<uint32_t>(blocks), 1, 64 * kExchangeWaves, s, TakeEnd(end), args);
+            return;
+        }
         if (m.PairRows.Get() != nullptr) {
             const size_t lds = PairTileLdsBytes(m.TileRowCount, maxd);
             const auto launch = [&](auto kernel) {
@@ -3943,13 +4026,15 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
         }
     } else if (m.TileRows.Get() != nullptr) {
         evaluate = "EvalObliviousRowTileKernel";
-    } else if (m.Oblivious && m.MaxDepth <= 8 && TileLdsBytes(m.LayoutBuckets, dchunk) <= kMaxTileLdsBytes) {
+    } else if (m.Oblivious && m.MaxDepth <= 8 && m.TileFits()) {
         evaluate = "EvalObliviousTileKernel";
     } else if (m.QuadRows.Get() != nullptr) {
         evaluate = "EvalObliviousQuadTileKernel";
     } else if (m.Oblivious && m.MaxDepth <= 8 && m.Dim == 1 && m.HalfTileLeaves.Get() != nullptr &&
-               TileLdsBytes(m.LayoutBuckets, 1) > kMaxTileLdsBytes && HalfTileLdsBytes(m.LayoutBuckets, 8) <= kMaxTileLdsBytes) {
-        evaluate = m.PairRows.Get() != nullptr ? "EvalObliviousPairTileKernel" : "EvalObliviousHalfTileKernel";
+               !m.TileFits() && HalfTileLdsBytes(m.LayoutBuckets, 8) <= kMaxTileLdsBytes) {
+        evaluate = m.TakesExchangeKernel(docCount) ? m.ExchangeName
+                   : m.PairRows.Get() != nullptr   ? "EvalObliviousPairTileKernel"
+                                                   : "EvalObliviousHalfTileKernel";
     } else if (m.DeepRows.Get() != nullptr) {
         evaluate = "EvalObliviousDeepTileKernel";
     } else if (m.Oblivious) {

@@ -92,6 +92,7 @@ typedef struct CbHipFeatures {
  *   CATBOOST_AMD_FUSED=0             binarize and evaluate always as two launches (no fused kernels)
  *   CATBOOST_AMD_PAIR_TILE=0         wide one-dimensional models (more buckets than an LDS tile of 256 documents
  *                                    holds): one tree per wave instead of two or four
+ *   CATBOOST_AMD_EXCHANGE=0          those models: two trees per wave also for batches that the exchange kernel would take
  *   CATBOOST_AMD_ROW_TILE=0          models outside the register kernels whose 256-document tile fits LDS: the tile
  *                                    kernel that broadcasts a tree's levels from a lane instead of the one that
  *                                    keeps a tree's row in registers (depth 9 to 16: the plain kernel)

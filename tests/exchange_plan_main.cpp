@@ -1,0 +1,54 @@
+// Prints the host tables of the exchange kernels for a model read from a file (test_exchange_kernel.py): all numbers
+// as text, one array per line.
+#include <cstdio>
+#include <fstream>
+#include <vector>
+
+#include "../catboost_amd/csrc/exchange_plan.h"
+
+int main(int argc, char** argv) {
+    if (argc != 2) {
+        return 2;
+    }
+    std::ifstream in(argv[1]);
+    size_t treeCount = 0;
+    uint32_t buckets = 0, maxDepth = 0, six = 0;
+    in >> treeCount >> buckets >> maxDepth >> six;
+    std::vector<cbamd::TExchangeTree> trees(treeCount);
+    std::vector<std::vector<double>> leaves(treeCount);
+    for (size_t t = 0; t < treeCount; ++t) {
+        size_t levels = 0;
+        in >> levels;
+        for (size_t d = 0; d < levels; ++d) {
+            cbamd::TExchangeLevel level;
+            in >> level.Bucket >> level.Add >> level.Xor >> level.IsXor >> level.Lopsided;
+            trees[t].Levels.push_back(level);
+        }
+        for (size_t i = 0; i < size_t(1) << levels; ++i) {
+            double value = 0.0;
+            in >> value;
+            leaves[t].push_back(value);
+        }
+        trees[t].Leaves = leaves[t].data();
+    }
+    if (!in) {
+        return 3;
+    }
+    cbamd::TExchangePlan plan;
+    if (!cbamd::BuildExchangePlan(trees, buckets, maxDepth, six != 0, &plan)) {
+        std::printf("refused\n");
+        return 0;
+    }
+    std::printf("%u\n", plan.Rounds);
+    for (const auto* table : {&plan.WaveTable, &plan.Records, &plan.ExtraRows}) {
+        for (uint32_t v : *table) {
+            std::printf("%u ", v);
+        }
+        std::printf("\n");
+    }
+    for (double v : plan.Leaves) {
+        std::printf("%.17g ", v);
+    }
+    std::printf("\n");
+    return 0;
+}

@@ -1,0 +1,66 @@
+"""The exchange kernels (wide one-dimensional models, most batches of more than 32768 documents) add a document's trees as the
+pair-tile kernel does: the same bits from both, and the oracle's values within the usual tolerance."""
+import numpy as np
+import pytest
+
+import catboost_amd as cb
+from oracle.oracle import OracleModel
+
+from .test_gpu_small_batch import _model_of_buckets
+
+pytestmark = pytest.mark.gpu
+
+
+def _evaluators(model, monkeypatch):
+    out = []
+    for switch in ("1", "0"):
+        monkeypatch.setenv("CATBOOST_AMD_EXCHANGE", switch)
+        g = cb.ModelCalcer()
+        g.load_from_dict(model)
+        g.enable_gpu_evaluation(0)
+        out.append(g)
+    return out
+
+
+# buckets: the most that the registers hold, ragged; trees: none, one and many of the sixteen waves' rounds of four, odd ones;
+# first: a bucket of more than 63 values takes the model out of the six-bit form
+@pytest.mark.parametrize("buckets,cats,trees,depth,first,kernel", [
+    (1024, 0, 300, 8, 1, "cbamd_eval_exchange_d8_s"),
+    (700, 10, 201, 8, 1, "cbamd_eval_exchange_d8_s"),
+    (990, 7, 1285, 7, 100, "cbamd_eval_exchange_d8"),
+    (640, 0, 129, 8, 120, "cbamd_eval_exchange_d8"),
+    (1000, 0, 250, 6, 1, "cbamd_eval_exchange_d6_s"),
+    (650, 16, 333, 5, 100, "cbamd_eval_exchange_d6"),
+    (600, 9, 150, 8, 100, "cbamd_eval_exchange_d8"),     # the 256-document tile fits LDS, but not with the row-tile kernel's regions
+])
+def test_exchange_kernel_gives_the_pair_tile_kernels_bits(buckets, cats, trees, depth, first, kernel, monkeypatch):
+    import torch
+
+    rng = np.random.default_rng(buckets + trees)
+    model, hashes = _model_of_buckets(rng, buckets, cats, trees, depth, 1, first)
+    exchange, pair = _evaluators(model, monkeypatch)
+    docs = 98_561                               # a workgroup per CU, and a generation of half as many behind them
+    x = rng.normal(size=(docs, buckets)).astype(np.float32)
+    for i in range(cats):
+        x[:, buckets - cats + i] = rng.choice(hashes[i], size=docs).view(np.float32)
+    flat = torch.from_numpy(x).to("cuda:0")
+    results = {}
+    for name, g in (("exchange", exchange), ("pair", pair)):
+        ev = g.evaluator()
+        feats = ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), flat.shape[1])
+        for n in (32768, 32769, 40_001, docs):
+            wanted = kernel if name == "exchange" and n > 32768 else "EvalObliviousPairTileKernel"
+            assert ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, n)["evaluate"] == wanted
+            out = torch.full((n + 1,), -3.0, dtype=torch.float64, device="cuda:0")
+            torch.cuda.synchronize()
+            ev.eval_data(feats, n, out.data_ptr())
+            assert out[n].item() == -3.0
+            results[name, n] = out[:n].clone()
+    for n in (32768, 32769, 40_001, docs):
+        assert torch.equal(results["exchange", n], results["pair", n]), n
+    sample = rng.choice(docs, size=300, replace=False)
+    np.testing.assert_allclose(results["exchange", docs].cpu().numpy()[sample], OracleModel(model).calc(x[sample]), rtol=1e-9, atol=1e-12)
+    # a range of the trees takes the pair-tile kernel, the whole model the exchange kernel
+    ranged = exchange.calc_flat(x[:33_000], tree_start=1, tree_end=trees)
+    np.testing.assert_allclose(ranged[sample[sample < 33_000]],
+                               OracleModel(model).calc(x[sample[sample < 33_000]], tree_start=1, tree_end=trees), rtol=1e-9, atol=1e-12)
