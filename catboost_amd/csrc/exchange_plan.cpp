@@ -1,6 +1,7 @@
 #include "exchange_plan.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <utility>
 
@@ -209,7 +210,7 @@ void Colour(std::vector<TEdge>* edges, size_t treeCount, size_t groupCount, bool
 }  // namespace
 
 bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketCount, uint32_t maxDepth, bool six,
-                       TExchangePlan* plan) {
+                       const std::vector<uint32_t>& columnOf, TExchangePlan* plan) {
     const size_t treeCount = trees.size();
     // ---- buckets to waves: the busiest first, each to the wave that compares the least
     std::vector<uint32_t> levelsOf(bucketCount, 0);
@@ -231,21 +232,35 @@ bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketC
         return false;
     }
     std::stable_sort(byLevels.begin(), byLevels.end(), [&](uint32_t a, uint32_t b) { return levelsOf[a] > levelsOf[b]; });
+    // (with tiles at most four of a tile's buckets to a wave: there are 64 of them at most)
+    const bool tiled = !columnOf.empty();
+    const uint32_t tileCount = tiled ? kExchangeTiles : 1, perTile = kExchangeWaveBuckets / tileCount;
     std::vector<uint32_t> waveOf(bucketCount, 0), registerOf(bucketCount, 0);
-    std::vector<uint32_t> taken(kExchangeWaves, 0);
+    std::vector<uint32_t> taken(kExchangeWaves * tileCount, 0);
     std::vector<size_t> load(kExchangeWaves, 0);
     plan->WaveTable.assign(size_t(kExchangeWaves) * kExchangeWaveDwords, 0);
+    plan->FusedWaveTable = plan->WaveTable;
     for (uint32_t b : byLevels) {
+        const uint32_t tile = tiled ? columnOf[b] / kExchangeTileColumns : 0;
+        if (tile >= tileCount) {
+            return false;
+        }
         uint32_t best = kExchangeWaves;
         for (uint32_t w = 0; w < kExchangeWaves; ++w) {
-            if (taken[w] < kExchangeWaveBuckets && (best == kExchangeWaves || load[w] < load[best])) {
+            if (taken[w * tileCount + tile] < perTile && (best == kExchangeWaves || load[w] < load[best])) {
                 best = w;
             }
         }
+        if (best == kExchangeWaves) {
+            return false;
+        }
         waveOf[b] = best;
-        registerOf[b] = taken[best]++;
+        registerOf[b] = tile * perTile + taken[best * tileCount + tile]++;
         load[best] += levelsOf[b];
         plan->WaveTable[best * kExchangeWaveDwords + registerOf[b]] = b * 256u;
+        if (tiled) {
+            plan->FusedWaveTable[best * kExchangeWaveDwords + registerOf[b]] = columnOf[b] % kExchangeTileColumns * kExchangeColumnBytes;
+        }
     }
 
     // ---- trees to the waves that sum them, and to steps
@@ -391,6 +406,7 @@ bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketC
         uint32_t* wave = plan->WaveTable.data() + w * kExchangeWaveDwords;
         wave[kExchangeWaveBuckets] = static_cast<uint32_t>(plan->ExtraRows.size() * sizeof(uint32_t));
         wave[kExchangeWaveBuckets + 1] = static_cast<uint32_t>(early[w].size());
+        std::copy_n(wave + kExchangeWaveBuckets, 2, plan->FusedWaveTable.data() + w * kExchangeWaveDwords + kExchangeWaveBuckets);
         const auto addExtra = [&](uint32_t g) {
             plan->ExtraRows.resize(plan->ExtraRows.size() + kExchangeGroupDwords);
             uint32_t* row = plan->ExtraRows.data() + plan->ExtraRows.size() - kExchangeGroupDwords;
@@ -436,6 +452,122 @@ bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketC
         for (size_t i = 0; i < leafCount; ++i) {
             values[i] = trees[t].Leaves[low[i & 15] | high[i >> 4]];
         }
+    }
+    return true;
+}
+
+void MakeExchangeGrid(bool six, TExchangeColumn* column) {
+    const uint32_t cells = ExchangeGridCells(six);
+    std::vector<float> borders(column->Values.size());
+    std::memcpy(borders.data(), column->Values.data(), borders.size() * sizeof(float));
+    column->Scale = column->Bias = 0.0f;
+    const float span = borders.empty() ? 0.0f : borders.back() - borders.front();
+    if (std::isfinite(span) && span > 0.0f) {
+        const float scale = 1.0f / span, bias = -borders.front() * scale;
+        if (std::isfinite(scale) && std::isfinite(bias)) {
+            column->Scale = scale;
+            column->Bias = bias;
+        }
+    }
+    column->Start.assign(cells, 0);
+    for (float border : borders) {
+        const float place = std::fma(border, column->Scale, column->Bias);
+        const float clamped = place > 0.0f ? std::min(place, 1.0f) : 0.0f;  // (NaN: 0)
+        const float cell = std::fma(clamped, static_cast<float>(cells - 1), 8388608.0f) - 8388608.0f;
+        ++column->Start[static_cast<uint32_t>(cell)];
+    }
+    const uint32_t tallest = *std::max_element(column->Start.begin(), column->Start.end());
+    column->Steps = 0;
+    while ((1u << column->Steps) - 1 < tallest) {
+        ++column->Steps;
+    }
+    uint32_t below = 0;
+    for (uint32_t& start : column->Start) {
+        const uint32_t here = start;
+        start = below;
+        below += here;
+    }
+}
+
+bool BuildExchangeTiles(const std::vector<TExchangeColumn>& columns, const std::vector<uint32_t>& pieces, bool six,
+                        std::vector<uint32_t>* table, std::vector<uint32_t>* oneHot) {
+    constexpr uint32_t kInfoDwords = 4, kOffsetsAt = 64, kHeaderDwords = 320;
+    constexpr uint32_t kParameterDwords = 12, kRecordDwords = 16;
+    const uint32_t slots = six ? 64 : 128;  // borders of a column, +inf behind the real ones
+    const uint32_t cells = ExchangeGridCells(six), columnDwords = slots + cells / 4;
+    const uint32_t pieceDwords = kExchangePieceColumns * columnDwords + 4;  // so that the pieces' tables start in different banks
+    const uint32_t parametersAt = kExchangeTilePieces * pieceDwords;
+    const uint32_t imageDwords = parametersAt + kExchangeTilePieces * kParameterDwords;
+    const size_t tiles = columns.size() / kExchangeTileColumns;
+    if (tiles == 0 || tiles > kExchangeTiles) {
+        return false;
+    }
+    table->assign(kHeaderDwords + tiles * imageDwords, 0);
+    oneHot->clear();
+    std::copy(pieces.begin(), pieces.end(), table->begin() + kOffsetsAt);
+    for (size_t t = 0; t < tiles; ++t) {
+        uint32_t* info = table->data() + t * kInfoDwords;
+        uint32_t* image = table->data() + kHeaderDwords + t * imageDwords;
+        const TExchangeColumn* tile = columns.data() + t * kExchangeTileColumns;
+        std::vector<uint32_t> hot;
+        uint32_t steps = 1;
+        for (uint32_t c = 0; c < kExchangeTileColumns; ++c) {
+            if (tile[c].Used && tile[c].OneHot) {
+                hot.push_back(c);
+            } else if (tile[c].Used) {
+                if (tile[c].Values.size() > slots || tile[c].Steps > kExchangeMaxSteps) {
+                    return false;
+                }
+                steps = std::max(steps, tile[c].Steps);
+            }
+        }
+        info[0] = steps;
+        info[1] = static_cast<uint32_t>(hot.size());
+        info[2] = static_cast<uint32_t>(oneHot->size() * sizeof(uint32_t));
+        for (uint32_t c = 0; c < kExchangeTileColumns; ++c) {
+            const bool searched = tile[c].Used && !tile[c].OneHot;
+            uint32_t* parameters = image + parametersAt + c / kExchangePieceColumns * kParameterDwords;
+            uint32_t* borders = image + c / kExchangePieceColumns * pieceDwords + c % kExchangePieceColumns * columnDwords;
+            uint8_t* lut = reinterpret_cast<uint8_t*>(borders + slots);
+            for (uint32_t k = 0; k < slots; ++k) {
+                borders[k] = searched && k < tile[c].Values.size() ? tile[c].Values[k] : 0x7f800000u;
+            }
+            if (searched) {
+                std::memcpy(parameters + c % kExchangePieceColumns, &tile[c].Scale, 4);
+                std::memcpy(parameters + kExchangePieceColumns + c % kExchangePieceColumns, &tile[c].Bias, 4);
+                for (uint32_t cell = 0; cell < cells; ++cell) {
+                    const uint32_t start = std::min(tile[c].Start[cell], slots + 1 - (1u << steps));  // the search ends inside the slots
+                    lut[cell] = static_cast<uint8_t>(six ? start * 4 : start);
+                }
+            }
+            if (c % kExchangePieceColumns == 0) {
+                parameters[2 * kExchangePieceColumns] = pieces[(t + 1) % tiles * kExchangeTilePieces + c / kExchangePieceColumns];
+            }
+        }
+        // the one-hot columns: where their records are, then the records (sixteen dwords each, and sixteen per eight values)
+        const size_t list = oneHot->size();
+        oneHot->resize(list + hot.size(), 0);
+        for (size_t k = 0; k < hot.size(); ++k) {
+            const TExchangeColumn& column = tile[hot[k]];
+            (*oneHot)[list + k] = static_cast<uint32_t>(oneHot->size() * sizeof(uint32_t));
+            const size_t chunks = (column.Values.size() + 7) / 8;
+            if (chunks == 0) {
+                return false;
+            }
+            const size_t record = oneHot->size();
+            oneHot->resize(record + (1 + chunks) * kRecordDwords, 0);
+            (*oneHot)[record] = column.RowByte;
+            (*oneHot)[record + 1] = hot[k] * kExchangeColumnBytes;
+            (*oneHot)[record + 2] = static_cast<uint32_t>(chunks);
+            for (size_t i = 0; i < 8 * chunks; ++i) {
+                const size_t value = i < column.Values.size() ? i : 0;  // the first one again behind the last
+                (*oneHot)[record + kRecordDwords + 2 * i] = column.Values[value];
+                (*oneHot)[record + kRecordDwords + 2 * i + 1] = static_cast<uint32_t>(value) + 1;
+            }
+        }
+    }
+    if (oneHot->empty()) {
+        oneHot->resize(1, 0);
     }
     return true;
 }

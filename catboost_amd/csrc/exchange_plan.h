@@ -31,6 +31,13 @@ constexpr uint32_t kExchangeRecordDwords = kExchangeRoundSteps * (kExchangeGroup
 constexpr uint32_t kExchangeWaveDwords = 80;     // per wave: 64 bucket offsets in bytes, offset of its first extra group row in
                                                  // bytes, how many of those come before the first step
 
+// Fused kernels: tiles of sixteen pieces of four neighbouring columns, the bins of a tile's 64 columns in a buffer in LDS
+constexpr uint32_t kExchangeTiles = 16;
+constexpr uint32_t kExchangeTilePieces = 16, kExchangePieceColumns = 4;
+constexpr uint32_t kExchangeTileColumns = kExchangeTilePieces * kExchangePieceColumns;
+constexpr uint32_t kExchangeColumnBytes = 260;   // of the buffer
+constexpr uint32_t kExchangeNoColumn = ~0u;
+
 struct TExchangeLevel {
     uint32_t Bucket = 0;
     uint32_t Add = 0;       // byte added to the (xored) bin: the level's result is the carry into bit 7
@@ -47,6 +54,7 @@ struct TExchangeTree {
 struct TExchangePlan {
     uint32_t Rounds = 0;
     std::vector<uint32_t> WaveTable;  // [wave][kExchangeWaveDwords]
+    std::vector<uint32_t> FusedWaveTable;  // the same with the registers' columns in the buffer for the buckets' offsets
     std::vector<uint32_t> Records;    // [round + 1][wave][kExchangeRecordDwords]: rows are fetched ahead
     std::vector<uint32_t> ExtraRows;  // [wave][its extra groups][kExchangeGroupDwords], and kExchangeEarlyRows spare ones
     std::vector<double> Leaves;       // [round + 1][wave][step][1 << maxDepth]
@@ -54,9 +62,36 @@ struct TExchangePlan {
 
 // maxDepth: 6 or 8, at least the deepest tree's. six: all bins are at most 63, and the levels of even places in a group
 // have their results in bit 6. Tree t of pair p = t / 2 is summed by wave p % 16, the last tree of an odd number by wave 0
-// behind its others: the sums and their order are the pair-tile kernel's. Returns false if the model does not fit (too many
+// behind its others: the sums and their order are the pair-tile kernel's. columnOf: empty, or per bucket tile * 64 + column for
+// a fused kernel (registers 4 t .. 4 t + 3 of a wave then hold buckets of tile t). Returns false if the model does not fit (too many
 // buckets, or groups that no slot is left for).
 bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketCount, uint32_t maxDepth, bool six,
-                       TExchangePlan* plan);
+                       const std::vector<uint32_t>& columnOf, TExchangePlan* plan);
+
+// A column of a tile of the fused kernels
+struct TExchangeColumn {
+    bool Used = false, OneHot = false;
+    uint32_t RowByte = 0;                // one-hot: where it is in a row
+    std::vector<uint32_t> Values;        // bits of the sorted borders, or hashes
+    float Scale = 0.0f, Bias = 0.0f;     // the borders' grid (MakeExchangeGrid), its search steps and the borders below each of its cells
+    uint32_t Steps = 0;
+    std::vector<uint32_t> Start;
+};
+
+constexpr uint32_t kExchangeMaxSteps = 4;
+
+// cells of a column's grid: what its 768 bytes of tables have room for beside 64 or 128 borders
+constexpr uint32_t ExchangeGridCells(bool six) {
+    return six ? 512 : 256;
+}
+
+// The grid over a column's sorted borders: a value's cell is fma(clamp(fma(value, Scale, Bias), 0, 1), cells - 1, 2^23) - 2^23, in fp32,
+// which rises with the value; so the borders of lower cells are below the value and those of higher cells are not.
+void MakeExchangeGrid(bool six, TExchangeColumn* column);
+
+// Tables of the fused kernels (gen_eval_exchange_kernel.py): infos and images of the tiles, and the one-hot columns' records.
+// columns: [tile][64]; pieces: [tile][16] byte offsets in a row. Returns false if a column's borders or steps do not fit.
+bool BuildExchangeTiles(const std::vector<TExchangeColumn>& columns, const std::vector<uint32_t>& pieces, bool six,
+                        std::vector<uint32_t>* table, std::vector<uint32_t>* oneHot);
 
 }  // namespace cbamd

@@ -27,14 +27,32 @@ buckets 0.70 ms; with half of the leaf values' copies left out 0.60, without the
 addressed by vector registers (nine more vector instructions) 0.72, leaf values through registers and ds_write_b128 0.78, one
 tree in four gathered from global memory 0.70. Some 13 us per workgroup go to its start (the bins, the first groups) and end.
 
-Kernel arguments (80 bytes):
+Fused variants ("cbamd_fused_exchange_...") take the documents' rows and make the bins themselves, tile by tile: a tile is sixteen
+*pieces* of four neighbouring columns (16 bytes of a row). A lane loads a piece of its four documents (sixteen lanes a row's
+pieces, so a load reads whole stretches of four rows), finds the bins as the other fused kernels do - cell of a grid of
+256, table of search starts, a branch-free search of 1 to 4 steps - with its columns' borders and start tables in LDS, and
+writes a dword of four documents' bins per column to a buffer [column][lane] in LDS, from which every wave takes the four of its
+64 buckets that are in this tile. A tile's tables come straight into LDS while the tile before is searched, its rows
+likewise into registers. One-hot columns are made behind that, by a wave per column. The phase takes some 55 us per workgroup of
+1016 columns: with all CUs in it at once 43 us are the rows' way from HBM (6.2 TB/s), with rows that sit in L2 it takes 45, at 43 %
+of the vector issue (12 instructions per value and search of two steps) and 36 % of LDS; the binarize launch and reading its bins took
+70 us of each workgroup's documents. Before the pieces' tables stood in different banks it took 80 us with few borders per column;
+four searches side by side instead of eight, a grid of 256 cells and a cell in five instructions instead of three: 5 to 8 us more each.
+1M documents over 1016 features, whole call, two launches -> fused: 500 trees of depth 8 1.53 -> 1.26 ms, 5000 3.77 -> 3.51.
+
+Kernel arguments (80 bytes, fused 112):
    0 bins const uint32* [docBlock][bucketCount][64]      8 wave table const uint32* [16][80]
   16 records const uint32* [rounds + 1][16][96]         24 extra group rows const uint32*
   32 leaves const double* [rounds + 1][16][4][1 << DEPTH]   40 out double* [docCount]
   48 bias const double*                                 56 scale double
   64 docCount uint32   68 rounds uint32 (>= 1)   72 bytes of a document block's bins uint32
+  fused: the bins are not there, the wave table's offsets are byte offsets of columns in the buffer
+  80 rows const float*   88 tile table const uint32* (TILE_HEADER bytes, then an image per tile)
+  96 row stride in bytes uint32   100 tiles uint32 (1 .. 16)   104 one-hot columns const uint32*
 grid = document blocks, 1024 threads; LDS: the slots, then sixteen times three leaf regions; at the end the partial sums.
 """
+
+import struct
 
 WAVES = 16
 WAVE_BUCKETS = 64
@@ -48,19 +66,51 @@ EARLY_ROWS = 3            # rows of the groups before the first step that are fe
 RECORD_BYTES = ROUND_STEPS * (GROUP_BYTES + TREE_ROW_BYTES)
 SKIP_FLAG = 0x20000000  # the lowest of a group row's flags
 
-SHAPES = [(depth, six) for depth in (8, 6) for six in (False, True)]
+# the fused kernels' binarize phase
+TILES = 16
+TILE_COLUMNS = 64
+COLUMN_BYTES = 260         # of the buffer: 64 dwords and one more, so that a tile's columns start in different banks
+OFFSETS_AT = 256           # behind the tiles' infos (16 bytes: search steps, one-hot columns, byte offset of their list): per tile the
+                           # byte offsets of its pieces in a row
+TILE_HEADER = OFFSETS_AT + TILES * 64
+PARAMETERS_BYTES = 768     # of an image: per piece 48 bytes, four scale, four bias, the next tile's piece, three spare dwords
+TABLE_BYTES = 768          # of a column in an image: its borders, then the search starts of its grid's cells
+ONE_HOT_BYTES = 64         # record of a one-hot column: byte offset in a row, offset in the buffer, records of values; then those
+MAX_STEPS = 4
+BUFFERS = [0, TILE_COLUMNS * COLUMN_BYTES]
+IMAGES_AT = 33 * 1024
+
+SHAPES = [(depth, six, fused) for fused in (False, True) for depth in (8, 6) for six in (False, True)]
 
 
-def kernel_name(depth, six):
-    return "cbamd_eval_exchange_d%d%s" % (depth, "_s" if six else "")
+def border_bytes(six):
+    return 256 if six else 512
 
 
-def lds_bytes(depth):
-    return SLOTS * 256 + WAVES * REGIONS * (8 << depth)
+def grid_cells(six):
+    return TABLE_BYTES - border_bytes(six)
 
 
-def gen_kernel(depth, six):
-    name = kernel_name(depth, six)
+# From one piece's tables to the next one's: sixteen bytes more than their size, so that pieces whose lanes look at the same place of
+# their tables (few borders, values that agree) look at different banks.
+PIECE_BYTES = 4 * TABLE_BYTES + 16
+
+
+def image_bytes():
+    return TILE_COLUMNS // 4 * PIECE_BYTES + PARAMETERS_BYTES
+
+
+def kernel_name(depth, six, fused=False):
+    return "cbamd_%s_exchange_d%d%s" % ("fused" if fused else "eval", depth, "_s" if six else "")
+
+
+def lds_bytes(depth, six=False, fused=False):
+    walk = SLOTS * 256 + WAVES * REGIONS * (8 << depth)
+    return max(walk, IMAGES_AT + 2 * image_bytes()) if fused else walk
+
+
+def gen_kernel(depth, six, fused=False):
+    name = kernel_name(depth, six, fused)
     leaf_bytes = 8 << depth
     round_leaf_bytes = WAVES * ROUND_STEPS * leaf_bytes
     round_record_bytes = WAVES * RECORD_BYTES
@@ -226,6 +276,295 @@ def gen_kernel(depth, six):
         fetch_leaves(regions[(number + 2) % REGIONS], i % 2 == 1)
         compare_group(groups[i % 2], "%s_t%d" % (name, number))
 
+    def binarize_tiles():
+        """The binarize phase: the wave's bins from the documents' rows. Vector registers below the bins but v1 are free,
+        scalar registers from 26 on."""
+        two, tile, following, left, table, wave_lists = 26, 27, 28, 29, 30, 32
+        stride, tiles, one_hot, register, last = 34, 35, 36, 38, 39
+        infos, lists = [64, 68], [72, 76]
+        highest_cell = 101
+        rows_base, rows_there = [80, 82, 84, 86], [88, 90, 92, 94]  # per document of a lane: its rows' base, the lanes that have one
+        table_of_float, two_to_23, tables = 0, 2, 3      # tables - the bits of 2^23; 2^23; LDS address of the piece's tables
+        scale, bias, offset, out = 4, 8, 12, 12
+        values, place, probe = [16, 32], 48, 56
+        image = image_bytes()
+        per_wave = image // WAVES // 1024 * 1024
+        copies = per_wave // 1024 + 1
+        assert image == WAVES * per_wave + 1024
+        assert IMAGES_AT >= BUFFERS[1] + TILE_COLUMNS * COLUMN_BYTES and IMAGES_AT % 1024 == image % 1024 == 0
+        # byte of a position's dword that belongs to the piece and not to the bin: (piece * PIECE_BYTES / 4) % 256 = 4 * piece
+        assert PIECE_BYTES // 4 % 256 == 4 and 4 * (TILE_COLUMNS // 4 - 1) + border_bytes(six) // 4 < 256
+
+        def copy_image(x):
+            """The following tile's image: the wave's share of it, the last 1 KB (with the parameters) by every wave alike."""
+            e("  v_lshlrev_b32_e32 v%d, 2, v1" % probe)
+            e("  s_mul_i32 s4, s3, 0x%x" % per_wave)
+            e("  s_mul_i32 s5, s%d, 0x%x" % (following, image))
+            e("  s_add_u32 s5, s5, 0x%x" % TILE_HEADER)
+            e("  s_add_u32 s6, s4, s5")
+            e("  s_add_u32 s6, s%d, s6" % table)
+            e("  s_addc_u32 s7, s%d, 0" % (table + 1))
+            e("  s_add_u32 m0, s4, 0x%x" % (IMAGES_AT + x * image))
+            e("  s_nop 0")
+            for piece in range(copies - 1):
+                e("  global_load_lds_dwordx4 v%d, s[6:7]%s" % (probe, " offset:%d" % (piece * 1024) if piece else ""))
+            e("  s_add_u32 s5, s5, 0x%x" % (image - 1024))
+            e("  s_add_u32 s6, s%d, s5" % table)
+            e("  s_addc_u32 s7, s%d, 0" % (table + 1))
+            e("  s_mov_b32 m0, 0x%x" % (IMAGES_AT + (x + 1) * image - 1024))
+            e("  s_nop 0")
+            e("  global_load_lds_dwordx4 v%d, s[6:7]" % probe)
+
+        def load_values(x):
+            """(A lane without a document keeps what its registers hold.)"""
+            e("  v_lshrrev_b32_e32 v%d, 6, v1" % probe)
+            e("  s_lshl_b32 s4, s3, 2")
+            e("  v_add_u32_e32 v%d, s4, v%d" % (probe, probe))
+            e("  v_mul_lo_u32 v%d, v%d, s%d" % (probe, probe, stride))
+            e("  v_add_u32_e32 v%d, v%d, v%d" % (probe, probe, offset))
+            for j in range(4):
+                e("  s_mov_b64 exec, s[%d:%d]" % (rows_there[j], rows_there[j] + 1))
+                e("  global_load_dwordx4 v[%d:%d], v%d, s[%d:%d]" % (values[x] + 4 * j, values[x] + 4 * j + 3, probe, rows_base[j], rows_base[j] + 1))
+            e("  s_mov_b64 exec, -1")
+
+        def load_infos(x):
+            """The following tile's."""
+            e("  s_lshl_b32 s4, s%d, 4" % following)
+            for regs, base in ((infos[x], table), (lists[x], wave_lists)):
+                e("  s_add_u32 s6, s%d, s4" % base)
+                e("  s_addc_u32 s7, s%d, 0" % (base + 1))
+                e("  s_load_dwordx4 s[%d:%d], s[6:7], 0x0" % (regs, regs + 3))
+
+        def next_tile():
+            """`tile` and `following` move on, round the end."""
+            e("  s_mov_b32 s%d, s%d" % (tile, following))
+            e("  s_add_u32 s%d, s%d, 1" % (following, following))
+            e("  s_cmp_eq_u32 s%d, s%d" % (following, tiles))
+            e("  s_cselect_b32 s%d, 0, s%d" % (following, following))
+
+        def search(label, x, j):
+            """The bins of the lane's documents j and j + 1 in its four columns, eight searches side by side, into bytes j and
+            j + 1 of the columns' dwords."""
+            value = values[x] + 4 * j
+
+            def step(number):
+                size = 4 << (number - 1)
+                for k in range(8):
+                    e("  ds_read_b32 v%d, v%d offset:%d" % (probe + k, place + k, k % 4 * TABLE_BYTES + size - 4))
+                e("  s_waitcnt lgkmcnt(0)")
+                for k in range(8):
+                    e("  v_cmp_lt_f32_e32 vcc, v%d, v%d" % (probe + k, value + k))
+                    e("  v_cndmask_b32_e64 v%d, 0, %d, vcc" % (probe + k, size))
+                    e("  v_add_u32_e32 v%d, v%d, v%d" % (place + k, place + k, probe + k))
+            for k in range(8):
+                c = k % 4
+                # the value's cell, 0 .. highest_cell, in the low bits of 2^23 + cell; NaN (and -inf) in the first one
+                e("  v_fma_f32 v%d, v%d, v%d, v%d clamp" % (probe + k, value + k, scale + c, bias + c))
+                e("  v_fma_f32 v%d, v%d, s%d, v%d" % (probe + k, probe + k, highest_cell, two_to_23))
+                e("  v_add_u32_e32 v%d, v%d, v%d" % (probe + k, probe + k, table_of_float))
+                e("  ds_read_u8 v%d, v%d offset:%d" % (place + k, probe + k, c * TABLE_BYTES + border_bytes(six)))
+            e("  s_waitcnt lgkmcnt(0)")
+            for k in range(8):
+                if six:
+                    e("  v_add_u32_e32 v%d, v%d, v%d" % (place + k, place + k, tables))
+                else:
+                    e("  v_lshl_add_u32 v%d, v%d, 2, v%d" % (place + k, place + k, tables))
+            for number in range(MAX_STEPS, 1, -1):
+                e("  s_cmp_lt_u32 s%d, %d" % (infos[x], number))
+                e("  s_cbranch_scc1 %s_%d_below%d" % (label, j, number))
+                step(number)
+                e("%s_%d_below%d:" % (label, j, number))
+            step(1)
+            for k in range(8):
+                # bits 2 .. 9: the bin and what the place of the piece's tables adds to it
+                e("  v_lshrrev_b32_sdwa v%d, s%d, v%d dst_sel:BYTE_%d dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD"
+                  % (out + k % 4, two, place + k, j + k // 4))
+
+        def one_hot_columns(label, x):
+            """A wave per one-hot column of the tile (column k of them by wave k % 16), behind the other columns."""
+            e("%s_hot:" % label)
+            e("  s_waitcnt lgkmcnt(0)")
+            e("  s_barrier")                       # the dwords of these columns that the lanes have written are overwritten
+            e("  s_mov_b32 s40, s3")
+            e("  s_lshl_b32 s4, s3, 2")
+            e("  s_add_u32 s6, s%d, s%d" % (one_hot, infos[x] + 2))
+            e("  s_addc_u32 s7, s%d, 0" % (one_hot + 1))
+            e("  s_add_u32 s6, s6, s4")
+            e("  s_addc_u32 s7, s7, 0")
+            e("%s_hot_next:" % label)
+            e("  s_cmp_ge_u32 s40, s%d" % (infos[x] + 1))
+            e("  s_cbranch_scc1 %s_hot_done" % label)
+            e("  s_load_dword s41, s[6:7], 0x0")   # byte offset of the column's record
+            e("  s_waitcnt lgkmcnt(0)")
+            e("  s_add_u32 s42, s%d, s41" % one_hot)
+            e("  s_addc_u32 s43, s%d, 0" % (one_hot + 1))
+            e("  s_load_dwordx4 s[44:47], s[42:43], 0x0")    # offset in a row, offset in the buffer, records of eight values
+            e("  s_waitcnt lgkmcnt(0)")
+            # all documents of the block, lane l's are l, l + 64 ..; the tile's own values are no longer needed
+            for j in range(4):
+                e("  v_lshrrev_b32_e32 v%d, 2, v1" % (place + j))
+                e("  v_add_u32_e32 v%d, %d, v%d" % (place + j, 64 * j, place + j))
+                e("  v_min_u32_e32 v%d, s%d, v%d" % (place + j, last, place + j))
+                e("  v_mul_lo_u32 v%d, v%d, s%d" % (place + j, place + j, stride))
+                e("  v_add_u32_e32 v%d, s44, v%d" % (place + j, place + j))
+            for j in range(4):
+                e("  global_load_dword v%d, v%d, s[%d:%d]" % (values[x] + j, place + j, rows_base[0], rows_base[0] + 1))
+            for j in range(4):
+                e("  v_mov_b32_e32 v%d, 0" % (probe + j))
+            e("  s_waitcnt vmcnt(0)")
+            e("%s_hot_values:" % label)
+            e("  s_add_u32 s42, s42, %d" % ONE_HOT_BYTES)
+            e("  s_addc_u32 s43, s43, 0")
+            e("  s_load_dwordx16 s[48:63], s[42:43], 0x0")   # eight times (value, bin)
+            e("  s_waitcnt lgkmcnt(0)")
+            for i in range(8):
+                e("  v_mov_b32_e32 v%d, s%d" % (place, 49 + 2 * i))
+                for j in range(4):
+                    e("  v_cmp_eq_u32_e32 vcc, s%d, v%d" % (48 + 2 * i, values[x] + j))
+                    e("  v_cndmask_b32_e32 v%d, v%d, v%d, vcc" % (probe + j, probe + j, place))
+            e("  s_sub_u32 s46, s46, 1")
+            e("  s_cmp_lg_u32 s46, 0")
+            e("  s_cbranch_scc1 %s_hot_values" % label)
+            for j in range(1, 4):
+                e("  v_lshl_or_b32 v%d, v%d, %d, v%d" % (probe, probe + j, 8 * j, probe))
+            e("  s_mov_b32 m0, s45")
+            e("  s_nop 0")
+            e("  ds_write_addtid_b32 v%d offset:%d" % (probe, BUFFERS[x]))
+            e("  s_add_u32 s40, s40, %d" % WAVES)
+            e("  s_add_u32 s6, s6, %d" % (4 * WAVES))
+            e("  s_addc_u32 s7, s7, 0")
+            e("  s_branch %s_hot_next" % label)
+            e("%s_hot_done:" % label)
+            e("  s_branch %s_hot_back" % label)
+
+        def read_bins(x):
+            """The wave's four columns of a tile, behind its barrier."""
+            for i in range(4):
+                e("  s_mov_b32 m0, s%d" % (lists[x] + i))
+                e("  s_nop 0")
+                e("  ds_read_addtid_b32 v%d offset:%d" % (place + i, BUFFERS[x]))
+
+        def take_bins():
+            """... into their registers (before the first tile: of no tile, into the first one's registers, which are written again)."""
+            e("  s_set_gpr_idx_on s%d, 0x8" % register)
+            for i in range(4):
+                e("  v_mov_b32_e32 v%d, v%d" % (b0 + i, place + i))
+            e("  s_set_gpr_idx_off")
+            e("  s_lshl_b32 s%d, s%d, 2" % (register, tile))
+
+        def lane_piece(piece, document):
+            """The lane's piece, and its first document of the block: 4 * wave + lane / 16."""
+            e("  v_lshrrev_b32_e32 v%d, 6, v1" % document)
+            e("  s_lshl_b32 s4, s3, 2")
+            e("  v_add_u32_e32 v%d, s4, v%d" % (document, document))
+            e("  v_bfe_u32 v%d, v1, 2, 4" % piece)
+
+        e("  s_load_dwordx8 s[40:47], s[0:1], 0x50")    # rows, tile table, stride, tiles, one-hot columns
+        e("  s_waitcnt lgkmcnt(0)")
+        e("  s_mov_b64 s[%d:%d], s[42:43]" % (table, table + 1))
+        e("  s_mov_b64 s[%d:%d], s[10:11]" % (wave_lists, wave_lists + 1))
+        e("  s_mov_b32 s%d, s44" % stride)
+        e("  s_mov_b32 s%d, s45" % tiles)
+        e("  s_mov_b64 s[%d:%d], s[46:47]" % (one_hot, one_hot + 1))
+        e("  s_lshl_b32 s4, s2, 8")
+        e("  s_sub_u32 s%d, s24, s4" % last)            # last row of the batch, counted from the block's first, at most 255
+        e("  s_sub_u32 s%d, s%d, 1" % (last, last))
+        e("  s_min_u32 s%d, s%d, 0xff" % (last, last))
+        e("  s_mul_i32 s5, s4, s%d" % stride)
+        e("  s_mul_hi_u32 s6, s4, s%d" % stride)
+        e("  s_add_u32 s%d, s40, s5" % rows_base[0])
+        e("  s_addc_u32 s%d, s41, s6" % (rows_base[0] + 1))
+        e("  s_lshl_b32 s4, s%d, 6" % stride)           # 64 rows
+        for j in range(1, 4):
+            e("  s_add_u32 s%d, s%d, s4" % (rows_base[j], rows_base[j - 1]))
+            e("  s_addc_u32 s%d, s%d, 0" % (rows_base[j] + 1, rows_base[j - 1] + 1))
+        lane_piece(probe, probe + 1)
+        for j in range(4):
+            e("  v_add_u32_e32 v%d, %d, v%d" % (place + j, 64 * j, probe + 1))
+            e("  v_cmp_ge_u32_e64 s[%d:%d], s%d, v%d" % (rows_there[j], rows_there[j] + 1, last, place + j))
+        # The workgroups start with different tiles: those that run side by side would otherwise all read the same columns of
+        # their rows, and rows of about 4 KB put these on few memory channels (262 000 documents, 500 trees: 431 -> 400 us).
+        e("  s_mov_b32 s%d, s%d" % (left, tiles))
+        e("  s_and_b32 s4, s2, 15")
+        e("  s_mul_i32 s4, s4, s%d" % tiles)
+        e("  s_lshr_b32 s%d, s4, 4" % following)
+        e("  s_lshl_b32 s%d, s%d, 2" % (register, following))
+        e("  s_lshl_b32 s4, s%d, 6" % following)
+        e("  s_add_u32 s4, s4, %d" % OFFSETS_AT)
+        e("  s_add_u32 s6, s%d, s4" % table)
+        e("  s_addc_u32 s7, s%d, 0" % (table + 1))
+        e("  v_lshlrev_b32_e32 v%d, 2, v%d" % (place, probe))
+        e("  global_load_dword v%d, v%d, s[6:7]" % (offset, place))
+        e("  v_mul_u32_u24_e32 v%d, 0x%x, v%d" % (tables, PIECE_BYTES, probe))
+        e("  v_add_u32_e32 v%d, 0x%x, v%d" % (tables, IMAGES_AT, tables))
+        e("  v_mov_b32_e32 v%d, 0x4b000000" % two_to_23)
+        e("  v_sub_u32_e32 v%d, v%d, v%d" % (table_of_float, tables, two_to_23))
+        copy_image(0)
+        load_infos(0)
+        next_tile()
+        e("  s_mov_b32 s%d, 2" % two)
+        e("  s_mov_b32 s%d, 0x%x" % (highest_cell, struct.unpack("<I", struct.pack("<f", grid_cells(six) - 1))[0]))
+        for i in range(4):
+            e("  s_mov_b32 s%d, 0" % (lists[1] + i))     # of the tile before the first
+        e("  s_waitcnt vmcnt(%d)" % copies)
+        load_values(0)
+        e("  s_waitcnt vmcnt(4) lgkmcnt(0)")
+        e("  s_barrier")
+        e("%s_tiles:" % name)
+        for x in range(2):
+            label = "%s_tile%d" % (name, x)
+            read_bins(1 - x)
+            e("  v_bfe_u32 v%d, v1, 2, 4" % probe)
+            e("  v_mul_u32_u24_e32 v%d, 48, v%d" % (probe, probe))
+            e("  v_add_u32_e32 v%d, 0x%x, v%d" % (probe, IMAGES_AT + (x + 1) * image - PARAMETERS_BYTES, probe))
+            for q in range(3):
+                e("  ds_read_b128 v[%d:%d], v%d%s" % (scale + 4 * q, scale + 4 * q + 3, probe, " offset:%d" % (16 * q) if q else ""))
+            copy_image(1 - x)
+            e("  s_waitcnt lgkmcnt(0)")
+            take_bins()
+            load_values(1 - x)
+            load_infos(1 - x)
+            next_tile()
+            e("  s_waitcnt vmcnt(%d)" % (copies + 4))  # this tile's values
+            for j in (0, 2):
+                search(label, x, j)
+            lane_piece(place, place + 1)
+            e("  v_mul_u32_u24_e32 v%d, 0x040404, v%d" % (place + 2, place))
+            e("  v_lshlrev_b32_e32 v%d, 26, v%d" % (place + 3, place))
+            e("  v_or_b32_e32 v%d, v%d, v%d" % (place + 2, place + 2, place + 3))
+            e("  v_lshlrev_b32_e32 v%d, 2, v%d" % (place + 1, place + 1))
+            e("  v_mul_u32_u24_e32 v%d, 0x%x, v%d" % (place, 4 * COLUMN_BYTES, place))
+            e("  v_add_u32_e32 v%d, v%d, v%d" % (place, place, place + 1))
+            for c in range(4):
+                e("  v_sub_u32_e32 v%d, v%d, v%d" % (out + c, out + c, place + 2))
+                e("  ds_write_b32 v%d, v%d offset:%d" % (place, out + c, BUFFERS[x] + c * COLUMN_BYTES))
+            e("  s_cmp_lg_u32 s%d, 0" % (infos[x] + 1))
+            e("  s_cbranch_scc1 %s_hot" % label)
+            e("%s_hot_back:" % label)
+            out_of_line.append(lambda label=label, x=x: one_hot_columns(label, x))
+            e("  s_waitcnt vmcnt(4) lgkmcnt(0)")      # the next tile's image, the bins
+            e("  s_barrier")
+            for base in (tables, table_of_float):
+                e("  v_%s_u32_e32 v%d, 0x%x, v%d" % ("add" if x == 0 else "subrev", base, image, base))
+            e("  s_sub_u32 s%d, s%d, 1" % (left, left))
+            e("  s_cmp_eq_u32 s%d, 0" % left)
+            e("  s_cbranch_scc1 %s_last%d" % (name, x))
+        e("  s_branch %s_tiles" % name)
+        for x in range(2):
+            e("%s_last%d:" % (name, x))
+            read_bins(x)
+            if x == 0:
+                e("  s_branch %s_binarized" % name)
+        e("%s_binarized:" % name)
+        e("  s_waitcnt vmcnt(0) lgkmcnt(0)")
+        take_bins()
+        e("  v_lshrrev_b32_e32 v0, 2, v1")
+        e("  s_lshl_b32 s4, s3, 6")
+        e("  v_add_u32_e32 v0, s4, v0")
+        e("  v_lshlrev_b32_e32 v2, 2, v1")
+        # the leaf regions and slots take the images' and buffers' place
+        e("  s_barrier")
+
     e(".text")
     e(".globl %s" % name)
     e(".p2align 8")
@@ -239,17 +578,14 @@ def gen_kernel(depth, six):
     e("  v_readfirstlane_b32 s3, v4")
     e("  v_lshlrev_b32_e32 v2, 4, v1")
     e("  v_lshlrev_b32_e32 v1, 2, v1")
-    for j in range(4):
-        e("  v_mov_b32_e32 v%d, 0x%x" % (sc0 + j, (1 << (3 - first_bit)) << (8 * j)))
-    for r in list(range(lv0, lv0 + 8)) + list(range(ac0, ac0 + 8)):
-        e("  v_mov_b32_e32 v%d, 0" % r)
     e("  s_mov_b32 s%d, 0x80808080" % high_bits)
     e("  s_mov_b32 s%d, 0xc0c0c0c0" % pair_bits)
     e("  s_waitcnt lgkmcnt(0)")
-    e("  s_mul_i32 s4, s2, s26")
-    e("  s_mul_hi_u32 s5, s2, s26")
-    e("  s_add_u32 s8, s8, s4")
-    e("  s_addc_u32 s9, s9, s5")
+    if not fused:
+        e("  s_mul_i32 s4, s2, s26")
+        e("  s_mul_hi_u32 s5, s2, s26")
+        e("  s_add_u32 s8, s8, s4")
+        e("  s_addc_u32 s9, s9, s5")
     e("  s_mov_b64 s[6:7], s[12:13]")               # records to s[14:15], extra rows to s[12:13]
     e("  s_mov_b64 s[12:13], s[14:15]")
     e("  s_mov_b64 s[14:15], s[6:7]")
@@ -257,20 +593,29 @@ def gen_kernel(depth, six):
         e("  s_mul_i32 s4, s3, 0x%x" % per_wave)
         e("  s_add_u32 s%d, s%d, s4" % (pointer, pointer))
         e("  s_addc_u32 s%d, s%d, 0" % (pointer + 1, pointer + 1))
+    if fused:
+        binarize_tiles()
+    for j in range(4):
+        e("  v_mov_b32_e32 v%d, 0x%x" % (sc0 + j, (1 << (3 - first_bit)) << (8 * j)))
+    for r in list(range(lv0, lv0 + 8)) + list(range(ac0, ac0 + 8)):
+        e("  v_mov_b32_e32 v%d, 0" % r)
     e("  s_load_dwordx2 s[6:7], s[10:11], 0x%x" % (4 * WAVE_BUCKETS))
     e("  s_mul_i32 s4, s3, 0x%x" % (REGIONS * leaf_bytes))
     for i in range(REGIONS):
         e("  s_add_u32 s%d, s4, 0x%x" % (regions[i], SLOTS * 256 + i * leaf_bytes))
     fetch_leaves(regions[0], False)
     fetch_leaves(regions[1], True)
-    # the block's bins: the offsets of the wave's buckets take all scalar registers from 32 on for a moment
-    for part in range(WAVE_BUCKETS // 16):
-        e("  s_load_dwordx16 s[%d:%d], s[10:11], 0x%x" % (32 + 16 * part, 47 + 16 * part, part * 64))
-    e("  s_waitcnt lgkmcnt(0)")
-    for i in range(WAVE_BUCKETS):
-        e("  s_add_u32 s4, s8, s%d" % (32 + i))
-        e("  s_addc_u32 s5, s9, 0")
-        e("  global_load_dword v%d, v1, s[4:5]" % (b0 + i))
+    if fused:
+        e("  s_waitcnt lgkmcnt(0)")
+    else:
+        # the block's bins: the offsets of the wave's buckets take all scalar registers from 32 on for a moment
+        for part in range(WAVE_BUCKETS // 16):
+            e("  s_load_dwordx16 s[%d:%d], s[10:11], 0x%x" % (32 + 16 * part, 47 + 16 * part, part * 64))
+        e("  s_waitcnt lgkmcnt(0)")
+        for i in range(WAVE_BUCKETS):
+            e("  s_add_u32 s4, s8, s%d" % (32 + i))
+            e("  s_addc_u32 s5, s9, 0")
+            e("  global_load_dword v%d, v1, s[4:5]" % (b0 + i))
     e("  s_add_u32 s12, s12, s6")
     e("  s_addc_u32 s13, s13, 0")
     # the groups that the first round looks at, EARLY_ROWS at a time, the first of them on their way while the bins come
@@ -353,9 +698,9 @@ def gen_kernel(depth, six):
     e(".rodata")
     e(".p2align 6")
     e(".amdhsa_kernel %s" % name)
-    e("  .amdhsa_group_segment_fixed_size %d" % lds_bytes(depth))
+    e("  .amdhsa_group_segment_fixed_size %d" % lds_bytes(depth, six, fused))
     e("  .amdhsa_private_segment_fixed_size 0")
-    e("  .amdhsa_kernarg_size 80")
+    e("  .amdhsa_kernarg_size %d" % (112 if fused else 80))
     e("  .amdhsa_user_sgpr_count 2")
     e("  .amdhsa_user_sgpr_kernarg_segment_ptr 1")
     e("  .amdhsa_system_sgpr_workgroup_id_x 1")
@@ -378,11 +723,15 @@ def gen_kernel(depth, six):
                         for at in range(0, 56, 8))
     arguments += "      - {.offset: 56, .size: 8, .value_kind: by_value}\n"
     arguments += "".join("      - {.offset: %d, .size: 4, .value_kind: by_value}\n" % at for at in (64, 68, 72, 76))
+    if fused:
+        arguments += "".join("      - {.address_space: global, .offset: %d, .size: 8, .value_kind: global_buffer}\n" % at for at in (80, 88))
+        arguments += "".join("      - {.offset: %d, .size: 4, .value_kind: by_value}\n" % at for at in (96, 100))
+        arguments += "      - {.address_space: global, .offset: 104, .size: 8, .value_kind: global_buffer}\n"
     meta = """  - .agpr_count: 0
     .args:
 %s    .group_segment_fixed_size: %d
     .kernarg_segment_align: 8
-    .kernarg_segment_size: 80
+    .kernarg_segment_size: %d
     .max_flat_workgroup_size: %d
     .name: %s
     .private_segment_fixed_size: 0
@@ -394,5 +743,5 @@ def gen_kernel(depth, six):
     .vgpr_count: %d
     .vgpr_spill_count: 0
     .wavefront_size: 64
-""" % (arguments, lds_bytes(depth), WAVES * 64, name, name, vgprs)
+""" % (arguments, lds_bytes(depth, six, fused), 112 if fused else 80, WAVES * 64, name, name, vgprs)
     return "\n".join(o), meta

@@ -1149,8 +1149,8 @@ def generate():
                     text, meta = gen_kernel(buckets, waves, 1, 256, False, six, fused=True, levels=levels, columns=columns)
                     parts.append(text)
                     metas.append(meta)
-    for depth, six in gen_eval_exchange_kernel.SHAPES:
-        text, meta = gen_eval_exchange_kernel.gen_kernel(depth, six)
+    for shape in gen_eval_exchange_kernel.SHAPES:
+        text, meta = gen_eval_exchange_kernel.gen_kernel(*shape)
         parts.append(text)
         metas.append(meta)
     parts.append(".amdgpu_metadata")

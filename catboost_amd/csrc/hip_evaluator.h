@@ -72,7 +72,8 @@ public:
     // (anyBatchSize: also where they are)
     bool EvalFusedDevice(const TFeatureBatch& batch, size_t docCount, size_t treeStart, size_t treeEnd,
                          double* results, void* stream, bool anyBatchSize = false, TStageEnd* end = nullptr);
-    // index of the fused kernel tables that such a call would use (0 flat rows, 1 split rows, 2 flat columns), -1 when it
+    // index of the fused kernel tables that such a call would use (0 flat rows, 1 split rows, 2 flat columns, 3 flat rows of wide
+    // models: the fused exchange kernel), -1 when it
     // takes the two launches (always with a stride of 2^20 floats or more between rows, of 2^30 or more between columns, and
     // from 2^29 documents on): the one test that EvalFusedDevice, the host pipeline and DescribeKernels share
     int FusedLayoutFor(int layout, size_t stride, size_t docCount, size_t treeStart, size_t treeEnd, bool anyBatchSize) const;

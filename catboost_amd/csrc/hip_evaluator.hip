@@ -245,6 +245,16 @@ struct TEvalExchangeArgs {
     uint32_t Unused;
 };
 static_assert(sizeof(TEvalExchangeArgs) == 80, "kernel argument block of the exchange kernels");
+struct TFusedExchangeArgs {
+    TEvalExchangeArgs Walk;  // no bins; the wave table of the fused kernels
+    const float* Rows;
+    const void* Tiles;
+    uint32_t StrideBytes;
+    uint32_t TileCount;
+    const void* OneHot;
+};
+static_assert(sizeof(TFusedExchangeArgs) == 112, "kernel argument block of the fused exchange kernels");
+constexpr int kFusedExchange = 3;  // FusedLayoutFor: flat rows, the fused exchange kernel
 
 struct TEvalRegVariant {
     uint32_t Buckets;
@@ -1576,6 +1586,10 @@ struct THipEvaluator::TImpl {
     bool PairBeforeTile = false;       // the tile kernel would hold the model's bins, but the pair-tile kernel takes it
     hipFunction_t ExchangeFunction = nullptr;  // nullptr: the model does not qualify
     const char* ExchangeName = "";
+    TDeviceVec<uint32_t> FusedExchangeWaves, FusedExchangeTiles, FusedExchangeOneHot;  // its form that makes the bins from flat rows
+    uint32_t FusedExchangeTileCount = 0;
+    hipFunction_t FusedExchangeFunction = nullptr;
+    std::string FusedExchangeName;
     TDeviceVec<uint32_t> QuadRows;     // quad-tile kernel: 16 dwords per tree, 64 bytes per row of the tile
     TDeviceVec<uint32_t> TileRows;     // row-tile kernel (whole tile, one tree per wave): the same with 256 bytes per bucket
     TDeviceVec<double> TileLeaves;     // its leaf values: [slice of the dimensions][tree][pair of dimensions][leaf][2]
@@ -1717,6 +1731,22 @@ struct THipEvaluator::TImpl {
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
         const size_t generations = (blocks + CuCount - 1) / CuCount, others = (2 * blocks + CuCount - 1) / CuCount;
         return generations * (MaxDepth <= 6 ? 36 : 29) < others * 20;
+    }
+
+    // The fused form instead of a binarize launch and either kernel. A generation of its workgroups takes some 50 us longer (per 1000
+    // columns), whatever part of the CUs has one; a binarize launch takes 70 us per 65 536 documents. Whole call over 1016 features,
+    // two launches -> fused, by the share of the generations' places that have a workgroup: 0.50 (66 000 documents), 500 trees
+    // 146 -> 150 us, 5000 trees 441 -> 457; 0.69 (90 000) 182 -> 168 and 469 -> 464, but 2000 trees of depth 5 over 700 features (pair-tile)
+    // 181 -> 190; 0.77 (50 000) 96 -> 89 and 251 -> 247; 0.99 (130 000) 234 -> 192 and 525 -> 484.
+    bool TakesFusedExchangeKernel(size_t docCount) const {
+        const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
+        return FusedExchangeFunction != nullptr && docCount < (size_t(1) << 32) &&
+               blocks * 10 >= (blocks + CuCount - 1) / CuCount * CuCount * 7;
+    }
+
+    TEvalExchangeArgs ExchangeArgs(size_t docCount, double* results) const {
+        return {nullptr, ExchangeWaves.Get(), ExchangeRecords.Get(), ExchangeExtra.Get(), ExchangeLeaves.Get(), results, Bias.Get(), Scale,
+                static_cast<uint32_t>(docCount), ExchangeRounds, LayoutBuckets * dev::kDocsPerBlock, 0};
     }
 
     // The tile kernel takes the model (of kernels on bins in an LDS tile of whole blocks, the one without a tree's row in registers).
@@ -2362,8 +2392,54 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                                                                 switches.LevelOrder ? std::fabs(share - 0.5) : 0.0});
                                 }
                             }
+                            // The fused form: the model's columns in pieces of four neighbouring ones, sixteen pieces a tile. A
+                            // piece that would leave the row is moved back over its neighbour.
+                            std::vector<uint32_t> columnOf, pieces, tileTable, oneHotTable;
+                            bool tiled = switches.Fused && m.CtrCount == 0 && m.BinarizeBuckets == BucketCount && BucketCount > 0 &&
+                                         m.FlatVectorSize >= kExchangePieceColumns;
+                            std::vector<std::pair<uint32_t, uint32_t>> byColumn;
+                            for (uint32_t b = 0; tiled && b < BucketCount; ++b) {
+                                byColumn.emplace_back(srcFlat[b], b);
+                                tiled = (flags[b] & dev::kBucketFlagNanToInf) == 0 && offsets[b + 1] > offsets[b];
+                            }
+                            std::sort(byColumn.begin(), byColumn.end());
+                            columnOf.assign(m.LayoutBuckets, kExchangeNoColumn);
+                            for (size_t i = 0; tiled && i < byColumn.size(); ++i) {
+                                const uint32_t column = byColumn[i].first;
+                                if (pieces.empty() || column * 4 >= pieces.back() + 4 * kExchangePieceColumns) {
+                                    pieces.push_back(4 * std::min<uint32_t>(column & ~3u, static_cast<uint32_t>(m.FlatVectorSize) - kExchangePieceColumns));
+                                }
+                                columnOf[byColumn[i].second] = static_cast<uint32_t>(pieces.size() - 1) * kExchangePieceColumns + column - pieces.back() / 4;
+                                tiled = (i == 0 || column != byColumn[i - 1].first) && pieces.size() <= kExchangeTiles * kExchangeTilePieces;
+                            }
+                            if (tiled) {
+                                pieces.resize((pieces.size() + kExchangeTilePieces - 1) / kExchangeTilePieces * kExchangeTilePieces, 0);
+                                std::vector<TExchangeColumn> columns(pieces.size() * kExchangePieceColumns);
+                                for (uint32_t b = 0; b < BucketCount; ++b) {
+                                    TExchangeColumn& column = columns[columnOf[b]];
+                                    column.Used = true;
+                                    column.OneHot = (flags[b] & dev::kBucketFlagOneHot) != 0;
+                                    column.RowByte = srcFlat[b] * 4;
+                                    column.Values.assign(values.begin() + offsets[b], values.begin() + offsets[b + 1]);
+                                    if (!column.OneHot) {
+                                        MakeExchangeGrid(m.PairSix, &column);
+                                    }
+                                }
+                                tiled = BuildExchangeTiles(columns, pieces, m.PairSix, &tileTable, &oneHotTable);
+                            }
+                            if (!tiled) {
+                                columnOf.clear();
+                            }
                             TExchangePlan plan;
-                            if (BuildExchangePlan(levels, m.LayoutBuckets, static_cast<uint32_t>(maxd), m.PairSix, &plan)) {
+                            if (BuildExchangePlan(levels, m.LayoutBuckets, static_cast<uint32_t>(maxd), m.PairSix, columnOf, &plan)) {
+                                if (tiled) {
+                                    m.FusedExchangeWaves.Upload(plan.FusedWaveTable);
+                                    m.FusedExchangeTiles.Upload(tileTable);
+                                    m.FusedExchangeOneHot.Upload(oneHotTable);
+                                    m.FusedExchangeTileCount = static_cast<uint32_t>(pieces.size()) / kExchangeTilePieces;
+                                    m.FusedExchangeName = std::string("cbamd_fused_exchange_d") + (maxd == 6 ? "6" : "8") + (m.PairSix ? "_s" : "");
+                                    HIP_CHECK(hipModuleGetFunction(&m.FusedExchangeFunction, SharedRegModule(kEvalRegCodeObject), m.FusedExchangeName.c_str()));
+                                }
                                 m.ExchangeRounds = plan.Rounds;
                                 m.ExchangeWaves.Upload(plan.WaveTable);
                                 m.ExchangeRecords.Upload(plan.Records);
@@ -3607,9 +3683,8 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
         const int maxd = m.MaxDepth <= 6 ? 6 : 8;
         if (m.TakesExchangeKernel(docCount) && tb == 0 && te == TreeCount && (reinterpret_cast<uintptr_t>(bins) & 3) == 0) {
-            TEvalExchangeArgs args = {bins, m.ExchangeWaves.Get(), m.ExchangeRecords.Get(), m.ExchangeExtra.Get(), m.ExchangeLeaves.Get(),
-                                      results, m.Bias.Get(), m.Scale, static_cast<uint32_t>(docCount), m.ExchangeRounds,
-                                      m.LayoutBuckets * dev::kDocsPerBlock, 0};
+            TEvalExchangeArgs args = m.ExchangeArgs(docCount, results);
+            args.Bins = bins;
             LaunchModuleWithEnd(m.ExchangeFunction, static_cast<uint32_t>(blocks), 1, 64 * kExchangeWaves, s, TakeEnd(end), args);
             return;
         }
@@ -3910,6 +3985,10 @@ static void AwaitSmallBatch(THipEvaluator::TImpl& m, const THipEvaluator::TImpl:
 int THipEvaluator::FusedLayoutFor(int layout, size_t stride, size_t docCount, size_t treeStart, size_t treeEnd, bool anyBatchSize) const {
     const TImpl& m = *Impl;
     const int layoutIndex = layout == TFeatureBatch::FlatRows ? 0 : layout == TFeatureBatch::SplitRows ? 1 : layout == TFeatureBatch::FlatColumns ? 2 : -1;
+    if (layoutIndex == 0 && !anyBatchSize && treeStart == 0 && treeEnd == TreeCount && stride < (size_t(1) << 20) &&
+        m.TakesFusedExchangeKernel(docCount)) {
+        return kFusedExchange;
+    }
     if (layoutIndex < 0 || !m.Fused[layoutIndex] || docCount == 0 || treeStart != 0 || treeEnd != TreeCount ||
         docCount >= (size_t(1) << 29) || stride >= (size_t(1) << (layoutIndex == 2 ? 30 : 20))) {
         return -1;
@@ -3930,6 +4009,16 @@ bool THipEvaluator::EvalFusedDevice(const TFeatureBatch& batch, size_t docCount,
     const int layoutIndex = FusedLayoutFor(batch.Layout, batch.Stride, docCount, treeStart, treeEnd, anyBatchSize);
     if (layoutIndex < 0) {
         return false;
+    }
+    if (layoutIndex == kFusedExchange) {
+        CBAMD_ENSURE(results != nullptr, "results pointer is null");
+        CheckBatch(batch, docCount);
+        TFusedExchangeArgs args = {m.ExchangeArgs(docCount, results), batch.Floats, m.FusedExchangeTiles.Get(),
+                                   static_cast<uint32_t>(batch.Stride * sizeof(float)), m.FusedExchangeTileCount, m.FusedExchangeOneHot.Get()};
+        args.Walk.WaveTable = m.FusedExchangeWaves.Get();
+        const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
+        LaunchModuleWithEnd(m.FusedExchangeFunction, static_cast<uint32_t>(blocks), 1, 64 * kExchangeWaves, m.Pick(stream), TakeEnd(end), args);
+        return true;
     }
     const TImpl::TFused& f = *m.Fused[layoutIndex];
     CBAMD_ENSURE(results != nullptr, "results pointer is null");
@@ -3990,7 +4079,7 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
     const TImpl& m = *Impl;
     // whole-model calls only: a call for a range of the trees may take other kernels
     if (const int fused = FusedLayoutFor(layout, stride, docCount, 0, TreeCount, false); fused >= 0) {
-        return std::string("fused=") + m.Fused[fused]->Name;
+        return "fused=" + (fused == kFusedExchange ? m.FusedExchangeName : m.Fused[fused]->Name);
     }
     if (TakesSmallBatchKernel(docCount, 0, TreeCount)) {
         const bool few = m.TakesFewDocumentsKernel(docCount);

@@ -12,8 +12,12 @@ int main(int argc, char** argv) {
     }
     std::ifstream in(argv[1]);
     size_t treeCount = 0;
-    uint32_t buckets = 0, maxDepth = 0, six = 0;
-    in >> treeCount >> buckets >> maxDepth >> six;
+    uint32_t buckets = 0, maxDepth = 0, six = 0, tiled = 0;
+    in >> treeCount >> buckets >> maxDepth >> six >> tiled;
+    std::vector<uint32_t> columnOf(tiled ? buckets : 0);
+    for (uint32_t& column : columnOf) {
+        in >> column;
+    }
     std::vector<cbamd::TExchangeTree> trees(treeCount);
     std::vector<std::vector<double>> leaves(treeCount);
     for (size_t t = 0; t < treeCount; ++t) {
@@ -31,16 +35,34 @@ int main(int argc, char** argv) {
         }
         trees[t].Leaves = leaves[t].data();
     }
+    std::vector<cbamd::TExchangeColumn> columns;
+    std::vector<uint32_t> pieces(tiled * cbamd::kExchangeTilePieces);
+    for (uint32_t& piece : pieces) {
+        in >> piece;
+    }
+    for (size_t c = 0; c < tiled * cbamd::kExchangeTileColumns; ++c) {
+        cbamd::TExchangeColumn column;
+        size_t values = 0;
+        in >> column.Used >> column.OneHot >> column.RowByte >> values;
+        column.Values.resize(values);
+        for (uint32_t& v : column.Values) {
+            in >> v;
+        }
+        if (column.Used && !column.OneHot) {
+            cbamd::MakeExchangeGrid(six != 0, &column);
+        }
+        columns.push_back(column);
+    }
     if (!in) {
         return 3;
     }
     cbamd::TExchangePlan plan;
-    if (!cbamd::BuildExchangePlan(trees, buckets, maxDepth, six != 0, &plan)) {
+    if (!cbamd::BuildExchangePlan(trees, buckets, maxDepth, six != 0, columnOf, &plan)) {
         std::printf("refused\n");
         return 0;
     }
     std::printf("%u\n", plan.Rounds);
-    for (const auto* table : {&plan.WaveTable, &plan.Records, &plan.ExtraRows}) {
+    for (const auto* table : {tiled ? &plan.FusedWaveTable : &plan.WaveTable, &plan.Records, &plan.ExtraRows}) {
         for (uint32_t v : *table) {
             std::printf("%u ", v);
         }
@@ -50,5 +72,14 @@ int main(int argc, char** argv) {
         std::printf("%.17g ", v);
     }
     std::printf("\n");
+    std::vector<uint32_t> table, oneHot;
+    if (tiled != 0 && cbamd::BuildExchangeTiles(columns, pieces, six != 0, &table, &oneHot)) {
+        for (const auto* t : {&table, &oneHot}) {
+            for (uint32_t v : *t) {
+                std::printf("%u ", v);
+            }
+            std::printf("\n");
+        }
+    }
     return 0;
 }

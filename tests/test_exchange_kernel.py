@@ -29,20 +29,28 @@ def planner(tmp_path_factory):
     return out
 
 
-def _plan(planner, path, trees, buckets, max_depth, six):
+def _plan(planner, path, trees, buckets, max_depth, six, tiles=None):
+    """tiles: (column of every bucket, byte offsets of the pieces, the columns) for a fused kernel."""
     with open(path, "w") as f:
-        f.write("%d %d %d %d\n" % (len(trees), buckets, max_depth, six))
+        f.write("%d %d %d %d %d\n" % (len(trees), buckets, max_depth, six, len(tiles[1]) // 16 if tiles else 0))
+        if tiles:
+            f.write(" ".join(map(str, tiles[0])) + "\n")
         for levels, leaves in trees:
             f.write("%d\n" % len(levels))
             for bucket, split, one_hot in levels:
                 add, xor = (1, ~split & 0x7f) if one_hot else (128 - split, 0)
                 f.write("%d %d %d %d %g\n" % (bucket, add, xor, one_hot, abs(split / 60.0 - 0.5)))
             f.write(" ".join("%.17g" % v for v in leaves) + "\n")
+        if tiles:
+            f.write(" ".join(map(str, tiles[1])) + "\n")
+            for used, one_hot, row_byte, values in tiles[2]:
+                f.write("%d %d %d %d %s\n" % (used, one_hot, row_byte, len(values), " ".join(map(str, values))))
     lines = subprocess.check_output([planner, path], text=True).split("\n")
     if lines[0] == "refused":
         return None
     tables = [np.array(line.split(), dtype=np.uint32) for line in lines[1:4]]
-    return int(lines[0]), tables[0], tables[1], tables[2], np.array(lines[4].split(), dtype=np.float64)
+    plan = (int(lines[0]), tables[0], tables[1], tables[2], np.array(lines[4].split(), dtype=np.float64))
+    return plan + tuple(np.array(line.split(), dtype=np.uint32) for line in lines[5:7]) if tiles else plan
 
 
 def _model(rng, tree_count, buckets, depths, bins_limit, one_hot_share, skew=False):
@@ -129,7 +137,7 @@ class _Wave:
     def vector(self, text, first=False):
         if re.match(r"v\d+$", text):
             r = int(text[1:])
-            if first and self.indexed:
+            if first and self.indexed and self.m0 >> 12 & 1:
                 r += self.m0 & 0xff
                 assert 64 <= r < 128
             return self.v[r]
@@ -211,7 +219,13 @@ class _Wave:
     def op_s_mov_b32(self, args):
         self.set_scalar(args[0], self.scalar(args[1]))
 
+    def op_s_cselect_b32(self, args):
+        self.set_scalar(args[0], self.scalar(args[1] if self.scc else args[2]))
+
     def op_s_mov_b64(self, args):
+        if args[0] == "exec":
+            self.exec = (1 << 64) - 1 if args[1] == "-1" else self.pair(args[1])
+            return
         to, source = (int(re.match(r"s\[(\d+):", a).group(1)) for a in args)
         self.s[to:to + 2] = self.s[source:source + 2]
 
@@ -266,6 +280,75 @@ class _Wave:
         if self.scc:
             self.pc = self.labels[args[0]]
 
+    def op_s_load_dword(self, args):
+        self._s_load(args, 1)
+
+    def op_s_min_u32(self, args):
+        self.set_scalar(args[0], min(self.scalar(args[1]), self.scalar(args[2])))
+
+    def op_s_cmp_lt_u32(self, args):
+        self.scc = int(self.scalar(args[0]) < self.scalar(args[1]))
+
+    def op_s_cmp_ge_u32(self, args):
+        self.scc = int(self.scalar(args[0]) >= self.scalar(args[1]))
+
+    def op_v_subrev_u32(self, args):
+        self._set(args, self.vector(args[2]) - self.vector(args[1], True))
+
+    def op_v_min_u32(self, args):
+        self._set(args, np.minimum(self.vector(args[1], True), self.vector(args[2])))
+
+    def op_v_or_b32(self, args):
+        self._set(args, self.vector(args[1], True) | self.vector(args[2]))
+
+    def op_v_sub_u32(self, args):
+        self._set(args, self.vector(args[1], True) - self.vector(args[2]))
+
+    def op_v_mul_u32_u24(self, args):
+        self._set(args, self.vector(args[1], True) * self.vector(args[2]))
+
+    op_v_mul_lo_u32 = op_v_mul_u32_u24
+
+    def op_v_lshl_add_u32(self, args):
+        self._set(args, (self.vector(args[1], True) << self.vector(args[2])) + self.vector(args[3]))
+
+    def op_v_lshl_or_b32(self, args):
+        self._set(args, (self.vector(args[1], True) << self.vector(args[2])) | self.vector(args[3]))
+
+    def op_v_lshrrev_b32_sdwa(self, args):
+        # the low byte of the result into one byte of the destination, the others stay
+        words = args[2].split()
+        byte = int(re.match(r"dst_sel:BYTE_(\d)", words[1]).group(1))
+        assert words[2:] == ["dst_unused:UNUSED_PRESERVE", "src0_sel:DWORD", "src1_sel:DWORD"]
+        value = (self.vector(words[0]) >> self.vector(args[1])) & np.uint32(255)
+        register = int(args[0][1:])
+        self.v[register] = self.v[register] & np.uint32(~(255 << 8 * byte) & 0xffffffff) | value << np.uint32(8 * byte)
+
+    def _floats(self, text):
+        return np.asarray(self.vector(text), dtype=np.uint32).view(np.float32)
+
+    def op_v_fma_f32(self, args):
+        last, _, clamp = args[3].partition(" ")
+        with np.errstate(all="ignore"):
+            a, b, c = (self._floats(x).astype(np.float64) for x in (args[1], args[2], last))
+            value = (a * b + c).astype(np.float32)
+            if clamp:
+                value = np.where(value > 0, np.minimum(value, np.float32(1)), np.float32(0)).astype(np.float32)
+        self._set(args, value.view(np.uint32))
+
+    def op_v_cmp_lt_f32(self, args):
+        assert args[0] == "vcc"
+        with np.errstate(all="ignore"):
+            self.vcc = sum(1 << int(i) for i in np.flatnonzero(self._floats(args[1]) < self._floats(args[2])))
+
+    def op_v_cmp_eq_u32(self, args):
+        self.vcc = sum(1 << int(i) for i in np.flatnonzero(self.vector(args[1]) == self.vector(args[2])))
+
+    def op_v_cndmask_b32(self, args):
+        assert args[3] == "vcc"
+        taken = np.array([self.vcc >> lane & 1 for lane in range(64)], dtype=bool)
+        self._set(args, np.where(taken, self.vector(args[2]), self.vector(args[1])))
+
     def op_s_cbranch_scc0(self, args):
         if not self.scc:
             self.pc = self.labels[args[0]]
@@ -292,7 +375,12 @@ class _Wave:
         self.v[int(args[0][1:])] = value
 
     def op_v_mov_b32(self, args):
-        self._set(args, self.vector(args[1], True))
+        if self.indexed and self.m0 >> 12 & 8:       # the destination is relative
+            register = int(args[0][1:]) + (self.m0 & 0xff)
+            assert 64 <= register < 128
+            self.v[register] = self.vector(args[1])
+        else:
+            self._set(args, self.vector(args[1], True))
 
     def op_v_and_b32(self, args):
         self._set(args, self.vector(args[1], True) & self.vector(args[2]))
@@ -331,6 +419,14 @@ class _Wave:
     def op_v_mul_f64(self, args):
         self._set_double(args, self.double(args[1]) * self.double(args[2]))
 
+    def op_v_cmp_ge_u32(self, args):
+        first = int(re.match(r"s\[(\d+):", args[0]).group(1))
+        mask = sum(1 << int(i) for i in np.flatnonzero(self.vector(args[1]) >= self.vector(args[2])))
+        self.s[first:first + 2] = [mask & 0xffffffff, mask >> 32]
+
+    def op_v_bfe_u32(self, args):
+        self._set(args, self.vector(args[1], True) >> self.vector(args[2]) & np.uint32((1 << int(args[3])) - 1))
+
     def op_v_cmp_gt_u32(self, args):
         hit = self.vector(args[1]) > self.vector(args[2])
         self.vcc = sum(1 << int(i) for i in np.flatnonzero(hit))
@@ -344,6 +440,7 @@ class _Wave:
     @staticmethod
     def _offset(args):
         found = re.search(r"offset:(\d+)", " ".join(args))
+        assert not found or int(found.group(1)) < 65536
         return int(found.group(1)) if found else 0
 
     def _ds_read(self, args, words):
@@ -362,6 +459,18 @@ class _Wave:
     def op_ds_read_b64(self, args):
         self._ds_read(args, 2)
 
+    def op_ds_read_b128(self, args):
+        self._ds_read(args, 4)
+
+    def op_ds_read_u8(self, args):
+        register = int(args[0][1:])
+        address = self.vector(args[1].split()[0]).astype(np.int64) + self._offset(args)
+        data = self.lds.data[self._lds(address, 1)][:, 0].astype(np.uint32)
+
+        def finish():
+            self.v[register] = data
+        self.issue(self.lgkm, {("v", register)}, finish)
+
     def _ds_write(self, args, words):
         first = int(re.match(r"v\[?(\d+)", args[1]).group(1))
         lanes = [lane for lane in range(64) if self.exec >> lane & 1]
@@ -379,8 +488,8 @@ class _Wave:
 
     # the lane's dword at M0
     def op_ds_read_addtid_b32(self, args):
-        register = int(args[0][1:])
-        address = (self.m0 & 0xffff) + 4 * np.arange(64)
+        register = int(args[0].split()[0][1:])
+        address = (self.m0 & 0xffff) + self._offset(args) + 4 * np.arange(64)
         data = self.lds.data[self._lds(address, 4)].copy().view(np.uint32)[:, 0]
 
         def finish():
@@ -388,14 +497,27 @@ class _Wave:
         self.issue(self.lgkm, {("v", register)}, finish)
 
     def op_ds_write_addtid_b32(self, args):
-        address = (self.m0 & 0xffff) + 4 * np.arange(64)
-        self.lds.data[self._lds(address, 4)] = self.v[int(args[0][1:])].copy().view(np.uint8).reshape(64, 4)
+        address = (self.m0 & 0xffff) + self._offset(args) + 4 * np.arange(64)
+        self.lds.data[self._lds(address, 4)] = self.v[int(args[0].split()[0][1:])].copy().view(np.uint8).reshape(64, 4)
         self.issue(self.lgkm, set(), lambda: None)
 
     # -- global memory
+    def op_global_load_dwordx4(self, args):
+        first = int(re.match(r"v\[(\d+):", args[0]).group(1))
+        base = self.pair(args[2].split()[0]) + self._offset(args)
+        values = self.v[first:first + 4].copy()
+        for lane in range(64):
+            if self.exec >> lane & 1:
+                data, at = self.memory.at(base + int(self.vector(args[1])[lane]), 16)
+                values[:, lane] = data[at:at + 16].copy().view(np.uint32)
+
+        def finish():
+            self.v[first:first + 4] = values
+        self.issue(self.vm, {("v", r) for r in range(first, first + 4)}, finish)
+
     def op_global_load_dword(self, args):
         register = int(args[0][1:])
-        base = self.pair(args[2])
+        base = self.pair(args[2].split()[0]) + self._offset(args)
         values = []
         for lane in range(64):
             data, at = self.memory.at(base + int(self.vector(args[1])[lane]), 4)
@@ -404,19 +526,6 @@ class _Wave:
         def finish():
             self.v[register] = np.array(values, dtype=np.uint32)
         self.issue(self.vm, {("v", register)}, finish)
-
-    def op_global_load_dwordx2(self, args):
-        first = int(re.match(r"v\[(\d+):", args[0]).group(1))
-        base = self.pair(args[2])
-        values = []
-        for lane in range(64):
-            data, at = self.memory.at(base + int(self.vector(args[1])[lane]), 8)
-            values.append(data[at:at + 8].copy().view(np.uint32))
-        values = np.array(values)
-
-        def finish():
-            self.v[first], self.v[first + 1] = values[:, 0], values[:, 1]
-        self.issue(self.vm, {("v", first), ("v", first + 1)}, finish)
 
     def op_global_load_lds_dwordx4(self, args):
         base, offset = self.pair(args[1].split()[0]), self._offset(args)
@@ -451,8 +560,8 @@ class _Lds:
         self.flying = np.zeros(size, dtype=bool)
 
 
-def _kernel(gen, depth, six):
-    text, _ = gen.gen_kernel(depth, six)
+def _kernel(gen, depth, six, fused=False):
+    text, _ = gen.gen_kernel(depth, six, fused)
     code, labels = [], {}
     for line in text.split("\n"):
         line = line.strip()
@@ -467,8 +576,9 @@ def _kernel(gen, depth, six):
     return code, labels
 
 
-def _run(gen, plan, bins, doc_count, buckets, depth, six, scale, bias, rng):
-    rounds, wave_table, records, extra_rows, leaves = plan
+def _run(gen, plan, bins, doc_count, buckets, depth, six, scale, bias, rng, rows=None):
+    """rows: the documents for a fused kernel, whose bins nobody gives it."""
+    rounds, wave_table, records, extra_rows, leaves = plan[:5]
     blocks = bins.shape[0] // 256
     # [block][bucket][lane][j] with document = block * 256 + j * 64 + lane
     tiled = np.ascontiguousarray(bins.reshape(blocks, 4, 64, buckets).transpose(0, 3, 2, 1)).reshape(-1).view(np.uint8)
@@ -476,14 +586,19 @@ def _run(gen, plan, bins, doc_count, buckets, depth, six, scale, bias, rng):
     out = np.full(doc_count, np.nan)
     addresses = [memory.add(np.ascontiguousarray(a).view(np.uint8)) for a in
                  (tiled, wave_table, records, extra_rows, leaves, out, np.array([bias]))]
-    kernarg = np.zeros(80, dtype=np.uint8)
+    kernarg = np.zeros(112, dtype=np.uint8)
     kernarg[:56] = np.array(addresses, dtype=np.uint64).view(np.uint8)
     kernarg[56:64] = np.array([scale]).view(np.uint8)
     kernarg[64:80] = np.array([doc_count, rounds, buckets * 256, 0], dtype=np.uint32).view(np.uint8)
+    if rows is not None:
+        fused = [memory.add(np.ascontiguousarray(a).reshape(-1).view(np.uint8)) for a in (rows, plan[5], plan[6])]
+        kernarg[80:96] = np.array(fused[:2], dtype=np.uint64).view(np.uint8)
+        kernarg[96:104] = np.array([rows.shape[1] * 4, (len(plan[5]) * 4 - gen.TILE_HEADER) // gen.image_bytes()], dtype=np.uint32).view(np.uint8)
+        kernarg[104:112] = np.array(fused[2:], dtype=np.uint64).view(np.uint8)
     where = memory.add(kernarg)
-    kernel = _kernel(gen, depth, six)
+    kernel = _kernel(gen, depth, six, rows is not None)
     for block in range(blocks):
-        lds = _Lds(gen.lds_bytes(depth), rng)
+        lds = _Lds(gen.lds_bytes(depth, six, rows is not None), rng)
         waves = [_Wave(kernel, memory, lds, where, block, w) for w in range(16)]
         running = list(range(16))
         while running:
@@ -522,6 +637,74 @@ def test_kernel_on_planned_tables(planner, tmp_path, case):
         assert plan is not None
         got = _run(gen, plan, bins, docs, buckets, depth, six, 0.5, 0.25, rng)
         np.testing.assert_array_equal(got, _expected(trees, bins)[:docs] * 0.5 + 0.25)
+
+
+# trees, columns, one-hot columns, depths, borders up to, documents
+FUSED_CASES = [
+    (40, 70, 0, [8], 60, 300),          # a last tile of two pieces, and documents behind the last row
+    (33, 1016, 16, [7, 8], 60, 256),    # sixteen tiles, one-hot columns in the last ones
+    (48, 200, 21, [6], 63, 41),         # more one-hot columns in a tile than waves
+    (35, 130, 5, [8], 127, 257),        # seven bits
+    (16, 66, 3, [5, 6], 120, 1),
+]
+
+
+@pytest.mark.parametrize("case", FUSED_CASES, ids=[str(c[:3]) for c in FUSED_CASES])
+def test_fused_kernel_on_rows(planner, tmp_path, case):
+    """A column in three is not used, some pieces are not: a piece that would leave the row is moved back over its neighbour. The
+    documents hold borders, values next to them, infinities, NaN, denormals and hashes of no category."""
+    tree_count, columns, one_hot, depths, limit, docs = case
+    gen = _generator()
+    rng = np.random.default_rng(tree_count * 1000 + columns)
+    used = np.flatnonzero(rng.random(columns) < (0.97 if columns > 900 else 0.7))
+    is_hot = np.zeros(columns, dtype=bool)
+    is_hot[rng.permutation(used[used > columns // 2] if columns > 900 else used)[:one_hot]] = True
+    pieces, column_of, covered = [], {}, -1
+    for c in used:
+        if c > covered:
+            start = min(c & ~3, columns - 4)
+            pieces.append(start)
+            covered = start + 3
+        column_of[c] = (len(pieces) - 1) // 16 * 64 + (len(pieces) - 1) % 16 * 4 + c - pieces[-1]
+    pieces += [0] * (-len(pieces) % 16)
+    assert len(pieces) <= 256
+    rows = rng.normal(size=(docs, columns)).astype(np.float32)
+    table = [(0, 0, 0, [])] * (4 * len(pieces))
+    bins = np.zeros(((docs + 255) // 256 * 256, len(used)), dtype=np.uint8)
+    six = limit <= 63
+    count = np.zeros(len(used), dtype=int)
+    for b, c in enumerate(used):
+        n = count[b] = int(rng.integers(1, limit + 1))
+        if is_hot[c]:
+            n = count[b] = min(n, 20)
+            values = rng.choice(2**31, size=n, replace=False).astype(np.uint32)
+            hashes = np.append(values, np.uint32(12345))[rng.integers(0, n + 1, size=docs)]
+            rows[:, c] = hashes.view(np.float32)
+            bins[:docs, b] = ((hashes[:, None] == values) * np.arange(1, n + 1)).max(axis=1)
+            table[column_of[c]] = (1, 1, 4 * c, values)
+            continue
+        # (normal values of a float's every size in a column or two, else at most fifteen borders may share a cell)
+        borders = np.unique(rng.normal(size=n).astype(np.float32)) if c % 3 else np.linspace(-1, 1, n).astype(np.float32)
+        if c % 7 == 0:
+            borders = np.float32([-3e38, 1e-40, 1.0, 3e38])
+        count[b] = len(borders)
+        special = np.concatenate([borders, np.nextafter(borders, np.float32(9)), [np.inf, -np.inf, np.nan, 1e-40, 3e38, -3e38]]).astype(np.float32)
+        at = rng.random(docs) < 0.3
+        rows[at, c] = rng.choice(special, size=at.sum())
+        with np.errstate(invalid="ignore"):
+            bins[:docs, b] = (rows[:, c:c + 1] > borders).sum(axis=1)
+        table[column_of[c]] = (1, 0, 0, borders.view(np.uint32))
+    depth = 6 if max(depths) <= 6 else 8
+    trees = []
+    for t in range(tree_count):
+        levels = [(int(b), int(rng.integers(1, count[b] + 1)), bool(is_hot[used[b]]))
+                  for b in rng.integers(0, len(used), size=int(rng.choice(depths)))]
+        trees.append((levels, rng.normal(size=1 << len(levels))))
+    tiles = ([column_of[c] for c in used], [4 * p for p in pieces], table)
+    plan = _plan(planner, str(tmp_path / "model.txt"), trees, len(used), depth, six, tiles)
+    assert plan is not None and len(plan) == 7
+    got = _run(gen, plan, bins, docs, len(used), depth, six, 0.5, 0.25, rng, rows=rows)
+    np.testing.assert_array_equal(got, _expected(trees, bins)[:docs] * 0.5 + 0.25)
 
 
 def test_plan_refuses_more_buckets_than_registers(planner, tmp_path):

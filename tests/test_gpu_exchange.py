@@ -1,5 +1,6 @@
 """The exchange kernels (wide one-dimensional models, most batches of more than 32768 documents) add a document's trees as the
-pair-tile kernel does: the same bits from both, and the oracle's values within the usual tolerance."""
+pair-tile kernel does, from bins or (the fused form) from flat rows: the same bits from all, and the oracle's values within the
+usual tolerance."""
 import numpy as np
 import pytest
 
@@ -13,8 +14,9 @@ pytestmark = pytest.mark.gpu
 
 def _evaluators(model, monkeypatch):
     out = []
-    for switch in ("1", "0"):
-        monkeypatch.setenv("CATBOOST_AMD_EXCHANGE", switch)
+    for fused, exchange in (("1", "1"), ("0", "1"), ("1", "0")):
+        monkeypatch.setenv("CATBOOST_AMD_FUSED", fused)
+        monkeypatch.setenv("CATBOOST_AMD_EXCHANGE", exchange)
         g = cb.ModelCalcer()
         g.load_from_dict(model)
         g.enable_gpu_evaluation(0)
@@ -38,26 +40,41 @@ def test_exchange_kernel_gives_the_pair_tile_kernels_bits(buckets, cats, trees, 
 
     rng = np.random.default_rng(buckets + trees)
     model, hashes = _model_of_buckets(rng, buckets, cats, trees, depth, 1, first)
-    exchange, pair = _evaluators(model, monkeypatch)
+    fused, exchange, pair = _evaluators(model, monkeypatch)
     docs = 98_561                               # a workgroup per CU, and a generation of half as many behind them
     x = rng.normal(size=(docs, buckets)).astype(np.float32)
+    borders = np.float32([f["borders"][len(f["borders"]) // 2] if len(f["borders"]) else 0 for f in model["float_features"]])
+    for value in (np.nan, np.inf, -np.inf, borders, np.nextafter(borders, np.float32(9))):
+        x[:, :buckets - cats] = np.where(rng.random((docs, 1)) < 0.1, value, x[:, :buckets - cats])
     for i in range(cats):
         x[:, buckets - cats + i] = rng.choice(hashes[i], size=docs).view(np.float32)
     flat = torch.from_numpy(x).to("cuda:0")
     results = {}
-    for name, g in (("exchange", exchange), ("pair", pair)):
+    for name, g in (("fused", fused), ("exchange", exchange), ("pair", pair)):
         ev = g.evaluator()
         feats = ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), flat.shape[1])
-        for n in (32768, 32769, 40_001, docs):
-            wanted = kernel if name == "exchange" and n > 32768 else "EvalObliviousPairTileKernel"
-            assert ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, n)["evaluate"] == wanted
+        for n in (32768, 32769, 46_081, docs):
+            kernels = ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, n)
+            if name == "fused" and n > 46_080:          # seven tenths of the CUs have a workgroup
+                assert kernels == {"fused": kernel.replace("eval", "fused")}
+            else:
+                assert kernels["evaluate"] == (kernel if name != "pair" and n > 32768 else "EvalObliviousPairTileKernel")
             out = torch.full((n + 1,), -3.0, dtype=torch.float64, device="cuda:0")
             torch.cuda.synchronize()
             ev.eval_data(feats, n, out.data_ptr())
             assert out[n].item() == -3.0
             results[name, n] = out[:n].clone()
-    for n in (32768, 32769, 40_001, docs):
+    for n in (32768, 32769, 46_081, docs):
         assert torch.equal(results["exchange", n], results["pair", n]), n
+        assert torch.equal(results["fused", n], results["pair", n]), n
+    # rows further apart than the model's features, and the last document's row at the end of its memory
+    wide = torch.full((docs * (buckets + 5) - 5,), float("nan"), device="cuda:0")
+    torch.as_strided(wide, (docs, buckets), (buckets + 5, 1)).copy_(flat)
+    out = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    ev = fused.evaluator()
+    ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, wide.data_ptr(), buckets + 5), docs, out.data_ptr())
+    assert torch.equal(out, results["pair", docs])
     sample = rng.choice(docs, size=300, replace=False)
     np.testing.assert_allclose(results["exchange", docs].cpu().numpy()[sample], OracleModel(model).calc(x[sample]), rtol=1e-9, atol=1e-12)
     # a range of the trees takes the pair-tile kernel, the whole model the exchange kernel
