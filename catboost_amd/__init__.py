@@ -19,8 +19,8 @@ LAYOUT_FLAT_ROWS, LAYOUT_FLAT_COLUMNS, LAYOUT_SPLIT_ROWS = range(3)
 
 _lib = None
 
-c_float_pp = ctypes.POINTER(ctypes.POINTER(ctypes.c_float))
-c_int_pp = ctypes.POINTER(ctypes.POINTER(ctypes.c_int))
+# pointers to rows and to results: an address (_address), or any ctypes pointer or array
+c_float_pp = c_int_pp = ctypes.c_void_p
 c_char_ppp = ctypes.POINTER(ctypes.POINTER(ctypes.c_char_p))
 
 
@@ -98,7 +98,7 @@ def load_library():
         except ImportError:
             pass
     lib = ctypes.CDLL(LIB_PATH)
-    vp, sz, dp = ctypes.c_void_p, ctypes.c_size_t, ctypes.POINTER(ctypes.c_double)
+    vp, sz, dp = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p
     sig = {
         "ModelCalcerCreate": (vp, []),
         "ModelCalcerDelete": (None, [vp]),
@@ -205,12 +205,31 @@ def integer_cat_feature_hash(v):
     return int(load_library().GetIntegerCatFeatureHash(int(v)))
 
 
-def _row_pointers(matrix, ctype):
-    """Array of per-row pointers into a C-contiguous 2-D numpy array."""
+def _address(array):
+    """Address of a C-contiguous numpy array's first element. (A call for one row takes some 18 us, of which `array.ctypes` for its
+    row, its row pointer and its result took 4.)"""
+    try:
+        return ctypes.addressof(ctypes.c_char.from_buffer(array))
+    except (TypeError, ValueError, BufferError):  # read-only or empty
+        return array.ctypes.data
+
+
+def _row_pointers(matrix):
+    """Array of per-row pointers into a C-contiguous 2-D numpy array, as an argument of a call."""
     n = matrix.shape[0]
-    addresses = matrix.ctypes.data + np.arange(max(n, 1), dtype=np.uint64) * np.uint64(matrix.strides[0])
-    # the ctypes array shares (and keeps alive) the numpy buffer of addresses
-    return (ctypes.POINTER(ctype) * max(n, 1)).from_buffer(addresses)
+    first = _address(matrix)
+    if n <= 1:
+        return _OneRow(first)
+    stride = matrix.strides[0]
+    if stride == 0 or first + n * stride >= 1 << 63:
+        addresses = np.full(n, first, dtype=np.uint64)
+    else:
+        addresses = np.arange(first, first + n * stride, stride, dtype=np.uint64)
+    # the argument keeps the numpy buffer of addresses alive
+    return ctypes.byref(ctypes.c_char.from_buffer(addresses))
+
+
+_OneRow = ctypes.c_void_p * 1
 
 
 def fast_exp(values, chunk=None):
@@ -650,7 +669,7 @@ class ModelCalcer:
 
     @staticmethod
     def _dp(a):
-        return a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+        return _address(a)
 
     def calc_flat(self, features, tree_start=None, tree_end=None, result_size=None):
         """CalcModelPredictionFlat[Staged]: features[doc][flat feature index]."""
@@ -659,7 +678,7 @@ class ModelCalcer:
             x = x.reshape(1, -1)
         n = x.shape[0]
         out = self._result(n) if result_size is None else np.zeros(result_size)
-        rows = _row_pointers(x, ctypes.c_float)
+        rows = _row_pointers(x)
         if tree_start is None and tree_end is None:
             _check(self._lib.CalcModelPredictionFlat(self._h, n, rows, x.shape[1], self._dp(out), out.size))
         else:
@@ -681,7 +700,7 @@ class ModelCalcer:
         x = np.ascontiguousarray(transposed_features, dtype=np.float32)
         n = x.shape[1]
         out = self._result(n)
-        cols = _row_pointers(x, ctypes.c_float)
+        cols = _row_pointers(x)
         if tree_start is None and tree_end is None:
             _check(self._lib.CalcModelPredictionFlatTransposed(self._h, n, cols, x.shape[0], self._dp(out), out.size))
         else:
@@ -706,7 +725,7 @@ class ModelCalcer:
             keep.append(row)
             cat_rows[i] = ctypes.cast(row, ctypes.POINTER(ctypes.c_char_p))
         out = self._result(n)
-        rows = _row_pointers(x, ctypes.c_float)
+        rows = _row_pointers(x)
         if tree_start is None and tree_end is None:
             _check(self._lib.CalcModelPrediction(self._h, n, rows, x.shape[1], cat_rows, n_cat, self._dp(out), out.size))
         else:
@@ -731,8 +750,8 @@ class ModelCalcer:
         c = np.ascontiguousarray(hashed_cat_features, dtype=np.int32)
         n = max(x.shape[0] if x.ndim == 2 else 0, c.shape[0] if c.ndim == 2 else 0)
         out = self._result(n)
-        frows = _row_pointers(x, ctypes.c_float) if x.ndim == 2 and x.shape[1] else None
-        crows = _row_pointers(c, ctypes.c_int) if c.ndim == 2 and c.shape[1] else None
+        frows = _row_pointers(x) if x.ndim == 2 and x.shape[1] else None
+        crows = _row_pointers(c) if c.ndim == 2 and c.shape[1] else None
         _check(self._lib.CalcModelPredictionWithHashedCatFeatures(
             self._h, n, frows, x.shape[1] if x.ndim == 2 else 0, crows, c.shape[1] if c.ndim == 2 else 0,
             self._dp(out), out.size))
@@ -742,7 +761,7 @@ class ModelCalcer:
         x = np.ascontiguousarray(features, dtype=np.float32)
         n = x.shape[0]
         out = np.zeros(n)
-        _check(self._lib.PredictSpecificClassFlat(self._h, n, _row_pointers(x, ctypes.c_float), x.shape[1], class_id,
+        _check(self._lib.PredictSpecificClassFlat(self._h, n, _row_pointers(x), x.shape[1], class_id,
                                                   self._dp(out), n))
         return out
 
@@ -751,7 +770,7 @@ class ModelCalcer:
         n = x.shape[0]
         te = self.tree_count if tree_end is None else tree_end
         out = np.zeros(max(n * (te - tree_start), 1), dtype=np.uint32)
-        _check(self._lib.CbHipCalcLeafIndexesFlat(self._h, n, _row_pointers(x, ctypes.c_float), x.shape[1], tree_start,
+        _check(self._lib.CbHipCalcLeafIndexesFlat(self._h, n, _row_pointers(x), x.shape[1], tree_start,
                                                   te, out.ctypes.data, n * (te - tree_start)))
         return out[:n * (te - tree_start)].reshape(n, te - tree_start)
 
@@ -761,7 +780,7 @@ class ModelCalcer:
         n = x.shape[0]
         size = n * self.bucket_count
         out = np.zeros(max(size, 1), dtype=np.uint8)
-        _check(self._lib.CbHipQuantizeFlat(self._h, n, _row_pointers(x, ctypes.c_float), x.shape[1], out.ctypes.data, size))
+        _check(self._lib.CbHipQuantizeFlat(self._h, n, _row_pointers(x), x.shape[1], out.ctypes.data, size))
         return out[:size]
 
     def quantize_hashed(self, float_features, hashed_cat_features):
@@ -770,8 +789,8 @@ class ModelCalcer:
         n = max(x.shape[0], c.shape[0])
         size = n * self.bucket_count
         out = np.zeros(max(size, 1), dtype=np.uint8)
-        frows = _row_pointers(x, ctypes.c_float) if x.shape[1] else None
-        crows = _row_pointers(c, ctypes.c_int) if c.shape[1] else None
+        frows = _row_pointers(x) if x.shape[1] else None
+        crows = _row_pointers(c) if c.shape[1] else None
         _check(self._lib.CbHipQuantizeWithHashedCatFeatures(self._h, n, frows, x.shape[1], crows, c.shape[1],
                                                             out.ctypes.data, size))
         return out[:size]
