@@ -1697,6 +1697,7 @@ struct THipEvaluator::TImpl {
     bool SmallUsable = false;
     uint32_t SmallCellCount = 0;
     TDeviceVec<uint32_t> SmallTable;
+    TDeviceVec<double> SmallLeaves;    // the leaf values, a tree's in the order of its levels in those rows
     size_t SmallCellsAt = 0, SmallFirstLeafAt = 0;
     // rows of the table without the null trees at its end, and those of a slice: a slice of the register kernels' (the whole
     // model when it is too short for slices), or a partial sum of SumOrder() with null trees up to the length of the longest
@@ -2187,6 +2188,15 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     }
     m.Bias.Upload(trees.Bias);
 
+    // How unevenly a level splits the documents, 0 (two halves) to 0.5, estimated from the rank of its border among the feature's borders
+    // (borders are quantiles of the training data). Kernels take a tree's levels in any order, leaf tables permuted to match.
+    const auto lopsidedness = [&](const TRepackedBin& rb) {
+        const uint32_t n = offsets[rb.FeatureIndex + 1] - offsets[rb.FeatureIndex];
+        const bool oneHot = (flags[rb.FeatureIndex] & dev::kBucketFlagOneHot) != 0 || rb.XorMask != 0;
+        const double share = oneHot ? 0.05 : static_cast<double>(rb.SplitIdx) / (n + 1.0);
+        return switches.LevelOrder ? std::fabs(share - 0.5) : 0.0;
+    };
+
     // The kernels that keep a tree's row in registers (two trees per wave on half a tile, one on a whole tile)
     // compare 7 bits. Their tile has a row per bucket, and two for a bucket of more than 127 values, which the
     // kernel makes while it copies the bins to LDS (tileMap): min(bin, 127) and max(bin - 127, 0) for a float
@@ -2385,11 +2395,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                                 for (int d = 0; d < trees.TreeSizes[t]; ++d) {
                                     const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + d];
                                     const TTileLevel level = tileLevelOf(rb);
-                                    // how evenly a level splits, estimated as for the register kernels (levelOrder below)
-                                    const uint32_t n = offsets[rb.FeatureIndex + 1] - offsets[rb.FeatureIndex];
-                                    const double share = level.IsXor ? 0.05 : static_cast<double>(rb.SplitIdx) / (n + 1.0);
-                                    levels[t].Levels.push_back({level.Row, level.Add & 0xffu, level.Xor, level.IsXor,
-                                                                switches.LevelOrder ? std::fabs(share - 0.5) : 0.0});
+                                    levels[t].Levels.push_back({level.Row, level.Add & 0xffu, level.Xor, level.IsXor, lopsidedness(rb)});
                                 }
                             }
                             // The fused form: the model's columns in pieces of four neighbouring ones, sixteen pieces a tile. A
@@ -2648,19 +2654,13 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         // gathers of a wave meet in the LDS banks that the low bits of the leaf indexes choose; lanes with the
         // same index share one access, lanes that differ only in high bits wait for each other. So the levels
         // that split the documents most evenly go to the low bits and the lopsided ones, on which most lanes
-        // agree, to the high bits: fewer lanes of a bank then differ. How evenly a level splits is estimated
-        // from the rank of its border among the feature's borders (borders are quantiles of the training data).
-        // The leaf tables are permuted to match; the sums and their order do not change.
+        // agree, to the high bits: fewer lanes of a bank then differ. The sums and their order do not change.
         std::vector<std::vector<int>> levelOrder(TreeCount);
         for (size_t t = 0; t < TreeCount; ++t) {
             const int depth = trees.TreeSizes[t];
             std::vector<std::pair<double, int>> lopsided;
             for (int d = 0; d < depth; ++d) {
-                const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + d];
-                const uint32_t n = offsets[rb.FeatureIndex + 1] - offsets[rb.FeatureIndex];
-                const bool oneHot = (flags[rb.FeatureIndex] & dev::kBucketFlagOneHot) != 0 || rb.XorMask != 0;
-                const double share = oneHot ? 0.05 : static_cast<double>(rb.SplitIdx) / (n + 1.0);
-                lopsided.emplace_back(switches.LevelOrder ? std::fabs(share - 0.5) : 0.0, d);
+                lopsided.emplace_back(lopsidedness(trees.RepackedBins[trees.TreeStartOffsets[t] + d]), d);
             }
             std::stable_sort(lopsided.begin(), lopsided.end(),
                              [](const auto& a, const auto& b) { return a.first < b.first; });
@@ -3078,6 +3078,11 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         order.resize(order.size() + dev::kSmallNullTrees, nullTree);
         std::vector<uint32_t> rows(order.size() * 16, 0);
         std::vector<uint32_t> first(order.size(), static_cast<uint32_t>(trees.LeafValues.size()));
+        // Sixteen documents of a tree read its leaf values together, from as many lines of 128 bytes as the high bits of their indexes
+        // differ: the lopsided levels, on which most documents agree, go there (6.9 lines -> 5.2 at depth 8). 1000 trees of depth 8,
+        // SmallBatchKernel for 4096 documents 12.5 -> 11.2 us, 16 384 38.7 -> 33.7; of depth 6 25.0 -> 24.0.
+        std::vector<double> smallLeaves(trees.LeafValues);
+        smallLeaves.resize(smallLeaves.size() + 256 * static_cast<size_t>(trees.ApproxDimension), 0.0);
         const uint32_t never = 0x7f800000u;
         bool usable = trees.LeafValues.size() < (size_t(1) << 32);
         for (size_t place = 0; place < order.size() && usable; ++place) {
@@ -3087,12 +3092,25 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             if (t < TreeCount) {
                 first[place] = static_cast<uint32_t>(trees.TreeFirstLeafOffsets[t]);
             }
+            std::vector<std::pair<double, int>> levels;
+            for (int d = 0; d < depth; ++d) {
+                levels.emplace_back(lopsidedness(trees.RepackedBins[trees.TreeStartOffsets[t] + d]), d);
+            }
+            std::stable_sort(levels.begin(), levels.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
+            for (size_t index = 0; t < TreeCount && index < (size_t(1) << depth); ++index) {
+                size_t leaf = 0;
+                for (int d = 0; d < depth; ++d) {
+                    leaf |= (index >> d & 1) << levels[d].second;
+                }
+                const size_t treeAt = trees.TreeFirstLeafOffsets[t], dim = static_cast<size_t>(m.Dim);
+                std::copy_n(trees.LeafValues.begin() + treeAt + leaf * dim, dim, smallLeaves.begin() + treeAt + index * dim);
+            }
             for (int d = 0; d < 8; ++d) {
                 row[8 + d] = never;
                 if (d >= depth) {
                     continue;
                 }
-                const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + d];
+                const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + levels[d].second];
                 const uint32_t b = rb.FeatureIndex, n = offsets[b + 1] - offsets[b];
                 // a damaged model may name a border that is not there: such a split stays with the kernels on bins
                 const bool oneHot = (flags[b] & dev::kBucketFlagOneHot) != 0;
@@ -3133,6 +3151,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             m.SmallFirstLeafAt = table.size();
             table.insert(table.end(), first.begin(), first.end());
             m.SmallTable.Upload(table);
+            m.SmallLeaves.Upload(smallLeaves);
             m.SmallCellCount = static_cast<uint32_t>(cells.size());
             m.SmallUsable = true;
         }
@@ -3910,7 +3929,7 @@ static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THos
     tab.Cells = reinterpret_cast<const dev::TSmallCell*>(m.SmallTable.Get() + m.SmallCellsAt);
     tab.TreeRows = m.SmallTable.Get();
     tab.FirstLeaf = m.SmallTable.Get() + m.SmallFirstLeafAt;
-    tab.Leaves = m.Leaves.Get();
+    tab.Leaves = m.SmallLeaves.Get();
     tab.Bias = m.Bias.Get();
     tab.Scale = m.Scale;
     tab.CellCount = m.SmallCellCount;
