@@ -628,8 +628,8 @@ constexpr size_t kMaxTileLdsBytes = 160 * 1024;
 
 // Batches of SmallBatchKernel and FewDocumentsKernel, in documents times passes over the dimensions; beyond, the binarize
 // and register kernels in slices of the trees are faster. Whole call, 1000 trees of depth 8 over 200 features: 8192
-// documents 31 us against 46 on those, 16384 48 against 49, 32768 82 against 62 (200 trees of depth 6: 26 against 33 and
-// 39 against 37). FewDocumentsKernel against SmallBatchKernel: 512 documents 18 against 21 us, 1024 24 against 21.
+// documents 29 us, 16384 42 against 38 on those (1000 trees of depth 6 32 against 33, 500 26 against 28, 300 of depth 4 25
+// against 26). FewDocumentsKernel against SmallBatchKernel: 512 documents 18 against 21 us, 1024 24 against 21.
 constexpr size_t kSmallBatchDocs = 16384;
 constexpr size_t kFewDocs = 640;
 // ... of host calls, whose features are at most so many bytes: more go through the pipeline of chunks
@@ -3899,7 +3899,7 @@ void THipEvaluator::EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCou
         LaunchModuleWithEnd(l.Function, grid, shares, 64 * l.Waves, s, nullptr, launchArgs);
     }
     const size_t count = docCount * m.Dim;
-    LaunchWithEnd(dev::CombineSlicesKernel, dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0, s, TakeEnd(end),
+    LaunchWithEnd(dev::CombineSlicesKernel, dim3(static_cast<uint32_t>((count + 63) / 64)), dim3(64), 0, s, TakeEnd(end),
                   static_cast<const double*>(partials), slices, count, m.Scale, m.Bias.Get(), m.Dim, results);
     HIP_CHECK(hipGetLastError());
 }

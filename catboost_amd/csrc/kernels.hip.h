@@ -729,16 +729,33 @@ __global__ __launch_bounds__(256) void EvalObliviousKernel(const uint32_t* __res
 
 // Small batches on the register-resident kernels: every slice of the trees left its raw sums in
 // partials[slice][count]; adds them in slice order and finishes like ApplyScaleAndBias. One thread per value.
-__global__ __launch_bounds__(256) void CombineSlicesKernel(const double* __restrict__ partials, uint32_t slices,
+// What bounds it: the latency of the loads. A loop of load and add had one in flight; now sixteen are (a whole turn past the last
+// slice reads that one again), in workgroups of one wave, which a batch of 17 000 documents spreads over every CU. Evaluation
+// (register kernel and this one) of 1000 trees of depth 6, 32 slices: 17 000 documents 22.2 -> 16.1 us, 100 000 48.2 -> 43.6; of 500 trees
+// and three dimensions 21.8 -> 17.6 and 41.5 -> 39.4. Workgroups of four waves 16.3 and 43.9, 19.2 and 40.5; 32 loads 16.0 and 43.7, 18.3
+// and 40.7.
+constexpr uint32_t kCombineInFlight = 16;
+
+__global__ __launch_bounds__(64) void CombineSlicesKernel(const double* __restrict__ partials, uint32_t slices,
                                                            size_t count, double scale, const double* __restrict__ bias,
                                                            int dim, double* __restrict__ out) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+    const size_t i = static_cast<size_t>(blockIdx.x) * 64 + threadIdx.x;
     if (i >= count) {
         return;
     }
     double sum = partials[i];
-    for (uint32_t s = 1; s < slices; ++s) {
-        sum = __dadd_rn(sum, partials[s * count + i]);
+    for (uint32_t first = 1; first < slices; first += kCombineInFlight) {
+        double part[kCombineInFlight];
+#pragma unroll
+        for (uint32_t k = 0; k < kCombineInFlight; ++k) {
+            part[k] = partials[min(first + k, slices - 1) * count + i];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kCombineInFlight; ++k) {
+            if (first + k < slices) {
+                sum = __dadd_rn(sum, part[k]);
+            }
+        }
     }
     out[i] = Finish(sum, scale, bias[i % static_cast<size_t>(dim)], true);
 }

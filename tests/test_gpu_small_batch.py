@@ -521,3 +521,32 @@ def test_which_wait_ends_calls_of_few_host_documents(monkeypatch, ticket, wait_u
     for docs in (17, 40):
         np.testing.assert_array_equal(m.calc_flat(x[:docs]), expected[:docs])
     assert flagged() - began == (50 if wait_us != "0" else 0)
+
+
+@pytest.mark.parametrize("trees,dim", [(64, 1), (513, 3), (544, 1), (545, 1), (1056, 2), (1057, 1)])
+def test_slices_are_added_in_order(trees, dim):
+    """The kernel that adds the slices keeps sixteen loads in flight: two slices, a whole turn of sixteen after the first
+    and one slice more, the same after two turns. The small batches' kernel adds the same slices in the same order."""
+    import torch
+
+    from tests.test_oracle import _random_flat_data, _random_oblivious
+
+    rng = np.random.default_rng(trees)
+    model, cat_values = _random_oblivious(rng, n_float=12, n_cat=1, trees=trees, max_depth=4, dim=dim, scale=0.5,
+                                          bias=rng.normal(size=dim))
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    docs = 16_641
+    assert "CombineSlicesKernel" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"]
+    assert "SmallBatchKernel" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, 4000)["evaluate"]
+    flat = torch.from_numpy(_random_flat_data(rng, model, cat_values, docs)).to("cuda:0")
+    out = torch.full((docs * dim + 8,), -3.0, dtype=torch.float64, device="cuda:0")
+    part = torch.zeros(4000 * dim, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), flat.shape[1]), docs, out.data_ptr())
+    for begin in (0, docs - 4000):
+        ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, flat[begin:].data_ptr(), flat.shape[1]), 4000, part.data_ptr())
+        assert torch.equal(part, out[begin * dim:(begin + 4000) * dim])
+    assert bool((out[docs * dim:] == -3.0).all())
