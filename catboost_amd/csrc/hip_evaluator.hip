@@ -4253,8 +4253,8 @@ void THipEvaluator::ApplyPredictionTypeDevice(int predictionType, size_t firstDo
     c.Mantissa = m.ExpMantissa.Get();
     c.Scale = constants.Scale;
     c.InvScale = constants.InvScale;
-    CBAMD_ENSURE((docCount + 255) / 256 <= 0x7fffffffu, "too many documents in one batch");
-    hipLaunchKernelGGL(dev::ApplyPredictionTypeKernel, dim3(static_cast<uint32_t>((docCount + 255) / 256)), dim3(256), 0, s,
+    CBAMD_ENSURE((docCount + 63) / 64 <= 0x7fffffffu, "too many documents in one batch");
+    hipLaunchKernelGGL(dev::ApplyPredictionTypeKernel, dim3(static_cast<uint32_t>((docCount + 63) / 64)), dim3(64), 0, s,
                        predictionType, dim, firstDoc, totalDocs, docCount, c, raw, result);
     HIP_CHECK(hipGetLastError());
 }

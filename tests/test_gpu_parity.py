@@ -345,6 +345,32 @@ def test_prediction_types_on_the_device(golden_dir, dim):
             ev.apply_prediction_type(cb.APT_MULTI_PROBABILITY, 1, 0, 0)
 
 
+@pytest.mark.parametrize("dim", [4, 5, 6, 7, 8, 9])
+def test_softmax_of_few_dimensions_in_registers(golden_dir, dim):
+    """Up to eight dimensions a document's values stay in registers (2 and 3 above), nine take the general loop: bit for
+    bit the oracle's, out of place and in place, with clamps, infinities, NaN and documents around a workgroup's 64."""
+    import torch
+
+    from oracle.oracle import apply_prediction_type
+
+    rng = np.random.default_rng(dim)
+    ev = _gpu_model(_random_oblivious(rng, trees=2, dim=dim)[0]).evaluator()
+    pool = np.load(os.path.join(golden_dir, "fmath_exp_vectors.npz"))["x"]
+    for docs in (1, 63, 64, 65, 129, len(pool) // dim):
+        raw = pool[rng.permutation(len(pool))[:docs * dim]].copy()
+        raw[:dim] = raw[0]
+        expected = apply_prediction_type(raw, dim, "Probability")
+        x = torch.from_numpy(raw).to("cuda:0")
+        out = torch.full((docs * dim + 8,), 777.0, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        ev.apply_prediction_type(cb.APT_PROBABILITY, docs, x.data_ptr(), out.data_ptr())
+        ev.apply_prediction_type(cb.APT_PROBABILITY, docs, x.data_ptr(), x.data_ptr())
+        ev.synchronize()
+        _same_bits(out.cpu().numpy()[:docs * dim], expected, "dim %d docs %d" % (dim, docs))
+        assert bool((out[docs * dim:] == 777.0).all())
+        _same_bits(x.cpu().numpy(), expected, "in place")
+
+
 # -------------------------------------------------------- CTR (target statistics) features ----
 
 def _hashed(rows):
