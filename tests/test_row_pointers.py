@@ -17,7 +17,8 @@ def test_row_pointers(shape, kind):
         x = np.concatenate([x, x])[2:2 + shape[0]]
     x.setflags(write=kind != "read-only")
     assert cb._address(x) == x.ctypes.data
-    rows = ctypes.cast(cb._row_pointers(x), ctypes.POINTER(ctypes.c_void_p))
+    argument = cb._row_pointers(x)  # owns the addresses; a cast of it does not
+    rows = ctypes.cast(argument, ctypes.POINTER(ctypes.c_void_p))
     for i in range(shape[0]):
         assert rows[i] == x.ctypes.data + i * x.strides[0]
         if shape[1]:
