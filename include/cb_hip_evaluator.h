@@ -88,7 +88,8 @@ typedef struct CbHipFeatures {
  *   CATBOOST_AMD_REG_SPLIT=0         a float feature keeps to one bins register: more than 127 used borders send the
  *                                    model to the mixed (8-bit compare) kernels (else: more than 128 take two)
  *   CATBOOST_AMD_SMALL_BATCH=0       the start value of CbHipSetSmallBatchSlicing is "off"
- *   CATBOOST_AMD_LEVEL_ORDER=0       register-resident kernels keep the model's order of a tree's levels
+ *   CATBOOST_AMD_LEVEL_ORDER=0       register-resident, exchange and small-batch kernels keep the
+ *                                    order of a tree's levels that the model has
  *   CATBOOST_AMD_FUSED=0             binarize and evaluate always as two launches (no fused kernels)
  *   CATBOOST_AMD_PAIR_TILE=0         wide one-dimensional models (more buckets than an LDS tile of 256 documents
  *                                    holds): one tree per wave instead of two or four
