@@ -4253,9 +4253,28 @@ void THipEvaluator::ApplyPredictionTypeDevice(int predictionType, size_t firstDo
     c.Mantissa = m.ExpMantissa.Get();
     c.Scale = constants.Scale;
     c.InvScale = constants.InvScale;
-    CBAMD_ENSURE((docCount + 63) / 64 <= 0x7fffffffu, "too many documents in one batch");
-    hipLaunchKernelGGL(dev::ApplyPredictionTypeKernel, dim3(static_cast<uint32_t>((docCount + 63) / 64)), dim3(64), 0, s,
-                       predictionType, dim, firstDoc, totalDocs, docCount, c, raw, result);
+    CBAMD_ENSURE((docCount + 255) / 256 <= 0x7fffffffu, "too many documents in one batch");
+    const dim3 grid(static_cast<uint32_t>((docCount + 255) / 256));
+    const auto softmax = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, docCount, c, raw, result); };
+    const bool isSoftmax = predictionType == dev::kPredProbability && dim > 1;
+    if (isSoftmax && dim <= 8) {
+        switch (dim) {
+            case 2: softmax(dev::SoftmaxKernel<2>); break;
+            case 3: softmax(dev::SoftmaxKernel<3>); break;
+            case 4: softmax(dev::SoftmaxKernel<4>); break;
+            case 5: softmax(dev::SoftmaxKernel<5>); break;
+            case 6: softmax(dev::SoftmaxKernel<6>); break;
+            case 7: softmax(dev::SoftmaxKernel<7>); break;
+            default: softmax(dev::SoftmaxKernel<8>); break;
+        }
+    } else if (isSoftmax || (predictionType == dev::kPredClass && dim >= dev::kManyDimsClass) ||
+               (predictionType == dev::kPredMultiProbability && dim >= dev::kManyDimsMultiProbability)) {
+        hipLaunchKernelGGL(dev::ApplyPredictionTypeManyKernel, dim3(static_cast<uint32_t>((docCount + 63) / 64)), dim3(64), 0, s,
+                           predictionType, dim, firstDoc, totalDocs, docCount, c, raw, result);
+    } else {
+        hipLaunchKernelGGL(dev::ApplyPredictionTypeKernel, grid, dim3(256), 0, s, predictionType, dim, firstDoc, totalDocs, docCount, c,
+                           raw, result);
+    }
     HIP_CHECK(hipGetLastError());
 }
 

@@ -3339,39 +3339,10 @@ __device__ __forceinline__ double FastExpAt(const TFastExpDev& c, double v, size
 constexpr int kPredRaw = 0, kPredExponent = 1, kPredRmseWithUncertainty = 2, kPredProbability = 3, kPredClass = 4,
               kPredMultiProbability = 5;  // EApiPredictionType, catboost/libs/model_interface/c_api.h:50-57
 
-// CalcSoftmax of one document (eval_processing.h:15-27) with its values in registers; r == o is allowed.
-// In the loops over `dim` every exponential was stored and, as o may be r, loaded again for the division, and no load went
-// past a store; so they wait for memory, and here a document's loads are in flight together. In workgroups of one wave, which
-// spread small batches. A launch: 100 000 documents of three dimensions 4.2 -> 3.1 us, 500 000 of eight 92.7 -> 18.4 (64 MB;
-// a copy takes 12), 1 000 000 of two 11.7 -> 7.3. Eight dimensions are 16 registers per array; more take the loops.
-template <uint32_t DIM>
-__device__ __forceinline__ void SoftmaxInRegisters(const TFastExpDev& c, const double* r, double* o) {
-    double v[DIM];
-#pragma unroll
-    for (uint32_t k = 0; k < DIM; ++k) {
-        v[k] = r[k];
-    }
-    double top = v[0];
-#pragma unroll
-    for (uint32_t k = 1; k < DIM; ++k) {
-        top = top < v[k] ? v[k] : top;
-    }
-    double sum = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < DIM; ++k) {
-        v[k] = FastExpAt(c, v[k] - top, k, DIM);
-        sum += v[k];
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < DIM; ++k) {
-        o[k] = v[k] / sum;
-    }
-}
-
 // One thread per document of a chunk that starts at document `firstDoc` of `totalDocs`.
 // raw[doc * dim + k] -> out (doc values for Class, doc * dim values otherwise). raw == out is allowed
-// except for Class with dim > 1.
-__global__ __launch_bounds__(64) void ApplyPredictionTypeKernel(int type, uint32_t dim, size_t firstDoc,
+// except for Class with dim > 1. Softmax, and Class and MultiProbability of many dimensions, have the kernels below.
+__global__ __launch_bounds__(256) void ApplyPredictionTypeKernel(int type, uint32_t dim, size_t firstDoc,
                                                                  size_t totalDocs, size_t docCount, TFastExpDev c,
                                                                  const double* raw, double* out) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -3420,30 +3391,6 @@ __global__ __launch_bounds__(64) void ApplyPredictionTypeKernel(int type, uint32
             }
             o[k] = v;
         }
-    } else if (type == kPredProbability) {  // CalcSoftmax, eval_processing.h:15-27
-        switch (dim) {
-            case 2: SoftmaxInRegisters<2>(c, r, o); return;
-            case 3: SoftmaxInRegisters<3>(c, r, o); return;
-            case 4: SoftmaxInRegisters<4>(c, r, o); return;
-            case 5: SoftmaxInRegisters<5>(c, r, o); return;
-            case 6: SoftmaxInRegisters<6>(c, r, o); return;
-            case 7: SoftmaxInRegisters<7>(c, r, o); return;
-            case 8: SoftmaxInRegisters<8>(c, r, o); return;
-        }
-        double top = r[0];
-        for (uint32_t k = 1; k < dim; ++k) {
-            const double v = r[k];
-            top = top < v ? v : top;
-        }
-        double sum = 0;
-        for (uint32_t k = 0; k < dim; ++k) {
-            const double e = FastExpAt(c, r[k] - top, k, dim);
-            o[k] = e;
-            sum += e;
-        }
-        for (uint32_t k = 0; k < dim; ++k) {
-            o[k] = o[k] / sum;
-        }
     } else if (type == kPredMultiProbability) {
         for (uint32_t k = 0; k < dim; ++k) {
             o[k] = 1. / (1. + FastExpAt(c, -r[k], inBlock * dim + k, blockDocs * dim));
@@ -3453,6 +3400,104 @@ __global__ __launch_bounds__(64) void ApplyPredictionTypeKernel(int type, uint32
             o[k] = r[k];
         }
     }
+}
+
+// CalcSoftmax (eval_processing.h:15-27) of two to eight dimensions, a document's values in the registers of its thread; raw == out
+// is allowed. In loops over a dimension of the call's every exponential was stored and, as out may be raw, loaded again for the
+// division, and no load went past a store, so they waited for memory; here a document's loads are in flight together. A launch:
+// 100 000 documents of three dimensions 4.3 -> 2.7 us, 500 000 of eight 92.3 -> 17.8 (64 MB; a copy takes 12), 1 000 000 of two
+// 11.9 -> 6.4. Eight dimensions are 16 registers per array; more take the kernel below. A kernel of its own, since its registers
+// cost the other types' waves (Class of 1 000 000 documents of two dimensions 4.0 -> 4.5 us with both in one).
+template <uint32_t DIM>
+__global__ __launch_bounds__(256) void SoftmaxKernel(size_t docCount, TFastExpDev c, const double* raw, double* out) {
+    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= docCount) {
+        return;
+    }
+    const double* r = raw + i * DIM;
+    double* o = out + i * DIM;
+    double v[DIM];
+#pragma unroll
+    for (uint32_t k = 0; k < DIM; ++k) {
+        v[k] = r[k];
+    }
+    double top = v[0];
+#pragma unroll
+    for (uint32_t k = 1; k < DIM; ++k) {
+        top = top < v[k] ? v[k] : top;
+    }
+    double sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < DIM; ++k) {
+        v[k] = FastExpAt(c, v[k] - top, k, DIM);
+        sum += v[k];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < DIM; ++k) {
+        o[k] = v[k] / sum;
+    }
+}
+
+// f(k, r[k]) for k = 0 .. dim - 1, the loads of a turn of eight in flight together and before what f stores in its places of r
+template <typename F>
+__device__ __forceinline__ void ForEachInTurns(const double* r, uint32_t dim, const F& f) {
+    constexpr uint32_t kTurn = 8;
+    for (uint32_t first = 0; first < dim; first += kTurn) {
+        double v[kTurn];
+#pragma unroll
+        for (uint32_t j = 0; j < kTurn; ++j) {
+            v[j] = r[min(first + j, dim - 1)];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kTurn; ++j) {
+            if (first + j < dim) {
+                f(first + j, v[j]);
+            }
+        }
+    }
+}
+
+// Many dimensions: softmax of more than eight (its exponentials computed twice, which costs less than storing and loading them),
+// Class and MultiProbability from the two lines on. Arguments as ApplyPredictionTypeKernel, whose loop has one load in flight.
+// Workgroups of one wave: few documents of many dimensions spread over every CU. A launch, that loop -> this kernel: Class of
+// 500 000 documents of eight dimensions 9.5 -> 7.1 us (400 000 of five 4.2 -> 4.4, 1 000 000 of two 4.0 -> 5.9), MultiProbability of
+// 500 000 of eight 65 -> 28, 15 000 of four 3.3 -> 2.8 (100 000 of three 3.4 -> 3.5); softmax of 200 000 of ten 51 -> 22,
+// of 20 000 of a hundred 114 -> 55 (71 with workgroups of four waves).
+constexpr uint32_t kManyDimsClass = 8, kManyDimsMultiProbability = 4;
+
+__global__ __launch_bounds__(64) void ApplyPredictionTypeManyKernel(int type, uint32_t dim, size_t firstDoc, size_t totalDocs,
+                                                                    size_t docCount, TFastExpDev c, const double* raw, double* out) {
+    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= docCount) {
+        return;
+    }
+    const double* r = raw + i * dim;
+    double* o = out + i * dim;
+    if (type == kPredMultiProbability) {
+        const size_t doc = firstDoc + i;
+        const size_t blockSize = totalDocs < 128 ? totalDocs : 128;
+        const size_t inBlock = doc % blockSize;
+        const size_t blockDocs = min(blockSize, totalDocs - (doc - inBlock));  // documents of this document's block
+        ForEachInTurns(r, dim, [&](uint32_t k, double v) {
+            o[k] = 1. / (1. + FastExpAt(c, -v, inBlock * dim + k, blockDocs * dim));
+        });
+        return;
+    }
+    uint32_t best = 0;
+    double top = r[0];
+    ForEachInTurns(r, dim, [&](uint32_t k, double v) {
+        if (top < v) {  // std::max_element: the first largest
+            top = v;
+            best = k;
+        }
+    });
+    if (type == kPredClass) {
+        out[i] = static_cast<double>(best);
+        return;
+    }
+    double sum = 0;
+    ForEachInTurns(r, dim, [&](uint32_t k, double v) { sum += FastExpAt(c, v - top, k, dim); });
+    ForEachInTurns(r, dim, [&](uint32_t k, double v) { o[k] = FastExpAt(c, v - top, k, dim) / sum; });
 }
 
 __global__ void FillBiasKernel(double* __restrict__ out, size_t count, const double* __restrict__ bias, int dim) {

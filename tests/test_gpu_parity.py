@@ -345,10 +345,11 @@ def test_prediction_types_on_the_device(golden_dir, dim):
             ev.apply_prediction_type(cb.APT_MULTI_PROBABILITY, 1, 0, 0)
 
 
-@pytest.mark.parametrize("dim", [4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("dim", [4, 5, 6, 7, 8, 9, 16, 17])
 def test_softmax_of_few_dimensions_in_registers(golden_dir, dim):
-    """Up to eight dimensions a document's values stay in registers (2 and 3 above), nine take the general loop: bit for
-    bit the oracle's, out of place and in place, with clamps, infinities, NaN and documents around a workgroup's 64."""
+    """Softmax of up to eight dimensions (2 and 3 above) keeps a document's values in registers; more, Class of eight
+    and MultiProbability of four and more take them in turns of eight: bit for bit the oracle's, out of place and in place,
+    with clamps, infinities, NaN and documents around a workgroup's 64 and 256."""
     import torch
 
     from oracle.oracle import apply_prediction_type
@@ -359,16 +360,19 @@ def test_softmax_of_few_dimensions_in_registers(golden_dir, dim):
     for docs in (1, 63, 64, 65, 129, len(pool) // dim):
         raw = pool[rng.permutation(len(pool))[:docs * dim]].copy()
         raw[:dim] = raw[0]
-        expected = apply_prediction_type(raw, dim, "Probability")
-        x = torch.from_numpy(raw).to("cuda:0")
-        out = torch.full((docs * dim + 8,), 777.0, dtype=torch.float64, device="cuda:0")
-        torch.cuda.synchronize()
-        ev.apply_prediction_type(cb.APT_PROBABILITY, docs, x.data_ptr(), out.data_ptr())
-        ev.apply_prediction_type(cb.APT_PROBABILITY, docs, x.data_ptr(), x.data_ptr())
-        ev.synchronize()
-        _same_bits(out.cpu().numpy()[:docs * dim], expected, "dim %d docs %d" % (dim, docs))
-        assert bool((out[docs * dim:] == 777.0).all())
-        _same_bits(x.cpu().numpy(), expected, "in place")
+        for name, kind in (("Probability", cb.APT_PROBABILITY), ("MultiProbability", cb.APT_MULTI_PROBABILITY), ("Class", cb.APT_CLASS)):
+            expected = apply_prediction_type(raw, dim, name)
+            x = torch.from_numpy(raw).to("cuda:0")
+            out = torch.full((len(expected) + 8,), 777.0, dtype=torch.float64, device="cuda:0")
+            torch.cuda.synchronize()
+            ev.apply_prediction_type(kind, docs, x.data_ptr(), out.data_ptr())
+            if name != "Class":
+                ev.apply_prediction_type(kind, docs, x.data_ptr(), x.data_ptr())
+            ev.synchronize()
+            _same_bits(out.cpu().numpy()[:len(expected)], expected, "%s dim %d docs %d" % (name, dim, docs))
+            assert bool((out[len(expected):] == 777.0).all())
+            if name != "Class":
+                _same_bits(x.cpu().numpy(), expected, "in place")
 
 
 # -------------------------------------------------------- CTR (target statistics) features ----
