@@ -3097,13 +3097,16 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 levels.emplace_back(lopsidedness(trees.RepackedBins[trees.TreeStartOffsets[t] + d]), d);
             }
             std::stable_sort(levels.begin(), levels.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
-            for (size_t index = 0; t < TreeCount && index < (size_t(1) << depth); ++index) {
-                size_t leaf = 0;
-                for (int d = 0; d < depth; ++d) {
-                    leaf |= (index >> d & 1) << levels[d].second;
-                }
+            if (t < TreeCount) {
                 const size_t treeAt = trees.TreeFirstLeafOffsets[t], dim = static_cast<size_t>(m.Dim);
-                std::copy_n(trees.LeafValues.begin() + treeAt + leaf * dim, dim, smallLeaves.begin() + treeAt + index * dim);
+                uint32_t leafOf[256] = {};  // by the index in the order of the rows; this kernel's trees have up to eight levels
+                for (uint32_t index = 0; index < (1u << depth); ++index) {
+                    if (index != 0) {  // of the index without its lowest bit, and that bit's level
+                        leafOf[index] = leafOf[index & (index - 1)] | 1u << levels[__builtin_ctz(index)].second;
+                    }
+                    const double* leaf = trees.LeafValues.data() + treeAt + leafOf[index] * dim;
+                    std::copy(leaf, leaf + dim, smallLeaves.data() + treeAt + index * dim);
+                }
             }
             for (int d = 0; d < 8; ++d) {
                 row[8 + d] = never;
