@@ -4007,12 +4007,15 @@ static void AwaitSmallBatch(THipEvaluator::TImpl& m, const THipEvaluator::TImpl:
 int THipEvaluator::FusedLayoutFor(int layout, size_t stride, size_t docCount, size_t treeStart, size_t treeEnd, bool anyBatchSize) const {
     const TImpl& m = *Impl;
     const int layoutIndex = layout == TFeatureBatch::FlatRows ? 0 : layout == TFeatureBatch::SplitRows ? 1 : layout == TFeatureBatch::FlatColumns ? 2 : -1;
+    if (layoutIndex < 0 || docCount == 0) {
+        return -1;
+    }
     if (layoutIndex == 0 && !anyBatchSize && treeStart == 0 && treeEnd == TreeCount && stride < (size_t(1) << 20) &&
         m.TakesFusedExchangeKernel(docCount)) {
         return kFusedExchange;
     }
-    if (layoutIndex < 0 || !m.Fused[layoutIndex] || docCount == 0 || treeStart != 0 || treeEnd != TreeCount ||
-        docCount >= (size_t(1) << 29) || stride >= (size_t(1) << (layoutIndex == 2 ? 30 : 20))) {
+    if (!m.Fused[layoutIndex] || treeStart != 0 || treeEnd != TreeCount || docCount >= (size_t(1) << 29) ||
+        stride >= (size_t(1) << (layoutIndex == 2 ? 30 : 20))) {
         return -1;
     }
     if (!anyBatchSize && docCount < m.FusedMinDocs()) {

@@ -81,3 +81,31 @@ def test_exchange_kernel_gives_the_pair_tile_kernels_bits(buckets, cats, trees, 
     ranged = exchange.calc_flat(x[:33_000], tree_start=1, tree_end=trees)
     np.testing.assert_allclose(ranged[sample[sample < 33_000]],
                                OracleModel(model).calc(x[sample[sample < 33_000]], tree_start=1, tree_end=trees), rtol=1e-9, atol=1e-12)
+
+
+def test_empty_batches():
+    """No documents: every call returns without touching a buffer, null pointers among them."""
+    import torch
+
+    model, _ = _model_of_buckets(np.random.default_rng(2), 700, 3, 201, 8, 1, 1)
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    assert "fused" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, 60_000)
+    assert "fused" not in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, 0)
+    assert g.calc_flat(np.zeros((0, 700), np.float32)).size == 0
+    assert g.calc_flat_transposed(np.zeros((700, 0), np.float32)).size == 0
+    assert g.quantize_flat(np.zeros((0, 700), np.float32)).size == 0
+    assert g.calc_leaf_indexes_flat(np.zeros((0, 700), np.float32)).size == 0
+    guard = torch.full((16,), 7.0, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    for pointer in (guard.data_ptr(), 0):
+        for layout in (cb.LAYOUT_FLAT_ROWS, cb.LAYOUT_FLAT_COLUMNS):
+            feats = ev.features(layout, pointer, 700)
+            ev.eval_data(feats, 0, pointer)
+            ev.eval_data_no_alloc(feats, 0, pointer)
+            ev.quantize(feats, 0, pointer)
+        ev.eval_quantized(pointer, 0, pointer)
+    ev.synchronize()
+    assert bool((guard == 7.0).all())
