@@ -3,6 +3,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <future>
+#include <numeric>
 #include <utility>
 
 namespace cbamd {
@@ -13,9 +15,18 @@ namespace {
 struct TEdge {
     uint32_t Tree = 0, Group = 0;
     const TExchangeLevel* Level = nullptr;
-    uint32_t ModelLevel = 0;  // which level of its tree
-    bool High = false;        // one of the places behind the first five
-    int Place = -1;           // place in its group, later the order of the compares
+    float Lopsided = 0.0f;
+    uint8_t ModelLevel = 0;  // which level of its tree
+    bool High = false;       // one of the places behind the first five
+    int8_t Place = -1;       // place in its group, later the order of the compares
+};
+
+// A tree's edges follow one another: all trees are in the order of their steps (At: place of a tree in that order)
+struct TTreeEdges {
+    std::vector<uint32_t> First;  // per place in the order, and the end
+    std::vector<uint32_t> At;
+    uint32_t Begin(uint32_t tree) const { return First[At[tree]]; }
+    uint32_t End(uint32_t tree) const { return First[At[tree] + 1]; }
 };
 
 struct TGroup {
@@ -33,20 +44,22 @@ constexpr uint32_t kEvenPlaces = 5;
 
 class TSides {
 public:
-    TSides(std::vector<TEdge>* edges, const std::vector<std::vector<uint32_t>>& ofTree, const std::vector<TGroup>& groups,
-           uint32_t places)
-        : Edges(*edges), OfTree(ofTree), Groups(groups), Places{kEvenPlaces, places - kEvenPlaces}, TreeCount{std::vector<uint32_t>(ofTree.size(), 0), std::vector<uint32_t>(ofTree.size(), 0)}
-        , GroupCount{std::vector<uint32_t>(groups.size(), 0), std::vector<uint32_t>(groups.size(), 0)} {
+    TSides(std::vector<TEdge>* edges, const TTreeEdges& ofTree, const std::vector<TGroup>& groups, uint32_t places)
+        : Edges(*edges), OfTree(ofTree), Groups(groups), Places{kEvenPlaces, places - kEvenPlaces}
+        , TreeCount{std::vector<uint8_t>(ofTree.At.size(), 0), std::vector<uint8_t>(ofTree.At.size(), 0)}
+        , GroupCount{std::vector<uint8_t>(groups.size(), 0), std::vector<uint8_t>(groups.size(), 0)}, Seen(groups.size(), 0) {
     }
 
     bool Assign() {
-        for (size_t t = 0; t < OfTree.size(); ++t) {
-            std::vector<uint32_t> order(OfTree[t]);
-            std::stable_sort(order.begin(), order.end(),
-                             [&](uint32_t a, uint32_t b) { return Edges[a].Level->Lopsided < Edges[b].Level->Lopsided; });
-            for (size_t i = 0; i < order.size(); ++i) {
-                Edges[order[i]].High = i >= kEvenPlaces;
-                Count(order[i], 1);
+        for (uint32_t t = 0; t < OfTree.At.size(); ++t) {
+            const uint32_t begin = OfTree.Begin(t), end = OfTree.End(t);
+            for (uint32_t e = begin; e < end; ++e) {
+                uint32_t before = 0;  // edges of the tree that come before this one, evenest first
+                for (uint32_t o = begin; o < end; ++o) {
+                    before += Edges[o].Lopsided < Edges[e].Lopsided || (o < e && Edges[o].Lopsided == Edges[e].Lopsided);
+                }
+                Edges[e].High = before >= kEvenPlaces;
+                Count(e, 1);
             }
         }
         for (uint32_t g = 0; g < Groups.size(); ++g) {
@@ -71,8 +84,8 @@ private:
         Edges[e].High = !Edges[e].High;
         Count(e, 1);
     }
-    double Cost(uint32_t e) const {  // of moving the edge to the other side
-        return Edges[e].High ? -Edges[e].Level->Lopsided : Edges[e].Level->Lopsided;
+    float Cost(uint32_t e) const {  // of moving the edge to the other side
+        return Edges[e].High ? -Edges[e].Lopsided : Edges[e].Lopsided;
     }
 
     // One edge of `side` less in group g: along a shortest chain of swaps (an edge of the group leaves `side`, another
@@ -81,9 +94,9 @@ private:
         Steps.clear();
         At.assign(1, g);
         Via.assign(1, -1);
-        Seen.assign(1, g);
+        Seen[g] = ++Search;
         while (!At.empty()) {
-            double bestCost = 0.0;
+            float bestCost = 0.0f;
             int best = -1;
             Next.clear();
             NextVia.clear();
@@ -101,20 +114,20 @@ private:
                         }
                         continue;
                     }
-                    for (uint32_t in : OfTree[t]) {
+                    for (uint32_t in = OfTree.Begin(t); in < OfTree.End(t); ++in) {
                         const uint32_t to = Edges[in].Group;
                         if (Edges[in].High == side || to == At[i]) {
                             continue;
                         }
                         if (GroupCount[side][to] < Places[side]) {
-                            const double cost = Cost(out) + Cost(in);
+                            const float cost = Cost(out) + Cost(in);
                             Steps.push_back({out, in, Via[i]});
                             if (best < 0 || cost < bestCost) {
                                 best = static_cast<int>(Steps.size()) - 1;
                                 bestCost = cost;
                             }
-                        } else if (std::find(Seen.begin(), Seen.end(), to) == Seen.end()) {
-                            Seen.push_back(to);
+                        } else if (Seen[to] != Search) {
+                            Seen[to] = Search;
                             Steps.push_back({out, in, Via[i]});
                             Next.push_back(to);
                             NextVia.push_back(static_cast<int>(Steps.size()) - 1);
@@ -142,68 +155,66 @@ private:
         int Parent;        // step before
     };
     std::vector<TStep> Steps;              // of Relieve
-    std::vector<uint32_t> At, Next, Seen;  // groups of the frontier, of the next one, and all that were on one
+    std::vector<uint32_t> At, Next;        // groups of the frontier and of the next one
     std::vector<int> Via, NextVia;         // steps that led there
     std::vector<TEdge>& Edges;
-    const std::vector<std::vector<uint32_t>>& OfTree;
+    const TTreeEdges& OfTree;
     const std::vector<TGroup>& Groups;
     const uint32_t Places[2];
-    std::vector<uint32_t> TreeCount[2], GroupCount[2];
+    std::vector<uint8_t> TreeCount[2], GroupCount[2];
+    std::vector<uint32_t> Seen;            // per group the last search that had it on a frontier
+    uint32_t Search = 0;
 };
 
 // Places base .. base + colours - 1 for the edges of one side: each edge takes a place that is free at its tree and at its group, after
 // swapping two places along the alternating path that starts at the group when there is no such place.
 void Colour(std::vector<TEdge>* edges, size_t treeCount, size_t groupCount, bool high, uint32_t colours, uint32_t base) {
-    std::vector<int> tree(treeCount * colours, -1), group(groupCount * colours, -1);
-    const auto slot = [&](bool isTree, uint32_t vertex, uint32_t colour) -> int& {
-        return (isTree ? tree : group)[vertex * colours + colour];
+    std::vector<uint32_t> slots((treeCount + groupCount) * colours);  // a colour's edge at a vertex, the trees' first
+    std::vector<uint8_t> freeOf(treeCount + groupCount, static_cast<uint8_t>((1u << colours) - 1));
+    std::vector<uint32_t> path;
+    const auto take = [&](uint32_t e, uint32_t vertex, uint32_t colour) {
+        slots[vertex * colours + colour] = e;
+        freeOf[vertex] &= ~(1u << colour);
     };
     for (size_t i = 0; i < edges->size(); ++i) {
         TEdge& e = (*edges)[i];
         if (e.High != high) {
             continue;
         }
-        int atTree = -1, atGroup = -1, both = -1;
-        for (uint32_t c = 0; c < colours; ++c) {
-            const bool freeTree = slot(true, e.Tree, c) < 0, freeGroup = slot(false, e.Group, c) < 0;
-            if (freeTree && atTree < 0) {
-                atTree = static_cast<int>(c);
-            }
-            if (freeGroup && atGroup < 0) {
-                atGroup = static_cast<int>(c);
-            }
-            if (freeTree && freeGroup && both < 0) {
-                both = static_cast<int>(c);
-            }
-        }
-        if (both < 0) {
+        const uint32_t tree = e.Tree, group = static_cast<uint32_t>(treeCount) + e.Group;
+        uint32_t colour;
+        if (const uint32_t both = freeOf[tree] & freeOf[group]; both != 0) {
+            colour = __builtin_ctz(both);
+        } else {
             // the path from the group along the colours atTree, atGroup, atTree ... never comes to the edge's tree
-            std::vector<uint32_t> path;
+            const uint32_t atTree = __builtin_ctz(freeOf[tree]), atGroup = __builtin_ctz(freeOf[group]);
+            path.clear();
             bool isTree = false;
-            uint32_t vertex = e.Group;
-            int colour = atTree;
-            for (int next = slot(isTree, vertex, colour); next >= 0; next = slot(isTree, vertex, colour)) {
-                path.push_back(static_cast<uint32_t>(next));
+            uint32_t vertex = group, along = atTree;
+            while ((freeOf[vertex] >> along & 1) == 0) {
+                path.push_back(slots[vertex * colours + along]);
                 isTree = !isTree;
-                vertex = isTree ? (*edges)[next].Tree : (*edges)[next].Group;
-                colour = colour == atTree ? atGroup : atTree;
+                vertex = isTree ? (*edges)[path.back()].Tree : static_cast<uint32_t>(treeCount) + (*edges)[path.back()].Group;
+                along ^= atTree ^ atGroup;
             }
             for (uint32_t p : path) {
                 const TEdge& on = (*edges)[p];
-                slot(true, on.Tree, on.Place - base) = -1;
-                slot(false, on.Group, on.Place - base) = -1;
+                const uint32_t bit = 1u << (on.Place - base);
+                freeOf[on.Tree] |= bit;
+                freeOf[treeCount + on.Group] |= bit;
             }
             for (uint32_t p : path) {
                 TEdge& on = (*edges)[p];
-                on.Place = static_cast<int>(base) + (on.Place - static_cast<int>(base) == atTree ? atGroup : atTree);
-                slot(true, on.Tree, on.Place - base) = static_cast<int>(p);
-                slot(false, on.Group, on.Place - base) = static_cast<int>(p);
+                const uint32_t other = on.Place - base == atTree ? atGroup : atTree;
+                on.Place = static_cast<int8_t>(base + other);
+                take(p, on.Tree, other);
+                take(p, static_cast<uint32_t>(treeCount) + on.Group, other);
             }
-            both = atTree;
+            colour = atTree;
         }
-        e.Place = static_cast<int>(base) + both;
-        slot(true, e.Tree, both) = static_cast<int>(i);
-        slot(false, e.Group, both) = static_cast<int>(i);
+        e.Place = static_cast<int8_t>(base + colour);
+        take(static_cast<uint32_t>(i), tree, colour);
+        take(static_cast<uint32_t>(i), group, colour);
     }
 }
 
@@ -290,10 +301,14 @@ bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketC
     }
     std::stable_sort(byStep.begin(), byStep.end(), [&](uint32_t a, uint32_t b) { return stepOf[a] < stepOf[b]; });
     std::vector<TEdge> edges;
+    edges.reserve(std::accumulate(levelsOf.begin(), levelsOf.end(), size_t(0)));
     std::vector<TGroup> groups;
-    std::vector<std::vector<uint32_t>> edgesOfTree(treeCount), groupsOf(kExchangeWaves);
+    std::vector<std::vector<uint32_t>> groupsOf(kExchangeWaves);
+    TTreeEdges edgesOfTree;
+    edgesOfTree.At.resize(treeCount);
     for (uint32_t t : byStep) {
-        edgesOfTree[t].reserve(trees[t].Levels.size());
+        edgesOfTree.At[t] = static_cast<uint32_t>(edgesOfTree.First.size());
+        edgesOfTree.First.push_back(static_cast<uint32_t>(edges.size()));
         for (uint32_t d = 0; d < trees[t].Levels.size(); ++d) {
             const TExchangeLevel& level = trees[t].Levels[d];
             const uint32_t w = waveOf[level.Bucket];
@@ -306,23 +321,29 @@ bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketC
             edge.Tree = t;
             edge.Group = groupsOf[w].back();
             edge.Level = &level;
-            edge.ModelLevel = d;
+            edge.Lopsided = level.Lopsided;
+            edge.ModelLevel = static_cast<uint8_t>(d);
             TGroup& group = groups[edge.Group];
             const uint32_t round = stepOf[t] / kExchangeRoundSteps;
             group.FirstRound = std::min(group.FirstRound, round);
             group.LastRound = std::max(group.LastRound, round);
             group.Edges.push_back(static_cast<uint32_t>(edges.size()));
-            edgesOfTree[t].push_back(static_cast<uint32_t>(edges.size()));
             edges.push_back(edge);
         }
     }
+    edgesOfTree.First.push_back(static_cast<uint32_t>(edges.size()));
 
     // ---- places in the groups
     if (!TSides(&edges, edgesOfTree, groups, maxDepth).Assign()) {
         return false;
     }
-    Colour(&edges, treeCount, groups.size(), false, kEvenPlaces, 0);
-    Colour(&edges, treeCount, groups.size(), true, maxDepth - kEvenPlaces, kEvenPlaces);
+    {
+        // of either side on its own, which touch no edge in common: on two threads where there are many
+        std::future<void> low = std::async(edges.size() < 8192 ? std::launch::deferred : std::launch::async | std::launch::deferred,
+                                           [&] { Colour(&edges, treeCount, groups.size(), false, kEvenPlaces, 0); });
+        Colour(&edges, treeCount, groups.size(), true, maxDepth - kEvenPlaces, kEvenPlaces);
+        low.get();
+    }
 
     // ---- when a group is compared, and in which slot it stands. A wave compares a group at the end of a step. The barrier of
     // round r stands at the beginning of its last step; behind it come the reads for the next round's first tree. So
@@ -431,26 +452,17 @@ bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketC
         }
     }
     plan->ExtraRows.resize(plan->ExtraRows.size() + kExchangeEarlyRows * kExchangeGroupDwords, 0);
-    const size_t leafCount = size_t(1) << maxDepth;
-    plan->Leaves.assign((size_t(plan->Rounds) + 1) * kExchangeWaves * kExchangeRoundSteps * leafCount, 0.0);
+    plan->LeafRows.assign((size_t(plan->Rounds) + 1) * kExchangeWaves * kExchangeRoundSteps, TExchangeLeafRow());
     for (size_t t = 0; t < treeCount; ++t) {
         const size_t step = stepOf[t], inRound = step % kExchangeRoundSteps;
         const uint32_t w = sumWaveOf[t];
         uint32_t* row = recordOf(step, w) + kExchangeRoundSteps * kExchangeGroupDwords + inRound * kExchangeTreeDwords;
-        double* values = plan->Leaves.data() + ((step / kExchangeRoundSteps * kExchangeWaves + w) * kExchangeRoundSteps + inRound) * leafCount;
-        for (uint32_t e : edgesOfTree[t]) {
-            row[edges[e].Place] = groups[edges[e].Group].Slot * 256u;
-        }
-        // a place without a level holds another group's bit: the values are the same for either
-        uint32_t low[16] = {}, high[16] = {};  // what the lower and the upper four bits of an index say of the leaf
-        for (uint32_t i = 0; i < 16; ++i) {
-            for (uint32_t e : edgesOfTree[t]) {
-                const uint32_t place = static_cast<uint32_t>(edges[e].Place);
-                (place < 4 ? low : high)[i] |= (i >> place % 4 & 1) << edges[e].ModelLevel;
-            }
-        }
-        for (size_t i = 0; i < leafCount; ++i) {
-            values[i] = trees[t].Leaves[low[i & 15] | high[i >> 4]];
+        TExchangeLeafRow& leaves = plan->LeafRows[(step / kExchangeRoundSteps * kExchangeWaves + w) * kExchangeRoundSteps + inRound];
+        leaves.Tree = static_cast<uint32_t>(t);
+        for (uint32_t e = edgesOfTree.Begin(static_cast<uint32_t>(t)); e < edgesOfTree.End(static_cast<uint32_t>(t)); ++e) {
+            const TEdge& edge = edges[e];
+            row[edge.Place] = groups[edge.Group].Slot * 256u;
+            leaves.Levels ^= (kExchangeNoLevel ^ edge.ModelLevel) << 4 * edge.Place;
         }
     }
     return true;

@@ -43,12 +43,19 @@ struct TExchangeLevel {
     uint32_t Add = 0;       // byte added to the (xored) bin: the level's result is the carry into bit 7
     uint32_t Xor = 0;       // seven bits
     bool IsXor = false;
-    double Lopsided = 0.0;  // 0: splits the documents evenly
+    float Lopsided = 0.0f;  // 0: splits the documents evenly
 };
 
 struct TExchangeTree {
     std::vector<TExchangeLevel> Levels;
-    const double* Leaves = nullptr;  // 1 << Levels.size() values
+};
+
+// Where a row of 1 << maxDepth leaf values comes from
+constexpr uint32_t kExchangeNoTree = ~0u, kExchangeNoLevel = 15;
+struct TExchangeLeafRow {
+    uint32_t Tree = kExchangeNoTree;  // none: a row of zeros
+    uint32_t Levels = ~0u;            // four bits per bit of the row's index: the level of the model whose result that bit is, or
+                                      // kExchangeNoLevel: the bit is another group's, the values are the same for either
 };
 
 struct TExchangePlan {
@@ -57,7 +64,7 @@ struct TExchangePlan {
     std::vector<uint32_t> FusedWaveTable;  // the same with the registers' columns in the buffer for the buckets' offsets
     std::vector<uint32_t> Records;    // [round + 1][wave][kExchangeRecordDwords]: rows are fetched ahead
     std::vector<uint32_t> ExtraRows;  // [wave][its extra groups][kExchangeGroupDwords], and kExchangeEarlyRows spare ones
-    std::vector<double> Leaves;       // [round + 1][wave][step][1 << maxDepth]
+    std::vector<TExchangeLeafRow> LeafRows;  // [round + 1][wave][step]
 };
 
 // maxDepth: 6 or 8, at least the deepest tree's. six: all bins are at most 63, and the levels of even places in a group

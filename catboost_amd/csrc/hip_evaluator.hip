@@ -7,6 +7,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -14,6 +15,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <exception>
+#include <future>
 #include <limits>
 #include <map>
 #include <numeric>
@@ -1078,6 +1080,36 @@ void RunOnThreads(size_t count, size_t threads, const TWork& work) {
     }
 }
 
+// Host tables of the exchange kernels, which take longer than all others of such a model together: made on threads of their own
+// meanwhile. Building an evaluator of 5000 trees of depth 8 over 1016 features 16 -> 7.5 ms (with their leaf values copied on the device; the
+// plan alone 9 -> 4 ms, one of its threads), 3.1 without them.
+struct TExchangeTables {
+    std::vector<TExchangeTree> Trees;
+    std::vector<TExchangeColumn> Columns;      // fused form: none if the model does not qualify
+    std::vector<uint32_t> ColumnOf, Pieces;
+    uint32_t BucketCount = 0, MaxDepth = 0;
+    bool Six = false;
+
+    TExchangePlan Plan;
+    std::vector<uint32_t> Tiles, OneHot;
+    bool Planned = false, Tiled = false;
+
+    void Build() {
+        RunOnThreads(2, 2, [&](size_t part) {
+            if (part == 0) {
+                Planned = BuildExchangePlan(Trees, BucketCount, MaxDepth, Six, ColumnOf, &Plan);
+            } else if (!Columns.empty()) {
+                for (TExchangeColumn& column : Columns) {
+                    if (column.Used && !column.OneHot) {
+                        MakeExchangeGrid(Six, &column);
+                    }
+                }
+                Tiled = BuildExchangeTiles(Columns, Pieces, Six, &Tiles, &OneHot);
+            }
+        });
+    }
+};
+
 // One feature's value of one row of its table, static_ctr_provider.cpp:52-126: one branch per CTR type, the row null
 // where the table does not know the hash. Single roundings throughout, as TModelCtr::Calc (online_ctr.h:290-293).
 float CtrValueOfRow(const TModelCtr& ctr, const TCtrValueTable& table, const uint8_t* row) {
@@ -1585,7 +1617,7 @@ struct THipEvaluator::TImpl {
     uint32_t ExchangeRounds = 0;
     bool PairBeforeTile = false;       // the tile kernel would hold the model's bins, but the pair-tile kernel takes it
     hipFunction_t ExchangeFunction = nullptr;  // nullptr: the model does not qualify
-    const char* ExchangeName = "";
+    std::string ExchangeName;
     TDeviceVec<uint32_t> FusedExchangeWaves, FusedExchangeTiles, FusedExchangeOneHot;  // its form that makes the bins from flat rows
     uint32_t FusedExchangeTileCount = 0;
     hipFunction_t FusedExchangeFunction = nullptr;
@@ -2180,12 +2212,6 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     m.FirstLeaf.Upload(firstLeaf);
     m.StepNodes.Upload(steps);
     m.NodeToLeaf.Upload(trees.NonSymmetricNodeIdToLeafId);
-    {
-        // the tile kernel copies (1 << 8) * dim doubles per tree: keep that much readable behind the end
-        std::vector<double> padded = trees.LeafValues;
-        padded.resize(padded.size() + 256 * static_cast<size_t>(trees.ApproxDimension), 0.0);
-        m.Leaves.Upload(padded);
-    }
     m.Bias.Upload(trees.Bias);
 
     // How unevenly a level splits the documents, 0 (two halves) to 0.5, estimated from the rank of its border among the feature's borders
@@ -2195,6 +2221,70 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         const bool oneHot = (flags[rb.FeatureIndex] & dev::kBucketFlagOneHot) != 0 || rb.XorMask != 0;
         const double share = oneHot ? 0.05 : static_cast<double>(rb.SplitIdx) / (n + 1.0);
         return switches.LevelOrder ? std::fabs(share - 0.5) : 0.0;
+    };
+
+    // Order of a tree's levels in the tables of the register and small-batch kernels (levelOrder[t][position] = level of the
+    // model). The leaf gathers of a wave meet in the LDS banks that the low bits of the leaf indexes choose; lanes with the
+    // same index share one access, lanes that differ only in high bits wait for each other. So the levels
+    // that split the documents most evenly go to the low bits and the lopsided ones, on which most lanes
+    // agree, to the high bits: fewer lanes of a bank then differ. The sums and their order do not change.
+    std::vector<std::array<uint8_t, kRegMaxDepth>> levelOrder;
+    if (m.Oblivious && m.MaxDepth <= kRegMaxDepth) {
+        levelOrder.resize(TreeCount);
+        for (size_t t = 0; t < TreeCount; ++t) {
+            double keys[kRegMaxDepth];
+            for (int d = 0; d < trees.TreeSizes[t]; ++d) {
+                const double key = lopsidedness(trees.RepackedBins[trees.TreeStartOffsets[t] + d]);
+                int at = d;
+                for (; at > 0 && key < keys[at - 1]; --at) {
+                    keys[at] = keys[at - 1];
+                    levelOrder[t][at] = levelOrder[t][at - 1];
+                }
+                keys[at] = key;
+                levelOrder[t][at] = static_cast<uint8_t>(d);
+            }
+        }
+    }
+
+    // Leaf values in other layouts are copied by a kernel from those on the device, when all tables stand (PlaceLeavesKernel).
+    std::vector<dev::TLeafRow> leafRows;
+    std::vector<std::pair<double*, size_t>> leafCopies;  // where, and how many rows of leafRows up to there
+    const auto placeLeaves = [&](TDeviceVec<double>* to, size_t size) {  // leafRows has got the rows
+        to->Reserve(std::max<size_t>(size, 1));
+        leafCopies.emplace_back(to->Get(), leafRows.size());
+    };
+
+    TExchangeTables exchangeTables;
+    std::future<void> exchangeBuilt;
+    const auto finishExchange = [&] {
+        exchangeBuilt.get();
+        const TExchangeTables& x = exchangeTables;
+        if (!x.Planned) {
+            return;
+        }
+        const std::string shape = std::string(x.MaxDepth == 6 ? "d6" : "d8") + (x.Six ? "_s" : "");
+        if (x.Tiled) {
+            m.FusedExchangeWaves.Upload(x.Plan.FusedWaveTable);
+            m.FusedExchangeTiles.Upload(x.Tiles);
+            m.FusedExchangeOneHot.Upload(x.OneHot);
+            m.FusedExchangeTileCount = static_cast<uint32_t>(x.Pieces.size()) / kExchangeTilePieces;
+            m.FusedExchangeName = "cbamd_fused_exchange_" + shape;
+            HIP_CHECK(hipModuleGetFunction(&m.FusedExchangeFunction, SharedRegModule(kEvalRegCodeObject), m.FusedExchangeName.c_str()));
+        }
+        m.ExchangeRounds = x.Plan.Rounds;
+        m.ExchangeWaves.Upload(x.Plan.WaveTable);
+        m.ExchangeRecords.Upload(x.Plan.Records);
+        m.ExchangeExtra.Upload(x.Plan.ExtraRows);
+        const size_t pitch = size_t(1) << x.MaxDepth;
+        for (size_t r = 0; r < x.Plan.LeafRows.size(); ++r) {
+            const TExchangeLeafRow& row = x.Plan.LeafRows[r];
+            const bool tree = row.Tree != kExchangeNoTree;
+            leafRows.push_back({r * pitch, tree ? firstLeaf[row.Tree] : 0u, row.Levels, tree ? static_cast<uint32_t>(pitch) : 0u,
+                                static_cast<uint32_t>(pitch)});
+        }
+        placeLeaves(&m.ExchangeLeaves, x.Plan.LeafRows.size() * pitch);
+        m.ExchangeName = "cbamd_eval_exchange_" + shape;
+        HIP_CHECK(hipModuleGetFunction(&m.ExchangeFunction, SharedRegModule(kEvalRegCodeObject), m.ExchangeName.c_str()));
     };
 
     // The kernels that keep a tree's row in registers (two trees per wave on half a tile, one on a whole tile)
@@ -2372,12 +2462,12 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             if (!m.TileFits()) {
                 const size_t pitch = m.MaxDepth <= 6 ? 64 : 256;
                 // zeros at the end: the pair-tile and quad-tile kernels fetch ahead of their trees without a bound
-                std::vector<double> fixed((trees.GetTreeCount() + dev::kQuadTreePadding) * pitch, 0.0);
-                for (size_t t = 0; t < trees.GetTreeCount(); ++t) {
-                    std::copy_n(trees.LeafValues.begin() + trees.TreeFirstLeafOffsets[t], size_t(1) << trees.TreeSizes[t],
-                                fixed.begin() + t * pitch);
+                const size_t rowCount = trees.GetTreeCount() + dev::kQuadTreePadding;
+                for (size_t t = 0; t < rowCount; ++t) {
+                    leafRows.push_back({t * pitch, t < TreeCount ? firstLeaf[t] : 0u, dev::kLeafRowInOrder,
+                                        t < TreeCount ? 1u << trees.TreeSizes[t] : 0u, static_cast<uint32_t>(pitch)});
                 }
-                m.HalfTileLeaves.Upload(fixed);
+                placeLeaves(&m.HalfTileLeaves, rowCount * pitch);
                 // two trees per wave: every bin of the tile's rows below 128 (the one-hot test then fits 7 bits too)
                 const int maxd = m.MaxDepth <= 6 ? 6 : 8;
                 const bool pairFits = PairTileLdsBytes(tileRowCount, 8) <= kMaxTileLdsBytes;
@@ -2389,18 +2479,21 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                         m.PairSix = m.MaxBucketValues <= 63 && !tileRowsSplit && switches.RegSix;
                         m.PairRows.Upload(pairTileRows(m.PairSix));
                         if (switches.Exchange && !tileRowsSplit) {
-                            std::vector<TExchangeTree> levels(trees.GetTreeCount());
-                            for (size_t t = 0; t < levels.size(); ++t) {
-                                levels[t].Leaves = trees.LeafValues.data() + trees.TreeFirstLeafOffsets[t];
+                            TExchangeTables& x = exchangeTables;
+                            x.BucketCount = m.LayoutBuckets;
+                            x.MaxDepth = static_cast<uint32_t>(maxd);
+                            x.Six = m.PairSix;
+                            x.Trees.resize(trees.GetTreeCount());
+                            for (size_t t = 0; t < x.Trees.size(); ++t) {
+                                x.Trees[t].Levels.reserve(trees.TreeSizes[t]);
                                 for (int d = 0; d < trees.TreeSizes[t]; ++d) {
                                     const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + d];
                                     const TTileLevel level = tileLevelOf(rb);
-                                    levels[t].Levels.push_back({level.Row, level.Add & 0xffu, level.Xor, level.IsXor, lopsidedness(rb)});
+                                    x.Trees[t].Levels.push_back({level.Row, level.Add & 0xffu, level.Xor, level.IsXor, static_cast<float>(lopsidedness(rb))});
                                 }
                             }
                             // The fused form: the model's columns in pieces of four neighbouring ones, sixteen pieces a tile. A
                             // piece that would leave the row is moved back over its neighbour.
-                            std::vector<uint32_t> columnOf, pieces, tileTable, oneHotTable;
                             bool tiled = switches.Fused && m.CtrCount == 0 && m.BinarizeBuckets == BucketCount && BucketCount > 0 &&
                                          m.FlatVectorSize >= kExchangePieceColumns;
                             std::vector<std::pair<uint32_t, uint32_t>> byColumn;
@@ -2409,52 +2502,30 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                                 tiled = (flags[b] & dev::kBucketFlagNanToInf) == 0 && offsets[b + 1] > offsets[b];
                             }
                             std::sort(byColumn.begin(), byColumn.end());
-                            columnOf.assign(m.LayoutBuckets, kExchangeNoColumn);
+                            x.ColumnOf.assign(m.LayoutBuckets, kExchangeNoColumn);
                             for (size_t i = 0; tiled && i < byColumn.size(); ++i) {
                                 const uint32_t column = byColumn[i].first;
-                                if (pieces.empty() || column * 4 >= pieces.back() + 4 * kExchangePieceColumns) {
-                                    pieces.push_back(4 * std::min<uint32_t>(column & ~3u, static_cast<uint32_t>(m.FlatVectorSize) - kExchangePieceColumns));
+                                if (x.Pieces.empty() || column * 4 >= x.Pieces.back() + 4 * kExchangePieceColumns) {
+                                    x.Pieces.push_back(4 * std::min<uint32_t>(column & ~3u, static_cast<uint32_t>(m.FlatVectorSize) - kExchangePieceColumns));
                                 }
-                                columnOf[byColumn[i].second] = static_cast<uint32_t>(pieces.size() - 1) * kExchangePieceColumns + column - pieces.back() / 4;
-                                tiled = (i == 0 || column != byColumn[i - 1].first) && pieces.size() <= kExchangeTiles * kExchangeTilePieces;
+                                x.ColumnOf[byColumn[i].second] = static_cast<uint32_t>(x.Pieces.size() - 1) * kExchangePieceColumns + column - x.Pieces.back() / 4;
+                                tiled = (i == 0 || column != byColumn[i - 1].first) && x.Pieces.size() <= kExchangeTiles * kExchangeTilePieces;
                             }
                             if (tiled) {
-                                pieces.resize((pieces.size() + kExchangeTilePieces - 1) / kExchangeTilePieces * kExchangeTilePieces, 0);
-                                std::vector<TExchangeColumn> columns(pieces.size() * kExchangePieceColumns);
+                                x.Pieces.resize((x.Pieces.size() + kExchangeTilePieces - 1) / kExchangeTilePieces * kExchangeTilePieces, 0);
+                                x.Columns.resize(x.Pieces.size() * kExchangePieceColumns);
                                 for (uint32_t b = 0; b < BucketCount; ++b) {
-                                    TExchangeColumn& column = columns[columnOf[b]];
+                                    TExchangeColumn& column = x.Columns[x.ColumnOf[b]];
                                     column.Used = true;
                                     column.OneHot = (flags[b] & dev::kBucketFlagOneHot) != 0;
                                     column.RowByte = srcFlat[b] * 4;
                                     column.Values.assign(values.begin() + offsets[b], values.begin() + offsets[b + 1]);
-                                    if (!column.OneHot) {
-                                        MakeExchangeGrid(m.PairSix, &column);
-                                    }
                                 }
-                                tiled = BuildExchangeTiles(columns, pieces, m.PairSix, &tileTable, &oneHotTable);
+                            } else {
+                                x.ColumnOf.clear();
                             }
-                            if (!tiled) {
-                                columnOf.clear();
-                            }
-                            TExchangePlan plan;
-                            if (BuildExchangePlan(levels, m.LayoutBuckets, static_cast<uint32_t>(maxd), m.PairSix, columnOf, &plan)) {
-                                if (tiled) {
-                                    m.FusedExchangeWaves.Upload(plan.FusedWaveTable);
-                                    m.FusedExchangeTiles.Upload(tileTable);
-                                    m.FusedExchangeOneHot.Upload(oneHotTable);
-                                    m.FusedExchangeTileCount = static_cast<uint32_t>(pieces.size()) / kExchangeTilePieces;
-                                    m.FusedExchangeName = std::string("cbamd_fused_exchange_d") + (maxd == 6 ? "6" : "8") + (m.PairSix ? "_s" : "");
-                                    HIP_CHECK(hipModuleGetFunction(&m.FusedExchangeFunction, SharedRegModule(kEvalRegCodeObject), m.FusedExchangeName.c_str()));
-                                }
-                                m.ExchangeRounds = plan.Rounds;
-                                m.ExchangeWaves.Upload(plan.WaveTable);
-                                m.ExchangeRecords.Upload(plan.Records);
-                                m.ExchangeExtra.Upload(plan.ExtraRows);
-                                m.ExchangeLeaves.Upload(plan.Leaves);
-                                m.ExchangeName = maxd == 6 ? (m.PairSix ? "cbamd_eval_exchange_d6_s" : "cbamd_eval_exchange_d6")
-                                                           : (m.PairSix ? "cbamd_eval_exchange_d8_s" : "cbamd_eval_exchange_d8");
-                                HIP_CHECK(hipModuleGetFunction(&m.ExchangeFunction, SharedRegModule(kEvalRegCodeObject), m.ExchangeName));
-                            }
+                            // (run by get() where there is no thread to be had)
+                            exchangeBuilt = std::async(std::launch::async | std::launch::deferred, [&x] { x.Build(); });
                         }
                     } else {
                         m.QuadRows.Upload(rowsInRegisters(64));
@@ -2650,24 +2721,6 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         std::vector<uint32_t> rows(std::max(tableTrees, tailTableTrees) * rowDwords, 0);
         std::vector<double> leaves((tailVariant ? launches - 1 : launches) * m.RegLaunchLeaves, 0.0);
         std::vector<double> tailLeaves(tailVariant ? tailTableTrees * rowsPerTree * tailPitch : 0, 0.0);
-        // Order of a tree's levels in these tables (levelOrder[t][position] = level of the model). The leaf
-        // gathers of a wave meet in the LDS banks that the low bits of the leaf indexes choose; lanes with the
-        // same index share one access, lanes that differ only in high bits wait for each other. So the levels
-        // that split the documents most evenly go to the low bits and the lopsided ones, on which most lanes
-        // agree, to the high bits: fewer lanes of a bank then differ. The sums and their order do not change.
-        std::vector<std::vector<int>> levelOrder(TreeCount);
-        for (size_t t = 0; t < TreeCount; ++t) {
-            const int depth = trees.TreeSizes[t];
-            std::vector<std::pair<double, int>> lopsided;
-            for (int d = 0; d < depth; ++d) {
-                lopsided.emplace_back(lopsidedness(trees.RepackedBins[trees.TreeStartOffsets[t] + d]), d);
-            }
-            std::stable_sort(lopsided.begin(), lopsided.end(),
-                             [](const auto& a, const auto& b) { return a.first < b.first; });
-            for (const auto& item : lopsided) {
-                levelOrder[t].push_back(item.second);
-            }
-        }
         // The register of a level's bins and the split index there: a float bucket that takes two registers answers
         // "bin >= s" in the first for s <= 127 and as "bin - 127 >= s - 127" in the second.
         const auto registerOf = [&](const TRepackedBin& rb) -> std::pair<uint32_t, uint32_t> {
@@ -3081,8 +3134,6 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         // Sixteen documents of a tree read its leaf values together, from as many lines of 128 bytes as the high bits of their indexes
         // differ: the lopsided levels, on which most documents agree, go there (6.9 lines -> 5.2 at depth 8). 1000 trees of depth 8,
         // SmallBatchKernel for 4096 documents 12.5 -> 11.2 us, 16 384 38.7 -> 33.7; of depth 6 25.0 -> 24.0.
-        std::vector<double> smallLeaves(trees.LeafValues);
-        smallLeaves.resize(smallLeaves.size() + 256 * static_cast<size_t>(trees.ApproxDimension), 0.0);
         const uint32_t never = 0x7f800000u;
         bool usable = trees.LeafValues.size() < (size_t(1) << 32);
         for (size_t place = 0; place < order.size() && usable; ++place) {
@@ -3092,28 +3143,12 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             if (t < TreeCount) {
                 first[place] = static_cast<uint32_t>(trees.TreeFirstLeafOffsets[t]);
             }
-            std::vector<std::pair<double, int>> levels;
-            for (int d = 0; d < depth; ++d) {
-                levels.emplace_back(lopsidedness(trees.RepackedBins[trees.TreeStartOffsets[t] + d]), d);
-            }
-            std::stable_sort(levels.begin(), levels.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
-            if (t < TreeCount) {
-                const size_t treeAt = trees.TreeFirstLeafOffsets[t], dim = static_cast<size_t>(m.Dim);
-                uint32_t leafOf[256] = {};  // by the index in the order of the rows; this kernel's trees have up to eight levels
-                for (uint32_t index = 0; index < (1u << depth); ++index) {
-                    if (index != 0) {  // of the index without its lowest bit, and that bit's level
-                        leafOf[index] = leafOf[index & (index - 1)] | 1u << levels[__builtin_ctz(index)].second;
-                    }
-                    const double* leaf = trees.LeafValues.data() + treeAt + leafOf[index] * dim;
-                    std::copy(leaf, leaf + dim, smallLeaves.data() + treeAt + index * dim);
-                }
-            }
             for (int d = 0; d < 8; ++d) {
                 row[8 + d] = never;
                 if (d >= depth) {
                     continue;
                 }
-                const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + levels[d].second];
+                const auto& rb = trees.RepackedBins[trees.TreeStartOffsets[t] + levelOrder[t][d]];
                 const uint32_t b = rb.FeatureIndex, n = offsets[b + 1] - offsets[b];
                 // a damaged model may name a border that is not there: such a split stays with the kernels on bins
                 const bool oneHot = (flags[b] & dev::kBucketFlagOneHot) != 0;
@@ -3154,10 +3189,42 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             m.SmallFirstLeafAt = table.size();
             table.insert(table.end(), first.begin(), first.end());
             m.SmallTable.Upload(table);
-            m.SmallLeaves.Upload(smallLeaves);
+            for (size_t t = 0; t < TreeCount; ++t) {
+                uint32_t levels = ~0u;
+                for (int d = 0; d < trees.TreeSizes[t]; ++d) {
+                    levels ^= (dev::kLeafRowNoLevel ^ levelOrder[t][d]) << 4 * d;
+                }
+                leafRows.push_back({firstLeaf[t], firstLeaf[t], levels, 1u << trees.TreeSizes[t], 1u << trees.TreeSizes[t]});
+            }
+            leafRows.push_back({trees.LeafValues.size(), 0u, ~0u, 0u, 256u});  // null trees' values
+            placeLeaves(&m.SmallLeaves, trees.LeafValues.size() + 256 * static_cast<size_t>(trees.ApproxDimension));
             m.SmallCellCount = static_cast<uint32_t>(cells.size());
             m.SmallUsable = true;
         }
+    }
+
+    {
+        // the tile kernel copies (1 << 8) * dim doubles per tree: keep that much readable behind the end
+        std::vector<double> padded;
+        padded.reserve(trees.LeafValues.size() + 256 * static_cast<size_t>(trees.ApproxDimension));
+        padded = trees.LeafValues;
+        padded.resize(padded.size() + 256 * static_cast<size_t>(trees.ApproxDimension), 0.0);
+        m.Leaves.Upload(padded);
+    }
+    if (exchangeBuilt.valid()) {
+        finishExchange();
+    }
+    if (!leafCopies.empty()) {
+        TDeviceVec<dev::TLeafRow> rows;
+        rows.Upload(leafRows);
+        size_t first = 0;
+        for (const auto& [to, end] : leafCopies) {
+            hipLaunchKernelGGL(dev::PlaceLeavesKernel, dim3(static_cast<uint32_t>(end - first)), dim3(64), 0, m.Stream, rows.Get() + first,
+                               static_cast<uint32_t>(m.Dim), static_cast<const double*>(m.Leaves.Get()), to);
+            HIP_CHECK(hipGetLastError());
+            first = end;
+        }
+        HIP_CHECK(hipStreamSynchronize(m.Stream));
     }
 }
 
@@ -4146,9 +4213,10 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
         evaluate = "EvalObliviousQuadTileKernel";
     } else if (m.Oblivious && m.MaxDepth <= 8 && m.Dim == 1 && m.HalfTileLeaves.Get() != nullptr &&
                !m.TileFits() && HalfTileLdsBytes(m.LayoutBuckets, 8) <= kMaxTileLdsBytes) {
-        evaluate = m.TakesExchangeKernel(docCount) ? m.ExchangeName
-                   : m.PairRows.Get() != nullptr   ? "EvalObliviousPairTileKernel"
-                                                   : "EvalObliviousHalfTileKernel";
+        evaluate = m.PairRows.Get() != nullptr ? "EvalObliviousPairTileKernel" : "EvalObliviousHalfTileKernel";
+        if (m.TakesExchangeKernel(docCount)) {
+            evaluate = m.ExchangeName;
+        }
     } else if (m.DeepRows.Get() != nullptr) {
         evaluate = "EvalObliviousDeepTileKernel";
     } else if (m.Oblivious) {

@@ -3500,6 +3500,35 @@ __global__ __launch_bounds__(64) void ApplyPredictionTypeManyKernel(int type, ui
     ForEachInTurns(r, dim, [&](uint32_t k, double v) { o[k] = FastExpAt(c, v - top, k, dim) / sum; });
 }
 
+// Leaf values of a model in another layout, a workgroup per row: what other kernels' tables of them are made of, once per model. On the
+// host each table was a second pass over the leaves and a transfer of them: building an evaluator of 1000 trees of depth 8 over 200
+// features (one such table) 3.25 -> 2.45 ms, of 2000 of depth 6 and ten dimensions 7.7 -> 5.9.
+struct TLeafRow {
+    uint64_t Destination;  // of its first value, in values
+    uint32_t Source;       // of the tree's first value
+    uint32_t Levels;       // four bits per bit of the row's index: the bit of the tree's leaf index that it is, or kLeafRowNoLevel
+    uint32_t Leaves;       // of the row that are the tree's, the others are zeros
+    uint32_t Pitch;        // leaves of the row
+};
+constexpr uint32_t kLeafRowNoLevel = 15, kLeafRowInOrder = 0x76543210u;
+
+__global__ __launch_bounds__(64) void PlaceLeavesKernel(const TLeafRow* __restrict__ rows, uint32_t dim, const double* __restrict__ leaves,
+                                                        double* __restrict__ out) {
+    const TLeafRow row = rows[blockIdx.x];
+    for (uint32_t leaf = threadIdx.x; leaf < row.Pitch; leaf += 64) {
+        uint32_t from = 0;
+#pragma unroll
+        for (uint32_t bit = 0; bit < 8; ++bit) {
+            const uint32_t level = row.Levels >> 4 * bit & 15;
+            from |= level != kLeafRowNoLevel ? (leaf >> bit & 1) << level : 0u;
+        }
+        for (uint32_t k = 0; k < dim; ++k) {
+            out[row.Destination + static_cast<size_t>(leaf) * dim + k] =
+                leaf < row.Leaves ? leaves[row.Source + static_cast<size_t>(from) * dim + k] : 0.0;
+        }
+    }
+}
+
 __global__ void FillBiasKernel(double* __restrict__ out, size_t count, const double* __restrict__ bias, int dim) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < count) {

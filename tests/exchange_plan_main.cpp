@@ -33,7 +33,6 @@ int main(int argc, char** argv) {
             in >> value;
             leaves[t].push_back(value);
         }
-        trees[t].Leaves = leaves[t].data();
     }
     std::vector<cbamd::TExchangeColumn> columns;
     std::vector<uint32_t> pieces(tiled * cbamd::kExchangeTilePieces);
@@ -68,8 +67,15 @@ int main(int argc, char** argv) {
         }
         std::printf("\n");
     }
-    for (double v : plan.Leaves) {
-        std::printf("%.17g ", v);
+    for (const cbamd::TExchangeLeafRow& row : plan.LeafRows) {
+        for (uint32_t i = 0; i < 1u << maxDepth; ++i) {
+            uint32_t leaf = 0;
+            for (uint32_t bit = 0; bit < 8; ++bit) {
+                const uint32_t level = row.Levels >> 4 * bit & 15;
+                leaf |= level != cbamd::kExchangeNoLevel ? (i >> bit & 1) << level : 0;
+            }
+            std::printf("%.17g ", row.Tree != cbamd::kExchangeNoTree ? leaves[row.Tree][leaf] : 0.0);
+        }
     }
     std::printf("\n");
     std::vector<uint32_t> table, oneHot;
