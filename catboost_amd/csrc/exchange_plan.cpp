@@ -358,6 +358,7 @@ bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketC
     std::vector<std::vector<uint32_t>> freedAfter(plan->Rounds);
     std::vector<size_t> next(kExchangeWaves, 0);
     const int64_t rounds = plan->Rounds;
+    plan->CompareSteps = 0;
     for (int64_t phase = -1; phase < rounds; ++phase) {
         std::vector<std::vector<uint32_t>> now(kExchangeWaves);
         const auto nextRound = [&](uint32_t w) {  // first round that needs the wave's next group
@@ -388,6 +389,12 @@ bool BuildExchangePlan(const std::vector<TExchangeTree>& trees, uint32_t bucketC
                 }
             }
         }
+        size_t busiest = 0, together = 0;
+        for (const std::vector<uint32_t>& groupsNow : now) {
+            busiest = std::max(busiest, groupsNow.size());
+            together += groupsNow.size();
+        }
+        plan->CompareSteps += static_cast<uint32_t>(phase < 0 ? busiest - together / kExchangeWaves : std::max<size_t>(busiest, stepCount));
         for (uint32_t w = 0; w < kExchangeWaves; ++w) {
             for (size_t i = 0; i < now[w].size(); ++i) {
                 (phase < 0 ? early[w] : groupsAt[(firstStep + i % stepCount) * kExchangeWaves + w]).push_back(now[w][i]);

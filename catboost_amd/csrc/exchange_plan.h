@@ -60,6 +60,8 @@ struct TExchangeLeafRow {
 
 struct TExchangePlan {
     uint32_t Rounds = 0;
+    uint32_t CompareSteps = 0;        // the rounds' steps and what the wave with the most groups of a round compares beyond them: a
+                                      // bucket's levels are all its wave's, so a model that looks at few buckets most takes longer
     std::vector<uint32_t> WaveTable;  // [wave][kExchangeWaveDwords]
     std::vector<uint32_t> FusedWaveTable;  // the same with the registers' columns in the buffer for the buckets' offsets
     std::vector<uint32_t> Records;    // [round + 1][wave][kExchangeRecordDwords]: rows are fetched ahead

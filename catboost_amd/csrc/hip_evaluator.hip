@@ -1615,6 +1615,8 @@ struct THipEvaluator::TImpl {
     TDeviceVec<uint32_t> ExchangeWaves, ExchangeRecords, ExchangeExtra;  // exchange kernel (exchange_plan.h)
     TDeviceVec<double> ExchangeLeaves;
     uint32_t ExchangeRounds = 0;
+    double ExchangeGeneration = 0.0;   // how many generations of the pair-tile kernel's workgroups one of its own lasts
+    bool FusedExchangeBalanced = false;  // few enough levels look at the same buckets for the fused form
     bool PairBeforeTile = false;       // the tile kernel would hold the model's bins, but the pair-tile kernel takes it
     hipFunction_t ExchangeFunction = nullptr;  // nullptr: the model does not qualify
     std::string ExchangeName;
@@ -1763,7 +1765,7 @@ struct THipEvaluator::TImpl {
         }
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
         const size_t generations = (blocks + CuCount - 1) / CuCount, others = (2 * blocks + CuCount - 1) / CuCount;
-        return generations * (MaxDepth <= 6 ? 36 : 29) < others * 20;
+        return static_cast<double>(generations) * ExchangeGeneration < static_cast<double>(others);
     }
 
     // The fused form instead of a binarize launch and either kernel. A generation of its workgroups takes some 50 us longer (per 1000
@@ -1773,8 +1775,25 @@ struct THipEvaluator::TImpl {
     // 181 -> 190; 0.77 (50 000) 96 -> 89 and 251 -> 247; 0.99 (130 000) 234 -> 192 and 525 -> 484.
     bool TakesFusedExchangeKernel(size_t docCount) const {
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
-        return FusedExchangeFunction != nullptr && docCount < (size_t(1) << 32) &&
+        return FusedExchangeFunction != nullptr && FusedExchangeBalanced && docCount < (size_t(1) << 32) &&
                blocks * 10 >= (blocks + CuCount - 1) / CuCount * CuCount * 7;
+    }
+
+    // What a model's levels on few buckets cost the exchange kernels. A CU's walk over 256 documents takes, in us, 11 and 0.0335 per tree
+    // of depth 7 or 8 (13 and 0.021 up to 6), the pair-tile kernel's two 17 and 0.047 (18 and 0.021). When the busiest waves have `turns`
+    // groups to compare for a step, it takes 8 and 0.0188 (0.0165) * turns per tree, where that is more. Whole calls for 1M
+    // documents, binarize and pair-tile launches, binarize and exchange, fused, by the share of the levels on one bucket (and turns): 2000 trees of
+    // depth 8 over 1016 features, 10 % (1.9) 2708, 2305, 2076 us; 16 % (2.7) 2717, 2687, 2483; 20 % (3.3) 2733, 3018, 2778; 30 % (4.7)
+    // 2714, 3832, 3572; 2000 of depth 6 over 700, 7 % (1.5) 1672, 1603, 1412; 10 % (2.0) 1665, 1687, 1590; 13 % (2.4) 1686, 1844, 1836; 500 of
+    // depth 8 over 600, 30 % (4.2) 1246, 1254, 1087. The fused form saves more of a binarize launch than it takes itself, 19 us for 65 536
+    // documents of 1000 columns, whatever the walk does.
+    void SetExchangeCosts(size_t trees, double turns) {
+        const bool shallow = MaxDepth <= 6;
+        const double count = static_cast<double>(trees), even = shallow ? 13.0 + 0.021 * count : 11.0 + 0.0335 * count;
+        const double walk = std::max(even, 8.0 + (shallow ? 0.0165 : 0.0188) * turns * count);
+        const double pairs = shallow ? 18.0 + 0.021 * count : 17.0 + 0.047 * count;
+        ExchangeGeneration = (shallow ? 1.8 : 1.45) * walk / even;
+        FusedExchangeBalanced = walk - pairs <= 0.019 * LayoutBuckets;
     }
 
     TEvalExchangeArgs ExchangeArgs(size_t docCount, double* results) const {
@@ -2272,6 +2291,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             HIP_CHECK(hipModuleGetFunction(&m.FusedExchangeFunction, SharedRegModule(kEvalRegCodeObject), m.FusedExchangeName.c_str()));
         }
         m.ExchangeRounds = x.Plan.Rounds;
+        m.SetExchangeCosts(TreeCount, static_cast<double>(x.Plan.CompareSteps) / (x.Plan.Rounds * kExchangeRoundSteps));
         m.ExchangeWaves.Upload(x.Plan.WaveTable);
         m.ExchangeRecords.Upload(x.Plan.Records);
         m.ExchangeExtra.Upload(x.Plan.ExtraRows);

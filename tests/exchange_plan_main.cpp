@@ -7,7 +7,7 @@
 #include "../catboost_amd/csrc/exchange_plan.h"
 
 int main(int argc, char** argv) {
-    if (argc != 2) {
+    if (argc != 2 && argc != 3) {  // a second argument: only the steps of the rounds, and those with the busiest waves' groups
         return 2;
     }
     std::ifstream in(argv[1]);
@@ -58,6 +58,10 @@ int main(int argc, char** argv) {
     cbamd::TExchangePlan plan;
     if (!cbamd::BuildExchangePlan(trees, buckets, maxDepth, six != 0, columnOf, &plan)) {
         std::printf("refused\n");
+        return 0;
+    }
+    if (argc == 3) {
+        std::printf("%u %u\n", plan.Rounds * cbamd::kExchangeRoundSteps, plan.CompareSteps);
         return 0;
     }
     std::printf("%u\n", plan.Rounds);

@@ -727,3 +727,18 @@ def test_plan_of_a_large_model(planner, tmp_path):
     assert groups.max() <= 1.02 * groups.mean() and levels <= groups.sum() * 8 < levels + 16 * 8
     late = extra - wave_table.reshape(16, 80)[:, 65]           # more than one group in a step
     assert (late >= 0).all() and late.sum() < 0.03 * groups.sum()
+
+
+@pytest.mark.parametrize("trees,share,least,most", [
+    (2000, 0.0, 1.0, 1.4), (2000, 0.1, 1.5, 2.1), (2000, 0.3, 4.0, 5.2),
+    (60, 0.0, 0.75, 1.8), (60, 0.5, 5.0, 9.0),          # one round: all groups are compared before it, none behind its last step
+])
+def test_plan_says_how_much_longer_the_busiest_waves_compare(planner, tmp_path, trees, share, least, most):
+    """A bucket's levels are all compared by the wave that holds it: with `share` of them on one bucket, 16 * share of a wave's part."""
+    rng = np.random.default_rng(3)
+    model = [([(0 if rng.random() < share else int(rng.integers(0, 1000)), 60, False) for _ in range(8)], np.zeros(256))
+             for _ in range(trees)]
+    path = str(tmp_path / "model.txt")
+    _plan(planner, path, model, 1000, 8, True)
+    steps, compared = map(int, subprocess.check_output([planner, path, "steps"], text=True).split())
+    assert least <= compared / steps <= most

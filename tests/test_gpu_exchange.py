@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import catboost_amd as cb
+from oracle import model_builder as mb
 from oracle.oracle import OracleModel
 
 from .test_gpu_small_batch import _model_of_buckets
@@ -81,6 +82,40 @@ def test_exchange_kernel_gives_the_pair_tile_kernels_bits(buckets, cats, trees, 
     ranged = exchange.calc_flat(x[:33_000], tree_start=1, tree_end=trees)
     np.testing.assert_allclose(ranged[sample[sample < 33_000]],
                                OracleModel(model).calc(x[sample[sample < 33_000]], tree_start=1, tree_end=trees), rtol=1e-9, atol=1e-12)
+
+
+@pytest.mark.parametrize("share,depth,exchange", [(0.0, 8, True), (0.1, 8, True), (0.35, 8, False), (0.05, 6, True), (0.3, 6, False)])
+def test_models_that_look_at_one_bucket_most_keep_the_pair_tile_kernel(share, depth, exchange, monkeypatch):
+    """One wave compares all levels of a bucket, so the exchange kernels are slower than the pair-tile kernel when a bucket has too many of
+    them. The values are the same bits whatever kernel takes the batch."""
+    import torch
+
+    rng = np.random.default_rng(17)
+    buckets, trees, docs = 700, 600, 130_000
+    at = list(rng.permutation(buckets))
+    tree_list = []
+    for _ in range(trees):
+        columns = [0 if rng.random() < share else int(at.pop() if at else rng.integers(0, buckets)) for _ in range(depth)]
+        tree_list.append(([("float", c, float(np.float32(rng.integers(-30, 31) / 20))) for c in columns], rng.normal(size=1 << depth)))
+    model = mb.build_oblivious([mb.float_feature(f) for f in range(buckets)], [], 1, tree_list)
+    x = rng.normal(size=(docs, buckets)).astype(np.float32)
+    flat = torch.from_numpy(x).to("cuda:0")
+    results = []
+    for g in _evaluators(model, monkeypatch):
+        ev = g.evaluator()
+        kernels = ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)
+        if len(results) < 2 and exchange:
+            assert "exchange" in kernels.get("fused", kernels.get("evaluate"))
+            assert ("fused" in kernels) == (len(results) == 0)
+        else:
+            assert kernels["evaluate"] == "EvalObliviousPairTileKernel"
+        out = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), buckets), docs, out.data_ptr())
+        results.append(out)
+    assert torch.equal(results[0], results[2]) and torch.equal(results[1], results[2])
+    sample = rng.choice(docs, size=200, replace=False)
+    np.testing.assert_allclose(results[0].cpu().numpy()[sample], OracleModel(model).calc(x[sample]), rtol=1e-9, atol=1e-12)
 
 
 def test_empty_batches():
