@@ -1773,10 +1773,11 @@ struct THipEvaluator::TImpl {
     // two launches -> fused, by the share of the generations' places that have a workgroup: 0.50 (66 000 documents), 500 trees
     // 146 -> 150 us, 5000 trees 441 -> 457; 0.69 (90 000) 182 -> 168 and 469 -> 464, but 2000 trees of depth 5 over 700 features (pair-tile)
     // 181 -> 190; 0.77 (50 000) 96 -> 89 and 251 -> 247; 0.99 (130 000) 234 -> 192 and 525 -> 484.
-    bool TakesFusedExchangeKernel(size_t docCount) const {
+    // (anyBatchSize: also where the two launches are the faster)
+    bool TakesFusedExchangeKernel(size_t docCount, bool anyBatchSize) const {
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
-        return FusedExchangeFunction != nullptr && FusedExchangeBalanced && docCount < (size_t(1) << 32) &&
-               blocks * 10 >= (blocks + CuCount - 1) / CuCount * CuCount * 7;
+        return FusedExchangeFunction != nullptr && docCount < (size_t(1) << 32) &&
+               (anyBatchSize || (FusedExchangeBalanced && blocks * 10 >= (blocks + CuCount - 1) / CuCount * CuCount * 7));
     }
 
     // What a model's levels on few buckets cost the exchange kernels. A CU's walk over 256 documents takes, in us, 11 and 0.0335 per tree
@@ -4097,8 +4098,8 @@ int THipEvaluator::FusedLayoutFor(int layout, size_t stride, size_t docCount, si
     if (layoutIndex < 0 || docCount == 0) {
         return -1;
     }
-    if (layoutIndex == 0 && !anyBatchSize && treeStart == 0 && treeEnd == TreeCount && stride < (size_t(1) << 20) &&
-        m.TakesFusedExchangeKernel(docCount)) {
+    if (layoutIndex == 0 && treeStart == 0 && treeEnd == TreeCount && stride < (size_t(1) << 20) &&
+        m.TakesFusedExchangeKernel(docCount, anyBatchSize)) {
         return kFusedExchange;
     }
     if (!m.Fused[layoutIndex] || treeStart != 0 || treeEnd != TreeCount || docCount >= (size_t(1) << 29) ||

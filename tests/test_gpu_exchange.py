@@ -118,6 +118,44 @@ def test_models_that_look_at_one_bucket_most_keep_the_pair_tile_kernel(share, de
     np.testing.assert_allclose(results[0].cpu().numpy()[sample], OracleModel(model).calc(x[sample]), rtol=1e-9, atol=1e-12)
 
 
+def test_no_alloc_entry_point_takes_batches_beyond_its_buffer(monkeypatch):
+    """eval_data_no_alloc: a wide model of a fused kernel uses no bin buffer, so it is refused at no size, also where eval_data takes
+    two launches (few workgroups in the last generation, or no batch at all is faster fused); eager and replayed from a graph."""
+    import torch
+
+    model, _ = _model_of_buckets(np.random.default_rng(4), 700, 3, 320, 8, 1, 1)
+    fused, _, pair = _evaluators(model, monkeypatch)
+    ev = fused.evaluator()
+    limit = (32 << 20) // ev.quantized_bytes(256) * 256
+    docs = 70_001
+    assert limit < 50_000 and "fused" not in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)
+    x = torch.from_numpy(np.random.default_rng(5).normal(size=(docs, 700)).astype(np.float32)).to("cuda:0")
+    feats = ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), 700)
+    expected = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+    out = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    pair.evaluator().eval_data(feats, docs, expected.data_ptr())
+    for n in (limit, limit + 1, docs):
+        out.fill_(-1.0)
+        torch.cuda.synchronize()
+        ev.eval_data_no_alloc(feats, n, out.data_ptr())
+        ev.synchronize()
+        assert torch.equal(out[:n], expected[:n]) and bool((out[n:] == -1.0).all()), n
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ev.eval_data_no_alloc(feats, docs, out.data_ptr(), stream=torch.cuda.current_stream().cuda_stream)
+    for replay in range(3):
+        x.copy_(x.flip(0))
+        out.fill_(-1.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        pair.evaluator().eval_data(feats, docs, expected.data_ptr())
+        assert torch.equal(out, expected), replay
+    with pytest.raises(cb.CatBoostError, match="exceeds the fixed bin buffer"):
+        ev.eval_data_no_alloc(feats, docs, out.data_ptr(), tree_start=1)      # a range of the trees has no fused kernel
+
+
 def test_empty_batches():
     """No documents: every call returns without touching a buffer, null pointers among them."""
     import torch
