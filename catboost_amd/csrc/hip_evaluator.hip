@@ -494,7 +494,8 @@ void LaunchWithEnd(TKernel kernel, dim3 grid, dim3 block, size_t lds, hipStream_
     }
 }
 
-// The same for a kernel of the code object, `args` its argument block.
+// The same for a kernel of the code object, `args` its argument block. (gridX * threads has 32 bits, which a batch of less than 2^29
+// documents does not leave: 1024 threads for 256 documents at the most.)
 template <typename TArgs>
 void LaunchModuleWithEnd(hipFunction_t kernel, uint32_t gridX, uint32_t gridY, uint32_t threads, hipStream_t s, hipEvent_t end,
                          TArgs& args) {
@@ -1760,7 +1761,7 @@ struct THipEvaluator::TImpl {
     // 240 -> 170 us, 66 000 363 -> 334, 130 000 493 -> 351, 1M 3633 -> 2659; 2000 of depth 5 over 700: 50 000 documents 61 -> 52 us,
     // 130 000 124 -> 113, 1M 887 -> 810, but 66 000 88 -> 96 and 140 000 147 -> 155, which stay where they were.
     bool TakesExchangeKernel(size_t docCount) const {
-        if (ExchangeFunction == nullptr || docCount >= (size_t(1) << 32)) {
+        if (ExchangeFunction == nullptr || docCount >= (size_t(1) << 29)) {
             return false;
         }
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
@@ -1776,7 +1777,7 @@ struct THipEvaluator::TImpl {
     // (anyBatchSize: also where the two launches are the faster)
     bool TakesFusedExchangeKernel(size_t docCount, bool anyBatchSize) const {
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
-        return FusedExchangeFunction != nullptr && docCount < (size_t(1) << 32) &&
+        return FusedExchangeFunction != nullptr && docCount < (size_t(1) << 29) &&
                (anyBatchSize || (FusedExchangeBalanced && blocks * 10 >= (blocks + CuCount - 1) / CuCount * CuCount * 7));
     }
 
@@ -4348,9 +4349,12 @@ void THipEvaluator::ApplyPredictionTypeDevice(int predictionType, size_t firstDo
     c.Mantissa = m.ExpMantissa.Get();
     c.Scale = constants.Scale;
     c.InvScale = constants.InvScale;
-    CBAMD_ENSURE((docCount + 255) / 256 <= 0x7fffffffu, "too many documents in one batch");
-    const dim3 grid(static_cast<uint32_t>((docCount + 255) / 256));
-    const auto softmax = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, docCount, c, raw, result); };
+    const auto gridOf = [&](size_t threads) {
+        const size_t groups = (docCount + threads - 1) / threads;
+        CBAMD_ENSURE(groups <= 0x7fffffffu, "too many documents in one batch");
+        return dim3(static_cast<uint32_t>(groups));
+    };
+    const auto softmax = [&](auto kernel) { hipLaunchKernelGGL(kernel, gridOf(256), dim3(256), 0, s, docCount, c, raw, result); };
     const bool isSoftmax = predictionType == dev::kPredProbability && dim > 1;
     if (isSoftmax && dim <= 8) {
         switch (dim) {
@@ -4364,11 +4368,11 @@ void THipEvaluator::ApplyPredictionTypeDevice(int predictionType, size_t firstDo
         }
     } else if (isSoftmax || (predictionType == dev::kPredClass && dim >= dev::kManyDimsClass) ||
                (predictionType == dev::kPredMultiProbability && dim >= dev::kManyDimsMultiProbability)) {
-        hipLaunchKernelGGL(dev::ApplyPredictionTypeManyKernel, dim3(static_cast<uint32_t>((docCount + 63) / 64)), dim3(64), 0, s,
-                           predictionType, dim, firstDoc, totalDocs, docCount, c, raw, result);
+        hipLaunchKernelGGL(dev::ApplyPredictionTypeManyKernel, gridOf(64), dim3(64), 0, s, predictionType, dim, firstDoc,
+                           totalDocs, docCount, c, raw, result);
     } else {
-        hipLaunchKernelGGL(dev::ApplyPredictionTypeKernel, grid, dim3(256), 0, s, predictionType, dim, firstDoc, totalDocs, docCount, c,
-                           raw, result);
+        hipLaunchKernelGGL(dev::ApplyPredictionTypeKernel, gridOf(256), dim3(256), 0, s, predictionType, dim, firstDoc, totalDocs,
+                           docCount, c, raw, result);
     }
     HIP_CHECK(hipGetLastError());
 }

@@ -156,6 +156,28 @@ def test_no_alloc_entry_point_takes_batches_beyond_its_buffer(monkeypatch):
         ev.eval_data_no_alloc(feats, docs, out.data_ptr(), tree_start=1)      # a range of the trees has no fused kernel
 
 
+def test_batches_of_more_documents_than_a_launch_can_count():
+    """2^29 documents and more: the exchange kernels are not chosen (their launch counts work-items in 32 bits); prediction types whose kernel
+    has 64 documents a workgroup refuse what that grid cannot hold."""
+    import torch
+
+    model, _ = _model_of_buckets(np.random.default_rng(2), 700, 3, 201, 8, 1, 1)
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    for layout in (cb.LAYOUT_FLAT_ROWS, cb.LAYOUT_FLAT_COLUMNS):
+        assert "exchange" in str(ev.describe_kernels(layout, (1 << 29) - 1))
+        assert "exchange" not in str(ev.describe_kernels(layout, 1 << 29))
+    dims = cb.ModelCalcer()
+    dims.build_oblivious([dict(index=0, flat_index=0)], [], 9, [([("float", 0, 0.5)], [0.25] * 18)])
+    dims.enable_gpu_evaluation(0)
+    raw, result = torch.zeros(9, dtype=torch.float64, device="cuda:0"), torch.zeros(9, dtype=torch.float64, device="cuda:0")
+    for kind in (cb.APT_PROBABILITY, cb.APT_CLASS, cb.APT_MULTI_PROBABILITY):
+        with pytest.raises(cb.CatBoostError, match="too many documents"):
+            dims.evaluator().apply_prediction_type(kind, (1 << 37) + 64, raw.data_ptr(), result.data_ptr())
+
+
 def test_empty_batches():
     """No documents: every call returns without touching a buffer, null pointers among them."""
     import torch
