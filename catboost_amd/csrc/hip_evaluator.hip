@@ -809,6 +809,15 @@ size_t PairTileLdsBytes(uint32_t buckets, int maxd) {
            static_cast<size_t>(dev::kPairWaves) * std::max<size_t>(size_t(1) << maxd, 128) * sizeof(double);
 }
 
+// Trees from which the pair-tile kernel is the faster of it and the tile kernel where both could take a model of one dimension, by the
+// evaluate launch for 100 000 and 1M documents, tile and pair-tile: 625 buckets, ranges of 300 trees of depth 8 53 and 54, 431 and 456 us, 600
+// trees 89 and 82, 722 and 660; 100 of depth 6 28 and 27, 232 and 232, 200 39 and 32, 312 and 266. 620 buckets, one of more than 127 values,
+// 400 trees of depth 8 74 and 80, 606 and 631 us, 600 90 and 83, 715 and 656; 300 of these and 8000 trees 1011 and 791, 8040 and 6083.
+// (Up to 32 768 documents, a workgroup per CU, the pair-tile kernel is ahead with any number: 300 trees 28 and 17.)
+constexpr uint32_t PairTrees(uint32_t maxDepth) {
+    return maxDepth <= 6 ? 150 : 500;
+}
+
 // dimensions the tile kernel accumulates per pass over the trees (and the pitch of its padded leaf rows)
 int TileChunk(int dim) {
     return dim == 1 ? 1 : dim == 2 ? 2 : dim <= 4 ? 4 : dim <= 8 ? 8 : dim <= 12 ? 12 : 16;
@@ -1803,9 +1812,10 @@ struct THipEvaluator::TImpl {
                 static_cast<uint32_t>(docCount), ExchangeRounds, LayoutBuckets * dev::kDocsPerBlock, 0};
     }
 
-    // The tile kernel takes the model (of kernels on bins in an LDS tile of whole blocks, the one without a tree's row in registers).
-    bool TileFits() const {
-        return !PairBeforeTile && TileLdsBytes(LayoutBuckets, TileChunk(Dim)) <= kMaxTileLdsBytes;
+    // The tile kernel takes the model, or a range of its trees (of kernels on bins in an LDS tile of whole blocks, the one without a tree's
+    // row in registers).
+    bool TileFits(uint32_t rangeTrees = ~0u) const {
+        return (!PairBeforeTile || rangeTrees < PairTrees(MaxDepth)) && TileLdsBytes(LayoutBuckets, TileChunk(Dim)) <= kMaxTileLdsBytes;
     }
 
     int SmallDims() const { return Dim == 1 ? 1 : Dim == 2 ? 2 : 4; }
@@ -2477,10 +2487,12 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 }
             }
             m.PackedMixed.Upload(mixed);
-            // Some 577 to 632 buckets: the tile fits LDS, but not with the regions of the row-tile kernel. Two trees per wave on
-            // half a tile, or the exchange kernel, are the faster there.
+            // The tile fits LDS up to 632 buckets, but not with the regions of the row-tile kernel beyond 568 rows (trees of depth 7 and 8) or
+            // 616: two trees per wave on half a tile there, or the exchange kernel, if the model has trees enough or the latter takes its
+            // large batches (a bucket of more than 127 values keeps that off). Few trees on rows of their own: the tile kernel.
+            const bool fewTrees = TreeCount < PairTrees(m.MaxDepth);
             m.PairBeforeTile = switches.RowTile && switches.PairTile && PairTileLdsBytes(tileRowCount, 8) <= kMaxTileLdsBytes &&
-                               RowTileWaves(tileRowCount, m.MaxDepth, 1) == 0;
+                               RowTileWaves(tileRowCount, m.MaxDepth, 1) == 0 && !(fewTrees && tileRowsSplit);
             if (!m.TileFits()) {
                 const size_t pitch = m.MaxDepth <= 6 ? 64 : 256;
                 // zeros at the end: the pair-tile and quad-tile kernels fetch ahead of their trees without a bound
@@ -2555,6 +2567,15 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     m.TileRowCount = tileRowsSplit ? tileRowCount : m.LayoutBuckets;  // (a model without splits: its one zero bucket)
                     if (tileRowsSplit) {
                         m.TileMap.Upload(tileMap);
+                    }
+                }
+                if (fewTrees && m.PairBeforeTile && exchangeBuilt.valid()) {
+                    finishExchange();
+                    if (m.ExchangeFunction == nullptr || (m.ExchangeGeneration >= 2.0 && !m.FusedExchangeBalanced)) {
+                        m.PairBeforeTile = TileLdsBytes(m.LayoutBuckets, 1) > kMaxTileLdsBytes;
+                        if (!m.PairBeforeTile) {
+                            m.ExchangeFunction = m.FusedExchangeFunction = nullptr;  // their sums are not the tile kernel's
+                        }
                     }
                 }
             }
@@ -3752,7 +3773,7 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
         HIP_CHECK(hipGetLastError());
         return;
     }
-    if (m.Oblivious && m.MaxDepth <= 8 && m.TileFits()) {
+    if (m.Oblivious && m.MaxDepth <= 8 && m.TileFits(tb != 0 || te != TreeCount ? te - tb : ~0u)) {
         // byte-parallel kernel over an LDS tile of bins
         const TTileArgs args{bins, docCount, m.LayoutBuckets, m.PackedTrees.Get(),
                              m.Dim == 1 ? m.Leaves.Get() : m.LeavesPadded.Get(), m.Bias.Get(), m.Scale, m.Dim, tb, te,

@@ -118,6 +118,54 @@ def test_models_that_look_at_one_bucket_most_keep_the_pair_tile_kernel(share, de
     np.testing.assert_allclose(results[0].cpu().numpy()[sample], OracleModel(model).calc(x[sample]), rtol=1e-9, atol=1e-12)
 
 
+@pytest.mark.parametrize("buckets,trees,depth,first,share,kernel", [
+    (575, 499, 8, 200, 0.0, "EvalObliviousTileKernel"),       # a bucket of two rows: no exchange kernel
+    (575, 500, 8, 200, 0.0, "EvalObliviousPairTileKernel"),
+    (620, 149, 6, 200, 0.0, "EvalObliviousTileKernel"),
+    (620, 499, 7, 1, 0.0, "cbamd_eval_exchange_d8_s"),
+    (620, 300, 8, 1, 0.45, "EvalObliviousTileKernel"),        # too many levels on one bucket for the exchange kernels
+    (620, 500, 8, 1, 0.45, "EvalObliviousPairTileKernel"),
+    (700, 300, 8, 1, 0.45, "EvalObliviousPairTileKernel"),    # more buckets than the tile holds
+])
+def test_models_of_few_trees_keep_the_tile_kernel(buckets, trees, depth, first, share, kernel, monkeypatch):
+    """Models whose tile of 256 documents fits LDS without the row-tile kernel's regions. Whatever kernel takes the model, the same bits
+    at every batch size; ranges of few and of many trees."""
+    import torch
+
+    monkeypatch.setenv("CATBOOST_AMD_FUSED", "0")
+    rng = np.random.default_rng(trees)
+    model, _ = _model_of_buckets(rng, buckets, 0, trees, depth, 1, first)
+    if share:
+        at = list(rng.permutation(buckets))
+        model = mb.build_oblivious([mb.float_feature(f) for f in range(buckets)], [], 1, [
+            ([("float", 0 if rng.random() < share else int(at.pop() if at else rng.integers(0, buckets)),
+               float(np.float32(rng.integers(-20, 21) / 20))) for _ in range(depth)], rng.normal(size=1 << depth)) for _ in range(trees)])
+    g = cb.ModelCalcer()
+    g.load_from_dict(model)
+    g.enable_gpu_evaluation(0)
+    ev = g.evaluator()
+    docs = 66_000
+    assert ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"] == kernel
+    x = rng.normal(size=(docs, buckets)).astype(np.float32)
+    flat = torch.from_numpy(x).to("cuda:0")
+    feats = ev.features(cb.LAYOUT_FLAT_ROWS, flat.data_ptr(), buckets)
+    sample = rng.choice(3000, size=200, replace=False)
+    oracle = OracleModel(model)
+    whole = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+    out = torch.zeros(docs, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    ev.eval_data(feats, docs, whole.data_ptr())
+    np.testing.assert_allclose(whole.cpu().numpy()[sample], oracle.calc(x[sample]), rtol=1e-9, atol=1e-12)
+    for n in (100, 3000, 20_000, 40_000):
+        ev.eval_data(feats, n, out.data_ptr())
+        assert torch.equal(out[:n], whole[:n]), n
+    for tree_range in ((0, trees - 1), (1, trees), (5, 6), (7, 7), (0, trees // 3), (trees // 2, trees)):
+        for n in (3000, docs):
+            ev.eval_data(feats, n, out.data_ptr(), tree_start=tree_range[0], tree_end=tree_range[1])
+            np.testing.assert_allclose(out.cpu().numpy()[sample], oracle.calc(x[sample], tree_start=tree_range[0], tree_end=tree_range[1]),
+                                       rtol=1e-9, atol=1e-12)
+
+
 def test_no_alloc_entry_point_takes_batches_beyond_its_buffer(monkeypatch):
     """eval_data_no_alloc: a wide model of a fused kernel uses no bin buffer, so it is refused at no size, also where eval_data takes
     two launches (few workgroups in the last generation, or no batch at all is faster fused); eager and replayed from a graph."""
