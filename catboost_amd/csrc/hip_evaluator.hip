@@ -4012,8 +4012,11 @@ void THipEvaluator::EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCou
         LaunchModuleWithEnd(l.Function, grid, shares, 64 * l.Waves, s, nullptr, launchArgs);
     }
     const size_t count = docCount * m.Dim;
-    LaunchWithEnd(dev::CombineSlicesKernel, dim3(static_cast<uint32_t>((count + 63) / 64)), dim3(64), 0, s, TakeEnd(end),
-                  static_cast<const double*>(partials), slices, count, m.Scale, m.Bias.Get(), m.Dim, results);
+    const auto combine = [&](auto kernel) {
+        LaunchWithEnd(kernel, dim3(static_cast<uint32_t>((count + 63) / 64)), dim3(64), 0, s, TakeEnd(end),
+                      static_cast<const double*>(partials), slices, count, m.Scale, m.Bias.Get(), m.Dim, results);
+    };
+    slices <= dev::kFewSlices ? combine(dev::CombineSlicesKernel<3>) : combine(dev::CombineSlicesKernel<16>);
     HIP_CHECK(hipGetLastError());
 }
 

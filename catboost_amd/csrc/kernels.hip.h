@@ -729,13 +729,15 @@ __global__ __launch_bounds__(256) void EvalObliviousKernel(const uint32_t* __res
 
 // Small batches on the register-resident kernels: every slice of the trees left its raw sums in
 // partials[slice][count]; adds them in slice order and finishes like ApplyScaleAndBias. One thread per value.
-// What bounds it: the latency of the loads. A loop of load and add had one in flight; now sixteen are (a whole turn past the last
-// slice reads that one again), in workgroups of one wave, which a batch of 17 000 documents spreads over every CU. Evaluation
-// (register kernel and this one) of 1000 trees of depth 6, 32 slices: 17 000 documents 22.2 -> 16.1 us, 100 000 48.2 -> 43.6; of 500 trees
-// and three dimensions 21.8 -> 17.6 and 41.5 -> 39.4. Workgroups of four waves 16.3 and 43.9, 19.2 and 40.5; 32 loads 16.0 and 43.7, 18.3
-// and 40.7.
-constexpr uint32_t kCombineInFlight = 16;
+// What bounds it: the latency of the loads. A loop of load and add had one in flight; now IN_FLIGHT are (a whole turn past the last
+// slice reads that one again), in workgroups of one wave, which a batch of 17 000 documents spreads over every CU. Sixteen for many
+// slices; evaluation (register kernel and this one) of 1000 trees of depth 6, 32 slices: 17 000 documents 22.2 -> 16.1 us, 100 000 48.2 ->
+// 43.6; of 500 trees and three dimensions, 16 slices, 21.8 -> 17.6 and 41.5 -> 39.4. Workgroups of four waves 16.3 and 43.9, 19.2 and 40.5; 32
+// loads 16.0 and 43.7, 18.3 and 40.7. Three up to kFewSlices, where most of sixteen would be of the last slice; 200 000 documents, one in
+// flight, three, sixteen: two slices of three dimensions 22.1, 22.1, 25.0 us, four 31.2, 30.3, 32.3, ten of one 30.7, 29.6, 30.0.
+constexpr uint32_t kFewSlices = 10;
 
+template <uint32_t IN_FLIGHT>
 __global__ __launch_bounds__(64) void CombineSlicesKernel(const double* __restrict__ partials, uint32_t slices,
                                                            size_t count, double scale, const double* __restrict__ bias,
                                                            int dim, double* __restrict__ out) {
@@ -744,14 +746,14 @@ __global__ __launch_bounds__(64) void CombineSlicesKernel(const double* __restri
         return;
     }
     double sum = partials[i];
-    for (uint32_t first = 1; first < slices; first += kCombineInFlight) {
-        double part[kCombineInFlight];
+    for (uint32_t first = 1; first < slices; first += IN_FLIGHT) {
+        double part[IN_FLIGHT];
 #pragma unroll
-        for (uint32_t k = 0; k < kCombineInFlight; ++k) {
+        for (uint32_t k = 0; k < IN_FLIGHT; ++k) {
             part[k] = partials[min(first + k, slices - 1) * count + i];
         }
 #pragma unroll
-        for (uint32_t k = 0; k < kCombineInFlight; ++k) {
+        for (uint32_t k = 0; k < IN_FLIGHT; ++k) {
             if (first + k < slices) {
                 sum = __dadd_rn(sum, part[k]);
             }

@@ -550,3 +550,9 @@ def test_slices_are_added_in_order(trees, dim):
         ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, flat[begin:].data_ptr(), flat.shape[1]), 4000, part.data_ptr())
         assert torch.equal(part, out[begin * dim:(begin + 4000) * dim])
     assert bool((out[docs * dim:] == -3.0).all())
+
+
+@pytest.mark.parametrize("trees,dim", [(96, 1), (128, 3), (160, 1), (320, 2), (321, 1)])
+def test_few_slices_are_added_in_order(trees, dim):
+    """Three loads in flight up to ten slices: a turn that ends in the last slice's again, whole turns, the first number with sixteen."""
+    test_slices_are_added_in_order(trees, dim)
