@@ -19,8 +19,8 @@ LAYOUT_FLAT_ROWS, LAYOUT_FLAT_COLUMNS, LAYOUT_SPLIT_ROWS = range(3)
 
 _lib = None
 
-# pointers to rows and to results: an address (_address), or any ctypes pointer or array
-c_float_pp = c_int_pp = ctypes.c_void_p
+c_float_pp = ctypes.POINTER(ctypes.POINTER(ctypes.c_float))
+c_int_pp = ctypes.POINTER(ctypes.POINTER(ctypes.c_int))
 c_char_ppp = ctypes.POINTER(ctypes.POINTER(ctypes.c_char_p))
 
 
@@ -98,7 +98,7 @@ def load_library():
         except ImportError:
             pass
     lib = ctypes.CDLL(LIB_PATH)
-    vp, sz, dp = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p
+    vp, sz, dp = ctypes.c_void_p, ctypes.c_size_t, ctypes.POINTER(ctypes.c_double)
     sig = {
         "ModelCalcerCreate": (vp, []),
         "ModelCalcerDelete": (None, [vp]),
@@ -206,30 +206,41 @@ def integer_cat_feature_hash(v):
 
 
 def _address(array):
-    """Address of a C-contiguous numpy array's first element. (A call for one row takes some 18 us, of which `array.ctypes` for its
-    row, its row pointer and its result took 4.)"""
+    """Address of a C-contiguous numpy array's first element."""
     try:
         return ctypes.addressof(ctypes.c_char.from_buffer(array))
     except (TypeError, ValueError, BufferError):  # read-only or empty
         return array.ctypes.data
 
 
+# by numpy's code of a type: the C type and its pointer
+_C_TYPES = {np.dtype(t).char: (c, ctypes.POINTER(c)) for t, c in (
+    (np.float32, ctypes.c_float), (np.int32, ctypes.c_int), (np.float64, ctypes.c_double))}
+
+
+def _pointer(array):
+    """A C-contiguous numpy array's first element, as an argument of a call that takes a pointer to such elements. The array has to
+    outlive it. (A call for one row takes some 17 us, of which `array.ctypes` for its row, its row pointer and its result took 4.)"""
+    element, pointer = _C_TYPES[array.dtype.char]
+    try:
+        return element.from_buffer(array)
+    except (TypeError, ValueError, BufferError):  # read-only or empty
+        return ctypes.cast(array.ctypes.data, pointer)
+
+
 def _row_pointers(matrix):
     """Array of per-row pointers into a C-contiguous 2-D numpy array, as an argument of a call."""
     n = matrix.shape[0]
-    first = _address(matrix)
     if n <= 1:
-        return _OneRow(first)
-    stride = matrix.strides[0]
+        first = _pointer(matrix)
+        return ctypes.byref(first if isinstance(first, ctypes._Pointer) else ctypes.pointer(first))
+    first, stride = _address(matrix), matrix.strides[0]
     if stride == 0 or first + n * stride >= 1 << 63:
-        addresses = np.full(n, first, dtype=np.uint64)
+        addresses = np.uint64(first) + np.arange(n, dtype=np.uint64) * np.uint64(stride)
     else:
         addresses = np.arange(first, first + n * stride, stride, dtype=np.uint64)
     # the argument keeps the numpy buffer of addresses alive
-    return ctypes.byref(ctypes.c_char.from_buffer(addresses))
-
-
-_OneRow = ctypes.c_void_p * 1
+    return ctypes.byref(_C_TYPES[matrix.dtype.char][1].from_buffer(addresses))
 
 
 def fast_exp(values, chunk=None):
@@ -667,9 +678,7 @@ class ModelCalcer:
     def _result(self, doc_count):
         return np.zeros(doc_count * self.prediction_dimensions_count, dtype=np.float64)
 
-    @staticmethod
-    def _dp(a):
-        return _address(a)
+    _dp = staticmethod(_pointer)
 
     def calc_flat(self, features, tree_start=None, tree_end=None, result_size=None):
         """CalcModelPredictionFlat[Staged]: features[doc][flat feature index]."""
