@@ -629,10 +629,10 @@ TBucketGrid MakeBucketGrid(const std::vector<float>& borders) {
 
 constexpr size_t kMaxTileLdsBytes = 160 * 1024;
 
-// Batches of SmallBatchKernel and FewDocumentsKernel, in documents times passes over the dimensions; beyond, the binarize
-// and register kernels in slices of the trees are faster. Whole call, 1000 trees of depth 8 over 200 features: 8192
-// documents 29 us, 16384 42 against 38 on those (1000 trees of depth 6 32 against 33, 500 26 against 28, 300 of depth 4 25
-// against 26). FewDocumentsKernel against SmallBatchKernel: 512 documents 18 against 21 us, 1024 24 against 21.
+// Batches of SmallBatchKernel and FewDocumentsKernel, in documents times passes over the dimensions; beyond come the binarize
+// and register kernels in slices of the trees, which one limit cannot meet at every model's crossing. Whole call for 16384
+// documents against those: 1000 trees of depth 8 over 200 features 40.5 and 38.5 us (14336 documents 39, 12288 34, 8192 28), 1000 of depth 6
+// 32 and 33, 500 26 and 28, 300 of depth 4 25 and 26. FewDocumentsKernel against SmallBatchKernel: 512 documents 18 against 21 us, 1024 24 against 21.
 constexpr size_t kSmallBatchDocs = 16384;
 constexpr size_t kFewDocs = 640;
 // ... of host calls, whose features are at most so many bytes: more go through the pipeline of chunks
@@ -1741,6 +1741,7 @@ struct THipEvaluator::TImpl {
     bool SmallUsable = false;
     uint32_t SmallCellCount = 0;
     TDeviceVec<uint32_t> SmallTable;
+    TDeviceVec<dev::TLeafRow> LeafRows;  // of the copies of the leaf values (kept: to free them there would take 40 to 60 us)
     TDeviceVec<double> SmallLeaves;    // the leaf values, a tree's in the order of its levels in those rows
     size_t SmallCellsAt = 0, SmallFirstLeafAt = 0;
     // rows of the table without the null trees at its end, and those of a slice: a slice of the register kernels' (the whole
@@ -3258,11 +3259,10 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         finishExchange();
     }
     if (!leafCopies.empty()) {
-        TDeviceVec<dev::TLeafRow> rows;
-        rows.Upload(leafRows);
+        m.LeafRows.Upload(leafRows);
         size_t first = 0;
         for (const auto& [to, end] : leafCopies) {
-            hipLaunchKernelGGL(dev::PlaceLeavesKernel, dim3(static_cast<uint32_t>(end - first)), dim3(64), 0, m.Stream, rows.Get() + first,
+            hipLaunchKernelGGL(dev::PlaceLeavesKernel, dim3(static_cast<uint32_t>(end - first)), dim3(64), 0, m.Stream, m.LeafRows.Get() + first,
                                static_cast<uint32_t>(m.Dim), static_cast<const double*>(m.Leaves.Get()), to);
             HIP_CHECK(hipGetLastError());
             first = end;
