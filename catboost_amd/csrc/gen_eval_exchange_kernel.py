@@ -30,7 +30,7 @@ tree in four gathered from global memory 0.70. Some 13 us per workgroup go to it
 Fused variants ("cbamd_fused_exchange_...") take the documents' rows and make the bins themselves, tile by tile: a tile is sixteen
 *pieces* of four neighbouring columns (16 bytes of a row). A lane loads a piece of its four documents (sixteen lanes a row's
 pieces, so a load reads whole stretches of four rows), finds the bins as the other fused kernels do - cell of a grid of
-256, table of search starts, a branch-free search of 1 to 4 steps - with its columns' borders and start tables in LDS, and
+256 (six-bit form 512), table of search starts, a branch-free search of 1 to 4 steps - with its columns' borders and start tables in LDS, and
 writes a dword of four documents' bins per column to a buffer [column][lane] in LDS, from which every wave takes the four of its
 64 buckets that are in this tile. A tile's tables come straight into LDS while the tile before is searched, its rows
 likewise into registers. One-hot columns are made behind that, by a wave per column. The phase takes some 55 us per workgroup of
