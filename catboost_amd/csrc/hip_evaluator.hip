@@ -2560,7 +2560,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                                 x.ColumnOf.clear();
                             }
                             // (run by get() where there is no thread to be had)
-                            exchangeBuilt = std::async(std::launch::async | std::launch::deferred, [&x] { x.Build(); });
+                            exchangeBuilt = std::async(std::launch::async | std::launch::deferred, [&exchangeTables] { exchangeTables.Build(); });
                         }
                     } else {
                         m.QuadRows.Upload(rowsInRegisters(64));
