@@ -23,7 +23,18 @@ Layout of the work:
   * a tree's levels come from a table of 16 dwords per tree, (bucket, (128 - splitIdx) * 0x01010101)
     per level, read with one scalar load two trees ahead; kernels for LEAVES = 64 use the first six.
     Six-bit variants: the even levels' constant is (64 - splitIdx) * 0x01010101, which puts the level's
-    bit in bit 6 of every byte (all bins are at most 64), next to the following level's in bit 7.
+    bit in bit 6 of every byte (all bins are at most 64), next to the following level's in bit 7. The other
+    variants get it there with v_lerp_u8, (bin + constant) >> 1 for every byte from sums of nine bits.
+    A tree's eight sums come first, in index mode; behind them the mode is off, and the merges, the
+    product that turns indexes into places of leaf values and the sums of the tree before follow.
+    What bounds a tree is vector issue (and LDS with tables of 256 leaves): in index mode any
+    instruction takes its SIMD 1.8 ns, outside of it shifts to the right, ands and v_bitop3 of vector
+    registers take 0.9 (and 0.4 beside another wave's slow one), but v_bfi, v_lerp, SDWA, shifts to the
+    left, fp64 and whatever names a scalar register 1.8. Measured per tree, wave and SIMD with the
+    merges as v_bfi with a scalar mask in index mode and SDWA multiplications for the places, and now
+    (2M documents, 1024 trees, made-up tables): 200 registers, 256 leaves, six-bit 72.3 -> 69.8 ns, 64
+    leaves 58.1 -> 56; 128 registers, 64 leaves, plain 53.6 -> 46; 96 registers, 64 leaves, six-bit
+    48.7 -> 44.5. (With the mode on for the merges 71.8, 57.8, 48.6, 47.2; with SDWA 72.1, 61, 50, 48.)
     Mixed variants: 32 dwords per tree. Bit 31 of the first dword clear: the 7-bit form above (the
     tree has no xor mask and no bin of its buckets is above 128). Set: 4 dwords per level, bucket,
     xorMask, splitIdx & 0x7f (both times 0x01010101) and 0x80808080 if splitIdx < 128 else 0; the
@@ -177,6 +188,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     block = tree_block(pitch, leaves)
     buf_bytes = block * tree_bytes
     lds_bytes = 2 * buf_bytes
+    unpack_scale = (8 if pitch == 1 else 16) >> max(8 - depth, 0)  # bytes of a table per unit of an index byte
     assert buf_bytes % row_bytes == 0 and lds_bytes <= 65536
     # A wave copies its own contiguous share of a tree block, 1 KB (16 bytes per lane) per instruction;
     # up to four instructions of a group differ only in the immediate offset, which moves the source
@@ -199,6 +211,8 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     te0 = ga0 + 4                         # two scratch registers of the epilogue
     wd0 = te0 + 2                         # deep kernels: the ten-bit leaf indexes of documents 0, 1 and 2, 3 as words
     b0 = wd0 + (2 if deep else 0)         # the bins
+    # eight registers for a tree's level sums: scratch, and what the epilogue and the gathers use at other times
+    sums = [4, 5, te0, te0 + 1, ga0, ga0 + 1, ga0 + 2, ga0 + 3]
     vgprs = b0 + buckets
     if fused:
         # registers of the binarize phase: those below the bins except v0 and v2, and 20 above the bins
@@ -215,11 +229,18 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     def waves_per_simd(registers):
         return 512 // ((registers + 7) // 8 * 8)
     # (not where the eight registers would cost a wave per SIMD: the 96-register shape runs four)
+    # behind the bins: the two masks of the merges and the left operand of the product that turns indexes into addresses
+    # (fused: registers that only the binarize phase uses)
+    mask80 = high if fused else vgprs
+    mask_c0, unpack = mask80 + 1, mask80 + 2
+    if not fused:
+        vgprs += 2 if deep else 3
     two_sets = pitch == 1 and block % 2 == 0 and (fused or (vgprs + 8 <= 256 and waves_per_simd(vgprs + 8) == waves_per_simd(vgprs)))
     if two_sets:
         if fused:
             lw0 = high + 8
         else:
+            vgprs += vgprs % 2                    # (register pairs start at even registers)
             lw0 = vgprs
             vgprs += 8
     assert vgprs <= 256
@@ -236,8 +257,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     def stage(buffer_offset, g):
         """Group g of the wave's pieces of a tree block, global memory -> LDS without passing through
         registers: lane l writes 16 bytes at buffer_offset + wave * wave_bytes + piece * 1024 + l * 16 (M0
-        holds the wave's base). M0 doubles as the VGPR index register, so its index-mode value is put
-        back after."""
+        holds the wave's base; outside of a tree's levels nothing else needs it)."""
         first, count = groups[g]
         e("  s_add_u32 m0, s100, %d" % (buffer_offset + first * 1024))
         # the thread's offset moves on to the group's first piece; the instruction also fills the wait
@@ -247,12 +267,10 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             e("  global_load_lds_dwordx4 v2, s[26:27]%s" % (" offset:%d" % (piece * 1024) if piece else ""))
 
     def add_leaf_values(other=False):
-        # sum + leaf as 1.0 * leaf + sum: the same single rounding, and with a constant in src0 the
-        # instruction does not depend on the register index that the levels leave in M0
         for j in range(4):
             for k in range(pitch):
-                e("  v_fma_f64 v[%d:%d], 1.0, v[%d:%d], v[%d:%d]" % (ac(j, k), ac(j, k) + 1, lv(j, k, other), lv(j, k, other) + 1,
-                                                                      ac(j, k), ac(j, k) + 1))
+                e("  v_add_f64 v[%d:%d], v[%d:%d], v[%d:%d]" % (ac(j, k), ac(j, k) + 1, lv(j, k, other), lv(j, k, other) + 1,
+                                                                 ac(j, k), ac(j, k) + 1))
 
     def load_rows(regs, tree):
         """Level table of tree `tree` (counted from the table position in s[6:7]) -> registers."""
@@ -260,22 +278,20 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             e("  s_load_dwordx16 s[%d:%d], s[6:7], 0x%x" % (regs + 16 * part, regs + 16 * part + 15,
                                                             tree * tree_row_bytes + 64 * part))
 
-    # With eight levels the first level's sum needs no masking: each later level shifts the index
-    # right by one and replaces bit 7 of every byte, so the seven low bits of the first sum leave
-    # their byte one by one through bit 0, land on bit 7 of the byte below and are overwritten there.
-    # Six-level kernels keep the mask: two of those bits would stay below the index.
+    # Six-level kernels clear what the first pair leaves below its two bits: two of those bits would stay below the
+    # index. With eight levels they leave their byte through bit 0, land on the upper bits of the byte below and are
+    # overwritten there.
     first_level_masked = depth < 8
 
     def levels_high(rows):
         """Levels 8 and 9 of a deep tree (constants (128 - splitIdx) in every form): their bits become bits 0 and
         1 of a second byte per document, and the two bytes of a document one 16-bit word: v[wd0] holds the
-        indexes of documents 0 and 1, v[wd0 + 1] those of 2 and 3. The index register is set to 0 behind the
-        last level, so that the instructions that follow may name vector registers in src0."""
-        e("  s_set_gpr_idx_idx s%d" % (rows + 16))
+        indexes of documents 0 and 1, v[wd0 + 1] those of 2 and 3."""
+        index_mode(True, rows + 16)
         e("  v_add_u32_e64 v4, v%d, s%d" % (b0, rows + 17))
         e("  s_set_gpr_idx_idx s%d" % (rows + 18))
         e("  v_add_u32_e64 v5, v%d, s%d" % (b0, rows + 19))
-        e("  s_set_gpr_idx_idx 0")
+        index_mode(False)
         e("  v_lshrrev_b32_e32 v4, 7, v4")
         e("  v_lshrrev_b32_e32 v5, 6, v5")
         e("  v_and_b32_e32 v4, 0x01010101, v4")
@@ -284,56 +300,62 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  v_perm_b32 v%d, v4, v3, s24" % wd0)        # bytes: index 0 low, high, index 1 low, high
         e("  v_perm_b32 v%d, v4, v3, s25" % (wd0 + 1))
 
-    def levels_seven_bit(rows):
-        for d in range(min(depth, 8)):
-            e("  s_set_gpr_idx_idx s%d" % (rows + 2 * d))
-            if d == 0 and not first_level_masked:
-                e("  v_add_u32_e64 v3, v%d, s%d" % (b0, rows + 2 * d + 1))
-                continue
-            e("  v_add_u32_e64 v4, v%d, s%d" % (b0, rows + 2 * d + 1))
-            if d == 0:
-                e("  v_and_b32_e32 v3, s22, v4")
-            else:
-                e("  v_lshrrev_b32_e32 v3, 1, v3")
-                e("  v_bfi_b32 v3, s22, v4, v3")
+    def select(to, mask, ones, zeros, invert=False):
+        """Bits of `ones` (inverted: of its complement) where the mask is set, of `zeros` elsewhere."""
+        e("  v_bitop3_b32 v%d, v%d, v%d, v%d bitop3:0x%x" % (to, mask, ones, zeros, 0x3a if invert else 0xca))
 
-    def levels_six_bit(rows):
-        """Bins of at most 64 everywhere: the host gives the even levels the constant (64 - splitIdx), whose sum
-        has the level's bit in bit 6 (and bit 7 clear), the odd levels (128 - splitIdx) as in the 7-bit
-        form. A pair of levels is then merged into the index with one shift: five instructions for two
-        levels instead of six. What the first pair leaves below its two bits goes the way the 7-bit
-        form's first sum goes; six-level kernels mask it."""
-        for pair in range(min(depth, 8) // 2):
-            even, odd = rows + 4 * pair, rows + 4 * pair + 2
-            e("  s_set_gpr_idx_idx s%d" % even)
-            e("  v_add_u32_e64 v4, v%d, s%d" % (b0, even + 1))
-            e("  s_set_gpr_idx_idx s%d" % odd)
-            e("  v_add_u32_e64 v%d, v%d, s%d" % (3 if pair == 0 else 5, b0, odd + 1))
-            if pair == 0:
-                e("  v_bfi_b32 v3, s22, v3, v4")           # bit 7 of the odd level's sum over the even level's
-                if first_level_masked:
-                    e("  v_and_b32_e32 v3, s29, v3")
+    def index_mode(on, register=None):
+        """Index mode: src0 of vector instructions becomes relative to a level's bucket."""
+        e("  s_set_gpr_idx_on s%d, 0x1" % register if on else "  s_set_gpr_idx_off")
+
+    def levels_in_pairs(rows, invert_top):
+        """A pair of levels puts its bits into bits 6 and 7 of a document's byte, and one shift and one select bring
+        them into the index. Bins of at most 64 (six-bit variants): the host gives the even levels the constant
+        (64 - splitIdx), whose sum has the level's bit in bit 6 and bit 7 clear. Else every level has (128 -
+        splitIdx), and v_lerp_u8, bytewise (bin + constant) >> 1 from a sum of nine bits, leaves the even level's bit in
+        bit 6 and bit 7 clear.
+        invert_top: the top bit of every index comes inverted (see gather_addresses)."""
+        count = min(depth, 8)
+        for d in range(count):
+            if d == 0:
+                index_mode(True, rows)
             else:
-                e("  v_bfi_b32 v4, s22, v5, v4")
-                e("  v_lshrrev_b32_e32 v3, 2, v3")
-                e("  v_bfi_b32 v3, s29, v4, v3")
+                e("  s_set_gpr_idx_idx s%d" % (rows + 2 * d))
+            if d % 2 == 0 and not six:
+                e("  v_lerp_u8 v%d, v%d, s%d, 0" % (sums[d], b0, rows + 2 * d + 1))
+            else:
+                e("  v_add_u32_e64 v%d, v%d, s%d" % (sums[d], b0, rows + 2 * d + 1))
+        index_mode(False)
+        for pair in range(count // 2):
+            select(sums[2 * pair], mask80, sums[2 * pair + 1], sums[2 * pair], invert_top and pair == count // 2 - 1)
+        if first_level_masked:
+            e("  v_and_b32_e32 v%d, v%d, v%d" % (sums[0], mask_c0, sums[0]))
+        for pair in range(1, count // 2):
+            e("  v_lshrrev_b32_e32 v3, 2, v%d" % (sums[0] if pair == 1 else 3))
+            select(3, mask_c0, sums[2 * pair], 3)
 
     def levels_eight_bit(rows):
         for d in range(depth):
             level = rows + 4 * d
-            e("  s_set_gpr_idx_idx s%d" % level)                      # index = bits 0..7 of the bucket dword
+            # index = bits 0..7 of the bucket dword
+            if d == 0:
+                index_mode(True, level)
+            else:
+                e("  s_set_gpr_idx_idx s%d" % level)
             e("  v_xor_b32_e64 v4, v%d, s%d" % (b0, level + 1))       # x = bin ^ xorMask
             e("  v_or_b32_e32 v5, s22, v4")
             e("  v_subrev_u32_e32 v5, s%d, v5" % (level + 2))         # (x | 0x80) - (splitIdx & 0x7f), per byte
             if d == 0 and not first_level_masked:
                 e("  v_bitop3_b32 v3, s%d, v4, v5 bitop3:0xe8" % (level + 3))  # majority
                 continue
-            e("  v_bitop3_b32 v4, s%d, v4, v5 bitop3:0xe8" % (level + 3))  # majority
+            # majority; of the top level its complement
+            e("  v_bitop3_b32 v4, s%d, v4, v5 bitop3:0x%x" % (level + 3, 0x17 if d == depth - 1 else 0xe8))
             if d == 0:
                 e("  v_and_b32_e32 v3, s22, v4")
             else:
                 e("  v_lshrrev_b32_e32 v3, 1, v3")
                 e("  v_bfi_b32 v3, s22, v4, v3")
+        index_mode(False)
 
     # ---- the binarize phase's search, shared by the rows' and the columns' form
     out_of_line = []
@@ -744,14 +766,13 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  s_nop 1")
     e("  v_readfirstlane_b32 s20, v5")           # wave of the workgroup
     e("  s_mov_b32 s22, 0x80808080")
-    if six:
-        e("  s_mov_b32 s29, 0xc0c0c0c0")
-    # byte j of the leaf indexes times s23 = offset of the document's leaf row in a tree's table
-    # (a six-level index sits in bits 2..7 of its byte)
+    # byte j of the leaf indexes times the unpacking weight = offset of the document's leaf row in a tree's table
+    # (a six-level index sits in bits 2..7 of its byte); deep kernels: a ten-bit index times s23
     # (tables of several dimensions hold a tree's values as pieces of two dimensions, each piece an array of
     # 16 bytes per leaf: a wave's 16-byte gathers then spread over all sixteen groups of four LDS banks, which
     # leaf rows of 32 bytes would not; an odd last dimension is a piece of eight bytes per leaf)
-    e("  s_mov_b32 s23, %d" % ((8 if pitch == 1 else 16) >> max(8 - depth, 0)))
+    if deep:
+        e("  s_mov_b32 s23, 8")
     e("  s_mul_i32 s100, s20, %d" % wave_bytes)  # offset of the wave's share of a tree block
     # one step back: every group of copies steps forward first
     e("  s_sub_u32 s28, s100, %d" % group_step(0))
@@ -885,6 +906,13 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     load_rows(rows_b, 1)
     for r in list(range(lv0, ga0)) + (list(range(lw0, lw0 + 8)) if two_sets else []):
         e("  v_mov_b32_e32 v%d, 0" % r)          # leaf values in flight and the sums
+    e("  v_mov_b32_e32 v%d, 0x80808080" % mask80)
+    e("  v_mov_b32_e32 v%d, 0xc0c0c0c0" % mask_c0)
+    if not deep:
+        # row i of a product's left operand is lane i's of the four, byte k of it stands for byte k of the index
+        e("  v_and_b32_e32 v5, 3, v0")
+        e("  v_lshlrev_b32_e32 v5, 3, v5")
+        e("  v_lshlrev_b32_e64 v%d, v5, %d" % (unpack, unpack_scale))
     # a launch that continues the sums of earlier trees takes them from `out`
     e("  s_bitcmp1_b32 s15, 1")
     e("  s_cbranch_scc0 %s_fresh" % name)
@@ -907,7 +935,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("%s_fresh:" % name)
     e("  s_waitcnt vmcnt(0) lgkmcnt(0)")
     e("  s_barrier")
-    e("  s_set_gpr_idx_on s22, 0x1")             # src0 of VALU instructions becomes index relative
     # every wave warms its own share of a tree block's level tables, every WARM_WAYS-th 64-byte line
     # from line (wave mod WARM_WAYS) on: s[30:31] = table + that line
     warm_lines = block * tree_row_bytes // 64
@@ -917,8 +944,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  s_lshl_b32 s28, s28, 6")
     e("  s_add_u32 s30, s6, s28")
     e("  s_addc_u32 s31, s7, 0")
-    if odd:
-        e("  s_mov_b32 s24, %d" % (8 >> max(8 - depth, 0)))  # the odd dimension's piece (s24 and s25 are free from here to the epilogue)
     if deep:
         # byte selectors of the two index words (s24 and s25 are free from here to the epilogue)
         e("  s_mov_b32 s24, 0x05010400")
@@ -931,65 +956,58 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 label = "%s_t%d_%d" % (name, buf, i)
                 e("  s_bitcmp1_b32 s%d, 31" % rows)
                 e("  s_cbranch_scc1 %s_x" % label)
-                levels_seven_bit(rows)
+                levels_in_pairs(rows, True)
                 e("  s_branch %s_j" % label)
                 e("%s_x:" % label)
                 levels_eight_bit(rows)
                 e("%s_j:" % label)
-            elif six:
-                levels_six_bit(rows)
             else:
-                levels_seven_bit(rows)
+                levels_in_pairs(rows, not deep)
             if deep:
                 levels_high(rows)
             tree_offset = buf * buf_bytes + i * tree_bytes
+            if not deep:
+                tree_offset += unpack_scale * 128
 
-            def gather_address(j, scale="s23"):
-                if deep:
+            # The previous tree's leaf values have arrived (its levels and addresses were issued in between), and so has
+            # the next tree's row. With two sets of leaf values the trees of a block alternate between them (a block has
+            # an even number of trees, so the first tree of a block finds the last one's values in the second set).
+            mine = two_sets and i % 2 == 1
+            if deep:
+                for j in range(4):
                     e("  v_mul_u32_u24_sdwa v%d, s23, v%d dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_%d"
                       % (ga0 + j, wd0 + j // 2, j % 2))
-                else:
-                    e("  v_mul_u32_u24_sdwa v%d, %s, v3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_%d"
-                      % (ga0 + j, scale, j))
-            if two_sets:
-                # The trees of a block alternate between the two sets of leaf values (a block has an even number
-                # of trees, so the first tree of a block finds the last one's values in the second set). The wait
-                # sits right in front of the tree's own gathers: the previous tree's had its levels and addresses to
-                # arrive, and so had the next tree's row. Gathers in one batch, sums behind them: interleaved they
-                # took longer (1.137 against 1.090 ms per 4M documents and 1000 trees).
-                mine = i % 2 == 1
-                for j in range(4):
-                    gather_address(j)
                 e("  s_waitcnt lgkmcnt(0)")
-                for j in range(4):
-                    e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, 0, mine), lv(j, 0, mine) + 1, ga0 + j, tree_offset))
+                add_leaf_values(two_sets and not mine)
                 load_rows(rows, buf * block + i + 2)
-                add_leaf_values(not mine)
             else:
-                # previous tree's leaf values have arrived (and so has the next tree's row)
+                # Places of the four documents' leaf values in the tree's table, a byte of the index for each document: a
+                # product of 4 x 4 bytes for every four lanes, whose left operand has the bytes' weight on its diagonal,
+                # leaves weight * byte in the four registers of every lane: one instruction instead of four SDWA
+                # multiplications. Its bytes have a sign: with the top bit inverted they are index - 128, and the reads'
+                # offsets add what is missing. The product needs two wait states behind the last select, the reads five
+                # behind the product: the sums and the next row's request.
                 e("  s_waitcnt lgkmcnt(0)")
-                add_leaf_values()
-                for j in range(4):
-                    gather_address(j)
-                    if pitch == 1:
-                        e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, 0), lv(j, 0) + 1, ga0 + j, tree_offset))
-                    else:
-                        for k in range(0, pitch - 1, 2):
-                            e("  ds_read_b128 v[%d:%d], v%d offset:%d" % (lv(j, k), lv(j, k) + 3, ga0 + j,
-                                                                         tree_offset + (k // 2) * leaves * 16))
-                        if odd:
-                            gather_address(j, "s24")
-                            e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, pitch - 1), lv(j, pitch - 1) + 1, ga0 + j,
-                                                                        tree_offset + (pitch // 2) * leaves * 16))
+                e("  s_nop 0")
+                e("  v_mfma_i32_4x4x4_16b_i8 v[%d:%d], v%d, v3, 0" % (ga0, ga0 + 3, unpack))
+                add_leaf_values(two_sets and not mine)
                 load_rows(rows, buf * block + i + 2)
+            for j in range(4):
+                if pitch == 1:
+                    e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, 0, mine), lv(j, 0, mine) + 1, ga0 + j, tree_offset))
+                    continue
+                for k in range(0, pitch - 1, 2):
+                    e("  ds_read_b128 v[%d:%d], v%d offset:%d" % (lv(j, k), lv(j, k) + 3, ga0 + j,
+                                                                 tree_offset + (k // 2) * leaves * 16))
+                if odd:
+                    # half the place: pieces of eight bytes
+                    e("  v_ashrrev_i32_e32 v%d, 1, v%d" % (te0, ga0 + j))
+                    e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, pitch - 1), lv(j, pitch - 1) + 1, te0,
+                                                                tree_offset + (pitch // 2) * leaves * 16 - unpack_scale * 64))
             # copy of the next tree block into the other buffer, spread over this block's trees
-            staged = False
             for g in range(len(groups)):
                 if g * block // len(groups) == i:
                     stage((1 - buf) * buf_bytes, g)
-                    staged = True
-            if staged:
-                e("  s_mov_b32 m0, 0x1000")      # index mode value again: src0 relative, index 0
             if i == 0:
                 # the rows of the next tree block are pulled into the scalar cache now, so that the
                 # per-tree row loads of that block do not each wait for a miss. The waves of a workgroup
@@ -1011,7 +1029,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  s_branch %s_loop" % name)
     e("%s_done:" % name)
     add_leaf_values(two_sets)                # the last tree of a block: second set
-    e("  s_set_gpr_idx_off")
     e("  s_bitcmp1_b32 s15, 2")                  # raw sums for a launch that continues them
     e("  s_cbranch_scc1 %s_store" % name)
     # scale, bias of the launch's dimensions (rows registers are free now)
@@ -1063,7 +1080,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  s_addc_u32 s31, s31, 0")
         for r in list(range(lv0, ga0)) + (list(range(lw0, lw0 + 8)) if two_sets else []):
             e("  v_mov_b32_e32 v%d, 0" % r)
-        e("  s_set_gpr_idx_on s22, 0x1")
         e("  s_branch %s_loop" % name)
         e("%s_end:" % name)
     e("  s_endpgm")

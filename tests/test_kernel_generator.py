@@ -262,3 +262,113 @@ def test_only_the_fused_kernels_of_rows_start_late():
         for buckets, waves in shapes:
             text, _ = gen.gen_kernel(buckets, waves, 1, 256, False, True, fused=True, columns=columns)
             assert ("s_sleep" in text) == (not columns)
+
+
+def _signed(byte):
+    return byte - 256 if byte >= 128 else byte
+
+
+def _places(code, scalars, bins, bins_at, weight):
+    """Follows one lane through the vector instructions of a tree (up to its first leaf gather) and gives the LDS offsets that
+    the gathers of the four documents name. `bins`: dwords of the bins registers from register `bins_at` on. Also checks what
+    the hardware asks for: two instructions between the last write of the product's index and the product, five between the
+    product and the first gather, no vector register in src0 of anything but a level's compare in index mode."""
+    v = {bins_at + i: dword for i, dword in enumerate(bins)}
+    index, written, product_at, gathers = None, {}, None, []
+    bytes_of = lambda x: [(x >> (8 * j)) & 255 for j in range(4)]  # noqa: E731
+    dword = lambda b: sum(x << (8 * j) for j, x in enumerate(b))   # noqa: E731
+
+    def value(operand):
+        if operand.startswith("v"):
+            return v[int(operand[1:])]
+        return scalars[int(operand[1:])] if operand.startswith("s") else int(operand, 0)
+
+    masks = [m.group(1) for m in (re.match(r"v_bitop3_b32 v\d+, v(\d+),", c) for c in code) if m]
+    lows = [m.group(1) for m in (re.match(r"v_bitop3_b32 v3, v(\d+),", c) for c in code) if m]
+    low = int(lows[0])
+    v[int(next(m for m in masks if int(m) != low))], v[low] = 0x80808080, 0xc0c0c0c0
+    for at, c in enumerate(code):
+        op, _, rest = c.partition(" ")
+        args = [x.strip() for x in rest.split(",")]
+        if op == "s_set_gpr_idx_on":
+            index = scalars[int(args[0][1:])] & 255
+        elif op == "s_set_gpr_idx_idx":
+            index = scalars[int(args[0][1:])] & 255
+        elif op == "s_set_gpr_idx_off":
+            index = None
+        elif op in ("v_add_u32_e64", "v_lerp_u8"):
+            assert index is not None and int(args[1][1:]) == bins_at
+            a, b = bytes_of(v[bins_at + index]), bytes_of(value(args[2]))
+            sums = [x + y for x, y in zip(a, b)]
+            assert op == "v_lerp_u8" or max(sums) < 256
+            v[int(args[0][1:])] = dword([x >> 1 for x in sums]) if op == "v_lerp_u8" else dword(sums)
+            written[int(args[0][1:])] = at
+        elif op.startswith(("v_bitop3", "v_lshrrev", "v_and_b32")):
+            assert index is None
+            if op.startswith("v_bitop3"):
+                last, table = args[3].split()
+                table = int(table.split(":")[1], 16)
+                x, y, z = value(args[1]), value(args[2]), value(last)
+                out = sum(((table >> (((x >> b & 1) << 2) | ((y >> b & 1) << 1) | (z >> b & 1))) & 1) << b for b in range(32))
+            elif op.startswith("v_lshrrev"):
+                out = value(args[2]) >> int(args[1])
+            else:
+                out = value(args[1]) & value(args[2])
+            v[int(args[0][1:])] = out
+            written[int(args[0][1:])] = at
+        elif op.startswith("v_mfma"):
+            assert at - written[3] > 2 and index is None
+            first = int(re.match(r"v\[(\d+):", args[0]).group(1))
+            for j in range(4):
+                v[first + j] = weight * _signed(bytes_of(v[3])[j])
+            product_at = at
+        elif op == "v_ashrrev_i32_e32":
+            v[int(args[0][1:])] = v[int(args[2][1:])] >> int(args[1])
+        elif op.startswith("ds_read"):
+            assert at - product_at > 5
+            found = re.match(r"ds_read_b(64|128) v\[\d+:\d+\], v(\d+) offset:(\d+)$", c)
+            gathers.append(v[int(found.group(2))] + int(found.group(3)))
+        else:
+            assert op in ("s_waitcnt", "s_nop", "v_add_f64", "s_load_dwordx16"), c
+    return gathers
+
+
+@pytest.mark.parametrize("shape", [(128, 4, 1, 64), (96, 8, 1, 64), (200, 4, 1, 256), (104, 4, 3, 64), (56, 4, 6, 64)])
+@pytest.mark.parametrize("six", [False, True])
+def test_places_of_leaf_values(shape, six):
+    """The levels' compares, their merges and the product, followed for one lane: the gathers name the leaves that comparing
+    bins with splits gives, at the edges of what the compare holds (bins and splits of 1 and 127 or 63, a bin of 128 or 64,
+    a level that stands for none: constant 0, true for that bin alone)."""
+    import random
+    gen = _generator()
+    buckets, waves, pitch, leaves = shape
+    text, _ = gen.gen_kernel(buckets, waves, pitch, leaves, False, six)
+    lines = [line.strip() for line in text.split("\n")]
+    start = next(i for i, line in enumerate(lines) if line.endswith("_loop:")) + 1
+    gathers = 4 * ((pitch + 1) // 2)
+    code = []
+    for line in lines[start:]:
+        code.append(line)
+        if sum(c.startswith("ds_read") for c in code) == gathers:
+            break
+    depth, top = (6 if leaves == 64 else 8), (64 if six else 128)
+    bins_at = int(re.search(r"v_add_u32_e64 v\d+, v(\d+), s", text).group(1))
+    weight = (8 if pitch == 1 else 16) >> (8 - depth)
+    rng = random.Random(7)
+    for _ in range(200):
+        bins = [[rng.choice([0, 1, top // 2, top - 1, top, rng.randrange(top + 1)]) for _ in range(4)] for _ in range(buckets)]
+        scalars, expected = {}, [0] * 4
+        for d in range(depth):
+            bucket, split = rng.randrange(buckets), rng.choice([1, 2, top - 1, top, rng.randrange(1, top + 1)])
+            scalars[32 + 2 * d] = bucket
+            scalars[33 + 2 * d] = ((64 if six and d % 2 == 0 else 128) - split) * 0x01010101
+            for j in range(4):
+                expected[j] |= int(bins[bucket][j] >= split) << d
+        got = _places(code, scalars, [sum(x << (8 * j) for j, x in enumerate(b)) for b in bins], bins_at, weight)
+        if pitch == 1:
+            assert got == [8 * x for x in expected]
+        else:
+            for j in range(4):
+                for k in range((pitch + 1) // 2):
+                    piece = (16 if 2 * k + 1 < pitch else 8) * expected[j] + k * leaves * 16
+                    assert got[j * ((pitch + 1) // 2) + k] == piece
