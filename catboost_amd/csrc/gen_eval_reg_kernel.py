@@ -51,7 +51,7 @@ Layout of the work:
 Kernel arguments (80 bytes):
    0 bins        const uint32*   [docBlock][bucketCount][64]
    8 rows        const uint32*   [(treeBlocks + 2) * TREE_BLOCK][16 or 32]  (null trees behind the model's)
-  16 leaves      const double*   [(treeBlocks + 2) * TREE_BLOCK][LEAVES][PITCH]
+  16 leaves      const double*   [(treeBlocks + 2) * TREE_BLOCK][LEAVES][PITCH] (fused kernels of six levels: [whole buffers of 64 trees, and two][64])
   24 out         double*         [docCount][dim]
   32 docCount    uint32          36 blockCount uint32 (ceil(docCount / 256), >= 1)
   40 treeBlocks  uint32 (>= 1)   44 flags uint32 (bit 0: add the bias)
@@ -125,8 +125,10 @@ VARIANTS += [shape + (False, six) for six in (False, True) for shape in DEEP_SHA
 # units, up to 96 buckets, runs its separate evaluate kernel at four waves per SIMD, which a fused kernel of 96
 # bins registers (144: three) does not match: measured, two launches are the faster there.
 FUSED_SHAPES = [(208, 4), (64, 8), (80, 8)]
-# Every shape also in a form that walks six levels ("_d6": models of depth <= 6; the leaf tables keep the 256 rows
-# per tree that the border images' buffers are sized for, the index reaches the first 64 of them).
+# Every shape also in a form that walks six levels ("_d6": models of depth <= 6): leaf tables of 64 rows per tree, 64 trees to a
+# buffer, whose walk may end behind any sixteenth tree. That is a quarter of the leaf values' way and of the barriers that tables
+# of 256 rows, sixteen trees to a buffer, took: 1M documents, 1000 trees over 150 columns 308 -> 293 us a call, 200 trees over rows of
+# 50 features 100.2 -> 99.
 FUSED_SIX_LEVEL_BUCKETS = 208
 # Fused kernels of column-major documents ("cbamd_fused_cols_..."), every shape in the same four forms. A load is a column's value
 # for 64 neighbouring documents: a line comes whole and, where the columns start on line boundaries, once (else a wave's load
@@ -184,8 +186,11 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     odd = pitch > 1 and pitch % 2 == 1    # the last dimension's values stand alone, eight bytes per leaf
     threads = waves * 64
     row_bytes = threads * 16              # one 16-byte piece per thread of a leaf table copy
-    tree_bytes = leaves * pitch * 8
-    block = tree_block(pitch, leaves)
+    # (six-level fused kernels: the 32 KB buffers of the border images hold 64 trees of 64 leaves)
+    table_leaves = levels and 1 << levels or leaves
+    tree_bytes = table_leaves * pitch * 8
+    step = tree_block(pitch, leaves)      # trees that the tree blocks of the arguments count
+    block = step * leaves // table_leaves  # trees of a buffer: whole steps
     buf_bytes = block * tree_bytes
     lds_bytes = 2 * buf_bytes
     unpack_scale = (8 if pitch == 1 else 16) >> max(8 - depth, 0)  # bytes of a table per unit of an index byte
@@ -935,9 +940,9 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("%s_fresh:" % name)
     e("  s_waitcnt vmcnt(0) lgkmcnt(0)")
     e("  s_barrier")
-    # every wave warms its own share of a tree block's level tables, every WARM_WAYS-th 64-byte line
+    # every wave warms its own share of a step's level tables, every WARM_WAYS-th 64-byte line
     # from line (wave mod WARM_WAYS) on: s[30:31] = table + that line
-    warm_lines = block * tree_row_bytes // 64
+    warm_lines = step * tree_row_bytes // 64
     warm_ways = min(waves, warm_lines)
     assert warm_ways & (warm_ways - 1) == 0 and warm_lines % warm_ways == 0
     e("  s_and_b32 s28, s20, %d" % (warm_ways - 1))
@@ -1008,14 +1013,18 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             for g in range(len(groups)):
                 if g * block // len(groups) == i:
                     stage((1 - buf) * buf_bytes, g)
-            if i == 0:
-                # the rows of the next tree block are pulled into the scalar cache now, so that the
-                # per-tree row loads of that block do not each wait for a miss. The waves of a workgroup
+            if i % step == 0:
+                # the rows of the next step's trees are pulled into the scalar cache now, so that the
+                # per-tree row loads there do not each wait for a miss. The waves of a workgroup
                 # share the cache and reach this point together, so each touches a share of the lines
                 # (a scalar load is dear here: sixteen per wave and block cost 5 % of the launch)
                 for k in range(warm_lines // warm_ways):
-                    e("  s_load_dword s3, s[30:31], 0x%x" % ((buf * block + block + 2) * tree_row_bytes
+                    e("  s_load_dword s3, s[30:31], 0x%x" % ((buf * block + i + step + 2) * tree_row_bytes
                                                             + 64 * warm_ways * k))
+            if (i + 1) % step == 0 and i + 1 < block:
+                e("  s_add_u32 s14, s14, -1")
+                e("  s_cmp_eq_u32 s14, 0")
+                e("  s_cbranch_scc1 %s_done" % name)
         # every wave is done reading this buffer and writing the other one
         e("  s_waitcnt vmcnt(0) lgkmcnt(0)")
         e("  s_barrier")
@@ -1028,6 +1037,8 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  s_addc_u32 s31, s31, 0")
     e("  s_branch %s_loop" % name)
     e("%s_done:" % name)
+    if step < block:
+        e("  s_waitcnt vmcnt(0) lgkmcnt(0)")     # the last gathers, and the copies into the other buffer
     add_leaf_values(two_sets)                # the last tree of a block: second set
     e("  s_bitcmp1_b32 s15, 2")                  # raw sums for a launch that continues them
     e("  s_cbranch_scc1 %s_store" % name)

@@ -2887,21 +2887,15 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         // Models of the 96-register shape take the fused kernel of 64 or 80 bins registers when their units fit it (112
         // and 128 registers: four waves per SIMD like their evaluate kernel); with more units they stay on two launches
         // (a fused kernel of 96 bins registers would run at three waves per SIMD and is the slower - measured on
-        // 50 and 90 buckets). The fused kernels copy 256 leaf rows per tree: a model on the six-level kernel gets
-        // a leaf table of that pitch for them (its level rows have the eight slots anyway) and the form of the
-        // fused kernel that walks six levels (4M documents x 1000 trees of depth 6 over 70 features: 1.06 ms
-        // against 1.15 on two launches; with the eight-level walk 1.19).
+        // 50 and 90 buckets). A model on the six-level kernel takes the form of the fused kernel that walks six levels, whose
+        // buffers hold 64 trees: null trees up to whole buffers, and two more.
         const bool fusedCandidate = switches.Fused && !regMapped && !variant->Mixed && variant->Pitch == 1 && variant->Leaves <= 256 && m.Dim == 1 && !m.HasCats &&
                                     m.CtrCount == 0 && m.BinarizeBuckets == BucketCount && BucketCount > 0 &&
                                     (TreeCount / block + 3) * block * 256 * 8 + 16 * kFusedImageBytes < (uint64_t(1) << 32) - (1u << 20);
-        std::vector<double> fusedLeaves;  // 256 rows per tree
-        if (fusedCandidate && variant->Leaves == 64) {
-            fusedLeaves.assign(tableTrees * 256, 0.0);
-            for (size_t t = 0; t < TreeCount; ++t) {
-                std::copy(leaves.begin() + t * 64, leaves.begin() + (t + 1) * 64, fusedLeaves.begin() + t * 256);
-            }
-        }
-        const std::vector<double>& fusedLeafTable = variant->Leaves == 64 ? fusedLeaves : leaves;
+        const size_t bufferTrees = kFusedImageBytes / (variant->Leaves * sizeof(double));
+        const size_t fusedTrees = fusedCandidate ? ((TreeCount + bufferTrees - 1) / bufferTrees + 2) * bufferTrees : 0;
+        std::vector<double> fusedLeafTable(leaves.begin(), leaves.begin() + (fusedCandidate ? std::min(leaves.size(), fusedTrees * variant->Leaves) : 0));
+        fusedLeafTable.resize(fusedTrees * variant->Leaves, 0.0);
         for (int layoutIndex = 0; layoutIndex < 3 && fusedCandidate; ++layoutIndex) {
             const bool columnMajor = layoutIndex == 2;  // a value is a load of its own: units of any sixteen buckets
             const std::vector<uint32_t>& columns = layoutIndex == 1 ? srcSplit : srcFlat;
@@ -2947,7 +2941,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 // (of the rows' shapes the wide one is for the models of the wide evaluate kernels; columns over 88
                 // buckets: 1M documents, 200 trees 164 us on two launches, 126 on the shape of 160, 1000 trees 329 and 301)
                 if (v.Columns == columnMajor && v.Six == variant->Six && unitStart.size() * kFusedUnitColumns <= v.Buckets && !fused &&
-                    (variant->Waves == 4 || v.Buckets <= 80 || columnMajor) && m.MaxDepth <= v.Levels) {
+                    (variant->Waves == 4 || v.Buckets <= 80 || columnMajor) && variant->Leaves == 1u << v.Levels) {
                     fused = &v;
                 }
             }
@@ -3032,6 +3026,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             std::memcpy(table.data() + images * kFusedImageBytes, fusedLeafTable.data(), fusedLeafTable.size() * sizeof(double));
             // level rows of the same form as the register kernel's, naming bins registers of this layout
             std::vector<uint32_t> fusedRows(rows);
+            fusedRows.resize(std::max(fusedRows.size(), fusedTrees * rowDwords), 0);
             for (size_t t = 0; t < TreeCount; ++t) {
                 const int depth = trees.TreeSizes[t];
                 uint32_t* row = fusedRows.data() + t * rowDwords;
