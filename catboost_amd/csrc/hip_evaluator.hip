@@ -16,6 +16,7 @@
 #include <cstring>
 #include <exception>
 #include <future>
+#include <iterator>
 #include <limits>
 #include <map>
 #include <numeric>
@@ -711,7 +712,7 @@ struct TNsUnit {
     uint32_t Height;
 };
 
-// Groups the trees (rows: first entry, height, entry count, unused) into units of at most `limit` entries.
+// Groups the trees (rows: first entry, steps behind the exits, entry count, unused) into units of at most `limit` entries.
 // A unit takes as many steps as its tallest tree, so the trees go in by falling height, and every tree joins
 // the fullest of the recently opened units that still has room for it (trees need not be neighbours in the
 // model: the kernel's sums are partial sums per wave anyway). False when a tree exceeds the limit.
@@ -832,7 +833,7 @@ int TileChunk(int dim) {
 // has at most 1023 buckets and no tree above dev::kNsLdsEntries entries (one-hot splits count two).
 void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<uint32_t>& firstLeaf,
                           TDeviceVec<uint32_t>* entriesOut, TDeviceVec<uint32_t>* rowsOut, bool* usable, bool* noXor,
-                          std::vector<uint32_t>* compactEntries, std::vector<uint32_t>* compactRows,
+                          std::vector<uint32_t>* compactEntries, std::vector<uint32_t>* compactRows, std::vector<uint32_t>* topNodes,
                           std::vector<double>* valuesByEntry, bool* compactUsable) {
     struct TItem {
         uint32_t Node;        // model node, or the parent node of a synthetic terminal
@@ -961,7 +962,7 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
         rows[t * 4 + 0] = static_cast<uint32_t>(firstEntry);
         rows[t * 4 + 1] = plain.Height;
         rows[t * 4 + 2] = firstLeaf[t];
-        // compact layout: root at 0, entry 1 unused, so that every pair of children starts even
+        // compact layout: the top nodes apart, the eight exits behind them, then pairs of children, so that every pair starts even
         if (!*compactUsable || !*usable) {
             *compactUsable = false;
             continue;
@@ -969,37 +970,81 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
         const TUnfolded split = *noXor ? TUnfolded() : unfold(root, true);
         const TUnfolded& compact = *noXor ? plain : split;
         *compactUsable = compact.Fits && compact.Order.size() + 1 <= static_cast<size_t>(dev::kNsLdsEntries);
-        if (*compactUsable) {
-            const auto compactIndex = [](size_t i) { return static_cast<uint32_t>(i == 0 ? 0 : i + 1); };
-            (*compactRows)[t * 4 + 0] = static_cast<uint32_t>(compactEntries->size());
-            (*compactRows)[t * 4 + 1] = compact.Height;
-            (*compactRows)[t * 4 + 2] = static_cast<uint32_t>(compact.Order.size() + 1);
-            for (size_t i = 0; i < compact.Order.size(); ++i) {
-                const TItem item = compact.Order[i];
-                const uint32_t self = compactIndex(i);
-                if (item.Terminal) {
-                    const bool odd = (self & 1u) != 0;
-                    compactEntries->push_back((odd ? 0u : 255u) | ((self & ~1u) << 21));
-                    const double* leaf = trees.LeafValues.data() + trees.NonSymmetricNodeIdToLeafId[item.Node];
-                    valuesByEntry->insert(valuesByEntry->end(), leaf, leaf + dim);
-                } else {
-                    const auto& rb = trees.RepackedBins[item.Node];
-                    // a one-hot split holds ~value in its xor mask (and 255 as its split index)
-                    uint32_t splitIdx = rb.SplitIdx;
-                    if (rb.XorMask != 0) {
-                        const uint32_t value = (~static_cast<uint32_t>(rb.XorMask)) & 0xffu;
-                        splitIdx = item.Second ? value + 1 : value;
-                        *compactUsable = *compactUsable && splitIdx <= 255;
-                    }
-                    // the true side always follows the false side in the order
-                    compactEntries->push_back(splitIdx | (static_cast<uint32_t>(rb.FeatureIndex) << 8) |
-                                              (compactIndex(compact.Children[i].first) << 21));
-                    valuesByEntry->insert(valuesByEntry->end(), static_cast<size_t>(dim), 0.0);
-                }
-                if (i == 0) {
-                    compactEntries->push_back(255u);  // the unused entry
-                    valuesByEntry->insert(valuesByEntry->end(), static_cast<size_t>(dim), 0.0);
-                }
+        if (!*compactUsable) {
+            continue;
+        }
+        // the item that a path of `levels` decisions (the root's the highest bit) leads to, a leaf if it ends there earlier
+        const auto follow = [&](uint32_t path, int levels) {
+            size_t i = 0;
+            for (int level = levels - 1; level >= 0 && !compact.Order[i].Terminal; --level) {
+                i = compact.Children[i].first + (path >> level & 1);  // the true side always follows the false side in the order
+            }
+            return i;
+        };
+        const auto splitOf = [&](size_t i) {
+            const auto& rb = trees.RepackedBins[compact.Order[i].Node];
+            if (rb.XorMask == 0) {
+                return static_cast<uint32_t>(rb.SplitIdx);
+            }
+            // a one-hot split holds ~value in its xor mask (and 255 as its split index)
+            return ((~static_cast<uint32_t>(rb.XorMask)) & 0xffu) + (compact.Order[i].Second ? 1u : 0u);
+        };
+        const auto bucketOf = [&](size_t i) { return static_cast<uint32_t>(trees.RepackedBins[compact.Order[i].Node].FeatureIndex); };
+        // the seven nodes of the top levels; false for every bin where there is none
+        for (uint32_t n = 0; n < 8; ++n) {
+            const int level = n == 0 ? 0 : n < 3 ? 1 : 2;
+            const size_t i = follow(n + 1 - (1u << level), level);
+            const bool none = n == 7 || compact.Order[i].Terminal;
+            *compactUsable = *compactUsable && (none || splitOf(i) <= 255);
+            topNodes->push_back(none ? 0u : bucketOf(i) << 8 | (256u - splitOf(i)));
+        }
+        // the exits, then the pairs of children below them; a pair has one place, whichever entries name it (those that a one-hot
+        // split repeats name their original's)
+        std::vector<size_t> placed;  // the item at each place
+        placed.reserve(compact.Order.size() + 8);
+        for (uint32_t exit = 0; exit < 8; ++exit) {
+            placed.push_back(follow(exit, 3));
+        }
+        std::vector<uint32_t> placeOfPair(compact.Order.size(), 0);  // by the left child's item; 0: none yet
+        for (size_t at = 0; at < placed.size(); ++at) {
+            const size_t i = placed[at];
+            if (!compact.Order[i].Terminal && placeOfPair[compact.Children[i].first] == 0) {
+                placeOfPair[compact.Children[i].first] = static_cast<uint32_t>(placed.size());
+                placed.push_back(compact.Children[i].first);
+                placed.push_back(compact.Children[i].first + 1);
+            }
+        }
+        // steps from each item to the farthest leaf
+        std::vector<uint32_t> stepsFrom(compact.Order.size(), UINT32_MAX);
+        const auto steps = [&](const auto& self, size_t i) -> uint32_t {
+            if (stepsFrom[i] == UINT32_MAX) {
+                const uint32_t left = compact.Children[i].first;
+                stepsFrom[i] = compact.Order[i].Terminal ? 0 : 1 + std::max(self(self, left), self(self, left + 1));
+            }
+            return stepsFrom[i];
+        };
+        uint32_t height = 0;
+        for (uint32_t exit = 0; exit < 8; ++exit) {
+            height = std::max(height, steps(steps, placed[exit]));
+        }
+        const size_t count = (placed.size() + 7) / 8 * 8;  // (a tree's exits start at a multiple of 32 bytes)
+        (*compactRows)[t * 4 + 0] = static_cast<uint32_t>(compactEntries->size());
+        (*compactRows)[t * 4 + 1] = height;
+        (*compactRows)[t * 4 + 2] = static_cast<uint32_t>(count);
+        *compactUsable = *compactUsable && count <= static_cast<size_t>(dev::kNsLdsEntries);
+        for (uint32_t at = 0; at < count; ++at) {
+            if (at >= placed.size() || compact.Order[placed[at]].Terminal) {
+                compactEntries->push_back((at % 2 != 0 ? 0u : 255u) | ((at & ~1u) << 21));
+            } else {
+                *compactUsable = *compactUsable && splitOf(placed[at]) <= 255;
+                compactEntries->push_back((splitOf(placed[at]) & 0xffu) | bucketOf(placed[at]) << 8 |
+                                          placeOfPair[compact.Children[placed[at]].first] << 21);
+            }
+            if (at < placed.size() && compact.Order[placed[at]].Terminal) {
+                const double* leaf = trees.LeafValues.data() + trees.NonSymmetricNodeIdToLeafId[compact.Order[placed[at]].Node];
+                valuesByEntry->insert(valuesByEntry->end(), leaf, leaf + dim);
+            } else {
+                valuesByEntry->insert(valuesByEntry->end(), static_cast<size_t>(dim), 0.0);
             }
         }
     }
@@ -1659,7 +1704,7 @@ struct THipEvaluator::TImpl {
     TDeviceVec<uint32_t> NsRows;     // 4 dwords per tree
     bool NsLdsUsable = false;        // compact entries walked out of LDS (one-dimensional, no xor)
     TDeviceVec<uint32_t> NsCompactEntries;
-    TDeviceVec<uint32_t> NsCompactRows;  // 8 dwords per unit of trees
+    TDeviceVec<uint32_t> NsCompactRows;  // dev::kNsUnitDwords per unit of trees
     uint32_t NsUnitCount = 0;
     uint32_t NsEntryCount = 0;       // entries of all units: rows of NsValuesByEntry per slice of the dimensions
     TNsLdsShape NsLdsShape{0, 0};    // waves and entries per region of EvalNonSymmetricLdsKernel for this model
@@ -2588,10 +2633,10 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
     }
 
     if (!m.Oblivious) {
-        std::vector<uint32_t> compactEntries, compactRows;
+        std::vector<uint32_t> compactEntries, compactRows, topNodes;
         std::vector<double> valuesByEntry;
         BuildLevelOrderTrees(trees, m.Dim, firstLeaf, &m.NsEntries, &m.NsRows, &m.NsTileUsable, &m.NsNoXor,
-                             &compactEntries, &compactRows, &valuesByEntry, &m.NsLdsUsable);
+                             &compactEntries, &compactRows, &topNodes, &valuesByEntry, &m.NsLdsUsable);
         if (m.NsLdsUsable) {
             // the shape whose units take the least time: more waves hide more of the walk's latency (steps per
             // unit of time relative to 8 waves, measured on 500 trees of about 430 entries: 12 waves 1.26), smaller
@@ -2610,7 +2655,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 }
                 uint64_t steps = 0;
                 for (const TNsUnit& unit : plan) {
-                    steps += unit.Height;
+                    steps += unit.Height + 3;  // the top three levels, which the shapes' speeds were measured with as steps
                 }
                 const double cost = static_cast<double>(steps) / shape.Speed;
                 if (!m.NsLdsUsable || cost < bestCost) {
@@ -2621,17 +2666,17 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 }
             }
             if (m.NsLdsUsable) {
-                // the entries in the order of the units; child indexes (bits 21-31) count from the unit's first entry
+                // the entries in the order of the units; child indexes (bits 21-31) count from the unit's first entry (trees are
+                // whole pieces of eight entries, as a wave's copy of a unit, sixteen bytes per lane, needs pieces of four)
                 std::vector<uint32_t> entries, units;
                 std::vector<double> values;
                 entries.reserve(compactEntries.size());
                 values.reserve(valuesByEntry.size());
+                // the bucket (bits 8-17 of an entry or node) becomes the LDS row of its bins in this shape
+                const auto withTileRow = [&](uint32_t entry) {
+                    return (entry & ~0x3ff00u) | dev::NsLdsTileRow((entry >> 8) & 0x3ffu, m.NsLdsShape.Waves, m.NsLdsShape.Entries) << 8;
+                };
                 for (const TNsUnit& unit : bestUnits) {
-                    // a wave copies a unit sixteen bytes per lane: every unit starts at a multiple of four entries
-                    while (entries.size() % 4 != 0) {
-                        entries.push_back(255u);
-                        values.insert(values.end(), static_cast<size_t>(m.Dim), 0.0);
-                    }
                     const uint32_t first = static_cast<uint32_t>(entries.size());
                     uint32_t start[dev::kNsUnitTrees] = {};
                     uint32_t count = 0;
@@ -2640,18 +2685,23 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                         const uint32_t treeFirst = compactRows[t * 4], treeEntries = compactRows[t * 4 + 2];
                         start[i] = count;
                         for (uint32_t e = 0; e < treeEntries; ++e) {
-                            // the bucket (bits 8-17) becomes the LDS row of its bins in this shape
-                            const uint32_t entry = compactEntries[treeFirst + e];
-                            const uint32_t tileRow = dev::NsLdsTileRow((entry >> 8) & 0x3ffu, m.NsLdsShape.Waves, m.NsLdsShape.Entries);
-                            entries.push_back((entry & ~0x3ff00u) + (tileRow << 8) + (count << 21));
+                            entries.push_back(withTileRow(compactEntries[treeFirst + e]) + (count << 21));
                             const double* value = valuesByEntry.data() + static_cast<size_t>(treeFirst + e) * m.Dim;
                             values.insert(values.end(), value, value + m.Dim);
                         }
                         count += treeEntries;
                     }
-                    const uint32_t row[8] = {first, unit.Height, count, start[1], start[2] | (unit.TreeCount << 16),
+                    const uint32_t row[8] = {first, unit.Height, first, start[1], start[2] | (unit.TreeCount << 16),
                                              unit.Trees[0], unit.Trees[1], unit.Trees[2]};
                     units.insert(units.end(), row, row + 8);
+                    for (uint32_t i = 0; i < static_cast<uint32_t>(dev::kNsUnitTrees); ++i) {
+                        const uint32_t* nodes = topNodes.data() + unit.Trees[i < unit.TreeCount ? i : 0] * 8;  // (a tree too few: the first again)
+                        std::transform(nodes, nodes + 8, std::back_inserter(units), withTileRow);
+                    }
+                }
+                // the first entry of the unit that a unit's wave takes next
+                for (size_t u = 0; u + m.NsLdsShape.Waves < bestUnits.size(); ++u) {
+                    units[u * dev::kNsUnitDwords + 2] = units[(u + m.NsLdsShape.Waves) * dev::kNsUnitDwords];
                 }
                 m.NsUnitCount = static_cast<uint32_t>(bestUnits.size());
                 m.NsEntryCount = static_cast<uint32_t>(entries.size());
@@ -2662,14 +2712,17 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     m.NsCompactEntries.Upload(padded);
                 }
                 m.NsCompactRows.Upload(units);
-                if (m.Dim > 1) {
-                    // [slice of the dimensions][entry][dimension of the slice], zeros past the last dimension
-                    const uint32_t dims = NsLdsDims(m.Dim), slices = (static_cast<uint32_t>(m.Dim) + dims - 1) / dims;
-                    std::vector<double> bySlice(static_cast<size_t>(slices) * entries.size() * dims, 0.0);
+                // [slice of the dimensions][entry][dimension of the slice], zeros past the last dimension and behind the last entry
+                const uint32_t dims = NsLdsDims(m.Dim), slices = (static_cast<uint32_t>(m.Dim) + dims - 1) / dims;
+                const size_t sliceRows = entries.size() + m.NsLdsShape.Entries;
+                if (m.Dim == 1) {
+                    values.resize(sliceRows, 0.0);
+                } else {
+                    std::vector<double> bySlice(slices * sliceRows * dims, 0.0);
                     for (uint32_t slice = 0; slice < slices; ++slice) {
                         for (size_t e = 0; e < entries.size(); ++e) {
                             for (uint32_t k = 0; k < dims && slice * dims + k < static_cast<uint32_t>(m.Dim); ++k) {
-                                bySlice[(slice * entries.size() + e) * dims + k] = values[e * m.Dim + slice * dims + k];
+                                bySlice[(slice * sliceRows + e) * dims + k] = values[e * m.Dim + slice * dims + k];
                             }
                         }
                     }
@@ -3860,9 +3913,10 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
             const dim3 grid(static_cast<uint32_t>(blocks), (static_cast<uint32_t>(m.Dim) + dims - 1) / dims);
             hipLaunchKernelGGL(kernel, grid, dim3(64 * m.NsLdsShape.Waves), lds, s,
                                reinterpret_cast<const uint32_t*>(bins), docCount, m.LayoutBuckets,
-                               m.NsCompactEntries.Get(), reinterpret_cast<const uint4*>(m.NsCompactRows.Get()),
+                               m.NsCompactEntries.Get(), m.NsCompactRows.Get(),
                                m.NsUnitCount, m.NsValuesByEntry.Get(), m.Bias.Get(), m.Scale,
-                               static_cast<uint32_t>(m.Dim), m.NsEntryCount, tb, te, results);
+                               static_cast<uint32_t>(m.Dim), m.NsEntryCount, tb, te,
+                               static_cast<uint32_t>(treeStart == 0 && treeEnd == TreeCount), results);
         };
         const auto tryShape = [&](auto waves, auto entries) {
             constexpr int W = decltype(waves)::value, E = decltype(entries)::value;

@@ -629,22 +629,37 @@ __device__ __forceinline__ void CopyInBatches(const T* __restrict__ src, uint32_
     }
 }
 
-// All `rows` of a block (256 bytes each), row r to the 64 dwords from tile + 64 * place(r) on; in pieces of 16 bytes
-// unless the bins start at an address that does not allow it (a caller's buffer).
+// All `rows` of a block (256 bytes each), row r to the 64 dwords from tile + 64 * place(r) on; four rows that start at a
+// multiple of four have places behind each other. In pieces of 16 bytes per lane, four rows to a wave's request, which go
+// into LDS without passing through registers, so that every request is on its way before the first has arrived; dword by dword
+// where the bins start at an address that does not allow it (a caller's buffer). A wave's requests have arrived behind
+// AwaitTile(); a barrier is the caller's. (Through registers, eight pieces to a batch, the compiler moved each load
+// behind the test of its own store: a trip to memory per piece. EvalNonSymmetricLdsKernel,
+// 1M documents * 500 trees over 300 features 1.240 -> 1.205 ms.)
 template <int THREADS, typename TPlace>
-__device__ __forceinline__ void CopyTile(const uint32_t* src, uint32_t rows, uint32_t tid, uint32_t* tile, const TPlace& place) {
+__device__ __forceinline__ void RequestTile(const uint32_t* src, uint32_t rows, uint32_t tid, uint32_t* tile, const TPlace& place) {
     if ((reinterpret_cast<uintptr_t>(src) & 15) == 0) {
-        CopyInBatches<THREADS>(reinterpret_cast<const uint4*>(src), rows * (kWave / 4), tid, [&](uint32_t i, const uint4& v) {
-            reinterpret_cast<uint4*>(tile)[place(i / (kWave / 4)) * (kWave / 4) + i % (kWave / 4)] = v;
-        });
+        const uint32_t lane = tid & (kWave - 1);
+        for (uint32_t row = __builtin_amdgcn_readfirstlane(tid / kWave) * 4; row < rows; row += THREADS / kWave * 4) {
+            if (row + lane / 16 < rows) {
+                __builtin_amdgcn_global_load_lds(
+                    reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(src + row * kWave + lane * 4)),
+                    (__attribute__((address_space(3))) void*)(tile + place(row) * kWave), 16, 0, 0);
+            }
+        }
     } else {
         CopyInBatches<THREADS>(src, rows * kWave, tid, [&](uint32_t i, uint32_t v) { tile[place(i / kWave) * kWave + i % kWave] = v; });
     }
 }
 
+__device__ __forceinline__ void AwaitTile() {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+}
+
 template <int THREADS>
 __device__ __forceinline__ void CopyTile(const uint32_t* src, uint32_t rows, uint32_t tid, uint32_t* tile) {
-    CopyTile<THREADS>(src, rows, tid, tile, [](uint32_t row) { return row; });
+    RequestTile<THREADS>(src, rows, tid, tile, [](uint32_t row) { return row; });
+    AwaitTile();
 }
 
 // Oblivious trees, any model: one wave per 256-document block, four documents per lane, leaf
@@ -2753,11 +2768,14 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalNonSymmetricTileKernel(
     }
 }
 
-// One-dimensional non-symmetric models without xor masks whose trees have at most kNsLdsEntries
-// entries, whole model: as EvalNonSymmetricTileKernel, but a wave walks its trees out of a copy in
-// its own LDS region (an LDS gather costs a fraction of a gather from global memory). Consecutive
-// trees are grouped into units of up to kNsUnitTrees trees and ENTRIES entries; a wave takes
-// a unit at a time and walks its trees side by side (4 documents x kNsUnitTrees chains per lane).
+// Non-symmetric models without xor masks whose trees have at most kNsLdsEntries entries: as EvalNonSymmetricTileKernel, but a
+// wave walks its trees out of a copy in its own LDS region (an LDS gather costs a fraction of a gather from global memory).
+// Trees are grouped into units of up to kNsUnitTrees trees and ENTRIES entries; a wave takes a unit at a time and walks its
+// trees side by side (4 documents x kNsUnitTrees chains per lane).
+// The top three levels of a tree are the same seven nodes for every document. They come with the unit's row in scalar
+// registers, padded to seven where a branch ends early (a node that is false for every bin), and are compared byte-parallel,
+// four documents to an instruction: a read of the bucket's bins and a v_lerp_u8 per node, whose bit 7 says bin >= split,
+// and selects by those bits. The three bits of a document choose one of the tree's first eight entries, its exits.
 // A compact entry is one dword:
 //   bits 0-7 splitIdx, bits 8-17 the 256-byte LDS row that holds the bucket's bins (so entry & 0x3ff00 is its
 //   address), bits 21-31 index of the left child relative to the unit's first entry.
@@ -2765,32 +2783,37 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalNonSymmetricTileKernel(
 // funnel shift {wave, entry} >> 19, because wave w keeps its entries at LDS address w * 8 KB. Regions shorter than
 // 8 KB leave gaps, and the rows of the bins fill them: NsLdsTileRow() says where bucket b goes, for the copy of
 // the tile here and for the entries on the host.
-// The kernel is bound by the latency of this chain of LDS reads, so the workgroup has as many waves as LDS has
-// room for: WAVES regions of ENTRIES entries, ENTRIES at least the largest tree of the model
-// (kNsLdsShapes in hip_evaluator.hip; 16 x 1024 to 4 x 2048).
-// The two children of a node sit side by side at an even index (the root is entry 0, entry 1 is
-// unused), so one 8-byte LDS read, issued together with the read of the node's bin, brings both
-// and the compare only selects: one LDS round trip per level. A terminal entry points at its own
+// The two children of a node sit side by side at an even index, so one 8-byte LDS read, issued together with the read of
+// the node's bin, brings both and the compare only selects: one LDS round trip per level. A terminal entry points at its own
 // pair and compares so that it selects itself (even index: splitIdx 255, false for every bin;
 // odd index: splitIdx 0, true for every bin, which no real split has). The next unit's entries
 // are fetched into registers while the current unit is walked: sixteen bytes per lane and whole rounds of
 // the wave, with neither bounds nor branches - every unit starts at a multiple of four entries and `entries`
 // ends with ENTRIES spare ones (a copy written with a test per round cost a taken branch each way per round,
 // a tenth of the kernel's time). valuesByEntry holds the leaf value of every terminal entry, indexed like
-// `entries`; a unit's values are requested behind its walk and added after the next unit's walk, two sets of
-// registers taking turns.
-// unitRows: 8 dwords per unit: first entry, height of the tallest tree, number of entries, first entry of the
-// second tree relative to the unit's, that of the third tree | number of trees << 16, and the model's numbers
+// `entries`, and ENTRIES rows of zeros behind them, which the trees that a unit lacks and those outside of the call's range
+// read; a unit's values are requested behind its walk and added after the next unit's walk. No load depends on a branch, so
+// that the wait for a unit's entries does not wait for the values requested behind them.
+// What bounds it: the walk's LDS reads and vector issue together (7.4 cycles of a CU for 64 chains' step; without bank conflicts
+// 6 % of the launch less, without the bins' reads 8 %, without the selects 12 %), and the values' gathers (12 of them a unit, some
+// 8 %). Whole call, with the root alone compared once for a lane's documents, the steps from there on, and values that a branch
+// guarded, and now: 4M documents, 500 trees of depth 10 over 300 features 6033 -> 5445 us; 1M, 500 of depth 6 over 60 686 -> 589, 300
+// of depth 8 over 150 675 -> 606, 500 of depth 9 over 20 (600 000 documents) 549 -> 491; three dimensions, 500 000 documents, 300
+// of depth 8 over 100 418 -> 413.
+// unitRows: 32 dwords per unit: first entry, steps behind the exits, first entry of the wave's next unit (WAVES on), first entry
+// of the second tree relative to the unit's, that of the third tree | number of trees << 16, and the model's numbers
 // of the three trees: a call for the trees [treeBegin, treeEnd) adds the values of those only and passes over
-// the units that hold none of them.
+// the units that hold none of them; from dword 8 on eight dwords per tree, its seven nodes by level (children of node n: 2 n + 1
+// and 2 n + 2): LDS row of the bins << 8 | (256 - splitIdx), low byte 0: false for every bin.
 // Models of several dimensions: a workgroup sums DIMS of them, those from blockIdx.y * DIMS on (every slice of
-// the dimensions walks the trees again), and valuesByEntry is [slice][entryCount] rows of DIMS values (zeros past
+// the dimensions walks the trees again), and valuesByEntry is [slice][entryCount + ENTRIES] rows of DIMS values (zeros past
 // the last dimension), so that a leaf's values come with one aligned load; they are read and added right behind
 // the unit's walk, with the other waves of the SIMD to cover the wait.
 // grid = (doc blocks, ceil(dim / DIMS)), block = 64 * WAVES, dynamic LDS = NsLdsTileRows(buckets, WAVES, ENTRIES) * 256
 // + 256 * 8 * DIMS bytes; no other LDS in the kernel.
 constexpr int kNsLdsEntries = 2048;
 constexpr int kNsUnitTrees = 3;
+constexpr int kNsUnitDwords = 32;
 
 // The 256-byte LDS row of bucket b's bins: the 8 KB of a wave start with its entries (entries / 64 rows) and the
 // rows that are left take bins; the other buckets follow the last wave's 8 KB.
@@ -2822,14 +2845,30 @@ __device__ __forceinline__ double LeafRowValue(const double4& row, int k) {
     return k == 0 ? row.x : k == 1 ? row.y : k == 2 ? row.z : row.w;
 }
 
+// Bits of `ones` where those of `mask` are set, of `zeros` elsewhere: v_bitop3 of vector registers, which takes half the time of
+// the v_bfi that the expression compiles to.
+__device__ __forceinline__ uint32_t SelectBits(uint32_t mask, uint32_t ones, uint32_t zeros) {
+    uint32_t r;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xca" : "=v"(r) : "v"(mask), "v"(ones), "v"(zeros));
+    return r;
+}
+
+// (bits & mask) | base, in the same class of instruction
+__device__ __forceinline__ uint32_t AndOr(uint32_t bits, uint32_t mask, uint32_t base) {
+    uint32_t r;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xea" : "=v"(r) : "v"(bits), "v"(mask), "v"(base));
+    return r;
+}
+
 template <int WAVES, int ENTRIES, int DIMS>
 __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
     const uint32_t* __restrict__ bins, size_t docCount, uint32_t bucketCount, const uint32_t* __restrict__ entries,
-    const uint4* __restrict__ unitRows, uint32_t unitCount, const double* __restrict__ valuesByEntry,
+    const uint32_t* __restrict__ unitRows, uint32_t unitCount, const double* __restrict__ valuesByEntry,
     const double* __restrict__ bias, double scale, uint32_t dim, uint32_t entryCount, uint32_t treeBegin,
-    uint32_t treeEnd, double* __restrict__ out) {
+    uint32_t treeEnd, uint32_t wholeModel, double* __restrict__ out) {
     constexpr int kFetch = ENTRIES / (4 * kWave);  // rounds of a wave's copy, sixteen bytes per lane
     static_assert(ENTRIES <= kNsLdsEntries && ENTRIES % (4 * kWave) == 0, "a region holds whole rounds of a wave's copy");
+    static_assert((32 - ENTRIES / 64) % 4 == 0, "the tile is requested four rows at a time");
     extern __shared__ uint32_t sTile[];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (kWave - 1);
@@ -2846,32 +2885,41 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
     // unit's are never followed).
     using TEntries4 = uint32_t __attribute__((ext_vector_type(4)));
     TEntries4 fetched[kFetch];
-#define CBAMD_STORE_UNIT()                                                                                  \
-    do {                                                                                                    \
-        _Pragma("unroll") for (int i = 0; i < kFetch; ++i) {                                                \
-            reinterpret_cast<TEntries4*>(sEntries)[i * kWave + lane] = fetched[i];                          \
-        }                                                                                                   \
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");                                              \
-        __builtin_amdgcn_wave_barrier();                                                                    \
-    } while (0)
-#define CBAMD_FETCH_UNIT(rowValue)                                                                          \
-    do {                                                                                                    \
-        const uint32_t fFirst = __builtin_amdgcn_readfirstlane((rowValue).x);                               \
-        const TEntries4* fSource = reinterpret_cast<const TEntries4*>(entries + fFirst) + lane;             \
-        _Pragma("unroll") for (int i = 0; i < kFetch; ++i) {                                                \
-            fetched[i] = fSource[i * kWave];                                                                \
-        }                                                                                                   \
-    } while (0)
+    const auto fetchUnit = [&](uint32_t firstEntry) {
+        const TEntries4* source = reinterpret_cast<const TEntries4*>(entries + firstEntry) + lane;
+#pragma unroll
+        for (int i = 0; i < kFetch; ++i) {
+            fetched[i] = source[i * kWave];
+        }
+    };
+    // whether a unit holds a tree of the call's range
+    const auto anyWanted = [&](uint32_t unit) {
+        const uint32_t* r = unitRows + unit * kNsUnitDwords;
+        const uint32_t trees = r[4] >> 16, range = treeEnd - treeBegin;
+        return r[5] - treeBegin < range || (trees > 1 && r[6] - treeBegin < range) || (trees > 2 && r[7] - treeBegin < range);
+    };
+    const auto skipUnwanted = [&](uint32_t unit) {
+        while (unit < unitCount && !anyWanted(unit)) {
+            unit += WAVES;
+        }
+        return unit;
+    };
 
-    uint32_t u = wave;
-    uint4 row = make_uint4(0, 0, 0, 0), row2 = make_uint4(0, 0, 0, 0);
+    RequestTile<64 * WAVES>(src, bucketCount, tid, sTile, [](uint32_t bucket) { return NsLdsTileRow(bucket, WAVES, ENTRIES); });
+    const auto unitBehind = [&](uint32_t unit) { return wholeModel ? unit + WAVES : skipUnwanted(unit + WAVES); };
+    uint32_t u = wholeModel ? wave : skipUnwanted(wave);
+    uint32_t row[kNsUnitDwords];
+    const auto loadRow = [&](uint32_t unit) {
+#pragma unroll
+        for (int i = 0; i < kNsUnitDwords; ++i) {
+            row[i] = unitRows[unit * kNsUnitDwords + i];
+        }
+    };
     if (u < unitCount) {
-        row = unitRows[2 * u];
-        row2 = unitRows[2 * u + 1];
-        CBAMD_FETCH_UNIT(row);
+        loadRow(u);
+        fetchUnit(row[0]);
     }
-    // the tile, behind the request for the first unit
-    CopyTile<64 * WAVES>(src, bucketCount, tid, sTile, [](uint32_t bucket) { return NsLdsTileRow(bucket, WAVES, ENTRIES); });
+    AwaitTile();
     __syncthreads();  // tile is loaded
 
     double acc[4][DIMS];
@@ -2882,76 +2930,74 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
             acc[j][k] = 0.0;
         }
     }
-    // one dimension: a unit's values are requested behind its walk and added behind the next unit's. Two sets
-    // of them take turns (the loop below is written out for two units), so that the loads of one unit never
-    // wait for registers that the sums of the unit before still read.
-    double pending[2][kNsUnitTrees][4];
+    // one dimension: a unit's values are requested behind its walk and added behind the next unit's
+    double pending[kNsUnitTrees][4];
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
+    for (int g = 0; g < kNsUnitTrees; ++g) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            pending[g][j] = 0.0;
+        }
+    }
+    const auto addPending = [&]() {
 #pragma unroll
         for (int g = 0; g < kNsUnitTrees; ++g) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                pending[p][g][j] = 0.0;
+                acc[j][0] = __dadd_rn(acc[j][0], pending[g][j]);
             }
         }
-    }
-    int lastSet = -1;  // the set whose values are not added yet
+    };
+    uint32_t next = unitBehind(u);
     const uint32_t d0 = blockIdx.y * DIMS;
-    const double* sliceValues = valuesByEntry + static_cast<size_t>(blockIdx.y) * entryCount * DIMS;
-    const auto walkUnit = [&](double (&mineSet)[kNsUnitTrees][4], const double (&otherSet)[kNsUnitTrees][4]) {
-        const uint32_t first = __builtin_amdgcn_readfirstlane(row.x);
-        const uint32_t height = __builtin_amdgcn_readfirstlane(row.y);
-        const uint32_t packed = __builtin_amdgcn_readfirstlane(row2.x);
-        const uint32_t trees = packed >> 16;
+    const double* sliceValues = valuesByEntry + static_cast<size_t>(blockIdx.y) * (entryCount + ENTRIES) * DIMS;
+    const uint32_t mask80 = 0x80808080u, maskC0 = 0xc0c0c0c0u;
+    while (u < unitCount) {
+        const uint32_t first = row[0], steps = row[1], trees = row[4] >> 16;
         // trees the unit does not have walk its first tree again; their values are not added
-        const uint32_t start[kNsUnitTrees] = {0u, trees > 1 ? __builtin_amdgcn_readfirstlane(row.w) : 0u,
-                                              trees > 2 ? (packed & 0xffffu) : 0u};
-        const uint32_t treeOf[kNsUnitTrees] = {static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(row2.y)),
-                                               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(row2.z)),
-                                               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(row2.w))};
+        const uint32_t start[kNsUnitTrees] = {0u, row[3], row[4] & 0xffffu};
         bool wanted[kNsUnitTrees];
-        bool anyWanted = false;
 #pragma unroll
         for (int g = 0; g < kNsUnitTrees; ++g) {
-            wanted[g] = static_cast<uint32_t>(g) < trees && treeOf[g] - treeBegin < treeEnd - treeBegin;
-            anyWanted = anyWanted || wanted[g];
+            wanted[g] = static_cast<uint32_t>(g) < trees && row[5 + g] - treeBegin < treeEnd - treeBegin;
         }
-        if (anyWanted) {
-            // the previous unit's reads were issued before these stores and LDS serves one wave in order
-            CBAMD_STORE_UNIT();
+        // the previous unit's reads were issued before these stores and LDS serves one wave in order
+#pragma unroll
+        for (int i = 0; i < kFetch; ++i) {
+            reinterpret_cast<TEntries4*>(sEntries)[i * kWave + lane] = fetched[i];
         }
-        const uint32_t uNext = u + WAVES;
-        uint4 rowNext = make_uint4(0, 0, 0, 0), row2Next = make_uint4(0, 0, 0, 0);
-        if (uNext < unitCount) {
-            rowNext = unitRows[2 * uNext];
-            row2Next = unitRows[2 * uNext + 1];
-            CBAMD_FETCH_UNIT(rowNext);
-        }
-        // The first step starts at the root for all four documents of a lane: one read of the children, one of the
-        // four bins (a terminal root selects itself like any other terminal entry, so the step is safe for a tree
-        // of one leaf).
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        // (behind the last unit one again)
+        fetchUnit(wholeModel ? row[2] : unitRows[min(next, unitCount - 1) * kNsUnitDwords]);
+        // the top three levels
         uint32_t entry[kNsUnitTrees][4];
+        uint32_t bins4[kNsUnitTrees][7];
 #pragma unroll
         for (int g = 0; g < kNsUnitTrees; ++g) {
-            const uint32_t rootEntry = anyWanted ? sEntries[start[g]] : 0u;
-            if (anyWanted && height > 0) {
-                const uint64_t pair = LdsLoad<uint64_t>(__builtin_amdgcn_alignbit(wave, rootEntry, 19));
-                uint32_t binAddr;
-                asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(binAddr) : "v"(rootEntry), "s"(bucketMask), "v"(laneOff));
-                const uint32_t bins4 = LdsLoad<uint32_t>(binAddr);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    entry[g][j] = static_cast<uint32_t>(((bins4 >> (8 * j)) & 0xffu) >= (rootEntry & 0xffu) ? pair >> 32 : pair);
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    entry[g][j] = rootEntry;
-                }
+            for (int n = 0; n < 7; ++n) {
+                bins4[g][n] = LdsLoad<uint32_t>((row[8 + 8 * g + n] & bucketMask) | laneOff);
             }
         }
-        for (uint32_t step = 1; step < (anyWanted ? height : 0u); ++step) {
+#pragma unroll
+        for (int g = 0; g < kNsUnitTrees; ++g) {
+            uint32_t side[7];  // bit 7 of every byte: the document goes right
+#pragma unroll
+            for (int n = 0; n < 7; ++n) {
+                side[n] = __builtin_amdgcn_lerp(bins4[g][n], (row[8 + 8 * g + n] & 0xffu) * 0x01010101u, 0);
+            }
+            const uint32_t second = SelectBits(side[0], side[2], side[1]);
+            const uint32_t third = SelectBits(side[0], SelectBits(second, side[6], side[5]), SelectBits(second, side[4], side[3]));
+            const uint32_t path = SelectBits(maskC0, SelectBits(mask80, side[0], second >> 1), third >> 2);  // bits 5 to 7
+            const uint32_t exits = wave * (kNsLdsEntries * 4) + start[g] * 4;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                entry[g][j] = LdsLoad<uint32_t>(AndOr(path >> (8 * j + 3), 0x1cu, exits));
+            }
+        }
+        loadRow(min(next, unitCount - 1));
+        for (uint32_t step = 0; step < steps; ++step) {
             uint64_t pair[kNsUnitTrees][4];  // the two children of a chain's node, left in the low half
             uint32_t bin[kNsUnitTrees][4];
 #pragma unroll
@@ -2962,9 +3008,7 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
                     // bits 18-20 of an entry are clear: e >> 19 is the byte offset of the pair of children in
                     // the wave's region, whose number comes in from above (kNsLdsEntries * 4 = 1 << 13)
                     pair[g][j] = LdsLoad<uint64_t>(__builtin_amdgcn_alignbit(wave, e, 19));
-                    uint32_t binAddr;
-                    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(binAddr) : "v"(e), "s"(bucketMask), "v"(laneOff));
-                    bin[g][j] = LdsLoad<uint8_t>(binAddr + j);
+                    bin[g][j] = LdsLoad<uint8_t>(AndOr(e, bucketMask, laneOff) + j);
                 }
             }
 #pragma unroll
@@ -2975,34 +3019,27 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
                 }
             }
         }
-        uint32_t idx[kNsUnitTrees][4];
+        // eight times a terminal entry's place in the unit: that of its pair, and one more for the right one (splitIdx 0, else 255)
+        uint32_t place[kNsUnitTrees][4];
 #pragma unroll
         for (int g = 0; g < kNsUnitTrees; ++g) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                idx[g][j] = (entry[g][j] >> 21) + ((entry[g][j] & 0xffu) == 0 ? 1u : 0u);
+                place[g][j] = (entry[g][j] >> 18) | (~entry[g][j] & 8u);
             }
         }
         if constexpr (DIMS == 1) {
+            addPending();
 #pragma unroll
             for (int g = 0; g < kNsUnitTrees; ++g) {
+                // the requests stay behind the sums: the values then have the same registers in every turn, where other ones
+                // would be waited for and moved
+                asm volatile("" : "+v"(acc[0][0]), "+v"(acc[1][0]), "+v"(acc[2][0]), "+v"(acc[3][0]), "+v"(place[g][0]), "+v"(place[g][1]),
+                                  "+v"(place[g][2]), "+v"(place[g][3]));
+                const char* from = reinterpret_cast<const char*>(valuesByEntry + (wanted[g] ? first : entryCount));
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    acc[j][0] = __dadd_rn(acc[j][0], otherSet[g][j]);
-                }
-            }
-#pragma unroll
-            for (int g = 0; g < kNsUnitTrees; ++g) {
-                if (wanted[g]) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        mineSet[g][j] = valuesByEntry[first + idx[g][j]];
-                    }
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        mineSet[g][j] = 0.0;
-                    }
+                    pending[g][j] = *reinterpret_cast<const double*>(from + place[g][j]);
                 }
             }
         } else {
@@ -3013,7 +3050,7 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
                     TLeafRow value[4];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        value[j] = reinterpret_cast<const TLeafRow*>(sliceValues)[first + idx[g][j]];
+                        value[j] = reinterpret_cast<const TLeafRow*>(sliceValues)[first + place[g][j] / 8];
                     }
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
@@ -3026,34 +3063,11 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
             }
         }
         __builtin_amdgcn_wave_barrier();
-        u = uNext;
-        row = rowNext;
-        row2 = row2Next;
-    };
-    while (u < unitCount) {
-        walkUnit(pending[0], pending[1]);
-        lastSet = 0;
-        if (u >= unitCount) {
-            break;
-        }
-        walkUnit(pending[1], pending[0]);
-        lastSet = 1;
+        u = next;
+        next = unitBehind(u);
     }
-#undef CBAMD_FETCH_UNIT
-#undef CBAMD_STORE_UNIT
     if constexpr (DIMS == 1) {
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            if (lastSet == p) {
-#pragma unroll
-                for (int g = 0; g < kNsUnitTrees; ++g) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        acc[j][0] = __dadd_rn(acc[j][0], pending[p][g][j]);
-                    }
-                }
-            }
-        }
+        addPending();
     }
     // waves add their partial sums in wave order into the LDS accumulator; the last wave
     // finishes the values and writes them out

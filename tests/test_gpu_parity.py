@@ -130,6 +130,54 @@ def test_non_symmetric_models_with_one_hot_splits(seed, n_float, n_cat, trees, m
     _close(g.calc_flat(x), o.calc(x))
 
 
+@pytest.mark.parametrize("dim", [1, 2])
+@pytest.mark.parametrize("border_of", [30, 254])
+def test_non_symmetric_trees_that_end_in_their_top_levels(border_of, dim):
+    """The LDS walk compares the top three levels byte-parallel and continues from eight exits: trees of a single leaf, branches
+    that end at every level, chains to either side, levels that are all there, a one-hot split whose left side, which is repeated
+    behind its second test, is the deeper one; splits and bins up to the most borders a bucket has; ranges of the trees."""
+    rng = np.random.default_rng(border_of + dim)
+    borders = [float(b) for b in np.arange(border_of)]
+    ffs = [mb.float_feature(i) for i in range(6)]
+    cats = [mb.cat_feature(0, 6), mb.cat_feature(1, 7)]
+    hashes = [11, -5, 7]
+    leaf = lambda: mb.leaf_node([float(v) for v in rng.normal(size=dim)] if dim > 1 else float(rng.normal()))  # noqa: E731
+    split = lambda: ("float", int(rng.integers(6)), borders[int(rng.choice([0, border_of - 1, rng.integers(border_of)]))])  # noqa: E731
+
+    def grown(depth, p_leaf):
+        if depth == 0 or rng.random() < p_leaf:
+            return leaf()
+        return mb.split_node(split(), grown(depth - 1, p_leaf), grown(depth - 1, p_leaf))
+
+    def chain(depth, side):
+        node = leaf()
+        for _ in range(depth):
+            node = mb.split_node(split(), *((node, leaf()) if side == 0 else (leaf(), node)))
+        return node
+
+    heads = [leaf(), mb.split_node(split(), leaf(), leaf()), grown(3, 0.0), grown(4, 0.0)]
+    heads += [chain(depth, side) for depth in (2, 3, 4, 5, 9) for side in (0, 1)]
+    for h in (11, 7):
+        heads.append(mb.split_node(("onehot", 0, h), chain(4, 1), leaf()))
+        heads.append(mb.split_node(split(), leaf(), mb.split_node(("onehot", 1, h), chain(3, 0), leaf())))
+        heads.append(mb.split_node(("onehot", 0, h), mb.split_node(("onehot", 1, -5), grown(3, 0.0), leaf()), leaf()))
+    heads += [grown(int(rng.integers(1, 9)), 0.2) for _ in range(40)]
+    # every border and category in use, so that bins reach the largest value
+    heads += [mb.split_node(("float", 0, b), leaf(), leaf()) for b in borders]
+    heads += [mb.split_node(("onehot", c, h), leaf(), leaf()) for c in (0, 1) for h in hashes]
+    model = mb.build_non_symmetric(ffs, cats, dim, heads, scale=0.5, bias=list(rng.normal(size=dim)))
+    docs = 1100
+    x = np.empty((docs, 8), np.float32)
+    x[:, :6] = rng.integers(-1, border_of + 1, size=(docs, 6)) + rng.choice([0.0, 0.5], size=(docs, 6))
+    x[:, 6:] = rng.choice(np.array(hashes + [99], np.int32), size=(docs, 2)).astype(np.int32).view(np.float32)
+    o = OracleModel(model)
+    g = _gpu_model(model)
+    assert "EvalNonSymmetricLdsKernel" in g.evaluator().describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"]
+    _close(g.calc_flat(x), o.calc(x))
+    for begin, end in ((3, len(heads) - 1), (0, len(heads) // 2), (len(heads) // 3, len(heads))):
+        _close(g.calc_flat(x, tree_start=begin, tree_end=end), o.calc(x, tree_start=begin, tree_end=end))
+
+
 @pytest.mark.parametrize("seed,dim,n_float,n_cat,trees,max_depth,docs", [
     (1, 2, 30, 0, 120, 8, 3000), (2, 3, 150, 3, 60, 9, 1000), (3, 4, 8, 4, 25, 6, 257), (4, 5, 40, 0, 200, 5, 5000),
     (5, 10, 60, 2, 90, 7, 2049), (6, 13, 12, 0, 33, 10, 64),
