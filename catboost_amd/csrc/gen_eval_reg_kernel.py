@@ -108,8 +108,8 @@ SHAPES = [
     (224, 4, 1, 256), (208, 4, 1, 256), (200, 4, 1, 256), (96, 8, 1, 256),
     (224, 4, 1, 64), (208, 4, 1, 64), (200, 4, 1, 64), (128, 4, 1, 64), (96, 8, 1, 64),
     (192, 4, 2, 64), (160, 4, 4, 64), (128, 4, 6, 64),
-    # Fewer buckets: three or four waves per SIMD instead of two; and three dimensions, whose odd one is a piece of eight
-    # bytes per leaf: LDS bounds these kernels, and a fourth dimension of padding is a quarter of its reads. 1M documents,
+    # Fewer buckets: three or four waves per SIMD instead of two; and three dimensions: LDS bounds these kernels, and a
+    # fourth dimension of padding is a quarter of its reads. (Measured with pieces of two dimensions:) 1M documents,
     # 1000 trees: three dimensions, 60 buckets 559 -> 446 us, 100 621 -> 506, 120 636 -> 528; seven as 4 + 3 1125 -> 1009,
     # nine as 6 + 3 1388 -> 1271; two over 70 buckets 367 -> 350, six over 50 812 -> 791. (Of eight waves per workgroup: 30 000
     # documents 2 to 4 % slower than before. Four dimensions over 48 buckets at four waves: 1 %, not kept.)
@@ -183,7 +183,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     row_dwords = 32 if mixed or deep else 16      # level table of a tree
     tree_row_bytes = row_dwords * 4
     rows_a, rows_b = 32, 32 + row_dwords  # the two sets of scalar registers holding level tables
-    odd = pitch > 1 and pitch % 2 == 1    # the last dimension's values stand alone, eight bytes per leaf
     threads = waves * 64
     row_bytes = threads * 16              # one 16-byte piece per thread of a leaf table copy
     # (six-level fused kernels: the 32 KB buffers of the border images hold 64 trees of 64 leaves)
@@ -193,7 +192,14 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     block = step * leaves // table_leaves  # trees of a buffer: whole steps
     buf_bytes = block * tree_bytes
     lds_bytes = 2 * buf_bytes
-    unpack_scale = (8 if pitch == 1 else 16) >> max(8 - depth, 0)  # bytes of a table per unit of an index byte
+    # Several dimensions: with 64 leaves a tree's values are a piece of 64 doubles per dimension, with 256 pieces of two dimensions,
+    # 16 bytes per leaf. LDS serves 32 lanes' 8-byte reads at a time from 32 banks (and 16 lanes' 16-byte reads from 16): 64 random
+    # leaves of 8 bytes take 4.2 cycles a wave, of 16 bytes 10.1; 256 leaves 6.5 and 11.9 (conflict-free 2.4 and 4.4). Per tree, wave
+    # and SIMD, pieces of 16 bytes and of 8 (2M documents, 1024 trees): 64 leaves, six dimensions 227 and 202 ns, four 147
+    # and 129, three 113 and 101, two 72 and 64; 256 leaves, six dimensions 314 and 362, two 99 and 110.
+    piece_dims = 2 if pitch > 1 and leaves > 64 else 1
+    assert pitch % piece_dims == 0
+    unpack_scale = 8 * piece_dims >> max(8 - depth, 0)  # bytes of a table per unit of an index byte
     assert buf_bytes % row_bytes == 0 and lds_bytes <= 65536
     # A wave copies its own contiguous share of a tree block, 1 KB (16 bytes per lane) per instruction;
     # up to four instructions of a group differ only in the immediate offset, which moves the source
@@ -773,9 +779,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     e("  s_mov_b32 s22, 0x80808080")
     # byte j of the leaf indexes times the unpacking weight = offset of the document's leaf row in a tree's table
     # (a six-level index sits in bits 2..7 of its byte); deep kernels: a ten-bit index times s23
-    # (tables of several dimensions hold a tree's values as pieces of two dimensions, each piece an array of
-    # 16 bytes per leaf: a wave's 16-byte gathers then spread over all sixteen groups of four LDS banks, which
-    # leaf rows of 32 bytes would not; an odd last dimension is a piece of eight bytes per leaf)
     if deep:
         e("  s_mov_b32 s23, 8")
     e("  s_mul_i32 s100, s20, %d" % wave_bytes)  # offset of the wave's share of a tree block
@@ -998,17 +1001,10 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 add_leaf_values(two_sets and not mine)
                 load_rows(rows, buf * block + i + 2)
             for j in range(4):
-                if pitch == 1:
-                    e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, 0, mine), lv(j, 0, mine) + 1, ga0 + j, tree_offset))
-                    continue
-                for k in range(0, pitch - 1, 2):
-                    e("  ds_read_b128 v[%d:%d], v%d offset:%d" % (lv(j, k), lv(j, k) + 3, ga0 + j,
-                                                                 tree_offset + (k // 2) * leaves * 16))
-                if odd:
-                    # half the place: pieces of eight bytes
-                    e("  v_ashrrev_i32_e32 v%d, 1, v%d" % (te0, ga0 + j))
-                    e("  ds_read_b64 v[%d:%d], v%d offset:%d" % (lv(j, pitch - 1), lv(j, pitch - 1) + 1, te0,
-                                                                tree_offset + (pitch // 2) * leaves * 16 - unpack_scale * 64))
+                for k in range(0, pitch, piece_dims):
+                    first = lv(j, k, mine)
+                    e("  ds_read_b%d v[%d:%d], v%d offset:%d" % (64 * piece_dims, first, first + 2 * piece_dims - 1, ga0 + j,
+                                                                tree_offset + k * leaves * 8))
             # copy of the next tree block into the other buffer, spread over this block's trees
             for g in range(len(groups)):
                 if g * block // len(groups) == i:

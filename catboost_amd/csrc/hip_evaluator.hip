@@ -2887,10 +2887,10 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     for (int d = 0; d < depth; ++d) {
                         modelLeaf |= ((leaf >> d) & 1) << levelOrder[t][d];
                     }
-                    // pieces of two dimensions, 16 bytes per leaf and piece; an odd last dimension, as one alone: a value per leaf
+                    // 64 leaves: a piece per dimension; 256: pieces of two dimensions, 16 bytes per leaf
                     for (size_t k = 0; k < launchPitch && launch * pitch + k < static_cast<size_t>(m.Dim); ++k) {
-                        const bool alone = k + 1 == launchPitch && k % 2 == 0;  // the odd last dimension
-                        const size_t slot = (k / 2) * rowsPerTree * 2 + (alone ? leaf : leaf * 2 + k % 2);
+                        const size_t slot = rowsPerTree == 64 || launchPitch == 1 ? k * rowsPerTree + leaf
+                                                                                  : (k / 2) * rowsPerTree * 2 + leaf * 2 + k % 2;
                         table[slot] = values[modelLeaf * m.Dim + launch * pitch + k];
                     }
                 }

@@ -322,8 +322,6 @@ def _places(code, scalars, bins, bins_at, weight):
             for j in range(4):
                 v[first + j] = weight * _signed(bytes_of(v[3])[j])
             product_at = at
-        elif op == "v_ashrrev_i32_e32":
-            v[int(args[0][1:])] = v[int(args[2][1:])] >> int(args[1])
         elif op.startswith("ds_read"):
             assert at - product_at > 5
             found = re.match(r"ds_read_b(64|128) v\[\d+:\d+\], v(\d+) offset:(\d+)$", c)
@@ -333,7 +331,7 @@ def _places(code, scalars, bins, bins_at, weight):
     return gathers
 
 
-@pytest.mark.parametrize("shape", [(128, 4, 1, 64), (96, 8, 1, 64), (200, 4, 1, 256), (104, 4, 3, 64), (56, 4, 6, 64)])
+@pytest.mark.parametrize("shape", [(128, 4, 1, 64), (96, 8, 1, 64), (200, 4, 1, 256), (104, 4, 3, 64), (56, 4, 6, 64), (160, 4, 4, 256)])
 @pytest.mark.parametrize("six", [False, True])
 def test_places_of_leaf_values(shape, six):
     """The levels' compares, their merges and the product, followed for one lane: the gathers name the leaves that comparing
@@ -345,7 +343,8 @@ def test_places_of_leaf_values(shape, six):
     text, _ = gen.gen_kernel(buckets, waves, pitch, leaves, False, six)
     lines = [line.strip() for line in text.split("\n")]
     start = next(i for i, line in enumerate(lines) if line.endswith("_loop:")) + 1
-    gathers = 4 * ((pitch + 1) // 2)
+    dims = 2 if leaves > 64 and pitch > 1 else 1  # of a piece of the table
+    gathers = 4 * pitch // dims
     code = []
     for line in lines[start:]:
         code.append(line)
@@ -353,7 +352,7 @@ def test_places_of_leaf_values(shape, six):
             break
     depth, top = (6 if leaves == 64 else 8), (64 if six else 128)
     bins_at = int(re.search(r"v_add_u32_e64 v\d+, v(\d+), s", text).group(1))
-    weight = (8 if pitch == 1 else 16) >> (8 - depth)
+    weight = 8 * dims >> (8 - depth)
     rng = random.Random(7)
     for _ in range(200):
         bins = [[rng.choice([0, 1, top // 2, top - 1, top, rng.randrange(top + 1)]) for _ in range(4)] for _ in range(buckets)]
@@ -365,10 +364,4 @@ def test_places_of_leaf_values(shape, six):
             for j in range(4):
                 expected[j] |= int(bins[bucket][j] >= split) << d
         got = _places(code, scalars, [sum(x << (8 * j) for j, x in enumerate(b)) for b in bins], bins_at, weight)
-        if pitch == 1:
-            assert got == [8 * x for x in expected]
-        else:
-            for j in range(4):
-                for k in range((pitch + 1) // 2):
-                    piece = (16 if 2 * k + 1 < pitch else 8) * expected[j] + k * leaves * 16
-                    assert got[j * ((pitch + 1) // 2) + k] == piece
+        assert got == [8 * dims * x + k * leaves * 8 for x in expected for k in range(0, pitch, dims)]
