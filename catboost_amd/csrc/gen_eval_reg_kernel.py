@@ -76,13 +76,19 @@ go through the same two LDS buffers as the tree blocks that follow them:
   * a lane owns the documents block * 256 + lane + 64 * j as before and reads its own rows, 16 bytes (four
     columns) per load, 64 bytes (a "unit" of sixteen columns = sixteen bins registers) per document and
     turn; the two units that share a 128-byte stretch of the rows are taken one right after the other;
-  * a value's bin is found as the HIP binarize kernel finds it: the value's cell in the bucket's uniform
-    grid of 256 cells, min(255, u32((v - lo) * scale)), indexes a byte table of search starts, and a
-    branch-free binary search over the next 2^steps - 1 borders finishes the count of borders below the
-    value; four columns of a document go through it side by side. steps (at most FUSED_MAX_STEPS) is
-    common to the four columns of a load;
-  * per unit a record of 40 dwords: sixteen lo, sixteen scale, a flags dword (bit q: the unit's q-th four
-    columns need four steps, bit 4 + q: three or more, bit 8 + q: two or more, bit 16 + i: NaN counts
+  * a value's bin is found as the HIP binarize kernel finds it, with cells of its own: the value's cell in the bucket's
+    grid of 256 cells, the nearest whole number of 255 * clamp((v - lo) * scale), columns 255 * clamp(fma(v, scale, bias)),
+    indexes a byte table of search starts, and a branch-free binary search over the next 2^steps - 1 borders finishes the
+    count of borders below the value; four columns of a document go through it side by side (columns: four documents
+    of a column, whose bias is moved to a vector register once for the four). steps (at most FUSED_MAX_STEPS) is
+    common to four columns, which are passed over where no split looks at any of them. Vector issue bounds the searches where
+    they are not hidden by the loads: per value of two steps 11 instructions, columns 9.25, where a cell by four of its own and fours
+    that no split looks at took 12. Whole calls: rows, 1M documents, 200 trees over 50 columns 102 -> 97 us, over 20 65.5 -> 63.7, 2M
+    over 33 149 -> 144, 4M, 1000 trees over 200 1571 -> 1559; columns, 1M, 1000 trees over 150 310 -> 301. (More loads of rows in
+    flight, the first document's straight into the bins registers: 102 -> 105 and 1565 -> 1675 us; 256 bytes of a row at a time 1650: what
+    L2 misses move, 1.4 to 1.6 times the rows, is near the rate that memory has.)
+  * per unit a record of 40 dwords: sixteen lo (columns: bias), sixteen scale, a flags dword (bit q: the unit's q-th four
+    columns need four steps, bit 4 + q: three or more, bit 8 + q: two or more, bit 12 + q: one or more, bit 16 + i: NaN counts
     as +inf in column i); behind the BUCKETS / 16 + 1 records, the units' byte offsets in a row.
 Column-major documents ("cbamd_fused_cols_..."): the bins registers follow the buckets, sixteen to a unit; behind the records
 sit, per unit, its sixteen columns instead of the units' byte offsets, and argument 96 is the bytes from a column to the next.
@@ -232,6 +238,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         row_off = [1, 3, 4, 5]            # byte offset of the lane's four rows from the block's first row
         srch_p = [6, 7, 8, 9]             # four searches side by side: position, border / scratch
         srch_b = [10, 11, 12, 13]
+        srch_bias = 14                    # (columns)
         # two sets of four 16-byte loads (first registers of the quads)
         values = [[16, 20, 24, high], [high + 4, high + 8, high + 12, high + 16]]
         assert b0 == 28
@@ -371,63 +378,71 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     # ---- the binarize phase's search, shared by the rows' and the columns' form
     out_of_line = []
 
-    def search_step(step, vals):
+    def search_step(step, vals, border_at):
         """Step `step` (counted from the last one, 1) of the four searches: looks at the border 2^(step-1)
         places on and moves on behind it when it lies below the value."""
         size = 4 << (step - 1)
         for d in range(4):
-            e("  ds_read_b32 v%d, v%d offset:%d" % (srch_b[d], srch_p[d], search_step.border_at[d] + size - 4))
+            e("  ds_read_b32 v%d, v%d offset:%d" % (srch_b[d], srch_p[d], border_at[d] + size - 4))
         e("  s_waitcnt lgkmcnt(0)")
         for d in range(4):
-            e("  v_cmp_lt_f32_e32 vcc, v%d, v%d" % (srch_b[d], vals + d))
+            e("  v_cmp_lt_f32_e32 vcc, v%d, v%d" % (srch_b[d], vals[d]))
             e("  v_cndmask_b32_e64 v%d, 0, %d, vcc" % (srch_b[d], size))
             e("  v_add_u32_e32 v%d, v%d, v%d" % (srch_p[d], srch_p[d], srch_b[d]))
 
-    def search_group(label, unit, j, q, vals, lo, scale, flags, buf):
-        """Columns 4 q .. 4 q + 3 of a unit for the lane's document j, whose values are in v[vals] .. v[vals + 3]: their
-        bins into byte j of the bins registers."""
-        local = (unit % (fused_layout(six)[0] // 16)) * 16 + 4 * q
-        search_step.border_at = [buf * buf_bytes + (local + d) * fused_layout(six)[1] for d in range(4)]
-        for d in range(4):
-            i = 4 * q + d
-            # the value's cell in the column's grid and the search start stored for it
-            e("  v_subrev_f32_e32 v%d, s%d, v%d" % (srch_b[d], lo + i, vals + d))
-            e("  v_mul_f32_e32 v%d, s%d, v%d" % (srch_b[d], scale + i, srch_b[d]))
-            e("  v_cvt_u32_f32_e32 v%d, v%d" % (srch_b[d], srch_b[d]))
-            e("  v_min_u32_e32 v%d, 0xff, v%d" % (srch_b[d], srch_b[d]))
-            e("  ds_read_u8 v%d, v%d offset:%d" % (srch_p[d], srch_b[d],
-                                                   buf * buf_bytes + 16384 + (local + d) * 256))
+    def search_group(label, unit, q, values_of, lo, scale, flags, buf):
+        """Four searches side by side among the columns 4 q .. 4 q + 3 of a unit: `values_of` are (column of the unit, document j,
+        register of the value) of each; the bins go into byte j of the column's bins register, first those of document 0. A
+        value's cell is the nearest whole number of 255 times its place between the lowest border and the highest one:
+        a product with the denormal number whose bits are 255 leaves the cell's number as the result's bits."""
+        columns_of = [column for column, _, _ in values_of]
+        vals = [reg for _, _, reg in values_of]
+        local = unit % (fused_layout(six)[0] // 16) * 16
+        border_at = [buf * buf_bytes + (local + column) * fused_layout(six)[1] for column in columns_of]
+        e("  s_bitcmp1_b32 s%d, %d" % (flags, 12 + q))  # else no split looks at the four columns
+        e("  s_cbranch_scc0 %s_none" % label)
+        if columns:
+            # a column's four documents: the bias as the one vector register that a product and sum may take it from
+            e("  v_mov_b32_e32 v%d, s%d" % (srch_bias, lo + columns_of[0]))
+        for d, column in enumerate(columns_of):
+            if columns:
+                e("  v_fma_f32 v%d, v%d, s%d, v%d clamp" % (srch_b[d], vals[d], scale + column, srch_bias))
+            else:
+                e("  v_subrev_f32_e32 v%d, s%d, v%d" % (srch_b[d], lo + column, vals[d]))
+                e("  v_mul_f32_e64 v%d, s%d, v%d clamp" % (srch_b[d], scale + column, srch_b[d]))
+            e("  v_mul_f32_e32 v%d, s23, v%d" % (srch_b[d], srch_b[d]))
+            e("  ds_read_u8 v%d, v%d offset:%d" % (srch_p[d], srch_b[d], buf * buf_bytes + 16384 + (local + column) * 256))
         e("  s_waitcnt lgkmcnt(0)")
         if not six:
             for d in range(4):
                 e("  v_lshlrev_b32_e32 v%d, 2, v%d" % (srch_p[d], srch_p[d]))
         # the search: steps above two are rare and sit out of line
         e("  s_bitcmp1_b32 s%d, %d" % (flags, 4 + q))
-        e("  s_cbranch_scc1 %s_q%d_hi" % (label, q))
-        e("%s_q%d_back:" % (label, q))
+        e("  s_cbranch_scc1 %s_hi" % label)
+        e("%s_back:" % label)
         e("  s_bitcmp1_b32 s%d, %d" % (flags, 8 + q))
-        e("  s_cbranch_scc0 %s_q%d_one" % (label, q))
-        search_step(2, vals)
-        e("%s_q%d_one:" % (label, q))
-        search_step(1, vals)
-        for d in range(4):
-            reg = b0 + unit * 16 + 4 * q + d
+        e("  s_cbranch_scc0 %s_one" % label)
+        search_step(2, vals, border_at)
+        e("%s_one:" % label)
+        search_step(1, vals, border_at)
+        for d, (column, j, _) in enumerate(values_of):
+            reg = b0 + unit * 16 + column
             if j == 0:
                 e("  v_lshrrev_b32_e32 v%d, 2, v%d" % (reg, srch_p[d]))
             else:
                 e("  v_lshl_add_u32 v%d, v%d, %d, v%d" % (reg, srch_p[d], 8 * j - 2, reg))
-        out_of_line.append((label, q, vals, list(search_step.border_at), flags))
+        e("%s_none:" % label)
+        out_of_line.append((label, q, vals, border_at, flags))
 
     def emit_out_of_line():
         for label, q, vals, border_at, flags in out_of_line:
-            search_step.border_at = border_at
-            e("%s_q%d_hi:" % (label, q))
+            e("%s_hi:" % label)
             e("  s_bitcmp1_b32 s%d, %d" % (flags, q))
-            e("  s_cbranch_scc0 %s_q%d_three" % (label, q))
-            search_step(4, vals)
-            e("%s_q%d_three:" % (label, q))
-            search_step(3, vals)
-            e("  s_branch %s_q%d_back" % (label, q))
+            e("  s_cbranch_scc0 %s_three" % label)
+            search_step(4, vals, border_at)
+            e("%s_three:" % label)
+            search_step(3, vals, border_at)
+            e("  s_branch %s_back" % label)
         del out_of_line[:]
 
     def binarize_columns(rec_lo, rec_scale, rec_fo):
@@ -501,9 +516,9 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                     e("  v_cndmask_b32_e32 v%d, v%d, v%d, vcc" % (reg, reg, srch_b[0]))
                 e("%s_n%d:" % (label, c))
             e("%s_n:" % label)
-            for j in range(4):
-                for h in (0, 1):
-                    search_group("%s_%d" % (label, j), unit, j, 2 * half + h, value_set[turn][2 * j + h], lo, scale, flags, buf)
+            for c in range(8):
+                search_group("%s_%d" % (label, c), unit, 2 * half + c // 4,
+                             [(8 * half + c, j, value_set[turn][2 * j + c // 4] + c % 4) for j in range(4)], lo, scale, flags, buf)
 
         # sets of registers for the turns in flight, as in the rows' form
         plan = []
@@ -602,6 +617,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  s_mov_b32 s24, s86")                     # s[24:25]: unit records, s28: units of the model
         e("  s_mov_b32 s25, s87")
         e("  s_mov_b32 s28, s89")
+        e("  s_movk_i32 s23, 0xff")                   # of search_group
         if columns:
             binarize_columns(rec_lo, rec_scale, rec_fo)
             return
@@ -661,7 +677,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 e("%s_n%d:" % (label, i))
             e("%s_n:" % label)
             for q in range(4):
-                search_group(label, unit, j, q, value_set[n][q], lo, scale, flags, buf)
+                search_group("%s_q%d" % (label, q), unit, q, [(4 * q + d, j, value_set[n][q] + d) for d in range(4)], lo, scale, flags, buf)
 
         # Two neighbouring units of a document (128 bytes of its row) are loaded together, eight loads one
         # behind the other, so that a line of the row is asked for once (the cache merges requests that

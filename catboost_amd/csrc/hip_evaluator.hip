@@ -597,6 +597,19 @@ struct TBucketGrid {
     uint32_t Start[dev::kLutCells] = {};
 };
 
+// Steps and starts from the borders of each cell
+void SetGridStarts(const uint32_t* population, TBucketGrid* g) {
+    const uint32_t tallest = *std::max_element(population, population + dev::kLutCells);
+    while ((1u << g->Steps) - 1 < tallest) {
+        ++g->Steps;
+    }
+    uint32_t start = 0;
+    for (int c = 0; c < dev::kLutCells; ++c) {
+        g->Start[c] = start;
+        start += population[c];
+    }
+}
+
 TBucketGrid MakeBucketGrid(const std::vector<float>& borders) {
     TBucketGrid g;
     if (borders.empty()) {
@@ -616,15 +629,30 @@ TBucketGrid MakeBucketGrid(const std::vector<float>& borders) {
     for (float x : borders) {
         ++population[GridCell(x, g.Lo, g.Scale)];
     }
-    const uint32_t tallest = *std::max_element(population, population + dev::kLutCells);
-    while ((1u << g.Steps) - 1 < tallest) {
-        ++g.Steps;
+    SetGridStarts(population, &g);
+    return g;
+}
+
+// The grid of the fused kernels: a value's cell is the nearest whole number of 255 times its place, clamped to 0 .. 1, in fp32. The place
+// rises with the value, so the borders of lower cells are below the value and those of higher cells are not.
+TBucketGrid MakeFusedGrid(const std::vector<float>& borders, bool columnMajor) {
+    TBucketGrid g;
+    if (borders.empty()) {
+        return g;
     }
-    uint32_t start = 0;
-    for (int c = 0; c < dev::kLutCells; ++c) {
-        g.Start[c] = start;
-        start += population[c];
+    const float span = borders.back() - borders.front();
+    const float scale = 1.0f / span, bias = -borders.front() * scale;
+    if (std::isfinite(span) && span > 0.0f && std::isfinite(scale) && std::isfinite(bias)) {
+        g.Lo = columnMajor ? bias : borders.front();
+        g.Scale = scale;
     }
+    uint32_t population[dev::kLutCells] = {};
+    for (float x : borders) {
+        const float place = columnMajor ? std::fma(x, g.Scale, g.Lo) : (x - g.Lo) * g.Scale;
+        const double clamped = place > 0.0f ? std::min(place, 1.0f) : 0.0f;  // (NaN: 0)
+        ++population[static_cast<uint32_t>(std::nearbyint(clamped * (dev::kLutCells - 1)))];
+    }
+    SetGridStarts(population, &g);
     return g;
 }
 
@@ -3024,7 +3052,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 const uint32_t n = offsets[b + 1] - offsets[b];
                 bordersOfSlot[slot].resize(n);
                 std::memcpy(bordersOfSlot[slot].data(), values.data() + offsets[b], n * sizeof(float));
-                grids[slot] = MakeBucketGrid(bordersOfSlot[slot]);
+                grids[slot] = MakeFusedGrid(bordersOfSlot[slot], columnMajor);
                 groupSteps[slot / 4] = std::max(groupSteps[slot / 4], grids[slot].Steps);
                 fits = fits && n <= slots;
             }
@@ -3055,6 +3083,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 if (b == UINT32_MAX) {
                     continue;  // a column no split reads: all-zero record and tables, its register is never indexed
                 }
+                record[32] |= 4096u << group;
                 std::memcpy(&record[column], &grids[slot].Lo, 4);
                 std::memcpy(&record[16 + column], &grids[slot].Scale, 4);
                 if (flags[b] & dev::kBucketFlagNanToInf) {

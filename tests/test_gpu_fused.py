@@ -251,3 +251,39 @@ def test_fused_six_level_walks_end_behind_any_sixteenth_tree(columns, trees, mon
     rng = np.random.default_rng(trees * 7 + columns)
     model = _bytes(_random_model(rng, columns, list(range(columns)), trees, 6, lambda f: rng.normal(0, 1, size=12)))
     _compare(model, rng.normal(0, 1, size=(1100, columns)).astype(np.float32), monkeypatch)
+
+
+@pytest.mark.parametrize("columns,used", [(20, list(range(20))), (40, [3, 4, 9, 21, 22, 23, 24, 33, 39]), (17, [16]), (90, list(range(0, 90, 5)))])
+@pytest.mark.parametrize("few", [True, False])
+def test_fused_grids_at_their_edges(columns, used, few, monkeypatch):
+    """Borders far from zero, a few denormal numbers apart, further apart than a float holds, one border, many in one cell; values
+    on them and next to them, infinities and NaN; sixteens and fours of columns of which splits look at some or none. Rows and
+    columns."""
+    import torch
+
+    rng = np.random.default_rng(columns + few)
+    count = 15 if few else 70  # the six-bit form and the other one
+
+    def borders_of(f):
+        n = rng.integers(1, count)
+        return [1e6 + rng.integers(0, 64, size=n) / 16.0, rng.integers(-7, 7, size=n) * 1.5e-45, [-3e38, 0.0, 3e38], [0.25],
+                rng.normal(size=n), [-0.0, 1e-30, 1.0], -1e20 - rng.random(n) * 1e15][f % 7]
+
+    model = _random_model(rng, columns, used, trees=300, depth=6, borders_of=borders_of, nan_true=set(used[::3]))
+    borders = {f: model["float_features"][f]["borders"] for f in used}
+    x = rng.normal(size=(3000, columns)).astype(np.float32)
+    for f, b in borders.items():
+        if len(b):
+            near = np.concatenate([b, np.nextafter(b, np.float32(np.inf)), np.nextafter(b, np.float32(-np.inf))])
+            x[100:, f] = rng.choice(near, size=2900)
+    x[rng.random(x.shape) < 0.02] = np.nan
+    x[rng.random(x.shape) < 0.02] = np.inf
+    x[rng.random(x.shape) < 0.02] = -np.inf
+    rows = _compare(_bytes(model), x, monkeypatch)
+    (_, fev), _ = _evaluators(_bytes(model), monkeypatch)
+    dx = torch.from_numpy(np.ascontiguousarray(x.T)).to("cuda:0")
+    out = torch.zeros(len(x), dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    fev.eval_data(fev.features(cb.LAYOUT_FLAT_COLUMNS, dx.data_ptr(), len(x)), len(x), out.data_ptr())
+    assert fev.last_kernel_times()[0] == 0.0, "the fused kernel did not run"
+    assert torch.equal(out, rows)
