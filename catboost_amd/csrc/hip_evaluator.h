@@ -81,6 +81,7 @@ public:
     // the trees in the slices of TreeSlicesFor. `source` and `results` may be device or pinned host memory. True when
     // such a call takes it.
     bool TakesSmallBatchKernel(size_t docCount, size_t treeStart, size_t treeEnd) const;
+    bool TakesSmallBatchOnDevice(size_t docCount, size_t treeStart, size_t treeEnd) const;
     // Small batches (fewer than 256 workgroups of the register kernels) are cut into slices of the trees by the
     // calls that own their scratch memory; off: every sum is one pass in tree order, the CPU evaluator's
     // order of additions, at the price of the small-batch speed-up. Set it before the calls it should govern.

@@ -659,9 +659,7 @@ TBucketGrid MakeFusedGrid(const std::vector<float>& borders, bool columnMajor) {
 constexpr size_t kMaxTileLdsBytes = 160 * 1024;
 
 // Batches of SmallBatchKernel and FewDocumentsKernel, in documents times passes over the dimensions; beyond come the binarize
-// and register kernels in slices of the trees, which one limit cannot meet at every model's crossing. Whole call for 16384
-// documents against those: 1000 trees of depth 8 over 200 features 40.5 and 38.5 us (14336 documents 39, 12288 34, 8192 28), 1000 of depth 6
-// 32 and 33, 500 26 and 28, 300 of depth 4 25 and 26. FewDocumentsKernel against SmallBatchKernel: 512 documents 18 against 21 us, 1024 24 against 21.
+// and register kernels in slices of the trees, for some models before (TakesSmallBatchOnDevice). FewDocumentsKernel against SmallBatchKernel: 512 documents 18 against 21 us, 1024 24 against 21.
 constexpr size_t kSmallBatchDocs = 16384;
 constexpr size_t kFewDocs = 640;
 // ... of host calls, whose features are at most so many bytes: more go through the pipeline of chunks
@@ -4105,6 +4103,20 @@ bool THipEvaluator::TakesSmallBatchKernel(size_t docCount, size_t treeStart, siz
            treeEnd == TreeCount && m.SmallLdsBytes() <= kMaxTileLdsBytes;
 }
 
+// ... of calls whose features are on the device. Its time grows with the levels that a document walks, and by a step for every 4096
+// documents (a workgroup of sixteen more on every CU), the one of binarize and evaluate launches hardly, so models of many levels
+// take those earlier. Whole call, SmallBatchKernel and the launches: 1000 trees of depth 8 over 200 features, 8192 documents 29.5
+// and 32.4 us, 10 240 36.2 and 35.4, 12 400 43.2 and 36.9, 16 384 46.3 and 37.5 (columns of 50 features, 8300 documents 34.2 and 35.6, 16 384
+// 44.4 and 36.8); 1000 of depth 6 over 100, 12 288 30.1 and 31.5, 12 400 33.5 and 32.7, 16 384 35.3 and 32.8; 500 of depth 6
+// over 150, 16 384 28.1 and 30.7, 300 of depth 8 over 60 28.7 and 30.2. (One dimension on the register kernels; both add the same
+// slices. Other models keep the one limit.)
+bool THipEvaluator::TakesSmallBatchOnDevice(size_t docCount, size_t treeStart, size_t treeEnd) const {
+    const TImpl& m = *Impl;
+    const size_t levels = TreeCount * static_cast<size_t>(m.MaxDepth);
+    const size_t limit = levels <= 4000 ? kSmallBatchDocs : levels <= 6500 ? 12288 : 10240;
+    return TakesSmallBatchKernel(docCount, treeStart, treeEnd) && (m.Dim > 1 || TreeSlicesFor(docCount) <= 1 || docCount <= limit);
+}
+
 // One launch of the small-batch kernel whose end `stop` marks. `batch` and `results` may be device or pinned host memory.
 // `flagged`: the slot whose flags the workgroups of FewDocumentsKernel set (AwaitSmallBatch).
 static void LaunchSmallBatch(THipEvaluator::TImpl& m, THipEvaluator::TImpl::THostContext& ctx, const TFeatureBatch& batch,
@@ -4297,7 +4309,7 @@ std::string THipEvaluator::DescribeKernels(int layout, size_t docCount, size_t s
     if (const int fused = FusedLayoutFor(layout, stride, docCount, 0, TreeCount, false); fused >= 0) {
         return "fused=" + (fused == kFusedExchange ? m.FusedExchangeName : m.Fused[fused]->Name);
     }
-    if (TakesSmallBatchKernel(docCount, 0, TreeCount)) {
+    if (TakesSmallBatchOnDevice(docCount, 0, TreeCount)) {
         const bool few = m.TakesFewDocumentsKernel(docCount);
         return std::string("binarize=none;evaluate=") + (few ? "FewDocumentsKernel<" : "SmallBatchKernel<") + std::to_string(m.MaxDepth <= 6 ? 6 : 8) + ", " + std::to_string(m.SmallDims()) +
                ">, " + std::to_string(m.SmallSliceCount()) + " slices of the trees" +
@@ -4485,7 +4497,7 @@ void THipEvaluator::CalcDevice(const TFeatureBatch& batch, size_t docCount, size
     HIP_CHECK(hipSetDevice(m.DeviceId));
     TImpl::TContextLease ctx(m);
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : m.Stream;
-    if (TakesSmallBatchKernel(docCount, treeStart, treeEnd)) {
+    if (TakesSmallBatchOnDevice(docCount, treeStart, treeEnd)) {
         CheckBatch(batch, docCount);
         LaunchSmallBatch(m, *ctx, batch, docCount, results, s, ctx->Ev[2]);
         HIP_CHECK(hipEventSynchronize(ctx->Ev[2]));

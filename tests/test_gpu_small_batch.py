@@ -556,3 +556,24 @@ def test_slices_are_added_in_order(trees, dim):
 def test_few_slices_are_added_in_order(trees, dim):
     """Three loads in flight up to ten slices: a turn that ends in the last slice's again, whole turns, the first number with sixteen."""
     test_slices_are_added_in_order(trees, dim)
+
+
+@pytest.mark.parametrize("trees,limit", [(500, 16384), (501, 12288), (812, 12288), (813, 10240)])
+def test_small_batches_of_models_with_many_levels(trees, limit):
+    """Models of more levels leave the small-batch kernel for the binarize and register kernels earlier; both add the same slices."""
+    import torch
+
+    model, info = syn.build_model("C2", trees=trees)
+    model.enable_gpu_evaluation(0)
+    ev = model.evaluator()
+    x = syn.device_features(info, limit + 1)
+    out = []
+    for docs in (limit, limit + 1):
+        result = torch.full((docs,), -1.0, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        ev.eval_data(ev.features(cb.LAYOUT_FLAT_ROWS, x.data_ptr(), x.shape[1]), docs, result.data_ptr())
+        out.append(result)
+        assert ("SmallBatch" in ev.describe_kernels(cb.LAYOUT_FLAT_ROWS, docs)["evaluate"]) == (docs == limit)
+        assert (ev.last_kernel_times()[0] == 0.0) == (docs == limit)
+    assert torch.equal(out[0], out[1][:limit])
+    np.testing.assert_array_equal(model.calc_flat(x[-700:].cpu().numpy()), out[1][-700:].cpu().numpy())  # SmallBatchKernel, from host memory
