@@ -54,7 +54,7 @@ Kernel arguments (80 bytes):
   16 leaves      const double*   [(treeBlocks + 2) * TREE_BLOCK][LEAVES][PITCH] (fused kernels of six levels: [whole buffers of 64 trees, and two][64])
   24 out         double*         [docCount][dim]
   32 docCount    uint32          36 blockCount uint32 (ceil(docCount / 256), >= 1)
-  40 treeBlocks  uint32 (>= 1)   44 flags uint32 (bit 0: add the bias)
+  40 treeBlocks  uint32 (>= 1)   44 flags uint32 (bit 0: add the bias, bit 4: 64 leaves, several dimensions, the table is not folded)
   48 scale       double          56 bias const double* (first dimension of this launch)
   64 bucketCount uint32 (1 .. BUCKETS)                68 dim uint32
   72 first dimension of this launch uint32            76 dimensions to store uint32 (1 .. PITCH)
@@ -250,9 +250,14 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     # behind the bins: the two masks of the merges and the left operand of the product that turns indexes into addresses
     # (fused: registers that only the binarize phase uses)
     mask80 = high if fused else vgprs
-    mask_c0, unpack = mask80 + 1, mask80 + 2
+    mask_c0, unpack, fold = mask80 + 1, mask80 + 2, mask80 + 3
+    # Several dimensions: the leaf tables are folded (see the walk). Trees of five levels or less have no two rows to a bank, so the
+    # kernels of 64 leaves walk either kind of table (flags bit 4: as it is); the one of two dimensions and many buckets, whose
+    # vector issue is as busy, loses 4 % by it.
+    folded = pitch > 1 and not (leaves == 64 and buckets == 192)
+    both_tables = folded and leaves == 64
     if not fused:
-        vgprs += 2 if deep else 3
+        vgprs += 2 if deep else 4 if folded else 3
     two_sets = pitch == 1 and block % 2 == 0 and (fused or (vgprs + 8 <= 256 and waves_per_simd(vgprs + 8) == waves_per_simd(vgprs)))
     if two_sets:
         if fused:
@@ -932,6 +937,8 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  v_mov_b32_e32 v%d, 0" % r)          # leaf values in flight and the sums
     e("  v_mov_b32_e32 v%d, 0x80808080" % mask80)
     e("  v_mov_b32_e32 v%d, 0xc0c0c0c0" % mask_c0)
+    if folded:
+        e("  v_mov_b32_e32 v%d, 0x%x" % (fold, 0x01010101 * (0x80 - (1 << max(8 - depth, 0)))))
     if not deep:
         # row i of a product's left operand is lane i's of the four, byte k of it stands for byte k of the index
         e("  v_and_b32_e32 v5, 3, v0")
@@ -972,82 +979,99 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         # byte selectors of the two index words (s24 and s25 are free from here to the epilogue)
         e("  s_mov_b32 s24, 0x05010400")
         e("  s_mov_b32 s25, 0x07030602")
-    e("%s_loop:" % name)
-    for buf in range(2):
-        for i in range(block):
-            rows = rows_a if i % 2 == 0 else rows_b
-            if mixed:
-                label = "%s_t%d_%d" % (name, buf, i)
-                e("  s_bitcmp1_b32 s%d, 31" % rows)
-                e("  s_cbranch_scc1 %s_x" % label)
-                levels_in_pairs(rows, True)
-                e("  s_branch %s_j" % label)
-                e("%s_x:" % label)
-                levels_eight_bit(rows)
-                e("%s_j:" % label)
-            else:
-                levels_in_pairs(rows, not deep)
-            if deep:
-                levels_high(rows)
-            tree_offset = buf * buf_bytes + i * tree_bytes
-            if not deep:
-                tree_offset += unpack_scale * 128
+    def enter_loop():
+        if both_tables:
+            e("  s_bitcmp1_b32 s15, 4")
+            e("  s_cbranch_scc1 %s_plain" % name)
 
-            # The previous tree's leaf values have arrived (its levels and addresses were issued in between), and so has
-            # the next tree's row. With two sets of leaf values the trees of a block alternate between them (a block has
-            # an even number of trees, so the first tree of a block finds the last one's values in the second set).
-            mine = two_sets and i % 2 == 1
-            if deep:
+    enter_loop()
+    for fold_here, loop in ((folded, "_loop"), (False, "_plain"))[:2 if both_tables else 1]:
+        e("%s%s:" % (name, loop))
+        for buf in range(2):
+            for i in range(block):
+                rows = rows_a if i % 2 == 0 else rows_b
+                if mixed:
+                    label = "%s%s_t%d_%d" % (name, loop, buf, i)
+                    e("  s_bitcmp1_b32 s%d, 31" % rows)
+                    e("  s_cbranch_scc1 %s_x" % label)
+                    levels_in_pairs(rows, True)
+                    e("  s_branch %s_j" % label)
+                    e("%s_x:" % label)
+                    levels_eight_bit(rows)
+                    e("%s_j:" % label)
+                else:
+                    levels_in_pairs(rows, not deep)
+                if deep:
+                    levels_high(rows)
+                tree_offset = buf * buf_bytes + i * tree_bytes
+                if not deep:
+                    tree_offset += unpack_scale * 128
+
+                # The previous tree's leaf values have arrived (its levels and addresses were issued in between), and so has
+                # the next tree's row. With two sets of leaf values the trees of a block alternate between them (a block has
+                # an even number of trees, so the first tree of a block finds the last one's values in the second set).
+                mine = two_sets and i % 2 == 1
+                if deep:
+                    for j in range(4):
+                        e("  v_mul_u32_u24_sdwa v%d, s23, v%d dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_%d"
+                          % (ga0 + j, wd0 + j // 2, j % 2))
+                    e("  s_waitcnt lgkmcnt(0)")
+                    add_leaf_values(two_sets and not mine)
+                    load_rows(rows, buf * block + i + 2)
+                else:
+                    if fold_here:
+                        # The place of leaf l in its table is l ^ (l >> 1): the result of every level but the top one is compared with the
+                        # next one's. The leaves of an LDS bank are those that share the low bits of their places, and two of them
+                        # in neighbouring rows differ in every level: where levels are lopsided, the likely leaves of the rows fall on
+                        # different banks. 64 lanes' reads of 8 bytes among 64 leaves (borders drawn evenly) take 2.6 to 2.7 cycles of
+                        # LDS instead of 3.3 to 3.5. 2M documents x 2000 trees of depth 6: ten dimensions 4550 -> 4035 us, six 2838 ->
+                        # 2570, four 2005 -> 1875; of depth 8, three dimensions, 1M x 2000 1518 -> 1469. (One dimension, which vector issue
+                    # bounds: the two instructions cost 2 to 5 %.)
+                        e("  v_lshrrev_b32_e32 v4, 1, v3")
+                        e("  v_bitop3_b32 v3, v4, v%d, v3 bitop3:0x6a" % fold)
+                    # Places of the four documents' leaf values in the tree's table, a byte of the index for each document: a
+                    # product of 4 x 4 bytes for every four lanes, whose left operand has the bytes' weight on its diagonal,
+                    # leaves weight * byte in the four registers of every lane: one instruction instead of four SDWA
+                    # multiplications. Its bytes have a sign: with the top bit inverted they are index - 128, and the reads'
+                    # offsets add what is missing. The product needs two wait states behind the last select, the reads five
+                    # behind the product: the sums and the next row's request.
+                    e("  s_waitcnt lgkmcnt(0)")
+                    e("  s_nop 0")
+                    e("  v_mfma_i32_4x4x4_16b_i8 v[%d:%d], v%d, v3, 0" % (ga0, ga0 + 3, unpack))
+                    add_leaf_values(two_sets and not mine)
+                    load_rows(rows, buf * block + i + 2)
                 for j in range(4):
-                    e("  v_mul_u32_u24_sdwa v%d, s23, v%d dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_%d"
-                      % (ga0 + j, wd0 + j // 2, j % 2))
-                e("  s_waitcnt lgkmcnt(0)")
-                add_leaf_values(two_sets and not mine)
-                load_rows(rows, buf * block + i + 2)
-            else:
-                # Places of the four documents' leaf values in the tree's table, a byte of the index for each document: a
-                # product of 4 x 4 bytes for every four lanes, whose left operand has the bytes' weight on its diagonal,
-                # leaves weight * byte in the four registers of every lane: one instruction instead of four SDWA
-                # multiplications. Its bytes have a sign: with the top bit inverted they are index - 128, and the reads'
-                # offsets add what is missing. The product needs two wait states behind the last select, the reads five
-                # behind the product: the sums and the next row's request.
-                e("  s_waitcnt lgkmcnt(0)")
-                e("  s_nop 0")
-                e("  v_mfma_i32_4x4x4_16b_i8 v[%d:%d], v%d, v3, 0" % (ga0, ga0 + 3, unpack))
-                add_leaf_values(two_sets and not mine)
-                load_rows(rows, buf * block + i + 2)
-            for j in range(4):
-                for k in range(0, pitch, piece_dims):
-                    first = lv(j, k, mine)
-                    e("  ds_read_b%d v[%d:%d], v%d offset:%d" % (64 * piece_dims, first, first + 2 * piece_dims - 1, ga0 + j,
-                                                                tree_offset + k * leaves * 8))
-            # copy of the next tree block into the other buffer, spread over this block's trees
-            for g in range(len(groups)):
-                if g * block // len(groups) == i:
-                    stage((1 - buf) * buf_bytes, g)
-            if i % step == 0:
-                # the rows of the next step's trees are pulled into the scalar cache now, so that the
-                # per-tree row loads there do not each wait for a miss. The waves of a workgroup
-                # share the cache and reach this point together, so each touches a share of the lines
-                # (a scalar load is dear here: sixteen per wave and block cost 5 % of the launch)
-                for k in range(warm_lines // warm_ways):
-                    e("  s_load_dword s3, s[30:31], 0x%x" % ((buf * block + i + step + 2) * tree_row_bytes
-                                                            + 64 * warm_ways * k))
-            if (i + 1) % step == 0 and i + 1 < block:
-                e("  s_add_u32 s14, s14, -1")
-                e("  s_cmp_eq_u32 s14, 0")
-                e("  s_cbranch_scc1 %s_done" % name)
-        # every wave is done reading this buffer and writing the other one
-        e("  s_waitcnt vmcnt(0) lgkmcnt(0)")
-        e("  s_barrier")
-        e("  s_add_u32 s14, s14, -1")
-        e("  s_cmp_eq_u32 s14, 0")
-        e("  s_cbranch_scc1 %s_done" % name)
-    e("  s_add_u32 s6, s6, %d" % (2 * block * tree_row_bytes))
-    e("  s_addc_u32 s7, s7, 0")
-    e("  s_add_u32 s30, s30, %d" % (2 * block * tree_row_bytes))
-    e("  s_addc_u32 s31, s31, 0")
-    e("  s_branch %s_loop" % name)
+                    for k in range(0, pitch, piece_dims):
+                        first = lv(j, k, mine)
+                        e("  ds_read_b%d v[%d:%d], v%d offset:%d" % (64 * piece_dims, first, first + 2 * piece_dims - 1, ga0 + j,
+                                                                    tree_offset + k * leaves * 8))
+                # copy of the next tree block into the other buffer, spread over this block's trees
+                for g in range(len(groups)):
+                    if g * block // len(groups) == i:
+                        stage((1 - buf) * buf_bytes, g)
+                if i % step == 0:
+                    # the rows of the next step's trees are pulled into the scalar cache now, so that the
+                    # per-tree row loads there do not each wait for a miss. The waves of a workgroup
+                    # share the cache and reach this point together, so each touches a share of the lines
+                    # (a scalar load is dear here: sixteen per wave and block cost 5 % of the launch)
+                    for k in range(warm_lines // warm_ways):
+                        e("  s_load_dword s3, s[30:31], 0x%x" % ((buf * block + i + step + 2) * tree_row_bytes
+                                                                + 64 * warm_ways * k))
+                if (i + 1) % step == 0 and i + 1 < block:
+                    e("  s_add_u32 s14, s14, -1")
+                    e("  s_cmp_eq_u32 s14, 0")
+                    e("  s_cbranch_scc1 %s_done" % name)
+            # every wave is done reading this buffer and writing the other one
+            e("  s_waitcnt vmcnt(0) lgkmcnt(0)")
+            e("  s_barrier")
+            e("  s_add_u32 s14, s14, -1")
+            e("  s_cmp_eq_u32 s14, 0")
+            e("  s_cbranch_scc1 %s_done" % name)
+        e("  s_add_u32 s6, s6, %d" % (2 * block * tree_row_bytes))
+        e("  s_addc_u32 s7, s7, 0")
+        e("  s_add_u32 s30, s30, %d" % (2 * block * tree_row_bytes))
+        e("  s_addc_u32 s31, s31, 0")
+        e("  s_branch %s%s" % (name, loop))
     e("%s_done:" % name)
     if step < block:
         e("  s_waitcnt vmcnt(0) lgkmcnt(0)")     # the last gathers, and the copies into the other buffer
@@ -1103,6 +1127,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         e("  s_addc_u32 s31, s31, 0")
         for r in list(range(lv0, ga0)) + (list(range(lw0, lw0 + 8)) if two_sets else []):
             e("  v_mov_b32_e32 v%d, 0" % r)
+        enter_loop()
         e("  s_branch %s_loop" % name)
         e("%s_end:" % name)
     e("  s_endpgm")

@@ -229,6 +229,7 @@ struct TEvalRegLaunchArgs {
 };
 static_assert(sizeof(TEvalRegLaunchArgs) == 96, "kernel argument block of the register-resident kernels");
 constexpr uint32_t kRegFlagMapped = 8;
+constexpr uint32_t kRegFlagPlainTable = 16;  // kernels of several dimensions and 64 leaves: the leaf table is not folded
 // what a mapped bins register holds of its bucket's bins (bits 16.. of a map entry)
 constexpr uint32_t kRegMapAsIs = 0, kRegMapLow = 1, kRegMapHigh = 2;  // bin, min(bin, 127), max(bin - 127, 0)
 
@@ -415,6 +416,11 @@ uint32_t RegSlicesPerGroup(size_t groups, uint32_t slices, size_t resident) {
         }
     }
     return best;
+}
+
+// Whether a variant's leaf tables are folded for trees of this depth: leaf l at l ^ (l >> 1) (gen_eval_reg_kernel.py: which kernels do)
+bool FoldsLeaves(const TEvalRegVariant& v, int depth) {
+    return v.Pitch > 1 && (v.Leaves == 256 || (v.Leaves == 64 && depth == 6 && v.Buckets != 192));
 }
 
 // trees per LDS buffer of a variant: a power of two, at most 16, buffer at most 32 KB
@@ -1760,6 +1766,7 @@ struct THipEvaluator::TImpl {
         uint32_t StoreDims = 1;
         uint32_t TreeBlock = 16;         // trees per LDS buffer of this kernel
         uint32_t GroupsPerCu = 1;        // workgroups that a CU holds at a time
+        uint32_t Flags = 0;              // kRegFlagPlainTable or none
         size_t TreeLeafDoubles = 0;      // doubles of a tree in Leaves
         const double* Leaves = nullptr;  // the launch's leaf table
     };
@@ -2907,16 +2914,17 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 double* table = tailTable ? tailLeaves.data() + t * rowsPerTree * tailPitch
                                           : leaves.data() + launch * m.RegLaunchLeaves + t * rowsPerTree * pitch;
                 for (size_t leaf = 0; leaf < rowsPerTree; ++leaf) {
-                    // the leaf of the model whose level bits are this table row's position bits (those behind the tree's
-                    // levels may be anything)
+                    // where the kernel looks for it (the top bit of what it folds comes inverted), and the leaf of the model whose level
+                    // bits are these (those behind the tree's levels may be anything)
+                    const size_t place = FoldsLeaves(tailTable ? *tailVariant : *variant, m.MaxDepth) ? leaf ^ (leaf >> 1) ^ (rowsPerTree >> 2) : leaf;
                     size_t modelLeaf = 0;
                     for (int d = 0; d < depth; ++d) {
                         modelLeaf |= ((leaf >> d) & 1) << levelOrder[t][d];
                     }
                     // 64 leaves: a piece per dimension; 256: pieces of two dimensions, 16 bytes per leaf
                     for (size_t k = 0; k < launchPitch && launch * pitch + k < static_cast<size_t>(m.Dim); ++k) {
-                        const size_t slot = rowsPerTree == 64 || launchPitch == 1 ? k * rowsPerTree + leaf
-                                                                                  : (k / 2) * rowsPerTree * 2 + leaf * 2 + k % 2;
+                        const size_t slot = rowsPerTree == 64 || launchPitch == 1 ? k * rowsPerTree + place
+                                                                                  : (k / 2) * rowsPerTree * 2 + place * 2 + k % 2;
                         table[slot] = values[modelLeaf * m.Dim + launch * pitch + k];
                     }
                 }
@@ -2953,6 +2961,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 l.TreeLeafDoubles = rowsPerTree * pitch;
                 l.Leaves = m.RegLeaves.Get() + launch * m.RegLaunchLeaves;
             }
+            l.Flags = FoldsLeaves(tailVariant && launch + 1 == launches ? *tailVariant : *variant, m.MaxDepth) ? 0u : kRegFlagPlainTable;
             int groupsPerCu = 0;
             HIP_CHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&groupsPerCu, l.Function, static_cast<int>(64 * l.Waves), 0));
             l.GroupsPerCu = static_cast<uint32_t>(std::max(1, groupsPerCu));
@@ -3789,12 +3798,13 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
         args.Out = results;
         args.DocCount = static_cast<uint32_t>(docCount);
         args.BlockCount = static_cast<uint32_t>((docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock);
-        args.Flags = (biased && !tail ? 1u : 0u) | (head ? 2u : 0u) | (tail ? 4u : 0u) | (m.RegMap.Get() != nullptr ? kRegFlagMapped : 0u);
+        const uint32_t flags = (biased && !tail ? 1u : 0u) | (head ? 2u : 0u) | (tail ? 4u : 0u) | (m.RegMap.Get() != nullptr ? kRegFlagMapped : 0u);
         launchArgs.RegMap = m.RegMap.Get();
         args.Scale = m.Scale;
         args.BucketCount = m.LayoutBuckets;
         args.Dim = static_cast<uint32_t>(m.Dim);
         for (const TImpl::TRegLaunch& l : m.RegLaunches) {
+            args.Flags = flags | l.Flags;
             args.TreeBlocks = (wholeEnd - wholeBegin + l.TreeBlock - 1) / l.TreeBlock;
             launchArgs.TreeBlocksPerSlice = args.TreeBlocks;
             launchArgs.SlicesPerGroup = 1;
@@ -4068,7 +4078,7 @@ void THipEvaluator::EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCou
     args.Out = partials;
     args.DocCount = static_cast<uint32_t>(docCount);
     args.BlockCount = static_cast<uint32_t>((docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock);
-    args.Flags = 4 | (m.RegMap.Get() != nullptr ? kRegFlagMapped : 0u);  // raw sums per slice
+    const uint32_t flags = 4 | (m.RegMap.Get() != nullptr ? kRegFlagMapped : 0u);  // raw sums per slice
     launchArgs.RegMap = m.RegMap.Get();
     args.Scale = m.Scale;
     args.BucketCount = m.LayoutBuckets;
@@ -4076,6 +4086,7 @@ void THipEvaluator::EvalQuantizedSlicedDevice(const uint8_t* bins, size_t docCou
     // a slice is the same number of trees in every launch
     const uint32_t sliceTrees = RegSliceTrees(m.RegTreeBlockSize);
     for (const TImpl::TRegLaunch& l : m.RegLaunches) {
+        args.Flags = flags | l.Flags;
         args.TreeBlocks = static_cast<uint32_t>((TreeCount + l.TreeBlock - 1) / l.TreeBlock);
         launchArgs.TreeBlocksPerSlice = sliceTrees / l.TreeBlock;
         args.Leaves = l.Leaves;

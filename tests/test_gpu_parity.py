@@ -880,6 +880,20 @@ def test_random_oblivious_models(seed, dim):
     _close(g.calc_hashed(floats, cats), o.calc(floats, cats, layout="split"))
 
 
+@pytest.mark.parametrize("six", ["1", "0"])
+@pytest.mark.parametrize("dim,max_depth,n_float,trees,docs", [(2, 5, 70, 20, 700), (3, 5, 100, 30, 1030), (4, 4, 150, 40, 300), (6, 5, 50, 33, 600),
+                                                              (7, 5, 30, 20, 2049), (2, 6, 190, 60, 600), (9, 1, 20, 20, 257)])
+def test_register_kernel_multi_dimensional_shallow_trees(monkeypatch, dim, max_depth, n_float, trees, docs, six):
+    """The walk of trees of five levels and less (leaf tables that are not folded), and the kernel that has no other."""
+    monkeypatch.setenv("CATBOOST_AMD_REG_SIX", six)
+    rng = np.random.default_rng(31 * dim + trees)
+    model = _float_only_model(rng, n_float, trees, max_depth, bias=list(rng.normal(size=dim)), dim=dim)
+    x = rng.normal(size=(docs, n_float)).astype(np.float32)
+    g = _gpu_model(model)
+    assert "_l64" in g.evaluator().describe_kernels(cb.LAYOUT_FLAT_ROWS, 1 << 20)["evaluate"]
+    np.testing.assert_array_equal(g.calc_flat(x), OracleModel(model).calc(x))
+
+
 def _float_only_model(rng, n_float, trees, max_depth, scale=1.0, bias=None, dim=1, max_borders=40):
     """Oblivious model over float features only (fewer than `max_borders` borders each), every feature used."""
     ffs = [mb.float_feature(i, i) for i in range(n_float)]

@@ -287,6 +287,9 @@ def _places(code, scalars, bins, bins_at, weight):
     lows = [m.group(1) for m in (re.match(r"v_bitop3_b32 v3, v(\d+),", c) for c in code) if m]
     low = int(lows[0])
     v[int(next(m for m in masks if int(m) != low))], v[low] = 0x80808080, 0xc0c0c0c0
+    for fold in (re.match(r"v_bitop3_b32 v3, v4, v(\d+), v3 bitop3:0x6a$", c) for c in code):
+        if fold:
+            v[int(fold.group(1))] = 0x7c7c7c7c if len(scalars) == 12 else 0x7f7f7f7f
     for at, c in enumerate(code):
         op, _, rest = c.partition(" ")
         args = [x.strip() for x in rest.split(",")]
@@ -364,4 +367,35 @@ def test_places_of_leaf_values(shape, six):
             for j in range(4):
                 expected[j] |= int(bins[bucket][j] >= split) << d
         got = _places(code, scalars, [sum(x << (8 * j) for j, x in enumerate(b)) for b in bins], bins_at, weight)
-        assert got == [8 * dims * x + k * leaves * 8 for x in expected for k in range(0, pitch, dims)]
+        # (several dimensions: a leaf's place is the levels' results, each but the last one compared with the next; the top one comes inverted)
+        places = [x ^ (x >> 1) ^ (leaves >> 2) if pitch > 1 else x for x in expected]
+        assert got == [8 * dims * x + k * leaves * 8 for x in places for k in range(0, pitch, dims)]
+
+
+@pytest.mark.parametrize("shape", [(104, 4, 3, 64), (56, 4, 6, 64), (192, 4, 2, 64)])
+def test_places_of_leaf_values_in_tables_that_are_not_folded(shape):
+    """The other walk of the kernels of several dimensions and 64 leaves (trees of five levels and less), and the one kernel that has no other."""
+    import random
+    gen = _generator()
+    buckets, waves, pitch, leaves = shape
+    text, _ = gen.gen_kernel(buckets, waves, pitch, leaves, False, False)
+    lines = [line.strip() for line in text.split("\n")]
+    both = any(line.endswith("_plain:") for line in lines)
+    assert both == (buckets != 192) and sum(line.endswith("_plain") for line in lines) == (3 if both else 0)  # two ways in, and its own turns
+    code = []
+    for line in lines[next(i for i, line in enumerate(lines) if line.endswith("_plain:" if both else "_loop:")) + 1:]:
+        code.append(line)
+        if sum(c.startswith("ds_read") for c in code) == 4 * pitch:
+            break
+    bins_at = int(re.search(r"v_add_u32_e64 v\d+, v(\d+), s", text).group(1))
+    rng = random.Random(3)
+    for _ in range(50):
+        bins = [[rng.randrange(129) for _ in range(4)] for _ in range(buckets)]
+        scalars, expected = {}, [0] * 4
+        for d in range(6):
+            bucket, split = rng.randrange(buckets), rng.randrange(1, 129)
+            scalars[32 + 2 * d], scalars[33 + 2 * d] = bucket, (128 - split) * 0x01010101
+            for j in range(4):
+                expected[j] |= int(bins[bucket][j] >= split) << d
+        got = _places(code, scalars, [sum(x << (8 * j) for j, x in enumerate(b)) for b in bins], bins_at, 2)
+        assert got == [8 * x + k * 512 for x in expected for k in range(pitch)]
