@@ -1214,7 +1214,7 @@ def generate():
                     parts.append(text)
                     metas.append(meta)
     for shape in gen_eval_exchange_kernel.SHAPES:
-        text, meta = gen_eval_exchange_kernel.gen_kernel(*shape)
+        text, meta = gen_eval_exchange_kernel.gen_kernel(*shape, folded=gen_eval_exchange_kernel.folds_leaves(shape[0]))
         parts.append(text)
         metas.append(meta)
     parts.append(".amdgpu_metadata")

@@ -2391,7 +2391,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             const TExchangeLeafRow& row = x.Plan.LeafRows[r];
             const bool tree = row.Tree != kExchangeNoTree;
             leafRows.push_back({r * pitch, tree ? firstLeaf[row.Tree] : 0u, row.Levels, tree ? static_cast<uint32_t>(pitch) : 0u,
-                                static_cast<uint32_t>(pitch)});
+                                static_cast<uint32_t>(pitch) | (x.MaxDepth == 8 ? dev::kLeafRowFolded : 0u)});
         }
         placeLeaves(&m.ExchangeLeaves, x.Plan.LeafRows.size() * pitch);
         m.ExchangeName = "cbamd_eval_exchange_" + shape;

@@ -3525,14 +3525,15 @@ struct TLeafRow {
     uint32_t Source;       // of the tree's first value
     uint32_t Levels;       // four bits per bit of the row's index: the bit of the tree's leaf index that it is, or kLeafRowNoLevel
     uint32_t Leaves;       // of the row that are the tree's, the others are zeros
-    uint32_t Pitch;        // leaves of the row
+    uint32_t Pitch;        // leaves of the row, with kLeafRowFolded
 };
 constexpr uint32_t kLeafRowNoLevel = 15, kLeafRowInOrder = 0x76543210u;
+constexpr uint32_t kLeafRowFolded = 0x80000000u;  // index i of the row stands at i ^ (i >> 1)
 
 __global__ __launch_bounds__(64) void PlaceLeavesKernel(const TLeafRow* __restrict__ rows, uint32_t dim, const double* __restrict__ leaves,
                                                         double* __restrict__ out) {
     const TLeafRow row = rows[blockIdx.x];
-    for (uint32_t leaf = threadIdx.x; leaf < row.Pitch; leaf += 64) {
+    for (uint32_t leaf = threadIdx.x; leaf < (row.Pitch & ~kLeafRowFolded); leaf += 64) {
         uint32_t from = 0;
 #pragma unroll
         for (uint32_t bit = 0; bit < 8; ++bit) {
@@ -3540,7 +3541,7 @@ __global__ __launch_bounds__(64) void PlaceLeavesKernel(const TLeafRow* __restri
             from |= level != kLeafRowNoLevel ? (leaf >> bit & 1) << level : 0u;
         }
         for (uint32_t k = 0; k < dim; ++k) {
-            out[row.Destination + static_cast<size_t>(leaf) * dim + k] =
+            out[row.Destination + static_cast<size_t>(row.Pitch & kLeafRowFolded ? leaf ^ (leaf >> 1) : leaf) * dim + k] =
                 leaf < row.Leaves ? leaves[row.Source + static_cast<size_t>(from) * dim + k] : 0.0;
         }
     }

@@ -707,6 +707,32 @@ def test_fused_kernel_on_rows(planner, tmp_path, case):
     np.testing.assert_array_equal(got, _expected(trees, bins)[:docs] * 0.5 + 0.25)
 
 
+@pytest.mark.parametrize("docs,six,depths", [(256, True, [8]), (255, False, [1, 5, 7, 8])])
+def test_kernel_on_folded_leaf_rows(planner, tmp_path, monkeypatch, docs, six, depths):
+    """The form that is built for depth 8: leaf l of a row stands at l ^ (l >> 1)."""
+    import functools
+
+    def bitop3(wave, args):
+        last, table = args[3].split()
+        x, y, z = wave.vector(args[1], True), wave.vector(args[2]), wave.vector(last)
+        assert table == "bitop3:0x6a"
+        wave._set(args, (x & y) ^ z)
+    monkeypatch.setattr(_Wave, "op_v_bitop3_b32", bitop3, raising=False)
+    gen = _generator()
+    assert gen.folds_leaves(8) and not gen.folds_leaves(6)
+    monkeypatch.setattr(gen, "gen_kernel", functools.partial(gen.gen_kernel, folded=True))
+    rng = np.random.default_rng(docs)
+    trees = _model(rng, 70, 600, depths, 63 if six else 127, 0.0)
+    bins = rng.integers(0, 64 if six else 128, size=(256, 600)).astype(np.uint8)
+    plan = list(_plan(planner, str(tmp_path / "model.txt"), trees, 600, 8, six))
+    place = np.arange(256) ^ (np.arange(256) >> 1)
+    folded = np.empty((plan[4].size // 256, 256))
+    folded[:, place] = plan[4].reshape(-1, 256)
+    plan[4] = folded.reshape(-1)
+    got = _run(gen, plan, bins, docs, 600, 8, six, 0.5, 0.25, rng)
+    np.testing.assert_array_equal(got, _expected(trees, bins)[:docs] * 0.5 + 0.25)
+
+
 def test_plan_refuses_more_buckets_than_registers(planner, tmp_path):
     rng = np.random.default_rng(5)
     trees = [([(b, 1, False)], rng.normal(size=2)) for b in range(1025)]
