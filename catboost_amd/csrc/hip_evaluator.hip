@@ -3,6 +3,7 @@
 #include "exchange_plan.h"
 #include "fast_exp.h"
 #include "kernels.hip.h"
+#include "ns_layout.h"
 
 #include <hip/hip_ext.h>
 
@@ -1005,14 +1006,6 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
         if (!*compactUsable) {
             continue;
         }
-        // the item that a path of `levels` decisions (the root's the highest bit) leads to, a leaf if it ends there earlier
-        const auto follow = [&](uint32_t path, int levels) {
-            size_t i = 0;
-            for (int level = levels - 1; level >= 0 && !compact.Order[i].Terminal; --level) {
-                i = compact.Children[i].first + (path >> level & 1);  // the true side always follows the false side in the order
-            }
-            return i;
-        };
         const auto splitOf = [&](size_t i) {
             const auto& rb = trees.RepackedBins[compact.Order[i].Node];
             if (rb.XorMask == 0) {
@@ -1022,55 +1015,30 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
             return ((~static_cast<uint32_t>(rb.XorMask)) & 0xffu) + (compact.Order[i].Second ? 1u : 0u);
         };
         const auto bucketOf = [&](size_t i) { return static_cast<uint32_t>(trees.RepackedBins[compact.Order[i].Node].FeatureIndex); };
+        std::vector<uint32_t> left(compact.Order.size());
+        for (size_t i = 0; i < left.size(); ++i) {
+            left[i] = compact.Order[i].Terminal ? kNsNoItem : compact.Children[i].first;  // the true side always follows the false side
+        }
+        const TNsTreeLayout layout = LayOutNsTree(left);
         // the seven nodes of the top levels; false for every bin where there is none
-        for (uint32_t n = 0; n < 8; ++n) {
-            const int level = n == 0 ? 0 : n < 3 ? 1 : 2;
-            const size_t i = follow(n + 1 - (1u << level), level);
-            const bool none = n == 7 || compact.Order[i].Terminal;
-            *compactUsable = *compactUsable && (none || splitOf(i) <= 255);
-            topNodes->push_back(none ? 0u : bucketOf(i) << 8 | (256u - splitOf(i)));
+        for (const uint32_t i : layout.TopItems) {
+            *compactUsable = *compactUsable && (i == kNsNoItem || splitOf(i) <= 255);
+            topNodes->push_back(i == kNsNoItem ? 0u : bucketOf(i) << 8 | (256u - splitOf(i)));
         }
-        // the exits, then the pairs of children below them; a pair has one place, whichever entries name it (those that a one-hot
-        // split repeats name their original's)
-        std::vector<size_t> placed;  // the item at each place
-        placed.reserve(compact.Order.size() + 8);
-        for (uint32_t exit = 0; exit < 8; ++exit) {
-            placed.push_back(follow(exit, 3));
-        }
-        std::vector<uint32_t> placeOfPair(compact.Order.size(), 0);  // by the left child's item; 0: none yet
-        for (size_t at = 0; at < placed.size(); ++at) {
-            const size_t i = placed[at];
-            if (!compact.Order[i].Terminal && placeOfPair[compact.Children[i].first] == 0) {
-                placeOfPair[compact.Children[i].first] = static_cast<uint32_t>(placed.size());
-                placed.push_back(compact.Children[i].first);
-                placed.push_back(compact.Children[i].first + 1);
-            }
-        }
-        // steps from each item to the farthest leaf
-        std::vector<uint32_t> stepsFrom(compact.Order.size(), UINT32_MAX);
-        const auto steps = [&](const auto& self, size_t i) -> uint32_t {
-            if (stepsFrom[i] == UINT32_MAX) {
-                const uint32_t left = compact.Children[i].first;
-                stepsFrom[i] = compact.Order[i].Terminal ? 0 : 1 + std::max(self(self, left), self(self, left + 1));
-            }
-            return stepsFrom[i];
-        };
-        uint32_t height = 0;
-        for (uint32_t exit = 0; exit < 8; ++exit) {
-            height = std::max(height, steps(steps, placed[exit]));
-        }
+        topNodes->push_back(0u);
+        const std::vector<uint32_t>& placed = layout.Items;
         const size_t count = (placed.size() + 7) / 8 * 8;  // (a tree's exits start at a multiple of 32 bytes)
         (*compactRows)[t * 4 + 0] = static_cast<uint32_t>(compactEntries->size());
-        (*compactRows)[t * 4 + 1] = height;
+        (*compactRows)[t * 4 + 1] = layout.Steps;
         (*compactRows)[t * 4 + 2] = static_cast<uint32_t>(count);
         *compactUsable = *compactUsable && count <= static_cast<size_t>(dev::kNsLdsEntries);
         for (uint32_t at = 0; at < count; ++at) {
+            const uint32_t next = at < placed.size() ? layout.Next[at] : at;
             if (at >= placed.size() || compact.Order[placed[at]].Terminal) {
-                compactEntries->push_back((at % 2 != 0 ? 0u : 255u) | ((at & ~1u) << 21));
+                compactEntries->push_back((next % 2 != 0 ? 0u : 255u) | ((next & ~1u) << 21));
             } else {
                 *compactUsable = *compactUsable && splitOf(placed[at]) <= 255;
-                compactEntries->push_back((splitOf(placed[at]) & 0xffu) | bucketOf(placed[at]) << 8 |
-                                          placeOfPair[compact.Children[placed[at]].first] << 21);
+                compactEntries->push_back((splitOf(placed[at]) & 0xffu) | bucketOf(placed[at]) << 8 | next << 21);
             }
             if (at < placed.size() && compact.Order[placed[at]].Terminal) {
                 const double* leaf = trees.LeafValues.data() + trees.NonSymmetricNodeIdToLeafId[compact.Order[placed[at]].Node];
