@@ -2699,6 +2699,11 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                         const uint32_t* nodes = topNodes.data() + unit.Trees[i < unit.TreeCount ? i : 0] * 8;  // (a tree too few: the first again)
                         std::transform(nodes, nodes + 8, std::back_inserter(units), withTileRow);
                     }
+                    const bool third = std::any_of(unit.Trees, unit.Trees + unit.TreeCount, [&](uint32_t t) {
+                        const uint32_t* nodes = topNodes.data() + t * 8;
+                        return std::any_of(nodes + 3, nodes + 7, [](uint32_t node) { return (node & 0xffu) != 0; });
+                    });
+                    units[units.size() - dev::kNsUnitDwords + 15] = third ? 0u : 1u;
                 }
                 // the first entry of the unit that a unit's wave takes next
                 for (size_t u = 0; u + m.NsLdsShape.Waves < bestUnits.size(); ++u) {

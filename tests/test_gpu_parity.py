@@ -178,6 +178,31 @@ def test_non_symmetric_trees_that_end_in_their_top_levels(border_of, dim):
         _close(g.calc_flat(x, tree_start=begin, tree_end=end), o.calc(x, tree_start=begin, tree_end=end))
 
 
+@pytest.mark.parametrize("dim", [1, 2, 3, 5])
+@pytest.mark.parametrize("trees", [1, 3, 4, 48, 49, 151])
+def test_non_symmetric_trees_of_two_levels_and_less(trees, dim):
+    """Units of the LDS walk without a node on the third level, beside a few that have one; waves with no unit, one, several; ranges."""
+    rng = np.random.default_rng(trees * 10 + dim)
+    ffs = [mb.float_feature(i) for i in range(5)]
+    leaf = lambda: mb.leaf_node([float(v) for v in rng.normal(size=dim)] if dim > 1 else float(rng.normal()))  # noqa: E731
+
+    def grown(depth):
+        if depth == 0 or rng.random() < 0.15:
+            return leaf()
+        return mb.split_node(("float", int(rng.integers(5)), float(rng.integers(20))), grown(depth - 1), grown(depth - 1))
+
+    heads = [grown(3 if t % 50 == 49 else int(rng.integers(1, 3))) for t in range(trees)]
+    heads[0] = mb.split_node(("float", 0, 4.0), mb.split_node(("float", 1, 7.0), leaf(), leaf()), mb.split_node(("float", 2, 9.0), leaf(), leaf()))
+    model = mb.build_non_symmetric(ffs, [], dim, heads, scale=1.5, bias=list(rng.normal(size=dim)))
+    x = (rng.integers(-1, 21, size=(1025, 5)) + rng.choice([0.0, 0.5], size=(1025, 5))).astype(np.float32)
+    o = OracleModel(model)
+    g = _gpu_model(model)
+    assert "EvalNonSymmetricLdsKernel" in g.evaluator().describe_kernels(cb.LAYOUT_FLAT_ROWS, 1025)["evaluate"]
+    _close(g.calc_flat(x), o.calc(x))
+    for begin, end in ((0, (trees + 1) // 2), (trees // 3, trees)):
+        _close(g.calc_flat(x, tree_start=begin, tree_end=end), o.calc(x, tree_start=begin, tree_end=end))
+
+
 @pytest.mark.parametrize("seed,dim,n_float,n_cat,trees,max_depth,docs", [
     (1, 2, 30, 0, 120, 8, 3000), (2, 3, 150, 3, 60, 9, 1000), (3, 4, 8, 4, 25, 6, 257), (4, 5, 40, 0, 200, 5, 5000),
     (5, 10, 60, 2, 90, 7, 2049), (6, 13, 12, 0, 33, 10, 64),
