@@ -54,7 +54,8 @@ Kernel arguments (80 bytes):
   16 leaves      const double*   [(treeBlocks + 2) * TREE_BLOCK][LEAVES][PITCH] (fused kernels of six levels: [whole buffers of 64 trees, and two][64])
   24 out         double*         [docCount][dim]
   32 docCount    uint32          36 blockCount uint32 (ceil(docCount / 256), >= 1)
-  40 treeBlocks  uint32 (>= 1)   44 flags uint32 (bit 0: add the bias, bit 4: 64 leaves, several dimensions, the table is not folded)
+  40 treeBlocks  uint32 (>= 1)   44 flags uint32 (bit 0: add the bias, bit 4: 64 leaves, several dimensions, the table is not folded,
+                                 bit 5: nor that, but in pieces of two dimensions)
   48 scale       double          56 bias const double* (first dimension of this launch)
   64 bucketCount uint32 (1 .. BUCKETS)                68 dim uint32
   72 first dimension of this launch uint32            76 dimensions to store uint32 (1 .. PITCH)
@@ -256,6 +257,11 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     # vector issue is as busy, loses 4 % by it.
     folded = pitch > 1 and not (leaves == 64 and buckets == 192)
     both_tables = folded and leaves == 64
+    # Four and six dimensions, trees of four levels and less: pieces of two dimensions as with 256 leaves, and no fold (flags bit 5). Their
+    # 16 leaves of 16 bytes fill two rows of the banks, and one read does what two of 8 bytes do. 600 001 documents, 400 trees of depth
+    # 4 over 100 features, pieces of one dimension and of two: four dimensions 217 and 191 us a call, six 273 and 260, ten 420 and 391 (of
+    # depth 5, 300 trees, 300 001 documents, pieces of one are the faster: four 101 and 106, six 123 and 139; three dimensions at any depth).
+    pair_tables = both_tables and pitch >= 4 and pitch % 2 == 0
     if not fused:
         vgprs += 2 if deep else 4 if folded else 3
     two_sets = pitch == 1 and block % 2 == 0 and (fused or (vgprs + 8 <= 256 and waves_per_simd(vgprs + 8) == waves_per_simd(vgprs)))
@@ -943,7 +949,12 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         # row i of a product's left operand is lane i's of the four, byte k of it stands for byte k of the index
         e("  v_and_b32_e32 v5, 3, v0")
         e("  v_lshlrev_b32_e32 v5, 3, v5")
-        e("  v_lshlrev_b32_e64 v%d, v5, %d" % (unpack, unpack_scale))
+        if pair_tables:
+            e("  s_bitcmp1_b32 s15, 5")
+            e("  s_cselect_b32 s24, %d, %d" % (2 * unpack_scale, unpack_scale))
+            e("  v_lshlrev_b32_e64 v%d, v5, s24" % unpack)
+        else:
+            e("  v_lshlrev_b32_e64 v%d, v5, %d" % (unpack, unpack_scale))
     # a launch that continues the sums of earlier trees takes them from `out`
     e("  s_bitcmp1_b32 s15, 1")
     e("  s_cbranch_scc0 %s_fresh" % name)
@@ -983,9 +994,17 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         if both_tables:
             e("  s_bitcmp1_b32 s15, 4")
             e("  s_cbranch_scc1 %s_plain" % name)
+        if pair_tables:
+            e("  s_bitcmp1_b32 s15, 5")
+            e("  s_cbranch_scc1 %s_pairs" % name)
 
     enter_loop()
-    for fold_here, loop in ((folded, "_loop"), (False, "_plain"))[:2 if both_tables else 1]:
+    walks = [(folded, piece_dims, "_loop")]
+    if both_tables:
+        walks.append((False, piece_dims, "_plain"))
+    if pair_tables:
+        walks.append((False, 2, "_pairs"))
+    for fold_here, walk_dims, loop in walks:
         e("%s%s:" % (name, loop))
         for buf in range(2):
             for i in range(block):
@@ -1005,7 +1024,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                     levels_high(rows)
                 tree_offset = buf * buf_bytes + i * tree_bytes
                 if not deep:
-                    tree_offset += unpack_scale * 128
+                    tree_offset += unpack_scale * walk_dims // piece_dims * 128
 
                 # The previous tree's leaf values have arrived (its levels and addresses were issued in between), and so has
                 # the next tree's row. With two sets of leaf values the trees of a block alternate between them (a block has
@@ -1041,9 +1060,9 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                     add_leaf_values(two_sets and not mine)
                     load_rows(rows, buf * block + i + 2)
                 for j in range(4):
-                    for k in range(0, pitch, piece_dims):
+                    for k in range(0, pitch, walk_dims):
                         first = lv(j, k, mine)
-                        e("  ds_read_b%d v[%d:%d], v%d offset:%d" % (64 * piece_dims, first, first + 2 * piece_dims - 1, ga0 + j,
+                        e("  ds_read_b%d v[%d:%d], v%d offset:%d" % (64 * walk_dims, first, first + 2 * walk_dims - 1, ga0 + j,
                                                                     tree_offset + k * leaves * 8))
                 # copy of the next tree block into the other buffer, spread over this block's trees
                 for g in range(len(groups)):

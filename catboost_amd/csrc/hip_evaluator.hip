@@ -231,6 +231,7 @@ struct TEvalRegLaunchArgs {
 static_assert(sizeof(TEvalRegLaunchArgs) == 96, "kernel argument block of the register-resident kernels");
 constexpr uint32_t kRegFlagMapped = 8;
 constexpr uint32_t kRegFlagPlainTable = 16;  // kernels of several dimensions and 64 leaves: the leaf table is not folded
+constexpr uint32_t kRegFlagPairTable = 32;   // kernels of four and six dimensions and 64 leaves: nor that, but in pieces of two dimensions
 // what a mapped bins register holds of its bucket's bins (bits 16.. of a map entry)
 constexpr uint32_t kRegMapAsIs = 0, kRegMapLow = 1, kRegMapHigh = 2;  // bin, min(bin, 127), max(bin - 127, 0)
 
@@ -422,6 +423,11 @@ uint32_t RegSlicesPerGroup(size_t groups, uint32_t slices, size_t resident) {
 // Whether a variant's leaf tables are folded for trees of this depth: leaf l at l ^ (l >> 1) (gen_eval_reg_kernel.py: which kernels do)
 bool FoldsLeaves(const TEvalRegVariant& v, int depth) {
     return v.Pitch > 1 && (v.Leaves == 256 || (v.Leaves == 64 && depth == 6 && v.Buckets != 192));
+}
+
+// ... or, of 64 leaves, hold pieces of two dimensions, 16 bytes per leaf (those of 256 leaves always do)
+bool PairsDimensions(const TEvalRegVariant& v, int depth) {
+    return v.Pitch > 1 && (v.Leaves == 256 || (v.Leaves == 64 && depth <= 4 && v.Pitch >= 4));
 }
 
 // trees per LDS buffer of a variant: a power of two, at most 16, buffer at most 32 KB
@@ -2886,18 +2892,19 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 const size_t launchPitch = tailTable ? tailPitch : pitch;
                 double* table = tailTable ? tailLeaves.data() + t * rowsPerTree * tailPitch
                                           : leaves.data() + launch * m.RegLaunchLeaves + t * rowsPerTree * pitch;
+                const TEvalRegVariant& kernel = tailTable ? *tailVariant : *variant;
+                const bool folds = FoldsLeaves(kernel, m.MaxDepth), pairs = PairsDimensions(kernel, m.MaxDepth);
                 for (size_t leaf = 0; leaf < rowsPerTree; ++leaf) {
                     // where the kernel looks for it (the top bit of what it folds comes inverted), and the leaf of the model whose level
                     // bits are these (those behind the tree's levels may be anything)
-                    const size_t place = FoldsLeaves(tailTable ? *tailVariant : *variant, m.MaxDepth) ? leaf ^ (leaf >> 1) ^ (rowsPerTree >> 2) : leaf;
+                    const size_t place = folds ? leaf ^ (leaf >> 1) ^ (rowsPerTree >> 2) : leaf;
                     size_t modelLeaf = 0;
                     for (int d = 0; d < depth; ++d) {
                         modelLeaf |= ((leaf >> d) & 1) << levelOrder[t][d];
                     }
-                    // 64 leaves: a piece per dimension; 256: pieces of two dimensions, 16 bytes per leaf
+                    // pieces of two dimensions, 16 bytes per leaf, or one per dimension
                     for (size_t k = 0; k < launchPitch && launch * pitch + k < static_cast<size_t>(m.Dim); ++k) {
-                        const size_t slot = rowsPerTree == 64 || launchPitch == 1 ? k * rowsPerTree + place
-                                                                                  : (k / 2) * rowsPerTree * 2 + place * 2 + k % 2;
+                        const size_t slot = pairs ? (k / 2) * rowsPerTree * 2 + place * 2 + k % 2 : k * rowsPerTree + place;
                         table[slot] = values[modelLeaf * m.Dim + launch * pitch + k];
                     }
                 }
@@ -2934,7 +2941,8 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 l.TreeLeafDoubles = rowsPerTree * pitch;
                 l.Leaves = m.RegLeaves.Get() + launch * m.RegLaunchLeaves;
             }
-            l.Flags = FoldsLeaves(tailVariant && launch + 1 == launches ? *tailVariant : *variant, m.MaxDepth) ? 0u : kRegFlagPlainTable;
+            const TEvalRegVariant& kernel = tailVariant && launch + 1 == launches ? *tailVariant : *variant;
+            l.Flags = FoldsLeaves(kernel, m.MaxDepth) ? 0u : PairsDimensions(kernel, m.MaxDepth) ? kRegFlagPairTable : kRegFlagPlainTable;
             int groupsPerCu = 0;
             HIP_CHECK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&groupsPerCu, l.Function, static_cast<int>(64 * l.Waves), 0));
             l.GroupsPerCu = static_cast<uint32_t>(std::max(1, groupsPerCu));

@@ -919,6 +919,27 @@ def test_register_kernel_multi_dimensional_shallow_trees(monkeypatch, dim, max_d
     np.testing.assert_array_equal(g.calc_flat(x), OracleModel(model).calc(x))
 
 
+@pytest.mark.parametrize("six", ["1", "0"])
+@pytest.mark.parametrize("max_depth", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("dim,n_float,n_cat", [(4, 20, 0), (5, 100, 0), (6, 30, 3), (8, 150, 0), (10, 40, 5), (11, 120, 0)])
+def test_register_kernel_tables_of_shallow_trees(monkeypatch, dim, n_float, n_cat, max_depth, six):
+    """Four levels and less: kernels of four and six dimensions read pieces of two dimensions, those of two and three a piece per dimension, as all of
+    them do at five levels; one-hot levels; one pass, slices of the trees, and ranges."""
+    monkeypatch.setenv("CATBOOST_AMD_REG_SIX", six)
+    rng = np.random.default_rng(dim * 100 + max_depth)
+    model, cat_values = _random_oblivious(rng, n_float=n_float, n_cat=n_cat, trees=70, max_depth=max_depth, dim=dim, scale=0.5, bias=rng.normal(size=dim))
+    x = _random_flat_data(rng, model, cat_values, 9001)
+    o = OracleModel(model)
+    expected = o.calc(x)
+    g = _gpu_model(model)
+    assert "_l64" in g.evaluator().describe_kernels(cb.LAYOUT_FLAT_ROWS, 1 << 20)["evaluate"]
+    _close(g.calc_flat(x), expected)
+    g.set_small_batch_slicing(False)
+    np.testing.assert_array_equal(g.calc_flat(x), expected)
+    np.testing.assert_array_equal(g.calc_flat(x[:1001], tree_start=0, tree_end=64), o.calc(x[:1001], tree_start=0, tree_end=64))
+    _close(g.calc_flat(x[:700], tree_start=5, tree_end=60), o.calc(x[:700], tree_start=5, tree_end=60))
+
+
 def _float_only_model(rng, n_float, trees, max_depth, scale=1.0, bias=None, dim=1, max_borders=40):
     """Oblivious model over float features only (fewer than `max_borders` borders each), every feature used."""
     ffs = [mb.float_feature(i, i) for i in range(n_float)]

@@ -399,3 +399,39 @@ def test_places_of_leaf_values_in_tables_that_are_not_folded(shape):
                 expected[j] |= int(bins[bucket][j] >= split) << d
         got = _places(code, scalars, [sum(x << (8 * j) for j, x in enumerate(b)) for b in bins], bins_at, 2)
         assert got == [8 * x + k * 512 for x in expected for k in range(pitch)]
+
+
+@pytest.mark.parametrize("shape", [(160, 4, 4, 64), (56, 4, 6, 64), (128, 4, 6, 64)])
+@pytest.mark.parametrize("six", [False, True])
+def test_places_of_leaf_values_in_pieces_of_two_dimensions(shape, six):
+    """The third walk of the kernels of four and six dimensions and 64 leaves (trees of four levels and less): 16 bytes per leaf, not folded;
+    the product's weight and the way in follow the same flag. Kernels of two and three dimensions have none."""
+    import random
+    gen = _generator()
+    buckets, waves, pitch, leaves = shape
+    text, _ = gen.gen_kernel(buckets, waves, pitch, leaves, False, six)
+    assert all("_pairs" not in gen.gen_kernel(b, 4, p, n, False, six)[0] for b, p, n in ((104, 3, 64), (80, 2, 64), (192, 2, 64), (160, 4, 256)))
+    lines = [line.strip() for line in text.split("\n")]
+    assert sum(line.endswith("_pairs") for line in lines) == 3  # two ways in, and its own turns
+    assert all(lines[i - 1] == "s_bitcmp1_b32 s15, 5" for i, line in enumerate(lines) if re.match(r"s_cbranch_scc1 .*_pairs$", line))
+    at = lines.index("s_cselect_b32 s24, 4, 2")
+    assert lines[at - 1] == "s_bitcmp1_b32 s15, 5" and re.match(r"v_lshlrev_b32_e64 v\d+, v5, s24$", lines[at + 1])
+    code = []
+    for line in lines[next(i for i, line in enumerate(lines) if line.endswith("_pairs:")) + 1:]:
+        code.append(line)
+        if sum(c.startswith("ds_read") for c in code) == 2 * pitch:
+            break
+    assert all(c.startswith("ds_read_b128") for c in code if c.startswith("ds_read"))
+    bins_at = int(re.search(r"v_add_u32_e64 v\d+, v(\d+), s", text).group(1))
+    top = 64 if six else 128
+    rng = random.Random(5)
+    for _ in range(50):
+        bins = [[rng.randrange(top + 1) for _ in range(4)] for _ in range(buckets)]
+        scalars, expected = {}, [0] * 4
+        for d in range(6):
+            bucket, split = rng.randrange(buckets), rng.randrange(1, top + 1)
+            scalars[32 + 2 * d], scalars[33 + 2 * d] = bucket, ((64 if six and d % 2 == 0 else 128) - split) * 0x01010101
+            for j in range(4):
+                expected[j] |= int(bins[bucket][j] >= split) << d
+        got = _places(code, scalars, [sum(x << (8 * j) for j, x in enumerate(b)) for b in bins], bins_at, 4)
+        assert got == [16 * x + k * 512 for x in expected for k in range(0, pitch, 2)]
