@@ -4096,17 +4096,16 @@ bool THipEvaluator::TakesSmallBatchKernel(size_t docCount, size_t treeStart, siz
 }
 
 // ... of calls whose features are on the device. Its time grows with the levels that a document walks, and by a step for every 4096
-// documents (a workgroup of sixteen more on every CU), the one of binarize and evaluate launches hardly with either, but with the columns
-// to binarize. Models of many levels take those earlier, later the more columns there are. Whole call, SmallBatchKernel and the
-// launches: 12 289 documents, 501 trees of depth 8, 20 columns 28.6 and 30.3 us, 200 28.6 and 33.1, 563 trees, 60 columns 31.7 and 28.3, 140 32.0
-// and 31.8, 222 32.2 and 33.4, 833 of depth 6, 60 columns 29.8 and 27.9, 222 31.2 and 35.5; 10 241 documents, 875 of depth 8, 60 columns
-// 32.0 and 28.3, 180 32.7 and 33.9, 1250 of depth 8, 222 columns 41.7 and 35.8. Of 696 such batches (4000 to 16 000 levels, 20 to 222 columns) these
-// lines give the launches 462, none of which they take longer for. (One dimension on the register kernels;
-// both add the same slices. Other models keep the one limit.)
+// documents (a workgroup of sixteen more on every CU), the one of binarize and evaluate launches hardly, so models of many levels
+// take those earlier. Whole call, SmallBatchKernel and the launches: 1000 trees of depth 8 over 200 features, 8192 documents 29.5
+// and 32.4 us, 10 240 36.2 and 35.4, 12 400 43.2 and 36.9, 16 384 46.3 and 37.5 (columns of 50 features, 8300 documents 34.2 and 35.6, 16 384
+// 44.4 and 36.8); 1000 of depth 6 over 100, 12 288 30.1 and 31.5, 12 400 33.5 and 32.7, 16 384 35.3 and 32.8; 500 of depth 6
+// over 150, 16 384 28.1 and 30.7, 300 of depth 8 over 60 28.7 and 30.2. (One dimension on the register kernels; both add the same
+// slices. Other models keep the one limit.)
 bool THipEvaluator::TakesSmallBatchOnDevice(size_t docCount, size_t treeStart, size_t treeEnd) const {
     const TImpl& m = *Impl;
-    const size_t levels = TreeCount * static_cast<size_t>(m.MaxDepth), columns = BucketCount > 100 ? BucketCount - 100 : 0;
-    const size_t limit = 2 * levels <= 10000 + 25 * columns ? kSmallBatchDocs : levels <= 6500 + 20 * columns ? 12288 : 10240;
+    const size_t levels = TreeCount * static_cast<size_t>(m.MaxDepth);
+    const size_t limit = levels <= 4000 ? kSmallBatchDocs : levels <= 6500 ? 12288 : 10240;
     return TakesSmallBatchKernel(docCount, treeStart, treeEnd) && (m.Dim > 1 || TreeSlicesFor(docCount) <= 1 || docCount <= limit);
 }
 

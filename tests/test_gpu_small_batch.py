@@ -558,16 +558,12 @@ def test_few_slices_are_added_in_order(trees, dim):
     test_slices_are_added_in_order(trees, dim)
 
 
-@pytest.mark.parametrize("name,trees,limit", [("C2N", 501, 16384), ("C2N", 625, 16384), ("C2N", 626, 12288), ("C2N", 812, 12288),
-                                              ("C2N", 813, 10240), ("C2", 501, 16384), ("C2", 781, 16384), ("C2", 782, 12288),
-                                              ("C2", 1062, 12288), ("C2", 1063, 10240)])
-def test_small_batches_of_models_with_many_levels(name, trees, limit):
-    """Models of more levels leave the small-batch kernel for the binarize and register kernels earlier, those of 200 columns (C2) later
-    than those of 90 (C2N), as the launches take longer for them; both add the same slices."""
+@pytest.mark.parametrize("trees,limit", [(500, 16384), (501, 12288), (812, 12288), (813, 10240)])
+def test_small_batches_of_models_with_many_levels(trees, limit):
+    """Models of more levels leave the small-batch kernel for the binarize and register kernels earlier; both add the same slices."""
     import torch
 
-    model, info = syn.build_model(name, trees=trees)
-    assert model.bucket_count == {"C2N": 90, "C2": 200}[name]
+    model, info = syn.build_model("C2", trees=trees)
     model.enable_gpu_evaluation(0)
     ev = model.evaluator()
     x = syn.device_features(info, limit + 1)
