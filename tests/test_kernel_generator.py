@@ -435,3 +435,152 @@ def test_places_of_leaf_values_in_pieces_of_two_dimensions(shape, six):
                 expected[j] |= int(bins[bucket][j] >= split) << d
         got = _places(code, scalars, [sum(x << (8 * j) for j, x in enumerate(b)) for b in bins], bins_at, 4)
         assert got == [16 * x + k * 512 for x in expected for k in range(0, pitch, 2)]
+
+
+def _follow(lines, start, scalars, v, bins_at, weight):
+    """As _places, for the trees that branch or have more than eight levels: follows a lane from line `start` on, branches taken as the
+    scalars say, up to the next tree's first instruction behind the gathers, and gives the LDS offsets that they name. `v`: the vector
+    registers' dwords. In index mode src0 may be a vector register in nothing but a level's read of its bucket."""
+    labels = {line[:-1]: i for i, line in enumerate(lines) if line.endswith(":")}
+    index, scc, step, product_step, gathers = None, 0, 0, None, []
+    written = {}
+    at = start
+
+    def value(operand):
+        if operand.startswith("v"):
+            return v[int(operand[1:])]
+        return scalars[int(operand[1:])] if operand.startswith("s") else int(operand, 0)
+
+    while True:
+        line = lines[at]
+        at += 1
+        if line.endswith(":"):
+            continue
+        op, _, rest = line.partition(" ")
+        args = [x.strip() for x in rest.split(",")]
+        if gathers and not op.startswith("ds_read"):
+            return gathers
+        step += 1
+        if op.startswith("s_set_gpr_idx_o") or op == "s_set_gpr_idx_idx":
+            index = None if op.endswith("off") else scalars[int(args[0][1:])] & 255
+        elif op == "s_bitcmp1_b32":
+            scc = scalars[int(args[0][1:])] >> int(args[1]) & 1
+        elif op in ("s_branch", "s_cbranch_scc1"):
+            at = labels[args[0]] if op == "s_branch" or scc else at
+        elif op.startswith("v_mfma"):
+            assert step - written[3] > 2 and index is None
+            first = int(re.match(r"v\[(\d+):", args[0]).group(1))
+            for j in range(4):
+                v[first + j] = weight * _signed(v[3] >> (8 * j) & 255)
+            product_step = step
+        elif op == "v_mul_u32_u24_sdwa":
+            word = int(args[2].split()[-1][-1])
+            v[int(args[0][1:])] = scalars[int(args[1][1:])] * (v[int(args[2].split()[0][1:])] >> (16 * word) & 0xffff)
+        elif op.startswith("ds_read"):
+            assert product_step is None or step - product_step > 5
+            found = re.match(r"ds_read_b(64|128) v\[\d+:\d+\], v(\d+) offset:(\d+)$", line)
+            gathers.append(v[int(found.group(2))] + int(found.group(3)))
+        elif op in ("s_waitcnt", "s_nop", "v_add_f64", "s_load_dwordx16"):
+            continue
+        else:
+            last, _, table = args[-1].partition(" ")
+            sources = args[1:-1] + [last]
+            if index is not None and sources[0].startswith("v"):
+                assert op in ("v_add_u32_e64", "v_lerp_u8", "v_xor_b32_e64") and sources[0] == "v%d" % bins_at
+                sources[0] = "v%d" % (bins_at + index)
+            x = [value(s) for s in sources]
+            if op in ("v_add_u32_e64", "v_lerp_u8"):
+                sums = [(x[0] >> (8 * j) & 255) + (x[1] >> (8 * j) & 255) for j in range(4)]
+                out = sum((s >> 1 if op == "v_lerp_u8" else s) << (8 * j) for j, s in enumerate(sums))
+                assert op == "v_lerp_u8" or max(sums) < 256
+            elif op == "v_subrev_u32_e32":
+                out = (x[1] - x[0]) & 0xffffffff
+            elif op == "v_bitop3_b32":
+                truth = int(table.split(":")[1], 16)
+                out = sum((truth >> ((x[0] >> b & 1) << 2 | (x[1] >> b & 1) << 1 | x[2] >> b & 1) & 1) << b for b in range(32))
+            elif op == "v_bfi_b32":
+                out = (x[0] & x[1]) | (~x[0] & x[2] & 0xffffffff)
+            elif op == "v_perm_b32":
+                both = x[1] | x[0] << 32  # selectors 0 to 3: bytes of the second operand, 4 to 7: of the first
+                out = sum((both >> (8 * (x[2] >> (8 * j) & 7)) & 255) << (8 * j) for j in range(4))
+            else:
+                out = {"v_xor_b32_e64": lambda: x[0] ^ x[1], "v_or_b32_e32": lambda: x[0] | x[1], "v_and_b32_e32": lambda: x[0] & x[1],
+                       "v_lshrrev_b32_e32": lambda: x[1] >> x[0]}[op]()
+            v[int(args[0][1:])] = out
+            written[int(args[0][1:])] = step
+
+
+def _constants(lines, end):
+    """Scalar and vector registers that hold a constant where the walk starts (the last move to each)."""
+    scalars, v = {}, {}
+    for line in lines[:end]:
+        found = re.match(r"(s_mov_b32 s|v_mov_b32_e32 v)(\d+), (0x[0-9a-f]+|\d+)$", line)
+        if found:
+            (scalars if found.group(1)[0] == "s" else v)[int(found.group(2))] = int(found.group(3), 0)
+    return scalars, v
+
+
+@pytest.mark.parametrize("shape", [(96, 8, 1, 64), (208, 4, 1, 256), (56, 4, 6, 64), (104, 4, 3, 64), (192, 4, 2, 64), (160, 4, 4, 256)])
+def test_places_of_leaf_values_of_mixed_trees(shape):
+    """Both forms of a mixed kernel's tree: bit 31 of its first dword clear (pairs of levels) and set (eight bits a level, with and without a
+    xor mask, splits on both sides of 128, and levels that stand for none: splitIdx 255), in every walk that the kernel has."""
+    import random
+    gen = _generator()
+    buckets, waves, pitch, leaves = shape
+    lines = [line.strip() for line in gen.gen_kernel(buckets, waves, pitch, leaves, True)[0].split("\n")]
+    depth = 6 if leaves == 64 else 8
+    rng = random.Random(11)
+    walks = [i for i, line in enumerate(lines) if re.search(r"_(loop|plain|pairs):$", line)]
+    assert len(walks) == (3 if leaves == 64 and pitch in (4, 6) else 2 if leaves == 64 and pitch == 3 else 1)
+    for start in walks:
+        folded = lines[start].endswith("_loop:") and pitch > 1 and buckets != 192
+        dims = 2 if pitch > 1 and (leaves == 256 or lines[start].endswith("_pairs:")) else 1
+        constants, vectors = _constants(lines, start)
+        bins_at = next(int(m.group(1)) for m in (re.match(r"v_xor_b32_e64 v4, v(\d+), s", line) for line in lines) if m)
+        for turn in range(120):
+            wide = turn % 2 == 1
+            top = 255 if wide else 128
+            bins = [[rng.choice([0, 1, 127, 128, top, rng.randrange(top + 1)]) % (top + 1) for _ in range(4)] for _ in range(buckets)]
+            scalars, expected = dict(constants), [0] * 4
+            for d in range(depth):
+                bucket = rng.randrange(buckets)
+                split = rng.choice([1, 2, 127, 128, 129, 254, 255, rng.randrange(1, 256)]) if wide else rng.choice([1, 127, 128, rng.randrange(1, 129)])
+                mask = rng.choice([0, 0, rng.randrange(256)]) if wide else 0
+                if wide:
+                    scalars.update({32 + 4 * d: bucket | (0x80000000 if d == 0 else 0), 33 + 4 * d: mask * 0x01010101,
+                                    34 + 4 * d: (split & 0x7f) * 0x01010101, 35 + 4 * d: 0x80808080 if split < 128 else 0})
+                else:
+                    scalars.update({32 + 2 * d: bucket, 33 + 2 * d: (128 - split) * 0x01010101})
+                for j in range(4):
+                    expected[j] |= int(bins[bucket][j] ^ mask >= split) << d
+            v = dict(vectors)
+            v.update({bins_at + i: sum(x << (8 * j) for j, x in enumerate(b)) for i, b in enumerate(bins)})
+            got = _follow(lines, start, scalars, v, bins_at, 8 * dims >> (8 - depth))
+            places = [x ^ (x >> 1) ^ (leaves >> 2) if folded else x for x in expected]
+            assert got == [8 * dims * x + k * leaves * 8 for x in places for k in range(0, pitch, dims)]
+
+
+@pytest.mark.parametrize("shape", [(96, 8, 1, 1024), (208, 4, 1, 1024)])
+@pytest.mark.parametrize("six", [False, True])
+def test_places_of_leaf_values_of_ten_levels(shape, six):
+    """Trees of depth 9 and 10: the ninth and tenth level join the eight merged in pairs, whose top bit is not inverted there."""
+    import random
+    gen = _generator()
+    buckets, waves, pitch, leaves = shape
+    lines = [line.strip() for line in gen.gen_kernel(buckets, waves, pitch, leaves, False, six)[0].split("\n")]
+    start = next(i for i, line in enumerate(lines) if line.endswith("_loop:"))
+    bins_at = next(int(m.group(1)) for m in (re.match(r"v_add_u32_e64 v\d+, v(\d+), s", line) for line in lines[start:]) if m)
+    constants, vectors = _constants(lines, start)
+    top = 64 if six else 128
+    rng = random.Random(13)
+    for _ in range(120):
+        bins = [[rng.choice([0, 1, top - 1, top, rng.randrange(top + 1)]) for _ in range(4)] for _ in range(buckets)]
+        scalars, expected = dict(constants), [0] * 4
+        for d in range(10):
+            bucket, split = rng.randrange(buckets), rng.choice([1, 2, top - 1, top, rng.randrange(1, top + 1)])
+            scalars.update({32 + 2 * d: bucket, 33 + 2 * d: ((64 if six and d % 2 == 0 and d < 8 else 128) - split) * 0x01010101})
+            for j in range(4):
+                expected[j] |= int(bins[bucket][j] >= split) << d
+        v = dict(vectors)
+        v.update({bins_at + i: sum(x << (8 * j) for j, x in enumerate(b)) for i, b in enumerate(bins)})
+        assert _follow(lines, start, scalars, v, bins_at, 8) == [8 * x for x in expected]
