@@ -40,14 +40,14 @@ def _run(cmd):
 
 
 def _build_eval_reg_code_object():
-    """gen_eval_reg_kernel.py -> assembly -> gfx950 code object -> byte list included by hip_evaluator.hip"""
+    """gen_eval_reg_kernel.py -> assembly -> gfx950 code object -> byte list included by hip_evaluator.hip, and the kernels' table"""
     llvm = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(_hipcc()))), "llvm", "bin")
     if not os.path.isdir(llvm):
         llvm = "/opt/rocm/llvm/bin"
     asm = os.path.join(OBJ_DIR, "eval_reg_kernel.s")
     obj = os.path.join(OBJ_DIR, "eval_reg_kernel.o")
     co = os.path.join(OBJ_DIR, "eval_reg_kernel.co")
-    _run([sys.executable, os.path.join(CSRC, "gen_eval_reg_kernel.py"), asm])
+    _run([sys.executable, os.path.join(CSRC, "gen_eval_reg_kernel.py"), asm, os.path.join(OBJ_DIR, "eval_reg_tables.inc")])
     _run([os.path.join(llvm, "clang"), "-x", "assembler", "-target", "amdgcn-amd-amdhsa", "-mcpu=gfx950", "-c", asm,
           "-o", obj])
     _run([os.path.join(llvm, "ld.lld"), "-shared", "-o", co, obj])

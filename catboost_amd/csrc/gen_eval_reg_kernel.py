@@ -98,7 +98,7 @@ Additional kernel arguments (104 bytes in all):
  100 unitCount uint32 (1 .. BUCKETS / 16)
 and argument 0 is the delay of workgroups 256 .. 511 in turns of 4096 cycles (rows; unused for columns), argument 16 points at the border table images.
 
-Usage: gen_eval_reg_kernel.py OUT.s
+Usage: gen_eval_reg_kernel.py OUT.s TABLES.inc
 """
 import os
 import sys
@@ -178,6 +178,21 @@ def tree_block(pitch, leaves):
     return block
 
 
+def folds_leaves(buckets, pitch, leaves):
+    """Several dimensions: a kernel's leaf tables are folded (see the walk). Trees of five levels or less have no two rows to a bank, so the
+    kernels of 64 leaves walk either kind of table (flags bit 4: as it is); the one of two dimensions and many buckets, whose
+    vector issue is as busy, loses 4 % by it."""
+    return pitch > 1 and not (leaves == 64 and buckets == 192)
+
+
+def has_pair_walk(buckets, pitch, leaves):
+    """Four and six dimensions, trees of four levels and less: pieces of two dimensions as with 256 leaves, and no fold (flags bit 5). Their
+    16 leaves of 16 bytes fill two rows of the banks, and one read does what two of 8 bytes do. 600 001 documents, 400 trees of depth
+    4 over 100 features, pieces of one dimension and of two: four dimensions 217 and 191 us a call, six 273 and 260, ten 420 and 391 (of
+    depth 5, 300 trees, 300 001 documents, pieces of one are the faster: four 101 and 106, six 123 and 139; three dimensions at any depth)."""
+    return folds_leaves(buckets, pitch, leaves) and leaves == 64 and pitch >= 4 and pitch % 2 == 0
+
+
 def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, levels=None, columns=False):
     assert not (mixed and six)
     assert fused or not columns
@@ -252,16 +267,8 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     # (fused: registers that only the binarize phase uses)
     mask80 = high if fused else vgprs
     mask_c0, unpack, fold = mask80 + 1, mask80 + 2, mask80 + 3
-    # Several dimensions: the leaf tables are folded (see the walk). Trees of five levels or less have no two rows to a bank, so the
-    # kernels of 64 leaves walk either kind of table (flags bit 4: as it is); the one of two dimensions and many buckets, whose
-    # vector issue is as busy, loses 4 % by it.
-    folded = pitch > 1 and not (leaves == 64 and buckets == 192)
+    folded, pair_tables = folds_leaves(buckets, pitch, leaves), has_pair_walk(buckets, pitch, leaves)
     both_tables = folded and leaves == 64
-    # Four and six dimensions, trees of four levels and less: pieces of two dimensions as with 256 leaves, and no fold (flags bit 5). Their
-    # 16 leaves of 16 bytes fill two rows of the banks, and one read does what two of 8 bytes do. 600 001 documents, 400 trees of depth
-    # 4 over 100 features, pieces of one dimension and of two: four dimensions 217 and 191 us a call, six 273 and 260, ten 420 and 391 (of
-    # depth 5, 300 trees, 300 001 documents, pieces of one are the faster: four 101 and 106, six 123 and 139; three dimensions at any depth).
-    pair_tables = both_tables and pitch >= 4 and pitch % 2 == 0
     if not fused:
         vgprs += 2 if deep else 4 if folded else 3
     two_sets = pitch == 1 and block % 2 == 0 and (fused or (vgprs + 8 <= 256 and waves_per_simd(vgprs + 8) == waves_per_simd(vgprs)))
@@ -1045,7 +1052,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                         # different banks. 64 lanes' reads of 8 bytes among 64 leaves (borders drawn evenly) take 2.6 to 2.7 cycles of
                         # LDS instead of 3.3 to 3.5. 2M documents x 2000 trees of depth 6: ten dimensions 4550 -> 4035 us, six 2838 ->
                         # 2570, four 2005 -> 1875; of depth 8, three dimensions, 1M x 2000 1518 -> 1469. (One dimension, which vector issue
-                    # bounds: the two instructions cost 2 to 5 %.)
+                        # bounds: the two instructions cost 2 to 5 %.)
                         e("  v_lshrrev_b32_e32 v4, 1, v3")
                         e("  v_bitop3_b32 v3, v4, v%d, v3 bitop3:0x6a" % fold)
                     # Places of the four documents' leaf values in the tree's table, a byte of the index for each document: a
@@ -1249,6 +1256,22 @@ def generate():
     return "\n".join(parts) + "\n"
 
 
+def generate_tables():
+    """What the host lays leaf tables out by, for hip_evaluator.hip: its table of the register kernels, those of fewer registers
+    first, and which exchange kernels read folded rows."""
+    flag = {False: "false", True: "true"}
+    rows = ['    {%d, %d, %d, %d, %s, %s, %s, %s, "%s"},' % (buckets, waves, pitch, leaves, flag[mixed], flag[six], flag[folds_leaves(buckets, pitch, leaves)],
+                                                             flag[has_pair_walk(buckets, pitch, leaves)],
+                                                             kernel_name(buckets, waves, pitch, leaves, mixed, six))
+            for buckets, waves, pitch, leaves, mixed, six in sorted(VARIANTS, key=lambda v: v[0])]
+    depths = sorted({shape[0] for shape in gen_eval_exchange_kernel.SHAPES})
+    folded = [depth for depth in depths if gen_eval_exchange_kernel.folds_leaves(depth)]
+    return "\n".join(["constexpr TEvalRegVariant kEvalRegVariants[] = {"] + rows + [
+        "};", "constexpr bool ExchangeFoldsLeaves(int depth) { return %s; }" % (" || ".join("depth == %d" % d for d in folded) or "false"), ""])
+
+
 if __name__ == "__main__":
     with open(sys.argv[1], "w") as f:
         f.write(generate())
+    with open(sys.argv[2], "w") as f:
+        f.write(generate_tables())

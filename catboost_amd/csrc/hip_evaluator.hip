@@ -269,72 +269,13 @@ struct TEvalRegVariant {
     uint32_t Leaves;  // leaf rows per tree (64: trees of depth <= 6)
     bool Mixed;       // 32-dword level tables, compare form chosen per tree
     bool Six;         // every bin at most 64: even levels compare into bit 6, two levels share a merge
+    bool Folds;       // the leaf tables are folded (64 leaves: or as they are, by a flag)
+    bool PairWalk;    // 64 leaves: or in pieces of two dimensions, by another
     const char* Name;
 };
-constexpr TEvalRegVariant kEvalRegVariants[] = {
-    {96, 8, 1, 256, false, false, "cbamd_eval_reg_b96_w8_p1_l256"},
-    {96, 8, 1, 64, false, false, "cbamd_eval_reg_b96_w8_p1_l64"},
-    {128, 4, 1, 64, false, false, "cbamd_eval_reg_b128_w4_p1_l64"},
-    {200, 4, 1, 64, false, false, "cbamd_eval_reg_b200_w4_p1_l64"},
-    {208, 4, 1, 64, false, false, "cbamd_eval_reg_b208_w4_p1_l64"},
-    {224, 4, 1, 64, false, false, "cbamd_eval_reg_b224_w4_p1_l64"},
-    {200, 4, 1, 256, false, false, "cbamd_eval_reg_b200_w4_p1_l256"},
-    {208, 4, 1, 256, false, false, "cbamd_eval_reg_b208_w4_p1_l256"},
-    {224, 4, 1, 256, false, false, "cbamd_eval_reg_b224_w4_p1_l256"},
-    {80, 4, 2, 64, false, false, "cbamd_eval_reg_b80_w4_p2_l64"},
-    {104, 4, 3, 64, false, false, "cbamd_eval_reg_b104_w4_p3_l64"},
-    {176, 4, 3, 64, false, false, "cbamd_eval_reg_b176_w4_p3_l64"},
-    {56, 4, 6, 64, false, false, "cbamd_eval_reg_b56_w4_p6_l64"},
-    {192, 4, 2, 64, false, false, "cbamd_eval_reg_b192_w4_p2_l64"},
-    {160, 4, 4, 64, false, false, "cbamd_eval_reg_b160_w4_p4_l64"},
-    {128, 4, 6, 64, false, false, "cbamd_eval_reg_b128_w4_p6_l64"},
-    {192, 4, 2, 256, false, false, "cbamd_eval_reg_b192_w4_p2_l256"},
-    {160, 4, 4, 256, false, false, "cbamd_eval_reg_b160_w4_p4_l256"},
-    {128, 4, 6, 256, false, false, "cbamd_eval_reg_b128_w4_p6_l256"},
-    {96, 8, 1, 256, true, false, "cbamd_eval_reg_b96_w8_p1_l256_m"},
-    {96, 8, 1, 64, true, false, "cbamd_eval_reg_b96_w8_p1_l64_m"},
-    {128, 4, 1, 64, true, false, "cbamd_eval_reg_b128_w4_p1_l64_m"},
-    {200, 4, 1, 64, true, false, "cbamd_eval_reg_b200_w4_p1_l64_m"},
-    {208, 4, 1, 64, true, false, "cbamd_eval_reg_b208_w4_p1_l64_m"},
-    {224, 4, 1, 64, true, false, "cbamd_eval_reg_b224_w4_p1_l64_m"},
-    {200, 4, 1, 256, true, false, "cbamd_eval_reg_b200_w4_p1_l256_m"},
-    {208, 4, 1, 256, true, false, "cbamd_eval_reg_b208_w4_p1_l256_m"},
-    {224, 4, 1, 256, true, false, "cbamd_eval_reg_b224_w4_p1_l256_m"},
-    {80, 4, 2, 64, true, false, "cbamd_eval_reg_b80_w4_p2_l64_m"},
-    {104, 4, 3, 64, true, false, "cbamd_eval_reg_b104_w4_p3_l64_m"},
-    {176, 4, 3, 64, true, false, "cbamd_eval_reg_b176_w4_p3_l64_m"},
-    {56, 4, 6, 64, true, false, "cbamd_eval_reg_b56_w4_p6_l64_m"},
-    {192, 4, 2, 64, true, false, "cbamd_eval_reg_b192_w4_p2_l64_m"},
-    {160, 4, 4, 64, true, false, "cbamd_eval_reg_b160_w4_p4_l64_m"},
-    {128, 4, 6, 64, true, false, "cbamd_eval_reg_b128_w4_p6_l64_m"},
-    {192, 4, 2, 256, true, false, "cbamd_eval_reg_b192_w4_p2_l256_m"},
-    {160, 4, 4, 256, true, false, "cbamd_eval_reg_b160_w4_p4_l256_m"},
-    {128, 4, 6, 256, true, false, "cbamd_eval_reg_b128_w4_p6_l256_m"},
-    {96, 8, 1, 256, false, true, "cbamd_eval_reg_b96_w8_p1_l256_s"},
-    {96, 8, 1, 64, false, true, "cbamd_eval_reg_b96_w8_p1_l64_s"},
-    {128, 4, 1, 64, false, true, "cbamd_eval_reg_b128_w4_p1_l64_s"},
-    {200, 4, 1, 64, false, true, "cbamd_eval_reg_b200_w4_p1_l64_s"},
-    {208, 4, 1, 64, false, true, "cbamd_eval_reg_b208_w4_p1_l64_s"},
-    {224, 4, 1, 64, false, true, "cbamd_eval_reg_b224_w4_p1_l64_s"},
-    {200, 4, 1, 256, false, true, "cbamd_eval_reg_b200_w4_p1_l256_s"},
-    {208, 4, 1, 256, false, true, "cbamd_eval_reg_b208_w4_p1_l256_s"},
-    {224, 4, 1, 256, false, true, "cbamd_eval_reg_b224_w4_p1_l256_s"},
-    {80, 4, 2, 64, false, true, "cbamd_eval_reg_b80_w4_p2_l64_s"},
-    {104, 4, 3, 64, false, true, "cbamd_eval_reg_b104_w4_p3_l64_s"},
-    {176, 4, 3, 64, false, true, "cbamd_eval_reg_b176_w4_p3_l64_s"},
-    {56, 4, 6, 64, false, true, "cbamd_eval_reg_b56_w4_p6_l64_s"},
-    {192, 4, 2, 64, false, true, "cbamd_eval_reg_b192_w4_p2_l64_s"},
-    {160, 4, 4, 64, false, true, "cbamd_eval_reg_b160_w4_p4_l64_s"},
-    {128, 4, 6, 64, false, true, "cbamd_eval_reg_b128_w4_p6_l64_s"},
-    {192, 4, 2, 256, false, true, "cbamd_eval_reg_b192_w4_p2_l256_s"},
-    {160, 4, 4, 256, false, true, "cbamd_eval_reg_b160_w4_p4_l256_s"},
-    {128, 4, 6, 256, false, true, "cbamd_eval_reg_b128_w4_p6_l256_s"},
-    // trees of depth 9 and 10 (one dimension, 1024 leaf rows; gen_eval_reg_kernel.py's DEEP_SHAPES)
-    {96, 8, 1, 1024, false, false, "cbamd_eval_reg_b96_w8_p1_l1024"},
-    {208, 4, 1, 1024, false, false, "cbamd_eval_reg_b208_w4_p1_l1024"},
-    {96, 8, 1, 1024, false, true, "cbamd_eval_reg_b96_w8_p1_l1024_s"},
-    {208, 4, 1, 1024, false, true, "cbamd_eval_reg_b208_w4_p1_l1024_s"},
-};
+// kEvalRegVariants: gen_eval_reg_kernel.py's kernels, those of fewer registers first, with what their leaf tables have to look like;
+// ExchangeFoldsLeaves: whether the exchange kernels of a depth read folded rows. Written by the generator beside the kernels.
+#include "eval_reg_tables.inc"
 constexpr int kRegMaxDepth = 10;  // deepest tree of the register kernels (one-dimensional models; 8 otherwise)
 
 // Fused kernels (binarize + evaluate in one launch, bins only ever in registers): shapes of
@@ -420,14 +361,14 @@ uint32_t RegSlicesPerGroup(size_t groups, uint32_t slices, size_t resident) {
     return best;
 }
 
-// Whether a variant's leaf tables are folded for trees of this depth: leaf l at l ^ (l >> 1) (gen_eval_reg_kernel.py: which kernels do)
+// Whether a variant's leaf tables are folded for trees of this depth: leaf l at l ^ (l >> 1)
 bool FoldsLeaves(const TEvalRegVariant& v, int depth) {
-    return v.Pitch > 1 && (v.Leaves == 256 || (v.Leaves == 64 && depth == 6 && v.Buckets != 192));
+    return v.Folds && (v.Leaves == 256 || depth == 6);
 }
 
 // ... or, of 64 leaves, hold pieces of two dimensions, 16 bytes per leaf (those of 256 leaves always do)
 bool PairsDimensions(const TEvalRegVariant& v, int depth) {
-    return v.Pitch > 1 && (v.Leaves == 256 || (v.Leaves == 64 && depth <= 4 && v.Pitch >= 4));
+    return v.Pitch > 1 && (v.Leaves == 256 || (v.PairWalk && depth <= 4));
 }
 
 // trees per LDS buffer of a variant: a power of two, at most 16, buffer at most 32 KB
@@ -2365,7 +2306,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             const TExchangeLeafRow& row = x.Plan.LeafRows[r];
             const bool tree = row.Tree != kExchangeNoTree;
             leafRows.push_back({r * pitch, tree ? firstLeaf[row.Tree] : 0u, row.Levels, tree ? static_cast<uint32_t>(pitch) : 0u,
-                                static_cast<uint32_t>(pitch) | (x.MaxDepth == 8 ? dev::kLeafRowFolded : 0u)});
+                                static_cast<uint32_t>(pitch) | (ExchangeFoldsLeaves(x.MaxDepth) ? dev::kLeafRowFolded : 0u)});
         }
         placeLeaves(&m.ExchangeLeaves, x.Plan.LeafRows.size() * pitch);
         m.ExchangeName = "cbamd_eval_exchange_" + shape;

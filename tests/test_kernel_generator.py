@@ -584,3 +584,26 @@ def test_places_of_leaf_values_of_ten_levels(shape, six):
         v = dict(vectors)
         v.update({bins_at + i: sum(x << (8 * j) for j, x in enumerate(b)) for i, b in enumerate(bins)})
         assert _follow(lines, start, scalars, v, bins_at, 8) == [8 * x for x in expected]
+
+
+def test_the_hosts_table_says_how_the_kernels_read_their_leaves():
+    """Leaf tables are laid out on the host by the table that the generator writes: which kernels fold them, and which have the walk of
+    pieces of two dimensions, has to be what the kernels' instructions do; those of exchange kernels likewise."""
+    gen = _generator()
+    rows = re.findall(r'\{(\d+), (\d+), (\d+), (\d+), (\w+), (\w+), (\w+), (\w+), "(\w+)"\}', gen.generate_tables())
+    assert len(rows) == len(gen.VARIANTS) and [int(r[0]) for r in rows] == sorted(int(r[0]) for r in rows)
+    for buckets, waves, pitch, leaves, mixed, six, folds, pairs, name in rows:
+        text, _ = gen.gen_kernel(int(buckets), int(waves), int(pitch), int(leaves), mixed == "true", six == "true")
+        assert name + "_loop:" in text
+        assert ("bitop3:0x6a" in text) == (folds == "true") and (name + "_pairs:" in text) == (pairs == "true")
+        assert (name + "_plain:" in text) == (folds == "true" and leaves == "64")
+        assert pitch != "1" or folds == pairs == "false"
+    found = re.search(r"ExchangeFoldsLeaves\(int depth\) \{ return (.*); \}", gen.generate_tables()).group(1)
+    exchange = gen.gen_eval_exchange_kernel
+    for depth, six, fused in {(shape + (False,))[:3] for shape in exchange.SHAPES}:
+        folded = exchange.folds_leaves(depth)
+        assert folded == ("depth == %d" % depth in found.split(" || "))
+        assert ("bitop3:0x6a" in exchange.gen_kernel(depth, six, fused, folded=folded)[0]) == folded
+    with open(os.path.join(ROOT, "catboost_amd", "csrc", "hip_evaluator.hip")) as f:
+        host = f.read()
+    assert '#include "eval_reg_tables.inc"' in host and "cbamd_eval_reg_b" not in host and host.count("ExchangeFoldsLeaves(") == 1
