@@ -1653,7 +1653,7 @@ struct THipEvaluator::TImpl {
     TDeviceVec<uint32_t> NsCompactEntries;
     TDeviceVec<uint32_t> NsCompactRows;  // dev::kNsUnitDwords per unit of trees
     uint32_t NsUnitCount = 0;
-    uint32_t NsEntryCount = 0;       // entries of all units: rows of NsValuesByEntry per slice of the dimensions
+    uint32_t NsEntryCount = 0;       // entries of all units: rows of NsValuesByEntry per slice of the dimensions (NsSliceRows)
     TNsLdsShape NsLdsShape{0, 0};    // waves and entries per region of EvalNonSymmetricLdsKernel for this model
     TDeviceVec<double> NsValuesByEntry;
 
@@ -2665,9 +2665,9 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     m.NsCompactEntries.Upload(padded);
                 }
                 m.NsCompactRows.Upload(units);
-                // [slice of the dimensions][entry][dimension of the slice], zeros past the last dimension and behind the last entry
+                // [slice of the dimensions][entry][dimension of the slice], zeros past the last dimension and, of one, behind the last entry
                 const uint32_t dims = NsLdsDims(m.Dim), slices = (static_cast<uint32_t>(m.Dim) + dims - 1) / dims;
-                const size_t sliceRows = entries.size() + m.NsLdsShape.Entries;
+                const size_t sliceRows = NsSliceRows(entries.size(), dims, m.NsLdsShape.Entries);
                 if (m.Dim == 1) {
                     values.resize(sliceRows, 0.0);
                 } else {

@@ -2793,10 +2793,10 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalNonSymmetricTileKernel(
 // the wave, with neither bounds nor branches - every unit starts at a multiple of four entries and `entries`
 // ends with ENTRIES spare ones (a copy written with a test per round cost a taken branch each way per round,
 // a tenth of the kernel's time). valuesByEntry holds the leaf value of every terminal entry, indexed like
-// `entries`, and ENTRIES rows of zeros behind them, which the trees that a unit lacks and those outside of the call's range
-// read; a unit's values are requested behind its walk and added after the next unit's walk. No load of values depends on a branch, so
-// that the wait for a unit's entries does not wait for the values requested behind them. (One dimension.) Behind a wave's last unit
-// no entries are fetched: a region's 4 KB and more, with one again 1M documents, 100 trees of depth 3 over 60 features took 202 us, now 191.
+// `entries`. One dimension: ENTRIES zeros behind them, which the trees that a unit lacks and those outside of the call's range
+// read; a unit's values are requested behind its walk and added after the next unit's walk, and no load of them depends on a branch, so
+// that the wait for a unit's entries does not wait for the values requested behind them. Behind a wave's last unit no entries are
+// fetched: a region's 4 KB and more, with one again 1M documents, 100 trees of depth 3 over 60 features took 202 us, now 191.
 // What bounds it: the walk's LDS reads and vector issue together (7.4 cycles of a CU for 64 chains' step; without bank conflicts
 // 6 % of the launch less, without the bins' reads 8 %, without the selects 12 %), and the values' gathers (12 of them a unit, some
 // 8 %). Whole call, with the root alone compared once for a lane's documents, the steps from there on, and values that a branch
@@ -2810,8 +2810,8 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalNonSymmetricTileKernel(
 // and 2 n + 2): LDS row of the bins << 8 | (256 - splitIdx), low byte 0: false for every bin; the eighth dword of the first tree: no
 // node of the unit's trees is on the third level.
 // Models of several dimensions: a workgroup sums DIMS of them, those from blockIdx.y * DIMS on (every slice of
-// the dimensions walks the trees again), and valuesByEntry is [slice][entryCount + ENTRIES] rows of DIMS values (zeros past
-// the last dimension), so that a leaf's values come with one aligned load; they are read and added right behind
+// the dimensions walks the trees again), and valuesByEntry is [slice][entryCount] rows of DIMS values (zeros past
+// the last dimension), so that a leaf's values come with one aligned load; those of the range's trees are read and added right behind
 // the unit's walk, with the other waves of the SIMD to cover the wait.
 // grid = (doc blocks, ceil(dim / DIMS)), block = 64 * WAVES, dynamic LDS = NsLdsTileRows(buckets, WAVES, ENTRIES) * 256
 // + 256 * 8 * DIMS bytes; no other LDS in the kernel.
@@ -2954,7 +2954,7 @@ __global__ __launch_bounds__(64 * WAVES) void EvalNonSymmetricLdsKernel(
     };
     uint32_t next = unitBehind(u);
     const uint32_t d0 = blockIdx.y * DIMS;
-    const double* sliceValues = valuesByEntry + static_cast<size_t>(blockIdx.y) * (entryCount + ENTRIES) * DIMS;
+    const double* sliceValues = valuesByEntry + static_cast<size_t>(blockIdx.y) * entryCount * DIMS;
     const uint32_t mask80 = 0x80808080u, maskC0 = 0xc0c0c0c0u;
     while (u < unitCount) {
         const uint32_t first = row[0], steps = row[1], trees = row[4] >> 16;

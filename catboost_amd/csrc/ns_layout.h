@@ -85,4 +85,10 @@ inline TNsTreeLayout LayOutNsTree(const std::vector<uint32_t>& left) {
     return layout;
 }
 
+// Rows of the leaf values of a slice of the dimensions. Of one dimension a region's zeros follow, which trees that a unit lacks or that the
+// call's range leaves out read; of several such trees' rows are not read at all.
+constexpr size_t NsSliceRows(size_t entries, uint32_t dims, uint32_t regionEntries) {
+    return dims == 1 ? entries + regionEntries : entries;
+}
+
 }  // namespace cbamd

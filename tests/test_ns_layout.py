@@ -90,3 +90,15 @@ def test_leaves_of_small_trees_have_one_place(lay_out):
         else:
             assert places == shared and len(items) <= len(left) + 1
     assert seen > 100
+
+
+def test_rows_of_leaf_values(tmp_path):
+    """One dimension reads a region's zeros behind the last entry; several read the range's trees alone, and nothing lies behind theirs."""
+    source = tmp_path / "rows.cpp"
+    source.write_text('#include "ns_layout.h"\n'
+                      "static_assert(cbamd::NsSliceRows(1000, 1, 2048) == 3048);\n"
+                      "static_assert(cbamd::NsSliceRows(1000, 2, 2048) == 1000 && cbamd::NsSliceRows(1000, 4, 1024) == 1000);\n"
+                      "int main() {}\n")
+    subprocess.check_call(["g++", "-std=c++17", "-I", os.path.join(ROOT, "catboost_amd", "csrc"), "-fsyntax-only", str(source)])
+    with open(os.path.join(ROOT, "catboost_amd", "csrc", "hip_evaluator.hip")) as f:
+        assert "sliceRows = NsSliceRows(entries.size(), dims, m.NsLdsShape.Entries)" in f.read()
