@@ -48,10 +48,12 @@ Layout of the work:
     fp64 in tree order, exactly like the CPU evaluator (cpu/evaluator_impl.cpp:362-460), and
     finished as ApplyScaleAndBias does (scale_and_bias.cpp:4-50).
 
-Kernel arguments (80 bytes):
+Kernel arguments (96 bytes; fused kernels 104, see below):
    0 bins        const uint32*   [docBlock][bucketCount][64]
    8 rows        const uint32*   [(treeBlocks + 2) * TREE_BLOCK][16 or 32]  (null trees behind the model's)
-  16 leaves      const double*   [(treeBlocks + 2) * TREE_BLOCK][LEAVES][PITCH] (fused kernels of six levels: [whole buffers of 64 trees, and two][64])
+  16 leaves      const double*   [(treeBlocks + 2) * TREE_BLOCK] tables of LEAVES * PITCH values: [LEAVES] of one dimension; of several [PITCH][LEAVES]
+                                 with 64 leaves, [PITCH / 2][LEAVES][2] with 256 and by flags bit 5, the leaves in the order that the flags
+                                 say (fused kernels of six levels: [whole buffers of 64 trees, and two][64])
   24 out         double*         [docCount][dim]
   32 docCount    uint32          36 blockCount uint32 (ceil(docCount / 256), >= 1)
   40 treeBlocks  uint32 (>= 1)   44 flags uint32 (bit 0: add the bias, bit 4: 64 leaves, several dimensions, the table is not folded,
@@ -60,8 +62,7 @@ Kernel arguments (80 bytes):
   64 bucketCount uint32 (1 .. BUCKETS)                68 dim uint32
   72 first dimension of this launch uint32            76 dimensions to store uint32 (1 .. PITCH)
   80 tree blocks per slice uint32                     84 slices per workgroup uint32 (kernels that are not fused)
-  88 map of the bins registers const uint32* (kernels that are not fused, read when flags bit 3 is set;
-     96 bytes in all)
+  88 map of the bins registers const uint32* (kernels that are not fused, read when flags bit 3 is set)
 grid = (ceil(blockCount / WAVES), ceil(slices / slices per workgroup)) workgroups of WAVES * 64 threads, LDS =
 2 * TREE_BLOCK * LEAVES * PITCH * 8 bytes. Slice s takes the tree blocks from s * (tree blocks per slice) on, at most
 that many, and writes to out + s * docCount * dim: a small batch is spread over the chip by giving the slices of
@@ -127,7 +128,7 @@ SHAPES = [
 DEEP_SHAPES = [(208, 4, 1, 1024), (96, 8, 1, 1024)]
 VARIANTS = [shape + (mixed, six) for mixed, six in ((False, False), (False, True), (True, False)) for shape in SHAPES]
 VARIANTS += [shape + (False, six) for six in (False, True) for shape in DEEP_SHAPES]
-# shapes of the fused kernels (one dimension, 256 leaf rows), each in a plain and a six-bit form. The wide shape,
+# shapes of the fused kernels (one dimension), each in a plain and a six-bit form, leaf tables of 256 rows. The wide shape,
 # and two of 64 and 80 bins registers that still run four waves per SIMD (112 and 128 registers); a model of more
 # units, up to 96 buckets, runs its separate evaluate kernel at four waves per SIMD, which a fused kernel of 96
 # bins registers (144: three) does not match: measured, two launches are the faster there.
@@ -892,58 +893,57 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             e("  s_add_u32 s34, s32, s24")
             e("  s_addc_u32 s35, s33, 0")
             e("  global_load_dword v%d, v1, s[34:35]" % (b0 + i))
-        if True:
-            # Flags bit 3: the bins registers follow a map, one dword per register: bits 0..15 the bucket it
-            # is loaded from, bits 16.. what becomes of the bins there: 0 as they are, 1 min(bin, 127), 2
-            # max(bin - 127, 0). A float bucket with more than 128 values then takes two registers, and a level
-            # "bin >= s" reads the first (s <= 127) or the second (with s - 127): every tree without xor
-            # masks runs in the 7-bit form. The map has ceil(BUCKETS / 16) * 16 entries.
-            e("  s_branch %s_loaded" % name)
-            e("%s_mapped:" % name)
-            e("  s_load_dwordx2 s[52:53], s[0:1], 0x58")
-            e("  s_mov_b32 s25, 0x7f7f7f7f")
-            batches = (buckets + 15) // 16
-            for batch in range(batches):
-                e("  s_waitcnt lgkmcnt(0)")
-                e("  s_load_dwordx16 s[36:51], s[52:53], 0x%x" % (64 * batch))
-                e("  s_waitcnt lgkmcnt(0)")
-                for k in range(16):
-                    i = 16 * batch + k
-                    if i >= buckets:
-                        break
-                    e("  s_and_b32 s24, s%d, 0xffff" % (36 + k))
-                    e("  s_lshl_b32 s24, s24, 8")
-                    e("  s_add_u32 s34, s32, s24")
-                    e("  s_addc_u32 s35, s33, 0")
-                    e("  global_load_dword v%d, v1, s[34:35]" % (b0 + i))
-            e("  s_waitcnt vmcnt(0)")
-            for batch in range(batches):
-                e("  s_load_dwordx16 s[36:51], s[52:53], 0x%x" % (64 * batch))
-                e("  s_waitcnt lgkmcnt(0)")
-                for k in range(16):
-                    i = 16 * batch + k
-                    if i >= buckets:
-                        break
-                    reg = b0 + i
-                    label = "%s_map%d" % (name, i)
-                    e("  s_lshr_b32 s24, s%d, 16" % (36 + k))
-                    e("  s_cmp_eq_u32 s24, 0")
-                    e("  s_cbranch_scc1 %s" % label)
-                    # bytes of 128 and more -> 0xff
-                    e("  v_and_b32_e32 v4, 0x80808080, v%d" % reg)
-                    e("  v_lshrrev_b32_e32 v5, 7, v4")
-                    e("  v_sub_u32_e32 v5, v4, v5")
-                    e("  v_or_b32_e32 v4, v4, v5")
-                    e("  s_cmp_eq_u32 s24, 1")
-                    e("  s_cbranch_scc1 %s_low" % label)
-                    e("  v_and_b32_e32 v5, 0x7f7f7f7f, v%d" % reg)      # those bytes: (bin & 127) + 1 = bin - 127
-                    e("  v_add_u32_e32 v5, 0x1010101, v5")
-                    e("  v_and_b32_e32 v%d, v4, v5" % reg)
-                    e("  s_branch %s" % label)
-                    e("%s_low:" % label)
-                    e("  v_bfi_b32 v%d, v4, s25, v%d" % (reg, reg))      # those bytes: 127
-                    e("%s:" % label)
-            e("%s_loaded:" % name)
+        # Flags bit 3: the bins registers follow a map, one dword per register: bits 0..15 the bucket it
+        # is loaded from, bits 16.. what becomes of the bins there: 0 as they are, 1 min(bin, 127), 2
+        # max(bin - 127, 0). A float bucket with more than 128 values then takes two registers, and a level
+        # "bin >= s" reads the first (s <= 127) or the second (with s - 127): every tree without xor
+        # masks runs in the 7-bit form. The map has ceil(BUCKETS / 16) * 16 entries.
+        e("  s_branch %s_loaded" % name)
+        e("%s_mapped:" % name)
+        e("  s_load_dwordx2 s[52:53], s[0:1], 0x58")
+        e("  s_mov_b32 s25, 0x7f7f7f7f")
+        batches = (buckets + 15) // 16
+        for batch in range(batches):
+            e("  s_waitcnt lgkmcnt(0)")
+            e("  s_load_dwordx16 s[36:51], s[52:53], 0x%x" % (64 * batch))
+            e("  s_waitcnt lgkmcnt(0)")
+            for k in range(16):
+                i = 16 * batch + k
+                if i >= buckets:
+                    break
+                e("  s_and_b32 s24, s%d, 0xffff" % (36 + k))
+                e("  s_lshl_b32 s24, s24, 8")
+                e("  s_add_u32 s34, s32, s24")
+                e("  s_addc_u32 s35, s33, 0")
+                e("  global_load_dword v%d, v1, s[34:35]" % (b0 + i))
+        e("  s_waitcnt vmcnt(0)")
+        for batch in range(batches):
+            e("  s_load_dwordx16 s[36:51], s[52:53], 0x%x" % (64 * batch))
+            e("  s_waitcnt lgkmcnt(0)")
+            for k in range(16):
+                i = 16 * batch + k
+                if i >= buckets:
+                    break
+                reg = b0 + i
+                label = "%s_map%d" % (name, i)
+                e("  s_lshr_b32 s24, s%d, 16" % (36 + k))
+                e("  s_cmp_eq_u32 s24, 0")
+                e("  s_cbranch_scc1 %s" % label)
+                # bytes of 128 and more -> 0xff
+                e("  v_and_b32_e32 v4, 0x80808080, v%d" % reg)
+                e("  v_lshrrev_b32_e32 v5, 7, v4")
+                e("  v_sub_u32_e32 v5, v4, v5")
+                e("  v_or_b32_e32 v4, v4, v5")
+                e("  s_cmp_eq_u32 s24, 1")
+                e("  s_cbranch_scc1 %s_low" % label)
+                e("  v_and_b32_e32 v5, 0x7f7f7f7f, v%d" % reg)      # those bytes: (bin & 127) + 1 = bin - 127
+                e("  v_add_u32_e32 v5, 0x1010101, v5")
+                e("  v_and_b32_e32 v%d, v4, v5" % reg)
+                e("  s_branch %s" % label)
+                e("%s_low:" % label)
+                e("  v_bfi_b32 v%d, v4, s25, v%d" % (reg, reg))      # those bytes: 127
+                e("%s:" % label)
+        e("%s_loaded:" % name)
     load_rows(rows_a, 0)
     load_rows(rows_b, 1)
     for r in list(range(lv0, ga0)) + (list(range(lw0, lw0 + 8)) if two_sets else []):

@@ -809,8 +809,8 @@ int TileChunk(int dim) {
 // from a node, the chosen side's diff leads to the next node and a zero diff ends the walk at the
 // node's own leaf (NonSymmetricNodeIdToLeafId). A zero side becomes a terminal entry of its own.
 // usable = false when a tree does not fit the 16-bit offsets of an entry.
-// The compact tables (EvalNonSymmetricLdsKernel) are filled when the model is one-dimensional,
-// has at most 1023 buckets and no tree above dev::kNsLdsEntries entries (one-hot splits count two).
+// The compact tables (EvalNonSymmetricLdsKernel) are filled when the model, of any dimension, has at most 1023 buckets and
+// no tree above dev::kNsLdsEntries entries (one-hot splits count two).
 void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<uint32_t>& firstLeaf,
                           TDeviceVec<uint32_t>* entriesOut, TDeviceVec<uint32_t>* rowsOut, bool* usable, bool* noXor,
                           std::vector<uint32_t>* compactEntries, std::vector<uint32_t>* compactRows, std::vector<uint32_t>* topNodes,
@@ -1649,7 +1649,7 @@ struct THipEvaluator::TImpl {
     bool NsNoXor = false;
     TDeviceVec<uint32_t> NsEntries;  // pairs of dwords
     TDeviceVec<uint32_t> NsRows;     // 4 dwords per tree
-    bool NsLdsUsable = false;        // compact entries walked out of LDS (one-dimensional, no xor)
+    bool NsLdsUsable = false;        // compact entries walked out of LDS (xor masks as splits of their own)
     TDeviceVec<uint32_t> NsCompactEntries;
     TDeviceVec<uint32_t> NsCompactRows;  // dev::kNsUnitDwords per unit of trees
     uint32_t NsUnitCount = 0;
@@ -2898,7 +2898,8 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         // and 128 registers: four waves per SIMD like their evaluate kernel); with more units they stay on two launches
         // (a fused kernel of 96 bins registers would run at three waves per SIMD and is the slower - measured on
         // 50 and 90 buckets). A model on the six-level kernel takes the form of the fused kernel that walks six levels, whose
-        // buffers hold 64 trees: null trees up to whole buffers, and two more.
+        // buffers hold 64 trees: null trees up to whole buffers, and two more. (The limit on the table's bytes, which the kernels address by
+        // 32 bits, counts 256 rows a tree for either form: some two million trees.)
         const bool fusedCandidate = switches.Fused && !regMapped && !variant->Mixed && variant->Pitch == 1 && variant->Leaves <= 256 && m.Dim == 1 && !m.HasCats &&
                                     m.CtrCount == 0 && m.BinarizeBuckets == BucketCount && BucketCount > 0 &&
                                     (TreeCount / block + 3) * block * 256 * 8 + 16 * kFusedImageBytes < (uint64_t(1) << 32) - (1u << 20);

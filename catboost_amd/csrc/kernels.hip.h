@@ -2768,7 +2768,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void EvalNonSymmetricTileKernel(
     }
 }
 
-// Non-symmetric models without xor masks whose trees have at most kNsLdsEntries entries: as EvalNonSymmetricTileKernel, but a
+// Non-symmetric models whose trees have at most kNsLdsEntries entries (a split by a xor mask is two of plain bins): as EvalNonSymmetricTileKernel, but a
 // wave walks its trees out of a copy in its own LDS region (an LDS gather costs a fraction of a gather from global memory).
 // Trees are grouped into units of up to kNsUnitTrees trees and ENTRIES entries; a wave takes a unit at a time and walks its
 // trees side by side (4 documents x kNsUnitTrees chains per lane).
