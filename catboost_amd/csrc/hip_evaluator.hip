@@ -650,26 +650,27 @@ size_t NsLdsKernelBytes(uint32_t buckets, uint32_t waves, uint32_t entries, uint
     return static_cast<size_t>(dev::NsLdsTileRows(buckets, waves, entries)) * 256 + dev::kDocsPerBlock * sizeof(double) * dims;
 }
 
-// The shapes of EvalNonSymmetricLdsKernel, most waves first
 // dimensions that one workgroup of EvalNonSymmetricLdsKernel sums (a model of more walks its trees once per slice)
 uint32_t NsLdsDims(int dim) {
     return dim == 1 ? 1 : dim == 2 ? 2 : 4;
 }
 
 // Few buckets leave LDS for larger regions (fewer units, larger trees) at a given number of waves, and 249 to 312 buckets
-// for ten or eleven waves where trees of more than 1536 entries used to leave eight. Evaluate launch, 1M documents, trees
-// of depth 10: 500 trees over 100 features 1250 us with eight waves of 2048 entries, 1131 with twelve of 1536, 1062 with
-// twelve of 2048, 1027 with sixteen of 2048; 500 over 300 features 1298 with eight, 1223 with ten, 1201 with eleven of 1792,
-// 1196 with twelve of 1536; 300 of three dimensions over 100 features 975 with eight, 832 with twelve of 2048, 812 with
-// sixteen of 1536.
-// The model's shape is the one with the least steps / speed. Steps (a unit takes as many as its tallest tree) per time,
-// relative to eight waves, measured over eleven models of depth 6 to 10, 20 to 300 features, one and three dimensions:
-//   16 x 1024 1.33 .. 1.41   16 x 1536 1.23 .. 1.40   16 x 2048 1.18 .. 1.25   12 x 1536 1.14 .. 1.32
-//   12 x 2048 1.12 .. 1.19   11 x 1792 1.11 .. 1.18   10 x 2048 1.05 .. 1.09
-// (a region that is fuller takes longer per step, so a shape's speed falls as its units shrink). The figures below, set on
-// two models, differ from these by up to 0.1; they gave nine of the eleven models the fastest shape and one (three
-// dimensions over 100 features) the second, 2 % behind. The last one has 20 features: there two workgroups of eight waves
-// share a CU (870 us against 999 with the 16 x 2048 that is taken), which the rule does not know.
+// for ten or eleven waves where trees of more than 1536 entries would leave eight. Evaluate launch, 500 000 documents, 500 trees
+// of depth 10 over 100 features: 580 us with eight waves of 2048 entries, 544 with twelve of 1536, 506 with twelve of 2048, 508 with
+// sixteen of 1536, 484 with sixteen of 2048; over 300 features 598 with eight, 559 with ten, 544 with eleven of 1792, 557 with
+// twelve of 1536; 1M, 500 of depth 6 over 60 753 with eight, 630 with twelve of 1536, 546 with sixteen of 1024; three dimensions, 500 000, 300 of
+// depth 8 over 100 408 with eight, 369 with twelve of 1536, 351 with sixteen of 1024.
+// The model's shape is the one with the least steps / speed. Steps (a unit takes as many as its tallest tree, and the three top levels for
+// three more) per time, relative to eight waves, measured over eight models of depth 6 to 10, 100 to 300 features, one to three dimensions:
+//   16 x 1024 1.16 .. 1.38   16 x 1536 1.09 .. 1.34   16 x 2048 1.20 .. 1.23   12 x 1536 1.11 .. 1.23   12 x 2048 1.09 .. 1.15
+//   11 x 1792 1.08 .. 1.17   10 x 2048 1.05 .. 1.09   (counting the top levels as no step or as five: the same within 0.04)
+// (a region that is fuller takes longer per step, so a shape's speed falls as its units shrink). The figures below were set on
+// two models and a walk that began at the root; they still give seven of these eight the fastest shape and one (depth 10 over 300
+// features) the second, 2 % behind. Of five models of 20 to 60 features two had a faster one: there two workgroups of eight waves
+// share a CU (100 trees of depth 8 over 50 features 163 us against the 189 of the 16 x 1024 that is taken, 500 of depth 9 over 20 476 against
+// 487), which the rule does not know.
+// The shapes of EvalNonSymmetricLdsKernel, most waves first.
 struct TNsLdsShape {
     uint32_t Waves;
     uint32_t Entries;
@@ -2586,9 +2587,8 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
         BuildLevelOrderTrees(trees, m.Dim, firstLeaf, &m.NsEntries, &m.NsRows, &m.NsTileUsable, &m.NsNoXor,
                              &compactEntries, &compactRows, &topNodes, &valuesByEntry, &m.NsLdsUsable);
         if (m.NsLdsUsable) {
-            // the shape whose units take the least time: more waves hide more of the walk's latency (steps per
-            // unit of time relative to 8 waves, measured on 500 trees of about 430 entries: 12 waves 1.26), smaller
-            // regions hold fewer trees per unit
+            // the shape whose units take the least time: more waves hide more of the walk's latency, smaller
+            // regions hold fewer trees per unit (kNsLdsShapes)
             m.NsLdsUsable = false;
             double bestCost = 0.0;
             std::vector<TNsUnit> bestUnits;
@@ -2603,7 +2603,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 }
                 uint64_t steps = 0;
                 for (const TNsUnit& unit : plan) {
-                    steps += unit.Height + 3;  // the top three levels, which the shapes' speeds were measured with as steps
+                    steps += unit.Height + 3;  // the top three levels
                 }
                 const double cost = static_cast<double>(steps) / shape.Speed;
                 if (!m.NsLdsUsable || cost < bestCost) {
@@ -3862,8 +3862,11 @@ void THipEvaluator::EvalQuantizedDevice(const uint8_t* bins, size_t docCount, si
         return;
     }
     // A unit holds trees of like height from anywhere in the model, so a range of the trees still walks most
-    // units: below about a third of the trees the kernel that walks the range's trees alone is the faster
-    // (C4, 1M documents: all trees 1.4 against 3.5 ms, half of them 1.3 against 1.8, a fifth 0.9 against 0.7).
+    // units: the kernel that walks the range's trees alone is the faster for about a tenth of them. Evaluate launch, that kernel and this
+    // one, three tenths, a fifth and a tenth of the trees: 500 of depth 10 over 300 features (500 000 documents) 483 and 365, 326 and 303, 191
+    // and 234 us; 500 of depth 6 over 60 (1M) 552 and 292, 377 and 279, 203 and 215; three dimensions, 300 of depth 8 over 100 (500 000) 293
+    // and 196, 204 and 166, 115 and 123; 100 of depth 8 over 50 (1M) 161 and 147, 110 and 142, 71 and 115. (The line is where it was with the
+    // walk from the root; of the seven models measured the smallest alone crosses above a fifth.)
     if (!m.Oblivious && m.NsLdsUsable && (treeEnd - treeStart) * 10 >= TreeCount * 3) {
         const size_t blocks = (docCount + dev::kDocsPerBlock - 1) / dev::kDocsPerBlock;
         const uint32_t dims = NsLdsDims(m.Dim);
