@@ -18,11 +18,11 @@ block are too many for one wave's registers (up to 1024 buckets) but fit the reg
     values gathered before the step's group is compared, and added behind the next step's wait;
   * a tree's leaf values go from global memory to the wave's own LDS region (three regions per wave, two steps ahead).
 
-What bounds it: LDS. Per tree and 256 documents 36 vector and 26 scalar instructions, and of the 102 cycles (of 2.4 GHz) that a step of
-sixteen waves takes for each 61 of reads (by its counters before the leaf rows were folded: four gathers and nine dwords, the bins' tables in the fused
-form; 28 of them bank conflicts) and 32 for the 2 KB of leaf values, which come in at 64 bytes per clock; the pair-tile kernel, in which only
-128 documents share a copy of the leaf values and every level reads its bins, issues 82 vector instructions. 262 144 documents x 5000 trees x 1016
-buckets 0.70 ms; with half of the leaf values' copies left out 0.60, without the gathers 0.60, without reading the groups' dwords
+What bounds it: LDS. Per tree and 256 documents 36 vector and 26 scalar instructions, and of the 100 cycles (at the 2.34 GHz it runs at, fused
+form) that a step of sixteen waves takes for each 56 of reads (by its counters: four gathers and nine dwords, the bins' tables; 23 of them bank
+conflicts, 28 before the leaf rows were folded) and 32 for the 2 KB of leaf values, which come in at 64 bytes per clock; the pair-tile kernel, in which only
+128 documents share a copy of the leaf values and every level reads its bins, issues 82 vector instructions. Over bins from memory and before
+the fold (84 cycles of 2.4 GHz), 262 144 documents x 5000 trees x 1016 buckets 0.70 ms; with half of the leaf values' copies left out 0.60, without the gathers 0.60, without reading the groups' dwords
 0.59, without the barriers 0.68, without loading rows 0.69. Tried: every request in the step that waits for it 0.77, slots
 addressed by vector registers (nine more vector instructions) 0.72, leaf values through registers and ds_write_b128 0.78, one
 tree in four gathered from global memory 0.70. Some 13 us per workgroup go to its start (the bins, the first groups) and end.
