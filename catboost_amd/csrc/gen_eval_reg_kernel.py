@@ -37,9 +37,11 @@ Layout of the work:
     48.7 -> 44.5. (With the mode on for the merges 71.8, 57.8, 48.6, 47.2; with SDWA 72.1, 61, 50, 48.)
     Mixed variants: 32 dwords per tree. Bit 31 of the first dword clear: the 7-bit form above (the
     tree has no xor mask and no bin of its buckets is above 128). Set: 4 dwords per level, bucket,
-    xorMask, splitIdx & 0x7f (both times 0x01010101) and 0x80808080 if splitIdx < 128 else 0; the
-    unsigned byte compare (bin ^ xorMask) >= splitIdx is then bit 7 of
-    majority(x, (x | 0x80) - (splitIdx & 0x7f), splitIdx < 128) taken per byte, x = bin ^ xorMask;
+    xorMask, 256 - splitIdx (both times 0x01010101) and one that nothing reads; the unsigned byte compare
+    (bin ^ xorMask) >= splitIdx is the ninth bit of a sum, which v_lerp_u8 leaves in bit 7. (As the majority of the byte,
+    its difference from the split and a flag, and with a merge per level in index mode, six vector instructions a level where four
+    are now: 1M documents, 1000 trees, ten one-hot columns beside 190 features 340 -> 303 us a launch at depth 8, 276 -> 260 at 6; eight beside 60,
+    two dimensions, depth 6 307 -> 256; ten dimensions, 54 743 documents, 39 trees of depth 6 over eight 31.4 -> 29.1.)
   * the leaf gathers of a tree (four documents per lane) are issued behind its levels and consumed
     after the levels of the next tree, so their LDS latency is covered. One-dimensional kernels with
     eight registers to spare keep two sets of leaf values: a tree's gathers go out in one batch right
@@ -345,15 +347,12 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
         """Index mode: src0 of vector instructions becomes relative to a level's bucket."""
         e("  s_set_gpr_idx_on s%d, 0x1" % register if on else "  s_set_gpr_idx_off")
 
-    def levels_in_pairs(rows, invert_top):
-        """A pair of levels puts its bits into bits 6 and 7 of a document's byte, and one shift and one select bring
-        them into the index. Bins of at most 64 (six-bit variants): the host gives the even levels the constant
-        (64 - splitIdx), whose sum has the level's bit in bit 6 and bit 7 clear. Else every level has (128 -
-        splitIdx), and v_lerp_u8, bytewise (bin + constant) >> 1 from a sum of nine bits, leaves the even level's bit in
-        bit 6 and bit 7 clear.
-        invert_top: the top bit of every index comes inverted (see gather_addresses)."""
-        count = min(depth, 8)
-        for d in range(count):
+    def pair_sums(rows):
+        """A pair of levels puts its bits into bits 6 and 7 of a document's byte. Bins of at most 64 (six-bit variants): the
+        host gives the even levels the constant (64 - splitIdx), whose sum has the level's bit in bit 6 and bit 7 clear. Else
+        every level has (128 - splitIdx), and v_lerp_u8, bytewise (bin + constant) >> 1 from a sum of nine bits, leaves the even
+        level's bit in bit 6 and bit 7 clear."""
+        for d in range(min(depth, 8)):
             if d == 0:
                 index_mode(True, rows)
             else:
@@ -363,6 +362,11 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             else:
                 e("  v_add_u32_e64 v%d, v%d, s%d" % (sums[d], b0, rows + 2 * d + 1))
         index_mode(False)
+
+    def merge_pairs(invert_top):
+        """One select joins the bits of a pair, a shift and a select bring them into the index.
+        invert_top: the top bit of every index comes inverted (see gather_addresses)."""
+        count = min(depth, 8)
         for pair in range(count // 2):
             select(sums[2 * pair], mask80, sums[2 * pair + 1], sums[2 * pair], invert_top and pair == count // 2 - 1)
         if first_level_masked:
@@ -371,7 +375,9 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
             e("  v_lshrrev_b32_e32 v3, 2, v%d" % (sums[0] if pair == 1 else 3))
             select(3, mask_c0, sums[2 * pair], 3)
 
-    def levels_eight_bit(rows):
+    def eight_bit_sums(rows):
+        """The sums that merge_pairs takes, of a tree of the mixed kernels whose levels compare eight bits: with a constant of
+        256 - splitIdx, v_lerp_u8 leaves the ninth bit of the sum, bin ^ xorMask >= splitIdx, in bit 7 of every byte."""
         for d in range(depth):
             level = rows + 4 * d
             # index = bits 0..7 of the bucket dword
@@ -379,20 +385,11 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                 index_mode(True, level)
             else:
                 e("  s_set_gpr_idx_idx s%d" % level)
-            e("  v_xor_b32_e64 v4, v%d, s%d" % (b0, level + 1))       # x = bin ^ xorMask
-            e("  v_or_b32_e32 v5, s22, v4")
-            e("  v_subrev_u32_e32 v5, s%d, v5" % (level + 2))         # (x | 0x80) - (splitIdx & 0x7f), per byte
-            if d == 0 and not first_level_masked:
-                e("  v_bitop3_b32 v3, s%d, v4, v5 bitop3:0xe8" % (level + 3))  # majority
-                continue
-            # majority; of the top level its complement
-            e("  v_bitop3_b32 v4, s%d, v4, v5 bitop3:0x%x" % (level + 3, 0x17 if d == depth - 1 else 0xe8))
-            if d == 0:
-                e("  v_and_b32_e32 v3, s22, v4")
-            else:
-                e("  v_lshrrev_b32_e32 v3, 1, v3")
-                e("  v_bfi_b32 v3, s22, v4, v3")
+            e("  v_xor_b32_e64 v3, v%d, s%d" % (b0, level + 1))
+            e("  v_lerp_u8 v%d, s%d, v3, 0" % (sums[d], level + 2))
         index_mode(False)
+        for d in range(0, depth, 2):
+            e("  v_lshrrev_b32_e32 v%d, 1, v%d" % (sums[d], sums[d]))
 
     # ---- the binarize phase's search, shared by the rows' and the columns' form
     out_of_line = []
@@ -811,7 +808,6 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
     # the three instructions above and the s_nop keep it well clear
     e("  s_nop 1")
     e("  v_readfirstlane_b32 s20, v5")           # wave of the workgroup
-    e("  s_mov_b32 s22, 0x80808080")
     # byte j of the leaf indexes times the unpacking weight = offset of the document's leaf row in a tree's table
     # (a six-level index sits in bits 2..7 of its byte); deep kernels: a ten-bit index times s23
     if deep:
@@ -1020,13 +1016,14 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
                     label = "%s%s_t%d_%d" % (name, loop, buf, i)
                     e("  s_bitcmp1_b32 s%d, 31" % rows)
                     e("  s_cbranch_scc1 %s_x" % label)
-                    levels_in_pairs(rows, True)
+                    pair_sums(rows)
                     e("  s_branch %s_j" % label)
                     e("%s_x:" % label)
-                    levels_eight_bit(rows)
+                    eight_bit_sums(rows)
                     e("%s_j:" % label)
                 else:
-                    levels_in_pairs(rows, not deep)
+                    pair_sums(rows)
+                merge_pairs(not deep)
                 if deep:
                     levels_high(rows)
                 tree_offset = buf * buf_bytes + i * tree_bytes

@@ -2822,8 +2822,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     }
                     row[4 * d] = bucket;
                     row[4 * d + 1] = xorMask * 0x01010101u;
-                    row[4 * d + 2] = (splitIdx & 0x7fu) * 0x01010101u;
-                    row[4 * d + 3] = splitIdx < 128 ? 0x80808080u : 0u;
+                    row[4 * d + 2] = (256u - splitIdx) * 0x01010101u;  // (a split's index is at least 1)
                 }
                 row[0] |= 0x80000000u;
             }

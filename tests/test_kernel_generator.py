@@ -536,7 +536,7 @@ def test_places_of_leaf_values_of_mixed_trees(shape):
         folded = lines[start].endswith("_loop:") and pitch > 1 and buckets != 192
         dims = 2 if pitch > 1 and (leaves == 256 or lines[start].endswith("_pairs:")) else 1
         constants, vectors = _constants(lines, start)
-        bins_at = next(int(m.group(1)) for m in (re.match(r"v_xor_b32_e64 v4, v(\d+), s", line) for line in lines) if m)
+        bins_at = next(int(m.group(1)) for m in (re.match(r"v_xor_b32_e64 v3, v(\d+), s", line) for line in lines) if m)
         for turn in range(120):
             wide = turn % 2 == 1
             top = 255 if wide else 128
@@ -548,7 +548,7 @@ def test_places_of_leaf_values_of_mixed_trees(shape):
                 mask = rng.choice([0, 0, rng.randrange(256)]) if wide else 0
                 if wide:
                     scalars.update({32 + 4 * d: bucket | (0x80000000 if d == 0 else 0), 33 + 4 * d: mask * 0x01010101,
-                                    34 + 4 * d: (split & 0x7f) * 0x01010101, 35 + 4 * d: 0x80808080 if split < 128 else 0})
+                                    34 + 4 * d: (256 - split) * 0x01010101})
                 else:
                     scalars.update({32 + 2 * d: bucket, 33 + 2 * d: (128 - split) * 0x01010101})
                 for j in range(4):
