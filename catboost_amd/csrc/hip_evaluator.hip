@@ -983,7 +983,7 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
         for (uint32_t at = 0; at < count; ++at) {
             const uint32_t next = at < placed.size() ? layout.Next[at] : at;
             if (at >= placed.size() || compact.Order[placed[at]].Terminal) {
-                compactEntries->push_back((next % 2 != 0 ? 0u : 255u) | ((next & ~1u) << 21));
+                compactEntries->push_back(NsTerminalEntry(next));
             } else {
                 *compactUsable = *compactUsable && splitOf(placed[at]) <= 255;
                 compactEntries->push_back((splitOf(placed[at]) & 0xffu) | bucketOf(placed[at]) << 8 | next << 21);
@@ -2638,6 +2638,17 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                             values.insert(values.end(), value, value + m.Dim);
                         }
                         count += treeEntries;
+                    }
+                    if (unit.Height == 0) {
+                        std::vector<uint32_t> from;
+                        for (uint32_t i = 0; i < unit.TreeCount; ++i) {
+                            CompactNsExits(entries.data() + first + start[i], &from);
+                        }
+                        const size_t dim = static_cast<size_t>(m.Dim);
+                        const std::vector<double> old(values.begin() + static_cast<std::ptrdiff_t>(first * dim), values.end());
+                        for (size_t r = 0; r < from.size(); ++r) {
+                            std::copy_n(old.data() + from[r] * dim, dim, values.data() + (first + r) * dim);
+                        }
                     }
                     const uint32_t row[8] = {first, unit.Height, first, start[1], start[2] | (unit.TreeCount << 16),
                                              unit.Trees[0], unit.Trees[1], unit.Trees[2]};

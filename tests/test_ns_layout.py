@@ -102,3 +102,48 @@ def test_rows_of_leaf_values(tmp_path):
     subprocess.check_call(["g++", "-std=c++17", "-I", os.path.join(ROOT, "catboost_amd", "csrc"), "-fsyntax-only", str(source)])
     with open(os.path.join(ROOT, "catboost_amd", "csrc", "hip_evaluator.hip")) as f:
         assert "sliceRows = NsSliceRows(entries.size(), dims, m.NsLdsShape.Entries)" in f.read()
+
+
+def test_rows_of_trees_that_end_at_their_exits(tmp_path):
+    """Units without a step: every exit names a row with its own leaf's value, the rows of a unit's trees lie behind each other from the
+    first on, one per leaf that an exit holds, and their entries read as the kernel reads them."""
+    source = tmp_path / "exits.cpp"
+    source.write_text(r'''
+#include "ns_layout.h"
+#include <cstdio>
+int main() {
+    for (unsigned seed = 1; seed < 2000; ++seed) {
+        unsigned state = seed * 2654435761u;
+        const auto draw = [&](unsigned n) { state = state * 1664525u + 1013904223u; return (state >> 10) % n; };
+        std::vector<uint32_t> from;
+        size_t rows = 0;
+        for (unsigned tree = 0, trees = 1 + draw(3); tree < trees; ++tree) {
+            const unsigned start = 16 * tree, leaves = 1 + draw(8);
+            uint32_t exits[8], places[8];
+            bool held[16] = {};
+            for (unsigned exit = 0; exit < 8; ++exit) {
+                places[exit] = start + draw(leaves) * 2 % 16 + (leaves > 4 ? draw(2) : 0);
+                held[places[exit] - start] = true;
+                exits[exit] = cbamd::NsTerminalEntry(places[exit]);
+            }
+            cbamd::CompactNsExits(exits, &from);
+            for (bool h : held) {
+                rows += h;
+            }
+            if (from.size() != rows) {
+                return 1;
+            }
+            for (unsigned exit = 0; exit < 8; ++exit) {
+                const uint32_t row = ((exits[exit] >> 18) | (~exits[exit] & 8u)) / 8;
+                if (row >= rows || from[row] != places[exit] || (exits[exit] & 0x1fff00u) != 0) {
+                    return 2;
+                }
+            }
+        }
+    }
+    return 0;
+}
+''')
+    program = str(tmp_path / "exits")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-I", os.path.join(ROOT, "catboost_amd", "csrc"), str(source), "-o", program])
+    subprocess.check_call([program])
