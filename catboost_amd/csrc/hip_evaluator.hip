@@ -693,21 +693,23 @@ struct TNsUnit {
     uint32_t Height;
 };
 
-// Groups the trees (rows: first entry, steps behind the exits, entry count, unused) into units of at most `limit` entries.
-// A unit takes as many steps as its tallest tree, so the trees go in by falling height, and every tree joins
-// the fullest of the recently opened units that still has room for it (trees need not be neighbours in the
-// model: the kernel's sums are partial sums per wave anyway). False when a tree exceeds the limit.
-bool PackNsUnits(const std::vector<uint32_t>& rows, size_t treeCount, uint32_t limit, std::vector<TNsUnit>* units) {
+// The trees (rows: first entry, steps behind the exits, entry count, unused) by falling height, the order in which PackNsUnits takes them
+std::vector<uint32_t> OrderNsTrees(const std::vector<uint32_t>& rows, size_t treeCount) {
     std::vector<uint32_t> order(treeCount);
-    for (size_t t = 0; t < treeCount; ++t) {
-        if (rows[t * 4 + 2] > limit) {
-            return false;
-        }
-        order[t] = static_cast<uint32_t>(t);
-    }
+    std::iota(order.begin(), order.end(), 0u);
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
         return rows[a * 4 + 1] != rows[b * 4 + 1] ? rows[a * 4 + 1] > rows[b * 4 + 1] : rows[a * 4 + 2] > rows[b * 4 + 2];
     });
+    return order;
+}
+
+// Groups the trees into units of at most `limit` entries. A unit takes as many steps as its tallest tree, so the trees go in by
+// falling height, and every tree joins the fullest of the recently opened units that still has room for it (trees need not be
+// neighbours in the model: the kernel's sums are partial sums per wave anyway). False when a tree exceeds the limit.
+bool PackNsUnits(const std::vector<uint32_t>& rows, const std::vector<uint32_t>& order, uint32_t limit, std::vector<TNsUnit>* units) {
+    if (std::any_of(order.begin(), order.end(), [&](uint32_t t) { return rows[t * 4 + 2] > limit; })) {
+        return false;
+    }
     constexpr size_t kWindow = 64;  // open units looked at per tree
     std::vector<size_t> open;
     for (const uint32_t t : order) {
@@ -838,8 +840,12 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
     // them: "bin >= v" (false: the model's left side) and behind its true side "bin >= v + 1" (false: the
     // model's right side, the bins are equal; true: the left side again). The entry of the left side is
     // repeated there, not its subtree: the copy names the same pair of children.
-    const auto unfold = [&](uint32_t root, bool splitOneHot) {
-        TUnfolded u;
+    const auto unfold = [&](uint32_t root, bool splitOneHot, TUnfolded* unfolded) {
+        TUnfolded& u = *unfolded;
+        u.Order.clear();
+        u.Level.clear();
+        u.Children.clear();
+        u.Height = 0;
         u.Order.push_back({root, false});
         u.Level.push_back(0);
         for (size_t i = 0; i < u.Order.size() && u.Order.size() * 8 <= 0xffffu; ++i) {
@@ -898,7 +904,6 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
             u.Children.emplace_back(child[0], child[1]);
         }
         u.Fits = u.Order.size() * 8 <= 0xffffu;
-        return u;
     };
     const size_t treeCount = trees.GetTreeCount();
     *noXor = true;
@@ -909,10 +914,13 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
     *usable = true;
     *compactUsable = trees.EffectiveBinFeaturesBucketCount <= 1023;
     compactRows->assign(treeCount * 4, 0);
+    TUnfolded plain, split;  // (these are filled anew by every tree)
+    std::vector<uint32_t> left;
+    TNsTreeLayout layout;
     for (size_t t = 0; t < treeCount && *usable; ++t) {
         const uint32_t root = static_cast<uint32_t>(trees.TreeStartOffsets[t]);
         const size_t firstEntry = entries.size() / 2;
-        const TUnfolded plain = unfold(root, false);
+        unfold(root, false, &plain);
         if (!plain.Fits) {
             *usable = false;
             break;
@@ -948,7 +956,9 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
             *compactUsable = false;
             continue;
         }
-        const TUnfolded split = *noXor ? TUnfolded() : unfold(root, true);
+        if (!*noXor) {
+            unfold(root, true, &split);
+        }
         const TUnfolded& compact = *noXor ? plain : split;
         *compactUsable = compact.Fits && compact.Order.size() + 1 <= static_cast<size_t>(dev::kNsLdsEntries);
         if (!*compactUsable) {
@@ -963,11 +973,11 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
             return ((~static_cast<uint32_t>(rb.XorMask)) & 0xffu) + (compact.Order[i].Second ? 1u : 0u);
         };
         const auto bucketOf = [&](size_t i) { return static_cast<uint32_t>(trees.RepackedBins[compact.Order[i].Node].FeatureIndex); };
-        std::vector<uint32_t> left(compact.Order.size());
+        left.resize(compact.Order.size());
         for (size_t i = 0; i < left.size(); ++i) {
             left[i] = compact.Order[i].Terminal ? kNsNoItem : compact.Children[i].first;  // the true side always follows the false side
         }
-        const TNsTreeLayout layout = LayOutNsTree(left);
+        LayOutNsTree(left, &layout);
         // the seven nodes of the top levels; false for every bin where there is none
         for (const uint32_t i : layout.TopItems) {
             *compactUsable = *compactUsable && (i == kNsNoItem || splitOf(i) <= 255);
@@ -980,19 +990,20 @@ void BuildLevelOrderTrees(const TModelTrees& trees, int dim, const std::vector<u
         (*compactRows)[t * 4 + 1] = layout.Steps;
         (*compactRows)[t * 4 + 2] = static_cast<uint32_t>(count);
         *compactUsable = *compactUsable && count <= static_cast<size_t>(dev::kNsLdsEntries);
+        compactEntries->resize(compactEntries->size() + count);
+        valuesByEntry->resize(compactEntries->size() * dim, 0.0);
+        uint32_t* entryAt = compactEntries->data() + compactEntries->size() - count;
+        double* valueAt = valuesByEntry->data() + valuesByEntry->size() - count * dim;
         for (uint32_t at = 0; at < count; ++at) {
-            const uint32_t next = at < placed.size() ? layout.Next[at] : at;
-            if (at >= placed.size() || compact.Order[placed[at]].Terminal) {
-                compactEntries->push_back(NsTerminalEntry(next));
+            if (at >= placed.size()) {
+                entryAt[at] = NsTerminalEntry(at);
+            } else if (compact.Order[placed[at]].Terminal) {
+                entryAt[at] = NsTerminalEntry(layout.Next[at]);
+                std::copy_n(trees.LeafValues.data() + trees.NonSymmetricNodeIdToLeafId[compact.Order[placed[at]].Node], dim, valueAt + static_cast<size_t>(at) * dim);
             } else {
-                *compactUsable = *compactUsable && splitOf(placed[at]) <= 255;
-                compactEntries->push_back((splitOf(placed[at]) & 0xffu) | bucketOf(placed[at]) << 8 | next << 21);
-            }
-            if (at < placed.size() && compact.Order[placed[at]].Terminal) {
-                const double* leaf = trees.LeafValues.data() + trees.NonSymmetricNodeIdToLeafId[compact.Order[placed[at]].Node];
-                valuesByEntry->insert(valuesByEntry->end(), leaf, leaf + dim);
-            } else {
-                valuesByEntry->insert(valuesByEntry->end(), static_cast<size_t>(dim), 0.0);
+                const uint32_t split = splitOf(placed[at]);
+                *compactUsable = *compactUsable && split <= 255;
+                entryAt[at] = (split & 0xffu) | bucketOf(placed[at]) << 8 | layout.Next[at] << 21;
             }
         }
     }
@@ -2591,14 +2602,23 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             // regions hold fewer trees per unit (kNsLdsShapes)
             m.NsLdsUsable = false;
             double bestCost = 0.0;
-            std::vector<TNsUnit> bestUnits;
+            struct TPlan {
+                bool Fits = false;
+                std::vector<TNsUnit> Units;
+            };
+            std::map<uint32_t, TPlan> plans;  // by the entries of a region
+            const std::vector<uint32_t> order = OrderNsTrees(compactRows, TreeCount);
             for (const TNsLdsShape& shape : kNsLdsShapes) {
                 if ((switches.NsWaves != 0 && switches.NsWaves != shape.Waves) ||
                     NsLdsKernelBytes(m.LayoutBuckets, shape.Waves, shape.Entries, NsLdsDims(m.Dim)) > kMaxTileLdsBytes) {
                     continue;
                 }
-                std::vector<TNsUnit> plan;
-                if (!PackNsUnits(compactRows, TreeCount, shape.Entries, &plan)) {
+                const auto [known, fresh] = plans.try_emplace(shape.Entries);
+                std::vector<TNsUnit>& plan = known->second.Units;
+                if (fresh) {
+                    known->second.Fits = PackNsUnits(compactRows, order, shape.Entries, &plan);
+                }
+                if (!known->second.Fits) {
                     continue;  // a tree larger than a region
                 }
                 uint64_t steps = 0;
@@ -2610,10 +2630,10 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     m.NsLdsUsable = true;
                     m.NsLdsShape = shape;
                     bestCost = cost;
-                    bestUnits.swap(plan);
                 }
             }
             if (m.NsLdsUsable) {
+                const std::vector<TNsUnit>& bestUnits = plans[m.NsLdsShape.Entries].Units;
                 // the entries in the order of the units; child indexes (bits 21-31) count from the unit's first entry (trees are
                 // whole pieces of eight entries, as a wave's copy of a unit, sixteen bytes per lane, needs pieces of four)
                 std::vector<uint32_t> entries, units;
@@ -2624,6 +2644,8 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                 const auto withTileRow = [&](uint32_t entry) {
                     return (entry & ~0x3ff00u) | dev::NsLdsTileRow((entry >> 8) & 0x3ffu, m.NsLdsShape.Waves, m.NsLdsShape.Entries) << 8;
                 };
+                std::vector<uint32_t> from;
+                std::vector<double> old;
                 for (const TNsUnit& unit : bestUnits) {
                     const uint32_t first = static_cast<uint32_t>(entries.size());
                     uint32_t start[dev::kNsUnitTrees] = {};
@@ -2634,18 +2656,18 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                         start[i] = count;
                         for (uint32_t e = 0; e < treeEntries; ++e) {
                             entries.push_back(withTileRow(compactEntries[treeFirst + e]) + (count << 21));
-                            const double* value = valuesByEntry.data() + static_cast<size_t>(treeFirst + e) * m.Dim;
-                            values.insert(values.end(), value, value + m.Dim);
                         }
+                        const double* value = valuesByEntry.data() + static_cast<size_t>(treeFirst) * m.Dim;
+                        values.insert(values.end(), value, value + static_cast<size_t>(treeEntries) * m.Dim);
                         count += treeEntries;
                     }
                     if (unit.Height == 0) {
-                        std::vector<uint32_t> from;
+                        from.clear();
                         for (uint32_t i = 0; i < unit.TreeCount; ++i) {
                             CompactNsExits(entries.data() + first + start[i], &from);
                         }
                         const size_t dim = static_cast<size_t>(m.Dim);
-                        const std::vector<double> old(values.begin() + static_cast<std::ptrdiff_t>(first * dim), values.end());
+                        old.assign(values.begin() + static_cast<std::ptrdiff_t>(first * dim), values.end());
                         for (size_t r = 0; r < from.size(); ++r) {
                             std::copy_n(old.data() + from[r] * dim, dim, values.data() + (first + r) * dim);
                         }
@@ -2915,8 +2937,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                                     (TreeCount / block + 3) * block * 256 * 8 + 16 * kFusedImageBytes < (uint64_t(1) << 32) - (1u << 20);
         const size_t bufferTrees = kFusedImageBytes / (variant->Leaves * sizeof(double));
         const size_t fusedTrees = fusedCandidate ? ((TreeCount + bufferTrees - 1) / bufferTrees + 2) * bufferTrees : 0;
-        std::vector<double> fusedLeafTable(leaves.begin(), leaves.begin() + (fusedCandidate ? std::min(leaves.size(), fusedTrees * variant->Leaves) : 0));
-        fusedLeafTable.resize(fusedTrees * variant->Leaves, 0.0);
+        const size_t fusedLeaves = fusedTrees * variant->Leaves;  // zeros behind the register kernel's
         for (int layoutIndex = 0; layoutIndex < 3 && fusedCandidate; ++layoutIndex) {
             const bool columnMajor = layoutIndex == 2;  // a value is a load of its own: units of any sixteen buckets
             const std::vector<uint32_t>& columns = layoutIndex == 1 ? srcSplit : srcFlat;
@@ -3013,7 +3034,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
             for (uint32_t b = 0; b < BucketCount && columnMajor; ++b) {
                 units[recordDwords + b] = columns[b];
             }
-            std::vector<uint8_t> table(images * kFusedImageBytes + fusedLeafTable.size() * sizeof(double), 0);
+            std::vector<uint8_t> table(images * kFusedImageBytes + fusedLeaves * sizeof(double), 0);
             for (uint32_t slot = 0; slot < fused->Buckets; ++slot) {
                 const uint32_t unit = slot / kFusedUnitColumns, column = slot % kFusedUnitColumns;
                 uint32_t* record = units.data() + static_cast<size_t>(unit) * kFusedUnitDwords;
@@ -3045,7 +3066,7 @@ THipEvaluator::THipEvaluator(const TModelTrees& trees, int deviceId, const std::
                     lut[c] = static_cast<uint8_t>(fused->Six ? start * 4 : start);  // the six-bit form stores byte offsets
                 }
             }
-            std::memcpy(table.data() + images * kFusedImageBytes, fusedLeafTable.data(), fusedLeafTable.size() * sizeof(double));
+            std::memcpy(table.data() + images * kFusedImageBytes, leaves.data(), std::min(leaves.size(), fusedLeaves) * sizeof(double));
             // level rows of the same form as the register kernel's, naming bins registers of this layout
             std::vector<uint32_t> fusedRows(rows);
             fusedRows.resize(std::max(fusedRows.size(), fusedTrees * rowDwords), 0);

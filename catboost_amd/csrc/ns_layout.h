@@ -22,11 +22,12 @@ struct TNsTreeLayout {
     // depth 2 over 100 features, values of three dimensions spread over 256 bytes instead of 128, 322 us a call, now 278.)
     std::vector<uint32_t> Next;
     uint32_t Steps = 0;           // from the exits to the farthest leaf
+    std::vector<uint32_t> PlaceOfPair, StepsFrom;  // scratch, by item and by place
 };
 
-// left: per item (the root first) the left child's item, which the right child follows; kNsNoItem: a leaf
-inline TNsTreeLayout LayOutNsTree(const std::vector<uint32_t>& left) {
-    TNsTreeLayout layout;
+// left: per item (the root first) the left child's item, which the right child follows; kNsNoItem: a leaf. A layout is filled anew by every
+// tree: models have thousands, and allocating five vectors for each takes longer than laying out a tree of one level.
+inline void LayOutNsTree(const std::vector<uint32_t>& left, TNsTreeLayout* layout) {
     // the item that a path of `levels` decisions (the root's the highest bit) leads to, a leaf if it ends there earlier
     const auto follow = [&](uint32_t path, int levels) {
         uint32_t item = 0;
@@ -38,23 +39,48 @@ inline TNsTreeLayout LayOutNsTree(const std::vector<uint32_t>& left) {
     for (uint32_t n = 0; n < 7; ++n) {
         const int level = n == 0 ? 0 : n < 3 ? 1 : 2;
         const uint32_t item = follow(n + 1 - (1u << level), level);
-        layout.TopItems[n] = left[item] == kNsNoItem ? kNsNoItem : item;
+        layout->TopItems[n] = left[item] == kNsNoItem ? kNsNoItem : item;
     }
     // a pair has one place, whichever items name it (those that a one-hot split repeats name their original's)
-    std::vector<uint32_t>& items = layout.Items;
-    items.reserve(left.size() + 8);
+    std::vector<uint32_t>&items = layout->Items, &next = layout->Next, &placeOfPair = layout->PlaceOfPair, &stepsFrom = layout->StepsFrom;
+    items.clear();
+    next.clear();
     for (uint32_t exit = 0; exit < 8; ++exit) {
         items.push_back(follow(exit, 3));
     }
-    std::vector<uint32_t> placeOfPair(left.size(), 0);  // by the left child's item; 0: none yet
+    placeOfPair.assign(left.size(), 0);  // by the left child's item; 0: none yet
+    bool repeats = false;
     for (uint32_t at = 0; at < items.size(); ++at) {
         const uint32_t child = left[items[at]];
-        if (child != kNsNoItem && placeOfPair[child] == 0) {
+        if (child == kNsNoItem) {
+            next.push_back(at);
+            continue;
+        }
+        if (placeOfPair[child] == 0) {
             placeOfPair[child] = static_cast<uint32_t>(items.size());
             items.push_back(child);
             items.push_back(child + 1);
+        } else {
+            repeats = true;
         }
-        layout.Next.push_back(child != kNsNoItem ? placeOfPair[child] : at);
+        next.push_back(placeOfPair[child]);
+    }
+    // A pair stands behind the place that names it but for repeated ones, whose steps are found by following the names
+    stepsFrom.assign(items.size(), repeats ? kNsNoItem : 0);
+    const auto follows = [&](const auto& self, uint32_t at) -> uint32_t {
+        if (stepsFrom[at] == kNsNoItem) {
+            stepsFrom[at] = left[items[at]] == kNsNoItem ? 0 : 1 + std::max(self(self, next[at]), self(self, next[at] + 1));
+        }
+        return stepsFrom[at];
+    };
+    for (uint32_t at = static_cast<uint32_t>(items.size()); !repeats && at-- > 0;) {
+        if (left[items[at]] != kNsNoItem) {
+            stepsFrom[at] = 1 + std::max(stepsFrom[next[at]], stepsFrom[next[at] + 1]);
+        }
+    }
+    layout->Steps = 0;
+    for (uint32_t exit = 0; exit < 8; ++exit) {
+        layout->Steps = std::max(layout->Steps, follows(follows, exit));
     }
     if (left.size() <= kNsSmallTreeItems) {
         for (uint32_t exit = 0; exit < 8; ++exit) {
@@ -64,25 +90,14 @@ inline TNsTreeLayout LayOutNsTree(const std::vector<uint32_t>& left) {
                 continue;
             }
             if (first < exit) {
-                layout.Next[exit] = layout.Next[first];
+                next[exit] = next[first];
             } else if (std::count(items.begin() + exit + 1, items.begin() + 8, item) > 0) {
-                layout.Next[exit] = static_cast<uint32_t>(items.size());
-                layout.Next.push_back(layout.Next[exit]);
+                next[exit] = static_cast<uint32_t>(items.size());
+                next.push_back(next[exit]);
                 items.push_back(item);
             }
         }
     }
-    std::vector<uint32_t> stepsFrom(left.size(), kNsNoItem);
-    const auto steps = [&](const auto& self, uint32_t item) -> uint32_t {
-        if (stepsFrom[item] == kNsNoItem) {
-            stepsFrom[item] = left[item] == kNsNoItem ? 0 : 1 + std::max(self(self, left[item]), self(self, left[item] + 1));
-        }
-        return stepsFrom[item];
-    };
-    for (uint32_t exit = 0; exit < 8; ++exit) {
-        layout.Steps = std::max(layout.Steps, steps(steps, items[exit]));
-    }
-    return layout;
 }
 
 // A terminal entry at a place: it selects itself from its pair (even: splitIdx 255, odd: splitIdx 0), and names the row of its leaf's values

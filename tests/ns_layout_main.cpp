@@ -9,13 +9,14 @@
 
 int main() {
     std::string line;
+    cbamd::TNsTreeLayout layout;  // the same for all of them, as in an evaluator
     while (std::getline(std::cin, line)) {
         std::istringstream in(line);
         std::vector<uint32_t> left;
         for (long item; in >> item;) {
             left.push_back(item < 0 ? cbamd::kNsNoItem : static_cast<uint32_t>(item));
         }
-        const cbamd::TNsTreeLayout layout = cbamd::LayOutNsTree(left);
+        cbamd::LayOutNsTree(left, &layout);
         std::printf("%u", layout.Steps);
         for (uint32_t item : layout.TopItems) {
             std::printf(" %d", static_cast<int>(item));
