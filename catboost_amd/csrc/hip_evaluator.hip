@@ -4077,7 +4077,10 @@ bool THipEvaluator::TakesSmallBatchKernel(size_t docCount, size_t treeStart, siz
 // and 32.4 us, 10 240 36.2 and 35.4, 12 400 43.2 and 36.9, 16 384 46.3 and 37.5 (columns of 50 features, 8300 documents 34.2 and 35.6, 16 384
 // 44.4 and 36.8); 1000 of depth 6 over 100, 12 288 30.1 and 31.5, 12 400 33.5 and 32.7, 16 384 35.3 and 32.8; 500 of depth 6
 // over 150, 16 384 28.1 and 30.7, 300 of depth 8 over 60 28.7 and 30.2. (One dimension on the register kernels; both add the same
-// slices. Other models keep the one limit.)
+// slices. Other models keep the one limit.) The columns to binarize are not looked at, and many of them cost the launches more than the lines suppose:
+// 12 289 documents, 501 trees of depth 8 over 200 columns 28.6 and 33.1 us, 833 of depth 6 over 222 31.2 and 35.5, where 563 of depth
+// 8 over 60 take 31.7 and 28.3. Of 696 batches of 4000 to 16 000 levels and 20 to 222 columns none is longer on the launches with lines at
+// 5000 and 6500 levels, and 12.5 and 20 more for every column beyond 100.
 bool THipEvaluator::TakesSmallBatchOnDevice(size_t docCount, size_t treeStart, size_t treeEnd) const {
     const TImpl& m = *Impl;
     const size_t levels = TreeCount * static_cast<size_t>(m.MaxDepth);
