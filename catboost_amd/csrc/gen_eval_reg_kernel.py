@@ -365,7 +365,7 @@ def gen_kernel(buckets, waves, pitch, leaves, mixed, six=False, fused=False, lev
 
     def merge_pairs(invert_top):
         """One select joins the bits of a pair, a shift and a select bring them into the index.
-        invert_top: the top bit of every index comes inverted (see gather_addresses)."""
+        invert_top: the top bit of every index comes inverted, for the product that makes places of them."""
         count = min(depth, 8)
         for pair in range(count // 2):
             select(sums[2 * pair], mask80, sums[2 * pair + 1], sums[2 * pair], invert_top and pair == count // 2 - 1)
